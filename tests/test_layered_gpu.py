@@ -202,6 +202,31 @@ def test_unequal_requests_share_passes_pages_and_slots(cases, dtype, tol):
     assert s.cache_usage() == (0, 8)
 
 
+@pytest.mark.parametrize("dim,vdim", [(5, 3), (64, 16), (65, 33), (128, 17), (129, 16), (256, 250)])
+@pytest.mark.parametrize("steep", [False, True])
+def test_runs_in_chunks_beside_short_ones(gpu, tmp_path, dim, vdim, steep):
+    """the recurrence in chunks of 16: runs around the line where it begins and around a chunk's end, beside shorter runs and single rows of the same
+    pass, twice in a row.  Steep: decays of down to exp(-90) a token, their products vanish inside a chunk"""
+    cfg = config(40, 50, [layer(attention(2, 2, 8, 8, 4, 7, 1), delta(3, 1, dim, vdim, 4), None, 0.0, 1.0)])
+    w = U.random_weights(cfg, dim + vdim)
+    if steep:
+        w["l0.mix.right.dt_bias"] = w["l0.mix.right.dt_bias"] + 16.0
+    c = Case(gpu, tmp_path, cfg, w=w)
+    first, second = (40, 1, 41, 39, 48, 83, 2), (1, 49, 57, 40, 3, 40, 64)
+    prompts = [tokens_for(cfg, a + b, i) for i, (a, b) in enumerate(zip(first, second))]
+    s = c.session("float32", len(prompts), 160)
+    got = [[] for _ in prompts]
+    for at, ns in (([0] * 7, first), (first, second)):
+        seq = [i for i, n in enumerate(ns) for _ in range(n)]
+        pos = [a + j for a, n in zip(at, ns) for j in range(n)]
+        lg, _ = s.forward_rows(seq, pos, [prompts[i][p] for i, p in zip(seq, pos)], range(len(seq)))
+        for r, i in enumerate(seq):
+            got[i].append(lg[r])
+    for p, rows in zip(prompts, got):
+        # steep: where next to nothing is left of a head's state its norm enlarges the rounding of single rows (token by token up to 3e-5 too)
+        assert U.rel_rms(np.array(rows), c.want(p)[0], 0.9 if steep else 1.0) < F32
+
+
 @pytest.mark.parametrize("dim,vdim", [(20, 20), (40, 36), (70, 17), (130, 20)])
 def test_many_heads_and_sequences(gpu, tmp_path, dim, vdim):
     """the recurrence's form for many columns at once: eight sequences of unequal length x 32 heads in one pass, then portions and single tokens"""

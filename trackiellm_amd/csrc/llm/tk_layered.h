@@ -96,7 +96,7 @@ protected:
 
 private:
     struct Seq { int len = 0, prev = -1, side = 0; std::vector<int32_t> pages; };
-    struct Pass { int nrows = 0, nseg = 0, ntiles = 0, nblocks = 0, nsums = 0; bool single = true, singles = true; }; /* all segments, or any, are single rows */
+    struct Pass { int nrows = 0, nseg = 0, longest = 0, shortest = 1 << 30, ntiles = 0, nblocks = 0, nsums = 0; bool single = true, singles = true; }; /* all segments, or any, are single rows */
     TkLayeredModel* m_ = nullptr;
     std::mutex mu_; /* seqs_, free_pages_, host page table */
     std::vector<Seq> seqs_;
@@ -111,7 +111,7 @@ private:
     size_t tab_ints_ = 0;
     TkPassTab tab_{};
     float *x_ = nullptr, *proj_ = nullptr, *low_ = nullptr, *y_ = nullptr, *router_ = nullptr, *scratch_ = nullptr;
-    float* sums_ = nullptr;
+    float *sums_ = nullptr, *chunks_ = nullptr;
     float *dq_ = nullptr, *dk_ = nullptr, *dv_ = nullptr, *dg_ = nullptr, *db_ = nullptr, *do_ = nullptr;
     void *img_x_ = nullptr, *img_low_ = nullptr, *img_mix_ = nullptr, *img_ff_ = nullptr, *img_gather_ = nullptr, *img_head_ = nullptr, *q_ = nullptr;
     TkMoeTab moe_{};

@@ -97,7 +97,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     h_pages_.assign((size_t)mseq * max_pages_, 0);
     for (int i = n_pages_ - 1; i >= 0; --i) free_pages_.push_back(i);
 
-    size_t proj = 16, low = 16, mix = 0, lowk = 0, q = 0, dq = 0, dv = 0, dg = 0, dh = 0, ff = 0, scratch = 0, E = 0, gather = 0, moe_ff = 0, assign = 0, moe_rows = 0, sums = 0;
+    size_t proj = 16, low = 16, mix = 0, lowk = 0, q = 0, dq = 0, dv = 0, dg = 0, dh = 0, ff = 0, scratch = 0, E = 0, gather = 0, moe_ff = 0, assign = 0, moe_rows = 0, sums = 0, chunks = 0;
     for (const TkLayerSpec& s : c.layers)
         for (const TkBranchSpec& b : s.branches)
             if (b.kind == TkBranchSpec::RETENTION) ret_heads_ = std::max(ret_heads_, b.retention.heads);
@@ -148,6 +148,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
                 dg = std::max(dg, (size_t)d.heads * d.dim);
                 dv = std::max(dv, (size_t)d.heads * d.vdim);
                 dh = std::max(dh, (size_t)d.heads);
+                chunks = std::max(chunks, tk_delta_chunk_floats(d.heads, d.dim, R, mseq));
             }
         }
         const TkMlpSpec& f = s.mlp;
@@ -167,7 +168,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
         !alloc((void**)&y_, yrows * c.width * 4, true) || !alloc(&img_x_, tk_img_bytes(type, R, c.width), true) || !alloc(&img_low_, lowk, true) ||
         !alloc(&img_mix_, mix, true) || !alloc(&img_ff_, std::max(ff, moe_ff), true) || !alloc(&img_head_, tk_img_bytes(type, TK_MAX_ROWS, c.width), true) ||
         !alloc(&q_, (size_t)R * q * esz, true) || !alloc((void**)&dq_, (size_t)R * dq * 4) || !alloc((void**)&dk_, (size_t)R * dq * 4) || !alloc((void**)&dv_, (size_t)R * dv * 4) ||
-        !alloc((void**)&sums_, sums * 4) || !alloc((void**)&dg_, (size_t)R * dg * 4) || !alloc((void**)&db_, (size_t)R * dh * 4) || !alloc((void**)&do_, (size_t)R * dv * 4) || !alloc((void**)&scratch_, scratch * 4))
+        !alloc((void**)&sums_, sums * 4) || (chunks && !alloc((void**)&chunks_, chunks * 4)) || !alloc((void**)&dg_, (size_t)R * dg * 4) || !alloc((void**)&db_, (size_t)R * dh * 4) || !alloc((void**)&do_, (size_t)R * dv * 4) || !alloc((void**)&scratch_, scratch * 4))
         return false;
     if (E && (!alloc((void**)&router_, (size_t)R * ((E + 15) / 16 * 16) * 4) || !alloc(&img_gather_, gather, true) || !alloc((void**)&moe_.count, E * 4, true) ||
               !alloc((void**)&moe_.expert, assign * 4) || !alloc((void**)&moe_.rank, assign * 4) || !alloc((void**)&moe_.weight, assign * 4) || !alloc((void**)&moe_.tile0, E * 4) ||
@@ -270,6 +271,8 @@ bool TkLayeredSession::describe(int nrows, const int32_t* seq, const int32_t* po
         sout[p->nseg] = 2 * id + (side ^ 1);
         for (int t = 0; t < n; t += 64, ++p->ntiles) { tiles[2 * p->ntiles] = r + t; tiles[2 * p->ntiles + 1] = std::min(64, n - t); }
         for (int i = 0; i < n; ++i) { h_seq[r + i] = id; h_pos[r + i] = pos[r + i]; h_tok[r + i] = tok[r + i]; h_seg[r + i] = p->nseg; }
+        p->longest = std::max(p->longest, n);
+        p->shortest = std::min(p->shortest, n);
         if (n > 1) {
             p->single = false;
             const int nb = (n + per - 1) / per;
@@ -377,7 +380,7 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
                 TkDeltaArgs d{};
                 d.heads = sp.heads; d.kv_heads = sp.kv_heads; d.dim = sp.dim; d.vdim = sp.vdim; d.taps = sp.taps; d.out_scale = bs.scale; d.eps = c.eps; d.unit_eps = sp.unit_eps;
                 d.col = B.col; d.conv = B.conv; d.a_log = B.a_log; d.dt_bias = B.dt_bias; d.norm = B.norm; d.low = low_; d.low_ld = L.low.N; d.low_a = B.low_a; d.low_g = B.low_g;
-                d.q = dq_; d.k = dk_; d.v = dv_; d.g = dg_; d.beta = db_; d.o = do_; d.conv_state = st.conv; d.state = st.state;
+                d.q = dq_; d.k = dk_; d.v = dv_; d.g = dg_; d.beta = db_; d.o = do_; d.conv_state = st.conv; d.state = st.state; d.chunks = chunks_;
                 d.out_img = img_mix_; d.out_k0 = B.out_k0; d.out_ktiles = L.out.K / kt;
                 ds.push_back(d);
             }
@@ -389,7 +392,7 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             tk_launch_mixer_prep(type, proj_, pitch, a, d, tab_, n, s);
             if (!p.single) {
                 if (a) tk_launch_attn_tiles(type, *a, tab_, d_tiles_, p.ntiles, s);
-                if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, n, s);
+                if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, p.shortest, p.longest, n, s);
                 continue;
             }
             const int splits = a ? tk_attn_rows_splits(*a, visible[ai], n) : 1;

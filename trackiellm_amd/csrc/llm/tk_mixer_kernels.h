@@ -57,6 +57,7 @@ struct TkDeltaArgs {
     float *q, *k, *v, *g, *beta, *o;  /* [rows][kv_heads dim], same, [rows][heads vdim], [rows][heads dim], [rows][heads], [rows][heads vdim] */
     float* conv_state;                /* [copies][channels][taps - 1] */
     float* state;                     /* [copies][heads][dim][vdim padded to 4] */
+    float* chunks;                    /* tk_delta_chunk_floats(): what the chunked scan knows of a chunk before its state */
     void* out_img;
     int out_k0, out_ktiles;
 };
@@ -92,8 +93,13 @@ void tk_launch_attn_rows(int type, const TkAttnArgs& a, const TkPassTab& t, int 
 int tk_attn_rows_splits(const TkAttnArgs& a, int pages, int nrows); /* for at most `pages` visible pages */
 size_t tk_attn_rows_scratch_floats(const TkAttnArgs& a, int nrows, int splits);
 
-/* the recurrence over every segment, token by token, and the gated per-head norm of its output */
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int nrows, hipStream_t s);
+/* the recurrence over every segment and the gated per-head norm of its output; shortest, longest: rows of the pass's shortest and longest segment.
+ * Segments of TK_DELTA_CHUNKED rows and more go in chunks, others token by token: a four-layer pass of one run takes 646 / 672 / 778 / 839 us token by
+ * token and 670 / 680 / 772 / 819 us in chunks at 24 / 32 / 48 / 64 rows */
+#define TK_DELTA_CHUNKED 40
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int longest, int nrows, hipStream_t s);
+/* of a pass of at most `rows` rows in at most `segments` segments (<= 256) */
+size_t tk_delta_chunk_floats(int heads, int dim, int rows, int segments);
 /* the same for passes whose segments are single rows: one launch */
 void tk_launch_delta_step(int type, const TkDeltaArgs& d, const TkPassTab& t, int nrows, hipStream_t s);
 

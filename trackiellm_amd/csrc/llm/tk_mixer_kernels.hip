@@ -799,13 +799,14 @@ __global__ __launch_bounds__(64) void k_attn_merge(TkAttnArgs a, int splits, con
  * leaves the wave.  q, k, decays, v and step sizes of TC tokens at a time go through LDS, the next TC in flight in registers.  32 lanes a column
  * where columns are few (the shorter chain), 16 where they are many (fewer operand reads per column). */
 template <int LN, int RPL>
-__global__ __launch_bounds__(256) void k_delta_scan(TkDeltaArgs d, TkPassTab t) {
+__global__ __launch_bounds__(256) void k_delta_scan(TkDeltaArgs d, TkPassTab t, int below /* segments of fewer rows */) {
     constexpr int DP = LN * RPL, TC = DP > 128 ? 8 : 16, NL = TC * DP / 256, CW = 64 / LN, NC = 4 * CW;
     __shared__ __attribute__((aligned(16))) float lq[2][TC][DP], lk[2][TC][DP], lg[2][TC][DP];
     __shared__ float lv[2][TC][NC], lb[2][TC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = blockIdx.y, seg = blockIdx.z, kvh = h / (d.heads / d.kv_heads), vp = (d.vdim + 3) & ~3;
     const int row0 = t.seg_row0[seg], n = t.seg_n[seg], in = t.seg_in[seg], out = t.seg_out[seg];
+    if (n >= below) return;
     const int cl = wave * CW + lane / LN, col = blockIdx.x * NC + cl, r0 = (lane % LN) * RPL;
     const bool live = col < d.vdim;
     float S[RPL];
@@ -862,6 +863,231 @@ __global__ __launch_bounds__(256) void k_delta_scan(TkDeltaArgs d, TkPassTab t) 
 #pragma unroll
         for (int i = 0; i < RPL; ++i)
             if (r0 + i < d.dim) d.state[(((size_t)out * d.heads + h) * d.dim + r0 + i) * vp + col] = S[i];
+}
+
+/* ---- the same in chunks of 16 tokens, for long runs ----
+ * With G_t = g_1 .. g_t (per key row) inside a chunk that starts from S, the corrections u_t = beta_t (v_t - S_t'^T k_t) solve a unit lower triangular
+ * system, and everything else is four small products:
+ *   u = T v - W S,   W = T (G k),   T = (I + L)^-1 diag(beta),   L[t][j] = beta_t k_t . (G_t / G_j) k_j   (j < t)
+ *   o = (G q) S + B u,              B[t][j] = q_t . (G_t / G_j) k_j                                      (j <= t)
+ *   S <- G_16 S + sum_j (G_16 / G_j) k_j u_j^T
+ * Ratios are running products of decays, never quotients or logarithms: a decay of zero is as good as any other.  All of it is f32 (v_mfma_f32_16x16x4).
+ * Token by token a step is one dependent chain of ~650 cycles whatever the chip has free (558 us for 2047 tokens x 16 heads of 128 x 128); here what
+ * does not depend on the state is done for all chunks at once (k_delta_chunk, 31 us), and the chain is ~2000 cycles for 16 tokens (k_delta_chain, 108 us).
+ * Its error against 64 bits is that of the token by token form (2.8e-6 of the logits of float32 models, 2.7e-6). */
+constexpr int DC = 16; /* tokens of a chunk */
+constexpr size_t delta_slot_floats(int dp) { return (size_t)(3 * DC + 1) * dp + 2 * DC * DC; }
+static int delta_pad(int dim) { return dim <= 64 ? 64 : dim <= 128 ? 128 : 256; }
+/* a segment's chunks are consecutive slots; room for every segment's last, partly filled one */
+__device__ __forceinline__ int delta_slot0(int row0, int seg) { return row0 / DC + seg; }
+
+/* lane i of every four: its elements 0 .. 3 -> element i of the lanes 0 .. 3 */
+__device__ __forceinline__ tk_v4f quad_transpose(tk_v4f v) {
+    const bool b0 = threadIdx.x & 1, b1 = threadIdx.x & 2;
+    const float s0 = tk_dpp<0xB1>(b0 ? v[0] : v[1]), s1 = tk_dpp<0xB1>(b0 ? v[2] : v[3]);
+    v = b0 ? tk_v4f{s0, v[1], s1, v[3]} : tk_v4f{v[0], s0, v[2], s1};
+    const float t0 = tk_dpp<0x4E>(b1 ? v[0] : v[2]), t1 = tk_dpp<0x4E>(b1 ? v[1] : v[3]);
+    return b1 ? tk_v4f{t0, t1, v[2], v[3]} : tk_v4f{v[0], v[1], t0, t1};
+}
+
+/* One chunk of one head: W, G q and the decayed keys (each as the operand k_delta_chain wants it, 16 bytes a lane), G_16, T, B.
+ * Bound by LDS reads and the vector work they feed; 2047 tokens x 16 heads are eight workgroups per CU, 31 us (53 us with one token j and eight key
+ * rows a thread and results stored four bytes at a time). */
+template <int DP>
+__global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t, int nseg) {
+    constexpr int PE = DP / 32; /* key rows of a thread in the pair products */
+    __shared__ __attribute__((aligned(16))) float lq[DC][DP], lk[DC][DP], lg[DC][DP], L[DC][DC], B[DC][DC], lb[DC];
+    const int tid = threadIdx.x, slot = blockIdx.y, h = blockIdx.x, kvh = h / (d.heads / d.kv_heads);
+    const int seg = __syncthreads_count(tid < nseg && delta_slot0(t.seg_row0[tid < nseg ? tid : 0], tid) <= slot) - 1;
+    if (seg < 0) return;
+    const int t0 = (slot - delta_slot0(t.seg_row0[seg], seg)) * DC, n = t.seg_n[seg];
+    if (t0 >= n || n < TK_DELTA_CHUNKED) return;
+    const int m = n - t0 < DC ? n - t0 : DC, row0 = t.seg_row0[seg] + t0;
+    float* const w = d.chunks + ((size_t)slot * d.heads + h) * delta_slot_floats(DP);
+    float *const wq = w + DC * DP, *const wk = wq + DC * DP, *const wg = wk + DC * DP, *const wt = wg + DP, *const wb = wt + DC * DC;
+#pragma unroll
+    for (int i = 0; i < DC * DP / 256; ++i) {
+        const int idx = tid + 256 * i, tt = idx / DP, e = idx % DP;
+        const bool ok = tt < m && e < d.dim;
+        const size_t row = row0 + (ok ? tt : 0), at = ok ? e : 0; /* no branch around a load: all of them are in flight together */
+        const float q = d.q[(row * d.kv_heads + kvh) * d.dim + at], k = d.k[(row * d.kv_heads + kvh) * d.dim + at], g = d.g[(row * d.heads + h) * d.dim + at];
+        lq[tt][e] = ok ? q : 0.0f;
+        lk[tt][e] = ok ? k : 0.0f;
+        lg[tt][e] = ok ? g : 1.0f;
+    }
+    if (tid < DC) lb[tid] = tid < m ? d.beta[(size_t)(row0 + tid) * d.heads + h] : 0.0f;
+    L[tid / DC][tid % DC] = 0.0f;
+    B[tid / DC][tid % DC] = 0.0f;
+    __syncthreads();
+    { /* a thread has two tokens j and PE key rows, a wave four tokens: those that have not come yet wait */
+        const int j = tid / 32 * 2, e0 = tid % 32 * PE, jw = __builtin_amdgcn_readfirstlane(tid / 64 * 4);
+        float p[2][PE];
+#pragma unroll
+        for (int e = 0; e < PE; ++e) { p[0][e] = lk[j][e0 + e]; p[1][e] = lk[j + 1][e0 + e]; }
+        for (int tt = jw; tt < m; ++tt) {
+            float a[2] = {0.0f, 0.0f}, b[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int e = 0; e < PE; ++e) {
+                const float g = lg[tt][e0 + e], k = lk[tt][e0 + e], q = lq[tt][e0 + e];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    p[i][e] *= tt > j + i ? g : 1.0f;
+                    a[i] = fmaf(p[i][e], k, a[i]);
+                    b[i] = fmaf(p[i][e], q, b[i]);
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i) { a[i] = tk_row32_sum(a[i]); b[i] = tk_row32_sum(b[i]); }
+            if (tid % 32 < 2) {
+                const int i = tid % 32, jj = j + i;
+                if (tt > jj) L[tt][jj] = lb[tt] * (i ? a[1] : a[0]);
+                if (tt >= jj) B[tt][jj] = i ? b[1] : b[0];
+            }
+        }
+        /* tokens past the run's end decay nothing.  The halves of the wave trade so that a lane has the four tokens of PE / 2 key rows */
+#pragma unroll
+        for (int e = 0; e < PE / 2; ++e) {
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[0][e]), __float_as_uint(p[0][e + PE / 2]), false, false);
+            const auto y = __builtin_amdgcn_permlane32_swap(__float_as_uint(p[1][e]), __float_as_uint(p[1][e + PE / 2]), false, false);
+            const int k = e0 + e + (tid & 32 ? PE / 2 : 0);
+            *(tk_v4f*)(wk + ((k >> 4) * 64 + (jw >> 2) * 16 + (k & 15)) * 4) =
+                tk_v4f{__uint_as_float(x[0]), __uint_as_float(y[0]), __uint_as_float(x[1]), __uint_as_float(y[1])};
+        }
+    }
+    __syncthreads();
+    /* columns of W (key rows) and of T (tokens): forward substitution, a thread a column */
+    for (int c = tid; c < DP + DC; c += 256) {
+        float x[DC], q[DC];
+        if (c < DP) {
+            float g = 1.0f;
+#pragma unroll
+            for (int tt = 0; tt < DC; ++tt) {
+                g *= lg[tt][c];
+                x[tt] = lb[tt] * (g * lk[tt][c]);
+                q[tt] = g * lq[tt][c];
+            }
+            wg[c] = g;
+        } else {
+#pragma unroll
+            for (int tt = 0; tt < DC; ++tt) x[tt] = tt == c - DP ? lb[tt] : 0.0f;
+        }
+#pragma unroll
+        for (int tt = 1; tt < DC; ++tt)
+#pragma unroll
+            for (int j = 0; j < tt; ++j) x[tt] = fmaf(-L[tt][j], x[j], x[tt]);
+        if (c < DP) { /* whole waves: four lanes trade their columns for tokens and store 16 bytes each */
+            const size_t at = ((c >> 4) * 64 + ((c >> 2) & 3) * 16 + (c & 3)) * 4;
+#pragma unroll
+            for (int i = 0; i < DC; i += 4) {
+                *(tk_v4f*)(w + at + 4 * i) = quad_transpose(tk_v4f{-x[i], -x[i + 1], -x[i + 2], -x[i + 3]});
+                *(tk_v4f*)(wq + at + 4 * i) = quad_transpose(tk_v4f{q[i], q[i + 1], q[i + 2], q[i + 3]});
+            }
+        } else {
+            const int k = c - DP;
+#pragma unroll
+            for (int tt = 0; tt < DC; ++tt) wt[((k >> 2) * 16 + tt) * 4 + (k & 3)] = x[tt];
+        }
+    }
+    wb[((tid % DC >> 2) * 16 + tid / DC) * 4 + (tid & 3)] = B[tid / DC][tid % DC];
+}
+
+/* The chunks of a segment in order: a workgroup owns 16 columns of one head's state, each of its four waves a quarter of the key rows, in
+ * accumulator registers, which are at once the products' right-hand operands.  Per chunk 26 MFMAs a wave and one barrier: the partial sums of W S
+ * meet in LDS, every wave adds them up (ascending) and goes on; those of the output are added a chunk later, off the chain.  Operands are requested
+ * three chunks ahead. */
+template <int DP>
+__global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t) {
+    constexpr int NT = DP / 64, AHEAD = 3;
+    __shared__ tk_v4f pu[2][4][64], po[2][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4;
+    const int h = blockIdx.x, seg = blockIdx.z, vp = (d.vdim + 3) & ~3, col = blockIdx.y * 16 + (lane & 15);
+    const int row0 = t.seg_row0[seg], n = t.seg_n[seg], in = t.seg_in[seg], out = t.seg_out[seg];
+    if (n < TK_DELTA_CHUNKED) return;
+    const bool live = col < d.vdim;
+    const int nc = (n + DC - 1) / DC;
+    tk_v4f S[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int e = (wave * NT + i) * 16 + 4 * g + r;
+            S[i][r] = in >= 0 && live && e < d.dim ? d.state[(((size_t)in * d.heads + h) * d.dim + e) * vp + col] : 0.0f;
+        }
+    struct Ops { tk_v4f w[NT], q[NT], k[NT], g[NT]; float t, b, v; } ops[AHEAD + 1];
+    const size_t step = (size_t)d.heads * delta_slot_floats(DP);
+    const float* const base = d.chunks + ((size_t)delta_slot0(row0, seg) * d.heads + h) * delta_slot_floats(DP);
+    auto fetch = [&](Ops& o, int c) {
+        const float* p = base + (size_t)c * step;
+        const int tile = wave * NT;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            o.w[i] = *(const tk_v4f*)(p + ((tile + i) * 64 + lane) * 4);
+            o.q[i] = *(const tk_v4f*)(p + DC * DP + ((tile + i) * 64 + lane) * 4);
+            o.k[i] = *(const tk_v4f*)(p + 2 * DC * DP + ((tile + i) * 64 + lane) * 4);
+            o.g[i] = *(const tk_v4f*)(p + 3 * DC * DP + (tile + i) * 16 + 4 * g);
+        }
+        /* T v and B u: wave w adds the tokens 4 g + w */
+        o.t = p[(3 * DC + 1) * DP + lane * 4 + wave];
+        o.b = p[(3 * DC + 1) * DP + DC * DC + lane * 4 + wave];
+        const int tt = c * DC + 4 * g + wave;
+        /* past the run's end, and in columns that do not exist, any number will do: their T is zero, their results are not stored */
+        o.v = d.v[((size_t)(row0 + (tt < n ? tt : c * DC)) * d.heads + h) * d.vdim + (live ? col : 0)];
+    };
+    const int ot = tid >> 4, oc = blockIdx.y * 16 + (tid & 15); /* the output element this thread finishes */
+    auto finish = [&](int c) {
+        const int l = (ot >> 2) * 16 + (tid & 15), b = c & 1;
+        const float o = ((po[b][0][l][ot & 3] + po[b][1][l][ot & 3]) + po[b][2][l][ot & 3]) + po[b][3][l][ot & 3];
+        if (c >= 0 && c * DC + ot < n && oc < d.vdim) d.o[((size_t)(row0 + c * DC + ot) * d.heads + h) * d.vdim + oc] = o;
+    };
+    auto chunk = [&](Ops& o, Ops& next, int c) {
+        fetch(next, c + AHEAD < nc ? c + AHEAD : nc - 1); /* never skipped: a branch here would make every wait one for the youngest request */
+        tk_v4f u = {0.0f, 0.0f, 0.0f, 0.0f}, y = u;
+        u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t, o.v, u, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.w[i][r], S[i][r], u, 0, 0, 0);
+        const int b = c & 1;
+        pu[b][wave][lane] = u;
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) y = __builtin_amdgcn_mfma_f32_16x16x4f32(o.q[i][r], S[i][r], y, 0, 0, 0);
+        /* pu[b] was last read two chunks ago, po[b] one barrier ago */
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        u = ((pu[b][0][lane] + pu[b][1][lane]) + pu[b][2][lane]) + pu[b][3][lane];
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            S[i] *= o.g[i];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[i][r], u[r], S[i], 0, 0, 0);
+        }
+        y = __builtin_amdgcn_mfma_f32_16x16x4f32(o.b, u[wave & 3], y, 0, 0, 0);
+        finish(c - 1);
+        po[b][wave][lane] = y;
+    };
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) fetch(ops[i], i < nc ? i : nc - 1);
+    int c = 0;
+    for (; c + 4 <= nc; c += 4) {
+        chunk(ops[0], ops[3], c);
+        chunk(ops[1], ops[0], c + 1);
+        chunk(ops[2], ops[1], c + 2);
+        chunk(ops[3], ops[2], c + 3);
+    }
+    if (c < nc) chunk(ops[0], ops[3], c);
+    if (c + 1 < nc) chunk(ops[1], ops[0], c + 1);
+    if (c + 2 < nc) chunk(ops[2], ops[1], c + 2);
+    __syncthreads();
+    finish(nc - 1);
+    if (live)
+#pragma unroll
+        for (int i = 0; i < NT; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = (wave * NT + i) * 16 + 4 * g + r;
+                if (e < d.dim) d.state[(((size_t)out * d.heads + h) * d.dim + e) * vp + col] = S[i][r];
+            }
 }
 
 /* o over its root mean square, times the norm's weight, times the gate: one wave per (row, head) */
@@ -1639,15 +1865,29 @@ bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, 
     return true;
 }
 
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int nrows, hipStream_t s) {
-    const bool many = (int64_t)((d.vdim + 15) / 16) * d.heads * n_segments >= 512;
-    const dim3 grid(many ? (d.vdim + 15) / 16 : (d.vdim + 7) / 8, d.heads, n_segments);
-#define TK_SCAN(RPL) do { if (many) hipLaunchKernelGGL((k_delta_scan<16, 2 * RPL>), grid, dim3(256), 0, s, d, t); else hipLaunchKernelGGL((k_delta_scan<32, RPL>), grid, dim3(256), 0, s, d, t); } while (0)
-    if (d.dim <= 32) TK_SCAN(1);
-    else if (d.dim <= 64) TK_SCAN(2);
-    else if (d.dim <= 128) TK_SCAN(4);
-    else TK_SCAN(8);
+size_t tk_delta_chunk_floats(int heads, int dim, int rows, int segments) { return (size_t)(rows / DC + segments) * heads * delta_slot_floats(delta_pad(dim)); }
+
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int longest, int nrows, hipStream_t s) {
+    if (longest >= TK_DELTA_CHUNKED) {
+        const dim3 chunks(d.heads, nrows / DC + n_segments), chain(d.heads, (d.vdim + 15) / 16, n_segments); /* heads first: a head's workgroups share an XCD's L2 */
+#define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_segments); hipLaunchKernelGGL((k_delta_chain<DP>), chain, dim3(256), 0, s, d, t); } while (0)
+        switch (delta_pad(d.dim)) {
+            case 64: TK_CHUNKED(64); break;
+            case 128: TK_CHUNKED(128); break;
+            default: TK_CHUNKED(256);
+        }
+#undef TK_CHUNKED
+    }
+    if (shortest < TK_DELTA_CHUNKED) {
+        const bool many = (int64_t)((d.vdim + 15) / 16) * d.heads * n_segments >= 512;
+        const dim3 grid(many ? (d.vdim + 15) / 16 : (d.vdim + 7) / 8, d.heads, n_segments);
+#define TK_SCAN(RPL) do { if (many) hipLaunchKernelGGL((k_delta_scan<16, 2 * RPL>), grid, dim3(256), 0, s, d, t, TK_DELTA_CHUNKED); else hipLaunchKernelGGL((k_delta_scan<32, RPL>), grid, dim3(256), 0, s, d, t, TK_DELTA_CHUNKED); } while (0)
+        if (d.dim <= 32) TK_SCAN(1);
+        else if (d.dim <= 64) TK_SCAN(2);
+        else if (d.dim <= 128) TK_SCAN(4);
+        else TK_SCAN(8);
 #undef TK_SCAN
+    }
     TK_TYPED(type, hipLaunchKernelGGL((k_delta_out<T>), dim3((d.heads + 3) / 4, nrows), dim3(256), 0, s, d));
 }
 
