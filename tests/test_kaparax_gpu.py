@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 
 import layered_util as U
-from layered_util import LO, Case, chunked, greedy, kaparax, no_end, retention, runner_ids, serial, tokens_for
+from layered_util import F32, LO, Case, chunked, greedy, kaparax, no_end, retention, runner_ids, serial, tokens_for
 
 pytestmark = pytest.mark.gpu
 
@@ -411,3 +411,19 @@ def test_trace_runner(cases, tmp_path):
         read = lambda i: np.fromfile(out / ("%d.f32" % i), "<f4").reshape(-1, c.cfg["vocab"])
         assert near(read(0), A[[69, 3, 3]], dtype) and near(read(1), A[[70]], dtype)
         assert near(read(2), A[[89]], dtype) and near(read(3), B[[32, 31]], dtype)
+
+
+@pytest.mark.parametrize("dtype,tol", [("float32", F32), ("bfloat16", 0.007)])
+@pytest.mark.parametrize("width,ff,rows", [(2064, 8190, 901), (2064, 8190, 1303), (1040, 5000, 1100), (1040, 2000, 2047), (528, 1500, 1100), (528, 1500, 300), (528, 700, 81)])
+def test_products_in_large_blocks(gpu, width, ff, rows, dtype, tol):
+    """passes whose products take 256 x 256, 256 x 128, 128 x 128, 128 x 64 and 128 x 32 blocks, with rows, columns and k that fill none of them, against
+    the same rows in passes of 61, which take another kernel (other tests hold that one against the restatement).  bf16: where a sum rounds to the other
+    neighbour the next products carry 2^-8 of that element on (0.0018 measured; a block with one wrong tile of sixteen is off by 0.2)"""
+    n = width // 16
+    cfg = kaparax(width, 64, [serial(chunked(n, n, 16, 16, 16, 48, 2, 20.0), (ff, 7.0))])
+    m = gpu.LlmModel(config=cfg, dtype=dtype, seed=3)
+    toks = tokens_for(cfg, rows, 5)
+    s = gpu.LlmSession(m, 2, 2048)
+    whole = s.forward_streams([0] * rows, range(rows), toks)[0]
+    parts = [s.forward_streams([1] * len(toks[i:i + 61]), range(i, i + len(toks[i:i + 61])), toks[i:i + 61])[0] for i in range(0, rows, 61)]
+    assert U.rel_rms(whole, np.concatenate(parts)) < tol

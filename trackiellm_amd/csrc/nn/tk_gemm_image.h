@@ -10,7 +10,7 @@
  *   instruction are element t of the four lane groups on both sides, an order of the same sum).
  *
  * Two kernels: a skinny one (up to 64 rows per block: the waves of a workgroup split K and stream the weights once from HBM to registers) and a
- * wide one (128 rows x 32 .. 128 columns per workgroup, both operands through a double-buffered LDS image filled by LDS-DMA).  Either can take
+ * wide one (128 or 256 rows x 32 .. 256 columns per workgroup, both operands through a ring of LDS stages filled by LDS-DMA).  Either can take
  * its row blocks from a table that names a weight matrix per block (mixture of experts: one launch over all experts).
  */
 #ifndef TK_GEMM_IMAGE_H
@@ -34,7 +34,7 @@ struct TkImgBlock { int32_t group, tile0, ntiles, pad; };
 struct TkImgGemm {
     int type;            /* TkImgType of both operands */
     const void* w;       /* image [N][K] */
-    const void* a;       /* image [rows][K]; allocated for rows rounded up to 128 */
+    const void* a;       /* image [rows][K] */
     int K;               /* padded */
     int N;               /* rows of the weight image, padded to 16 (32 with swiglu) */
     int nrows;           /* rows of A (grouped: unused) */

@@ -3,6 +3,7 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "tk_image_device.h"
 
@@ -134,12 +135,19 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
 /* s_waitcnt vmcnt(N): all but this wave's N youngest vector-memory requests are done */
 template <int N> __device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | (N >> 4) << 14); }
 
-/* ---- wide: 128 rows x 16 * NBT columns per workgroup, waves 2 x 2, two k tiles per stage, a ring of LDS stages filled by LDS-DMA ---- */
-template <int NBT> constexpr int wide_ring() { return NBT == 8 ? 2 : NBT == 4 ? 3 : 4; } /* stages: as many as let two workgroups share a CU */
-template <typename T, int NBT /* column tiles of the workgroup: 2, 4, 8 */, bool SWIGLU, bool GROUPED>
-__global__ __launch_bounds__(256) void k_gemm_wide(TkImgGemm a, int nblk_n, int nblk_m, int ks) {
-    constexpr int MBT = 8, NW = NBT / 2, MW = MBT / 2; /* tiles of one wave */
-    constexpr int STAGE = (MBT + NBT) * 2 * 1024, RING = wide_ring<NBT>();
+/* ---- wide: 16 MBT rows x 16 NBT columns per workgroup of WM x WN waves, two k tiles per stage, a ring of LDS stages filled by LDS-DMA ----
+ * A block of R x C reads (R + C) k operands for R C k products, so large blocks are what the L2s can feed; a wave of MW x NW tiles takes (MW + NW) KiB of
+ * LDS for MW NW MFMAs.  What is left is latency: all waves of a CU meet at the same barrier, and whatever stands between it and the next MFMA is lost
+ * by all of them.  So a k tile's operands are read while the tile before it is multiplied, the requests for a later stage are spread between MFMAs, and
+ * the loop over them has no branch.  2048 x 28672 x 4096 (gate | up): 502 us with 128 x 128 blocks read and multiplied in turn, 414 us with 256 x 256
+ * ones, 382 us (1.26 PF/s) with the reads and requests between the MFMAs; 2047 x 4096 x 14336 (down): 214 -> 180 us (1.33 PF/s). */
+constexpr int wide_stage(int mbt, int nbt) { return (mbt + nbt) * 2048; }
+template <typename T, int MBT, int NBT, int WM, int WN, int RING, bool SWIGLU, bool GROUPED>
+__global__ __launch_bounds__(64 * WM * WN) void k_gemm_wide(TkImgGemm a, int nblk_n, int nblk_m, int ks) {
+    constexpr int NW = NBT / WN, MW = MBT / WM; /* tiles of one wave */
+    constexpr int STAGE = wide_stage(MBT, NBT);
+    static_assert(!SWIGLU || NW % 2 == 0, "a wave has gate and up tiles in pairs");
+    static_assert(MW >= 1 && NW >= 1 && (MBT + NBT) * 2 % (WM * WN) == 0, "every wave has tiles, and as many pieces of a stage as the others");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     /* workgroups go to the eight XCDs in turn: give each XCD a contiguous range of blocks (row blocks fastest) so that it re-reads the same
@@ -163,56 +171,87 @@ __global__ __launch_bounds__(256) void k_gemm_wide(TkImgGemm a, int nblk_n, int 
     }
     if (mlive > MBT) mlive = MBT;
     const int ntot = a.N / 16, n0 = bn * NBT;
-    constexpr int PIECES = (MBT + NBT) * 2, PPW = PIECES / 4;
-    const uint8_t* src[PPW];
+    constexpr int PPW = (MBT + NBT) * 2 / (WM * WN); /* pieces of a stage per wave */
+    const uint8_t* src[PPW]; /* the same for all lanes */
 #pragma unroll
     for (int i = 0; i < PPW; ++i) { /* piece p: tile p / 2 (M-tiles first, then column tiles), k tile p % 2 of the stage */
         const int p = wave * PPW + i, t = p >> 1, k0 = 2 * s0 + (p & 1);
-        if (t < MBT) src[i] = (const uint8_t*)a.a + ((size_t)(m0 + (t < mlive ? t : 0)) * ktiles + k0) * 1024 + lane * 16;
+        if (t < MBT) src[i] = (const uint8_t*)a.a + ((size_t)(m0 + (t < mlive ? t : 0)) * ktiles + k0) * 1024;
         else {
             const int nt = n0 + t - MBT < ntot ? n0 + t - MBT : ntot - 1;
-            src[i] = wbase + ((size_t)nt * ktiles + k0) * 1024 + lane * 16;
+            src[i] = wbase + ((size_t)nt * ktiles + k0) * 1024;
         }
     }
+    const int lane16 = lane * 16;
     auto stage = [&](int buf) {
 #pragma unroll
         for (int i = 0; i < PPW; ++i) {
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src[i],
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + lane16),
                                              (__attribute__((address_space(3))) void*)(lds + buf * STAGE + (wave * PPW + i) * 1024), 16, 0, 0);
             src[i] += 2048;
         }
     };
-    const int wm = (wave & 1) * MW, wn = (wave >> 1) * NW;
+    const int wm = wave % WM * MW, wn = wave / WM * NW;
     tk_v4f acc[NW][MW];
 #pragma unroll
     for (int n = 0; n < NW; ++n)
 #pragma unroll
         for (int m = 0; m < MW; ++m) acc[n][m] = tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    for (int s = 0; s < RING - 1 && s < stages; ++s) stage(s);
-    int cur = 0, fill = RING - 1;
-#pragma unroll 1
-    for (int s = 0; s < stages; ++s) {
-        /* stage s has landed when at most the RING - 2 younger ones are outstanding (at the end there are fewer: wait for all) */
-        if (s + RING - 1 <= stages) wait_vm<(RING - 2) * PPW>();
-        else wait_vm<0>();
-        asm volatile("s_barrier" ::: "memory"); /* every wave's pieces of stage s have landed, and every wave has read stage s - 1, whose place is filled next */
-        if (s + RING - 1 < stages) stage(fill);
-        const uint8_t* b = lds + cur * STAGE + lane * 16;
-        cur = cur + 1 < RING ? cur + 1 : 0;
-        fill = fill + 1 < RING ? fill + 1 : 0;
+    struct Ops { tk_v4u a[MW], w[NW]; } x, y;
+    auto read = [&](Ops& o, int buf, int k) {
+        const uint8_t* b = lds + buf * STAGE + lane16;
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            tk_v4u av[MW], wv[NW];
+        for (int n = 0; n < NW; ++n) o.w[n] = *(const tk_v4u*)(b + ((MBT + wn + n) * 2 + k) * 1024);
 #pragma unroll
-            for (int m = 0; m < MW; ++m) av[m] = *(const tk_v4u*)(b + ((wm + m) * 2 + k) * 1024);
+        for (int m = 0; m < MW; ++m) o.a[m] = *(const tk_v4u*)(b + ((wm + m) * 2 + k) * 1024);
+    };
+    auto multiply = [&](const Ops& o) {
 #pragma unroll
-            for (int n = 0; n < NW; ++n) wv[n] = *(const tk_v4u*)(b + ((MBT + wn + n) * 2 + k) * 1024);
+        for (int m = 0; m < MW; ++m)
 #pragma unroll
-            for (int n = 0; n < NW; ++n)
+            for (int n = 0; n < NW; ++n) acc[n][m] = TkImg<T>::mma(o.w[n], o.a[m], acc[n][m]);
+    };
+    /* a k tile's operands are read, and `dma` pieces of a later stage requested, between the MFMAs of the tile before it */
+    auto weave = [&](auto dma) {
+        constexpr int READS = MW + NW, MFMAS = MW * NW * (sizeof(T) == 4 ? 4 : 1), EACH = MFMAS / READS;
 #pragma unroll
-                for (int m = 0; m < MW; ++m) acc[n][m] = TkImg<T>::mma(wv[n], av[m], acc[n][m]);
+        for (int i = 0; i < READS; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x8, EACH, 0);
+            if (i < dma.value) __builtin_amdgcn_sched_group_barrier(0x10, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
-    }
+        if (MFMAS % READS) __builtin_amdgcn_sched_group_barrier(0x8, MFMAS % READS, 0);
+    };
+    /* stages s + 1 .. s + RING - 1 are in flight while stage s is multiplied; a stage's place is free once every wave has its operands in registers */
+    for (int s = 0; s < RING && s < stages; ++s) stage(s);
+    if (stages >= RING) wait_vm<(RING - 1) * PPW>();
+    else wait_vm<0>();
+    asm volatile("s_barrier" ::: "memory");
+    read(x, 0, 0);
+    int cur = 0;
+    auto step = [&](auto more) {
+        const int next = cur + 1 < RING ? cur + 1 : 0;
+        read(y, cur, 1);
+        multiply(x);
+        weave(std::integral_constant<int, 0>{});
+        if (more.value) wait_vm<(RING - 2) * PPW>(); /* the next stage: all but the RING - 2 after it */
+        else wait_vm<0>();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); /* the next stage is there, and this one is in everybody's registers */
+        if (more.value) stage(cur);
+        read(x, next, 0);
+        multiply(y);
+        weave(std::integral_constant<int, more.value ? PPW : 0>{});
+        cur = next;
+    };
+    int s = 0;
+#pragma unroll 1
+    for (; s + RING < stages; ++s) step(std::true_type{});
+#pragma unroll 1
+    for (; s + 1 < stages; ++s) step(std::false_type{});
+    read(y, cur, 1);
+    multiply(x);
+    weave(std::integral_constant<int, 0>{});
+    multiply(y);
 #pragma unroll
     for (int m = 0; m < MW; ++m) {
         const int64_t row = (int64_t)(m0 + wm + m) * 16 + (lane & 15);
@@ -240,6 +279,41 @@ __global__ void k_put_image(const void* src, int src_f32, int64_t N, int64_t K, 
     tk_img_put(img, row, (int)k0 + k, ktiles, v);
 }
 
+/* The forms of the wide kernel and what they cost: rounds of workgroups x (their start and end + k x time per k), fitted to products of 100 .. 2047 rows
+ * whose weights come from memory (within ~15 %).  Large blocks where they fill the chip once or several times, smaller ones where larger would leave CUs
+ * idle.  Of forms that run two to a CU a last round of at most 256 runs one to a CU. */
+struct WideForm { int mb, nb, per_cu; float start, k, start2, k2; }; /* tiles; us, ns per k of a round with one workgroup per CU, and with two */
+constexpr WideForm wide_forms[] = {
+    {16, 16, 1, 22.0f, 17.5f, 0.0f, 0.0f}, /* 1750 x 28672 x 4096: 372 us (next best 379) */
+    {16, 8, 1, 8.0f, 12.0f, 0.0f, 0.0f},   /* 2047 x 4096 x 14336: 182 us (242) */
+    {8, 8, 2, 6.0f, 11.8f, 8.0f, 15.0f},   /* 1100 x 28672 x 4096: 248 us (271) */
+    {8, 8, 1, 10.0f, 7.0f, 0.0f, 0.0f},    /* four stages instead of two.  1750 x 2048 x 8192: 68 us (93) */
+    {8, 4, 2, 7.0f, 5.5f, 8.0f, 9.6f},     /* 600 x 2048 x 8192: 50 us (64) */
+    {8, 2, 2, 6.0f, 3.9f, 6.0f, 7.2f},     /* 200 x 4096 x 14336: 61 us (84) */
+};
+struct WidePick { int form, ks; };
+WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
+    const int ntiles = g.N / 16, mtiles = (g.nrows + 15) / 16;
+    /* k in parts whose sums the consumer adds, at least 512 each: it reads, and this kernel writes, a slab more per part */
+    const int kt = tk_img_kt(g.type), most = swiglu || grouped || g.max_slabs < 1 ? 1 : g.max_slabs;
+    const float slab_us = (float)((double)g.nrows * g.n_valid * 8e-6 / 5.0);
+    WidePick best{2, 1};
+    float least = 1e30f;
+    for (int f = 0; f < (int)(sizeof wide_forms / sizeof wide_forms[0]); ++f) {
+        const WideForm& w = wide_forms[f];
+        if ((grouped && w.mb > 8) || (swiglu && w.nb < 4)) continue;
+        for (int ks = 1; ks <= most && (ks == 1 || g.K / kt / ks >= 16); ++ks) {
+            const int64_t blocks = (int64_t)(grouped ? g.max_blocks : (mtiles + w.mb - 1) / w.mb) * ((ntiles + w.nb - 1) / w.nb) * ks;
+            const float k = 1e-3f * (float)g.K / (float)ks, one = w.start + w.k * k, two = w.start2 + w.k2 * k;
+            float us = (float)(ks - 1) * slab_us;
+            if (w.per_cu == 1) us += (float)((blocks + 255) / 256) * one;
+            else us += (float)(blocks / 512) * two + (blocks % 512 == 0 ? 0.0f : blocks % 512 <= 256 ? one : two);
+            if (us < least) { least = us; best = WidePick{f, ks}; }
+        }
+    }
+    return best;
+}
+
 template <typename T, bool SWIGLU, bool GROUPED>
 const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
     const int ntiles = g.N / 16;
@@ -258,22 +332,18 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
 #undef TK_SK
         return nullptr;
     }
-    const int nblk_m = GROUPED ? g.max_blocks : (g.nrows + 127) / 128;
-    int nb = 8, ks = 1;
-    const int64_t full = (int64_t)nblk_m * ((ntiles + 7) / 8);
-    if (!SWIGLU && !GROUPED && g.max_slabs > 1 && full < 256) { /* large blocks of a part of K rather than small blocks of all of it: at least eight stages each */
-        ks = (int)(512 / full);
-        if (ks > g.max_slabs) ks = g.max_slabs;
-        const int most = g.K / TkImg<T>::KT / 16;
-        if (ks > most) ks = most;
-        if (ks < 1) ks = 1;
+    const WidePick pick = pick_wide(g, SWIGLU, GROUPED);
+    if (slabs) *slabs = pick.ks;
+#define TK_WD(MB, NB, WM, WN, RING) do { const int nbn = (ntiles + NB - 1) / NB, nbm = GROUPED ? g.max_blocks : (mtiles + MB - 1) / MB; \
+        hipLaunchKernelGGL((k_gemm_wide<T, MB, NB, WM, WN, RING, SWIGLU, GROUPED>), dim3(nbn * nbm * pick.ks), dim3(64 * WM * WN), (size_t)RING * wide_stage(MB, NB), s, g, nbn, nbm, pick.ks); } while (0)
+    switch (pick.form) {
+        case 0: if constexpr (!GROUPED) TK_WD(16, 16, 4, 2, 2); break;
+        case 1: if constexpr (!GROUPED) TK_WD(16, 8, 4, 2, 3); break;
+        case 2: TK_WD(8, 8, 2, 4, 2); break;
+        case 3: TK_WD(8, 8, 2, 4, 4); break;
+        case 4: TK_WD(8, 4, 4, 2, 3); break;
+        default: if constexpr (!SWIGLU) TK_WD(8, 2, 4, 1, 4);
     }
-    while (nb > (SWIGLU ? 4 : 2) && (int64_t)nblk_m * ((ntiles + nb - 1) / nb) * ks < 200) nb /= 2;
-    if (slabs) *slabs = ks;
-#define TK_WD(NB) do { const int nbn = (ntiles + NB - 1) / NB; hipLaunchKernelGGL((k_gemm_wide<T, NB, SWIGLU, GROUPED>), dim3(nbn * nblk_m * ks), dim3(256), (size_t)wide_ring<NB>() * (8 + NB) * 2048, s, g, nbn, nblk_m, ks); } while (0)
-    if (nb == 8) TK_WD(8);
-    else if (nb == 4 || SWIGLU) TK_WD(4);
-    else TK_WD((SWIGLU ? 4 : 2));
 #undef TK_WD
     return nullptr;
 }
@@ -297,9 +367,15 @@ const char* tk_launch_gemm_image(const TkImgGemm& g, hipStream_t s, int* slabs) 
 template <typename T>
 static hipError_t opt_in_wide() {
     hipError_t e = hipSuccess;
-#define TK_OPT(NB, S, G) if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k_gemm_wide<T, NB, S, G>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)
-    TK_OPT(2, false, false); TK_OPT(2, false, true);
-    TK_OPT(4, false, false); TK_OPT(4, false, true); TK_OPT(4, true, false); TK_OPT(4, true, true);
+#define TK_OPT(MB, NB, WM, WN, RING, S, G) if (e == hipSuccess) e = hipFuncSetAttribute((const void*)k_gemm_wide<T, MB, NB, WM, WN, RING, S, G>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)
+#define TK_OPT4(MB, NB, WM, WN, RING) TK_OPT(MB, NB, WM, WN, RING, false, false); TK_OPT(MB, NB, WM, WN, RING, false, true); TK_OPT(MB, NB, WM, WN, RING, true, false); TK_OPT(MB, NB, WM, WN, RING, true, true)
+    TK_OPT(16, 16, 4, 2, 2, false, false); TK_OPT(16, 16, 4, 2, 2, true, false);
+    TK_OPT(16, 8, 4, 2, 3, false, false); TK_OPT(16, 8, 4, 2, 3, true, false);
+    TK_OPT4(8, 8, 2, 4, 2);
+    TK_OPT4(8, 8, 2, 4, 4);
+    TK_OPT4(8, 4, 4, 2, 3);
+    TK_OPT(8, 2, 4, 1, 4, false, false); TK_OPT(8, 2, 4, 1, 4, false, true);
+#undef TK_OPT4
 #undef TK_OPT
     return e;
 }
