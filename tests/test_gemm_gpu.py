@@ -44,6 +44,25 @@ def test_tiled_equals_staged_bitwise(gpu, M, N, K, act, bias, res):
             assert ct[i, j] == want
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (1, 1, 128), (31, 17, 128), (401, 255, 1152), (33, 65, 2304),      # 32 x 32 blocks: one element, tails on both sides, a long chain
+    (6400, 80, 768), (6401, 16, 640),                                  # 64 x 16
+    (12800, 64, 1152), (3201, 257, 1152),                              # 64 x 32
+    (12801, 128, 640), (12800, 130, 1152),                             # 64 x 64
+    (12795, 80, 2304), (51201, 79, 1152),                              # 64 x 80 and 128 x 80
+    (25600, 32, 128), (51200, 33, 128), (9000, 384, 128),              # left to the 32 x 32 x 2 kernels
+])
+def test_block_forms_equal_the_chain(gpu, M, N, K):
+    """every block form of the staged kernels, at sizes that fill no block: the tiled kernel's bits, and the definition at the corners"""
+    a, w, b, r, cs, ct = _pair(gpu, M, N, K, seed=M + N)
+    assert np.array_equal(cs.view(np.uint32), ct.view(np.uint32))
+    for i, j in ((0, 0), (M - 1, N - 1), (0, N - 1), (M // 2, N // 2)):
+        acc = np.float32(0)
+        for k in range(K):
+            acc = np.float32(np.float64(a[i, k]) * np.float64(w[j, k]) + np.float64(acc))
+        assert cs[i, j] == np.float32(acc + b[j])
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 256, 1024), (48, 4096, 512), (256, 64, 256)])
 def test_f16_weight_tiles_equal_the_staged_f16_path(gpu, M, N, K):
     """fp16-checkpoint semantics: f16 weights, activations rounded through f16, fp32 chain"""

@@ -54,6 +54,16 @@ def test_detector_head_maps_bit_exact(gpu):
         assert np.array_equal(boxes, wb)
 
 
+@pytest.mark.parametrize("B,H,W", [(1, 32, 32), (1, 32, 416), (5, 96, 64), (2, 224, 352)])
+def test_detector_head_maps_bit_exact_at_other_sizes(gpu, B, H, W):
+    """input geometries whose layers fill no block of a convolution launch, down to one pixel"""
+    x = np.random.default_rng(H + W).standard_normal((B, H, W, 3)).astype(np.float32)
+    det = gpu.ObjectDetector(model="synthetic://yolov8n?seed=5&cls_bias=-0.5", width=W, height=H, max_batch=B)
+    raw = det.forward_raw(x)
+    orc = O.OracleYolo(80, 5, -0.5)
+    assert np.array_equal(raw, orc.forward(x))
+
+
 def test_detector_full_size_frame_bit_exact(gpu):
     """BASELINE geometry: one 640x640 network input (8400 anchors): head maps and NMS survivors equal the oracle's, bit for bit"""
     det = gpu.ObjectDetector(width=640, height=640, conf=0.05)

@@ -7,6 +7,7 @@
 #include "../common/tk_sample_device.h"
 
 typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 
 #define BM 64
 #define BN 64
@@ -446,6 +447,196 @@ __global__ __launch_bounds__(256) void k_gemm_f32_big(TkGemm g) {
         for (int i = 0; i < 2; ++i) store_tile(g, acc[i][j], C, R, m0 + wm * 64 + i * 32, n0 + wn * 64 + j * 32 + (lane & 31), lane);
 }
 
+/*
+ * The same chains on v_mfma_f32_16x16x4_f32, WM x WN waves of MT x NT 16 x 16 tiles.  Per output the pipe takes 8 cycles a k where the 32 x 32 x 2 form
+ * takes 32, and blocks can be small: what a launch of few rows (one frame, one utterance) waits for is a chain of K steps on a mostly idle chip.
+ * Columns come in 16s, so N = 16 or 80 wastes nothing.
+ * LDS holds both operands as the MFMA wants them: per 16 rows and 16 k, lane (row, g) has k = g, 4 + g, 8 + g, 12 + g in one 16-byte read; a group of
+ * four k from memory goes to the four g (64 floats apart).  [N][K] weights only.  Slabs of 16 BK16 k, the next two slabs' loads in flight.
+ */
+template <bool IM, int PATH, int WM, int WN, int MT, int NT, int BK16 /* 16-k groups of a slab */>
+__global__ __launch_bounds__(256) void k_gemm_f32_t16(TkGemm g) {
+    static_assert(WM * WN == 4, "four waves");
+    constexpr int TM = WM * MT, TN = WN * NT, SK = 16 * BK16;      /* tiles of the workgroup */
+    constexpr int NA = TM * 16 * SK / 4 / 256, NB = (TN * 16 * SK / 4 + 255) / 256; /* groups of four per thread */
+    constexpr int KG = SK / 4;                                     /* groups of a row */
+    static_assert(256 % KG == 0 && NA >= 1, "a thread keeps its place in k");
+    constexpr int RPT = 256 / KG;                                  /* rows that 256 threads cover */
+    extern __shared__ __attribute__((aligned(16))) float t16_lds[];
+    constexpr int BUF = (TM + TN) * BK16 * 256;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = blockIdx.y * TM * 16, n0 = blockIdx.x * TN * 16;
+    int64_t oA, oB, oC, oR;
+    batch_offsets(g, blockIdx.z, oA, oB, oC, oR);
+    const float* A = g.A + oA;
+    const float* B = g.B + oB;
+    float* C = g.C + oC;
+    const bool a_vec = (g.lda & 3) == 0 && (((uintptr_t)A) & 15) == 0;
+    const bool b_vec = (g.ldb & 3) == 0 && (((uintptr_t)B) & 15) == 0;
+    /* Two slabs are on their way.  Aligned operands: every lane loads from an address inside the matrix and what lies outside is made zero on the way
+     * into LDS, so that no branch stands between the requests of a slab and those of the next (a wait behind one would be for the youngest).
+     * Addresses are 32-bit offsets: of a row, fixed, and of a k, the same for all rows of a thread. */
+    struct Slab { float a[NA][4], b[NB][4]; uint32_t ok_a, ok_b; } s0, s1;
+    const int ar = tid / KG, akg = tid % KG;
+    int offa[NA], iy0[NA], ix0[NA], offb[NB];
+    /* tap of a k without a division: k, taps < 2^16 (the launcher's condition) */
+    const uint32_t by_c = IM ? (uint32_t)((0x100000000ull + g.im_C - 1) / g.im_C) : 0, by_kw = IM ? (uint32_t)((0x100000000ull + g.im_kw - 1) / g.im_kw) : 0;
+#pragma unroll
+    for (int h = 0; h < NA; ++h) {
+        const int m = m0 + ar + RPT * h;
+        if (IM) {
+            const ImRow r = im_row(g, m);
+            iy0[h] = r.iy0; ix0[h] = r.ix0;
+            offa[h] = ((int)r.pix0 + r.iy0 * g.im_W + r.ix0) * g.im_ldx;
+        } else {
+            offa[h] = (m < g.M ? m : 0) * g.lda;
+        }
+    }
+#pragma unroll
+    for (int h = 0; h < NB; ++h) {
+        const int n = n0 + ar + RPT * h;
+        offb[h] = (ar + RPT * h < TN * 16 && n < g.N ? n : 0) * g.ldb;
+    }
+    auto get4 = [](const float* p, int at, float out[4]) {
+        const float4 t = *(const float4*)((const char*)p + (uint32_t)at * 4u);
+        out[0] = t.x; out[1] = t.y; out[2] = t.z; out[3] = t.w;
+    };
+    auto gload = [&](Slab& s, int k0) {
+        const int k = k0 + akg * 4;
+        const bool in = k < g.K;
+        s.ok_a = s.ok_b = 0;
+        int at = in ? k : 0, ky = 0, kx = 0;
+        if (IM) {
+            const int tap = g.im_C == 1 ? k : (int)__umulhi((uint32_t)k, by_c);
+            ky = g.im_kw == 1 ? tap : (int)__umulhi((uint32_t)tap, by_kw);
+            kx = tap - ky * g.im_kw;
+            at = (ky * g.im_W + kx) * g.im_ldx + k - tap * g.im_C;
+        }
+#pragma unroll
+        for (int h = 0; h < NA; ++h) {
+            if (IM) {
+                const bool ok = (int)in & (int)((uint32_t)(iy0[h] + ky) < (uint32_t)g.im_H) & (int)((uint32_t)(ix0[h] + kx) < (uint32_t)g.im_W);
+                s.ok_a |= (uint32_t)ok << h;
+                get4(A, ok ? offa[h] + at : 0, s.a[h]);
+            } else if (PATH != 0) {
+                s.ok_a |= (uint32_t)in << h;
+                get4(A, offa[h] + at, s.a[h]);
+            } else {
+                load_a4<0>(g, A, a_vec, m0 + ar + RPT * h, k, s.a[h]);
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < NB; ++h) {
+            if (PATH != 0) {
+                s.ok_b |= (uint32_t)in << h;
+                get4(B, offb[h] + (in ? k : 0), s.b[h]);
+            } else {
+                load_b4_nk<0>(g, B, b_vec, ar + RPT * h < TN * 16 ? n0 + ar + RPT * h : g.N, k, s.b[h]);
+            }
+        }
+    };
+    auto put = [&](float* buf, int row, int kg, const float v[4]) { /* four k of a row */
+        float* p = buf + ((row >> 4) * BK16 + (kg >> 2)) * 256 + (row & 15) * 4 + (kg & 3);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[64 * i] = v[i];
+    };
+    auto lstore = [&](const Slab& s, int b) {
+        float* as = t16_lds + b * BUF;
+        float* bs = as + TM * BK16 * 256;
+#pragma unroll
+        for (int h = 0; h < NA; ++h) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = PATH == 0 || (s.ok_a >> h & 1) ? s.a[h][i] : 0.0f;
+            put(as, ar + RPT * h, akg, v);
+        }
+#pragma unroll
+        for (int h = 0; h < NB; ++h) {
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = PATH == 0 || (s.ok_b >> h & 1) ? s.b[h][i] : 0.0f;
+            if (ar + RPT * h < TN * 16) {
+                put(bs, ar + RPT * h, akg, v);
+            }
+        }
+    };
+    v4f acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    const int wm = wave % WM * MT, wn = wave / WM * NT;
+    const int slabs = (g.K + SK - 1) / SK;
+    auto multiply = [&](int b) {
+        const float* ap = t16_lds + b * BUF + wm * BK16 * 256 + lane * 4;
+        const float* bp = t16_lds + b * BUF + (TM + wn) * BK16 * 256 + lane * 4;
+        /* a 16-k group's operands are read while the one before it is multiplied */
+        v4f av[2][MT], bv[2][NT];
+        auto read = [&](int j) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) av[j & 1][m] = *(const v4f*)(ap + (m * BK16 + j) * 256);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) bv[j & 1][n] = *(const v4f*)(bp + (n * BK16 + j) * 256);
+        };
+        read(0);
+        __builtin_amdgcn_sched_group_barrier(0x100, MT + NT, 0);
+#pragma unroll
+        for (int j = 0; j < BK16; ++j) {
+            if (j + 1 < BK16) {
+                read(j + 1);
+                __builtin_amdgcn_sched_group_barrier(0x100, MT + NT, 0);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[j & 1][m][t], bv[j & 1][n][t], acc[m][n], 0, 0, 0);
+            __builtin_amdgcn_sched_group_barrier(0x8, 4 * MT * NT, 0);
+        }
+    };
+    gload(s0, 0);
+    gload(s1, SK);
+    lstore(s0, 0);
+    __syncthreads();
+    for (int i = 0; i < slabs; i += 2) { /* slabs past the end are zero: nothing is added */
+        gload(s0, (i + 2) * SK);
+        multiply(0);
+        lstore(s1, 1);
+        __syncthreads();
+        gload(s1, (i + 3) * SK);
+        if (i + 1 < slabs) multiply(1);
+        lstore(s0, 0);
+        __syncthreads();
+    }
+    const float* R = g.residual ? g.residual + oR : nullptr;
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int col = n0 + (wn + n) * 16 + (lane & 15);
+        if (col >= g.N) continue;
+        const float bias = g.bias ? g.bias[col] : 0.0f;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const int row = m0 + (wm + m) * 16 + 4 * (lane >> 4);
+            float v[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = acc[m][n][r];
+            if (g.alpha != 1.0f) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = v[r] * g.alpha;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r] + bias, g.act);
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (row + r < g.M) {
+                    if (R) v[r] = v[r] + R[(int64_t)(row + r) * g.ldr + col];
+                    C[(int64_t)(row + r) * g.ldc + col] = v[r];
+                }
+        }
+    }
+}
+
 /* ------------------------------------------------------------------------------------------
  * Opt-in fast contraction (TkGemm::fast): the same tiles, loaders and epilogue on the f16 matrix pipe.
  * v_mfma_f32_32x32x16_f16 retires 16 k per 8 passes where v_mfma_f32_32x32x2_f32 retires 2 per 16: 16 x the rate, with operands of 11
@@ -834,6 +1025,49 @@ static bool tk_gemm_fast(const TkGemm& g) {
     return true;
 }
 
+/* What an exact-chain launch costs, by kernel: start + K (a + b x more) + c x more, where more = workgroups per CU beyond the first (a workgroup alone on
+ * its CU waits for its own chain and loads, further ones share the pipe).  Fitted to the detector's layers at 1, 8 and 32 frames; us, ns per k. */
+struct F32Form { int rows, cols; float start, a, b, c; };
+constexpr F32Form f32_forms[] = {
+    {32, 32, 3.3f, 11.0f, 8.5f, 1.0f},   /* 400 x 256 x 1152: 16 us (128 x 128: 102), 400 x 64 x 2304: 27 us (64 x 64: 69) */
+    {64, 16, 4.5f, 11.5f, 8.6f, 1.2f},   /* 6400 x 80 x 720: 19 us (128 x 96: 57) */
+    {64, 32, 5.0f, 16.1f, 18.0f, 1.4f},  /* 12800 x 64 x 1152: 37 us (128 x 64: 64) */
+    {64, 64, 6.0f, 25.5f, 26.5f, 1.4f},  /* 12800 x 128 x 576: 33 us (128 x 128: 60) */
+    {64, 80, 7.0f, 31.0f, 32.5f, 2.2f},  /* 204800 x 80 x 720: 294 us (128 x 96: 328) */
+    {128, 80, 10.0f, 51.6f, 68.0f, 3.0f}, /* 51200 x 80 x 1152: 124 us (128 x 96: 136) */
+};
+static float f32_cost(const F32Form& f, const TkGemm& g, int nz) {
+    const float wgs = (float)((g.M + f.rows - 1) / f.rows) * (float)((g.N + f.cols - 1) / f.cols) * (float)nz;
+    const float more = wgs > 256.0f ? wgs / 256.0f - 1.0f : 0.0f;
+    return f.start + 1e-3f * (float)g.K * (f.a + f.b * more) + f.c * more;
+}
+/* the 16 x 16 x 4 form of a launch, or -1: one of the 32 x 32 x 2 kernels is expected to be quicker (high-resolution layers of few channels and many
+ * frames, scores of whole utterances), or the operands are not for it */
+static int f32_pick(const TkGemm& g, int nz) {
+    /* its offsets have 32 bits */
+    const int64_t most = 1 << 28;
+    if (g.b_f16 || g.b_kn || g.K < 1 || g.K > 60000) return -1; /* [K][N] matrices: 1500 x 64 x 1500 x 192 483 us with the 64 x 64 kernel, 580 and more here */
+    if (g.im_C > 0) {
+        const int64_t images = g.M / ((int64_t)g.im_Ho * g.im_Wo) + 1;
+        if (images * g.im_H * g.im_W * g.im_ldx >= most || g.im_C > 60000) return -1;
+    } else if ((int64_t)g.M * g.lda >= most) {
+        return -1;
+    }
+    if ((int64_t)g.N * g.ldb >= most) return -1;
+    F32Form old;
+    if (g.M >= 256 && g.N >= 96) old = F32Form{128, 128, 11.0f, 78.0f, 105.0f, 2.0f};
+    else if (g.N < 96 && g.M >= 4 * NBM && nz == 1 && g.batch_inner == 0)
+        old = g.N <= 32 ? F32Form{NBM, 32, 4.5f, 36.0f, 36.0f, 0.5f} : g.N <= 64 ? F32Form{NBM, 64, 6.0f, 50.0f, 50.0f, 2.4f} : F32Form{NBM, 96, 5.0f, 72.0f, 72.0f, 4.9f};
+    else old = F32Form{BM, BN, 2.0f, 29.0f, 40.0f, 1.0f};
+    int best = -1;
+    float least = f32_cost(old, g, nz);
+    for (int i = 0; i < (int)(sizeof f32_forms / sizeof f32_forms[0]); ++i) {
+        const float c = f32_cost(f32_forms[i], g, nz);
+        if (c < least && (g.M + f32_forms[i].rows - 1) / f32_forms[i].rows <= 65535) { least = c; best = i; }
+    }
+    return best;
+}
+
 void tk_launch_gemm(const TkGemm& g, hipStream_t s) {
     const int nz = g.batch > 0 ? g.batch : 1;
     const bool im = g.im_C > 0; /* validated by tk_gemm_im2col_ok(): aligned [N][K] f32 weights, C % 4 == 0, no batch */
@@ -869,6 +1103,23 @@ void tk_launch_gemm(const TkGemm& g, hipStream_t s) {
 #undef TK_TALL_H3
         return;
     }
+#define TK_T16(WM, WN, MT, NT, BK16) do {                                                                                                     \
+        const dim3 grid((g.N + WN * NT * 16 - 1) / (WN * NT * 16), (g.M + WM * MT * 16 - 1) / (WM * MT * 16), nz);                              \
+        const size_t lds = (size_t)2 * (WM * MT + WN * NT) * BK16 * 1024;                                                                      \
+        if (im) hipLaunchKernelGGL((k_gemm_f32_t16<true, 1, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                                \
+        else if (path == 1) hipLaunchKernelGGL((k_gemm_f32_t16<false, 1, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                   \
+        else hipLaunchKernelGGL((k_gemm_f32_t16<false, 0, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                                  \
+    } while (0)
+    switch (f32_pick(g, nz)) {
+        case 0: TK_T16(2, 2, 1, 1, 4); return;
+        case 1: TK_T16(4, 1, 1, 1, 4); return;
+        case 2: TK_T16(2, 2, 2, 1, 4); return;
+        case 3: TK_T16(2, 2, 2, 2, 2); return;
+        case 4: TK_T16(4, 1, 1, 5, 2); return;
+        case 5: TK_T16(4, 1, 2, 5, 2); return;
+        default: break;
+    }
+#undef TK_T16
     if (g.M >= 256 && g.N >= 96) {
         const size_t lds = (size_t)2 * (LBM + LBN) * LDS_LD * sizeof(float);
         (void)tk_nn_prepare_device();
