@@ -50,6 +50,27 @@ def test_whisper_tiny_en_full_size_encoder(gpu):
     assert np.array_equal(toks, wt) and np.array_equal(lg, wlg)
 
 
+@pytest.mark.parametrize("ctx,state,heads,clips,steps", [
+    (512, 64, 4, 1, 135),    # heads of 16; scores of cross attention in the same kernel for the last time; self attention past two blocks of 64 keys
+    (513, 96, 2, 3, 3),      # heads of 48 (not split); scores in their own kernel
+    (1536, 32, 2, 2, 2),     # the longest round of one tile of 16 columns
+    (1537, 64, 1, 1, 2),     # one key more; a head in four parts
+    (800, 288, 2, 1, 18),    # heads of 144: nine tiles for eight waves
+    (520, 512, 2, 2, 2),     # heads of 256
+    (2048, 128, 1, 1, 2), (2049, 64, 2, 1, 2),   # the most keys, and the general form beyond
+])
+def test_decoder_attention_over_contexts_and_heads(gpu, ctx, state, heads, clips, steps):
+    ohp = O.whisper_tiny_test()
+    ohp.n_audio_ctx, ohp.n_audio_state, ohp.n_audio_head, ohp.n_audio_layer = ctx, state, heads, 1
+    ohp.n_text_ctx, ohp.n_text_state, ohp.n_text_head, ohp.n_text_layer = 144, state, heads, 1
+    asr = gpu.Asr(hp=hp_of(gpu, ohp), seed=3, max_batch=clips)
+    pcm = np.clip(np.random.default_rng(ctx).normal(0, 3000, (clips, 9000)), -32768, 32767).astype(np.int16)
+    toks, _, _, lg = asr.transcribe_tokens(pcm, steps)
+    want, _, _, wlg = O.OracleWhisper(ohp, seed=3).transcribe(pcm, steps)
+    assert np.array_equal(lg, wlg), np.abs(lg - wlg).max()
+    assert np.array_equal(toks, want)
+
+
 def test_whisper_tiny_en_full_size_against_hf(gpu):
     """the HIP ASR engine itself against HF transformers at the tiny.en geometry (whisper_full_tiny_en.npz: sampled log-mel, encoder states,
     first-step logits; 2e-4 of the tensors' scale), without the oracle in between"""

@@ -4,6 +4,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <type_traits>
+
 #include "../nn/tk_gemm_tiled.h"
 #include "../nn/tk_nn_kernels.h"
 
@@ -68,112 +70,266 @@ __global__ __launch_bounds__(1024) void k_logmel_finish(float* mel, int per_b) {
 
 /* ---------------------------------------------------------------- decoder-step attention, fused
 
- * One query row per (sequence, head): scores, softmax and the value contraction in one workgroup, with exactly the arithmetic of the
+ * One query row per (sequence, head): scores, softmax and the value contraction in one launch or two, with exactly the arithmetic of the
  * three-launch form it replaces (tk_whisper_graph.h: attention()): score = (fp32 fma chain over the head dimension, ascending) * scale
  * + 0.0f (the GEMM epilogue's bias slot); softmax as k_softmax_rows evaluates it (256 strided partial maxima / sums, shuffle tree,
- * ((w0 + w1) + w2) + w3); output = one fp32 fma chain over the keys in ascending order, + 0.0f.  The decoder steps of 32 utterances were
- * sixteen 64x64-tile GEMM launches of one live row each per step; this is eight short launches. */
-#define TK_AT1_CK 64 /* keys per ring slot of the value stream */
-#define TK_AT1_NS 3  /* ring slots */
-/* s_waitcnt vmcnt(n) alone */
-__device__ __forceinline__ void at1_wait_vmcnt(int n) {
-#define TK_VMW(k) case k: __builtin_amdgcn_s_waitcnt(0x0F70 | ((k) & 15) | (((k) >> 4) << 14)); break;
-    switch (n) {
-        TK_VMW(0) TK_VMW(1) TK_VMW(2) TK_VMW(3) TK_VMW(4) TK_VMW(5) TK_VMW(6) TK_VMW(7) TK_VMW(8) TK_VMW(9) TK_VMW(10) TK_VMW(11) TK_VMW(12)
-        TK_VMW(13) TK_VMW(14) TK_VMW(15) TK_VMW(16)
-        default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-    }
-#undef TK_VMW
+ * ((w0 + w1) + w2) + w3); output = one fp32 fma chain over the keys in ascending order, + 0.0f.  */
+/* What bounds it: the value contraction is one fp32 chain over the keys per output, 8 cycles a key on the 16 x 16 x 4 MFMA (1500 keys: 5 us), and
+ * what one CU can fetch (about 40 KB a us).  So the chain must never wait for memory, and a head's K and V come in through several CUs:
+ *  - a workgroup takes hd / split outputs of one head, with its part of V only: few sequences leave most CUs idle, so the split grows while the
+ *    grid stays within the chip.  16 outputs are one wave's chain; its MFMAs take the weights as 16 equal rows of A.
+ *  - V goes through registers, requested before the scores are known (all of 1500 keys x 16 outputs; more in rounds, the next one under way during
+ *    a round's chain), into LDS in the order of four MFMAs' operands: a wave gets one LDS read in about 18 cycles, whatever its width, so it
+ *    must need few: 2 for 16 keys.
+ *  - over long contexts (cross attention) the scores come from a kernel of their own, 64 keys per wave over the whole chip; up to 512 keys
+ *    (self attention) every workgroup makes them itself, 64 keys per wave: a launch costs more.
+ * Scores: a key per lane.  K comes by LDS-DMA, 16 floats of each key per slot of 4 KiB (rows 64 bytes apart, their 16-byte units swapped by
+ * row so that the 64 lanes' reads spread over all banks).
+ * Cross attention of one sequence (6 heads, 1500 keys of 64): 18 us (4 + 14); with one workgroup of 4 waves per head, whose lanes read whole rows of K
+ * (64 lines per load) and whose chain ran on one vector unit: 49 us.  32 sequences: 42 us against 77. */
+#define TK_AT1_NW 8             /* waves */
+#define TK_AT1_RING (16 * 1024) /* bytes per wave: 64 keys of K in four slots of 16 floats */
+#define TK_AT1_SELF 512         /* longest context whose scores are made in the same kernel: 64 keys per wave */
+#define TK_AT1_MAX_KEYS 2048    /* 8 scores per thread */
+typedef float at1_f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void at1_wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); } /* s_waitcnt vmcnt(0) alone */
+__device__ __forceinline__ void at1_dma(const float* src, uint8_t* lds) {
+    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
-/* The value contraction is ONE fp32 chain over the keys per output (the canonical order), carried by hd threads; what the other threads
- * can do is move the values: all four waves stream V through a three-slot LDS ring by LDS-DMA (64 keys x hd floats per slot, 1 KiB pieces
- * of four 256-byte rows), the first two slots requested before the scores are even computed, so the chain reads LDS instead of waiting
- * for 32 global rows at a time (cross-attention over 1500 keys: the chain wave alone had 384 KB to pull through 32 loads in flight). */
-__global__ __launch_bounds__(256) void k_attend1(const float* q, const float* k, const float* v, float* out, int Tk, int64_t q_bstride, int64_t kv_bstride, int d,
-                                                 int hd, float scale, float* img /* optional: out also as the tiled GEMM's operand image [B rows][K = d] */) {
-    extern __shared__ __attribute__((aligned(16))) float att1_lds[];
-    __shared__ float red[4];
-    float* vring = att1_lds;                                   /* [NS][CK][hd] */
-    float* sc = att1_lds + (size_t)TK_AT1_NS * TK_AT1_CK * hd; /* [Tk] */
-    float* qs = sc + Tk;                                       /* [hd] */
-    const int h = blockIdx.x, b = blockIdx.y, t0 = threadIdx.x, lane = t0 & 63;
+/* the score of key 64 blk + lane (of the last key where there is none); q [hd] in LDS, hd * 256 bytes of ring per wave or 16 KiB, whichever is less */
+__device__ __forceinline__ float at1_score(const float* kp, int blk, int Tk, int d, int hd, float scale, const float* qs, uint8_t* ring, int lane) {
+    const int unit = (lane & 3) ^ ((lane >> 4) & 3), nsl = hd >> 4;
+    const float* src[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        int row = blk * 64 + p * 16 + (lane >> 2);
+        row = row < Tk ? row : Tk - 1;
+        src[p] = kp + (int64_t)row * d + unit * 4;
+    }
+    float a = 0.0f;
+    for (int s0 = 0; s0 < nsl; s0 += 4) {
+        for (int sl = s0; sl < s0 + 4 && sl < nsl; ++sl)
+#pragma unroll
+            for (int p = 0; p < 4; ++p) at1_dma(src[p] + sl * 16, ring + (sl & 3) * 4096 + p * 1024);
+        at1_wait_vm0();
+        for (int sl = s0; sl < s0 + 4 && sl < nsl; ++sl) {
+            const uint8_t* slot = ring + (sl & 3) * 4096 + lane * 64;
+            float4 kk[4], qq[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { kk[i] = *(const float4*)(slot + ((i ^ ((lane >> 2) & 3)) << 4)); qq[i] = *(const float4*)(qs + sl * 16 + 4 * i); }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                a = tk_fmaf(qq[i].x, kk[i].x, a); a = tk_fmaf(qq[i].y, kk[i].y, a); a = tk_fmaf(qq[i].z, kk[i].z, a); a = tk_fmaf(qq[i].w, kk[i].w, a);
+            }
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); /* the ring is read out */
+    }
+    a = a * scale;
+    return a + 0.0f;
+}
+
+/* scores [sequences][heads][pitch] of a long context: grid (64-key blocks / 4, heads, sequences), a block of keys per wave */
+__global__ __launch_bounds__(256) void k_attend1_scores(const float* q, const float* k, float* scores, int Tk, int pitch, int64_t q_bstride, int64_t kv_bstride, int d, int hd,
+                                                        float scale) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t att1_lds[];
+    const int h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    float* qs = (float*)(att1_lds + 4 * TK_AT1_RING);
+    for (int i = threadIdx.x; i < hd; i += 256) qs[i] = q[(int64_t)b * q_bstride + (int64_t)h * hd + i];
+    __syncthreads();
+    const int blk = blockIdx.x * 4 + wave;
+    if (blk * 64 >= Tk) return;
+    const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, blk, Tk, d, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
+    if (blk * 64 + lane < Tk) scores[((int64_t)b * gridDim.y + h) * pitch + blk * 64 + lane] = a;
+}
+
+/* tasks of a thread in a round of V (kernel below), and what a round takes of C columns: the whole of a self attention's usual context at once */
+constexpr int at1_tasks(bool self) { return self ? 1 : 3; }
+__host__ __device__ constexpr int at1_round_blocks(bool self, int C) { return at1_tasks(self) * 64 * TK_AT1_NW / C; }
+/* place of key k's weight in LDS: 16 keys' weights in the order in which four MFMAs take them, so that a lane's four are one read */
+__device__ __forceinline__ int at1_place(int k) { return (k & ~15) | (k & 3) << 2 | (k >> 2 & 3); }
+
+template <bool SELF>
+__global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, const float* k, const float* v, const float* scores, int pitch, float* out, int Tk,
+                                                           int64_t q_bstride, int64_t kv_bstride, int d, int hd, int split, float scale, int sc_at /* bytes */,
+                                                           float* img /* optional: out also as the tiled GEMM's operand image [B rows][K = d] */) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t att1_lds[];
+    const int h = blockIdx.x / split, part = blockIdx.x % split, b = blockIdx.y, t0 = threadIdx.x, lane = t0 & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t0 >> 6);
-    const float* qp = q + (int64_t)b * q_bstride + (int64_t)h * hd;
-    const float* kp = k + (int64_t)b * kv_bstride + (int64_t)h * hd;
-    const float* vp = v + (int64_t)b * kv_bstride + (int64_t)h * hd;
-    const int nchunk = (Tk + TK_AT1_CK - 1) / TK_AT1_CK;
-    const int upr = hd / 4;                       /* 16-byte units per row */
-    const int ppw = TK_AT1_CK * hd / 256 / 4;     /* DMA pieces per wave and chunk (the launcher admits hd % 16 == 0 only) */
-    auto issue = [&](int c) { /* rows past the last key re-read it: never used by the chain */
-        float* slot = vring + (size_t)(c % TK_AT1_NS) * TK_AT1_CK * hd;
-        for (int i = 0; i < ppw; ++i) {
-            const int p = wave + 4 * i, u = p * 64 + lane;
-            int row = c * TK_AT1_CK + u / upr;
-            row = row < Tk ? row : Tk - 1;
-            const auto gs = (const __attribute__((address_space(1))) void*)(vp + (int64_t)row * d + 4 * (u % upr));
-            const auto ls = (__attribute__((address_space(3))) void*)((uint8_t*)slot + p * 1024);
-            __builtin_amdgcn_global_load_lds(gs, ls, 16, 0, 0);
+    float* vbuf = (float*)att1_lds;         /* a round of V; before it the waves' rings of K */
+    float* sc = (float*)(att1_lds + sc_at); /* [Tk rounded up to 16] */
+    float* qs = sc + ((Tk + 15) & ~15);     /* [hd] */
+    float* red = qs + hd;                   /* [8] */
+    const int C = hd / split;               /* this workgroup's outputs: a multiple of 16 */
+    const float* vp = v + (int64_t)b * kv_bstride + (int64_t)h * hd + part * C;
+
+    /* 256 threads hold the scores: thread t those of keys t, t + 256, ...: the canonical partials */
+    constexpr int NS = SELF ? TK_AT1_SELF / 256 : TK_AT1_MAX_KEYS / 256;
+    float e[NS];
+    if (!SELF) {
+        const float* sp = scores + ((int64_t)b * (gridDim.x / split) + h) * pitch;
+#pragma unroll
+        for (int j = 0; j < NS; ++j) { const int t = (t0 & 255) + 256 * j; e[j] = sp[t < Tk ? t : Tk - 1]; }
+    }
+    /* V in rounds of 16 * rb keys.  A thread's task: keys 16 kb + 4 t + g, t = 0 .. 3, of four neighbouring columns.  LDS: [block of 16 keys]
+     * [16 columns][g][column ^ g][t], 1 KiB a tile (the XOR spreads the four g's writes over the banks) */
+    constexpr int NT = at1_tasks(SELF);
+    const int cu = C >> 2, nt = C >> 4, rb = at1_round_blocks(SELF, C), nblk = (Tk + 15) >> 4;
+    at1_f32x4 vv[NT][4];
+    auto load_v = [&](int kb0) { /* past the round or the last key: read again, not used */
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const int id = t0 + 64 * TK_AT1_NW * i, kq = id / cu, x = id - kq * cu;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                int row = (kb0 + (kq >> 2)) * 16 + 4 * t + (kq & 3);
+                row = row < Tk ? row : Tk - 1;
+                vv[i][t] = *(const at1_f32x4*)(vp + (int64_t)row * d + 4 * x);
+            }
         }
     };
-    for (int j = 0; j < TK_AT1_NS - 1 && j < nchunk; ++j) issue(j);
-    for (int i = t0; i < hd; i += 256) qs[i] = qp[i];
-    __syncthreads();
-    float m = -INFINITY;
-    for (int t = t0; t < Tk; t += 256) {
-        const float* kr = kp + (int64_t)t * d;
-        float a = 0.0f;
-        for (int i = 0; i < hd; i += 4) {
-            const float4 kk = *(const float4*)(kr + i);
-            a = tk_fmaf(qs[i], kk.x, a); a = tk_fmaf(qs[i + 1], kk.y, a); a = tk_fmaf(qs[i + 2], kk.z, a); a = tk_fmaf(qs[i + 3], kk.w, a);
+    auto store_v = [&](int blocks) {
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const int id = t0 + 64 * TK_AT1_NW * i, kq = id / cu, x = id - kq * cu, g = kq & 3;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(vv[i][t])); /* as loaded up to here: else the loads are turned, and waited for, where they are issued */
+            float* dst = vbuf + ((kq >> 2) * nt + (x >> 2)) * 256 + g * 64 + (x & 3) * 16;
+            if ((kq >> 2) < blocks) {
+                *(at1_f32x4*)(dst + (0 ^ g) * 4) = at1_f32x4{vv[i][0].x, vv[i][1].x, vv[i][2].x, vv[i][3].x};
+                *(at1_f32x4*)(dst + (1 ^ g) * 4) = at1_f32x4{vv[i][0].y, vv[i][1].y, vv[i][2].y, vv[i][3].y};
+                *(at1_f32x4*)(dst + (2 ^ g) * 4) = at1_f32x4{vv[i][0].z, vv[i][1].z, vv[i][2].z, vv[i][3].z};
+                *(at1_f32x4*)(dst + (3 ^ g) * 4) = at1_f32x4{vv[i][0].w, vv[i][1].w, vv[i][2].w, vv[i][3].w};
+            }
         }
-        a = a * scale;
-        a = a + 0.0f;
-        sc[t] = a;
-        m = tk_fmaxf(m, a);
+    };
+    load_v(0);
+    __builtin_amdgcn_sched_barrier(0);
+    if (SELF) {
+        const float* qp = q + (int64_t)b * q_bstride + (int64_t)h * hd;
+        for (int i = t0; i < hd; i += 64 * TK_AT1_NW) qs[i] = qp[i];
+        __syncthreads();
+        if (wave * 64 < Tk) {
+            const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, wave, Tk, d, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
+            if (t0 < Tk) sc[t0] = a;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < NS; ++j) { const int t = (t0 & 255) + 256 * j; e[j] = sc[t < Tk ? t : Tk - 1]; }
     }
+    const int tk = t0 & 255; /* threads 256 .. 511 do the same again: no wave waits for another's branch */
+    float m = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+        if (tk + 256 * j < Tk) m = tk_fmaxf(m, e[j]);
     for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, __shfl_xor(m, s, 64));
-    if ((t0 & 63) == 0) red[t0 >> 6] = m;
+    if (lane == 0) red[wave & 3] = m;
     __syncthreads();
     m = tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
-    __syncthreads();
     float s = 0.0f;
-    for (int t = t0; t < Tk; t += 256) { const float e = tk_expf(sc[t] - m); sc[t] = e; s = s + e; }
+#pragma unroll
+    for (int j = 0; j < NS; ++j)
+        if (tk + 256 * j < Tk) { e[j] = tk_expf(e[j] - m); s = s + e[j]; }
     for (int w = 32; w >= 1; w >>= 1) s = s + __shfl_xor(s, w, 64);
-    if ((t0 & 63) == 0) red[t0 >> 6] = s;
+    if (lane == 0) red[4 + (wave & 3)] = s;
     __syncthreads();
-    const float tot = ((red[0] + red[1]) + red[2]) + red[3];
-    for (int t = t0; t < Tk; t += 256) sc[t] = tk_divf(sc[t], tot);
-    float a = 0.0f;
-    for (int c = 0; c < nchunk; ++c) {
-        /* chunk c has landed once all but the chunks requested after it have; the barrier also says everybody is done with chunk c - 1,
-         * whose slot takes chunk c + NS - 1 (and, the first time, publishes the probabilities) */
-        const int ahead = nchunk - 1 - c < TK_AT1_NS - 2 ? nchunk - 1 - c : TK_AT1_NS - 2;
-        at1_wait_vmcnt(ahead * ppw);
+    const float tot = ((red[4] + red[5]) + red[6]) + red[7];
+    if (wave < 4) {
+#pragma unroll
+        for (int j = 0; j < NS; ++j)
+            if (t0 + 256 * j < Tk) sc[at1_place(t0 + 256 * j)] = tk_divf(e[j], tot);
+        if (t0 < (-Tk & 15)) sc[at1_place(Tk + t0)] = 0.0f;
+    }
+
+    at1_f32x4 acc[2] = {{0.0f, 0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f, 0.0f}}; /* outputs 16 wave .. and 16 (wave + 8) .. */
+    const int g = lane >> 4, col = lane & 15;
+    for (int kb0 = 0; kb0 < nblk; kb0 += rb) {
+        if (kb0) __syncthreads(); /* everybody is done with the round before */
+        const int nb = nblk - kb0 < rb ? nblk - kb0 : rb, n = Tk - kb0 * 16;
+        store_v(nb);
         __syncthreads();
-        if (c + TK_AT1_NS - 1 < nchunk) issue(c + TK_AT1_NS - 1);
-        if (t0 < hd) {
-            const float* vs = vring + (size_t)(c % TK_AT1_NS) * TK_AT1_CK * hd + t0;
-            const float* pc = sc + c * TK_AT1_CK;
-            const int n = Tk - c * TK_AT1_CK < TK_AT1_CK ? Tk - c * TK_AT1_CK : TK_AT1_CK;
+        if (kb0 + rb < nblk) load_v(kb0 + rb);
+        const float* pc = sc + kb0 * 16;
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const int tile = wave + TK_AT1_NW * w;
+            if (tile >= nt) break;
+            struct Stage { at1_f32x4 p[2], v[2]; } x, y; /* 32 keys */
+            const float* vt = vbuf + tile * 256 + g * 64 + (col ^ g) * 4;
+            auto read = [&](Stage& o, int u) { /* blocks u, u + 1 of 16 keys; the last one again past it */
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    const int kb = u + i < nb ? u + i : nb - 1;
+                    o.p[i] = *(const at1_f32x4*)(pc + kb * 16 + 4 * g);
+                    o.v[i] = *(const at1_f32x4*)(vt + kb * nt * 256);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto multiply = [&](Stage& o, int u, auto tail) {
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    if (tail.value) {
+                        if (u + i >= nb) break;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) o.v[i][j] = (u + i) * 16 + 4 * j + g < n ? o.v[i][j] : 0.0f; /* keys past the last add 0 x 0 */
+                    }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc[w] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.p[i][j], o.v[i][j], acc[w], 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            read(x, 0);
             int u = 0;
-            for (; u + 8 <= n; u += 8) {
-                float vv[8], pp[8];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { vv[e] = vs[(u + e) * hd]; pp[e] = pc[u + e]; }
-#pragma unroll
-                for (int e = 0; e < 8; ++e) a = tk_fmaf(pp[e], vv[e], a);
+            for (; u + 4 < nb; u += 4) {
+                read(y, u + 2);
+                multiply(x, u, std::false_type{});
+                read(x, u + 4);
+                multiply(y, u + 2, std::false_type{});
             }
-            for (; u < n; ++u) a = tk_fmaf(pc[u], vs[u * hd], a);
+            read(y, u + 2);
+            multiply(x, u, std::true_type{});
+            multiply(y, u + 2, std::true_type{});
         }
     }
-    if (t0 < hd) {
-        const float r = a + 0.0f;
-        out[(int64_t)b * q_bstride + (int64_t)h * hd + t0] = r;
-        if (img) {
-            const int kk = h * hd + t0;
-            img[(int64_t)(b >> 4) * 16 * d + (int64_t)(kk >> 4) * 256 + (kk & 3) * 64 + (b & 15) * 4 + ((kk & 15) >> 2)] = r;
-        }
+#pragma unroll
+    for (int w = 0; w < 2; ++w) {
+        const int c0 = (wave + TK_AT1_NW * w) * 16 + col;
+        if (c0 - col >= C || g != 0) break;
+        const int kk = h * hd + part * C + c0;
+        const float r = acc[w][0] + 0.0f;
+        out[(int64_t)b * q_bstride + kk] = r;
+        if (img) img[(int64_t)(b >> 4) * 16 * d + (int64_t)(kk >> 4) * 256 + (kk & 3) * 64 + (b & 15) * 4 + ((kk & 15) >> 2)] = r;
     }
+}
+/* bytes in front of the weights: the rings of K or a round of V, whichever is more */
+static int at1_buffer(int Tk, int C) {
+    const bool self = Tk <= TK_AT1_SELF;
+    const int blocks = (Tk + 15) / 16, rb = at1_round_blocks(self, C), round = (blocks < rb ? blocks : rb) * 64 * C, rings = self ? (Tk + 63) / 64 * TK_AT1_RING : 0;
+    return round > rings ? round : rings;
+}
+static bool at1_prepare_device() {
+    const int most = 160 * 1024;
+    return hipFuncSetAttribute((const void*)k_attend1<true>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+           hipFuncSetAttribute((const void*)k_attend1<false>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+           hipFuncSetAttribute((const void*)k_attend1_scores, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess;
+}
+/* scores: scratch [B][nh][pitch] */
+static bool at1_launch(const float* q, const float* k, const float* v, float* scores, int pitch, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh,
+                       float* img, hipStream_t s) {
+    const int hd = d / nh;
+    const float scale = tk_divf(1.0f, tk_sqrtf((float)hd));
+    int split = 1; /* workgroups per head: 16 outputs each at least, while all of them run at once */
+    while (hd % (32 * split) == 0 && 2 * split * nh * B <= 256) split *= 2;
+    const dim3 grid(nh * split, B), block(64 * TK_AT1_NW);
+    const int sc_at = at1_buffer(Tk, hd / split);
+    const size_t lds = (size_t)sc_at + (size_t)(((Tk + 15) & ~15) + hd + 8) * 4; /* <= 128 KiB + 3 KiB, 96 KiB + 10 KiB */
+    if (Tk <= TK_AT1_SELF) {
+        hipLaunchKernelGGL((k_attend1<true>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img);
+    } else {
+        hipLaunchKernelGGL(k_attend1_scores, dim3(((Tk + 63) / 64 + 3) / 4, nh, B), dim3(256), 4 * TK_AT1_RING + (size_t)hd * 4, s, q, k, scores, Tk, pitch, q_bstride, kv_bstride, d, hd, scale);
+        hipLaunchKernelGGL((k_attend1<false>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img);
+    }
+    return true;
 }
 
 /* ---------------------------------------------------------------- GPU ops for the shared graph */
@@ -308,14 +464,12 @@ struct TkAudioGpuOps {
         tk_launch_layernorm(x, rows, D, w, b, TK_WH_LN_EPS, y, s, img);
     }
     void softmax_rows(float* x, int rows, int cols, int ld) { drop_image(); tk_launch_softmax_rows(x, rows, cols, ld, s); }
-    bool attend1(const float* q, const float* k, const float* v, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh) {
+    bool attend1(const float* q, const float* k, const float* v, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh, float* scores, int pitch) {
         drop_image();
         const int hd = d / nh;
-        const size_t ldsb = ((size_t)TK_AT1_NS * TK_AT1_CK * hd + (size_t)Tk + (size_t)hd) * 4;
-        if (hd > 256 || (hd & 15) || (d & 3) || Tk < 1 || ldsb > 60 * 1024) return false; /* the three-launch form takes what does not fit */
+        if (hd > 256 || (hd & 15) || (d & 3) || Tk < 1 || Tk > TK_AT1_MAX_KEYS) return false; /* the three-launch form takes what does not fit */
         float* img = (short_pass(B) && d % 128 == 0 && q_bstride == d) ? image_for(out, B, d, d) : nullptr; /* the output projection's input, packed on the way out */
-        hipLaunchKernelGGL(k_attend1, dim3(nh, B), dim3(256), ldsb, s, q, k, v, out, Tk, q_bstride, kv_bstride, d, hd, tk_divf(1.0f, tk_sqrtf((float)hd)), img);
-        return true;
+        return at1_launch(q, k, v, scores, pitch, out, B, Tk, q_bstride, kv_bstride, d, nh, img, s);
     }
     /* the opt-in fast contraction's attention (TkAsr::fast): Q K^T, softmax and P V of a long pass in one kernel, no score matrix in HBM */
     bool attend_fused(const float* q, const float* k, const float* v, float* out, int B, int Tq, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh) {
@@ -377,7 +531,7 @@ struct TkAudioSizeOps {
     void im2col1d(const float*, int, int, int, int, int, int, int, float*) {}
     void layernorm(const float*, int rows, int D, const float*, const float*, float*) { image(rows, D); }
     void softmax_rows(float*, int, int, int) {}
-    bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int d, int) { image(B, d); return true; }
+    bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int d, int, float*, int) { image(B, d); return true; }
     bool attend_fused(const float*, const float*, const float*, float*, int, int, int, int64_t, int64_t, int, int) { return false; } /* sized for the exact form */
     void add_rows(float*, const float*, int, int, int) {}
     void embed_rows(const float*, const float*, const int32_t*, const int32_t*, int, int, float*) {}
@@ -515,7 +669,7 @@ bool TkAsr::init(TkWhisperModel* m, int mb) {
     (void)g.begin_decode(so, enc, mb);
     arena_floats = so.peak + 4096 + (size_t)3 * m->hp.n_text_ctx * mb + 64; /* + the decode loop's token / position / arg-max tables */
     if (!m->prepare_tiles()) { error = m->error; return false; }
-    if (!tk_gemm_tiled_prepare_device()) { error = "LDS opt-in of the tiled GEMM failed"; return false; }
+    if (!tk_gemm_tiled_prepare_device() || !at1_prepare_device()) { error = "LDS opt-in of the tiled GEMM or of the decoder's attention failed"; return false; }
     HIPQ(hipMalloc((void**)&arena, arena_floats * 4));
     return true;
 }

@@ -208,7 +208,7 @@ struct TkWhisperGraph {
     void attention(Ops& o, const float* q, const float* k, const float* v, float* out, int B, int Tq, int Tk, int64_t q_bstride, int64_t kv_bstride,
                    int d, int nh, float* scores) const {
         const int hd = d / nh;
-        if (Tq == 1 && o.attend1(q, k, v, out, B, Tk, q_bstride, kv_bstride, d, nh)) return; /* decoder steps: one kernel, same arithmetic */
+        if (Tq == 1 && o.attend1(q, k, v, out, B, Tk, q_bstride, kv_bstride, d, nh, scores, score_pitch(Tk))) return; /* decoder steps: same arithmetic */
         if (Tq > 1 && o.attend_fused(q, k, v, out, B, Tq, Tk, q_bstride, kv_bstride, d, nh)) return; /* opt-in fast path only */
         const int Tp = score_pitch(Tk);
         TkGemm s{};
