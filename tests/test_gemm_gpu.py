@@ -63,6 +63,17 @@ def test_block_forms_equal_the_chain(gpu, M, N, K):
         assert cs[i, j] == np.float32(acc + b[j])
 
 
+@pytest.mark.parametrize("M,N,K,f16", [
+    (1, 48, 384, 0), (16, 80, 2048, 0), (7, 64, 1536, 1),               # 16 rows: the whole range in the LDS, waves without a tile, the longest range
+    (16, 80, 2176, 0), (3, 48, 4096, 1),                                # in a ring
+    (17, 48, 1024, 0), (32, 80, 896, 1), (31, 96, 1152, 0),             # 32 rows: the longest whole range, one of 128s, a ring
+    (32, 4112, 256, 0), (1, 8208, 256, 1),                              # more than one tile per wave's workgroup
+])
+def test_few_rows_with_the_whole_range_or_a_ring(gpu, M, N, K, f16):
+    _, _, _, _, cs, ct = _pair(gpu, M, N, K, 0, f16, not f16, False, seed=K + M)
+    assert np.array_equal(cs.view(np.uint32), ct.view(np.uint32))
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 256, 1024), (48, 4096, 512), (256, 64, 256)])
 def test_f16_weight_tiles_equal_the_staged_f16_path(gpu, M, N, K):
     """fp16-checkpoint semantics: f16 weights, activations rounded through f16, fp32 chain"""

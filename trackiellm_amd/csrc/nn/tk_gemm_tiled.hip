@@ -22,7 +22,7 @@ __device__ __forceinline__ float tw_f16(uint32_t h) { return (float)__builtin_bi
 __device__ __forceinline__ void tw_wait_vmcnt(int n) {
 #define TK_VMW(k) case k: __builtin_amdgcn_s_waitcnt(0x0F70 | ((k) & 15) | (((k) >> 4) << 14)); break;
     switch (n) {
-        TK_VMW(0) TK_VMW(1) TK_VMW(2) TK_VMW(3) TK_VMW(4) TK_VMW(5) TK_VMW(6) TK_VMW(7) TK_VMW(8)
+        TK_VMW(0) TK_VMW(1) TK_VMW(2) TK_VMW(3) TK_VMW(4) TK_VMW(5) TK_VMW(6) TK_VMW(7) TK_VMW(8) TK_VMW(16)
         default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
     }
 #undef TK_VMW
@@ -37,10 +37,14 @@ __device__ __forceinline__ float tw_act(float v, int act) {
     }
 }
 
-/* WB = bytes per weight value (2: f16, 4: f32); MT = M-tiles per workgroup.  (Twelve weight pieces in flight for the Whisper decoder's
- * K = 384 launches — one round trip to the weights instead of three — measured 20 % SLOWER per launch: the whole activation image must
- * then land before the first MFMA, profiles/r04_perception.txt.) */
-template <int MT, int WB, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */>
+/* WB = bytes per weight value (2: f16, 4: f32); MT = M-tiles per workgroup.
+ * What bounds few rows: the chain, 8 cycles a k and M-tile, as long as weights and operands are there in time.  One LDS read takes a wave about 130
+ * cycles, so operands are read one pair of tiles ahead, also across the chunks of 32 k.  With a ring the compiler cannot count what is in flight
+ * behind the staging and lets the first weights of every PF chunks wait for all requests; where the activations of the whole K range fit the LDS
+ * (ONE: up to 2048 k at one M-tile, 1024 at two) there is no staging in the loop, and 8 pieces of weights stay in flight.
+ * Cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us, 384 x 1536 13.9 -> 10.2, 51872 x 384 24.0 -> 22.0; at 32 rows 8.6 -> 7.9, 20.8 -> 18.9
+ * (ring), 30.0 -> 27.0.  Twelve pieces: 384 x 384 at 1 row 5.6 (a wave's requests queue in front of the activations of the others). */
+template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */>
 __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, int total_row_tiles, int rk /* k per ring slot */, int slot_bytes /* ring slot pitch */) {
     constexpr int LPC = WB == 4 ? 2 : 1; /* 16-byte requests per piece and lane */
     constexpr int PIECE = 512 * WB;      /* bytes of one (row tile, 32 k) piece */
@@ -90,17 +94,36 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         if (LPC == 2) dst[LPC - 1] = tw_ldg_nt(p + 16);
     };
     stage(0, 0);
+    if (!active) { /* no tile of its own: its share of the staging */
+        for (int s = 0; s < nslots; ++s) {
+            tw_wait_vmcnt(0);
+            __syncthreads();
+            if (s + 1 < nslots) stage(s + 1, (s + 1) & 1);
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < PF; ++i) wload(i, wq[i]);
 
 #pragma unroll 1
-    for (int s = 0; s < nslots; ++s) {
+    for (int s = 0; s < (ONE ? 1 : nslots); ++s) {
         /* slot s has landed once all but the PF * LPC youngest requests are done: those are weight requests issued after its DMA
          * (cps >= PF chunks follow every slot's DMA, the PF initial ones the first) */
         tw_wait_vmcnt(PF * LPC);
         __syncthreads();
-        if (s + 1 < nslots) stage(s + 1, (s + 1) & 1);
-        const uint8_t* slot = lds + (size_t)(s & 1) * slot_bytes + lane * 16;
+        if (!ONE && s + 1 < nslots) stage(s + 1, (s + 1) & 1);
+        const uint8_t* slot = lds + (size_t)(ONE ? 0 : s & 1) * slot_bytes + lane * 16;
+        /* operands of M-tiles m, m + 1 (m alone of MT = 1) and chunk cc of the slot; [k half][tile] */
+        constexpr int PAIR = MT == 1 ? 1 : 2, PAIRS = MT / PAIR;
+        struct Ops { v4f a[2][PAIR]; } ops[2];
+        auto read = [&](Ops& o, int cc, int m) {
+            const uint8_t* ap = slot + (size_t)(2 * (cc < cps ? cc : cps - 1)) * MT * 1024 + m * 1024;
+#pragma unroll
+            for (int i = 0; i < PAIR; ++i)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) o.a[h][i] = *(const v4f*)(ap + (h * MT + i) * 1024);
+        };
+        read(ops[0], 0, 0);
 #pragma unroll 1
         for (int cc = 0; cc < cps; cc += PF) {
 #pragma unroll
@@ -116,52 +139,34 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                     wf[0] = __uint_as_float(w0.x); wf[1] = __uint_as_float(w0.y); wf[2] = __uint_as_float(w0.z); wf[3] = __uint_as_float(w0.w);
                     wf[4] = __uint_as_float(w1.x); wf[5] = __uint_as_float(w1.y); wf[6] = __uint_as_float(w1.z); wf[7] = __uint_as_float(w1.w);
                 }
-                wload(c + PF, wq[u]);
-                const uint8_t* ap = slot + (size_t)(2 * (cc + u)) * MT * 1024;
-                if (MT == 1) {
-                    const v4f a0 = *(const v4f*)ap, a1 = *(const v4f*)(ap + 1024);
-                    if (active) {
-                        v4f d = {acc[0][0], acc[0][1], acc[0][2], acc[0][3]};
+                if (WB == 2 || !ONE) wload(c + PF, wq[u]);
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) d = __builtin_amdgcn_mfma_f32_16x16x4f32(a0[t], wf[t], d, 0, 0, 0);
+                for (int p = 0; p < PAIRS; ++p) {
+                    /* the next pair's operand reads, the next chunk's behind the last pair, are issued before this pair's MFMAs; of two tiles the
+                     * chains alternate (a chain step's 40-cycle dependent latency hides behind the other chain's MFMA) */
+                    const int step = u * PAIRS + p, m = p * PAIR;
+                    Ops& o = ops[step & 1];
+                    if (p + 1 < PAIRS) read(ops[(step + 1) & 1], cc + u, m + PAIR);
+                    else read(ops[(step + 1) & 1], cc + u + 1, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    {
+                        v4f d[PAIR];
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) d = __builtin_amdgcn_mfma_f32_16x16x4f32(a1[t], wf[4 + t], d, 0, 0, 0);
-                        acc[0][0] = d[0]; acc[0][1] = d[1]; acc[0][2] = d[2]; acc[0][3] = d[3];
-                    }
-                } else {
-                    /* M-tiles in pairs: the two accumulators' chains alternate (a chain step's 40-cycle dependent latency hides behind the
-                     * other chain's MFMA) and the next pair's operand reads are issued before this pair's MFMAs */
-                    v4f A0[2][2], A1[2][2]; /* [buffer][tile of the pair] */
-                    A0[0][0] = *(const v4f*)(ap); A1[0][0] = *(const v4f*)(ap + MT * 1024);
-                    A0[0][1] = *(const v4f*)(ap + 1024); A1[0][1] = *(const v4f*)(ap + (MT + 1) * 1024);
+                        for (int i = 0; i < PAIR; ++i) d[i] = v4f{acc[m + i][0], acc[m + i][1], acc[m + i][2], acc[m + i][3]};
 #pragma unroll
-                    for (int m = 0; m < MT; m += 2) {
-                        const int cur = (m >> 1) & 1, nxt = cur ^ 1;
-                        if (m + 2 < MT) {
-                            A0[nxt][0] = *(const v4f*)(ap + (m + 2) * 1024); A1[nxt][0] = *(const v4f*)(ap + (MT + m + 2) * 1024);
-                            A0[nxt][1] = *(const v4f*)(ap + (m + 3) * 1024); A1[nxt][1] = *(const v4f*)(ap + (MT + m + 3) * 1024);
-                        }
-                        if (active) {
-                            v4f d0 = {acc[m][0], acc[m][1], acc[m][2], acc[m][3]}, d1 = {acc[m + 1][0], acc[m + 1][1], acc[m + 1][2], acc[m + 1][3]};
+                        for (int t = 0; t < 8; ++t)
 #pragma unroll
-                            for (int t = 0; t < 4; ++t) {
-                                d0 = __builtin_amdgcn_mfma_f32_16x16x4f32(A0[cur][0][t], wf[t], d0, 0, 0, 0);
-                                d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(A0[cur][1][t], wf[t], d1, 0, 0, 0);
-                            }
+                            for (int i = 0; i < PAIR; ++i) d[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.a[t >> 2][i][t & 3], wf[t], d[i], 0, 0, 0);
 #pragma unroll
-                            for (int t = 0; t < 4; ++t) {
-                                d0 = __builtin_amdgcn_mfma_f32_16x16x4f32(A1[cur][0][t], wf[4 + t], d0, 0, 0, 0);
-                                d1 = __builtin_amdgcn_mfma_f32_16x16x4f32(A1[cur][1][t], wf[4 + t], d1, 0, 0, 0);
-                            }
-                            acc[m][0] = d0[0]; acc[m][1] = d0[1]; acc[m][2] = d0[2]; acc[m][3] = d0[3];
-                            acc[m + 1][0] = d1[0]; acc[m + 1][1] = d1[1]; acc[m + 1][2] = d1[2]; acc[m + 1][3] = d1[3];
-                        }
+                        for (int i = 0; i < PAIR; ++i)
+#pragma unroll
+                            for (int r = 0; r < 4; ++r) acc[m + i][r] = d[i][r];
                     }
                 }
+                if (WB == 4 && ONE) wload(c + PF, wq[u]);
             }
         }
     }
-    if (!active) return;
     const int g = lane >> 4;
     const int n = col_base + rt * TK_TW_ROWS_PER_TILE + (lane & 15);
     if (n >= a.n_valid) return;
@@ -287,8 +292,9 @@ bool tk_gemm_tiled_prepare_device() {
     if (g_tw_opted[dev].load(std::memory_order_acquire)) return true;
     std::lock_guard<std::mutex> lk(g_tw_mu);
     hipError_t e = hipSuccess;
-#define TK_TW_OPT(MTV, PFV) do { if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<MTV, 2, PFV>); if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<MTV, 4, PFV>); } while (0)
-    TK_TW_OPT(1, 4); TK_TW_OPT(2, 4); TK_TW_OPT(4, 4); TK_TW_OPT(8, 4); TK_TW_OPT(16, 2); TK_TW_OPT(8, 2); TK_TW_OPT(6, 2);
+#define TK_TW_OPT(MTV, ONEV, PFV) do { if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<MTV, 2, ONEV, PFV>); if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<MTV, 4, ONEV, PFV>); } while (0)
+    TK_TW_OPT(1, true, 4); TK_TW_OPT(1, true, 8); TK_TW_OPT(2, true, 4); TK_TW_OPT(2, true, 8);
+    TK_TW_OPT(1, false, 4); TK_TW_OPT(2, false, 4); TK_TW_OPT(4, false, 4); TK_TW_OPT(8, false, 4); TK_TW_OPT(16, false, 2); TK_TW_OPT(8, false, 2); TK_TW_OPT(6, false, 2);
 #undef TK_TW_OPT
     if (e != hipSuccess) return false;
     g_tw_opted[dev].store(true, std::memory_order_release);
@@ -323,9 +329,10 @@ bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
         if (groups > row_tiles) groups = row_tiles;
         waves = (row_tiles + groups - 1) / groups;
         while (waves > 8) { groups *= 2; waves = (row_tiles + groups - 1) / groups; }
-        if (waves == 1 && row_tiles >= 4) { /* fewer tiles than CUs: four one-tile waves (one per SIMD) share a workgroup's ring staging */
-            waves = 4;
-            groups = (row_tiles + 3) / 4;
+        if (waves == 1 && row_tiles >= 4) { /* fewer tiles than CUs: one-tile waves that share a workgroup's staging.  More of them ask one CU for more weights at a time,
+             * fewer stage more each: 384 x 1536 at 1 row 10.9, 10.2, 10.8 us with 1, 2, 4 waves, at 32 rows 24.8, 20.7, 18.9 */
+            waves = mt == 1 ? 2 : 4;
+            groups = (row_tiles + waves - 1) / waves;
         }
     } else {
         waves = row_tiles < 8 ? row_tiles : 8;
@@ -333,28 +340,29 @@ bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
     }
     const int Kr = a.K / a.ks;
     /* k per ring slot: the largest multiple of 32 PF that divides the K range and fits a 64 KiB slot (rk / 16 * mt KiB) — a whole short
-     * range in one slot spares a small launch its ring hand-overs (Whisper decoder: K = 384 at two M-tiles is one 48 KiB slot).
+     * range in one slot (`one`, up to 128 KiB) needs no ring.
      * Many row blocks of 128 rows (the Whisper encoder's linears, 48000 rows): 32 KiB slots and two weight pieces in flight instead, so
      * that TWO workgroups share a CU and one's ring fill and epilogue run under the other's MFMAs. */
     const bool twin = ny > 1 && (mt == 8 || mt == 6) && Kr % 64 == 0;
-    const int pf = (mt == 16 || twin) ? 2 : 4;
+    const bool one = mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES;
+    const int pf = mt == 16 || twin ? 2 : one ? (Kr % 256 == 0 ? 8 : 4) : 4;
     const int slot_kib = twin ? 32 : 64;
-    int rk = 0;
-    for (int c = (slot_kib * 16 / mt) / (32 * pf) * (32 * pf); c >= 32 * pf; c -= 32 * pf)
+    int rk = one ? Kr : 0;
+    for (int c = (slot_kib * 16 / mt) / (32 * pf) * (32 * pf); rk == 0 && c >= 32 * pf; c -= 32 * pf)
         if (Kr % c == 0) { rk = c; break; }
     if (rk == 0) return false;
     if (Kr % rk) return false;
     const int slot_bytes = twin ? slot_kib * 1024 : TK_TW_SLOT_BYTES;
-    const size_t ldsb = (size_t)2 * slot_bytes;
-#define TK_TW_LAUNCH(MTV, WBV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, PFV>), dim3(groups * a.ks, ny), dim3(64 * waves), ldsb, s, a, groups, row_tiles, rk, slot_bytes)
-#define TK_TW_WB(MTV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, PFV); else TK_TW_LAUNCH(MTV, 4, PFV); } while (0)
+    const size_t ldsb = one ? (size_t)Kr * mt * 64 : (size_t)2 * slot_bytes;
+#define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(groups * a.ks, ny), dim3(64 * waves), ldsb, s, a, groups, row_tiles, rk, slot_bytes)
+#define TK_TW_WB(MTV, ONEV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, ONEV, PFV); else TK_TW_LAUNCH(MTV, 4, ONEV, PFV); } while (0)
     switch (mt) {
-        case 1: TK_TW_WB(1, 4); break;
-        case 2: TK_TW_WB(2, 4); break;
-        case 4: TK_TW_WB(4, 4); break;
-        case 6: TK_TW_WB(6, 2); break;
-        case 8: if (twin) TK_TW_WB(8, 2); else TK_TW_WB(8, 4); break;
-        default: TK_TW_WB(16, 2); break;
+        case 1: if (one) { if (pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
+        case 2: if (one) { if (pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
+        case 4: TK_TW_WB(4, false, 4); break;
+        case 6: TK_TW_WB(6, false, 2); break;
+        case 8: if (twin) TK_TW_WB(8, false, 2); else TK_TW_WB(8, false, 4); break;
+        default: TK_TW_WB(16, false, 2); break;
     }
 #undef TK_TW_WB
 #undef TK_TW_LAUNCH
