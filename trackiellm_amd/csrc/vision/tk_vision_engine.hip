@@ -256,9 +256,11 @@ struct TkSizeOps {
 
 /* ------------------------------------------------------------------------------------------ decode + NMS kernels */
 
-__global__ void k_yolo_decode(TkT h0, TkT h1, TkT h2, int nc, int n_anchors, float conf, tk_yolo_cand_t* cand) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x, b = blockIdx.y;
-    if (a >= n_anchors) return;
+/* Four lanes per anchor: lane q takes side q of the box and the classes q, q + 4, ... (first class on ties, as tk_yolo_decode_anchor).  One thread per
+ * anchor was a chain of 64 + nc exponentials on a tenth of the chip: 29 us for the 8400 anchors of one 640 x 640 frame, now 9. */
+__global__ __launch_bounds__(256) void k_yolo_decode(TkT h0, TkT h1, TkT h2, int nc, int n_anchors, float conf, tk_yolo_cand_t* cand) {
+    const int a = (blockIdx.x * 256 + threadIdx.x) >> 2, q = threadIdx.x & 3, b = blockIdx.y;
+    if (a >= n_anchors) return; /* all four lanes of an anchor */
     const int n0 = h0.H * h0.W, n1 = h1.H * h1.W;
     const TkT* h;
     int local;
@@ -267,11 +269,24 @@ __global__ void k_yolo_decode(TkT h0, TkT h1, TkT h2, int nc, int n_anchors, flo
     else if (a < n0 + n1) { h = &h1; local = a - n0; stride = 16.0f; }
     else { h = &h2; local = a - n0 - n1; stride = 32.0f; }
     const float ax = (float)(local % h->W) + 0.5f, ay = (float)(local / h->W) + 0.5f;
-    tk_yolo_cand_t c;
-    tk_yolo_decode_anchor(h->p + ((size_t)b * h->H * h->W + local) * h->ld, nc, ax, ay, stride, &c);
-    c.anchor = a;
-    if (!(c.score > conf)) c.cls = -1; /* not a candidate */
-    cand[(size_t)b * n_anchors + a] = c;
+    const float* o = h->p + ((size_t)b * h->H * h->W + local) * h->ld;
+    const float d = tk_yolo_dfl(o + 16 * q);
+    float best = -1.0f;
+    int bi = 0;
+    for (int k = q; k < nc; k += 4) {
+        const float s = tk_sigmoidf(o[64 + k]);
+        if (s > best) { best = s; bi = k; }
+    }
+#pragma unroll
+    for (int w = 1; w <= 2; w <<= 1) {
+        const float os = __shfl_xor(best, w, 64);
+        const int oi = __shfl_xor(bi, w, 64);
+        if (os > best || (os == best && oi < bi)) { best = os; bi = oi; }
+    }
+    const float at = q & 1 ? ay : ax, edge = (q < 2 ? at - d : at + d) * stride; /* x1 y1 x2 y2 */
+    tk_yolo_cand_t* c = cand + (size_t)b * n_anchors + a;
+    (&c->x1)[q] = edge;
+    if (q == 0) { c->score = best; c->cls = best > conf ? bi : -1 /* not a candidate */; c->anchor = a; }
 }
 
 /* a YOLO-class graph's own output [4 + nc][anchors] (Ultralytics export: box centre / size in input pixels, class probabilities already through
@@ -287,36 +302,64 @@ __global__ void k_yolo_decode_out(const float* out, int nc, int n_anchors, float
 }
 
 /* rank of every candidate among the candidates: (score desc, anchor asc); the best MAX_CAND are kept.  Most anchors fall below the
- * confidence threshold, so each 256-anchor tile is compacted in LDS first (ballot + prefix) and only its survivors are compared. */
+ * confidence threshold, so each 1024-anchor tile is compacted in LDS first (ballot + prefix) and only its survivors are compared.  A tile's scores are
+ * requested under the tile before, survivors are read
+ * eight at a time: 8400 anchors 41 -> 22 us. */
 __global__ __launch_bounds__(256) void k_yolo_rank(const tk_yolo_cand_t* cand, int n_anchors, int32_t* order, int32_t* n_cand) {
     const int b = blockIdx.y;
     const tk_yolo_cand_t* cb = cand + (size_t)b * n_anchors;
     const int a = blockIdx.x * blockDim.x + threadIdx.x;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    __shared__ float ss[256];
-    __shared__ int sj[256];
-    __shared__ int wcnt[4];
-    const bool valid = a < n_anchors && cb[a].cls >= 0;
-    const float mys = valid ? cb[a].score : 0.0f;
-    int rank = 0, total = 0;
-    for (int base = 0; base < n_anchors; base += 256) {
-        const int j = base + threadIdx.x;
-        const bool v = j < n_anchors && cb[j].cls >= 0;
-        const float sco = v ? cb[j].score : 0.0f;
-        const uint64_t bal = __ballot(v);
-        if (lane == 0) wcnt[wave] = __popcll(bal);
-        __syncthreads();
-        int off = 0, nt = 0;
+    __shared__ __attribute__((aligned(16))) float2 tile[1024 + 8]; /* score, anchor (as bits) */
+    __shared__ int wcnt[16];
+    const int own = a < n_anchors ? a : n_anchors - 1;
+    const bool valid = a < n_anchors && cb[own].cls >= 0;
+    const float mys = cb[own].score;
+    float sco[4];
+    int cls[4];
+    auto load = [&](int base) { /* past the last anchor: read again, not used */
 #pragma unroll
-        for (int w = 0; w < 4; ++w) { const int c = wcnt[w]; if (w < wave) off += c; nt += c; }
-        if (v) {
-            const int pos = off + __popcll(bal & ((1ull << lane) - 1ull));
-            ss[pos] = sco; sj[pos] = j;
+        for (int u = 0; u < 4; ++u) {
+            int j = base + u * 256 + (int)threadIdx.x;
+            j = j < n_anchors ? j : n_anchors - 1;
+            sco[u] = cb[j].score; cls[u] = cb[j].cls;
+        }
+    };
+    load(0);
+    int rank = 0, total = 0;
+    for (int base = 0; base < n_anchors; base += 1024) {
+        uint64_t bal[4];
+        float s0[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            s0[u] = sco[u];
+            bal[u] = __ballot(base + u * 256 + (int)threadIdx.x < n_anchors && cls[u] >= 0);
+            if (lane == 0) wcnt[u * 4 + wave] = __popcll(bal[u]);
         }
         __syncthreads();
+        if (base + 1024 < n_anchors) load(base + 1024);
+        int nt = 0, off[4];
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            if ((w & 3) == wave) off[w >> 2] = nt;
+            nt += wcnt[w];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (bal[u] >> lane & 1) {
+                const int pos = off[u] + __popcll(bal[u] & ((1ull << lane) - 1ull));
+                tile[pos] = make_float2(s0[u], __int_as_float(base + u * 256 + (int)threadIdx.x));
+            }
+        if (threadIdx.x < 8) tile[nt + threadIdx.x] = make_float2(-INFINITY, 0.0f); /* below every candidate */
+        __syncthreads();
         if (valid)
-            for (int k = 0; k < nt; ++k)
-                if (ss[k] > mys || (ss[k] == mys && sj[k] < a)) ++rank;
+            for (int k = 0; k < nt; k += 8) {
+                float2 o[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) o[u] = tile[k + u];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) rank += o[u].x > mys || (o[u].x == mys && __float_as_int(o[u].y) < a) ? 1 : 0;
+            }
         total += nt;
         __syncthreads();
     }
@@ -324,53 +367,77 @@ __global__ __launch_bounds__(256) void k_yolo_rank(const tk_yolo_cand_t* cand, i
     if (a == 0) n_cand[b] = total < TK_YOLO_MAX_CAND ? total : TK_YOLO_MAX_CAND;
 }
 
-/* suppression bit matrix: bit j of mask[i] set iff j > i, same class, IoU > thr */
-__global__ void k_yolo_mask(const tk_yolo_cand_t* cand, int n_anchors, const int32_t* order, const int32_t* n_cand, float iou_thr, uint64_t* mask) {
-    const int b = blockIdx.z;
+/* suppression bit matrix: bit j of mask[i] set iff j > i, same class, IoU > thr.  A wave holds 64 candidates j, one a lane, and takes 32 rows i: a row's
+ * word is the ballot.  (A thread per word, which fetched its 64 candidates one after the other: 27 us for some tens of candidates, now 10.) */
+__global__ __launch_bounds__(256) void k_yolo_mask(const tk_yolo_cand_t* cand, int n_anchors, const int32_t* order, const int32_t* n_cand, float iou_thr, uint64_t* mask) {
+    __shared__ tk_yolo_cand_t rows[32];
+    const int b = blockIdx.z, lane = threadIdx.x & 63, wj = blockIdx.x * 4 + (threadIdx.x >> 6), i0 = blockIdx.y * 32;
     const int n = n_cand[b];
-    const int i = blockIdx.y * blockDim.y + threadIdx.y;
-    const int wj = blockIdx.x * blockDim.x + threadIdx.x; /* 64-candidate word */
-    if (i >= n || wj * 64 >= n) return;
+    if (i0 >= n || blockIdx.x * 256 >= n) return;
     const tk_yolo_cand_t* cb = cand + (size_t)b * n_anchors;
     const int32_t* ob = order + (size_t)b * TK_YOLO_MAX_CAND;
-    const tk_yolo_cand_t ci = cb[ob[i]];
-    uint64_t bits = 0;
-    for (int k = 0; k < 64; ++k) {
-        const int j = wj * 64 + k;
-        if (j <= i || j >= n) continue;
-        const tk_yolo_cand_t cj = cb[ob[j]];
-        if (cj.cls == ci.cls && tk_yolo_iou(&ci, &cj) > iou_thr) bits |= 1ull << k;
+    if (threadIdx.x < 32 && i0 + (int)threadIdx.x < n) rows[threadIdx.x] = cb[ob[i0 + threadIdx.x]];
+    const int j = wj * 64 + lane;
+    const tk_yolo_cand_t cj = cb[ob[j < n ? j : n - 1]];
+    __syncthreads();
+    if (wj * 64 >= n) return;
+    for (int i = i0; i < n && i < i0 + 32; ++i) {
+        const tk_yolo_cand_t ci = rows[i - i0];
+        const uint64_t bits = __ballot(j > i && j < n && cj.cls == ci.cls && tk_yolo_iou(&ci, &cj) > iou_thr);
+        if (lane == 0) mask[((size_t)b * TK_YOLO_MAX_CAND + i) * (TK_YOLO_MAX_CAND / 64) + wj] = bits;
     }
-    mask[((size_t)b * TK_YOLO_MAX_CAND + i) * (TK_YOLO_MAX_CAND / 64) + wj] = bits;
 }
 
-/* greedy scan, one wave per frame */
-__global__ void k_yolo_scan(const tk_yolo_cand_t* cand, int n_anchors, const int32_t* order, const int32_t* n_cand, const uint64_t* mask,
-                            TkDetection* kept, int32_t* n_kept) {
+/* greedy scan, one wave per frame: 64 candidates at a time, whose words among themselves are in the lanes, so that a kept one costs a few scalar steps and
+ * no trip to memory (44 us for some tens of kept boxes, now 8); the later words take the kept rows eight loads at a time */
+__global__ __launch_bounds__(64) void k_yolo_scan(const tk_yolo_cand_t* cand, int n_anchors, const int32_t* order, const int32_t* n_cand, const uint64_t* mask,
+                                                  TkDetection* kept, int32_t* n_kept) {
     const int b = blockIdx.x, lane = threadIdx.x;
-    __shared__ uint64_t removed[TK_YOLO_MAX_CAND / 64];
+    constexpr int WORDS = TK_YOLO_MAX_CAND / 64;
+    static_assert(WORDS <= 64, "a lane per word");
     const int n = n_cand[b];
     const int words = (n + 63) / 64;
-    for (int w = lane; w < TK_YOLO_MAX_CAND / 64; w += 64) removed[w] = 0;
-    __syncthreads();
     const tk_yolo_cand_t* cb = cand + (size_t)b * n_anchors;
     const int32_t* ob = order + (size_t)b * TK_YOLO_MAX_CAND;
+    const uint64_t* mb = mask + (size_t)b * TK_YOLO_MAX_CAND * WORDS;
+    uint64_t removed = 0; /* lane w: word w */
     int nk = 0;
-    for (int i = 0; i < n && nk < TK_OBJECT_DETECTOR_MAX_DETECTIONS; ++i) {
-        const bool dead = (removed[i >> 6] >> (i & 63)) & 1;
-        if (!dead) {
-            const uint64_t* mrow = mask + ((size_t)b * TK_YOLO_MAX_CAND + i) * (TK_YOLO_MAX_CAND / 64);
-            for (int w = lane; w < words; w += 64) removed[w] |= mrow[w];
-            if (lane == 0) {
-                const tk_yolo_cand_t c = cb[ob[i]];
-                TkDetection dt{c.x1, c.y1, c.x2, c.y2, c.score, c.cls, c.anchor};
-                kept[(size_t)b * TK_OBJECT_DETECTOR_MAX_DETECTIONS + nk] = dt;
-            }
-            ++nk;
+    auto lane_of = [](uint64_t v, int l) {
+        return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, l) | (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), l) << 32;
+    };
+    for (int w = 0; w < words && nk < TK_OBJECT_DETECTOR_MAX_DETECTIONS; ++w) {
+        const int i = w * 64 + lane;
+        const uint64_t mine = i < n ? mb[(size_t)i * WORDS + w] : 0;
+        const tk_yolo_cand_t c = cb[ob[i < n ? i : n - 1]];
+        uint64_t left = ~lane_of(removed, w) & (n - w * 64 >= 64 ? ~0ull : (1ull << (n - w * 64)) - 1ull), keep = 0;
+        while (left != 0) {
+            const int k = __builtin_ctzll(left);
+            keep |= 1ull << k;
+            left &= ~(1ull << k) & ~lane_of(mine, k); /* a row marks later candidates only */
         }
-        __syncthreads();
+        const int at = nk + __popcll(keep & ((1ull << lane) - 1ull));
+        if ((keep >> lane & 1) && at < TK_OBJECT_DETECTOR_MAX_DETECTIONS) {
+            TkDetection dt{c.x1, c.y1, c.x2, c.y2, c.score, c.cls, c.anchor};
+            kept[(size_t)b * TK_OBJECT_DETECTOR_MAX_DETECTIONS + at] = dt;
+        }
+        nk += __popcll(keep);
+        if (w + 1 < words) {
+            const int word = lane < words ? lane : words - 1;
+            while (keep != 0) {
+                uint64_t r[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) { /* past the last kept one: it again */
+                    const int k = __builtin_ctzll(keep);
+                    r[u] = mb[(size_t)(w * 64 + k) * WORDS + word];
+                    const uint64_t rest = keep & (keep - 1);
+                    keep = u < 7 && rest == 0 ? keep : rest;
+                }
+#pragma unroll
+                for (int u = 0; u < 8; ++u) removed |= r[u];
+            }
+        }
     }
-    if (lane == 0) n_kept[b] = nk;
+    if (lane == 0) n_kept[b] = nk < TK_OBJECT_DETECTOR_MAX_DETECTIONS ? nk : TK_OBJECT_DETECTOR_MAX_DETECTIONS;
 }
 
 /* ------------------------------------------------------------------------------------------ detector */
@@ -453,7 +520,7 @@ bool TkDetector::forward_graph(int B, const float* nchw_host, std::vector<float>
     last_B = 0;
     if (!run_graph(B, out->data())) return false;
     hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
-    hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 64 / 8, TK_YOLO_MAX_CAND / 8, B), dim3(8, 8), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
+    hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
     hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept);
     HIPQ(hipGetLastError());
     HIPQ(hipStreamSynchronize(stream));
@@ -464,7 +531,7 @@ bool TkDetector::enqueue(int B) {
     if (model->generic) {
         if (!run_graph(B, nullptr)) return false;
         hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
-        hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 64 / 8, TK_YOLO_MAX_CAND / 8, B), dim3(8, 8), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
+        hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
         hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept);
         HIPQ(hipGetLastError());
         return true;
@@ -474,9 +541,9 @@ bool TkDetector::enqueue(int B) {
     TkT x;
     x.p = input; x.B = B; x.H = in_h; x.W = in_w; x.C = 3; x.ld = 3;
     TkYoloV8n<TkGpuOps>::forward(ops, x, heads, model->nc);
-    hipLaunchKernelGGL(k_yolo_decode, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, heads[0], heads[1], heads[2], model->nc, n_anchors, conf, cand);
+    hipLaunchKernelGGL(k_yolo_decode, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, heads[0], heads[1], heads[2], model->nc, n_anchors, conf, cand);
     hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
-    hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 64 / 8, TK_YOLO_MAX_CAND / 8, B), dim3(8, 8), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
+    hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
     hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept);
     HIPQ(hipGetLastError());
     return true;
