@@ -1326,8 +1326,45 @@ __global__ __launch_bounds__(256) void k_layernorm(const float* x, int D, const 
         if (ir) ir[(int64_t)(i >> 4) * 256 + (i & 3) * 64 + ((i & 15) >> 2)] = v;
     }
 }
+/* rows of up to 256 NV columns: k_layernorm on registers (thread j owns elements j, j + 256, ...), in the same order.  The row, w and b are requested
+ * together: one trip to memory instead of three in a row (384 columns: one row 2.7 against 3.6 us, 48 000 rows 78 against 111) */
+template <int NV>
+__global__ __launch_bounds__(256) void k_layernorm_reg(const float* x, int D, const float* w, const float* b, float eps, float* y, float* img) {
+    __shared__ float red[4];
+    const int64_t r = blockIdx.x;
+    const float* xr = x + r * D;
+    float v[NV], wv[NV], bv[NV];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        int i = threadIdx.x + 256 * u;
+        i = i < D ? i : D - 1;
+        v[u] = xr[i]; wv[u] = w[i]; bv[u] = b[i];
+    }
+    float s = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+        if (threadIdx.x + 256 * u < D) s = s + v[u];
+    const float mean = tk_divf(nn_block_sum256(s, red), (float)D);
+    float q = 0.0f;
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+        if (threadIdx.x + 256 * u < D) { const float d = v[u] - mean; q = tk_fmaf(d, d, q); }
+    const float var = tk_divf(nn_block_sum256(q, red), (float)D);
+    const float rstd = tk_divf(1.0f, tk_sqrtf(var + eps));
+    float* ir = img ? img + (r >> 4) * 16 * (int64_t)D + (r & 15) * 4 : nullptr;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int i = threadIdx.x + 256 * u;
+        if (i >= D) break;
+        const float o = ((v[u] - mean) * rstd) * wv[u] + bv[u];
+        y[r * D + i] = o;
+        if (ir) ir[(int64_t)(i >> 4) * 256 + (i & 3) * 64 + ((i & 15) >> 2)] = o;
+    }
+}
 void tk_launch_layernorm(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, hipStream_t s, float* img) {
-    hipLaunchKernelGGL(k_layernorm, dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
+    if (D <= 512) hipLaunchKernelGGL((k_layernorm_reg<2>), dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
+    else if (D <= 1280) hipLaunchKernelGGL((k_layernorm_reg<5>), dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
+    else hipLaunchKernelGGL(k_layernorm, dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
 }
 
 /* in-place row softmax over the first `cols` entries of every row (row pitch ld) */
