@@ -227,6 +227,30 @@ def test_runs_in_chunks_beside_short_ones(gpu, tmp_path, dim, vdim, steep):
         assert U.rel_rms(np.array(rows), c.want(p)[0], 0.9 if steep else 1.0) < F32
 
 
+@pytest.mark.parametrize("at", [0, 15, 16, 37, 57])
+@pytest.mark.parametrize("operand", ["v", "k", "q", "a1"])
+def test_non_finite_values_stay_with_their_position(gpu, tmp_path, operand, at):
+    """an overflow in one position's value, key, query or decay: the positions before it, of its own chunk too, and the other sequence of the
+    pass keep their bits"""
+    cfg = config(40, 50, [layer(attention(2, 2, 8, 8, 4, 70, 1), delta(3, 1, 20, 36, 4), None)])
+    w = U.random_weights(cfg, 3)
+    for name, m in w.items():
+        if m.ndim == 2 and m.shape[-1] == 40 and name not in ("embed", "head"):
+            m[:, 7] = 0.0
+    w["l0.mix.right." + operand][:, 7] = 16.0
+    w["embed"][:, 7] = 0.0
+    w["embed"][49, 7] = U.bf16_round(np.float32(3e38))
+    s = Case(gpu, tmp_path, cfg, w=w).session("float32", 2, 160)
+    a, b = ([t % 49 for t in tokens_for(cfg, n, n)] for n in (58, 45))
+    broken = a[:at] + [49] + a[at + 1:]
+
+    def run(x):
+        return s.forward_rows([0] * 58 + [1] * 45, [*range(58), *range(45)], x + b, range(103))[0]
+    good, got = run(a), run(broken)
+    assert np.isfinite(good).all() and not np.isfinite(got[at]).all()
+    assert np.array_equal(got[:at], good[:at]) and np.array_equal(got[58:], good[58:])
+
+
 @pytest.mark.parametrize("dim,vdim", [(20, 20), (40, 36), (70, 17), (130, 20)])
 def test_many_heads_and_sequences(gpu, tmp_path, dim, vdim):
     """the recurrence's form for many columns at once: eight sequences of unequal length x 32 heads in one pass, then portions and single tokens"""

@@ -994,8 +994,11 @@ __global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t,
 /* The chunks of a segment in order: a workgroup owns 16 columns of one head's state, each of its four waves a quarter of the key rows, in
  * accumulator registers, which are at once the products' right-hand operands.  Per chunk 26 MFMAs a wave and one barrier: the partial sums of W S
  * meet in LDS, every wave adds them up (ascending) and goes on; those of the output are added a chunk later, off the chain.  Operands are requested
- * three chunks ahead. */
-template <int DP>
+ * three chunks ahead.
+ * The zeros of T and B must not meet an infinity or NaN, which would reach the tokens before its own.  A test per chunk cost 18 us on top of the 108, so a
+ * second launch (AGAIN, 2 us) looks at the states that the first has left, where what is not finite stays (0 x infinity is NaN): it walks columns that
+ * have any once more, without those zeros, and leaves at once otherwise. */
+template <int DP, bool AGAIN>
 __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t) {
     constexpr int NT = DP / 64, AHEAD = 3;
     __shared__ tk_v4f pu[2][4][64], po[2][4][64];
@@ -1005,6 +1008,7 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
     if (n < TK_DELTA_CHUNKED) return;
     const bool live = col < d.vdim;
     const int nc = (n + DC - 1) / DC;
+    if (AGAIN && !__syncthreads_or(live && !__builtin_isfinite(d.state[((size_t)out * d.heads + h) * d.dim * vp + col]))) return;
     tk_v4f S[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i)
@@ -1039,10 +1043,24 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
         const float o = ((po[b][0][l][ot & 3] + po[b][1][l][ot & 3]) + po[b][2][l][ot & 3]) + po[b][3][l][ot & 3];
         if (c >= 0 && c * DC + ot < n && oc < d.vdim) d.o[((size_t)(row0 + c * DC + ot) * d.heads + h) * d.vdim + oc] = o;
     };
+    /* c + a b over this wave's four tokens, a = T or B: row t has the tokens up to t */
+    auto tokens_before = [&](float a, float b, tk_v4f c) -> tk_v4f {
+        if (!AGAIN) return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float bk = __shfl(b, 16 * k + (lane & 15), 64);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float ak = __shfl(a, 16 * k + 4 * g + r, 64);
+                if (4 * k + wave <= 4 * g + r) c[r] = fmaf(ak, bk, c[r]);
+            }
+        }
+        return c;
+    };
     auto chunk = [&](Ops& o, Ops& next, int c) {
         fetch(next, c + AHEAD < nc ? c + AHEAD : nc - 1); /* never skipped: a branch here would make every wait one for the youngest request */
         tk_v4f u = {0.0f, 0.0f, 0.0f, 0.0f}, y = u;
-        u = __builtin_amdgcn_mfma_f32_16x16x4f32(o.t, o.v, u, 0, 0, 0);
+        u = tokens_before(o.t, o.v, u);
 #pragma unroll
         for (int i = 0; i < NT; ++i)
 #pragma unroll
@@ -1062,7 +1080,7 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
 #pragma unroll
             for (int r = 0; r < 4; ++r) S[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(o.k[i][r], u[r], S[i], 0, 0, 0);
         }
-        y = __builtin_amdgcn_mfma_f32_16x16x4f32(o.b, u[wave & 3], y, 0, 0, 0);
+        y = tokens_before(o.b, u[wave & 3], y);
         finish(c - 1);
         po[b][wave][lane] = y;
     };
@@ -1870,7 +1888,8 @@ size_t tk_delta_chunk_floats(int heads, int dim, int rows, int segments) { retur
 void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int longest, int nrows, hipStream_t s) {
     if (longest >= TK_DELTA_CHUNKED) {
         const dim3 chunks(d.heads, nrows / DC + n_segments), chain(d.heads, (d.vdim + 15) / 16, n_segments); /* heads first: a head's workgroups share an XCD's L2 */
-#define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_segments); hipLaunchKernelGGL((k_delta_chain<DP>), chain, dim3(256), 0, s, d, t); } while (0)
+#define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_segments); \
+        hipLaunchKernelGGL((k_delta_chain<DP, false>), chain, dim3(256), 0, s, d, t); hipLaunchKernelGGL((k_delta_chain<DP, true>), chain, dim3(256), 0, s, d, t); } while (0)
         switch (delta_pad(d.dim)) {
             case 64: TK_CHUNKED(64); break;
             case 128: TK_CHUNKED(128); break;
