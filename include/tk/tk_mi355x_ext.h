@@ -250,6 +250,11 @@ TK_API const char* tk_mi355x_llm_runner_tool_call_text(struct tk_llm_runner_s* r
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_pair(int device, int M, int N, int K, const float* a, const float* w, const float* bias,
                                                         const float* residual, int act, int f16, float* c_staged, float* c_tiled);
 
+/* test hook: the blocks that a product of the layer-list decoders is cut into (csrc/nn/tk_gemm_image.h): rows x K against N x K, operands f32 or bf16;
+ * swiglu: N = gate and up rows together; experts > 0: every row goes to `top` of them; max_slabs: parts of k at most.  form = rows, columns and LDS
+ * stages of a block, parts of k; stages = 0: the kernel for few rows.  No GPU involved. */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,52 @@
+"""Which blocks a matrix product is cut into: the choice is made on the host, so it is held here; the kernels themselves are in the GPU tests."""
+import ctypes as C
+
+import pytest
+
+import trackiellm_amd as tk
+
+
+def image_form(f32, rows, n, k, swiglu=0, experts=0, top=0, slabs=1):
+    form = (C.c_int * 4)()
+    assert tk.lib().tk_mi355x_gemm_image_form(f32, rows, n, k, swiglu, experts, top, slabs, form) == 0
+    return tuple(form)
+
+
+@pytest.mark.parametrize("rows,n,k,swiglu,slabs,want", [
+    (2047, 7552, 4096, 0, 1, (256, 256, 2, 1)),
+    (1303, 7552, 4096, 0, 1, (128, 128, 2, 1)),   # 256 x 256: 180 blocks, one round of 940 us; three rounds of a quarter each: 715
+    (1303, 6192, 2080, 0, 1, (128, 64, 3, 1)),    # 318 us, 256 x 256 480
+    (2047, 3072, 2048, 0, 1, (128, 64, 3, 1)),    # 202 us, 256 x 128 257
+    (900, 4096, 14336, 0, 1, (128, 128, 4, 1)),
+    (900, 28672, 4096, 1, 1, (128, 128, 2, 1)),   # 1656 us, 256 x 256 1886
+    (256, 3072, 2048, 0, 8, (128, 128, 4, 5)),    # in parts of k: 36 us in four, 42 whole
+])
+def test_blocks_of_float32_products(rows, n, k, swiglu, slabs, want):
+    """the choice is that of measured times: an f32 MFMA takes sixteen times as long as a bf16 one for the same k, so rounds half empty cost more than anything else"""
+    assert image_form(1, rows, n, k, swiglu, slabs=slabs) == want
+
+
+@pytest.mark.parametrize("rows,n,k,swiglu,want", [
+    (1750, 28672, 4096, 1, (256, 256, 2, 1)), (2047, 4096, 14336, 0, (256, 128, 3, 1)), (1100, 28672, 4096, 1, (128, 128, 2, 1)),
+    (1750, 2048, 8192, 0, (128, 128, 4, 1)), (600, 2048, 8192, 0, (128, 64, 3, 1)), (200, 4096, 14336, 0, (128, 32, 4, 1)), (64, 4096, 4096, 0, (64, 0, 0, 1)),
+])
+def test_blocks_of_bf16_products(rows, n, k, swiglu, want):
+    assert image_form(0, rows, n, k, swiglu) == want
+
+
+@pytest.mark.parametrize("f32,rows,n,k,swiglu,experts,top,want", [
+    (1, 2047, 1024, 2048, 0, 8, 2, (128, 32, 4, 1)),    # 182 us, 128 x 128 242
+    (1, 1200, 512, 256, 1, 6, 3, (128, 64, 3, 1)),      # 31 blocks of 34 are live: 248 of 272 workgroups, one round.  13.5 us, 128 x 128 20.5
+    (0, 1200, 1024, 2048, 0, 8, 2, (128, 128, 4, 1)),
+    (0, 2047, 2048, 2048, 1, 64, 8, (128, 128, 2, 1)),
+])
+def test_blocks_of_experts(f32, rows, n, k, swiglu, experts, top, want):
+    """row blocks come from the router; how many there will be is estimated"""
+    assert image_form(f32, rows, n, k, swiglu, experts, top) == want
+
+
+def test_block_hooks_refuse_bad_sizes():
+    f = (C.c_int * 4)()
+    for args in ((0, 0, 16, 64, 0, 0, 0, 1), (0, 8, 0, 64, 0, 0, 0, 1), (0, 8, 16, 0, 0, 0, 0, 1), (0, 8, 16, 64, 0, 4, 0, 1), (0, 8, 16, 64, 0, 4, 5, 1)):
+        assert tk.lib().tk_mi355x_gemm_image_form(*args, f) != 0
+    assert tk.lib().tk_mi355x_gemm_image_form(0, 8, 16, 64, 0, 0, 0, 1, None) != 0

@@ -12,6 +12,7 @@
 
 #include "../vision/tk_vision_engine.h"
 #include "tk/tk_rocm_hal.h"
+#include "../nn/tk_gemm_image.h"
 #include "../nn/tk_gemm_tiled.h"
 #include "../nn/tk_nn_kernels.h"
 
@@ -170,6 +171,16 @@ tk_error_code_t tk_mi355x_gemm_pair(int device, int M, int N, int K, const float
     void* ptrs[] = {da, dw, db, dr, dc, dimg, dwh, dt};
     for (void* q : ptrs) if (q) (void)hipFree(q);
     return ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
+}
+
+tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]) {
+    if (rows <= 0 || N <= 0 || K <= 0 || experts < 0 || (experts > 0 && (top < 1 || top > experts)) || !form) return TK_ERROR_INVALID_ARGUMENT;
+    const int to = swiglu ? 32 : 16;
+    TkImgGemm g{};
+    g.type = f32 ? TK_IMG_F32 : TK_IMG_BF16; g.K = tk_img_pad_k(g.type, K); g.N = (N + to - 1) / to * to; g.n_valid = N; g.nrows = rows; g.swiglu = swiglu != 0; g.max_slabs = max_slabs;
+    if (experts) tk_img_expert_blocks(rows, top, experts, &g);
+    tk_gemm_image_form(g, form);
+    return TK_SUCCESS;
 }
 
 tk_error_code_t tk_kernels_depth_to_point_cloud(const tk_depth_to_points_params_t* p, tk_hip_stream_t stream) {

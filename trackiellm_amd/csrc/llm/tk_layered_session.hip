@@ -313,16 +313,13 @@ void TkLayeredSession::enqueue_moe(const TkLayerSpec& s, const TkLayeredLayer& L
     g.type = type; g.w = L.router.img; g.a = img_x_; g.K = L.router.K; g.N = L.router.N; g.nrows = nrows;
     g.out = router_; g.ldc = L.router.N; g.n_valid = f.experts;
     gemm(g);
-    const int64_t assign = (int64_t)nrows * f.top;
-    const int64_t per = assign / f.experts;
-    const int bt = per <= 16 ? 1 : per <= 32 ? 2 : per <= 64 ? 4 : 8;
-    tk_launch_moe_select(router_, L.router.N, f.experts, f.top, f.groups, f.keep, nrows, bt, moe_, stream);
-    tk_launch_moe_gather(img_x_, img_gather_, xkt, f.top, nrows, moe_, stream);
     TkImgGemm u{};
+    tk_img_expert_blocks(nrows, f.top, f.experts, &u);
+    tk_launch_moe_select(router_, L.router.N, f.experts, f.top, f.groups, f.keep, nrows, u.block_tiles, moe_, stream);
+    tk_launch_moe_gather(img_x_, img_gather_, xkt, f.top, nrows, moe_, stream);
     u.type = type; u.w = L.gate_up.img; u.a = img_gather_; u.K = L.gate_up.K; u.N = L.gate_up.N;
     u.swiglu = 1; u.act_img = img_ff_; u.act_ktiles = fkt; u.act_valid = f.ff;
-    u.blocks = moe_.blocks; u.n_blocks = moe_.n_blocks; u.block_tiles = bt; u.group_bytes = L.gate_up.bytes;
-    u.max_blocks = (int)(std::min<int64_t>(f.experts, assign) + assign / (16 * bt));
+    u.blocks = moe_.blocks; u.n_blocks = moe_.n_blocks; u.group_bytes = L.gate_up.bytes;
     gemm(u);
     TkImgGemm d = u;
     d.w = L.down.img; d.a = img_ff_; d.K = L.down.K; d.N = L.down.N; d.swiglu = 0; d.act_img = nullptr; d.group_bytes = L.down.bytes;

@@ -57,11 +57,24 @@ struct TkImgGemm {
     const TkImgBlock* blocks;
     const int32_t* n_blocks;
     int max_blocks, block_tiles;
+    int live_blocks;     /* how many are expected to be live (0: all of max_blocks); for the choice of a form only */
     size_t group_bytes;  /* between the weight images of two groups */
 };
 
 /* nullptr, or why the arguments are refused (nothing is launched then) */
 const char* tk_launch_gemm_image(const TkImgGemm& g, hipStream_t s, int* slabs = nullptr);
+
+/* rows, columns and LDS stages of the blocks that a launch with these sizes takes, and its k parts; stages = 0: the skinny kernel.  Reads no pointer. */
+void tk_gemm_image_form(const TkImgGemm& g, int form[4]);
+
+/* row blocks of `rows` rows sent to `top` of `experts` each: tiles of a block, the most there can be, and how many to expect (an expert's last block is half
+ * the time there) */
+static inline void tk_img_expert_blocks(int64_t rows, int top, int experts, TkImgGemm* g) {
+    const int64_t assign = rows * top, per = assign / experts, used = experts < assign ? experts : assign;
+    g->block_tiles = per <= 16 ? 1 : per <= 32 ? 2 : per <= 64 ? 4 : 8;
+    g->max_blocks = (int)(used + assign / (16 * g->block_tiles));
+    g->live_blocks = g->max_blocks - (int)(used / 2);
+}
 
 /* opts the kernels into their dynamic LDS on the calling thread's current device; nullptr or an error string.  Idempotent, thread-safe. */
 const char* tk_gemm_image_prepare_device();

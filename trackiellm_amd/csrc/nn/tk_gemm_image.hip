@@ -279,35 +279,52 @@ __global__ void k_put_image(const void* src, int src_f32, int64_t N, int64_t K, 
     tk_img_put(img, row, (int)k0 + k, ktiles, v);
 }
 
-/* The forms of the wide kernel and what they cost: rounds of workgroups x (their start and end + k x time per k), fitted to products of 100 .. 2047 rows
- * whose weights come from memory (within ~15 %).  Large blocks where they fill the chip once or several times, smaller ones where larger would leave CUs
- * idle.  Of forms that run two to a CU a last round of at most 256 runs one to a CU. */
-struct WideForm { int mb, nb, per_cu; float start, k, start2, k2; }; /* tiles; us, ns per k of a round with one workgroup per CU, and with two */
-constexpr WideForm wide_forms[] = {
-    {16, 16, 1, 22.0f, 17.5f, 0.0f, 0.0f}, /* 1750 x 28672 x 4096: 372 us (next best 379) */
-    {16, 8, 1, 8.0f, 12.0f, 0.0f, 0.0f},   /* 2047 x 4096 x 14336: 182 us (242) */
-    {8, 8, 2, 6.0f, 11.8f, 8.0f, 15.0f},   /* 1100 x 28672 x 4096: 248 us (271) */
-    {8, 8, 1, 10.0f, 7.0f, 0.0f, 0.0f},    /* four stages instead of two.  1750 x 2048 x 8192: 68 us (93) */
-    {8, 4, 2, 7.0f, 5.5f, 8.0f, 9.6f},     /* 600 x 2048 x 8192: 50 us (64) */
-    {8, 2, 2, 6.0f, 3.9f, 6.0f, 7.2f},     /* 200 x 4096 x 14336: 61 us (84) */
+/* The forms of the wide kernel and what they cost, fitted to products of 100 .. 2047 rows whose weights come from memory.  Large blocks where they fill the
+ * chip once or several times, smaller ones where larger would leave CUs idle.
+ * bf16 (within ~15 %): rounds of workgroups x (their start and end + k x time per k).  Of forms that run two to a CU a last round of at most 256 runs one
+ * to a CU.
+ * f32 (within 11 %): four MFMAs for 16 k where bf16 takes one for 32, so the matrix pipe is all there is, two workgroups of a CU take twice the time, and
+ * what counts is the blocks of the fullest CU: the first one's start and end once, + per further one, + k x time per k each. */
+struct WideForm {
+    int mb, nb, ring; /* tiles, stages */
+    int per_cu; float start, k, start2, k2;  /* bf16: us, ns per k of a round with one workgroup per CU, and with two */
+    float f32_start, f32_more, f32_k;        /* f32 */
 };
+constexpr WideForm wide_forms[] = {
+    /* bf16 1750 x 28672 x 4096: 372 us (next best 379); f32 2047 x 7552 x 4096: 942 us (947) */
+    {16, 16, 2, 1, 22.0f, 17.5f, 0.0f, 0.0f, 16.0f, 15.0f, 221.3f},
+    /* bf16 2047 x 4096 x 14336: 182 us (242); f32 256 x 16384 x 2048: as the next two, 0.25 us */
+    {16, 8, 3, 1, 8.0f, 12.0f, 0.0f, 0.0f, 12.0f, 6.0f, 115.7f},
+    /* bf16 1100 x 28672 x 4096: 248 us (271); f32 1303 x 7552 x 4096: 715 us (256 x 256: 940, which bf16's constants would take) */
+    {8, 8, 2, 2, 6.0f, 11.8f, 8.0f, 15.0f, 9.5f, 0.3f, 58.7f},
+    /* bf16 1750 x 2048 x 8192: 68 us (93); f32 900 x 4096 x 14336: 846 us (873) */
+    {8, 8, 4, 1, 10.0f, 7.0f, 0.0f, 0.0f, 9.5f, 4.0f, 58.6f},
+    /* bf16 600 x 2048 x 8192: 50 us (64); f32 2047 x 3072 x 2048: 202 us (128 x 128: 251) */
+    {8, 4, 3, 2, 7.0f, 5.5f, 8.0f, 9.6f, 8.5f, 0.5f, 31.2f},
+    /* bf16 200 x 4096 x 14336: 61 us (84); f32 1303 x 2048 x 8192: 422 us (128 x 128: 487) */
+    {8, 2, 4, 2, 6.0f, 3.9f, 6.0f, 7.2f, 7.5f, 1.0f, 17.1f},
+};
+float wide_us(const WideForm& w, bool f32, int64_t blocks, float k /* thousands */) {
+    if (f32) return w.f32_start + (float)((blocks + 255) / 256 - 1) * w.f32_more + (float)((blocks + 255) / 256) * w.f32_k * k;
+    const float one = w.start + w.k * k, two = w.start2 + w.k2 * k;
+    if (w.per_cu == 1) return (float)((blocks + 255) / 256) * one;
+    return (float)(blocks / 512) * two + (blocks % 512 == 0 ? 0.0f : blocks % 512 <= 256 ? one : two);
+}
 struct WidePick { int form, ks; };
 WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
     const int ntiles = g.N / 16, mtiles = (g.nrows + 15) / 16;
-    /* k in parts whose sums the consumer adds, at least 512 each: it reads, and this kernel writes, a slab more per part */
+    /* k in parts whose sums the consumer adds, at least 16 k tiles each: it reads, and this kernel writes, a slab more per part */
     const int kt = tk_img_kt(g.type), most = swiglu || grouped || g.max_slabs < 1 ? 1 : g.max_slabs;
     const float slab_us = (float)((double)g.nrows * g.n_valid * 8e-6 / 5.0);
+    const int row_blocks = g.live_blocks > 0 && g.live_blocks < g.max_blocks ? g.live_blocks : g.max_blocks;
     WidePick best{2, 1};
     float least = 1e30f;
     for (int f = 0; f < (int)(sizeof wide_forms / sizeof wide_forms[0]); ++f) {
         const WideForm& w = wide_forms[f];
         if ((grouped && w.mb > 8) || (swiglu && w.nb < 4)) continue;
         for (int ks = 1; ks <= most && (ks == 1 || g.K / kt / ks >= 16); ++ks) {
-            const int64_t blocks = (int64_t)(grouped ? g.max_blocks : (mtiles + w.mb - 1) / w.mb) * ((ntiles + w.nb - 1) / w.nb) * ks;
-            const float k = 1e-3f * (float)g.K / (float)ks, one = w.start + w.k * k, two = w.start2 + w.k2 * k;
-            float us = (float)(ks - 1) * slab_us;
-            if (w.per_cu == 1) us += (float)((blocks + 255) / 256) * one;
-            else us += (float)(blocks / 512) * two + (blocks % 512 == 0 ? 0.0f : blocks % 512 <= 256 ? one : two);
+            const int64_t blocks = (int64_t)(grouped ? row_blocks : (mtiles + w.mb - 1) / w.mb) * ((ntiles + w.nb - 1) / w.nb) * ks;
+            const float us = (float)(ks - 1) * slab_us + wide_us(w, g.type == TK_IMG_F32, blocks, 1e-3f * (float)g.K / (float)ks);
             if (us < least) { least = us; best = WidePick{f, ks}; }
         }
     }
@@ -349,6 +366,15 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
 }
 
 } // namespace
+
+void tk_gemm_image_form(const TkImgGemm& g, int form[4]) {
+    const bool grouped = g.max_blocks > 0;
+    form[0] = 64; form[1] = form[2] = 0; form[3] = 1;
+    if ((grouped ? g.block_tiles : (g.nrows + 15) / 16) <= 4) return;
+    const WidePick p = pick_wide(g, g.swiglu != 0, grouped);
+    const WideForm& w = wide_forms[p.form];
+    form[0] = 16 * w.mb; form[1] = 16 * w.nb; form[2] = w.ring; form[3] = p.ks;
+}
 
 const char* tk_launch_gemm_image(const TkImgGemm& g, hipStream_t s, int* slabs) {
     if (slabs) *slabs = 1;
