@@ -19,7 +19,8 @@ def image_form(f32, rows, n, k, swiglu=0, experts=0, top=0, slabs=1):
     (2047, 3072, 2048, 0, 1, (128, 64, 3, 1)),    # 202 us, 256 x 128 257
     (900, 4096, 14336, 0, 1, (128, 128, 4, 1)),
     (900, 28672, 4096, 1, 1, (128, 128, 2, 1)),   # 1656 us, 256 x 256 1886
-    (256, 3072, 2048, 0, 8, (128, 128, 4, 5)),    # in parts of k: 36 us in four, 42 whole
+    (256, 3072, 2048, 0, 8, (128, 64, 3, 8)),     # as many parts as 128 x 128 blocks leave room for: the error, not the time
+    (900, 2048, 8192, 0, 2, (128, 128, 4, 2)),
 ])
 def test_blocks_of_float32_products(rows, n, k, swiglu, slabs, want):
     """the choice is that of measured times: an f32 MFMA takes sixteen times as long as a bf16 one for the same k, so rounds half empty cost more than anything else"""
