@@ -227,6 +227,20 @@ def test_runs_in_chunks_beside_short_ones(gpu, tmp_path, dim, vdim, steep):
         assert U.rel_rms(np.array(rows), c.want(p)[0], 0.9 if steep else 1.0) < F32
 
 
+def test_sessions_take_memory_for_the_chunks_they_can_have(gpu, tmp_path):
+    """256 sequences of one position: a pass has 256 rows, of which 6 runs of 40 and more can be, 22 chunks at most"""
+    import torch
+    heads, dim = 32, 130
+    c = Case(gpu, tmp_path, config(32, 40, [layer(attention(1, 1, 8, 8, 4, 7, 1), delta(heads, 1, dim, 4, 2), None)]))
+    c.session("float32", 1, 1).close()
+    free = torch.cuda.mem_get_info()[0]
+    s = c.session("float32", 256, 1)
+    taken = free - torch.cuda.mem_get_info()[0]
+    s.close()
+    state, chunk = 2 * 256 * heads * dim * 4 * 4, heads * (49 * 256 + 512) * 4
+    assert taken < state + 22 * chunk + (32 << 20)   # a chunk for every sequence would be 427 MB
+
+
 @pytest.mark.parametrize("at", [0, 15, 16, 37, 57])
 @pytest.mark.parametrize("operand", ["v", "k", "q", "a1"])
 def test_non_finite_values_stay_with_their_position(gpu, tmp_path, operand, at):

@@ -875,11 +875,9 @@ __global__ __launch_bounds__(256) void k_delta_scan(TkDeltaArgs d, TkPassTab t, 
  * Token by token a step is one dependent chain of ~650 cycles whatever the chip has free (558 us for 2047 tokens x 16 heads of 128 x 128); here what
  * does not depend on the state is done for all chunks at once (k_delta_chunk, 31 us), and the chain is ~2000 cycles for 16 tokens (k_delta_chain, 108 us).
  * Its error against 64 bits is that of the token by token form (2.8e-6 of the logits of float32 models, 2.7e-6). */
-constexpr int DC = 16; /* tokens of a chunk */
-constexpr size_t delta_slot_floats(int dp) { return (size_t)(3 * DC + 1) * dp + 2 * DC * DC; }
+constexpr int DC = TK_DELTA_CHUNK;
+constexpr size_t delta_chunk_floats(int dp) { return (size_t)(3 * DC + 1) * dp + 2 * DC * DC; }
 static int delta_pad(int dim) { return dim <= 64 ? 64 : dim <= 128 ? 128 : 256; }
-/* a segment's chunks are consecutive slots; room for every segment's last, partly filled one */
-__device__ __forceinline__ int delta_slot0(int row0, int seg) { return row0 / DC + seg; }
 
 /* lane i of every four: its elements 0 .. 3 -> element i of the lanes 0 .. 3 */
 __device__ __forceinline__ tk_v4f quad_transpose(tk_v4f v) {
@@ -897,13 +895,11 @@ template <int DP>
 __global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t, int nseg) {
     constexpr int PE = DP / 32; /* key rows of a thread in the pair products */
     __shared__ __attribute__((aligned(16))) float lq[DC][DP], lk[DC][DP], lg[DC][DP], L[DC][DC], B[DC][DC], lb[DC];
-    const int tid = threadIdx.x, slot = blockIdx.y, h = blockIdx.x, kvh = h / (d.heads / d.kv_heads);
-    const int seg = __syncthreads_count(tid < nseg && delta_slot0(t.seg_row0[tid < nseg ? tid : 0], tid) <= slot) - 1;
-    if (seg < 0) return;
-    const int t0 = (slot - delta_slot0(t.seg_row0[seg], seg)) * DC, n = t.seg_n[seg];
-    if (t0 >= n || n < TK_DELTA_CHUNKED) return;
+    const int tid = threadIdx.x, chunk = blockIdx.y, h = blockIdx.x, kvh = h / (d.heads / d.kv_heads);
+    const int seg = __syncthreads_count(tid < nseg && t.seg_chunk0[tid < nseg ? tid : 0] <= chunk) - 1; /* the last one that begins here or before: it has chunks */
+    const int t0 = (chunk - t.seg_chunk0[seg]) * DC, n = t.seg_n[seg];
     const int m = n - t0 < DC ? n - t0 : DC, row0 = t.seg_row0[seg] + t0;
-    float* const w = d.chunks + ((size_t)slot * d.heads + h) * delta_slot_floats(DP);
+    float* const w = d.chunks + ((size_t)chunk * d.heads + h) * delta_chunk_floats(DP);
     float *const wq = w + DC * DP, *const wk = wq + DC * DP, *const wg = wk + DC * DP, *const wt = wg + DP, *const wb = wt + DC * DC;
 #pragma unroll
     for (int i = 0; i < DC * DP / 256; ++i) {
@@ -1018,8 +1014,8 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
             S[i][r] = in >= 0 && live && e < d.dim ? d.state[(((size_t)in * d.heads + h) * d.dim + e) * vp + col] : 0.0f;
         }
     struct Ops { tk_v4f w[NT], q[NT], k[NT], g[NT]; float t, b, v; } ops[AHEAD + 1];
-    const size_t step = (size_t)d.heads * delta_slot_floats(DP);
-    const float* const base = d.chunks + ((size_t)delta_slot0(row0, seg) * d.heads + h) * delta_slot_floats(DP);
+    const size_t step = (size_t)d.heads * delta_chunk_floats(DP);
+    const float* const base = d.chunks + ((size_t)t.seg_chunk0[seg] * d.heads + h) * delta_chunk_floats(DP);
     auto fetch = [&](Ops& o, int c) {
         const float* p = base + (size_t)c * step;
         const int tile = wave * NT;
@@ -1883,11 +1879,11 @@ bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, 
     return true;
 }
 
-size_t tk_delta_chunk_floats(int heads, int dim, int rows, int segments) { return (size_t)(rows / DC + segments) * heads * delta_slot_floats(delta_pad(dim)); }
+size_t tk_delta_chunk_floats(int heads, int dim, int rows) { return (size_t)(rows / DC + rows / TK_DELTA_CHUNKED) * heads * delta_chunk_floats(delta_pad(dim)); }
 
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int longest, int nrows, hipStream_t s) {
-    if (longest >= TK_DELTA_CHUNKED) {
-        const dim3 chunks(d.heads, nrows / DC + n_segments), chain(d.heads, (d.vdim + 15) / 16, n_segments); /* heads first: a head's workgroups share an XCD's L2 */
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_chunks, int nrows, hipStream_t s) {
+    if (n_chunks > 0) {
+        const dim3 chunks(d.heads, n_chunks), chain(d.heads, (d.vdim + 15) / 16, n_segments); /* heads first: a head's workgroups share an XCD's L2 */
 #define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_segments); \
         hipLaunchKernelGGL((k_delta_chain<DP, false>), chain, dim3(256), 0, s, d, t); hipLaunchKernelGGL((k_delta_chain<DP, true>), chain, dim3(256), 0, s, d, t); } while (0)
         switch (delta_pad(d.dim)) {
