@@ -57,7 +57,8 @@ def test_whisper_tiny_en_full_size_encoder(gpu):
     (1537, 64, 1, 1, 2),     # one key more; a head in four parts
     (800, 288, 2, 1, 18),    # heads of 144: nine tiles for eight waves
     (520, 512, 2, 2, 2),     # heads of 256
-    (2048, 128, 1, 1, 2), (2049, 64, 2, 1, 2),   # the most keys, and the general form beyond
+    (2048, 128, 1, 1, 2), (2049, 64, 2, 1, 2),   # the most keys whose scores are held, and scores read twice beyond
+    (3000, 128, 2, 3, 18), (4097, 48, 1, 1, 2), (12288, 16, 1, 1, 2), (12289, 16, 1, 1, 2),   # a second and third round of scores; the most keys, and the general form beyond
     (40, 528, 33, 1, 2), (40, 1280, 80, 2, 2), (40, 1296, 81, 1, 2),   # norms: rows in five registers a thread, the longest of these, read again
 ])
 def test_decoder_attention_over_contexts_and_heads(gpu, ctx, state, heads, clips, steps):

@@ -95,11 +95,13 @@ __global__ __launch_bounds__(256) void k_logmel_clamp(float* mel, int per_b, con
  * Scores: a key per lane.  K comes by LDS-DMA, 16 floats of each key per slot of 4 KiB (rows 64 bytes apart, their 16-byte units swapped by
  * row so that the 64 lanes' reads spread over all banks).
  * Cross attention of one sequence (6 heads, 1500 keys of 64): 18 us (4 + 14); with one workgroup of 4 waves per head, whose lanes read whole rows of K
- * (64 lines per load) and whose chain ran on one vector unit: 49 us.  32 sequences: 42 us against 77. */
+ * (64 lines per load) and whose chain ran on one vector unit: 49 us.  32 sequences: 42 us against 77.  Contexts beyond 2048 keys read their
+ * scores twice and keep the weights in LDS only: a decoder step of four layers over 6000 keys, 16 sequences: 0.65 ms, 1.30 in three launches. */
 #define TK_AT1_NW 8             /* waves */
 #define TK_AT1_RING (16 * 1024) /* bytes per wave: 64 keys of K in four slots of 16 floats */
 #define TK_AT1_SELF 512         /* longest context whose scores are made in the same kernel: 64 keys per wave */
-#define TK_AT1_MAX_KEYS 2048    /* 8 scores per thread */
+#define TK_AT1_HELD 2048        /* longest context whose scores stay in registers: 8 per thread */
+#define TK_AT1_MAX_KEYS 12288   /* a round of V and the weights in the LDS */
 typedef float at1_f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void at1_wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0F70); } /* s_waitcnt vmcnt(0) alone */
 __device__ __forceinline__ void at1_dma(const float* src, uint8_t* lds) {
@@ -158,7 +160,9 @@ __host__ __device__ constexpr int at1_round_blocks(bool self, int C) { return at
 /* place of key k's weight in LDS: 16 keys' weights in the order in which four MFMAs take them, so that a lane's four are one read */
 __device__ __forceinline__ int at1_place(int k) { return (k & ~15) | (k & 3) << 2 | (k >> 2 & 3); }
 
-template <bool SELF>
+/* where the scores are: made here; read from memory once and held; read from memory twice */
+enum { AT1_SELF, AT1_HELD, AT1_LONG };
+template <int FORM>
 __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, const float* k, const float* v, const float* scores, int pitch, float* out, int Tk,
                                                            int64_t q_bstride, int64_t kv_bstride, int d, int hd, int split, float scale, int sc_at /* bytes */,
                                                            float* img /* optional: out also as the tiled GEMM's operand image [B rows][K = d] */) {
@@ -173,13 +177,15 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
     const float* vp = v + (int64_t)b * kv_bstride + (int64_t)h * hd + part * C;
 
     /* 256 threads hold the scores: thread t those of keys t, t + 256, ...: the canonical partials */
-    constexpr int NS = SELF ? TK_AT1_SELF / 256 : TK_AT1_MAX_KEYS / 256;
+    constexpr bool SELF = FORM == AT1_SELF;
+    constexpr int NS = SELF ? TK_AT1_SELF / 256 : TK_AT1_HELD / 256;
     float e[NS];
-    if (!SELF) {
-        const float* sp = scores + ((int64_t)b * (gridDim.x / split) + h) * pitch;
+    const float* sp = scores + ((int64_t)b * (gridDim.x / split) + h) * pitch;
+    auto load_scores = [&](int k0) {
 #pragma unroll
-        for (int j = 0; j < NS; ++j) { const int t = (t0 & 255) + 256 * j; e[j] = sp[t < Tk ? t : Tk - 1]; }
-    }
+        for (int j = 0; j < NS; ++j) { const int t = k0 + (t0 & 255) + 256 * j; e[j] = sp[t < Tk ? t : Tk - 1]; }
+    };
+    if (FORM == AT1_HELD) load_scores(0);
     /* V in rounds of 16 * rb keys.  A thread's task: keys 16 kb + 4 t + g, t = 0 .. 3, of four neighbouring columns.  LDS: [block of 16 keys]
      * [16 columns][g][column ^ g][t], 1 KiB a tile (the XOR spreads the four g's writes over the banks) */
     constexpr int NT = at1_tasks(SELF);
@@ -227,26 +233,41 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
         for (int j = 0; j < NS; ++j) { const int t = (t0 & 255) + 256 * j; e[j] = sc[t < Tk ? t : Tk - 1]; }
     }
     const int tk = t0 & 255; /* threads 256 .. 511 do the same again: no wave waits for another's branch */
+    const int rounds = FORM == AT1_LONG ? (Tk + TK_AT1_HELD - 1) / TK_AT1_HELD * TK_AT1_HELD : 1;
     float m = -INFINITY;
+    for (int k0 = 0; k0 < rounds; k0 += TK_AT1_HELD) {
+        if (FORM == AT1_LONG) load_scores(k0);
 #pragma unroll
-    for (int j = 0; j < NS; ++j)
-        if (tk + 256 * j < Tk) m = tk_fmaxf(m, e[j]);
+        for (int j = 0; j < NS; ++j)
+            if (k0 + tk + 256 * j < Tk) m = tk_fmaxf(m, e[j]);
+    }
     for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, __shfl_xor(m, s, 64));
     if (lane == 0) red[wave & 3] = m;
     __syncthreads();
     m = tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
     float s = 0.0f;
+    for (int k0 = 0; k0 < rounds; k0 += TK_AT1_HELD) {
+        if (FORM == AT1_LONG) load_scores(k0);
 #pragma unroll
-    for (int j = 0; j < NS; ++j)
-        if (tk + 256 * j < Tk) { e[j] = tk_expf(e[j] - m); s = s + e[j]; }
+        for (int j = 0; j < NS; ++j)
+            if (k0 + tk + 256 * j < Tk) {
+                e[j] = tk_expf(e[j] - m);
+                s = s + e[j];
+                if (FORM == AT1_LONG && wave < 4) sc[at1_place(k0 + tk + 256 * j)] = e[j];
+            }
+    }
     for (int w = 32; w >= 1; w >>= 1) s = s + __shfl_xor(s, w, 64);
     if (lane == 0) red[4 + (wave & 3)] = s;
     __syncthreads();
     const float tot = ((red[4] + red[5]) + red[6]) + red[7];
     if (wave < 4) {
+        if (FORM == AT1_LONG) {
+            for (int t = t0; t < Tk; t += 256) sc[at1_place(t)] = tk_divf(sc[at1_place(t)], tot); /* its own */
+        } else {
 #pragma unroll
-        for (int j = 0; j < NS; ++j)
-            if (t0 + 256 * j < Tk) sc[at1_place(t0 + 256 * j)] = tk_divf(e[j], tot);
+            for (int j = 0; j < NS; ++j)
+                if (t0 + 256 * j < Tk) sc[at1_place(t0 + 256 * j)] = tk_divf(e[j], tot);
+        }
         if (t0 < (-Tk & 15)) sc[at1_place(Tk + t0)] = 0.0f;
     }
 
@@ -318,8 +339,9 @@ static int at1_buffer(int Tk, int C) {
 }
 static bool at1_prepare_device() {
     const int most = 160 * 1024;
-    return hipFuncSetAttribute((const void*)k_attend1<true>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
-           hipFuncSetAttribute((const void*)k_attend1<false>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+    return hipFuncSetAttribute((const void*)k_attend1<AT1_SELF>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+           hipFuncSetAttribute((const void*)k_attend1<AT1_HELD>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
+           hipFuncSetAttribute((const void*)k_attend1<AT1_LONG>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
            hipFuncSetAttribute((const void*)k_attend1_scores, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess;
 }
 /* scores: scratch [B][nh][pitch] */
@@ -331,12 +353,14 @@ static bool at1_launch(const float* q, const float* k, const float* v, float* sc
     while (hd % (32 * split) == 0 && 2 * split * nh * B <= 256) split *= 2;
     const dim3 grid(nh * split, B), block(64 * TK_AT1_NW);
     const int sc_at = at1_buffer(Tk, hd / split);
-    const size_t lds = (size_t)sc_at + (size_t)(((Tk + 15) & ~15) + hd + 8) * 4; /* <= 128 KiB + 3 KiB, 96 KiB + 10 KiB */
+    const size_t lds = (size_t)sc_at + (size_t)(((Tk + 15) & ~15) + hd + 8) * 4; /* <= 128 KiB + 3 KiB, 96 KiB + 10 KiB, 96 KiB + 50 KiB */
     if (Tk <= TK_AT1_SELF) {
-        hipLaunchKernelGGL((k_attend1<true>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img);
+        hipLaunchKernelGGL((k_attend1<AT1_SELF>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img);
     } else {
         hipLaunchKernelGGL(k_attend1_scores, dim3(((Tk + 63) / 64 + 3) / 4, nh, B), dim3(256), 4 * TK_AT1_RING + (size_t)hd * 4, s, q, k, scores, Tk, pitch, q_bstride, kv_bstride, d, hd, scale);
-        hipLaunchKernelGGL((k_attend1<false>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img);
+#define TK_AT1(FORM) hipLaunchKernelGGL((k_attend1<FORM>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img)
+        if (Tk <= TK_AT1_HELD) TK_AT1(AT1_HELD); else TK_AT1(AT1_LONG);
+#undef TK_AT1
     }
     return true;
 }
