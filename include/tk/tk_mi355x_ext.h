@@ -249,6 +249,13 @@ TK_API const char* tk_mi355x_llm_runner_tool_call_text(struct tk_llm_runner_s* r
  * act: 0 none, 1 SiLU, 2 GELU, 3 sigmoid. */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_pair(int device, int M, int N, int K, const float* a, const float* w, const float* bias,
                                                         const float* residual, int act, int f16, float* c_staged, float* c_tiled);
+/* test hook for the kernels behind the staged one: C[M][N] = act(A W^T + bias) + residual, A [M][lda], W [N][ldb], by the given form (0 .. 5: blocks of
+ * 16 x 16 x 4 MFMAs; 6 .. 8: 128 rows x 32, 64, 96 columns; 9: 128 x 128; 10: 64 x 64).  conv (may be NULL): A is a convolution's input [pixels][ldx],
+ * conv = {C, H, W, ldx, kernel, stride, padding, Ho, Wo}, M = images Ho Wo, K = kernel^2 C, lda unused. */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_f32(int device, int form, int M, int N, int K, int lda, int ldb, const float* a, const float* w, const float* bias,
+                                                       const float* residual, int act, const int conv[9], float* c);
+/* the form that such a product takes by itself, `batch` of them side by side, and the rows and columns of its block.  No GPU involved. */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_f32_form(int M, int N, int K, int lda, int ldb, int batch, const int conv[9], int* form, int block[2]);
 
 /* test hook: the blocks that a product of the layer-list decoders is cut into (csrc/nn/tk_gemm_image.h): rows x K against N x K, operands f32 or bf16;
  * swiglu: N = gate and up rows together; experts > 0: every row goes to `top` of them; max_slabs: parts of k at most.  form = rows, columns and LDS

@@ -46,6 +46,38 @@ def test_blocks_of_experts(f32, rows, n, k, swiglu, experts, top, want):
     assert image_form(f32, rows, n, k, swiglu, experts, top) == want
 
 
+def f32_form(m, n, k, pad=0, batch=1, conv=None):
+    form, block = C.c_int(), (C.c_int * 2)()
+    ld = k + pad
+    rc = tk.lib().tk_mi355x_gemm_f32_form(m, n, k, ld, k if conv else ld, batch, conv and (C.c_int * 9)(*conv), C.byref(form), block)
+    assert rc == 0
+    return form.value, tuple(block)
+
+
+def conv3(c, side, stride, images):
+    out = (side - 1) // stride + 1
+    return images * out * out, 9 * c, (c, side, side, c, 3, stride, 1, out, out)
+
+
+@pytest.mark.parametrize("m,n,k,pad,batch,block", [
+    # side by side, short or unaligned: 0.55 - 0.75 of the speed where the 16 x 16 x 4 forms took them
+    (255, 201, 400, 0, 48, (64, 64)), (1500, 80, 27, 1, 48, (64, 64)), (100, 1500, 64, 0, 48, (64, 64)), (102400, 80, 64, 0, 1, (128, 96)), (102400, 80, 64, 1, 1, (128, 96)),
+    (25600, 96, 27, 1, 1, (128, 128)), (1500, 16, 27, 1, 1, (128, 32)), (6400, 384, 27, 1, 1, (128, 128)), (255, 1500, 64, 0, 48, (64, 64)),
+    (400, 256, 1152, 0, 1, (32, 32)), (1, 1, 4608, 0, 1, (32, 32)), (1500, 201, 1152, 1, 6, (64, 80)), (33, 384, 400, 0, 6, (32, 32)),
+])
+def test_blocks_of_exact_products(m, n, k, pad, batch, block):
+    assert f32_form(m, n, k, pad, batch)[1] == block
+
+
+@pytest.mark.parametrize("c,side,stride,images,n,block", [
+    (16, 160, 1, 1, 16, (64, 16)), (128, 20, 1, 1, 128, (32, 32)), (64, 80, 1, 1, 80, (64, 16)), (512, 112, 1, 1, 64, (64, 32)), (32, 160, 2, 32, 64, (128, 64)), (80, 80, 1, 32, 80, (64, 80)),
+    (64, 40, 1, 8, 128, (64, 64)), (256, 20, 1, 32, 64, (64, 64)), (128, 80, 1, 8, 80, (128, 80)),
+])
+def test_blocks_of_convolutions(c, side, stride, images, n, block):
+    m, k, conv = conv3(c, side, stride, images)
+    assert f32_form(m, n, k, conv=conv)[1] == block
+
+
 def test_block_hooks_refuse_bad_sizes():
     f = (C.c_int * 4)()
     for args in ((0, 0, 16, 64, 0, 0, 0, 1), (0, 8, 0, 64, 0, 0, 0, 1), (0, 8, 16, 0, 0, 0, 0, 1), (0, 8, 16, 64, 0, 4, 0, 1), (0, 8, 16, 64, 0, 4, 5, 1)):

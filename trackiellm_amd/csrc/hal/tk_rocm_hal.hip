@@ -173,6 +173,48 @@ tk_error_code_t tk_mi355x_gemm_pair(int device, int M, int N, int K, const float
     return ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
 }
 
+/* false: sizes that do not belong together */
+static bool gemm_f32_sizes(TkGemm& g, int M, int N, int K, int lda, int ldb, const int* conv) {
+    if (M <= 0 || N <= 0 || K <= 0 || ldb < K || (!conv && lda < K)) return false;
+    g.M = M; g.N = N; g.K = K; g.lda = lda; g.ldb = ldb; g.ldc = N; g.ldr = N; g.alpha = 1.0f; g.batch = 1;
+    if (!conv) return true;
+    for (int i = 0; i < 9; ++i)
+        if (conv[i] < (i == 6 ? 0 : 1) || conv[i] > 16384) return false;
+    g.im_C = conv[0]; g.im_H = conv[1]; g.im_W = conv[2]; g.im_ldx = conv[3]; g.im_kw = conv[4]; g.im_stride = conv[5]; g.im_pad = conv[6]; g.im_Ho = conv[7]; g.im_Wo = conv[8];
+    /* taps of the last output pixel that lie inside the image: nothing else is read */
+    return g.im_C % 4 == 0 && g.im_ldx % 4 == 0 && g.im_ldx >= g.im_C && (int64_t)K == (int64_t)g.im_kw * g.im_kw * g.im_C && ldb % 4 == 0 && M % (g.im_Ho * g.im_Wo) == 0;
+}
+
+tk_error_code_t tk_mi355x_gemm_f32(int device, int form, int M, int N, int K, int lda, int ldb, const float* a, const float* w, const float* bias, const float* residual, int act,
+                                   const int conv[9], float* c) {
+    TkGemm g{};
+    if (!a || !w || !c || act < 0 || act > 3 || !gemm_f32_sizes(g, M, N, K, lda, ldb, conv) || !tk_gemm_form_takes(g, form)) return TK_ERROR_INVALID_ARGUMENT;
+    int n = 0;
+    if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return TK_ERROR_GPU_DEVICE_NOT_FOUND;
+    if (device < 0 || device >= n || hipSetDevice(device) != hipSuccess) return TK_ERROR_INVALID_ARGUMENT;
+    const size_t na = conv ? (size_t)(M / (g.im_Ho * g.im_Wo)) * g.im_H * g.im_W * g.im_ldx : (size_t)M * lda, nw = (size_t)N * ldb, nc = (size_t)M * N;
+    float *da = nullptr, *dw = nullptr, *db = nullptr, *dr = nullptr, *dc = nullptr;
+    auto put = [](float** d, const float* h, size_t n) { return hipMalloc((void**)d, n * 4) == hipSuccess && hipMemcpy(*d, h, n * 4, hipMemcpyHostToDevice) == hipSuccess; };
+    bool ok = tk_nn_prepare_device() && put(&da, a, na) && put(&dw, w, nw) && (!bias || put(&db, bias, N)) && (!residual || put(&dr, residual, nc)) &&
+              hipMalloc((void**)&dc, nc * 4) == hipSuccess;
+    if (ok) {
+        g.A = da; g.B = dw; g.C = dc; g.bias = db; g.residual = dr; g.act = act;
+        tk_launch_gemm_form(g, form, nullptr);
+        ok = hipGetLastError() == hipSuccess && hipMemcpy(c, dc, nc * 4, hipMemcpyDeviceToHost) == hipSuccess;
+    }
+    float* ptrs[] = {da, dw, db, dr, dc};
+    for (float* q : ptrs) if (q) (void)hipFree(q);
+    return ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
+}
+
+tk_error_code_t tk_mi355x_gemm_f32_form(int M, int N, int K, int lda, int ldb, int batch, const int conv[9], int* form, int block[2]) {
+    TkGemm g{};
+    if (!form || !block || batch < 1 || (conv && batch > 1) || !gemm_f32_sizes(g, M, N, K, lda, ldb, conv)) return TK_ERROR_INVALID_ARGUMENT;
+    g.batch = batch; g.sA = (int64_t)M * lda; g.sB = (int64_t)N * ldb; g.sC = (int64_t)M * N;
+    *form = tk_gemm_f32_form(g, block);
+    return TK_SUCCESS;
+}
+
 tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]) {
     if (rows <= 0 || N <= 0 || K <= 0 || experts < 0 || (experts > 0 && (top < 1 || top > experts)) || !form) return TK_ERROR_INVALID_ARGUMENT;
     const int to = swiglu ? 32 : 16;

@@ -20,6 +20,11 @@
 #include "../common/tk_gemm_desc.h"
 
 void tk_launch_gemm(const TkGemm& g, hipStream_t s);
+/* the exact kernel that tk_launch_gemm takes (0 .. 5: 16 x 16 x 4 forms, 6 .. 8: tall, 9: 128 x 128, 10: 64 x 64; reads no operand, only its alignment), and
+ * a launch of a given one that takes these operands: the same bits from each */
+int tk_gemm_f32_form(const TkGemm& g, int block[2]);
+bool tk_gemm_form_takes(const TkGemm& g, int form);
+void tk_launch_gemm_form(const TkGemm& g, int form, hipStream_t s);
 /* whether a convolution can be addressed by the GEMM itself (TkGemm::im_*): channels and pitch multiples of 4, input x and the [N][K]
  * f32 weights w 16-byte aligned */
 bool tk_gemm_im2col_ok(const float* x, int C, int ldx, const float* w);

@@ -1025,53 +1025,78 @@ static bool tk_gemm_fast(const TkGemm& g) {
     return true;
 }
 
-/* What an exact-chain launch costs, by kernel: start + K (a + b x more) + c x more, where more = workgroups per CU beyond the first (a workgroup alone on
- * its CU waits for its own chain and loads, further ones share the pipe).  Fitted to the detector's layers at 1, 8 and 32 frames; us, ns per k. */
-struct F32Form { int rows, cols; float start, a, b, c; };
+/* What an exact-chain launch costs, by kernel and load path: start + K (a + b x more) + c x more; us, ns per k.  more = workgroups per CU beyond the first, a
+ * last round that is partly filled counted half way to a full one (a workgroup alone on its CU waits for its own chain and loads, further ones share the
+ * pipe).  Fitted to 2089 products of 1 .. 102 400 rows, 1 .. 1500 columns, K 27 .. 4608, up to 48 of them side by side, and convolutions of 7 x 7 .. 112 x 112
+ * pixels, and the detector's layers at 1, 8 and 32 frames: the choice is 1.60 (the detector's layers 1.70) times as fast as the 32 x 32 x 2 kernels alone,
+ * the best choice would be 1.63 (1.71). */
+struct F32Cost { float start, a, b, c; };
+struct F32Form { int rows, cols; F32Cost general, aligned, conv; }; /* rows and columns of a block; PATH 0, PATH 1 and 2, implicit im2col */
 constexpr F32Form f32_forms[] = {
-    {32, 32, 3.3f, 11.0f, 8.5f, 1.0f},   /* 400 x 256 x 1152: 16 us (128 x 128: 102), 400 x 64 x 2304: 27 us (64 x 64: 69) */
-    {64, 16, 4.5f, 11.5f, 8.6f, 1.2f},   /* 6400 x 80 x 720: 19 us (128 x 96: 57) */
-    {64, 32, 5.0f, 16.1f, 18.0f, 1.4f},  /* 12800 x 64 x 1152: 37 us (128 x 64: 64) */
-    {64, 64, 6.0f, 25.5f, 26.5f, 1.4f},  /* 12800 x 128 x 576: 33 us (128 x 128: 60) */
-    {64, 80, 7.0f, 31.0f, 32.5f, 2.2f},  /* 204800 x 80 x 720: 294 us (128 x 96: 328) */
-    {128, 80, 10.0f, 51.6f, 68.0f, 3.0f}, /* 51200 x 80 x 1152: 124 us (128 x 96: 136) */
+    /* k_gemm_f32_t16 */
+    {32, 32, {4.6f, 16.1f, 12.9f, 0.7f}, {3.2f, 8.7f, 6.6f, 0.7f}, {4.8f, 10.0f, 6.4f, 1.3f}},     /* 400 x 256 x 1152: 16 us (128 x 128: 102) */
+    {64, 16, {4.8f, 16.5f, 15.6f, 0.7f}, {3.5f, 9.3f, 7.9f, 0.7f}, {5.3f, 11.4f, 7.2f, 1.5f}},     /* 6400 x 80 x 720: 19 us (128 x 96: 57) */
+    {64, 32, {5.6f, 23.6f, 22.4f, 1.4f}, {4.0f, 13.5f, 12.2f, 1.2f}, {6.5f, 15.8f, 11.7f, 2.4f}},  /* 12544 x 64 x 4608: 126 us (128 x 64: 236) */
+    {64, 64, {4.9f, 41.3f, 37.2f, 0.9f}, {3.8f, 22.3f, 18.3f, 1.4f}, {7.3f, 25.4f, 19.8f, 1.8f}},  /* 12800 x 128 x 576: 33 us (128 x 128: 60) */
+    {64, 80, {5.0f, 49.3f, 45.9f, 1.6f}, {4.0f, 30.2f, 23.4f, 1.5f}, {7.0f, 32.0f, 26.9f, 1.9f}},  /* 204800 x 80 x 720: 294 us (128 x 96: 328) */
+    {128, 80, {9.5f, 86.0f, 79.3f, 4.8f}, {8.5f, 55.1f, 47.4f, 4.7f}, {11.2f, 54.2f, 55.0f, 3.5f}}, /* 51200 x 80 x 1152: 124 us (128 x 96: 136) */
+    /* k_gemm_f32_tall, k_gemm_f32_big, k_gemm_f32 */
+    {128, 32, {3.1f, 47.1f, 37.7f, 0.2f}, {3.3f, 24.4f, 19.5f, 1.5f}, {5.8f, 34.0f, 21.0f, 2.3f}},
+    {128, 64, {4.0f, 68.8f, 63.2f, 0.5f}, {4.2f, 40.0f, 40.0f, 2.6f}, {8.5f, 49.2f, 41.8f, 2.9f}},
+    {128, 96, {4.3f, 91.2f, 89.7f, 1.1f}, {4.4f, 56.3f, 54.1f, 4.8f}, {9.1f, 65.6f, 54.9f, 7.1f}},
+    {128, 128, {4.6f, 150.3f, 118.4f, 3.6f}, {5.7f, 78.0f, 73.2f, 3.0f}, {13.1f, 78.8f, 74.9f, 6.1f}},
+    {64, 64, {2.6f, 48.5f, 28.6f, 0.5f}, {2.5f, 23.6f, 20.1f, 0.4f}, {4.9f, 27.7f, 22.0f, 1.0f}},
 };
-static float f32_cost(const F32Form& f, const TkGemm& g, int nz) {
-    const float wgs = (float)((g.M + f.rows - 1) / f.rows) * (float)((g.N + f.cols - 1) / f.cols) * (float)nz;
-    const float more = wgs > 256.0f ? wgs / 256.0f - 1.0f : 0.0f;
-    return f.start + 1e-3f * (float)g.K * (f.a + f.b * more) + f.c * more;
+enum { F32_T16 = 6, F32_TALL = 6, F32_BIG = 9, F32_SMALL = 10, F32_FORMS = 11 };
+static float f32_cost(const F32Form& f, const TkGemm& g, int path, int nz) {
+    const F32Cost& c = g.im_C > 0 ? f.conv : path ? f.aligned : f.general;
+    const float wgs = (float)((g.M + f.rows - 1) / f.rows) * (float)((g.N + f.cols - 1) / f.cols) * (float)nz * (1.0f / 256.0f);
+    const float more = wgs > 1.0f ? 0.5f * (wgs + ceilf(wgs)) - 1.0f : 0.0f;
+    return c.start + 1e-3f * (float)g.K * (c.a + c.b * more) + c.c * more;
 }
-/* the 16 x 16 x 4 form of a launch, or -1: one of the 32 x 32 x 2 kernels is expected to be quicker (high-resolution layers of few channels and many
- * frames, scores of whole utterances), or the operands are not for it */
-static int f32_pick(const TkGemm& g, int nz) {
-    /* its offsets have 32 bits */
+/* whether a form takes the operands at all */
+static bool f32_form_takes(const TkGemm& g, int nz, int form) {
+    if (form < 0 || form >= F32_FORMS) return false;
+    if (form >= F32_BIG) return true;
+    if (form >= F32_TALL) return g.N <= f32_forms[form].cols && !g.b_kn && !g.b_f16 && nz == 1 && g.batch_inner == 0;
+    /* [K][N] matrices: 1500 x 64 x 1500 x 192 483 us with the 64 x 64 kernel, 580 and more here.  Offsets have 32 bits, a k and its tap 16 */
     const int64_t most = 1 << 28;
-    if (g.b_f16 || g.b_kn || g.K < 1 || g.K > 60000) return -1; /* [K][N] matrices: 1500 x 64 x 1500 x 192 483 us with the 64 x 64 kernel, 580 and more here */
+    if (g.b_f16 || g.b_kn || g.M < 1 || g.N < 1 || g.K < 1 || g.K > 60000 || (g.M + f32_forms[form].rows - 1) / f32_forms[form].rows > 65535) return false;
     if (g.im_C > 0) {
         const int64_t images = g.M / ((int64_t)g.im_Ho * g.im_Wo) + 1;
-        if (images * g.im_H * g.im_W * g.im_ldx >= most || g.im_C > 60000) return -1;
+        if (images * g.im_H * g.im_W * g.im_ldx >= most || g.im_C > 60000) return false;
     } else if ((int64_t)g.M * g.lda >= most) {
-        return -1;
+        return false;
     }
-    if ((int64_t)g.N * g.ldb >= most) return -1;
-    F32Form old;
-    if (g.M >= 256 && g.N >= 96) old = F32Form{128, 128, 11.0f, 78.0f, 105.0f, 2.0f};
-    else if (g.N < 96 && g.M >= 4 * NBM && nz == 1 && g.batch_inner == 0)
-        old = g.N <= 32 ? F32Form{NBM, 32, 4.5f, 36.0f, 36.0f, 0.5f} : g.N <= 64 ? F32Form{NBM, 64, 6.0f, 50.0f, 50.0f, 2.4f} : F32Form{NBM, 96, 5.0f, 72.0f, 72.0f, 4.9f};
-    else old = F32Form{BM, BN, 2.0f, 29.0f, 40.0f, 1.0f};
-    int best = -1;
-    float least = f32_cost(old, g, nz);
-    for (int i = 0; i < (int)(sizeof f32_forms / sizeof f32_forms[0]); ++i) {
-        const float c = f32_cost(f32_forms[i], g, nz);
-        if (c < least && (g.M + f32_forms[i].rows - 1) / f32_forms[i].rows <= 65535) { least = c; best = i; }
+    return (int64_t)g.N * g.ldb < most;
+}
+/* the kernel of a launch: of the 32 x 32 x 2 ones by rows and columns, of the 16 x 16 x 4 ones the quickest, where it is expected to be clearly quicker (the
+ * costs hold within some 10 %) */
+static int f32_pick(const TkGemm& g, int path, int nz) {
+    int best = F32_SMALL;
+    if (g.M >= 256 && g.N >= 96) best = F32_BIG;
+    else if (g.M >= 4 * NBM && f32_form_takes(g, nz, F32_TALL + 2)) best = F32_TALL + (g.N <= 32 ? 0 : g.N <= 64 ? 1 : 2); /* narrow and tall: every column in one workgroup */
+    float least = 0.92f * f32_cost(f32_forms[best], g, path, nz);
+    for (int i = 0; i < F32_T16; ++i) {
+        if (!f32_form_takes(g, nz, i)) continue;
+        /* a slab or two of k on a full chip is a copy with some products: 204800 x 64 x 64 39 us in blocks of 128 rows, 43 and more in smaller ones */
+        if (g.K <= 64 && (int64_t)((g.M + f32_forms[i].rows - 1) / f32_forms[i].rows) * ((g.N + f32_forms[i].cols - 1) / f32_forms[i].cols) * nz > 512) continue;
+        const float c = f32_cost(f32_forms[i], g, path, nz);
+        if (c < least) { least = c; best = i; }
     }
     return best;
 }
+int tk_gemm_f32_form(const TkGemm& g, int block[2]) {
+    const int form = f32_pick(g, tk_gemm_fast(g) ? (g.b_kn ? 2 : 1) : 0, g.batch > 0 ? g.batch : 1);
+    block[0] = f32_forms[form].rows; block[1] = f32_forms[form].cols;
+    return form;
+}
 
-void tk_launch_gemm(const TkGemm& g, hipStream_t s) {
+static void launch_f32(const TkGemm& g, hipStream_t s, int form /* < 0: f32_pick() */) {
     const int nz = g.batch > 0 ? g.batch : 1;
     const bool im = g.im_C > 0; /* validated by tk_gemm_im2col_ok(): aligned [N][K] f32 weights, C % 4 == 0, no batch */
     const int path = tk_gemm_fast(g) ? (g.b_kn ? 2 : 1) : 0;
+    if (form < 0) form = f32_pick(g, path, nz);
 #define TK_GEMM_PATHS(KERNEL, GRID, LDS)                                                                      \
     do {                                                                                                      \
         if (im) hipLaunchKernelGGL((KERNEL<true, 1>), GRID, dim3(256), LDS, s, g);                            \
@@ -1079,11 +1104,57 @@ void tk_launch_gemm(const TkGemm& g, hipStream_t s) {
         else if (path == 2) hipLaunchKernelGGL((KERNEL<false, 2>), GRID, dim3(256), LDS, s, g);               \
         else hipLaunchKernelGGL((KERNEL<false, 0>), GRID, dim3(256), LDS, s, g);                              \
     } while (0)
+#define TK_T16(WM, WN, MT, NT, BK16) do {                                                                                                     \
+        const dim3 grid((g.N + WN * NT * 16 - 1) / (WN * NT * 16), (g.M + WM * MT * 16 - 1) / (WM * MT * 16), nz);                              \
+        const size_t lds = (size_t)2 * (WM * MT + WN * NT) * BK16 * 1024;                                                                      \
+        if (im) hipLaunchKernelGGL((k_gemm_f32_t16<true, 1, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                                \
+        else if (path == 1) hipLaunchKernelGGL((k_gemm_f32_t16<false, 1, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                   \
+        else hipLaunchKernelGGL((k_gemm_f32_t16<false, 0, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                                  \
+    } while (0)
+#define TK_TALL(NTV)                                                                                          \
+    do {                                                                                                      \
+        const dim3 grid(1, (g.M + NBM - 1) / NBM, 1);                                                         \
+        if (im) hipLaunchKernelGGL((k_gemm_f32_tall<true, 1, NTV>), grid, dim3(256), 0, s, g);                \
+        else if (path == 1) hipLaunchKernelGGL((k_gemm_f32_tall<false, 1, NTV>), grid, dim3(256), 0, s, g);   \
+        else hipLaunchKernelGGL((k_gemm_f32_tall<false, 0, NTV>), grid, dim3(256), 0, s, g);                  \
+    } while (0)
+    switch (form) {
+        case 0: TK_T16(2, 2, 1, 1, 4); break;
+        case 1: TK_T16(4, 1, 1, 1, 4); break;
+        case 2: TK_T16(2, 2, 2, 1, 4); break;
+        case 3: TK_T16(2, 2, 2, 2, 2); break;
+        case 4: TK_T16(4, 1, 1, 5, 2); break;
+        case 5: TK_T16(4, 1, 2, 5, 2); break;
+        case 6: TK_TALL(1); break;
+        case 7: TK_TALL(2); break;
+        case 8: TK_TALL(3); break;
+        case 9: {
+            const size_t lds = (size_t)2 * (LBM + LBN) * LDS_LD * sizeof(float);
+            (void)tk_nn_prepare_device();
+            const dim3 grid((g.N + LBN - 1) / LBN, (g.M + LBM - 1) / LBM, nz);
+            TK_GEMM_PATHS(k_gemm_f32_big, grid, lds);
+            break;
+        }
+        default: {
+            const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, nz);
+            TK_GEMM_PATHS(k_gemm_f32, grid, 0);
+        }
+    }
+#undef TK_TALL
+#undef TK_T16
+#undef TK_GEMM_PATHS
+}
+bool tk_gemm_form_takes(const TkGemm& g, int form) { return f32_form_takes(g, g.batch > 0 ? g.batch : 1, form); }
+void tk_launch_gemm_form(const TkGemm& g, int form, hipStream_t s) { launch_f32(g, s, form); }
+
+void tk_launch_gemm(const TkGemm& g, hipStream_t s) {
+    const int nz = g.batch > 0 ? g.batch : 1;
+    const bool im = g.im_C > 0;
     /* TkGemm::fast: the split-f16 kernels where the operands meet the one-load-per-group conditions ([N][K] f32 weights); every other
      * shape keeps the exact chain.  Which kernel runs depends on N and the batch layout only, NEVER on M: a row's result must not depend
      * on how many other rows (frames, utterances) share its launch — the two split kernels evaluate an element identically (the same 16-k
      * MFMA steps from k = 0), the exact ones differ from them, so a choice by M would make a fast handle's result depend on its batch. */
-    const bool fast = g.fast != 0 && !g.b_kn && (im || path == 1);
+    const bool fast = g.fast != 0 && !g.b_kn && (im || tk_gemm_fast(g));
     if (fast && g.N >= 96) {
         (void)tk_nn_prepare_device();
         const dim3 grid((g.N + LBN - 1) / LBN, (g.M + LBM - 1) / LBM, nz);
@@ -1103,46 +1174,7 @@ void tk_launch_gemm(const TkGemm& g, hipStream_t s) {
 #undef TK_TALL_H3
         return;
     }
-#define TK_T16(WM, WN, MT, NT, BK16) do {                                                                                                     \
-        const dim3 grid((g.N + WN * NT * 16 - 1) / (WN * NT * 16), (g.M + WM * MT * 16 - 1) / (WM * MT * 16), nz);                              \
-        const size_t lds = (size_t)2 * (WM * MT + WN * NT) * BK16 * 1024;                                                                      \
-        if (im) hipLaunchKernelGGL((k_gemm_f32_t16<true, 1, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                                \
-        else if (path == 1) hipLaunchKernelGGL((k_gemm_f32_t16<false, 1, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                   \
-        else hipLaunchKernelGGL((k_gemm_f32_t16<false, 0, WM, WN, MT, NT, BK16>), grid, dim3(256), lds, s, g);                                  \
-    } while (0)
-    switch (f32_pick(g, nz)) {
-        case 0: TK_T16(2, 2, 1, 1, 4); return;
-        case 1: TK_T16(4, 1, 1, 1, 4); return;
-        case 2: TK_T16(2, 2, 2, 1, 4); return;
-        case 3: TK_T16(2, 2, 2, 2, 2); return;
-        case 4: TK_T16(4, 1, 1, 5, 2); return;
-        case 5: TK_T16(4, 1, 2, 5, 2); return;
-        default: break;
-    }
-#undef TK_T16
-    if (g.M >= 256 && g.N >= 96) {
-        const size_t lds = (size_t)2 * (LBM + LBN) * LDS_LD * sizeof(float);
-        (void)tk_nn_prepare_device();
-        const dim3 grid((g.N + LBN - 1) / LBN, (g.M + LBM - 1) / LBM, nz);
-        TK_GEMM_PATHS(k_gemm_f32_big, grid, lds);
-        return;
-    }
-    if (g.N < 96 && g.M >= 4 * NBM && !g.b_kn && !g.b_f16 && nz == 1 && g.batch_inner == 0) { /* narrow and tall: every column in one workgroup */
-        const dim3 grid(1, (g.M + NBM - 1) / NBM, 1);
-        const int nt = (g.N + 31) / 32;
-#define TK_TALL(NTV)                                                                                          \
-    do {                                                                                                      \
-        if (im) hipLaunchKernelGGL((k_gemm_f32_tall<true, 1, NTV>), grid, dim3(256), 0, s, g);                \
-        else if (path == 1) hipLaunchKernelGGL((k_gemm_f32_tall<false, 1, NTV>), grid, dim3(256), 0, s, g);   \
-        else hipLaunchKernelGGL((k_gemm_f32_tall<false, 0, NTV>), grid, dim3(256), 0, s, g);                  \
-    } while (0)
-        if (nt == 1) TK_TALL(1); else if (nt == 2) TK_TALL(2); else TK_TALL(3);
-#undef TK_TALL
-        return;
-    }
-    const dim3 grid((g.N + BN - 1) / BN, (g.M + BM - 1) / BM, nz);
-    TK_GEMM_PATHS(k_gemm_f32, grid, 0);
-#undef TK_GEMM_PATHS
+    launch_f32(g, s, -1);
 }
 
 bool tk_gemm_im2col_ok(const float* x, int C, int ldx, const float* w) {
