@@ -96,7 +96,7 @@ protected:
 
 private:
     struct Seq { int len = 0, prev = -1, side = 0; std::vector<int32_t> pages; };
-    struct Pass { int nrows = 0, nseg = 0, nchunks = 0, shortest = 1 << 30, ntiles = 0, nblocks = 0, nsums = 0; bool single = true, singles = true; }; /* all segments, or any, are single rows */
+    struct Pass { int nrows = 0, nseg = 0, nruns = 0, nchunks = 0, shortest = 1 << 30, ntiles = 0, nblocks = 0, nsums = 0; bool single = true, singles = true; }; /* all segments, or any, are single rows */
     TkLayeredModel* m_ = nullptr;
     std::mutex mu_; /* seqs_, free_pages_, host page table */
     std::vector<Seq> seqs_;

@@ -74,7 +74,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     const int max_tiles = R / 64 + mseq;
     /* tables behind the base's rows: segment of a row, segments, wanted rows, attention tiles, retention blocks */
     int32_t* ext = nullptr;
-    const size_t block_ints = sizeof(TkRetentionBlock) / 4, extra = (size_t)R + 5 * (size_t)mseq + R + (2 + block_ints) * (size_t)max_tiles;
+    const size_t block_ints = sizeof(TkRetentionBlock) / 4, extra = (size_t)R + 4 * (size_t)mseq + 2 * (size_t)(R / TK_DELTA_CHUNKED) + R + (2 + block_ints) * (size_t)max_tiles;
     if (!init_tables(m->device, c.vocab, R, extra, &ext)) return false;
     tab_ints_ = 3 * (size_t)R + extra;
     d_tab_ = d_seq;
@@ -85,7 +85,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     tab_.seg_n = p; p += mseq;
     tab_.seg_in = p; p += mseq;
     tab_.seg_out = p; p += mseq;
-    tab_.seg_chunk0 = p; p += mseq;
+    tab_.chunked = p; p += 2 * (size_t)(R / TK_DELTA_CHUNKED);
     d_out_rows_ = p; p += R;
     d_tiles_ = p; p += 2 * (size_t)max_tiles;
     d_blocks_ = p;
@@ -232,7 +232,7 @@ bool TkLayeredSession::upload_pages() {
 bool TkLayeredSession::describe(int nrows, const int32_t* seq, const int32_t* pos, const int32_t* tok, Pass* p) {
     const int R = row_cap_;
     int32_t *h_seq = h_tab_, *h_pos = h_seq + R, *h_tok = h_pos + R, *h_seg = h_tok + R, *row0 = h_seg + R, *sn = row0 + max_seq, *sin = sn + max_seq, *sout = sin + max_seq,
-            *chunk0 = sout + max_seq, *tiles = chunk0 + max_seq + R;
+            *chunked = sout + max_seq, *tiles = chunked + 2 * (R / TK_DELTA_CHUNKED) + R;
     TkRetentionBlock* blocks = (TkRetentionBlock*)(h_tab_ + (d_blocks_ - d_tab_));
     *p = Pass();
     p->nrows = nrows; p->singles = false;
@@ -264,6 +264,10 @@ bool TkLayeredSession::describe(int nrows, const int32_t* seq, const int32_t* po
         need += want > have ? want - have : 0;
     }
     if (need > free_pages_.size()) { error = "cache pool exhausted: " + std::to_string(need) + " more pages wanted, " + std::to_string(free_pages_.size()) + " of " + std::to_string(n_pages_) + " are free"; return false; }
+    int longest = 0, many = 0;
+    for (const Run& u : runs)
+        if (u.n >= TK_DELTA_CHUNKED) { longest = std::max(longest, u.n); many += u.n; }
+    const bool chunks = longest >= TK_DELTA_LONG || many >= TK_DELTA_MANY;
     for (const Run& u : runs) {
         const int r = u.r, n = u.n, id = seq[r], side = u.side;
         need_pages(seqs_[(size_t)id], id, pos[r] + n - 1);
@@ -272,8 +276,11 @@ bool TkLayeredSession::describe(int nrows, const int32_t* seq, const int32_t* po
         sout[p->nseg] = 2 * id + (side ^ 1);
         for (int t = 0; t < n; t += 64, ++p->ntiles) { tiles[2 * p->ntiles] = r + t; tiles[2 * p->ntiles + 1] = std::min(64, n - t); }
         for (int i = 0; i < n; ++i) { h_seq[r + i] = id; h_pos[r + i] = pos[r + i]; h_tok[r + i] = tok[r + i]; h_seg[r + i] = p->nseg; }
-        chunk0[p->nseg] = p->nchunks;
-        p->nchunks += tk_delta_chunks(n);
+        if (chunks && n >= TK_DELTA_CHUNKED) {
+            chunked[2 * p->nruns] = p->nseg; chunked[2 * p->nruns + 1] = p->nchunks;
+            ++p->nruns;
+            p->nchunks += (n + TK_DELTA_CHUNK - 1) / TK_DELTA_CHUNK;
+        }
         p->shortest = std::min(p->shortest, n);
         if (n > 1) {
             p->single = false;
@@ -391,7 +398,7 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             tk_launch_mixer_prep(type, proj_, pitch, a, d, tab_, n, s);
             if (!p.single) {
                 if (a) tk_launch_attn_tiles(type, *a, tab_, d_tiles_, p.ntiles, s);
-                if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, p.shortest, p.nchunks, n, s);
+                if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, p.shortest, p.nruns, p.nchunks, n, s);
                 continue;
             }
             const int splits = a ? tk_attn_rows_splits(*a, visible[ai], n) : 1;

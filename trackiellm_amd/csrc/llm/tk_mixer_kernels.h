@@ -22,7 +22,7 @@ struct TkPassTab {
     const int32_t *seq, *pos, *tok; /* [rows] */
     const int32_t* seg;             /* [rows] */
     const int32_t *seg_row0, *seg_n; /* [segments] */
-    const int32_t* seg_chunk0;      /* [segments] first chunk of a segment's own, ascending; a segment that has none (tk_delta_chunks) the next one's */
+    const int32_t* chunked;         /* [runs][2] segments that the delta rule takes in chunks, and the first chunk of each; ascending */
     int32_t *seg_in, *seg_out;      /* [segments] state copies read (-1: the sequence starts here) and written; never the same copy */
     const int32_t* page_of;         /* [sequences][max_pages] page ids */
     int max_pages;
@@ -94,13 +94,18 @@ void tk_launch_attn_rows(int type, const TkAttnArgs& a, const TkPassTab& t, int 
 int tk_attn_rows_splits(const TkAttnArgs& a, int pages, int nrows); /* for at most `pages` visible pages */
 size_t tk_attn_rows_scratch_floats(const TkAttnArgs& a, int nrows, int splits);
 
-/* the recurrence over every segment and the gated per-head norm of its output; shortest: rows of the pass's shortest segment, n_chunks: of all segments.
- * Segments of TK_DELTA_CHUNKED rows and more go in chunks, others token by token: a four-layer pass of one run takes 646 / 672 / 778 / 839 us token by
- * token and 670 / 680 / 772 / 819 us in chunks at 24 / 32 / 48 / 64 rows */
-#define TK_DELTA_CHUNKED 40
+/* the recurrence over every segment and the gated per-head norm of its output; shortest: rows of the pass's shortest segment, n_runs, n_chunks: of TkPassTab::chunked.
+ *
+ * Segments of TK_DELTA_CHUNKED rows and more go in chunks, others token by token, in passes that have one of TK_DELTA_LONG rows or TK_DELTA_MANY rows of such
+ * segments; in other passes all go token by token.  Token by token a run takes its length, however many there are, until they fill the chip; chunks
+ * cost three launches more and so lose where the chain is short.  Four-layer passes, 16 heads of 128 x 128, token by token / in chunks: one run of 40, 48,
+ * 64, 128 rows 757 / 773, 766 / 785, 830 / 835, 897 / 855 us; 4 of 40 961 / 971; 8 of 64 1504 / 1458; 51 of 40 4584 / 4378; 100 single rows and one
+ * run of 40 1302 / 1371. */
 #define TK_DELTA_CHUNK 16
-static inline int tk_delta_chunks(int rows) { return rows < TK_DELTA_CHUNKED ? 0 : (rows + TK_DELTA_CHUNK - 1) / TK_DELTA_CHUNK; } /* of a segment */
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments /* <= 256 */, int shortest, int n_chunks, int nrows, hipStream_t s);
+#define TK_DELTA_CHUNKED 40
+#define TK_DELTA_LONG 72
+#define TK_DELTA_MANY 224
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_runs /* <= 256 */, int n_chunks, int nrows, hipStream_t s);
 /* scratch of a pass of at most `rows` rows: its chunks, and one that is partly filled per segment (16 heads of 128, 2048 rows: 78 MB) */
 size_t tk_delta_chunk_floats(int heads, int dim, int rows);
 /* the same for passes whose segments are single rows: one launch */

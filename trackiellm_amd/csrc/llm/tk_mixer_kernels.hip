@@ -892,12 +892,12 @@ __device__ __forceinline__ tk_v4f quad_transpose(tk_v4f v) {
  * Bound by LDS reads and the vector work they feed; 2047 tokens x 16 heads are eight workgroups per CU, 31 us (53 us with one token j and eight key
  * rows a thread and results stored four bytes at a time). */
 template <int DP>
-__global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t, int nseg) {
+__global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t, int nruns) {
     constexpr int PE = DP / 32; /* key rows of a thread in the pair products */
     __shared__ __attribute__((aligned(16))) float lq[DC][DP], lk[DC][DP], lg[DC][DP], L[DC][DC], B[DC][DC], lb[DC];
     const int tid = threadIdx.x, chunk = blockIdx.y, h = blockIdx.x, kvh = h / (d.heads / d.kv_heads);
-    const int seg = __syncthreads_count(tid < nseg && t.seg_chunk0[tid < nseg ? tid : 0] <= chunk) - 1; /* the last one that begins here or before: it has chunks */
-    const int t0 = (chunk - t.seg_chunk0[seg]) * DC, n = t.seg_n[seg];
+    const int run = __syncthreads_count(tid < nruns && t.chunked[2 * (tid < nruns ? tid : 0) + 1] <= chunk) - 1; /* the last one that begins here or before */
+    const int seg = t.chunked[2 * run], t0 = (chunk - t.chunked[2 * run + 1]) * DC, n = t.seg_n[seg];
     const int m = n - t0 < DC ? n - t0 : DC, row0 = t.seg_row0[seg] + t0;
     float* const w = d.chunks + ((size_t)chunk * d.heads + h) * delta_chunk_floats(DP);
     float *const wq = w + DC * DP, *const wk = wq + DC * DP, *const wg = wk + DC * DP, *const wt = wg + DP, *const wb = wt + DC * DC;
@@ -999,9 +999,8 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
     constexpr int NT = DP / 64, AHEAD = 3;
     __shared__ tk_v4f pu[2][4][64], po[2][4][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4;
-    const int h = blockIdx.x, seg = blockIdx.z, vp = (d.vdim + 3) & ~3, col = blockIdx.y * 16 + (lane & 15);
+    const int h = blockIdx.x, seg = t.chunked[2 * blockIdx.z], vp = (d.vdim + 3) & ~3, col = blockIdx.y * 16 + (lane & 15);
     const int row0 = t.seg_row0[seg], n = t.seg_n[seg], in = t.seg_in[seg], out = t.seg_out[seg];
-    if (n < TK_DELTA_CHUNKED) return;
     const bool live = col < d.vdim;
     const int nc = (n + DC - 1) / DC;
     if (AGAIN && !__syncthreads_or(live && !__builtin_isfinite(d.state[((size_t)out * d.heads + h) * d.dim * vp + col]))) return;
@@ -1015,7 +1014,7 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
         }
     struct Ops { tk_v4f w[NT], q[NT], k[NT], g[NT]; float t, b, v; } ops[AHEAD + 1];
     const size_t step = (size_t)d.heads * delta_chunk_floats(DP);
-    const float* const base = d.chunks + ((size_t)t.seg_chunk0[seg] * d.heads + h) * delta_chunk_floats(DP);
+    const float* const base = d.chunks + ((size_t)t.chunked[2 * blockIdx.z + 1] * d.heads + h) * delta_chunk_floats(DP);
     auto fetch = [&](Ops& o, int c) {
         const float* p = base + (size_t)c * step;
         const int tile = wave * NT;
@@ -1881,10 +1880,11 @@ bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, 
 
 size_t tk_delta_chunk_floats(int heads, int dim, int rows) { return (size_t)(rows / DC + rows / TK_DELTA_CHUNKED) * heads * delta_chunk_floats(delta_pad(dim)); }
 
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_chunks, int nrows, hipStream_t s) {
-    if (n_chunks > 0) {
-        const dim3 chunks(d.heads, n_chunks), chain(d.heads, (d.vdim + 15) / 16, n_segments); /* heads first: a head's workgroups share an XCD's L2 */
-#define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_segments); \
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_runs, int n_chunks, int nrows, hipStream_t s) {
+    const int below = n_runs > 0 ? TK_DELTA_CHUNKED : 1 << 30;
+    if (n_runs > 0) {
+        const dim3 chunks(d.heads, n_chunks), chain(d.heads, (d.vdim + 15) / 16, n_runs); /* heads first: a head's workgroups share an XCD's L2 */
+#define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_runs); \
         hipLaunchKernelGGL((k_delta_chain<DP, false>), chain, dim3(256), 0, s, d, t); hipLaunchKernelGGL((k_delta_chain<DP, true>), chain, dim3(256), 0, s, d, t); } while (0)
         switch (delta_pad(d.dim)) {
             case 64: TK_CHUNKED(64); break;
@@ -1893,10 +1893,10 @@ void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, in
         }
 #undef TK_CHUNKED
     }
-    if (shortest < TK_DELTA_CHUNKED) {
+    if (shortest < below) {
         const bool many = (int64_t)((d.vdim + 15) / 16) * d.heads * n_segments >= 512;
         const dim3 grid(many ? (d.vdim + 15) / 16 : (d.vdim + 7) / 8, d.heads, n_segments);
-#define TK_SCAN(RPL) do { if (many) hipLaunchKernelGGL((k_delta_scan<16, 2 * RPL>), grid, dim3(256), 0, s, d, t, TK_DELTA_CHUNKED); else hipLaunchKernelGGL((k_delta_scan<32, RPL>), grid, dim3(256), 0, s, d, t, TK_DELTA_CHUNKED); } while (0)
+#define TK_SCAN(RPL) do { if (many) hipLaunchKernelGGL((k_delta_scan<16, 2 * RPL>), grid, dim3(256), 0, s, d, t, below); else hipLaunchKernelGGL((k_delta_scan<32, RPL>), grid, dim3(256), 0, s, d, t, below); } while (0)
         if (d.dim <= 32) TK_SCAN(1);
         else if (d.dim <= 64) TK_SCAN(2);
         else if (d.dim <= 128) TK_SCAN(4);
