@@ -345,7 +345,9 @@ bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
      * that TWO workgroups share a CU and one's ring fill and epilogue run under the other's MFMAs. */
     const bool twin = ny > 1 && (mt == 8 || mt == 6) && Kr % 64 == 0;
     const bool one = mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES;
-    const int pf = mt == 16 || twin ? 2 : one ? (Kr % 256 == 0 ? 8 : 4) : 4;
+    /* whole range: eight pieces of weights in flight where they divide it, but not all of it at once: 51872 x 256, f32, 1 and 32 rows 14.9 and 18.9 us with
+     * four, 18.2 and 22.6 with eight */
+    const int pf = mt == 16 || twin ? 2 : one && Kr % 256 == 0 && Kr > 256 ? 8 : 4;
     const int slot_kib = twin ? 32 : 64;
     int rk = one ? Kr : 0;
     for (int c = (slot_kib * 16 / mt) / (32 * pf) * (32 * pf); rk == 0 && c >= 32 * pf; c -= 32 * pf)
