@@ -88,6 +88,8 @@ typedef struct {
 /* explicit geometry + batch (parity tests use a small geometry; bench uses tiny.en with max_batch = B); max_batch in [1, 256] */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_asr_create(tk_asr_whisper_context_t** out, const tk_mi355x_whisper_hparams_t* hp, uint64_t seed,
                                                          int device, int max_batch);
+/* device memory that such a context's passes work in.  No GPU involved. */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_asr_arena_bytes(const tk_mi355x_whisper_hparams_t* hp, int max_batch, uint64_t* bytes);
 /* B utterances of n_samples int16 each -> exactly n_steps greedy tokens per utterance (forced, EOT ignored);
  * optional outputs: mel [B][2*ctx][n_mels], enc [B][ctx][d], logits of the first sampled position [B][n_vocab] */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_asr_transcribe_tokens(tk_asr_whisper_context_t* ctx, int batch, const int16_t* pcm, int n_samples,

@@ -440,6 +440,16 @@ tk_error_code_t tk_mi355x_asr_create(tk_asr_whisper_context_t** out, const tk_mi
     return asr_new(out, h, "", seed, device, max_batch, false);
 }
 
+tk_error_code_t tk_mi355x_asr_arena_bytes(const tk_mi355x_whisper_hparams_t* hp, int max_batch, uint64_t* bytes) {
+    if (!hp || !bytes || max_batch < 1 || max_batch > 256 || hp->n_mels < 1 || hp->n_audio_ctx < 1 || hp->n_audio_state < 1 || hp->n_audio_head < 1 || hp->n_audio_layer < 0 ||
+        hp->n_text_ctx < 1 || hp->n_text_state < 1 || hp->n_text_head < 1 || hp->n_text_layer < 0 || hp->n_vocab < 1)
+        return TK_ERROR_INVALID_ARGUMENT;
+    const TkWhisperHP h{hp->n_mels, hp->n_audio_ctx, hp->n_audio_state, hp->n_audio_head, hp->n_audio_layer,
+                        hp->n_text_ctx, hp->n_text_state, hp->n_text_head, hp->n_text_layer, hp->n_vocab};
+    *bytes = (uint64_t)tk_asr_arena_floats(h, tk_whisper_manifest(h), max_batch) * 4;
+    return TK_SUCCESS;
+}
+
 tk_error_code_t tk_mi355x_asr_get_hparams(tk_asr_whisper_context_t* ctx, tk_mi355x_whisper_hparams_t* out) {
     if (!ctx || !out) return TK_ERROR_INVALID_ARGUMENT;
     const TkWhisperHP& h = ctx->sh->model.hp;

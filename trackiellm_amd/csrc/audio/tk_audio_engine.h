@@ -35,6 +35,9 @@ public:
     bool load_ggml(class TkWhisperGgml& g);
 };
 
+/* floats of scratch that a TkAsr of up to `max_batch` clips works in */
+size_t tk_asr_arena_floats(const TkWhisperHP& hp, const TkWhManifest& man, int max_batch);
+
 class TkAsr {
 public:
     TkWhisperModel* model = nullptr;

@@ -411,6 +411,10 @@ struct TkAudioGpuOps {
     }
     float* raw_alloc(size_t n) {
         n = (n + 63) & ~(size_t)63;
+        if (a->arena_used + n > a->arena_floats) { /* tk_asr_arena_floats() counts every allocation: not reached */
+            a->launch_error = "ASR arena too small";
+            return a->arena;
+        }
         float* p = a->arena + a->arena_used;
         a->arena_used += n;
         return p;
@@ -553,7 +557,7 @@ struct TkAudioSizeOps {
     size_t used = 0, peak = 0;
     float* alloc(size_t n) { used += (n + 63) & ~(size_t)63; if (used > peak) peak = used; return nullptr; }
     int32_t* alloc_i32(size_t n) { return (int32_t*)alloc(n); }
-    void gemm(const TkGemm& g) { /* the tiled path's activation image is scratch on top of the live allocations; fc1 of a short pass adds fc2's image */
+    void gemm(const TkGemm& g) { /* the tiled path's activation image is scratch on top of the live allocations; fc1 adds fc2's image */
         if (!tk_tiled_gemm_applies(g)) return;
         size_t top = used + ((tk_tiled_gemm_scratch(g) + 63) & ~(size_t)63);
         if (g.c_feeds_linear) { TkGemm nx{}; nx.M = g.M; nx.K = g.N; top += (tk_tiled_gemm_scratch(nx) + 63) & ~(size_t)63; }
@@ -692,19 +696,27 @@ TkAsr::~TkAsr() {
     if (stream) (void)hipStreamDestroy(stream);
 }
 
+/* all that a transcription of `mb` clips has in the arena at any time: the long passes, then the decode loop's token / position / arg-max tables and the
+ * operand images of a step on top of what the long passes leave */
+size_t tk_asr_arena_floats(const TkWhisperHP& hp, const TkWhManifest& man, int mb) {
+    TkAudioSizeOps so;
+    std::vector<float*> nullw(man.t.size(), nullptr);
+    TkWhisperGraph<TkAudioSizeOps> g{hp, man, nullw.data()};
+    float* ml = g.mel(so, nullptr, mb, 0, 0);
+    float* enc = g.encode(so, ml, mb);
+    auto st = g.begin_decode(so, enc, mb);
+    so.alloc_i32((size_t)3 * hp.n_text_ctx * mb);
+    g.decode_step(so, st, 0);
+    return so.peak + 4096;
+}
+
 bool TkAsr::init(TkWhisperModel* m, int mb) {
     model = m;
     max_batch = mb;
     if (!m || mb < 1 || mb > 256) { error = "max_batch must be in [1,256]"; return false; }
     HIPQ(hipSetDevice(m->device));
     HIPQ(tk_create_perception_stream(&stream));
-    TkAudioSizeOps so;
-    std::vector<float*> nullw(m->man.t.size(), nullptr);
-    TkWhisperGraph<TkAudioSizeOps> g{m->hp, m->man, nullw.data()};
-    float* ml = g.mel(so, nullptr, mb, 0, 0);
-    float* enc = g.encode(so, ml, mb);
-    (void)g.begin_decode(so, enc, mb);
-    arena_floats = so.peak + 4096 + (size_t)3 * m->hp.n_text_ctx * mb + 64; /* + the decode loop's token / position / arg-max tables */
+    arena_floats = tk_asr_arena_floats(m->hp, m->man, mb);
     if (!m->prepare_tiles()) { error = m->error; return false; }
     if (!tk_gemm_tiled_prepare_device() || !at1_prepare_device()) { error = "LDS opt-in of the tiled GEMM or of the decoder's attention failed"; return false; }
     HIPQ(hipMalloc((void**)&arena, arena_floats * 4));
