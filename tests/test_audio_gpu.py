@@ -73,6 +73,19 @@ def test_decoder_attention_over_contexts_and_heads(gpu, ctx, state, heads, clips
     assert np.array_equal(toks, want)
 
 
+@pytest.mark.parametrize("ctx,state,heads,layers,clips", [(200, 1344, 21, 1, 5), (300, 512, 2, 2, 32), (8, 128, 2, 3, 1)])
+def test_text_context_longer_than_the_audio(gpu, ctx, state, heads, layers, clips):
+    """geometries whose decoder steps need more scratch than the encoder leaves room for"""
+    ohp = O.whisper_tiny_test()
+    ohp.n_audio_ctx, ohp.n_audio_state, ohp.n_audio_head, ohp.n_audio_layer = ctx, state, heads, 1
+    ohp.n_text_ctx, ohp.n_text_state, ohp.n_text_head, ohp.n_text_layer = 448, state, heads, layers
+    asr = gpu.Asr(hp=hp_of(gpu, ohp), seed=3, max_batch=clips)
+    pcm = np.clip(np.random.default_rng(ctx).normal(0, 3000, (clips, 2500)), -32768, 32767).astype(np.int16)
+    toks, _, _, lg = asr.transcribe_tokens(pcm, 4)
+    want, _, _, wlg = O.OracleWhisper(ohp, seed=3).transcribe(pcm, 4)
+    assert np.array_equal(lg, wlg) and np.array_equal(toks, want)
+
+
 def test_whisper_tiny_en_full_size_against_hf(gpu):
     """the HIP ASR engine itself against HF transformers at the tiny.en geometry (whisper_full_tiny_en.npz: sampled log-mel, encoder states,
     first-step logits; 2e-4 of the tensors' scale), without the oracle in between"""
