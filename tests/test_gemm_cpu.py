@@ -29,7 +29,7 @@ def test_blocks_of_float32_products(rows, n, k, swiglu, slabs, want):
 
 @pytest.mark.parametrize("rows,n,k,swiglu,want", [
     (1750, 28672, 4096, 1, (256, 256, 2, 1)), (2047, 4096, 14336, 0, (256, 128, 3, 1)), (1100, 28672, 4096, 1, (128, 128, 2, 1)),
-    (1750, 2048, 8192, 0, (128, 128, 4, 1)), (600, 2048, 8192, 0, (128, 64, 3, 1)), (200, 4096, 14336, 0, (128, 32, 4, 1)), (64, 4096, 4096, 0, (64, 0, 0, 1)),
+    (1750, 2048, 8192, 0, (128, 128, 4, 1)), (600, 2048, 8192, 0, (128, 64, 3, 1)), (200, 4096, 14336, 0, (128, 32, 4, 1)), (2047, 1024, 512, 0, (128, 64, 3, 1)), (1100, 2048, 512, 0, (128, 128, 4, 1)), (64, 4096, 4096, 0, (64, 0, 0, 1)),
 ])
 def test_blocks_of_bf16_products(rows, n, k, swiglu, want):
     assert image_form(0, rows, n, k, swiglu) == want

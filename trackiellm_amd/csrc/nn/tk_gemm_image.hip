@@ -280,9 +280,9 @@ __global__ void k_put_image(const void* src, int src_f32, int64_t N, int64_t K, 
     tk_img_put(img, row, (int)k0 + k, ktiles, v);
 }
 
-/* The forms of the wide kernel and what they cost, fitted to products of 100 .. 2047 rows whose weights come from memory.  Large blocks where they fill the
- * chip once or several times, smaller ones where larger would leave CUs idle.
- * bf16 (within ~15 %): rounds of workgroups x (their start and end + k x time per k).  Of forms that run two to a CU a last round of at most 256 runs one
+/* The forms of the wide kernel and what they cost, fitted to products of 100 .. 2047 rows and k = 256 .. 14336
+ * whose weights come from memory.  Large blocks where they fill the chip once or several times, smaller ones where larger would leave CUs idle.
+ * bf16 (the choice costs 0.4 % on average over the best one; 171 products): rounds of workgroups x (their start and end + k x time per k).  Of forms that run two to a CU a last round of at most 256 runs one
  * to a CU.
  * f32 (within 11 %): four MFMAs for 16 k where bf16 takes one for 32, so the matrix pipe is all there is, two workgroups of a CU take twice the time, and
  * what counts is the blocks of the fullest CU: the first one's start and end once, + per further one, + k x time per k each. */
@@ -297,13 +297,13 @@ constexpr WideForm wide_forms[] = {
     /* bf16 2047 x 4096 x 14336: 182 us (242); f32 256 x 16384 x 2048: as the next two, 0.25 us */
     {16, 8, 3, 1, 8.0f, 12.0f, 0.0f, 0.0f, 12.0f, 6.0f, 115.7f},
     /* bf16 1100 x 28672 x 4096: 248 us (271); f32 1303 x 7552 x 4096: 715 us (256 x 256: 940, which bf16's constants would take) */
-    {8, 8, 2, 2, 6.0f, 11.8f, 8.0f, 15.0f, 9.5f, 0.3f, 58.7f},
+    {8, 8, 2, 2, 3.0f, 11.8f, 6.4f, 14.1f, 9.5f, 0.3f, 58.7f},
     /* bf16 1750 x 2048 x 8192: 68 us (93); f32 900 x 4096 x 14336: 846 us (873) */
-    {8, 8, 4, 1, 10.0f, 7.0f, 0.0f, 0.0f, 9.5f, 4.0f, 58.6f},
+    {8, 8, 4, 1, 4.6f, 7.3f, 0.0f, 0.0f, 9.5f, 4.0f, 58.6f},
     /* bf16 600 x 2048 x 8192: 50 us (64); f32 2047 x 3072 x 2048: 202 us (128 x 128: 251) */
-    {8, 4, 3, 2, 7.0f, 5.5f, 8.0f, 9.6f, 8.5f, 0.5f, 31.2f},
+    {8, 4, 3, 2, 3.4f, 5.3f, 3.8f, 9.8f, 8.5f, 0.5f, 31.2f},
     /* bf16 200 x 4096 x 14336: 61 us (84); f32 1303 x 2048 x 8192: 422 us (128 x 128: 487) */
-    {8, 2, 4, 2, 6.0f, 3.9f, 6.0f, 7.2f, 7.5f, 1.0f, 17.1f},
+    {8, 2, 4, 2, 3.2f, 4.0f, 2.8f, 7.4f, 7.5f, 1.0f, 17.1f},
 };
 float wide_us(const WideForm& w, bool f32, int64_t blocks, float k /* thousands */) {
     if (f32) return w.f32_start + (float)((blocks + 255) / 256 - 1) * w.f32_more + (float)((blocks + 255) / 256) * w.f32_k * k;
