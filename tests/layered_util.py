@@ -206,6 +206,11 @@ def close(got, want, tol):
     return rel_rms(got, want, 1.0 if tol < 1e-3 else 0.9) < tol
 
 
+# width, feed-forward, rows of passes whose products take every block form of the kernel for many rows (held in test_gemm_cpu.py)
+LARGE_PRODUCTS = [(2064, 8190, 901), (2064, 8190, 1303), (1040, 5000, 1100), (1040, 2000, 2047), (528, 1500, 1100), (528, 1500, 300), (528, 700, 81),
+                  (1040, 300, 2047), (1296, 5000, 600), (2576, 300, 2047)]
+
+
 def tokens_for(cfg, n, seed=11):
     return np.random.default_rng(seed).integers(0, cfg["vocab"], n).tolist()
 

@@ -4,6 +4,7 @@ import ctypes as C
 import pytest
 
 import trackiellm_amd as tk
+from layered_util import LARGE_PRODUCTS
 
 
 def image_form(f32, rows, n, k, swiglu=0, experts=0, top=0, slabs=1):
@@ -33,6 +34,18 @@ def test_blocks_of_float32_products(rows, n, k, swiglu, slabs, want):
 ])
 def test_blocks_of_bf16_products(rows, n, k, swiglu, want):
     assert image_form(0, rows, n, k, swiglu) == want
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+def test_sizes_of_the_large_products_reach_every_form(f32):
+    """the sizes that the GPU test takes (q, k, v in one product, then out, gate with up, down)"""
+    plain, swiglu = set(), set()
+    for width, ff, rows in LARGE_PRODUCTS:
+        slabs = min(8, 2048 // rows)
+        plain |= {image_form(f32, rows, 3 * width, width)[:3], image_form(f32, rows, width, width, slabs=slabs)[:3], image_form(f32, rows, width, ff, slabs=slabs)[:3]}
+        swiglu.add(image_form(f32, rows, 2 * ((ff + 15) // 16 * 16), width, 1)[:3])
+    forms = {(256, 256, 2), (256, 128, 3), (128, 128, 2), (128, 128, 4), (128, 64, 3)}
+    assert swiglu == forms and plain == forms | {(128, 32, 4)}
 
 
 @pytest.mark.parametrize("f32,rows,n,k,swiglu,experts,top,want", [

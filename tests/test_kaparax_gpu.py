@@ -414,7 +414,7 @@ def test_trace_runner(cases, tmp_path):
 
 
 @pytest.mark.parametrize("dtype,tol", [("float32", F32), ("bfloat16", 0.007)])
-@pytest.mark.parametrize("width,ff,rows", [(2064, 8190, 901), (2064, 8190, 1303), (1040, 5000, 1100), (1040, 2000, 2047), (528, 1500, 1100), (528, 1500, 300), (528, 700, 81)])
+@pytest.mark.parametrize("width,ff,rows", U.LARGE_PRODUCTS)
 def test_products_in_large_blocks(gpu, width, ff, rows, dtype, tol):
     """passes whose products take 256 x 256, 256 x 128, 128 x 128, 128 x 64 and 128 x 32 blocks, with rows, columns and k that fill none of them, against
     the same rows in passes of 61, which take another kernel (other tests hold that one against the restatement).  bf16: where a sum rounds to the other

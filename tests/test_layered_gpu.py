@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import layered_util as U
+from test_gemm_cpu import image_form
 from layered_util import BF16, F32, LO, Case, attention, close, config, delta, dense, greedy, layer, moe, no_end, runner_ids, tokens_for
 
 pytestmark = pytest.mark.gpu
@@ -351,6 +352,40 @@ def test_more_rows_than_a_pass_holds(gpu, tmp_path):
     parts = U.feed(s, 1, toks, [700, 1, 2, 997, 600])
     assert close(whole, parts, F32)
     assert close(whole[:200], c.want(toks[:200])[0], F32)
+
+
+@pytest.mark.parametrize("dtype,experts,top,rows,width,ff,up,down", [
+    ("bfloat16", 2, 1, 301, 80, 40, (128, 64, 3), (128, 32, 4)),
+    ("bfloat16", 3, 2, 2047, 80, 264, (128, 128, 2), (128, 32, 4)),
+    ("bfloat16", 3, 2, 2047, 272, 264, (128, 128, 2), (128, 64, 3)),
+    ("bfloat16", 3, 2, 2047, 528, 264, (128, 128, 4), (128, 128, 2)),
+    ("bfloat16", 3, 2, 2047, 528, 520, (128, 128, 2), (128, 128, 4)),
+    ("float32", 2, 1, 301, 80, 40, (128, 64, 3), (128, 32, 4)),
+    ("float32", 3, 2, 2047, 272, 40, (128, 64, 3), (128, 64, 3)),
+    ("float32", 3, 2, 2047, 144, 264, (128, 128, 4), (128, 32, 4)),
+    ("float32", 6, 3, 2047, 1040, 40, (128, 64, 3), (128, 128, 2)),
+    ("float32", 6, 3, 2047, 528, 136, (128, 64, 3), (128, 128, 4)),
+    ("float32", 6, 3, 2047, 80, 520, (128, 128, 2), (128, 32, 4)),
+])
+def test_experts_in_large_blocks(gpu, tmp_path, dtype, experts, top, rows, width, ff, up, down):
+    """every form of the expert products over many rows: ragged row blocks of one to eight tiles, columns and k that fill no block, against the same rows in
+    passes of 61, which take another kernel (other tests hold that one against the restatement).  The router reads dimensions that hold the token's choice
+    with gaps of 2 and that nothing else writes, so no rounding changes it.  bf16: as for the dense products"""
+    form = lambda n, k, swiglu: image_form(dtype == "float32", rows, n, k, swiglu, experts, top)[:3]
+    assert (form(2 * ((ff + 15) // 16 * 16), width, 1), form(width, ff, 0)) == (up, down)
+    cfg = config(width, 97, [layer(attention(1, 1, 8, 8, 4, 9, 1), delta(1, 1, 8, 8, 2), moe(ff, experts, top), 0.01, 0.0)])
+    w, rng = U.random_weights(cfg, ff), np.random.default_rng(rows)
+    w["embed"][:, :experts] = -4.0
+    for t in range(97):
+        w["embed"][t, rng.permutation(experts)[:top]] = 2.0 * np.arange(top)
+    w["l0.norm1"][:experts] = 0.0
+    w["l0.mlp.router"] = 0 * w["l0.mlp.router"]
+    w["l0.mlp.router"][:, :experts] = np.eye(experts)
+    s = Case(gpu, tmp_path, cfg, w=w).session(dtype, 2, 2048)
+    toks = tokens_for(cfg, rows, 5)
+    whole = s.forward_streams([0] * rows, range(rows), toks)[0]
+    parts = [s.forward_streams([1] * len(toks[i:i + 61]), range(i, i + len(toks[i:i + 61])), toks[i:i + 61])[0] for i in range(0, rows, 61)]
+    assert U.rel_rms(whole, np.concatenate(parts)) < (F32 if dtype == "float32" else 0.007)
 
 
 # ---- generation ----
