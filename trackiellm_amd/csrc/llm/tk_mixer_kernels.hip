@@ -992,7 +992,7 @@ __global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t,
  * meet in LDS, every wave adds them up (ascending) and goes on; those of the output are added a chunk later, off the chain.  Operands are requested
  * three chunks ahead.
  * The zeros of T and B must not meet an infinity or NaN, which would reach the tokens before its own.  A test per chunk cost 18 us on top of the 108, so a
- * second launch (AGAIN, 2 us) looks at the states that the first has left, where what is not finite stays (0 x infinity is NaN): it walks columns that
+ * second launch (AGAIN, 5 us) looks at the states that the first has left, where what is not finite stays (0 x infinity is NaN): it walks columns that
  * have any once more, without those zeros, and leaves at once otherwise. */
 template <int DP, bool AGAIN>
 __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t) {

@@ -140,8 +140,9 @@ template <int N> __device__ __forceinline__ void wait_vm() { __builtin_amdgcn_s_
  * A block of R x C reads (R + C) k operands for R C k products, so large blocks are what the L2s can feed; a wave of MW x NW tiles takes (MW + NW) KiB of
  * LDS for MW NW MFMAs.  What is left is latency: all waves of a CU meet at the same barrier, and whatever stands between it and the next MFMA is lost
  * by all of them.  So a k tile's operands are read while the tile before it is multiplied, the requests for a later stage are spread between MFMAs, and
- * the loop over them has no branch.  2048 x 28672 x 4096 (gate | up): 502 us with 128 x 128 blocks read and multiplied in turn, 414 us with 256 x 256
- * ones, 382 us (1.26 PF/s) with the reads and requests between the MFMAs; 2047 x 4096 x 14336 (down): 214 -> 180 us (1.33 PF/s). */
+ * the loop over them has no branch.  2047 x 28672 x 4096 (gate | up), launches in a row with weights from memory: 494 us with 128 x 128 blocks read and
+ * multiplied in turn, 414 with 256 x 256 ones, 379 (1.27 PF/s; 390 - 412 inside a prompt) with the reads and requests between the MFMAs;
+ * 2047 x 4096 x 14336 (down): 239 -> 190 us (1.27 PF/s).  Experts (the grouped form), 2047 rows to 8 of 64, 2048 x 2048: 254 -> 243 us. */
 constexpr int wide_stage(int mbt, int nbt) { return (mbt + nbt) * 2048; }
 template <typename T, int MBT, int NBT, int WM, int WN, int RING, bool SWIGLU, bool GROUPED>
 __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wide(TkImgGemm a, int nblk_n, int nblk_m, int ks) {

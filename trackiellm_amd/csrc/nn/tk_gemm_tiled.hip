@@ -41,9 +41,11 @@ __device__ __forceinline__ float tw_act(float v, int act) {
  * What bounds few rows: the chain, 8 cycles a k and M-tile, as long as weights and operands are there in time.  One LDS read takes a wave about 130
  * cycles, so operands are read one pair of tiles ahead, also across the chunks of 32 k.  With a ring the compiler cannot count what is in flight
  * behind the staging and lets the first weights of every PF chunks wait for all requests; where the activations of the whole K range fit the LDS
- * (ONE: up to 2048 k at one M-tile, 1024 at two) there is no staging in the loop, and 8 pieces of weights stay in flight.
- * Cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us, 384 x 1536 13.9 -> 10.2, 51872 x 384 24.0 -> 22.0; at 32 rows 8.6 -> 7.9, 20.8 -> 18.9
- * (ring), 30.0 -> 27.0.  Twelve pieces: 384 x 384 at 1 row 5.6 (a wave's requests queue in front of the activations of the others). */
+ * (ONE: multiples of 128 k, up to 2048 at one M-tile, 1024 at two) there is no staging in the loop, and four pieces of weights stay in flight, eight
+ * where k is a multiple of 256 from 512 on.
+ * Cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us and 51872 x 384 24.0 -> 22.0 with four, 384 x 1536 13.9 -> 10.2 with eight; at 32 rows
+ * 8.6 -> 7.9, 30.0 -> 27.0 with four, 20.8 -> 18.9 (ring).  Twelve pieces: 384 x 384 at 1 row 5.6 (a wave's requests queue in front of the activations
+ * of the others). */
 template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */>
 __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, int total_row_tiles, int rk /* k per ring slot */, int slot_bytes /* ring slot pitch */) {
     constexpr int LPC = WB == 4 ? 2 : 1; /* 16-byte requests per piece and lane */

@@ -303,8 +303,7 @@ __global__ void k_yolo_decode_out(const float* out, int nc, int n_anchors, float
 
 /* rank of every candidate among the candidates: (score desc, anchor asc); the best MAX_CAND are kept.  Most anchors fall below the
  * confidence threshold, so each 1024-anchor tile is compacted in LDS first (ballot + prefix) and only its survivors are compared.  A tile's scores are
- * requested under the tile before, survivors are read
- * eight at a time: 8400 anchors 41 -> 22 us. */
+ * requested under the tile before, survivors are read eight at a time: 8400 anchors 41 -> 22 us. */
 __global__ __launch_bounds__(256) void k_yolo_rank(const tk_yolo_cand_t* cand, int n_anchors, int32_t* order, int32_t* n_cand) {
     const int b = blockIdx.y;
     const tk_yolo_cand_t* cb = cand + (size_t)b * n_anchors;
