@@ -389,6 +389,20 @@ def _policy_geometry():
     return O.WhisperHP(80, 50, 64, 2, 2, 64, 64, 2, 2, 512)
 
 
+@pytest.mark.parametrize("vocab", [1023, 1024, 1025, 8192, 8193])
+def test_token_picks_by_vocabulary(gpu, vocab):
+    """a value a thread, one more, and around the eight that are read together: picks and their log-probabilities"""
+    ohp = _policy_geometry()
+    ohp.n_vocab = vocab
+    asr, orc = gpu.Asr(hp=hp_of(gpu, ohp), seed=6, max_batch=2), O.OracleWhisper(ohp, seed=6)
+    pcm = np.clip(np.random.default_rng(vocab).normal(0, 3000, (2, 9000)), -32768, 32767).astype(np.int16)
+    assert np.array_equal(asr.transcribe_tokens(pcm, 6)[0], orc.transcribe(pcm, 6)[0])
+    for temp in (0.0, 0.8):
+        toks, lp = asr.transcribe_policy(pcm, 6, temp, 3)
+        wt, wlp = orc.transcribe_policy(pcm, 6, temp, 3)
+        assert np.array_equal(toks, wt) and np.array_equal(lp.view(np.uint32), wlp.view(np.uint32))
+
+
 def test_asr_decode_policy_tokens_and_logprobs_bit_exact(gpu):
     """whisper.cpp's per-step bookkeeping (the reference arms its policy: tk_asr_whisper.c:126-138): tokens picked by temperature and their
     log-probabilities, device against oracle, bit for bit; temperature 0 is the greedy decode"""
