@@ -74,6 +74,32 @@ TK_HD float tk_fabsf(float x) { return tk_bits_f32(tk_f32_bits(x) & 0x7fffffffu)
 TK_HD float tk_fmaxf(float a, float b) { return a > b ? a : b; }
 TK_HD float tk_fminf(float a, float b) { return a < b ? a : b; }
 
+/*
+ * Device forms of exp, sigmoid and tanh: the same values in fewer instructions, without branches.  fp32 MFMAs and vector instructions take turns on a
+ * SIMD (gfx950: a wave of 16 x 16 x 4 MFMAs and a wave of fmas together take the sum of their times), so an epilogue's activation is time that the products wait.
+ *   2^n by ldexp instead of two multiplications; a round to integer instead of the magic sum (|x| < 2^22: the same);
+ *   1 / d and 2 / d for 1 <= d <= 2^126 by v_rcp_f32 and one residual (correctly rounded) instead of the general division; beyond, where 1 / d is subnormal, the
+ *   division as before.
+ * Bit for bit the host forms: exp, sigmoid, SiLU, tanh and GELU were compared over all 2^32 inputs.  SiLU 42 -> 22 vector instructions, GELU 50 -> 30:
+ * products of 204 800 x 64 x 64 with SiLU 35.4 -> 31.9 us, 819 200 x 32 x 32 48.3 -> 41.1, convolutions 204 800 x 80 x 720 265 -> 260.
+ */
+#if defined(__HIP_DEVICE_COMPILE__)
+TK_HD float tk_expf(float x) {
+    const float c = x > 88.0f ? 88.0f : x; /* NaN stays */
+    const float n = __builtin_rintf(c * 1.44269504088896341f);
+    float r = tk_fmaf(-n, 0.693145751953125f, c);
+    r = tk_fmaf(-n, 1.42860682030941723e-6f, r);
+    float p = 1.0f / 720.0f;
+    p = tk_fmaf(p, r, 1.0f / 120.0f);
+    p = tk_fmaf(p, r, 1.0f / 24.0f);
+    p = tk_fmaf(p, r, 1.0f / 6.0f);
+    p = tk_fmaf(p, r, 0.5f);
+    p = tk_fmaf(p, r, 1.0f);
+    p = tk_fmaf(p, r, 1.0f);
+    const float e = __builtin_ldexpf(p, (int32_t)n);
+    return x < -87.0f ? 0.0f : e;
+}
+#else
 /* exp(x): Cody-Waite reduction + degree-6 polynomial, <= 1 ulp on [-87, 88]. */
 TK_HD float tk_expf(float x) {
     if (x > 88.0f) x = 88.0f;
@@ -98,6 +124,7 @@ TK_HD float tk_expf(float x) {
     float s2 = tk_bits_f32((uint32_t)(n2 + 127) << 23);
     return (p * s1) * s2;
 }
+#endif
 
 /* natural log for x > 0 (normal range): x = m * 2^e, m in [sqrt(.5), sqrt(2)) */
 TK_HD float tk_logf(float x) {
@@ -124,13 +151,47 @@ TK_HD float tk_logf(float x) {
 
 TK_HD float tk_log10f(float x) { return tk_logf(x) * 0.434294481903251828f; }
 
-TK_HD float tk_sigmoidf(float x) { return tk_divf(1.0f, 1.0f + tk_expf(-x)); }
+TK_HD float tk_sigmoidf(float x) {
+    const float d = 1.0f + tk_expf(-x);
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float r = __builtin_amdgcn_rcpf(d);
+    float q = tk_fmaf(tk_fmaf(-d, r, 1.0f), r, r);
+    if (__builtin_expect(d > 8.50705917e37f /* 2^126 */, 0)) q = tk_divf(1.0f, d);
+    return q;
+#else
+    return tk_divf(1.0f, d);
+#endif
+}
 TK_HD float tk_siluf(float x) { return x * tk_sigmoidf(x); }
+#if defined(__HIPCC__)
+/* SiLU of N values at a time: one test for all of them, their chains side by side */
+template <int N> __device__ __forceinline__ void tk_silu_all(float* v) {
+    float d[N], q[N], top = 0.0f;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        d[i] = 1.0f + tk_expf(-v[i]);
+        const float r = __builtin_amdgcn_rcpf(d[i]);
+        q[i] = tk_fmaf(tk_fmaf(-d[i], r, 1.0f), r, r);
+        top = __builtin_fmaxf(top, d[i]);
+    }
+    if (__builtin_expect(top > 8.50705917e37f, 0)) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = tk_divf(1.0f, d[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = v[i] * q[i];
+}
+#endif
 
 TK_HD float tk_tanhf(float x) {
     /* tanh(x) = 1 - 2/(exp(2x)+1); saturates cleanly through tk_expf's clamps */
-    float e = tk_expf(2.0f * x);
-    return 1.0f - tk_divf(2.0f, e + 1.0f);
+    const float d = tk_expf(2.0f * x) + 1.0f;
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float r = __builtin_amdgcn_rcpf(d), q = 2.0f * r;
+    return 1.0f - tk_fmaf(tk_fmaf(-d, q, 2.0f), r, q);
+#else
+    return 1.0f - tk_divf(2.0f, d);
+#endif
 }
 
 /* GELU, tanh form (the form ggml/whisper.cpp evaluates) */

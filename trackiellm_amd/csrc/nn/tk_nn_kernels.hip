@@ -155,8 +155,12 @@ __device__ __forceinline__ void store_tile(const TkGemm& g, const v16f& acc, flo
 #pragma unroll
     for (int r = 0; r < 16; ++r) v[r] = v[r] + bias;
     if (g.act == TK_ACT_SILU) {
+        if (FASTACT) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) v[r] = FASTACT ? v[r] * fast_sigmoidf(v[r]) : tk_siluf(v[r]);
+            for (int r = 0; r < 16; ++r) v[r] = v[r] * fast_sigmoidf(v[r]);
+        } else {
+            tk_silu_all<16>(v);
+        }
     } else if (g.act == TK_ACT_GELU) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) v[r] = FASTACT ? fast_geluf(v[r]) : tk_geluf(v[r]);
@@ -626,7 +630,12 @@ __global__ __launch_bounds__(256) void k_gemm_f32_t16(TkGemm g) {
                 for (int r = 0; r < 4; ++r) v[r] = v[r] * g.alpha;
             }
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r] + bias, g.act);
+            for (int r = 0; r < 4; ++r) v[r] = v[r] + bias;
+            if (g.act == TK_ACT_SILU) tk_silu_all<4>(v);
+            else if (g.act != TK_ACT_NONE) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = apply_act(v[r], g.act);
+            }
 #pragma unroll
             for (int r = 0; r < 4; ++r)
                 if (row + r < g.M) {
