@@ -257,6 +257,12 @@ TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_f32(int device, int form, int
 /* the form that such a product takes by itself, `batch` of them side by side, and the rows and columns of its block.  No GPU involved. */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_f32_form(int M, int N, int K, int lda, int ldb, int batch, const int conv[9], int* form, int block[2]);
 
+/* test hook for the direct convolution (csrc/nn/tk_conv_direct.h): shape = {B, H, W, C, channels of the first source, its pitch, whether it is upsampled, the second's pitch
+ * (0: one source), whether that is, kernel, stride, N, pitch of y, pitch of the residual, act (0 none, 1 SiLU)}; cut = {tiles a wave, waves along pixels, along
+ * channels, rows, columns of a tile} or NULL for its own choice, which is stored in used[5] (may be NULL).  w [N][kernel^2 C] in k order. */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_conv_direct(int device, const int shape[15], const int* cut, const float* x0, const float* x1, const float* w, const float* bias,
+                                                          const float* residual, float* y, int* used);
+
 /* test hook: the blocks that a product of the layer-list decoders is cut into (csrc/nn/tk_gemm_image.h): rows x K against N x K, operands f32 or bf16;
  * swiglu: N = gate and up rows together; experts > 0: every row goes to `top` of them; max_slabs: parts of k at most.  form = rows, columns and LDS
  * stages of a block, parts of k; stages = 0: the kernel for few rows.  No GPU involved. */

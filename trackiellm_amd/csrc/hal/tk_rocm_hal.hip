@@ -14,6 +14,7 @@
 #include "tk/tk_rocm_hal.h"
 #include "../nn/tk_gemm_image.h"
 #include "../nn/tk_gemm_tiled.h"
+#include "../nn/tk_conv_direct.h"
 #include "../nn/tk_nn_kernels.h"
 
 struct tk_gpu_buffer_s {
@@ -213,6 +214,45 @@ tk_error_code_t tk_mi355x_gemm_f32_form(int M, int N, int K, int lda, int ldb, i
     g.batch = batch; g.sA = (int64_t)M * lda; g.sB = (int64_t)N * ldb; g.sC = (int64_t)M * N;
     *form = tk_gemm_f32_form(g, block);
     return TK_SUCCESS;
+}
+
+tk_error_code_t tk_mi355x_conv_direct(int device, const int shape[15], const int* cut, const float* x0, const float* x1, const float* w, const float* bias, const float* residual,
+                                      float* y, int* used) {
+    if (!shape || !x0 || !w || !y) return TK_ERROR_INVALID_ARGUMENT;
+    for (int i = 0; i < 15; ++i)
+        if (shape[i] < 0 || shape[i] > 16384) return TK_ERROR_INVALID_ARGUMENT;
+    TkConvDirect c{};
+    c.B = shape[0]; c.H = shape[1]; c.W = shape[2]; c.C = shape[3]; c.c_split = shape[7] > 0 ? shape[4] : c.C;
+    c.k = shape[9]; c.stride = shape[10]; c.pad = c.k / 2; c.N = shape[11]; c.ldy = shape[12]; c.ldr = shape[13]; c.act = shape[14];
+    if (c.stride < 1 || c.H < 1 || c.W < 1 || c.B < 1 || c.C < 16 || c.N < 1 || c.c_split > c.C || c.ldy < c.N || (residual && c.ldr < c.N) || (c.c_split < c.C && !x1) ||
+        shape[5] < c.c_split || (c.c_split < c.C && shape[7] < c.C - c.c_split) || shape[6] > 1 || shape[8] > 1)
+        return TK_ERROR_INVALID_ARGUMENT;
+    c.Ho = (c.H + 2 * c.pad - c.k) / c.stride + 1; c.Wo = (c.W + 2 * c.pad - c.k) / c.stride + 1;
+    const size_t pixels = (size_t)c.B * c.H * c.W, outs = (size_t)c.B * c.Ho * c.Wo, K = (size_t)c.k * c.k * c.C;
+    const size_t n0 = (pixels >> (2 * shape[6])) * shape[5], n1 = c.c_split < c.C ? (pixels >> (2 * shape[8])) * shape[7] : 0;
+    c.src[0] = TkConvSource{x0, shape[5], shape[6]}; c.src[1] = TkConvSource{x1, shape[7], shape[8]};
+    int n = 0;
+    if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return TK_ERROR_GPU_DEVICE_NOT_FOUND;
+    if (device < 0 || device >= n || hipSetDevice(device) != hipSuccess) return TK_ERROR_INVALID_ARGUMENT;
+    float *d0 = nullptr, *d1 = nullptr, *dw = nullptr, *dp = nullptr, *db = nullptr, *dr = nullptr, *dy = nullptr;
+    auto put = [](float** d, const float* h, size_t n) { return hipMalloc((void**)d, n * 4) == hipSuccess && hipMemcpy(*d, h, n * 4, hipMemcpyHostToDevice) == hipSuccess; };
+    bool ok = put(&d0, x0, n0) && (n1 == 0 || put(&d1, x1, n1)) && put(&dw, w, K * c.N) && (!bias || put(&db, bias, c.N)) && (!residual || put(&dr, residual, outs * c.ldr)) &&
+              put(&dy, y, outs * c.ldy) && hipMalloc((void**)&dp, tk_conv_weight_floats(c.N, (int)K) * 4) == hipSuccess;
+    bool fits = true;
+    if (ok) {
+        c.src[0].p = d0; c.src[1].p = d1; c.w = dp; c.bias = db; c.residual = dr; c.y = dy;
+        TkConvPlan plan{};
+        if (cut) plan = TkConvPlan{cut[0], cut[1], cut[2], cut[3], cut[4]};
+        fits = tk_conv_direct_takes(c) && (cut || tk_conv_direct_plan(c, &plan)) && tk_conv_plan_ok(c, plan);
+        if (fits) {
+            tk_launch_conv_weights(dw, c.N, (int)K, dp, nullptr);
+            ok = tk_launch_conv_direct(c, plan, nullptr) && hipGetLastError() == hipSuccess && hipMemcpy(y, dy, outs * c.ldy * 4, hipMemcpyDeviceToHost) == hipSuccess;
+            if (used) { used[0] = plan.mt; used[1] = plan.wm; used[2] = plan.wn; used[3] = plan.th; used[4] = plan.tw; }
+        }
+    }
+    float* ptrs[] = {d0, d1, dw, dp, db, dr, dy};
+    for (float* q : ptrs) if (q) (void)hipFree(q);
+    return !fits ? TK_ERROR_INVALID_ARGUMENT : ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
 }
 
 tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]) {

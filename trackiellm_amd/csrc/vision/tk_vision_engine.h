@@ -17,6 +17,7 @@
 #include "../common/tk_ggml_blocks.h"
 #include "../common/tk_yolo_post.h"
 #include "../common/tk_yolov8n_graph.h"
+#include "../nn/tk_conv_direct.h"
 #include "../nn/tk_onnx_exec.h"
 
 struct TkPreprocessArgs {
@@ -39,6 +40,7 @@ public:
     int device = 0, nc = TK_YOLO_NC;
     std::vector<TkConvSpec> specs;
     std::vector<float*> w, b; /* device: [cout][k*k*cin], [cout] */
+    std::vector<float*> wp;   /* device: the weights as pieces (tk_conv_direct.h) of the layers that have whole ones, null else */
     std::string error;
     ~TkYoloModel();
     bool init(int device, int nc);
@@ -101,6 +103,7 @@ private:
     float* col = nullptr;
     size_t col_floats = 0;
     TkT heads[3];
+    std::vector<std::vector<TkConvPlan>> plans; /* [B][layer] of the direct convolutions (mt == 0: not made yet); at most max_batch + 1 rows */
     tk_yolo_cand_t* cand = nullptr;     /* [B][n_anchors] decoded */
     int32_t* order = nullptr;           /* [B][MAX_CAND] anchor ids, sorted */
     int32_t* n_cand = nullptr;          /* [B] */
