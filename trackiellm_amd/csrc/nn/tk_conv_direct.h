@@ -52,6 +52,11 @@ bool tk_conv_direct_plan(const TkConvDirect& c, TkConvPlan* plan);
 bool tk_conv_plan_ok(const TkConvDirect& c, const TkConvPlan& plan);
 bool tk_launch_conv_direct(const TkConvDirect& c, const TkConvPlan& plan, hipStream_t s);
 
+/* up to TK_CONV_SET convolutions of one batch size that do not depend on each other, in one launch (cuts with the same tiles a wave and number of waves) */
+enum { TK_CONV_SET = 6 };
+bool tk_conv_direct_plan_set(const TkConvDirect* c, int n, TkConvPlan* plans);
+bool tk_launch_conv_direct_set(const TkConvDirect* c, const TkConvPlan* plans, int n, hipStream_t s);
+
 /* [N][K] row-major weights (device) -> pieces; K = k k C, a multiple of 16 */
 size_t tk_conv_weight_floats(int N, int K);
 void tk_launch_conv_weights(const float* w, int N, int K, float* pieces, hipStream_t s);

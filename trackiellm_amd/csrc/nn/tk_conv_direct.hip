@@ -25,7 +25,14 @@ struct CdArgs {
     int wn, th, tw, pw, ph;      /* waves along channels; tile; patch */
     int tiles_x, tiles;          /* spatial tiles of a row, of an image */
     int cp4;                     /* float4 of a pixel in the LDS: C / 4 + 1 */
-    uint32_t by_c4[2], by_pw, by_tw, by_wn, by_cj; /* cd_div() of a source's float4 of a pixel, ... */
+    uint32_t by_c4[2], by_pw, by_tw, by_wn, by_cj, by_tiles_x; /* cd_div() of a source's float4 of a pixel, ... */
+};
+
+/* up to P convolutions of one batch in a launch: block x counts through the (tile, channel group) pairs of the first, then of the second, ... */
+template <int P> struct CdSet {
+    int n, first[P];
+    uint32_t by_tiles[P];
+    CdArgs a[P];
 };
 
 template <int V> struct CdCount { static constexpr int value = V; };
@@ -36,17 +43,22 @@ template <int V> struct CdCount { static constexpr int value = V; };
  * instructions share: 71 % of it at 80 x 80 x 64 x 32 frames (139 us; the GEMM kernels 162), 57 % at 40 x 40 (43 us; 54), where patches and epilogues are a larger part.
  * Weights come from the L2 once per tile of pixels, operands from the LDS: a padding of 16 bytes a pixel turns 16 pixels into 16 different groups of banks.
  */
-template <int MT /* 16-pixel tiles a wave */, int PF /* pieces of weights in flight */, int RD /* operand sets, divides PF: read RD - 1 groups ahead */>
-__global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdArgs a) {
+template <int P, int MT /* 16-pixel tiles a wave */, int PF /* pieces of weights in flight */, int RD /* operand sets, divides PF: read RD - 1 groups ahead */>
+__global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdSet<P> set) {
     extern __shared__ __attribute__((aligned(16))) float cd_lds[];
+    int pi = 0;
+#pragma unroll
+    for (int i = 1; i < P; ++i) pi += i < set.n && (int)blockIdx.x >= set.first[i] ? 1 : 0;
+    const CdArgs& a = set.a[pi];
+    const int local = (int)blockIdx.x - set.first[pi], by = cd_quot(local, set.by_tiles[pi]), bx = local - by * a.tiles;
     const TkConvDirect& c = a.c;
     const int tid = threadIdx.x, nthreads = blockDim.x, lane = tid & 63, r = lane & 15, g = lane >> 4;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = cd_quot(wave, a.by_wn), wn = wave - wm * a.wn;
-    const int b = blockIdx.z, ty = blockIdx.x / a.tiles_x, tx = blockIdx.x - ty * a.tiles_x;
+    const int b = blockIdx.z, ty = cd_quot(bx, a.by_tiles_x), tx = bx - ty * a.tiles_x;
     const int oy0 = ty * a.th, ox0 = tx * a.tw;
     const int cj = c.C >> 4, G = c.k * c.k * cj; /* 16-k groups: of a tap, in all */
-    const int ntile = blockIdx.y * a.wn + wn;
+    const int ntile = by * a.wn + wn;
     const bool active = ntile * 16 < c.N;
 
     /* the first weights travel under the patch; requests past the chain read what lies behind it (tk_conv_weight_floats) */
@@ -70,7 +82,7 @@ __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdArgs a) 
             const int c4 = (si == 0 ? c.c_split : c.C - c.c_split) >> 2, total = a.ph * a.pw * c4, sh = s.shift;
             const int hs = c.H >> sh, ws = c.W >> sh, H = c.H, W = c.W, pw = a.pw, cp4 = a.cp4;
             const uint32_t ld = (uint32_t)s.ld, by_pw = a.by_pw;
-            const uint32_t by = a.by_c4[si];
+            const uint32_t by_c4 = a.by_c4[si];
             const float* image = s.p + (int64_t)b * hs * ws * s.ld;
             float* to = cd_lds + (si == 0 ? 0 : c.c_split);
             auto batch = [&](auto count, int e0) { /* past the end: the last float4 again */
@@ -81,7 +93,7 @@ __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdArgs a) 
                 for (int u = 0; u < U; ++u) {
                     int e = e0 + u * nthreads + tid;
                     e = e < total ? e : total - 1;
-                    const int pix = cd_quot(e, by), q = e - __mul24(pix, c4);
+                    const int pix = cd_quot(e, by_c4), q = e - __mul24(pix, c4);
                     const int py = cd_quot(pix, by_pw), px = pix - __mul24(py, pw);
                     const int iy = iy0 + py, ix = ix0 + px;
                     const bool in = (int)((uint32_t)iy < (uint32_t)H) & (int)((uint32_t)ix < (uint32_t)W);
@@ -220,7 +232,9 @@ static bool cd_fill(const TkConvDirect& c, const TkConvPlan& p, CdArgs* a) {
     a->cp4 = c.C / 4 + 1;
     /* (a patch has fewer than 10240 float4, a divisor is at most 10240) */
     a->by_c4[0] = cd_div(c.c_split / 4); a->by_c4[1] = cd_div(c.c_split < c.C ? (c.C - c.c_split) / 4 : 1);
-    a->by_pw = cd_div(a->pw); a->by_tw = cd_div(p.tw); a->by_wn = cd_div(p.wn); a->by_cj = cd_div(c.C / 16);
+    a->by_pw = cd_div(a->pw); a->by_tw = cd_div(p.tw); a->by_wn = cd_div(p.wn); a->by_cj = cd_div(c.C / 16); a->by_tiles_x = cd_div(a->tiles_x);
+    /* pairs of tile and channel group: their quotients by the tiles too */
+    if ((int64_t)a->tiles * ((c.N + 15) / 16) * a->tiles >= 0x7fffffff) return false;
     return cd_lds_bytes(c, a->ph, a->pw) <= TK_CD_LDS;
 }
 bool tk_conv_plan_ok(const TkConvDirect& c, const TkConvPlan& plan) {
@@ -231,7 +245,7 @@ bool tk_conv_plan_ok(const TkConvDirect& c, const TkConvPlan& plan) {
 /* Costs in cycles, fitted to 18 000 launches (the detector's 3 x 3 layers at 1, 3, 8 and 32 frames, every cut): the choice takes 1.4 % more than the best cut in the
  * mean, 15 % at most.  A workgroup's latency is its patch, its chains (32 cycles an MFMA) and its epilogue; the CU's further ones take turns on the pipe, which their
  * vector instructions share.  Five, six or seven waves load the SIMDs unevenly (64 -> 80 channels, 32 frames: 247 us with five, 190 with four). */
-bool tk_conv_direct_plan(const TkConvDirect& c, TkConvPlan* plan) {
+static float cd_plan(const TkConvDirect& c, int only_mt, int only_waves, TkConvPlan* plan) {
     const int ntiles = (c.N + 15) / 16;
     const float G = (float)(c.k * c.k * c.C / 16);
     float best = 3e38f;
@@ -241,8 +255,9 @@ bool tk_conv_direct_plan(const TkConvDirect& c, TkConvPlan* plan) {
         if (wn > ntiles) break;
         for (int wm = 1; wm * wn <= TK_CD_MAX_WAVES; wm *= 2) {
             const int w = wm * wn;
-            if ((w > 4 && w < 8) || (w < 2 && ntiles > 1)) continue;
+            if ((w > 4 && w < 8) || (w < 2 && ntiles > 1) || (only_waves && w != only_waves)) continue;
             for (int mt : mts) {
+                if (only_mt && mt != only_mt) continue;
                 const int rows = 16 * mt * wm;
                 for (int tw0 : widths) {
                     const int tw = tw0 < c.Wo ? tw0 : c.Wo;
@@ -264,6 +279,21 @@ bool tk_conv_direct_plan(const TkConvDirect& c, TkConvPlan* plan) {
             }
         }
     }
+    return best;
+}
+bool tk_conv_direct_plan(const TkConvDirect& c, TkConvPlan* plan) { return cd_plan(c, 0, 0, plan) < 3e38f; }
+/* one form for all: four waves, the tiles a wave that cost least in the sum */
+bool tk_conv_direct_plan_set(const TkConvDirect* c, int n, TkConvPlan* plans) {
+    float best = 3e38f;
+    for (int mt = 1; mt <= 4; mt *= 2) {
+        TkConvPlan p[TK_CONV_SET];
+        float sum = 0.0f;
+        for (int i = 0; i < n && i < TK_CONV_SET; ++i) sum += cd_plan(c[i], mt, 4, &p[i]);
+        if (sum < best) {
+            best = sum;
+            for (int i = 0; i < n && i < TK_CONV_SET; ++i) plans[i] = p[i];
+        }
+    }
     return best < 3e38f;
 }
 
@@ -274,23 +304,42 @@ bool tk_conv_direct_prepare_device() {
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
     if (g_cd_opted[dev].load(std::memory_order_acquire)) return true;
     std::lock_guard<std::mutex> lk(g_cd_mu);
-    const void* fns[3] = {(const void*)k_conv_direct<1, 8, 2>, (const void*)k_conv_direct<2, 8, 2>, (const void*)k_conv_direct<4, 4, 2>};
+    const void* fns[6] = {(const void*)k_conv_direct<1, 1, 8, 2>, (const void*)k_conv_direct<1, 2, 8, 2>, (const void*)k_conv_direct<1, 4, 4, 2>,
+                          (const void*)k_conv_direct<TK_CONV_SET, 1, 8, 2>, (const void*)k_conv_direct<TK_CONV_SET, 2, 8, 2>, (const void*)k_conv_direct<TK_CONV_SET, 4, 4, 2>};
     for (const void* f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, TK_CD_LDS) != hipSuccess) return false;
     g_cd_opted[dev].store(true, std::memory_order_release);
     return true;
 }
 
-bool tk_launch_conv_direct(const TkConvDirect& c, const TkConvPlan& p, hipStream_t s) {
-    CdArgs a;
-    if (!tk_conv_direct_takes(c) || !cd_fill(c, p, &a) || !tk_conv_direct_prepare_device()) return false;
-    const int ntiles = (c.N + 15) / 16;
-    const dim3 grid(a.tiles, (ntiles + p.wn - 1) / p.wn, c.B), block(64 * p.wm * p.wn);
-    const size_t lds = (size_t)cd_lds_bytes(c, a.ph, a.pw);
-    switch (p.mt) {
-        case 1: hipLaunchKernelGGL((k_conv_direct<1, 8, 2>), grid, block, lds, s, a); break;
-        case 2: hipLaunchKernelGGL((k_conv_direct<2, 8, 2>), grid, block, lds, s, a); break;
-        default: hipLaunchKernelGGL((k_conv_direct<4, 4, 2>), grid, block, lds, s, a); break;
+template <int P>
+static bool cd_launch(const TkConvDirect* c, const TkConvPlan* p, int n, hipStream_t s) {
+    CdSet<P> set;
+    set.n = n;
+    int blocks = 0;
+    size_t lds = 0;
+    for (int i = 0; i < P; ++i) {
+        const int j = i < n ? i : 0;
+        CdArgs& a = set.a[i];
+        if (!tk_conv_direct_takes(c[j]) || !cd_fill(c[j], p[j], &a) || c[j].B != c[0].B || p[j].mt != p[0].mt || p[j].wm * p[j].wn != p[0].wm * p[0].wn) return false;
+        set.first[i] = blocks;
+        set.by_tiles[i] = cd_div(a.tiles);
+        if (i >= n) continue;
+        blocks += a.tiles * (((c[j].N + 15) / 16 + p[j].wn - 1) / p[j].wn);
+        const size_t l = (size_t)cd_lds_bytes(c[j], a.ph, a.pw);
+        lds = l > lds ? l : lds;
+    }
+    if (!tk_conv_direct_prepare_device()) return false;
+    const dim3 grid(blocks, 1, c[0].B), block(64 * p[0].wm * p[0].wn);
+    switch (p[0].mt) {
+        case 1: hipLaunchKernelGGL((k_conv_direct<P, 1, 8, 2>), grid, block, lds, s, set); break;
+        case 2: hipLaunchKernelGGL((k_conv_direct<P, 2, 8, 2>), grid, block, lds, s, set); break;
+        default: hipLaunchKernelGGL((k_conv_direct<P, 4, 4, 2>), grid, block, lds, s, set); break;
     }
     return true;
+}
+bool tk_launch_conv_direct(const TkConvDirect& c, const TkConvPlan& p, hipStream_t s) { return cd_launch<1>(&c, &p, 1, s); }
+bool tk_launch_conv_direct_set(const TkConvDirect* c, const TkConvPlan* p, int n, hipStream_t s) {
+    if (n < 1 || n > TK_CONV_SET) return false;
+    return n == 1 ? cd_launch<1>(c, p, 1, s) : cd_launch<TK_CONV_SET>(c, p, n, s);
 }

@@ -254,24 +254,61 @@ struct TkGpuOps {
         if (back) c->src[1] = TkConvSource{back->x.p, back->x.ld, back->shift};
         return true;
     }
-    bool direct(const TkT& x, int idx, const TkT& y, const TkT* res) {
+    /* false: not a layer for the direct kernel */
+    bool describe(const TkT& x, int idx, const TkT& y, const TkT* res, TkConvDirect* out) const {
         const TkConvSpec& sp = d->model->specs[idx];
         if (d->fast || !d->model->wp[idx]) return false;
-        TkConvDirect c{};
+        TkConvDirect& c = *out;
+        c = TkConvDirect{};
         if (!sources(x, &c)) return false;
-        /* 1 x 1: the GEMM kernels are as quick or quicker (32 frames, 80 x 80 x 64: 31.9 us, 36.2 here) unless a copy and an upsampling fall away (5 us each and more) */
-        if (sp.k == 1 && c.c_split == x.C) return false;
         c.B = x.B; c.H = x.H; c.W = x.W; c.C = x.C; c.k = sp.k; c.stride = sp.s; c.pad = sp.k / 2; c.Ho = y.H; c.Wo = y.W; c.N = sp.cout;
         c.w = d->model->wp[idx]; c.bias = d->model->b[idx];
         c.residual = res ? res->p : nullptr; c.ldr = res ? res->ld : 0;
         c.y = y.p; c.ldy = y.ld; c.act = sp.act ? TK_ACT_SILU : TK_ACT_NONE;
-        if (!tk_conv_direct_takes(c)) return false;
+        return tk_conv_direct_takes(c);
+    }
+    bool direct(const TkT& x, int idx, const TkT& y, const TkT* res) {
+        TkConvDirect c;
+        if (!describe(x, idx, y, res, &c)) return false;
+        /* 1 x 1: the GEMM kernels are as quick or quicker (32 frames, 80 x 80 x 64: 31.9 us, 36.2 here) unless a copy and an upsampling fall away (5 us each and more) */
+        if (c.k == 1 && c.c_split == x.C) return false;
         TkConvPlan& plan = d->plans[x.B][idx];
         if (plan.mt == 0 && !tk_conv_direct_plan(c, &plan)) { plan.mt = 0; return false; }
         if (res) settle(*res);
         return tk_launch_conv_direct(c, plan, s);
     }
+    /* The last 18 layers are six chains of three, box and class branch of each scale: their first layers in one launch, then the second, then the third.  One frame:
+     * 18 launches of 170 us, now three of 73.  Up to four frames of 80 x 80: at 32 each layer fills the chip, and in one launch the largest patch (256 channels) would
+     * set how many workgroups a CU holds (1055 us for the first layers, 676 one by one). */
+    struct Layer { TkT x, y; int idx; };
+    std::vector<Layer> heads[3];
+    bool defer(const TkT& x, int idx, const TkT& y, const TkT* res) {
+        const int at = idx - ((int)d->model->specs.size() - 18);
+        if (at < 0 || res) return false;
+        heads[at % 3].push_back(Layer{x, y, idx});
+        if (at == 17) {
+            for (auto& stage : heads) {
+                TkConvDirect c[TK_CONV_SET];
+                bool ok = stage.size() == TK_CONV_SET;
+                for (size_t i = 0; ok && i < stage.size(); ++i) ok = describe(stage[i].x, stage[i].idx, stage[i].y, nullptr, &c[i]);
+                ok = ok && (int64_t)c[0].B * c[0].H * c[0].W <= 4 * 6400;
+                TkConvPlan p[TK_CONV_SET];
+                if (ok && d->plans[x.B][stage[0].idx].mt == 0) {
+                    ok = tk_conv_direct_plan_set(c, TK_CONV_SET, p);
+                    for (int i = 0; ok && i < TK_CONV_SET; ++i) d->plans[x.B][stage[i].idx] = p[i];
+                } else {
+                    for (int i = 0; ok && i < TK_CONV_SET; ++i) p[i] = d->plans[x.B][stage[i].idx];
+                }
+                if (ok && tk_launch_conv_direct_set(c, p, TK_CONV_SET, s)) continue;
+                for (const Layer& l : stage) run(l.x, l.idx, l.y, nullptr);
+            }
+        }
+        return true;
+    }
     void conv(const TkT& x, int idx, const TkT& y, const TkT* res) {
+        if (!defer(x, idx, y, res)) run(x, idx, y, res);
+    }
+    void run(const TkT& x, int idx, const TkT& y, const TkT* res) {
         const TkConvSpec& sp = d->model->specs[idx];
         if (direct(x, idx, y, res)) return;
         settle(x);
