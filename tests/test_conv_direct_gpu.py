@@ -80,3 +80,24 @@ def test_what_it_does_not_take(gpu):
     ok = (C.c_int * 15)(1, 64, 64, 16, 16, 16, 0, 0, 0, 3, 1, 16, 16, 0, 1)
     for cut in [(8, 1, 1, 4, 4), (1, 1, 1, 5, 5), (1, 3, 3, 4, 4), (1, 1, 0, 4, 4)]:
         assert gpu.lib().tk_mi355x_conv_direct(0, ok, (C.c_int * 5)(*cut), p(z), None, p(z), None, None, p(z), None) != 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("w,h,batch", [(32, 32, 1), (96, 64, 3), (1344, 32, 1), (32, 1056, 2), (1568, 1344, 1)])
+def test_stem_pools_and_heads_at_odd_maps(gpu, w, h, batch):
+    """whole network at maps that fill no tile of the stem (32 x 8 outputs), with a pooled map of one pixel to one that no longer fits the LDS: frames (the stem pre-processes)
+    against the pre-processed tensor, and a frame alone against the same frame in a batch"""
+    det = gpu.ObjectDetector(model="synthetic://yolov8n?seed=5&cls_bias=-0.5", width=w, height=h, max_batch=batch, conf=0.3)
+    rng = np.random.default_rng(w)
+    frames = [rng.integers(0, 256, (37, 53, 3), np.uint8) for _ in range(batch)]
+    got = det.detect_batch(frames) if batch > 1 else [det.detect(frames[0])]
+    planar = np.stack([gpu.preprocess(f, w, h) for f in frames])
+    raw = det.forward_raw(np.ascontiguousarray(planar.transpose(0, 2, 3, 1)))
+    for b, f in enumerate(frames):
+        one = gpu.ObjectDetector(model="synthetic://yolov8n?seed=5&cls_bias=-0.5", width=w, height=h, max_batch=1, conf=0.3)
+        assert one.detect(f) == got[b] and len(got[b]) > 0
+        boxes, cls, anchors = one.last_boxes()
+        det.detect_batch(frames) if batch > 1 else det.detect(f)
+        assert np.array_equal(one.forward_raw(np.ascontiguousarray(planar[b:b + 1].transpose(0, 2, 3, 1))).view(np.uint32), raw[b:b + 1].view(np.uint32))
+        again, cls2, anchors2 = one.last_boxes()
+        assert np.array_equal(boxes.view(np.uint32), again.view(np.uint32)) and np.array_equal(cls, cls2) and np.array_equal(anchors, anchors2)

@@ -28,10 +28,6 @@ void tk_launch_gemm_form(const TkGemm& g, int form, hipStream_t s);
 /* whether a convolution can be addressed by the GEMM itself (TkGemm::im_*): channels and pitch multiples of 4, input x and the [N][K]
  * f32 weights w 16-byte aligned */
 bool tk_gemm_im2col_ok(const float* x, int C, int ldx, const float* w);
-/* direct 3x3 convolution of a 3-channel image into 16 channels (the detector's stem), the GEMM's chain and epilogue (bias, act) per
- * output; false (nothing launched): another shape — use im2col + tk_launch_gemm */
-bool tk_launch_conv_stem(const float* x, int B, int H, int W, int C, int ldx, const float* w, const float* bias, int act, int N, int k, int stride, int pad, float* y,
-                         int ldy, hipStream_t s);
 /* opts the large-tile GEMM into its dynamic LDS on the calling thread's current device; idempotent, thread-safe.  tk_launch_gemm does
  * it on first use; callers that capture launches into a hipGraph call it beforehand. */
 bool tk_nn_prepare_device();
@@ -45,6 +41,8 @@ bool tk_launch_attention_h3(const float* q, const float* k, const float* v, floa
 void tk_launch_im2col(const float* x, int B, int H, int W, int C, int ldx, int kh, int kw, int stride, int pad, float* col, hipStream_t s);
 /* 1-D variant for conv1d over [T][C] rows */
 void tk_launch_maxpool5(const float* x, int B, int H, int W, int C, int ldx, float* y, int ldy, hipStream_t s);
+/* y0 = pool(x), y1 = pool(y0), y2 = pool(y1); false (nothing launched): channels or pitches that are no multiples of 4, unaligned bases, more than 2048 pixels */
+bool tk_launch_maxpool5_chain(const float* x, int B, int H, int W, int C, int ldx, float* y0, float* y1, float* y2, int ldy, hipStream_t s);
 void tk_launch_upsample2x(const float* x, int B, int H, int W, int C, int ldx, float* y, int ldy, hipStream_t s);
 void tk_launch_copy_cols(const float* x, int rows, int C, int ldx, float* y, int ldy, hipStream_t s);
 /* rows of [T][C] (row pitch ldx) -> col[b*To + t][(kx*C + c)], kernel width kw, zero padding `pad` on both ends */

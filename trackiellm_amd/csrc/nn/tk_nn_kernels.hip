@@ -1190,63 +1190,6 @@ bool tk_gemm_im2col_ok(const float* x, int C, int ldx, const float* w) {
     return C > 0 && (C & 3) == 0 && (ldx & 3) == 0 && ((((uintptr_t)x) | ((uintptr_t)w)) & 15) == 0;
 }
 
-/*
- * The detector's stem (3 input channels: no 16-byte groups for the implicit path, and its column matrix would be 9x the image): one thread
- * per output pixel evaluates all N output channels as the SAME chain the GEMM evaluates — acc = fma(a[k], w[n][k], acc) over
- * k = (ky kw + kx) C + c ascending from +0, padding taps taking part as a = 0 — then the GEMM's epilogue.  Weights sit in LDS.
- */
-template <int N, int C, int KW>
-__global__ __launch_bounds__(256) void k_conv_stem(const float* x, int H, int W, int ldx, const float* w, const float* bias, int act, int stride, int pad, int Ho,
-                                                   int Wo, uint32_t total, float* y, int ldy) {
-    constexpr int K = KW * KW * C;
-    __shared__ __attribute__((aligned(16))) float ws[K * N]; /* [k][n]: a wave reads one k of all n as 16-byte broadcasts */
-    for (int i = threadIdx.x; i < K * N; i += 256) ws[i] = w[(i % N) * K + i / N];
-    __syncthreads();
-    const uint32_t t = blockIdx.x * 256u + threadIdx.x;
-    if (t >= total) return;
-    const uint32_t ox = t % (uint32_t)Wo, r = t / (uint32_t)Wo, oy = r % (uint32_t)Ho, b = r / (uint32_t)Ho;
-    float acc[N];
-#pragma unroll
-    for (int n = 0; n < N; ++n) acc[n] = 0.0f;
-#pragma unroll
-    for (int ky = 0; ky < KW; ++ky)
-#pragma unroll
-        for (int kx = 0; kx < KW; ++kx) {
-            const int iy = (int)(oy * stride) + ky - pad, ix = (int)(ox * stride) + kx - pad;
-            const bool in = iy >= 0 && iy < H && ix >= 0 && ix < W;
-            const float* p = x + (((int64_t)b * H + (in ? iy : 0)) * W + (in ? ix : 0)) * ldx;
-#pragma unroll
-            for (int c = 0; c < C; ++c) {
-                const float a = in ? p[c] : 0.0f;
-                const float4* wk = (const float4*)(ws + ((ky * KW + kx) * C + c) * N);
-#pragma unroll
-                for (int n = 0; n < N; n += 4) {
-                    const float4 q = wk[n >> 2];
-                    acc[n] = __builtin_fmaf(a, q.x, acc[n]); acc[n + 1] = __builtin_fmaf(a, q.y, acc[n + 1]);
-                    acc[n + 2] = __builtin_fmaf(a, q.z, acc[n + 2]); acc[n + 3] = __builtin_fmaf(a, q.w, acc[n + 3]);
-                }
-            }
-        }
-    float4* o = (float4*)(y + (int64_t)t * ldy); /* ldy % 4 == 0 and y 16-byte aligned: checked by the launcher */
-#pragma unroll
-    for (int n = 0; n < N; n += 4) {
-        float4 v;
-        v.x = apply_act(acc[n] + (bias ? bias[n] : 0.0f), act); v.y = apply_act(acc[n + 1] + (bias ? bias[n + 1] : 0.0f), act);
-        v.z = apply_act(acc[n + 2] + (bias ? bias[n + 2] : 0.0f), act); v.w = apply_act(acc[n + 3] + (bias ? bias[n + 3] : 0.0f), act);
-        o[n >> 2] = v;
-    }
-}
-
-bool tk_launch_conv_stem(const float* x, int B, int H, int W, int C, int ldx, const float* w, const float* bias, int act, int N, int k, int stride, int pad, float* y,
-                         int ldy, hipStream_t s) {
-    if (!(N == 16 && C == 3 && k == 3) || (ldy & 3) || (((uintptr_t)y) & 15)) return false;
-    const int Ho = (H + 2 * pad - k) / stride + 1, Wo = (W + 2 * pad - k) / stride + 1;
-    const int64_t total = (int64_t)B * Ho * Wo;
-    if (total <= 0 || total >= ((int64_t)1 << 31)) return false;
-    hipLaunchKernelGGL((k_conv_stem<16, 3, 3>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x, H, W, ldx, w, bias, act, stride, pad, Ho, Wo, (uint32_t)total, y, ldy);
-    return true;
-}
-
 __global__ void k_im2col(const float* x, int B, int H, int W, int C, int ldx, int kh, int kw, int stride, int pad, int Ho, int Wo, float* col) {
     const int64_t K = (int64_t)kh * kw * C;
     const int64_t total = (int64_t)B * Ho * Wo * K;
@@ -1311,6 +1254,48 @@ __global__ void k_maxpool5(const float* x, int B, int H, int W, int C, int ldx, 
 void tk_launch_maxpool5(const float* x, int B, int H, int W, int C, int ldx, float* y, int ldy, hipStream_t s) {
     const int64_t total = (int64_t)B * H * W * C;
     hipLaunchKernelGGL(k_maxpool5, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, x, B, H, W, C, ldx, y, ldy);
+}
+
+/* SPPF's three poolings in a row as one launch: a workgroup holds four channels of a map in the LDS, twice, and a pooling is 25 reads of 16 bytes in the order of
+ * k_maxpool5.  Three launches of 9.4 us at one frame (20 x 20 x 128), 38 at 32: now one of 8.3 and of 26. */
+#define TK_POOL_MAX_PIXELS 2048
+__global__ __launch_bounds__(512) void k_maxpool5_chain(const float* x, int H, int W, int ldx, float* y0, float* y1, float* y2, int ldy) {
+    extern __shared__ __attribute__((aligned(16))) float pool_lds[];
+    const int n = H * W, c = blockIdx.x * 4;
+    const int64_t base = (int64_t)blockIdx.y * n;
+    v4f* cur = (v4f*)pool_lds;
+    v4f* nxt = cur + n;
+    for (int i = threadIdx.x; i < n; i += 512) cur[i] = *(const v4f*)(x + (base + i) * ldx + c);
+    __syncthreads();
+#pragma unroll 1
+    for (int t = 0; t < 3; ++t) {
+        float* y = t == 0 ? y0 : t == 1 ? y1 : y2;
+        for (int i = threadIdx.x; i < n; i += 512) {
+            const int oy = i / W, ox = i - oy * W;
+            v4f m = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+            for (int dy = -2; dy <= 2; ++dy)
+#pragma unroll
+                for (int dx = -2; dx <= 2; ++dx) {
+                    const int iy = oy + dy, ix = ox + dx;
+                    const bool in = (int)((uint32_t)iy < (uint32_t)H) & (int)((uint32_t)ix < (uint32_t)W);
+                    const v4f v = cur[in ? iy * W + ix : i];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) m[q] = in ? tk_fmaxf(m[q], v[q]) : m[q];
+                }
+            nxt[i] = m;
+            *(v4f*)(y + (base + i) * ldy + c) = m;
+        }
+        __syncthreads();
+        v4f* const swap = cur;
+        cur = nxt;
+        nxt = swap;
+    }
+}
+bool tk_launch_maxpool5_chain(const float* x, int B, int H, int W, int C, int ldx, float* y0, float* y1, float* y2, int ldy, hipStream_t s) {
+    if ((C & 3) || (ldx & 3) || (ldy & 3) || (((uintptr_t)x | (uintptr_t)y0 | (uintptr_t)y1 | (uintptr_t)y2) & 15) || (int64_t)H * W > TK_POOL_MAX_PIXELS || B > 65535) return false;
+    hipLaunchKernelGGL(k_maxpool5_chain, dim3(C / 4, B), dim3(512), (size_t)H * W * 32, s, x, H, W, ldx, y0, y1, y2, ldy);
+    return true;
 }
 
 __global__ void k_upsample2x(const float* x, int B, int H, int W, int C, int ldx, float* y, int ldy) {

@@ -40,7 +40,7 @@ public:
     int device = 0, nc = TK_YOLO_NC;
     std::vector<TkConvSpec> specs;
     std::vector<float*> w, b; /* device: [cout][k*k*cin], [cout] */
-    std::vector<float*> wp;   /* device: the weights as pieces (tk_conv_direct.h) of the layers that have whole ones, null else */
+    std::vector<float*> wp;   /* device: the weights as pieces (tk_conv_direct.h) of the layers that have whole ones, the stem's as [27][16], null else */
     std::string error;
     ~TkYoloModel();
     bool init(int device, int nc);
@@ -83,7 +83,8 @@ public:
      * color[n] = dominant-colour bin 0..8, door_closed[n] = 1 when the strong-vertical-edge density exceeds 10 % */
     bool classify_boxes(int b, int n, const int32_t* rects, int32_t* color, int32_t* door_closed);
 
-    bool enqueue(int B); /* pre-processed input already in `input`; network + decode + NMS on `stream` */
+    /* network + decode + NMS on `stream`, of the pre-processed tensor in `input` or (frames) of B device frames side by side, which the stem pre-processes on its way */
+    bool enqueue(int B, const TkPreprocessArgs* frames = nullptr);
     float* input = nullptr;        /* [B][H][W][3] */
     int n_anchors = 0;
 

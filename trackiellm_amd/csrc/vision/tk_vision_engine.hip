@@ -29,18 +29,14 @@ static inline hipError_t tk_create_perception_stream(hipStream_t* s) { return hi
  * One thread per output pixel, all three channels; u8 reads are served by L2 (the 4 taps of
  * neighbouring pixels overlap), fp32 writes are coalesced per plane.  HBM-bound: 1.23 MB in, 4.92 MB out.
  * ------------------------------------------------------------------------------------------ */
-__global__ void k_preprocess(TkPreprocessArgs a) {
-    const uint32_t ox = blockIdx.x * blockDim.x + threadIdx.x, oy = blockIdx.y * blockDim.y + threadIdx.y;
-    if (ox >= a.out_w || oy >= a.out_h) return;
-    const float x_ratio = tk_divf((float)a.in_w - 1.0f, (float)a.out_w);
-    const float y_ratio = tk_divf((float)a.in_h - 1.0f, (float)a.out_h);
+/* the three channels of output pixel (ox, oy) */
+__device__ __forceinline__ void preprocess_pixel(const TkPreprocessArgs& a, const uint8_t* src, float x_ratio, float y_ratio, uint32_t ox, uint32_t oy, float out[3]) {
     const float gx = x_ratio * (float)ox, gy = y_ratio * (float)oy;
     const int x = (int)gx, y = (int)gy;
     const float xd = gx - (float)x, yd = gy - (float)y;
     const int x1 = x + 1 < (int)a.in_w ? x + 1 : x, y1 = y + 1 < (int)a.in_h ? y + 1 : y; /* reference reads x+1/y+1 (always in range for w,h >= 2) */
-    const uint8_t* r0 = a.src + (size_t)y * a.in_stride;
-    const uint8_t* r1 = a.src + (size_t)y1 * a.in_stride;
-    const size_t np = (size_t)a.out_w * a.out_h, pix = (size_t)oy * a.out_w + ox;
+    const uint8_t* r0 = src + (size_t)y * a.in_stride;
+    const uint8_t* r1 = src + (size_t)y1 * a.in_stride;
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
         const float p1 = (float)r0[x * a.bpp + c], p2 = (float)r0[x1 * a.bpp + c];
@@ -49,9 +45,21 @@ __global__ void k_preprocess(TkPreprocessArgs a) {
         v = v + (p2 * xd) * (1.0f - yd);
         v = v + (p3 * (1.0f - xd)) * yd;
         v = v + (p4 * xd) * yd;
-        const float o = tk_divf(tk_divf(v, 255.0f) - a.mean[c], a.std_dev[c]);
-        if (a.nhwc) a.dst[pix * 3 + c] = o;
-        else a.dst[c * np + pix] = o;
+        out[c] = tk_divf(tk_divf(v, 255.0f) - a.mean[c], a.std_dev[c]);
+    }
+}
+__global__ void k_preprocess(TkPreprocessArgs a) {
+    const uint32_t ox = blockIdx.x * blockDim.x + threadIdx.x, oy = blockIdx.y * blockDim.y + threadIdx.y;
+    if (ox >= a.out_w || oy >= a.out_h) return;
+    const float x_ratio = tk_divf((float)a.in_w - 1.0f, (float)a.out_w);
+    const float y_ratio = tk_divf((float)a.in_h - 1.0f, (float)a.out_h);
+    const size_t np = (size_t)a.out_w * a.out_h, pix = (size_t)oy * a.out_w + ox;
+    float o[3];
+    preprocess_pixel(a, a.src, x_ratio, y_ratio, ox, oy, o);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        if (a.nhwc) a.dst[pix * 3 + c] = o[c];
+        else a.dst[c * np + pix] = o[c];
     }
 }
 
@@ -59,6 +67,63 @@ void tk_launch_preprocess(const TkPreprocessArgs& a, hipStream_t s) {
     dim3 block(64, 4);
     dim3 grid((a.out_w + 63) / 64, (a.out_h + 3) / 4);
     hipLaunchKernelGGL(k_preprocess, grid, block, 0, s, a);
+}
+
+/*
+ * The detector's stem, 3 -> 16 channels, 3 x 3, stride 2, padding 1: a thread per output pixel, all 16 channels as the GEMM's chain — acc = fma(a[k], w[n][k], acc) over
+ * k = (ky 3 + kx) 3 + c ascending from +0, padding as a = 0 — then bias and SiLU.  The input pixels under a tile of 32 x 8 outputs go through the LDS; from camera
+ * frames they are pre-processed on the way, so that the network's input tensor is never written or read.  Weights are read through the scalar cache ([27][16]).
+ * Vector instructions bound it (per output 432 fmas and 16 SiLUs, per input pixel ~110): one frame 15 us (pre-processing and stem as launches of their own:
+ * 24), 32 frames 546 -> 160 us.  All byte loads of a thread ahead of their use: 178 at 32 frames, no gain at one.
+ */
+#define TK_STEM_TW 32
+#define TK_STEM_TH 8
+template <bool FRAMES>
+__global__ __launch_bounds__(256) void k_stem(TkPreprocessArgs a, size_t frame_bytes, const float* tensor, int H, int W, int Ho, int Wo, const float* __restrict__ wt,
+                                              const float* __restrict__ bias, int silu, float* y, int ldy) {
+    constexpr int PW = 2 * TK_STEM_TW + 1, PH = 2 * TK_STEM_TH + 1, PN = PW * PH;
+    __shared__ float px[3 * PN];
+    const int tid = threadIdx.x, b = blockIdx.z;
+    const int iy0 = 2 * (int)blockIdx.y * TK_STEM_TH - 1, ix0 = 2 * (int)blockIdx.x * TK_STEM_TW - 1;
+    const float x_ratio = FRAMES ? tk_divf((float)a.in_w - 1.0f, (float)a.out_w) : 0.0f, y_ratio = FRAMES ? tk_divf((float)a.in_h - 1.0f, (float)a.out_h) : 0.0f;
+    const uint8_t* src = FRAMES ? a.src + frame_bytes * (size_t)b : nullptr;
+    for (int e = tid; e < PN; e += 256) {
+        const int py = e / PW, iy = iy0 + py, ix = ix0 + e - py * PW;
+        float v[3] = {0.0f, 0.0f, 0.0f};
+        if (iy >= 0 && iy < H && ix >= 0 && ix < W) {
+            if (FRAMES) preprocess_pixel(a, src, x_ratio, y_ratio, (uint32_t)ix, (uint32_t)iy, v);
+            else {
+                const float* p = tensor + (((int64_t)b * H + iy) * W + ix) * 3;
+                v[0] = p[0]; v[1] = p[1]; v[2] = p[2];
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 3; ++c) px[c * PN + e] = v[c];
+    }
+    __syncthreads();
+    const int ly = tid / TK_STEM_TW, lx = tid % TK_STEM_TW;
+    const int oy = blockIdx.y * TK_STEM_TH + ly, ox = blockIdx.x * TK_STEM_TW + lx;
+    float acc[16];
+#pragma unroll
+    for (int n = 0; n < 16; ++n) acc[n] = 0.0f;
+    const float* p = px + 2 * ly * PW + 2 * lx;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+        const float v = p[(k % 3) * PN + (k / 9) * PW + k / 3 % 3];
+#pragma unroll
+        for (int n = 0; n < 16; ++n) acc[n] = __builtin_fmaf(v, wt[k * 16 + n], acc[n]);
+    }
+    if (oy >= Ho || ox >= Wo) return;
+#pragma unroll
+    for (int n = 0; n < 16; ++n) acc[n] = acc[n] + bias[n];
+    if (silu) tk_silu_all<16>(acc);
+    float4* o = (float4*)(y + (((int64_t)b * Ho + oy) * Wo + ox) * ldy);
+#pragma unroll
+    for (int n = 0; n < 16; n += 4) o[n >> 2] = make_float4(acc[n], acc[n + 1], acc[n + 2], acc[n + 3]);
+}
+/* [16][27] -> [27][16] */
+__global__ void k_stem_weights(const float* w, float* wt) {
+    for (int i = threadIdx.x; i < 432; i += blockDim.x) wt[i] = w[(i % 16) * 27 + i / 16];
 }
 
 /* ------------------------------------------------------------------------------------------ model */
@@ -84,8 +149,9 @@ bool TkYoloModel::init(int dev, int n_classes) {
         const TkConvSpec& s = specs[i];
         HIPQ(hipMalloc((void**)&w[i], (size_t)s.cout * s.k * s.k * s.cin * 4));
         HIPQ(hipMalloc((void**)&b[i], (size_t)s.cout * 4));
-        if (s.cin % 16 == 0) {
-            const size_t n = tk_conv_weight_floats(s.cout, s.k * s.k * s.cin) * 4;
+        const bool stem = i == 0 && s.cin == 3 && s.cout == 16 && s.k == 3 && s.s == 2;
+        if (stem || s.cin % 16 == 0) {
+            const size_t n = stem ? 432 * 4 : tk_conv_weight_floats(s.cout, s.k * s.k * s.cin) * 4;
             HIPQ(hipMalloc((void**)&wp[i], n));
             HIPQ(hipMemset(wp[i], 0, n)); /* what lies behind the last piece is requested, not used */
         }
@@ -106,7 +172,8 @@ bool TkYoloModel::set_layer(int idx, const float* w_host, const float* b_host) {
     HIPQ(hipMemcpy(w[idx], w_host, (size_t)s.cout * s.k * s.k * s.cin * 4, hipMemcpyHostToDevice));
     HIPQ(hipMemcpy(b[idx], b_host, (size_t)s.cout * 4, hipMemcpyHostToDevice));
     if (wp[idx]) {
-        tk_launch_conv_weights(w[idx], s.cout, s.k * s.k * s.cin, wp[idx], nullptr);
+        if (s.cin == 3) hipLaunchKernelGGL(k_stem_weights, dim3(1), dim3(64), 0, nullptr, w[idx], wp[idx]);
+        else tk_launch_conv_weights(w[idx], s.cout, s.k * s.k * s.cin, wp[idx], nullptr);
         HIPQ(hipGetLastError());
         HIPQ(hipStreamSynchronize(nullptr)); /* the engines' streams do not wait for the null stream */
     }
@@ -217,6 +284,17 @@ struct TkGpuOps {
         d->arena_used += n;
         return t;
     }
+    const TkPreprocessArgs* frames = nullptr;
+    size_t frame_bytes = 0;
+    bool stem(const TkT& x, const TkT& y) {
+        const TkConvSpec& sp = d->model->specs[0];
+        if (!d->model->wp[0] || sp.cin != 3 || (y.ld & 3) || (((uintptr_t)y.p) & 15) || y.B > 65535) return false;
+        const dim3 grid((y.W + TK_STEM_TW - 1) / TK_STEM_TW, (y.H + TK_STEM_TH - 1) / TK_STEM_TH, y.B);
+        const TkPreprocessArgs a = frames ? *frames : TkPreprocessArgs{};
+        if (frames) hipLaunchKernelGGL((k_stem<true>), grid, dim3(256), 0, s, a, frame_bytes, x.p, x.H, x.W, y.H, y.W, d->model->wp[0], d->model->b[0], sp.act, y.p, y.ld);
+        else hipLaunchKernelGGL((k_stem<false>), grid, dim3(256), 0, s, a, frame_bytes, x.p, x.H, x.W, y.H, y.W, d->model->wp[0], d->model->b[0], sp.act, y.p, y.ld);
+        return true;
+    }
     /* A concatenation's copied and upsampled parts are not written: the convolution behind it reads them where they are (two sources).  Any other reader has them
      * written first. */
     struct Part { TkT x, y; int shift; };
@@ -257,7 +335,7 @@ struct TkGpuOps {
     /* false: not a layer for the direct kernel */
     bool describe(const TkT& x, int idx, const TkT& y, const TkT* res, TkConvDirect* out) const {
         const TkConvSpec& sp = d->model->specs[idx];
-        if (d->fast || !d->model->wp[idx]) return false;
+        if (d->fast || idx == 0 || !d->model->wp[idx]) return false;
         TkConvDirect& c = *out;
         c = TkConvDirect{};
         if (!sources(x, &c)) return false;
@@ -306,10 +384,12 @@ struct TkGpuOps {
         return true;
     }
     void conv(const TkT& x, int idx, const TkT& y, const TkT* res) {
+        pool();
         if (!defer(x, idx, y, res)) run(x, idx, y, res);
     }
     void run(const TkT& x, int idx, const TkT& y, const TkT* res) {
         const TkConvSpec& sp = d->model->specs[idx];
+        if (idx == 0 && stem(x, y)) return;
         if (direct(x, idx, y, res)) return;
         settle(x);
         if (res) settle(*res);
@@ -320,9 +400,6 @@ struct TkGpuOps {
             g.A = x.p; g.lda = 0;
             g.im_C = x.C; g.im_H = x.H; g.im_W = x.W; g.im_ldx = x.ld; g.im_kw = sp.k; g.im_stride = sp.s; g.im_pad = sp.k / 2;
             g.im_Ho = y.H; g.im_Wo = y.W;
-        } else if (!res && tk_launch_conv_stem(x.p, x.B, x.H, x.W, x.C, x.ld, d->model->w[idx], d->model->b[idx], sp.act ? TK_ACT_SILU : TK_ACT_NONE, sp.cout, sp.k,
-                                               sp.s, sp.k / 2, y.p, y.ld, s)) {
-            return; /* the 3-channel stem: a direct kernel, the GEMM's chain */
         } else {
             tk_launch_im2col(x.p, x.B, x.H, x.W, x.C, x.ld, sp.k, sp.k, sp.s, sp.k / 2, d->col, s);
             g.A = d->col; g.lda = g.K;
@@ -336,9 +413,24 @@ struct TkGpuOps {
         g.fast = d->fast ? 1 : 0;
         tk_launch_gemm(g, s);
     }
-    void maxpool5(const TkT& x, const TkT& y) { settle(x); tk_launch_maxpool5(x.p, x.B, x.H, x.W, x.C, x.ld, y.p, y.ld, s); }
-    void upsample2x(const TkT& x, const TkT& y) { settle(x); parts.push_back(Part{x, y, 1}); }
-    void copy(const TkT& x, const TkT& y) { settle(x); parts.push_back(Part{x, y, 0}); }
+    /* three poolings, each of the one before: one launch */
+    struct Pool { TkT x, y; };
+    std::vector<Pool> pools;
+    void maxpool5(const TkT& x, const TkT& y) {
+        if (!pools.empty() && (x.p != pools.back().y.p || x.C != y.C || x.ld != pools.back().y.ld || y.ld != x.ld)) pool();
+        if (pools.empty()) settle(x);
+        pools.push_back(Pool{x, y});
+        if (pools.size() == 3) pool();
+    }
+    void pool() {
+        const TkT x = pools.empty() ? TkT{} : pools[0].x;
+        const bool chain = pools.size() == 3 && tk_launch_maxpool5_chain(x.p, x.B, x.H, x.W, x.C, x.ld, pools[0].y.p, pools[1].y.p, pools[2].y.p, pools[0].y.ld, s);
+        if (!chain)
+            for (const Pool& q : pools) tk_launch_maxpool5(q.x.p, q.x.B, q.x.H, q.x.W, q.x.C, q.x.ld, q.y.p, q.y.ld, s);
+        pools.clear();
+    }
+    void upsample2x(const TkT& x, const TkT& y) { pool(); settle(x); parts.push_back(Part{x, y, 1}); }
+    void copy(const TkT& x, const TkT& y) { pool(); settle(x); parts.push_back(Part{x, y, 0}); }
 };
 
 /* sizing pass: same graph, counts arena floats and the largest im2col matrix */
@@ -633,7 +725,7 @@ bool TkDetector::forward_graph(int B, const float* nchw_host, std::vector<float>
     return true;
 }
 
-bool TkDetector::enqueue(int B) {
+bool TkDetector::enqueue(int B, const TkPreprocessArgs* frames) {
     if (model->generic) {
         if (!run_graph(B, nullptr)) return false;
         hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
@@ -644,6 +736,8 @@ bool TkDetector::enqueue(int B) {
     }
     TkGpuOps ops;
     ops.d = this; ops.s = stream;
+    ops.frames = frames;
+    ops.frame_bytes = frames ? (size_t)frames->in_stride * frames->in_h : 0;
     arena_used = 0;
     if (plans[B].empty()) plans[B].assign(model->specs.size(), TkConvPlan{});
     TkT x;
@@ -668,16 +762,21 @@ bool TkDetector::detect(int B, const uint8_t* const* frames, uint32_t w, uint32_
         HIPQ(hipMalloc((void**)&frame_dev, fb * max_batch));
         frame_cap = fb * max_batch;
     }
+    TkPreprocessArgs a{};
+    a.src = frame_dev; a.in_w = w; a.in_h = h; a.in_stride = stride; a.bpp = bpp;
+    a.dst = input; a.out_w = in_w; a.out_h = in_h; a.nhwc = model->generic ? 0 : 1; /* a file's graph takes planar NCHW */
+    for (int c = 0; c < 3; ++c) { a.mean[c] = mean[c]; a.std_dev[c] = std_dev[c]; }
+    const bool in_stem = !model->generic && model->wp[0]; /* else as a launch of its own per frame */
     for (int b = 0; b < B; ++b) {
         HIPQ(hipMemcpyAsync(frame_dev + fb * b, frames[b], fb, hipMemcpyHostToDevice, stream));
-        TkPreprocessArgs a{};
-        a.src = frame_dev + fb * b; a.in_w = w; a.in_h = h; a.in_stride = stride; a.bpp = bpp;
-        a.dst = input + (size_t)b * in_h * in_w * 3; a.out_w = in_w; a.out_h = in_h; a.nhwc = model->generic ? 0 : 1; /* a file's graph takes planar NCHW */
-        for (int c = 0; c < 3; ++c) { a.mean[c] = mean[c]; a.std_dev[c] = std_dev[c]; }
-        tk_launch_preprocess(a, stream);
+        if (in_stem) continue;
+        TkPreprocessArgs f = a;
+        f.src = frame_dev + fb * b;
+        f.dst = input + (size_t)b * in_h * in_w * 3;
+        tk_launch_preprocess(f, stream);
     }
     last_w = w; last_h = h; last_stride = stride; last_B = B;
-    if (!enqueue(B)) return false;
+    if (!enqueue(B, in_stem ? &a : nullptr)) return false;
     return fetch(B, out);
 }
 
