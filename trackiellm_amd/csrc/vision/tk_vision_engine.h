@@ -109,8 +109,15 @@ private:
     int32_t* order = nullptr;           /* [B][MAX_CAND] anchor ids, sorted */
     int32_t* n_cand = nullptr;          /* [B] */
     uint64_t* mask = nullptr;           /* [B][MAX_CAND][MAX_CAND/64] */
-    TkDetection* kept = nullptr;        /* [B][MAX_DET] */
-    int32_t* n_kept = nullptr;          /* [B] */
+    uint64_t* list = nullptr;           /* [B][n_anchors] keys of the anchors above the threshold, in any order (k_yolo_rank) */
+    int32_t* n_list = nullptr;          /* [B], zero between passes (the scan clears it) */
+    bool list_clear = false;            /* the last pass came to its end */
+    uint8_t* results = nullptr;         /* [B] counts, then [B][MAX_DET] boxes; the same in pinned host memory */
+    uint8_t* results_host = nullptr;
+    size_t kept_at = 0;
+    TkDetection* kept = nullptr;        /* in results */
+    int32_t* n_kept = nullptr;
+    bool begin_list();
 };
 
 /* the same classification on a host frame (tightly packed RGB8), temporary device buffers on `device`: the reference's stand-alone

@@ -454,11 +454,24 @@ struct TkSizeOps {
 
 /* ------------------------------------------------------------------------------------------ decode + NMS kernels */
 
-/* Four lanes per anchor: lane q takes side q of the box and the classes q, q + 4, ... (first class on ties, as tk_yolo_decode_anchor).  One thread per
- * anchor was a chain of 64 + nc exponentials on a tenth of the chip: 29 us for the 8400 anchors of one 640 x 640 frame, now 9. */
-__global__ __launch_bounds__(256) void k_yolo_decode(TkT h0, TkT h1, TkT h2, int nc, int n_anchors, float conf, tk_yolo_cand_t* cand) {
-    const int a = (blockIdx.x * 256 + threadIdx.x) >> 2, q = threadIdx.x & 3, b = blockIdx.y;
-    if (a >= n_anchors) return; /* all four lanes of an anchor */
+/* one lane of each anchor says whether it is a candidate: those of a wave are appended to the frame's list, in any order, as keys whose order is (score desc, anchor
+ * asc) from the largest down */
+__device__ __forceinline__ void append_candidate(bool is, float score, int anchor, uint64_t* list, int32_t* n_list) {
+    const uint64_t all = __ballot(is);
+    if (all == 0) return;
+    const int lane = threadIdx.x & 63, first = __builtin_ctzll(all);
+    int base = 0;
+    if (lane == first) base = atomicAdd(n_list, __popcll(all));
+    base = __shfl(base, first, 64);
+    const uint32_t u = tk_f32_bits(score + 0.0f), up = u >> 31 ? ~u : u | 0x80000000u; /* (-0 counts as +0) */
+    if (is) list[base + __popcll(all & ((1ull << lane) - 1ull))] = (uint64_t)up << 32 | (uint32_t)~(uint32_t)anchor;
+}
+
+/* Four lanes per anchor: lane q takes side q of the box and of every 16 classes the four from 4 q on (first class on ties, as tk_yolo_decode_anchor).  One thread per
+ * anchor was a chain of 64 + nc exponentials on a tenth of the chip: 29 us for the 8400 anchors of one 640 x 640 frame, now 8. */
+__global__ __launch_bounds__(256) void k_yolo_decode(TkT h0, TkT h1, TkT h2, int nc, int n_anchors, float conf, tk_yolo_cand_t* cand, uint64_t* list, int32_t* n_list) {
+    const int at = (blockIdx.x * 256 + threadIdx.x) >> 2, q = threadIdx.x & 3, b = blockIdx.y;
+    const int a = at < n_anchors ? at : n_anchors - 1; /* past the end: not stored */
     const int n0 = h0.H * h0.W, n1 = h1.H * h1.W;
     const TkT* h;
     int local;
@@ -468,100 +481,92 @@ __global__ __launch_bounds__(256) void k_yolo_decode(TkT h0, TkT h1, TkT h2, int
     else { h = &h2; local = a - n0 - n1; stride = 32.0f; }
     const float ax = (float)(local % h->W) + 0.5f, ay = (float)(local / h->W) + 0.5f;
     const float* o = h->p + ((size_t)b * h->H * h->W + local) * h->ld;
-    const float d = tk_yolo_dfl(o + 16 * q);
+    float side[16];
     float best = -1.0f;
     int bi = 0;
-    for (int k = q; k < nc; k += 4) {
-        const float s = tk_sigmoidf(o[64 + k]);
+    auto score = [&](float l, int k) {
+        const float s = tk_sigmoidf(l);
         if (s > best) { best = s; bi = k; }
+    };
+    if ((nc & 3) == 0) { /* pixels of 64 + nc floats: every group of four is aligned */
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float4 t = ((const float4*)(o + 16 * q))[i];
+            side[4 * i] = t.x; side[4 * i + 1] = t.y; side[4 * i + 2] = t.z; side[4 * i + 3] = t.w;
+        }
+        for (int k = 4 * q; k < nc; k += 16) {
+            const float4 t = *(const float4*)(o + 64 + k);
+            score(t.x, k); score(t.y, k + 1); score(t.z, k + 2); score(t.w, k + 3);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) side[i] = o[16 * q + i];
+        for (int k = q; k < nc; k += 4) score(o[64 + k], k);
     }
+    const float d = tk_yolo_dfl(side);
 #pragma unroll
     for (int w = 1; w <= 2; w <<= 1) {
         const float os = __shfl_xor(best, w, 64);
         const int oi = __shfl_xor(bi, w, 64);
         if (os > best || (os == best && oi < bi)) { best = os; bi = oi; }
     }
-    const float at = q & 1 ? ay : ax, edge = (q < 2 ? at - d : at + d) * stride; /* x1 y1 x2 y2 */
-    tk_yolo_cand_t* c = cand + (size_t)b * n_anchors + a;
-    (&c->x1)[q] = edge;
-    if (q == 0) { c->score = best; c->cls = best > conf ? bi : -1 /* not a candidate */; c->anchor = a; }
+    const float from = q & 1 ? ay : ax, edge = (q < 2 ? from - d : from + d) * stride; /* x1 y1 x2 y2 */
+    const bool is = at < n_anchors && best > conf;
+    if (at < n_anchors) {
+        tk_yolo_cand_t* c = cand + (size_t)b * n_anchors + a;
+        (&c->x1)[q] = edge;
+        if (q == 0) { c->score = best; c->cls = is ? bi : -1 /* not a candidate */; c->anchor = a; }
+    }
+    append_candidate(is && q == 0, best, a, list + (size_t)b * n_anchors, n_list + b);
 }
 
 /* a YOLO-class graph's own output [4 + nc][anchors] (Ultralytics export: box centre / size in input pixels, class probabilities already through
  * the sigmoid): xyxy = centre -/+ size / 2, score = max_c p_c (first class on ties), candidate iff score > confidence_threshold */
-__global__ void k_yolo_decode_out(const float* out, int nc, int n_anchors, float conf, tk_yolo_cand_t* cand) {
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    if (a >= n_anchors) return;
+__global__ void k_yolo_decode_out(const float* out, int nc, int n_anchors, float conf, tk_yolo_cand_t* cand, uint64_t* list, int32_t* n_list) {
+    const int at = blockIdx.x * blockDim.x + threadIdx.x, a = at < n_anchors ? at : n_anchors - 1;
     tk_yolo_cand_t c;
     tk_yolo_decode_out_anchor(out + a, n_anchors, nc, &c);
     c.anchor = a;
-    if (!(c.score > conf)) c.cls = -1;
-    cand[a] = c;
+    const bool is = at < n_anchors && c.score > conf;
+    if (!is) c.cls = -1;
+    if (at < n_anchors) cand[a] = c;
+    append_candidate(is, c.score, a, list, n_list);
 }
 
-/* rank of every candidate among the candidates: (score desc, anchor asc); the best MAX_CAND are kept.  Most anchors fall below the
- * confidence threshold, so each 1024-anchor tile is compacted in LDS first (ballot + prefix) and only its survivors are compared.  A tile's scores are
- * requested under the tile before, survivors are read eight at a time: 8400 anchors 41 -> 22 us. */
-__global__ __launch_bounds__(256) void k_yolo_rank(const tk_yolo_cand_t* cand, int n_anchors, int32_t* order, int32_t* n_cand) {
-    const int b = blockIdx.y;
-    const tk_yolo_cand_t* cb = cand + (size_t)b * n_anchors;
-    const int a = blockIdx.x * blockDim.x + threadIdx.x;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    __shared__ __attribute__((aligned(16))) float2 tile[1024 + 8]; /* score, anchor (as bits) */
-    __shared__ int wcnt[16];
-    const int own = a < n_anchors ? a : n_anchors - 1;
-    const bool valid = a < n_anchors && cb[own].cls >= 0;
-    const float mys = cb[own].score;
-    float sco[4];
-    int cls[4];
-    auto load = [&](int base) { /* past the last anchor: read again, not used */
+/* rank of every candidate among the candidates; the best MAX_CAND are kept.  Most anchors fall below the confidence threshold and are not in the list.  A workgroup
+ * takes 64 candidates, one a lane, and each of its waves a quarter of the list (1 000 candidates of 8 400 anchors: 20 us when every workgroup looked through all anchors,
+ * 13 with a lane that walked the whole list, now 6). */
+__global__ __launch_bounds__(256) void k_yolo_rank(const uint64_t* list, const int32_t* n_list, int n_anchors, int32_t* order, int32_t* n_cand) {
+    const int b = blockIdx.y, n = n_list[b], lane = threadIdx.x & 63, wave = threadIdx.x >> 6, i = blockIdx.x * 64 + lane;
+    if (blockIdx.x == 0 && threadIdx.x == 0) n_cand[b] = n < TK_YOLO_MAX_CAND ? n : TK_YOLO_MAX_CAND;
+    if (blockIdx.x * 64 >= n) return;
+    const uint64_t* lb = list + (size_t)b * n_anchors;
+    __shared__ __attribute__((aligned(16))) uint64_t tile[1024];
+    __shared__ int part[4][64];
+    const uint64_t own = lb[i < n ? i : n - 1];
+    int rank = 0;
+    for (int base = 0; base < n; base += 1024) {
+        if (base) __syncthreads();
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            int j = base + u * 256 + (int)threadIdx.x;
-            j = j < n_anchors ? j : n_anchors - 1;
-            sco[u] = cb[j].score; cls[u] = cb[j].cls;
-        }
-    };
-    load(0);
-    int rank = 0, total = 0;
-    for (int base = 0; base < n_anchors; base += 1024) {
-        uint64_t bal[4];
-        float s0[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            s0[u] = sco[u];
-            bal[u] = __ballot(base + u * 256 + (int)threadIdx.x < n_anchors && cls[u] >= 0);
-            if (lane == 0) wcnt[u * 4 + wave] = __popcll(bal[u]);
+            const int j = (int)threadIdx.x + u * 256;
+            tile[j] = base + j < n ? lb[base + j] : 0; /* below every candidate */
         }
         __syncthreads();
-        if (base + 1024 < n_anchors) load(base + 1024);
-        int nt = 0, off[4];
+        const int nt = n - base < 1024 ? n - base : 1024;
+        for (int k = wave * 8; k < nt; k += 32) { /* the waves take turns: eight keys each */
+            uint64_t o[8];
 #pragma unroll
-        for (int w = 0; w < 16; ++w) {
-            if ((w & 3) == wave) off[w >> 2] = nt;
-            nt += wcnt[w];
+            for (int u = 0; u < 8; ++u) o[u] = tile[k + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) rank += o[u] > own ? 1 : 0;
         }
-#pragma unroll
-        for (int u = 0; u < 4; ++u)
-            if (bal[u] >> lane & 1) {
-                const int pos = off[u] + __popcll(bal[u] & ((1ull << lane) - 1ull));
-                tile[pos] = make_float2(s0[u], __int_as_float(base + u * 256 + (int)threadIdx.x));
-            }
-        if (threadIdx.x < 8) tile[nt + threadIdx.x] = make_float2(-INFINITY, 0.0f); /* below every candidate */
-        __syncthreads();
-        if (valid)
-            for (int k = 0; k < nt; k += 8) {
-                float2 o[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) o[u] = tile[k + u];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) rank += o[u].x > mys || (o[u].x == mys && __float_as_int(o[u].y) < a) ? 1 : 0;
-            }
-        total += nt;
-        __syncthreads();
     }
-    if (valid && rank < TK_YOLO_MAX_CAND) order[(size_t)b * TK_YOLO_MAX_CAND + rank] = a;
-    if (a == 0) n_cand[b] = total < TK_YOLO_MAX_CAND ? total : TK_YOLO_MAX_CAND;
+    part[wave][lane] = rank;
+    __syncthreads();
+    if (wave != 0 || i >= n) return;
+    rank = part[0][lane] + part[1][lane] + part[2][lane] + part[3][lane];
+    if (rank < TK_YOLO_MAX_CAND) order[(size_t)b * TK_YOLO_MAX_CAND + rank] = (int32_t)~(uint32_t)own;
 }
 
 /* suppression bit matrix: bit j of mask[i] set iff j > i, same class, IoU > thr.  A wave holds 64 candidates j, one a lane, and takes 32 rows i: a row's
@@ -588,8 +593,9 @@ __global__ __launch_bounds__(256) void k_yolo_mask(const tk_yolo_cand_t* cand, i
 /* greedy scan, one wave per frame: 64 candidates at a time, whose words among themselves are in the lanes, so that a kept one costs a few scalar steps and
  * no trip to memory (44 us for some tens of kept boxes, now 8); the later words take the kept rows eight loads at a time */
 __global__ __launch_bounds__(64) void k_yolo_scan(const tk_yolo_cand_t* cand, int n_anchors, const int32_t* order, const int32_t* n_cand, const uint64_t* mask,
-                                                  TkDetection* kept, int32_t* n_kept) {
+                                                  TkDetection* kept, int32_t* n_kept, int32_t* n_list) {
     const int b = blockIdx.x, lane = threadIdx.x;
+    if (lane == 0) n_list[b] = 0; /* for the next pass */
     constexpr int WORDS = TK_YOLO_MAX_CAND / 64;
     static_assert(WORDS <= 64, "a lane per word");
     const int n = n_cand[b];
@@ -642,8 +648,9 @@ __global__ __launch_bounds__(64) void k_yolo_scan(const tk_yolo_cand_t* cand, in
 TkDetector::~TkDetector() {
     if (model) (void)hipSetDevice(model->device);
     if (stream) (void)hipStreamSynchronize(stream);
-    void* ptrs[] = {frame_dev, arena, col, input, cand, order, n_cand, mask, kept, n_kept, attr_dev};
+    void* ptrs[] = {frame_dev, arena, col, input, cand, order, n_cand, mask, results, list, n_list, attr_dev};
     for (void* p : ptrs) if (p) (void)hipFree(p);
+    if (results_host) (void)hipHostFree(results_host);
     if (exec) exec->unload(); /* before its stream goes */
     if (stream) (void)hipStreamDestroy(stream);
 }
@@ -677,8 +684,13 @@ bool TkDetector::init(TkYoloModel* m, int w, int h, int mb) {
     HIPQ(hipMalloc((void**)&order, (size_t)mb * TK_YOLO_MAX_CAND * 4));
     HIPQ(hipMalloc((void**)&n_cand, (size_t)mb * 4));
     HIPQ(hipMalloc((void**)&mask, (size_t)mb * TK_YOLO_MAX_CAND * (TK_YOLO_MAX_CAND / 64) * 8));
-    HIPQ(hipMalloc((void**)&kept, (size_t)mb * TK_OBJECT_DETECTOR_MAX_DETECTIONS * sizeof(TkDetection)));
-    HIPQ(hipMalloc((void**)&n_kept, (size_t)mb * 4));
+    HIPQ(hipMalloc((void**)&list, (size_t)mb * n_anchors * 8));
+    HIPQ(hipMalloc((void**)&n_list, (size_t)mb * 4));
+    kept_at = ((size_t)mb * 4 + 255) & ~(size_t)255;
+    HIPQ(hipMalloc((void**)&results, kept_at + (size_t)mb * TK_OBJECT_DETECTOR_MAX_DETECTIONS * sizeof(TkDetection)));
+    n_kept = (int32_t*)results;
+    kept = (TkDetection*)(results + kept_at);
+    HIPQ(hipHostMalloc((void**)&results_host, kept_at + (size_t)mb * TK_OBJECT_DETECTOR_MAX_DETECTIONS * sizeof(TkDetection), hipHostMallocDefault));
     return true;
 }
 
@@ -703,7 +715,7 @@ bool TkDetector::run_graph(int B, float* host_out) {
                     std::to_string(in_w) + " x " + std::to_string(in_h) + " at strides 8 / 16 / 32)";
             return false;
         }
-        hipLaunchKernelGGL(k_yolo_decode_out, dim3((n_anchors + 255) / 256), dim3(256), 0, stream, o->d, model->nc, n_anchors, conf, cand + (size_t)b * n_anchors);
+        hipLaunchKernelGGL(k_yolo_decode_out, dim3((n_anchors + 255) / 256), dim3(256), 0, stream, o->d, model->nc, n_anchors, conf, cand + (size_t)b * n_anchors, list + (size_t)b * n_anchors, n_list + b);
         if (host_out) HIPQ(hipMemcpyAsync(host_out + (size_t)b * o->count(), o->d, (size_t)o->count() * 4, hipMemcpyDeviceToHost, stream)); /* before the next run reuses the arena */
     }
     return true;
@@ -716,38 +728,49 @@ bool TkDetector::forward_graph(int B, const float* nchw_host, std::vector<float>
     HIPQ(hipMemcpyAsync(input, nchw_host, (size_t)B * 3 * in_h * in_w * 4, hipMemcpyHostToDevice, stream));
     out->assign((size_t)B * (4 + model->nc) * n_anchors, 0.0f);
     last_B = 0;
-    if (!run_graph(B, out->data())) return false;
-    hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
+    if (!begin_list() || !run_graph(B, out->data())) return false;
+    hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, list, n_list, n_anchors, order, n_cand);
     hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
-    hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept);
+    hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept, n_list);
     HIPQ(hipGetLastError());
+    list_clear = true;
     HIPQ(hipStreamSynchronize(stream));
     return true;
 }
 
+/* a pass that did not come to its end may have left counts behind */
+bool TkDetector::begin_list() {
+    if (!list_clear) HIPQ(hipMemsetAsync(n_list, 0, (size_t)max_batch * 4, stream));
+    list_clear = false;
+    return true;
+}
+
 bool TkDetector::enqueue(int B, const TkPreprocessArgs* frames) {
+    if (!begin_list()) return false;
     if (model->generic) {
         if (!run_graph(B, nullptr)) return false;
-        hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
+        hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, list, n_list, n_anchors, order, n_cand);
         hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
-        hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept);
+        hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept, n_list);
         HIPQ(hipGetLastError());
+        list_clear = true;
         return true;
     }
+    TkT x;
+    x.p = input; x.B = B; x.H = in_h; x.W = in_w; x.C = 3; x.ld = 3;
+    if (plans[B].empty()) plans[B].assign(model->specs.size(), TkConvPlan{});
     TkGpuOps ops;
     ops.d = this; ops.s = stream;
     ops.frames = frames;
     ops.frame_bytes = frames ? (size_t)frames->in_stride * frames->in_h : 0;
     arena_used = 0;
-    if (plans[B].empty()) plans[B].assign(model->specs.size(), TkConvPlan{});
-    TkT x;
-    x.p = input; x.B = B; x.H = in_h; x.W = in_w; x.C = 3; x.ld = 3;
     TkYoloV8n<TkGpuOps>::forward(ops, x, heads, model->nc);
-    hipLaunchKernelGGL(k_yolo_decode, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, heads[0], heads[1], heads[2], model->nc, n_anchors, conf, cand);
-    hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 255) / 256, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand);
+    hipLaunchKernelGGL(k_yolo_decode, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, heads[0], heads[1], heads[2], model->nc, n_anchors, conf, cand, list, n_list);
+    hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, list, n_list, n_anchors, order, n_cand);
     hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
-    hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept);
+    hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept, n_list);
     HIPQ(hipGetLastError());
+    list_clear = true;
     return true;
 }
 
@@ -905,14 +928,13 @@ bool tk_classify_boxes_host(int device, const uint8_t* frame, uint32_t w, uint32
 }
 
 bool TkDetector::fetch(int B, std::vector<std::vector<TkDetection>>* out) {
-    std::vector<int32_t> nk(B);
-    std::vector<TkDetection> hk((size_t)B * TK_OBJECT_DETECTOR_MAX_DETECTIONS);
-    HIPQ(hipMemcpyAsync(nk.data(), n_kept, B * 4, hipMemcpyDeviceToHost, stream));
-    HIPQ(hipMemcpyAsync(hk.data(), kept, hk.size() * sizeof(TkDetection), hipMemcpyDeviceToHost, stream));
+    /* counts and boxes in one copy to pinned memory (two to pageable memory were staged and waited for one by one) */
+    HIPQ(hipMemcpyAsync(results_host, results, kept_at + (size_t)B * TK_OBJECT_DETECTOR_MAX_DETECTIONS * sizeof(TkDetection), hipMemcpyDeviceToHost, stream));
     HIPQ(hipStreamSynchronize(stream));
+    const int32_t* nk = (const int32_t*)results_host;
+    const TkDetection* hk = (const TkDetection*)(results_host + kept_at);
     out->assign(B, {});
-    for (int b = 0; b < B; ++b)
-        (*out)[b].assign(hk.begin() + (size_t)b * TK_OBJECT_DETECTOR_MAX_DETECTIONS, hk.begin() + (size_t)b * TK_OBJECT_DETECTOR_MAX_DETECTIONS + nk[b]);
+    for (int b = 0; b < B; ++b) (*out)[b].assign(hk + (size_t)b * TK_OBJECT_DETECTOR_MAX_DETECTIONS, hk + (size_t)b * TK_OBJECT_DETECTOR_MAX_DETECTIONS + nk[b]);
     return true;
 }
 
