@@ -96,13 +96,15 @@ struct SharedDetector {
     }
     void run() {
         std::unique_lock<std::mutex> lk(mu);
+        int expect = 1;
         for (;;) {
             cv_req.wait(lk, [&] { return stop || !q.empty(); });
             if (stop) break;
-            /* give the other handles' callers a moment to arrive: a few hundred microseconds against a network of ~1.5 ms per frame */
-            if (handles > 1) {
+            /* give the other callers a moment to arrive, as many as there were last time: those of the last job and those that came while it ran.  (Waiting for every
+             * handle there is made a lone caller beside idle handles wait the 400 us each time, as long as half a network of one frame.) */
+            if (expect > 1) {
                 const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(400);
-                while ((int)q.size() < (handles < TK_DET_SHARED_MAX_BATCH ? handles : TK_DET_SHARED_MAX_BATCH) && !stop)
+                while ((int)q.size() < expect && !stop)
                     if (cv_req.wait_until(lk, until) == std::cv_status::timeout) break;
                 if (stop) break;
             }
@@ -153,6 +155,7 @@ struct SharedDetector {
             n_frames += job.size();
             if (job.size() > widest) widest = job.size();
             for (DetReq* r : job) r->done = true;
+            expect = (int)(job.size() + q.size()) < TK_DET_SHARED_MAX_BATCH ? (int)(job.size() + q.size()) : TK_DET_SHARED_MAX_BATCH;
             cv_done.notify_all();
         }
         /* whoever is still waiting is told so */
