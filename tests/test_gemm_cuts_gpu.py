@@ -1,0 +1,19 @@
+"""The tiled exact product in the cuts that its cost rule takes for small matrices (1, 2, 4, 6 and 8 M-tiles a workgroup over many blocks of rows): bit for bit the
+LDS-staged kernel, at row counts around the blocks' edges, with padded last tiles and columns, bias, activation and residual."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 15, 17, 33, 47, 65, 95, 97, 129, 200, 255, 257, 1500, 3001])
+@pytest.mark.parametrize("N,K,act,res", [(384, 384, 0, True), (1152, 384, 0, False), (1531, 384, 2, False), (384, 1536, 0, True), (50, 1152, 2, True), (768, 128, 0, False)])
+def test_cut_of_few_tiles_equals_staged(gpu, M, N, K, act, res):
+    rng = np.random.default_rng(M + N + K)
+    f = lambda *s: rng.normal(0, 1, s).astype(np.float32)
+    a, w, b, r = f(M, K), f(N, K) * np.float32(K ** -0.5), f(N), f(M, N) if res else None
+    cs, ct = np.empty((M, N), np.float32), np.empty((M, N), np.float32)
+    p = lambda x: x.ctypes.data_as(C.c_void_p) if x is not None else None
+    gpu.check(gpu.lib().tk_mi355x_gemm_pair(0, M, N, K, p(a), p(w), p(b), p(r), act, 0, p(cs), p(ct)))
+    assert np.array_equal(cs.view(np.uint32), ct.view(np.uint32))

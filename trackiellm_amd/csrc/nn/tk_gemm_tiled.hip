@@ -1,6 +1,8 @@
 /* tk_gemm_tiled.hip — see tk_gemm_tiled.h */
 #include "tk_gemm_tiled.h"
 
+#include <math.h>
+
 #include <atomic>
 #include <mutex>
 
@@ -303,15 +305,90 @@ bool tk_gemm_tiled_prepare_device() {
     return true;
 }
 
-bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
+static bool tw_valid(const TkTiledGemm& a) {
     if (a.nseg < 1 || a.nseg > 3 || a.ks < 1 || a.K <= 0 || a.K % (32 * a.ks) || a.nrows <= 0 || (a.wbytes != 2 && a.wbytes != 4) || (a.ks > 1 && a.nrows > TK_TW_MAX_BLOCK_ROWS)) return false;
     if ((a.per_seg || a.c_img) && a.ks != 1) return false;
     if (a.per_seg && (a.residual || a.c_img)) return false;
-    if (a.c_img && (a.n_valid % 16 || a.nseg != 1)) return false;
-    int row_tiles = 0;
-    for (int i = 0; i < a.nseg; ++i) row_tiles += a.row_tiles[i];
+    return !(a.c_img && (a.n_valid % 16 || a.nseg != 1));
+}
+static int tw_row_tiles(const TkTiledGemm& a) {
+    int n = 0;
+    for (int i = 0; i < a.nseg; ++i) n += a.row_tiles[i];
+    return n;
+}
+
+/* the rest of a cut, M-tiles of a workgroup and its waves given; false: no staging of this k range */
+static bool tw_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
+    if ((mt != 1 && mt != 2 && mt != 4 && mt != 6 && mt != 8 && mt != 16) || waves < 1 || waves > 8) return false;
+    const int row_tiles = tw_row_tiles(a), Kr = a.K / a.ks;
+    p->mt = mt;
+    p->waves = waves;
+    p->groups = (row_tiles + waves - 1) / waves;
+    p->ny = (a.nrows + mt * TK_TW_ROWS_PER_TILE - 1) / (mt * TK_TW_ROWS_PER_TILE);
+    /* k per ring slot: the largest multiple of 32 PF that divides the K range and fits a 64 KiB slot (rk / 16 * mt KiB) — a whole short
+     * range in one slot (`one`, up to 128 KiB) needs no ring.
+     * Many row blocks of 128 rows (the Whisper encoder's linears, 48000 rows): 32 KiB slots and two weight pieces in flight instead, so
+     * that TWO workgroups share a CU and one's ring fill and epilogue run under the other's MFMAs. */
+    const bool twin = p->ny > 1 && (mt == 8 || mt == 6) && Kr % 64 == 0;
+    p->one = mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES;
+    /* whole range: eight pieces of weights in flight where they divide it, but not all of it at once: 51872 x 256, f32, 1 and 32 rows 14.9 and 18.9 us with
+     * four, 18.2 and 22.6 with eight */
+    p->pf = mt == 16 || mt == 6 || twin ? 2 : p->one && Kr % 256 == 0 && Kr > 256 ? 8 : 4;
+    const int slot_kib = twin ? 32 : 64;
+    p->rk = p->one ? Kr : 0;
+    for (int c = (slot_kib * 16 / mt) / (32 * p->pf) * (32 * p->pf); p->rk == 0 && c >= 32 * p->pf; c -= 32 * p->pf)
+        if (Kr % c == 0) p->rk = c;
+    if (p->rk == 0) return false;
+    p->slot_bytes = twin ? slot_kib * 1024 : TK_TW_SLOT_BYTES;
+    p->lds = p->one ? (size_t)Kr * mt * 64 : (size_t)2 * p->slot_bytes;
+    return true;
+}
+
+/* What a launch costs, in cycles: a workgroup's staging (its whole activations, or a slot and the waits for the further ones), its chains of 8 cycles a k and M-tile, then the
+ * CU's further workgroups on the same pipe; or the weights, which every block of rows fetches from the L2 again, whichever is longer.  Fitted to 1 700 launches
+ * of 1 .. 48 000 rows against 384 x 384 .. 51 872 x 384. */
+static float tw_cost(const TkTiledGemm& a, const TkTiledPlan& p) {
+    const int row_tiles = tw_row_tiles(a), Kr = a.K / a.ks;
+    const float rounds = (float)p.groups * (float)p.ny * (float)a.ks * (1.0f / 256.0f), up = ceilf(rounds);
+    int side_by_side = (int)(163840 / p.lds) < 16 / p.waves ? (int)(163840 / p.lds) : 16 / p.waves;
+    if (side_by_side < 1) side_by_side = 1;
+    const int per = (p.waves + 3) / 4;
+    const float kib = (float)p.lds * (1.0f / 1024.0f), waits = p.one ? 0.0f : (float)(Kr / p.rk) * 1012.0f;
+    const float chain = (float)(per * p.mt * Kr) * 8.6f;
+    float turns = side_by_side > 1 ? 0.61f * rounds + 0.39f * up : up;
+    turns = turns > 1.0f ? turns - 1.0f : 0.0f;
+    const float again = 0.25f * (float)(p.waves * p.mt) * (float)Kr * 10.3f + 21.0f * (float)(p.waves * p.mt) + 0.5f * waits / (float)side_by_side + (p.one ? 24.0f * kib : 0.0f);
+    const float pipe = 1100.0f + (p.one ? 158.0f * kib : 1030.0f) + chain + waits + turns * again;
+    const float weights = 1100.0f + (float)p.ny * (float)row_tiles * 16.0f * (float)a.K * (float)a.wbytes * (1.0f / 4100.0f);
+    return pipe > weights ? pipe + 0.15f * weights : weights + 0.15f * pipe;
+}
+
+static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p);
+bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
+    if (!tw_valid(a)) return false;
+    if (mt > 0) return tw_plan(a, mt, waves, p);
+    if (!tw_usual(a, p)) return false;
+    /* As many rows as possible behind one reading of the weights is what counts where these are large.  Small matrices (up to 24 MB: they come from the caches) of few
+     * tiles leave most of the chip idle that way: fewer M-tiles a workgroup, where that is clearly quicker by the costs, measured 384 x 384 at 32, 256 and 1500 rows
+     * 7.8 -> 5.6, 41 -> 5.4, 26.5 -> 10.4 us, 384 x 1536 20.3 -> 11.9, 123 -> 12.0, 87 -> 36.  No cut reads rows of the image that the usual one does not. */
+    const TkTiledPlan usual = *p;
+    if ((size_t)tw_row_tiles(a) * 16 * (size_t)a.K * (size_t)a.wbytes > 24000000u || (int64_t)tw_row_tiles(a) * usual.ny * a.ks >= 4096) return true;
+    float least = 0.93f * tw_cost(a, usual);
+    const int mts[5] = {1, 2, 4, 6, 8}, wvs[3] = {2, 4, 8};
+    for (int m : mts)
+        for (int w : wvs) {
+            TkTiledPlan q;
+            if (!tw_plan(a, m, w, &q) || (m == 1 && !q.one) || q.ny * q.mt > usual.ny * usual.mt || q.ny > 65535) continue;
+            const float c = tw_cost(a, q);
+            if (c < least) { least = c; *p = q; }
+        }
+    return true;
+}
+static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
+    int mt, waves;
+    const int row_tiles = tw_row_tiles(a);
     const int rows_blk = a.nrows < TK_TW_MAX_BLOCK_ROWS ? a.nrows : TK_TW_MAX_BLOCK_ROWS;
-    int mt = rows_blk > 128 ? 16 : rows_blk > 64 ? 8 : rows_blk > 32 ? 4 : rows_blk > 16 ? 2 : 1;
+    mt = rows_blk > 128 ? 16 : rows_blk > 64 ? 8 : rows_blk > 32 ? 4 : rows_blk > 16 ? 2 : 1;
     if (mt == 16 && a.nrows > TK_TW_MAX_BLOCK_ROWS && (a.K / a.ks) % 64 == 0) {
         /* many row blocks: two workgroups per CU (below), 512 at a time on the chip; of 128- and 96-row blocks the one whose last round
          * wastes less (N = 384 at 48 000 rows: 1 125 workgroups = 3 rounds of 8 M-tiles against 1 500 = 3 rounds of 6) */
@@ -324,9 +401,8 @@ bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
     const int ny = (a.nrows + mt * TK_TW_ROWS_PER_TILE - 1) / (mt * TK_TW_ROWS_PER_TILE);
     /* one pass of <= 256 rows (the LLM): spread the row tiles over the CUs, K-split ranges side by side; many row blocks: eight tiles
      * per workgroup share one activation ring */
-    int groups, waves;
     if (ny == 1) {
-        groups = 256 / a.ks;
+        int groups = 256 / a.ks;
         if (groups < 1) groups = 1;
         if (groups > row_tiles) groups = row_tiles;
         waves = (row_tiles + groups - 1) / groups;
@@ -336,39 +412,30 @@ bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
             waves = mt == 1 ? 2 : 4;
             groups = (row_tiles + waves - 1) / waves;
         }
-    } else {
-        waves = row_tiles < 8 ? row_tiles : 8;
-        groups = (row_tiles + waves - 1) / waves;
+        if (!tw_plan(a, mt, waves, p)) return false;
+        p->groups = groups;
+        return true;
     }
-    const int Kr = a.K / a.ks;
-    /* k per ring slot: the largest multiple of 32 PF that divides the K range and fits a 64 KiB slot (rk / 16 * mt KiB) — a whole short
-     * range in one slot (`one`, up to 128 KiB) needs no ring.
-     * Many row blocks of 128 rows (the Whisper encoder's linears, 48000 rows): 32 KiB slots and two weight pieces in flight instead, so
-     * that TWO workgroups share a CU and one's ring fill and epilogue run under the other's MFMAs. */
-    const bool twin = ny > 1 && (mt == 8 || mt == 6) && Kr % 64 == 0;
-    const bool one = mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES;
-    /* whole range: eight pieces of weights in flight where they divide it, but not all of it at once: 51872 x 256, f32, 1 and 32 rows 14.9 and 18.9 us with
-     * four, 18.2 and 22.6 with eight */
-    const int pf = mt == 16 || twin ? 2 : one && Kr % 256 == 0 && Kr > 256 ? 8 : 4;
-    const int slot_kib = twin ? 32 : 64;
-    int rk = one ? Kr : 0;
-    for (int c = (slot_kib * 16 / mt) / (32 * pf) * (32 * pf); rk == 0 && c >= 32 * pf; c -= 32 * pf)
-        if (Kr % c == 0) { rk = c; break; }
-    if (rk == 0) return false;
-    if (Kr % rk) return false;
-    const int slot_bytes = twin ? slot_kib * 1024 : TK_TW_SLOT_BYTES;
-    const size_t ldsb = one ? (size_t)Kr * mt * 64 : (size_t)2 * slot_bytes;
-#define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(groups * a.ks, ny), dim3(64 * waves), ldsb, s, a, groups, row_tiles, rk, slot_bytes)
+    return tw_plan(a, mt, row_tiles < 8 ? row_tiles : 8, p);
+}
+
+bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipStream_t s) {
+    const int row_tiles = tw_row_tiles(a);
+#define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
 #define TK_TW_WB(MTV, ONEV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, ONEV, PFV); else TK_TW_LAUNCH(MTV, 4, ONEV, PFV); } while (0)
-    switch (mt) {
-        case 1: if (one) { if (pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
-        case 2: if (one) { if (pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
+    switch (p.mt) {
+        case 1: if (p.one) { if (p.pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
+        case 2: if (p.one) { if (p.pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
         case 4: TK_TW_WB(4, false, 4); break;
         case 6: TK_TW_WB(6, false, 2); break;
-        case 8: if (twin) TK_TW_WB(8, false, 2); else TK_TW_WB(8, false, 4); break;
+        case 8: if (p.pf == 2) TK_TW_WB(8, false, 2); else TK_TW_WB(8, false, 4); break;
         default: TK_TW_WB(16, false, 2); break;
     }
 #undef TK_TW_WB
 #undef TK_TW_LAUNCH
     return true;
+}
+bool tk_launch_gemm_tiled(const TkTiledGemm& a, hipStream_t s) {
+    TkTiledPlan p;
+    return tk_gemm_tiled_plan(a, 0, 0, &p) && tk_launch_gemm_tiled_plan(a, p, s);
 }
