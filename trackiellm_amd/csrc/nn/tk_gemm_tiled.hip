@@ -354,7 +354,8 @@ static float tw_cost(const TkTiledGemm& a, const TkTiledPlan& p) {
     if (side_by_side < 1) side_by_side = 1;
     const int per = (p.waves + 3) / 4;
     const float kib = (float)p.lds * (1.0f / 1024.0f), waits = p.one ? 0.0f : (float)(Kr / p.rk) * 1012.0f;
-    const float chain = (float)(per * p.mt * Kr) * 8.6f;
+    const float lone = (float)side_by_side < up ? (float)side_by_side : up;
+    const float chain = (float)(per * p.mt * Kr) * ((float)(per * p.mt) * lone <= 1.0f ? 6.0f : 8.6f);
     float turns = side_by_side > 1 ? 0.61f * rounds + 0.39f * up : up;
     turns = turns > 1.0f ? turns - 1.0f : 0.0f;
     const float again = 0.25f * (float)(p.waves * p.mt) * (float)Kr * 10.3f + 21.0f * (float)(p.waves * p.mt) + 0.5f * waits / (float)side_by_side + (p.one ? 24.0f * kib : 0.0f);
