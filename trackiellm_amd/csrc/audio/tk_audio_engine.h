@@ -88,9 +88,7 @@ private:
 class TkVadModel {
 public:
     int device = 0, window = 480, hidden = 64;
-    float *w1 = nullptr, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
-    float *x = nullptr, *hbuf = nullptr, *p = nullptr; /* grow-only scratch */
-    int cap = 0;
+    float *w1 = nullptr /* [window / 4][hidden][4] */, *b1 = nullptr, *w2 = nullptr, *b2 = nullptr;
     hipStream_t stream = nullptr;
     std::string error;
     ~TkVadModel();
@@ -98,6 +96,12 @@ public:
     bool fill_synthetic(uint64_t seed);
     /* windows: [n][window] float on the host -> probabilities[n] */
     bool infer(const float* windows_host, int n, float* prob_host);
+
+private:
+    enum { TK_VAD_CHUNK = 512 }; /* windows of a slot at most */
+    struct Slot { float* x = nullptr; int cap = 0; hipEvent_t done = nullptr; }; /* pinned: [cap][window], then [cap] probabilities */
+    Slot slots[2];
+    bool reserve(Slot& s, int n);
 };
 
 #endif

@@ -892,15 +892,20 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
 TkVadModel::~TkVadModel() {
     (void)hipSetDevice(device);
     if (stream) (void)hipStreamSynchronize(stream);
-    float* ptrs[] = {w1, b1, w2, b2, x, hbuf, p};
+    float* ptrs[] = {w1, b1, w2, b2};
     for (float* q : ptrs) if (q) (void)hipFree(q);
+    for (Slot& s : slots) {
+        if (s.x) (void)hipHostFree(s.x);
+        if (s.done) (void)hipEventDestroy(s.done);
+    }
     if (stream) (void)hipStreamDestroy(stream);
 }
 
 bool TkVadModel::init(int dev, int win, int hid) {
     device = dev; window = win; hidden = hid;
+    if (win < 4 || (win & 3) || hid < 1 || hid > 64) { error = "VAD windows are whole groups of four samples, its hidden layer has at most 64 units"; return false; }
     HIPQ(hipSetDevice(device));
-    HIPQ(hipMalloc((void**)&w1, (size_t)hid * win * 4));
+    HIPQ(hipMalloc((void**)&w1, (size_t)win * hid * 4));
     HIPQ(hipMalloc((void**)&b1, (size_t)hid * 4));
     HIPQ(hipMalloc((void**)&w2, (size_t)hid * 4));
     HIPQ(hipMalloc((void**)&b2, 4));
@@ -910,47 +915,111 @@ bool TkVadModel::init(int dev, int win, int hid) {
 bool TkVadModel::fill_synthetic(uint64_t seed) {
     std::vector<float> a((size_t)hidden * window), b(hidden), c(hidden), d(1);
     tk_vad_synth(seed, window, hidden, a.data(), b.data(), c.data(), d.data());
+    /* [hidden][window] -> [window / 4][hidden][4]: a lane per hidden unit reads four of its weights at a time */
+    std::vector<float> t(a.size());
+    for (int h = 0; h < hidden; ++h)
+        for (int k = 0; k < window; ++k) t[((size_t)(k >> 2) * hidden + h) * 4 + (k & 3)] = a[(size_t)h * window + k];
     HIPQ(hipSetDevice(device));
-    HIPQ(hipMemcpy(w1, a.data(), a.size() * 4, hipMemcpyHostToDevice));
+    HIPQ(hipMemcpy(w1, t.data(), t.size() * 4, hipMemcpyHostToDevice));
     HIPQ(hipMemcpy(b1, b.data(), b.size() * 4, hipMemcpyHostToDevice));
     HIPQ(hipMemcpy(w2, c.data(), c.size() * 4, hipMemcpyHostToDevice));
     HIPQ(hipMemcpy(b2, d.data(), 4, hipMemcpyHostToDevice));
     return true;
 }
 
-/* relu is not in TkAct: hidden = max(0, .) is folded into a tiny kernel together with the second layer */
-__global__ void k_vad_head(const float* hid, int n, int hidden, const float* w2, const float* b2, float* prob) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+/* A workgroup per window, a lane per hidden unit: its chain over the window, relu, then one lane's chain over the hidden units.  Windows are read from, and probabilities
+ * written to, pinned host memory: one launch and one wait make a call, where a copy, two launches, a copy and a wait took 47 us for 33 windows of 480.  What is left is the
+ * launch, the trip over the bus and the chain of `window` fmas. */
+#define TK_VAD_AHEAD 20 /* groups of four weights on their way, twice */
+__global__ __launch_bounds__(64) void k_vad(const float* x, int window, int hidden, const float* __restrict__ w1, const float* __restrict__ b1, const float* __restrict__ w2,
+                                            const float* __restrict__ b2, float* prob) {
+    extern __shared__ __attribute__((aligned(16))) float vad_lds[];
+    float* hs = vad_lds + window; /* [hidden] behind the window */
+    const int t = threadIdx.x, groups = window >> 2, unit = t < hidden ? t : hidden - 1;
+    const at1_f32x4* wp = (const at1_f32x4*)w1 + unit;
+    at1_f32x4 w[2][TK_VAD_AHEAD];
+    auto load = [&](int set, int g0) { /* past the end: the last group again */
+#pragma unroll
+        for (int i = 0; i < TK_VAD_AHEAD; ++i) w[set][i] = wp[(g0 + i < groups ? g0 + i : groups - 1) * hidden];
+    };
+    load(0, 0);
+    const at1_f32x4* row = (const at1_f32x4*)(x + (int64_t)blockIdx.x * window);
+    for (int i = t; i < groups; i += 64) ((at1_f32x4*)vad_lds)[i] = row[i];
+    __syncthreads();
     float acc = 0.0f;
-    for (int k = 0; k < hidden; ++k) acc = tk_fmaf(tk_fmaxf(hid[(int64_t)i * hidden + k], 0.0f), w2[k], acc);
-    prob[i] = tk_sigmoidf(acc + b2[0]);
+    for (int g0 = 0; g0 < groups; g0 += 2 * TK_VAD_AHEAD) {
+#pragma unroll
+        for (int set = 0; set < 2; ++set) {
+            const int base = g0 + set * TK_VAD_AHEAD;
+            load(set ^ 1, base + TK_VAD_AHEAD);
+#pragma unroll
+            for (int i = 0; i < TK_VAD_AHEAD; ++i)
+                if (base + i < groups) {
+                    const at1_f32x4 v = ((const at1_f32x4*)vad_lds)[base + i];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc = tk_fmaf(v[j], w[set][i][j], acc);
+                }
+        }
+    }
+    if (t < hidden) hs[t] = tk_fmaxf(acc + b1[unit], 0.0f);
+    __syncthreads();
+    if (t == 0) {
+        float a = 0.0f;
+        for (int k = 0; k < hidden; ++k) a = tk_fmaf(hs[k], w2[k], a);
+        prob[blockIdx.x] = tk_sigmoidf(a + b2[0]);
+    }
+}
+
+/* pinned memory for one slot's windows and, behind them, their probabilities */
+bool TkVadModel::reserve(Slot& s, int n) {
+    if (n > s.cap) {
+        if (s.x) (void)hipHostFree(s.x); /* (a slot grows between calls or before its first use) */
+        s.x = nullptr;
+        s.cap = 0;
+        const int want = n < 128 ? 128 : n;
+        HIPQ(hipHostMalloc((void**)&s.x, (size_t)want * (window + 1) * 4, hipHostMallocDefault));
+        s.cap = want;
+    }
+    if (!s.done) HIPQ(hipEventCreateWithFlags(&s.done, hipEventDisableTiming));
+    return true;
 }
 
 bool TkVadModel::infer(const float* windows_host, int n, float* prob_host) {
     if (n <= 0) return true;
     HIPQ(hipSetDevice(device));
     if (!stream) HIPQ(tk_create_perception_stream(&stream));
-    if (n > cap) { /* grow-only scratch: no allocation on the steady-state path */
-        if (x) (void)hipFree(x);
-        if (hbuf) (void)hipFree(hbuf);
-        if (p) (void)hipFree(p);
-        x = hbuf = p = nullptr;
-        cap = 0;
-        const int want = n < 128 ? 128 : n;
-        HIPQ(hipMalloc((void**)&x, (size_t)want * window * 4));
-        HIPQ(hipMalloc((void**)&hbuf, (size_t)want * hidden * 4));
-        HIPQ(hipMalloc((void**)&p, (size_t)want * 4));
-        cap = want;
+    auto launch = [&](Slot& s, int count) {
+        hipLaunchKernelGGL(k_vad, dim3(count), dim3(64), (size_t)(window + hidden) * 4, stream, s.x, window, hidden, w1, b1, w2, b2, s.x + (size_t)s.cap * window);
+        return hipGetLastError();
+    };
+    if (n <= TK_VAD_CHUNK) {
+        Slot& s = slots[0];
+        if (!reserve(s, n)) return false;
+        memcpy(s.x, windows_host, (size_t)n * window * 4);
+        HIPQ(launch(s, n));
+        HIPQ(hipStreamSynchronize(stream));
+        memcpy(prob_host, s.x + (size_t)s.cap * window, (size_t)n * 4);
+        return true;
     }
-    HIPQ(hipMemcpyAsync(x, windows_host, (size_t)n * window * 4, hipMemcpyHostToDevice, stream));
-    TkGemm g{};
-    g.A = x; g.B = w1; g.C = hbuf; g.bias = b1; g.M = n; g.N = hidden; g.K = window; g.lda = window; g.ldb = window; g.ldc = hidden;
-    g.alpha = 1.0f; g.batch = 1;
-    tk_launch_gemm(g, stream);
-    hipLaunchKernelGGL(k_vad_head, dim3((n + 63) / 64), dim3(64), 0, stream, hbuf, n, hidden, w2, b2, p);
-    HIPQ(hipGetLastError());
-    HIPQ(hipMemcpyAsync(prob_host, p, (size_t)n * 4, hipMemcpyDeviceToHost, stream));
-    HIPQ(hipStreamSynchronize(stream));
+    /* many windows: in turn through two slots, so that one is filled while the other is worked on */
+    int from[2] = {0, 0}, count[2] = {0, 0};
+    auto fetch = [&](int i) {
+        HIPQ(hipEventSynchronize(slots[i].done));
+        memcpy(prob_host + from[i], slots[i].x + (size_t)slots[i].cap * window, (size_t)count[i] * 4);
+        count[i] = 0;
+        return true;
+    };
+    int at = 0, i = 0;
+    for (; at < n; at += TK_VAD_CHUNK, i ^= 1) {
+        Slot& s = slots[i];
+        if ((count[i] > 0 && !fetch(i)) || !reserve(s, TK_VAD_CHUNK)) { (void)hipStreamSynchronize(stream); return false; }
+        from[i] = at;
+        count[i] = n - at < TK_VAD_CHUNK ? n - at : TK_VAD_CHUNK;
+        memcpy(s.x, windows_host + (size_t)at * window, (size_t)count[i] * window * 4);
+        const hipError_t e = launch(s, count[i]);
+        if (e != hipSuccess || hipEventRecord(s.done, stream) != hipSuccess) { (void)hipStreamSynchronize(stream); error = "launching the VAD failed"; return false; }
+    }
+    for (int k = 0; k < 2; ++k)
+        if (count[k] > 0 && !fetch(k)) { (void)hipStreamSynchronize(stream); return false; }
     return true;
 }
