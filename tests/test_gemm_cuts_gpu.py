@@ -17,3 +17,18 @@ def test_cut_of_few_tiles_equals_staged(gpu, M, N, K, act, res):
     p = lambda x: x.ctypes.data_as(C.c_void_p) if x is not None else None
     gpu.check(gpu.lib().tk_mi355x_gemm_pair(0, M, N, K, p(a), p(w), p(b), p(r), act, 0, p(cs), p(ct)))
     assert np.array_equal(cs.view(np.uint32), ct.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("width", [64, 128, 384, 768, 1024, 1152])
+def test_norms_inside_products_of_a_few_rows(gpu, width):
+    """a decoder's norms are made by the products behind them for up to four sequences and widths of 128 .. 1024 in steps of 128, as launches else: tokens and logits of
+    a clip are the same bits whatever number of clips runs with it"""
+    hp = gpu.WhisperHP(80, 40, 128, 2, 1, 24, width, width // 64, 2, 515)
+    asr = gpu.Asr(hp=hp, seed=9, max_batch=6)
+    pcm = np.random.default_rng(width).integers(-6000, 6000, (6, 5000)).astype(np.int16)
+    ids, mel, enc, logits = asr.transcribe_tokens(pcm, 5)
+    for n in (1, 2, 3, 4, 5):
+        i2, m2, e2, l2 = asr.transcribe_tokens(pcm[:n], 5)
+        assert np.array_equal(i2, ids[:n]) and np.array_equal(l2.view(np.uint32), logits[:n].view(np.uint32))
+        assert np.array_equal(m2.view(np.uint32), mel[:n].view(np.uint32)) and np.array_equal(e2.view(np.uint32), enc[:n].view(np.uint32))

@@ -389,6 +389,16 @@ struct TkAudioGpuOps {
      * once.  It sits on top of the arena and is dropped — its space handed back — by every other op, by any allocation of the graph and
      * by a GEMM that writes into the matrix it was made from. */
     struct { const float* A = nullptr; int M = 0, K = 0, lda = 0; float* img = nullptr; size_t mark = 0; bool live = false; } pk;
+    /* Decoder steps of few sequences: a norm is not launched; the linear layers on it make it themselves (TkTiledGemm::ln_x).  pk then names its output, which nobody else
+     * reads, and has no image.  A layer that cannot take it has it launched first. */
+    struct { const float *x = nullptr, *w = nullptr, *b = nullptr; float* y = nullptr; bool live = false, used = false; } norm;
+    static bool norm_fits(int rows, int D) { return rows <= TK_TW_LN_ROWS && D <= TK_TW_LN_MAX && D % 128 == 0; }
+    void make_norm() { /* as a launch after all, with its image */
+        const int M = pk.M, K = pk.K;
+        norm.live = false;
+        float* img = image_for(norm.y, M, K, K);
+        tk_launch_layernorm(norm.x, M, K, norm.w, norm.b, TK_WH_LN_EPS, norm.y, s, img);
+    }
     /* linear layers on the SAME packed input (q / k / v of a layer, the cross keys and values) are collected — up to three — and go out as ONE
      * launch with a destination per segment (q | k | v: the query buffer and row p of the two caches); anything else flushes the batch first */
     struct { TkTiledGemm t{}; int n = 0; } pend;
@@ -403,7 +413,9 @@ struct TkAudioGpuOps {
     }
     void drop_image() {
         flush();
-        if (pk.live) { a->arena_used = pk.mark; pk.live = false; }
+        if (norm.live && !norm.used) make_norm(); /* (its readers are not linear layers) */
+        if (pk.live && !norm.live) a->arena_used = pk.mark;
+        pk.live = norm.live = false;
     }
     float* alloc(size_t n) {
         drop_image();
@@ -442,7 +454,13 @@ struct TkAudioGpuOps {
             return;
         }
         const int idx = tk_tiled_gemm_applies(g) ? a->model->tensor_of(g.B) : -1;
-        if (idx < 0 || !a->model->wt[(size_t)idx]) { drop_image(); tk_launch_gemm(g, s); return; }
+        if (idx < 0 || !a->model->wt[(size_t)idx]) {
+            if (norm.live) make_norm();
+            drop_image();
+            tk_launch_gemm(g, s);
+            return;
+        }
+        if (norm.live && !(pk.A == g.A && pk.M == g.M && pk.K == g.K && pk.lda == g.lda)) drop_image();
         if (!(pk.live && pk.A == g.A && pk.M == g.M && pk.K == g.K && pk.lda == g.lda)) {
             drop_image();
             pk.mark = a->arena_used;
@@ -458,12 +476,13 @@ struct TkAudioGpuOps {
         const bool in_place = c0 < a1 && a0 < c1;
         const bool plain = !g.residual && !g.c_feeds_linear && g.N % 16 == 0 && !in_place; /* an in-place layer never joins a batch: it runs alone below */
         if (plain) { /* joins (or opens) the batch of layers on this input */
-            if (pend.n > 0 && (pend.t.a_img != pk.img || pend.t.K != g.K || pend.t.nrows != g.M || pend.t.act != g.act)) flush();
+            if (pend.n > 0 && (pend.t.a_img != (norm.live ? nullptr : pk.img) || pend.t.ln_x != (norm.live ? norm.x : nullptr) || pend.t.K != g.K || pend.t.nrows != g.M || pend.t.act != g.act)) flush();
             TkTiledGemm& t = pend.t;
             if (pend.n == 0) {
                 t = TkTiledGemm{};
-                t.wbytes = 4; t.K = g.K; t.ks = 1; t.nrows = g.M; t.slab_rows = 0; t.a_img = pk.img; t.a_ts = (size_t)g.K * 16;
+                t.wbytes = 4; t.K = g.K; t.ks = 1; t.nrows = g.M; t.slab_rows = 0; t.a_img = norm.live ? nullptr : pk.img; t.a_ts = (size_t)g.K * 16;
                 t.act = g.act; t.add_zero_bias = 1; t.per_seg = 1;
+                use_norm(t);
             }
             const int i = pend.n++;
             t.tiles[i] = a->model->wt[(size_t)idx]; t.row_tiles[i] = g.N / 16;
@@ -475,7 +494,8 @@ struct TkAudioGpuOps {
         TkTiledGemm t{};
         t.tiles[0] = a->model->wt[(size_t)idx]; t.row_tiles[0] = (g.N + 15) / 16; t.nseg = 1; t.wbytes = 4;
         t.K = g.K; t.ks = 1; t.ldc = g.ldc; t.n_valid = g.N; t.nrows = g.M; t.slab_rows = 0;
-        t.a_img = pk.img; t.a_ts = (size_t)g.K * 16; t.out = g.C;
+        t.a_img = norm.live ? nullptr : pk.img; t.a_ts = (size_t)g.K * 16; t.out = g.C;
+        use_norm(t);
         t.bias = g.bias; t.residual = g.residual; t.ldr = g.ldr; t.act = g.act; t.add_zero_bias = 1;
         /* fc1: its output is only ever the input of fc2 — written as fc2's operand image as well (on top of fc1's own), on long (encoder) passes
          * too: there the second image replaces a k_pack_a launch over B x 1500 x 4 d values (9.8 -> 9.4 ms per call, profiles/r04_perception.txt) */
@@ -484,19 +504,31 @@ struct TkAudioGpuOps {
         if (emit_img) {
             TkGemm nx{};
             nx.M = g.M; nx.K = g.N;
+            if (norm.live) pk.mark = a->arena_used; /* (the norm has no image below it) */
             cimg = raw_alloc(tk_tiled_gemm_scratch(nx));
             t.c_img = cimg;
         }
         if (!tk_launch_gemm_tiled(t, s)) tk_launch_gemm(g, s); /* not reached: tk_tiled_gemm_applies() admits only shapes the launcher takes */
         if (emit_img) { /* the image pair stays allocated from pk.mark up; the upper one is now the live image */
             pk.img = cimg; pk.A = g.C; pk.M = g.M; pk.K = g.N; pk.lda = g.ldc; pk.live = true;
+            norm.live = false;
             return;
         }
         if (in_place) drop_image(); /* the output overwrote the packed matrix: the image is stale */
     }
+    void use_norm(TkTiledGemm& t) {
+        if (!norm.live) return;
+        norm.used = true;
+        t.ln_x = norm.x; t.ln_w = norm.w; t.ln_b = norm.b; t.ln_eps = TK_WH_LN_EPS;
+    }
     void im2col1d(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* col) { drop_image(); tk_launch_im2col1d(x, B, T, C, ldx, kw, stride, pad, col, s); }
     void layernorm(const float* x, int rows, int D, const float* w, const float* b, float* y) {
         drop_image();
+        if (!long_ok && norm_fits(rows, D)) { /* a decoder step's: it feeds linear layers only */
+            norm.x = x; norm.w = w; norm.b = b; norm.y = y; norm.live = true; norm.used = false;
+            pk.A = y; pk.M = rows; pk.K = D; pk.lda = D; pk.img = nullptr; pk.mark = a->arena_used; pk.live = true;
+            return;
+        }
         float* img = D % 128 == 0 && !(a->fast && long_ok) ? image_for(y, rows, D, D) : nullptr; /* a norm feeds linear layers: packed on the way out */
         tk_launch_layernorm(x, rows, D, w, b, TK_WH_LN_EPS, y, s, img);
     }

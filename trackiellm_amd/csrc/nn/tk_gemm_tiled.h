@@ -55,7 +55,13 @@ struct TkTiledGemm {
     int seg_n[3];
     /* c_img: the output is ALSO written as the operand image of the next linear layer (K = n_valid), so no pack launch follows */
     float* c_img;
+    /* ln_x: the activations are the layer norm of its rows ([nrows][K], dense), made by every workgroup for itself (f32 tiles, ks == 1, at most TK_TW_LN_ROWS rows of at
+     * most TK_TW_LN_MAX columns, K % 128 == 0); a_img is not read */
+    const float *ln_x, *ln_w, *ln_b;
+    float ln_eps;
 };
+#define TK_TW_LN_ROWS 4
+#define TK_TW_LN_MAX 1024
 
 /* false (nothing launched): K / ks is not a multiple of the ring granularity (128 k; 64 k from 129 rows per block on) or a field is inconsistent */
 bool tk_launch_gemm_tiled(const TkTiledGemm& g, hipStream_t s);

@@ -48,7 +48,62 @@ __device__ __forceinline__ float tw_act(float v, int act) {
  * Cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us and 51872 x 384 24.0 -> 22.0 with four, 384 x 1536 13.9 -> 10.2 with eight; at 32 rows
  * 8.6 -> 7.9, 30.0 -> 27.0 with four, 20.8 -> 18.9 (ring).  Twelve pieces: 384 x 384 at 1 row 5.6 (a wave's requests queue in front of the activations
  * of the others). */
-template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */>
+/*
+ * Layer norm of the workgroup's rows into the one slot of activations (TkTiledGemm::ln_x): a wave a row, k_layernorm's arithmetic in its order — 256 partial sums over
+ * columns p, p + 256, ..., folded within groups of 64 by halves, the four groups left to right — with the four groups side by side in a wave's lanes.  A decoder step of
+ * one sequence has 13 norms; as launches of their own they took 2.9 us each, and the 12 products behind them waited for a trip to memory more.
+ */
+__device__ __forceinline__ void tw_layernorm(const TkTiledGemm& a, int row0, int rows, float* image, int wave, int nw, int lane) {
+    constexpr int NV = TK_TW_LN_MAX / 256;
+    const int D = a.K;
+    auto fold = [&](float (&s)[4]) {
+#pragma unroll
+        for (int m = 32; m >= 1; m >>= 1)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) s[w] = s[w] + __shfl_xor(s[w], m, 64);
+        return ((s[0] + s[1]) + s[2]) + s[3];
+    };
+    for (int r = wave; r < rows; r += nw) {
+        const float* xr = a.ln_x + (size_t)(row0 + r) * D;
+        float v[NV][4], wv[NV][4], bv[NV][4];
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                int i = 256 * u + 64 * w + lane;
+                i = i < D ? i : D - 1;
+                v[u][w] = xr[i]; wv[u][w] = a.ln_w[i]; bv[u][w] = a.ln_b[i];
+            }
+        float s[4];
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            s[w] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NV; ++u)
+                if (256 * u + 64 * w + lane < D) s[w] = s[w] + v[u][w];
+        }
+        const float mean = tk_divf(fold(s), (float)D);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            s[w] = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NV; ++u)
+                if (256 * u + 64 * w + lane < D) { const float d = v[u][w] - mean; s[w] = tk_fmaf(d, d, s[w]); }
+        }
+        const float var = tk_divf(fold(s), (float)D);
+        const float rstd = tk_divf(1.0f, tk_sqrtf(var + a.ln_eps));
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const int i = 256 * u + 64 * w + lane;
+                if (i < D) image[(i >> 4) * 256 + (i & 3) * 64 + r * 4 + ((i & 15) >> 2)] = ((v[u][w] - mean) * rstd) * wv[u][w] + bv[u][w];
+            }
+    }
+}
+
+template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */,
+          bool LN = false /* the activations are made here (MT = 1, ONE) */>
 __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, int total_row_tiles, int rk /* k per ring slot */, int slot_bytes /* ring slot pitch */) {
     constexpr int LPC = WB == 4 ? 2 : 1; /* 16-byte requests per piece and lane */
     constexpr int PIECE = 512 * WB;      /* bytes of one (row tile, 32 k) piece */
@@ -97,8 +152,18 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         dst[0] = tw_ldg_nt(p);
         if (LPC == 2) dst[LPC - 1] = tw_ldg_nt(p + 16);
     };
-    stage(0, 0);
-    if (!active) { /* no tile of its own: its share of the staging */
+    if (LN) {
+        if (active) {
+#pragma unroll
+            for (int i = 0; i < PF; ++i) wload(i, wq[i]);
+        }
+        tw_layernorm(a, row0, rows_here, (float*)lds, wave, nw, lane);
+        __syncthreads();
+        if (!active) return;
+    } else {
+        stage(0, 0);
+    }
+    if (!LN && !active) { /* no tile of its own: its share of the staging */
         for (int s = 0; s < nslots; ++s) {
             tw_wait_vmcnt(0);
             __syncthreads();
@@ -106,15 +171,19 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         }
         return;
     }
+    if (!LN) {
 #pragma unroll
-    for (int i = 0; i < PF; ++i) wload(i, wq[i]);
+        for (int i = 0; i < PF; ++i) wload(i, wq[i]);
+    }
 
 #pragma unroll 1
     for (int s = 0; s < (ONE ? 1 : nslots); ++s) {
         /* slot s has landed once all but the PF * LPC youngest requests are done: those are weight requests issued after its DMA
          * (cps >= PF chunks follow every slot's DMA, the PF initial ones the first) */
-        tw_wait_vmcnt(PF * LPC);
-        __syncthreads();
+        if (!LN) {
+            tw_wait_vmcnt(PF * LPC);
+            __syncthreads();
+        }
         if (!ONE && s + 1 < nslots) stage(s + 1, (s + 1) & 1);
         const uint8_t* slot = lds + (size_t)(ONE ? 0 : s & 1) * slot_bytes + lane * 16;
         /* operands of M-tiles m, m + 1 (m alone of MT = 1) and chunk cc of the slot; [k half][tile] */
@@ -300,6 +369,8 @@ bool tk_gemm_tiled_prepare_device() {
     TK_TW_OPT(1, true, 4); TK_TW_OPT(1, true, 8); TK_TW_OPT(2, true, 4); TK_TW_OPT(2, true, 8);
     TK_TW_OPT(1, false, 4); TK_TW_OPT(2, false, 4); TK_TW_OPT(4, false, 4); TK_TW_OPT(8, false, 4); TK_TW_OPT(16, false, 2); TK_TW_OPT(8, false, 2); TK_TW_OPT(6, false, 2);
 #undef TK_TW_OPT
+    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 4, true>);
+    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 8, true>);
     if (e != hipSuccess) return false;
     g_tw_opted[dev].store(true, std::memory_order_release);
     return true;
@@ -309,6 +380,7 @@ static bool tw_valid(const TkTiledGemm& a) {
     if (a.nseg < 1 || a.nseg > 3 || a.ks < 1 || a.K <= 0 || a.K % (32 * a.ks) || a.nrows <= 0 || (a.wbytes != 2 && a.wbytes != 4) || (a.ks > 1 && a.nrows > TK_TW_MAX_BLOCK_ROWS)) return false;
     if ((a.per_seg || a.c_img) && a.ks != 1) return false;
     if (a.per_seg && (a.residual || a.c_img)) return false;
+    if (a.ln_x && (a.ks != 1 || a.wbytes != 4 || a.K > TK_TW_LN_MAX || a.nrows > TK_TW_LN_ROWS || a.K % 128)) return false;
     return !(a.c_img && (a.n_valid % 16 || a.nseg != 1));
 }
 static int tw_row_tiles(const TkTiledGemm& a) {
@@ -422,6 +494,12 @@ static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
 
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipStream_t s) {
     const int row_tiles = tw_row_tiles(a);
+    if (a.ln_x) {
+        if (p.mt != 1 || !p.one) return false;
+        if (p.pf == 8) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 8, true>), dim3(p.groups, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+        else hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 4, true>), dim3(p.groups, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+        return true;
+    }
 #define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
 #define TK_TW_WB(MTV, ONEV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, ONEV, PFV); else TK_TW_LAUNCH(MTV, 4, ONEV, PFV); } while (0)
     switch (p.mt) {
