@@ -394,8 +394,7 @@ static tk_error_code_t asr_run_ref(tk_asr_whisper_context_s* c, const int16_t* p
 
 /* one decode of `batch` utterances for this context: through the scheduler (shared contexts, one utterance per call) or straight on the engine */
 static tk_error_code_t asr_run(tk_asr_whisper_context_s* c, int batch, const int16_t* pcm, int n_samples, const std::vector<int32_t>& prompt, int n_steps, bool policy,
-                               float temperature, uint64_t seed, int32_t* tokens_out, float* logprobs_out, std::vector<float>* mel, std::vector<float>* enc,
-                               std::vector<float>* lg) {
+                               float temperature, uint64_t seed, int32_t* tokens_out, float* logprobs_out, float* mel, float* enc, float* lg) {
     SharedAsr* sh = c->sh.get();
     if (sh->scheduled && batch == 1 && !mel && !enc && !lg) {
         AsrReq r;
@@ -535,14 +534,7 @@ tk_error_code_t tk_mi355x_asr_transcribe_tokens(tk_asr_whisper_context_t* c, int
     std::vector<int32_t> prompt;
     std::string why;
     if (!asr_prompt(c, &prompt, &why)) return afail(TK_ERROR_INFERENCE_FAILED, why); /* whisper_full fails the same way at decode time */
-    std::vector<float> mel, enc, lg;
-    tk_error_code_t rc = asr_run(c, batch, pcm, n_samples, prompt, n_steps, false, 0.0f, 0, tokens_out, nullptr, mel_out ? &mel : nullptr, enc_out ? &enc : nullptr,
-                                 logits_out ? &lg : nullptr);
-    if (rc != TK_SUCCESS) return rc;
-    if (mel_out) memcpy(mel_out, mel.data(), mel.size() * 4);
-    if (enc_out) memcpy(enc_out, enc.data(), enc.size() * 4);
-    if (logits_out) memcpy(logits_out, lg.data(), lg.size() * 4);
-    return TK_SUCCESS;
+    return asr_run(c, batch, pcm, n_samples, prompt, n_steps, false, 0.0f, 0, tokens_out, nullptr, mel_out, enc_out, logits_out);
 }
 
 tk_error_code_t tk_mi355x_asr_transcribe_policy(tk_asr_whisper_context_t* c, int batch, const int16_t* pcm, int n_samples, int n_steps, float temperature,

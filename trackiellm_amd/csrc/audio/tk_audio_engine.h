@@ -50,9 +50,9 @@ public:
     ~TkAsr();
     bool init(TkWhisperModel* m, int max_batch);
     /* pcm[B][n_samples] (host), greedy decode of exactly n_steps tokens after the start-of-transcript prompt;
-     * tokens_out[B][n_steps]; optional copies of the mel / encoder output for parity tests */
+     * tokens_out[B][n_steps]; optional copies of the mel [B][frames][mels], of the encoder's output [B][ctx][state] and of the first sampled position's logits [B][vocab] */
     bool transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* prompt, int n_prompt, int n_steps, int32_t* tokens_out,
-                    std::vector<float>* mel_out, std::vector<float>* enc_out, std::vector<float>* first_logits);
+                    float* mel_out, float* enc_out, float* first_logits);
     /* the same with whisper.cpp's per-step bookkeeping: temperature 0 = arg max, > 0 = one draw per step from softmax(l / temperature) by the
      * canonical sampler keyed by (seed, step x B + b); logprobs_out [B][n_steps] = log-probability of every produced token under that
      * distribution (what the policy's logprob / entropy thresholds are taken on) */
@@ -81,6 +81,12 @@ private:
     int32_t* wh_state = nullptr;     /* [max_batch][TK_WH_STATE_INTS] */
     float* lp_dev = nullptr;         /* [n_text_ctx][max_batch] log-probabilities of a policy / reference-parameter decode */
     bool ensure_decode_buffers();
+    enum { TK_ASR_AUX_KEPT = 16 << 20 };
+    float* aux_host = nullptr;       /* pinned: what a call copies out beside its tokens */
+    size_t aux_floats = 0;
+    hipStream_t aux_stream = nullptr;
+    hipEvent_t aux_ready = nullptr, aux_done = nullptr;
+    bool aux_reserve(size_t floats);
     std::vector<float> pick_logprobs; /* [total steps][B], read back by transcribe_policy */
 };
 

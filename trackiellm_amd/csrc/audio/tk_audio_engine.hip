@@ -725,6 +725,11 @@ TkAsr::~TkAsr() {
     if (suppress_dev) (void)hipFree(suppress_dev);
     if (lp_dev) (void)hipFree(lp_dev);
     if (wh_state) (void)hipFree(wh_state);
+    if (aux_stream) (void)hipStreamSynchronize(aux_stream);
+    if (aux_host) (void)hipHostFree(aux_host);
+    if (aux_ready) (void)hipEventDestroy(aux_ready);
+    if (aux_done) (void)hipEventDestroy(aux_done);
+    if (aux_stream) (void)hipStreamDestroy(aux_stream);
     if (stream) (void)hipStreamDestroy(stream);
 }
 
@@ -837,8 +842,22 @@ bool TkAsr::transcribe_ref(int B, const int16_t* pcm, int n_samples, const int32
     return ok && copied;
 }
 
+/* pinned memory of the last call's outputs is kept up to TK_ASR_AUX_KEPT floats; what is larger is given back by the next smaller call */
+bool TkAsr::aux_reserve(size_t floats) {
+    if (!aux_stream) HIPQ(tk_create_perception_stream(&aux_stream));
+    if (!aux_ready) HIPQ(hipEventCreateWithFlags(&aux_ready, hipEventDisableTiming));
+    if (!aux_done) HIPQ(hipEventCreateWithFlags(&aux_done, hipEventDisableTiming));
+    if (floats <= aux_floats && (aux_floats <= TK_ASR_AUX_KEPT || floats > TK_ASR_AUX_KEPT)) return true;
+    if (aux_host) (void)hipHostFree(aux_host);
+    aux_host = nullptr;
+    aux_floats = 0;
+    HIPQ(hipHostMalloc((void**)&aux_host, floats * 4, hipHostMallocDefault));
+    aux_floats = floats;
+    return true;
+}
+
 bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* prompt, int n_prompt, int n_steps, int32_t* tokens_out,
-                       std::vector<float>* mel_out, std::vector<float>* enc_out, std::vector<float>* first_logits) {
+                       float* mel_out, float* enc_out, float* first_logits) {
     const TkWhisperHP& h = model->hp;
     if (B < 1 || B > max_batch) { error = "batch larger than the ASR context was created for"; return false; }
     if (n_samples < 0 || n_samples > h.n_samples()) { error = "audio longer than the model window"; return false; }
@@ -863,8 +882,20 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     auto st = g.begin_decode(ops, enc, B);
     ops.long_ok = false;
     HIPQ(hipGetLastError());
-    if (mel_out) { mel_out->resize((size_t)B * h.n_frames() * h.n_mels); HIPQ(hipMemcpyAsync(mel_out->data(), ml, mel_out->size() * 4, hipMemcpyDeviceToHost, stream)); }
-    if (enc_out) { enc_out->resize((size_t)B * h.n_audio_ctx * h.n_audio_state); HIPQ(hipMemcpyAsync(enc_out->data(), enc, enc_out->size() * 4, hipMemcpyDeviceToHost, stream)); }
+    /* The mel, the encoder's output and the first logits travel to pinned memory on a stream of their own, and from there to the caller while the decoder's steps run:
+     * copies to pageable memory in between held back the launches behind them (one clip: 0.5 ms of 7). */
+    const size_t n_mel = mel_out ? (size_t)B * h.n_frames() * h.n_mels : 0, n_enc = enc_out ? (size_t)B * h.n_audio_ctx * h.n_audio_state : 0, n_lg = first_logits ? (size_t)B * h.n_vocab : 0;
+    float *mel_at = nullptr, *enc_at = nullptr, *lg_at = nullptr;
+    struct Wait { TkAsr* a; ~Wait() { if (a->aux_stream) (void)hipStreamSynchronize(a->aux_stream); } } wait{this}; /* whatever happens below */
+    if (n_mel + n_enc + n_lg > 0) {
+        if (!aux_reserve(n_mel + n_enc + n_lg)) return false;
+        mel_at = aux_host; enc_at = mel_at + n_mel; lg_at = enc_at + n_enc;
+        HIPQ(hipEventRecord(aux_ready, stream));
+        HIPQ(hipStreamWaitEvent(aux_stream, aux_ready, 0));
+        if (n_mel) HIPQ(hipMemcpyAsync(mel_at, ml, n_mel * 4, hipMemcpyDeviceToHost, aux_stream));
+        if (n_enc) HIPQ(hipMemcpyAsync(enc_at, enc, n_enc * 4, hipMemcpyDeviceToHost, aux_stream));
+        HIPQ(hipEventRecord(aux_done, aux_stream));
+    }
     /* The whole greedy loop is enqueued without touching the host: prompt tokens and positions sit in device tables uploaded once, step p
      * reads its token from the prompt table or from the previous step's arg-max slot and writes its own arg-max into slot p of an output
      * table; one copy and one synchronisation at the end.  (A synchronisation and three small copies per step made the 16 steps of 32
@@ -891,8 +922,8 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
         st.next = out_tab + (size_t)p * B;
         g.decode_step(ops, st, p);
         if (p == n_prompt - 1 && first_logits) {
-            first_logits->resize((size_t)B * h.n_vocab);
-            HIPQ(hipMemcpyAsync(first_logits->data(), st.logits, first_logits->size() * 4, hipMemcpyDeviceToHost, stream));
+            ops.flush();
+            HIPQ(hipMemcpyAsync(lg_at, st.logits, n_lg * 4, hipMemcpyDeviceToHost, stream)); /* (the next step writes them again) */
         }
         /* the reference-parameter decode ends where the rows' own bookkeeping says (whisper.cpp: up to n_text_ctx / 2 - 4 tokens): every 16 sampled
          * positions the rows' status words are read; once every row has completed or failed nothing more is enqueued — a finished row emits eot and
@@ -909,9 +940,15 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
         }
     }
     ops.flush();
+    if (n_mel + n_enc > 0) {
+        HIPQ(hipEventSynchronize(aux_done));
+        if (n_mel) memcpy(mel_out, mel_at, n_mel * 4);
+        if (n_enc) memcpy(enc_out, enc_at, n_enc * 4);
+    }
     std::vector<int32_t> outs((size_t)steps_run * B);
     HIPQ(hipMemcpyAsync(outs.data(), out_tab + (size_t)(n_prompt - 1) * B, outs.size() * 4, hipMemcpyDeviceToHost, stream));
     HIPQ(hipStreamSynchronize(stream)); /* host_tab and outs live until here */
+    if (n_lg) memcpy(first_logits, lg_at, n_lg * 4);
     for (int step = 0; step < n_steps; ++step)
         for (int b = 0; b < B; ++b) tokens_out[(size_t)b * n_steps + step] = step < steps_run ? outs[(size_t)step * B + b] : pick.eot;
     HIPQ(hipGetLastError());
