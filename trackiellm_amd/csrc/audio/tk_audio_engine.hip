@@ -6,6 +6,7 @@
 
 #include <type_traits>
 
+#include "../nn/tk_attention_images.h"
 #include "../nn/tk_gemm_tiled.h"
 #include "../nn/tk_nn_kernels.h"
 
@@ -486,7 +487,7 @@ struct TkAudioGpuOps {
             }
             const int i = pend.n++;
             t.tiles[i] = a->model->wt[(size_t)idx]; t.row_tiles[i] = g.N / 16;
-            t.seg_out[i] = g.C; t.seg_ldc[i] = g.ldc; t.seg_bias[i] = g.bias; t.seg_n[i] = g.N;
+            t.seg_out[i] = g.C; t.seg_ldc[i] = g.ldc; t.seg_bias[i] = g.bias; t.seg_n[i] = g.N; t.seg_img[i] = g.c_image;
             if (pend.n == 3) flush();
             return; /* none of these layers writes into its own input: `plain` excludes in-place layers */
         }
@@ -539,6 +540,21 @@ struct TkAudioGpuOps {
         if (hd > 256 || (hd & 15) || (d & 3) || Tk < 1 || Tk > TK_AT1_MAX_KEYS) return false; /* the three-launch form takes what does not fit */
         float* img = (short_pass(B) && d % 128 == 0 && q_bstride == d) ? image_for(out, B, d, d) : nullptr; /* the output projection's input, packed on the way out */
         return at1_launch(q, k, v, scores, pitch, out, B, Tk, q_bstride, kv_bstride, d, nh, img, s);
+    }
+    /* an encoder layer's attention on operand images: 16 rows of a head in one workgroup, no score matrix.  All contexts it has registers for take it (three launches
+     * and their score matrix else): at 1500 positions and six heads 97 -> 56 us a layer for one clip, 2106 -> 1194 us for 32 */
+    bool takes_images(const float* q_w, const float* k_w, const float* o_w, int Tc, int d, int nh) {
+        if ((a->fast && long_ok) || !long_ok || d % 128 || !tk_attention_images_fits(Tc, Tc, d, nh)) return false;
+        for (const float* w : {q_w, k_w, o_w}) {
+            const int i = a->model->tensor_of(w);
+            if (i < 0 || !a->model->wt[(size_t)i]) return false;
+        }
+        return true;
+    }
+    void attend_images(const float* q, const float* k, const float* v, float* out, int B, int Tc, int d, int nh) {
+        drop_image();
+        float* img = image_for(out, B * Tc, d, d);
+        if (!tk_launch_attention_images(q, k, v, img, B, nh, Tc, Tc, d, tk_divf(1.0f, tk_sqrtf((float)(d / nh))), s)) a->launch_error = "attention launch refused";
     }
     /* the opt-in fast contraction's attention (TkAsr::fast): Q K^T, softmax and P V of a long pass in one kernel, no score matrix in HBM */
     bool attend_fused(const float* q, const float* k, const float* v, float* out, int B, int Tq, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh) {
@@ -605,6 +621,8 @@ struct TkAudioSizeOps {
     void layernorm(const float*, int rows, int D, const float*, const float*, float*) { image(rows, D); }
     void softmax_rows(float*, int, int, int) {}
     bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int d, int, float*, int) { image(B, d); return true; }
+    bool takes_images(const float*, const float*, const float*, int, int, int) { return false; }
+    void attend_images(const float*, const float*, const float*, float*, int, int, int, int) {}
     bool attend_fused(const float*, const float*, const float*, float*, int, int, int, int64_t, int64_t, int, int) { return false; } /* sized for the exact form */
     void add_rows(float*, const float*, int, int, int) {}
     void embed_rows(const float*, const float*, const int32_t*, const int32_t*, int, int, float*) {}

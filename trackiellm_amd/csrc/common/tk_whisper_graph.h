@@ -14,6 +14,8 @@
  *   void layernorm(const float* x, int rows, int D, const float* w, const float* b, float* y);
  *   void softmax_rows(float* x, int rows, int cols, int ld);
  *   bool attend1(...): optional fused form of attention() for one query row per sequence (same arithmetic); false = not provided
+ *   bool takes_images(...) / attend_images(...): optional one-kernel form of attention() for all rows of an encoder layer, on q and k that
+ *     their linear layers wrote as operand images (TkGemm::c_image; same arithmetic); `out` then feeds linear layer `o` only
  *   bool attend_fused(...): optional one-kernel form of attention() for many query rows (the GPU's opt-in fast contraction: NOT the same
  *     arithmetic, ~1e-6 of scale off; the oracle and the exact path return false)
  *   void add_rows(float* x, const float* add, int rows, int D, int add_rows);
@@ -240,8 +242,9 @@ struct TkWhisperGraph {
         o.gemm(lin(col2, B * Tc, 3 * d, 3 * d, W[m.conv2_w], W[m.conv2_b], d, x, d, TK_ACT_GELU));
         o.add_rows(x, W[m.enc_pos], B * Tc, d, Tc);
         float* hb = o.alloc((size_t)B * Tc * d);
-        float* q = o.alloc((size_t)B * Tc * d);
-        float* k = o.alloc((size_t)B * Tc * d);
+        const size_t whole = ((size_t)B * Tc + 15) / 16 * 16 * d; /* rows of whole tiles: q and k may be operand images */
+        float* q = o.alloc(whole);
+        float* k = o.alloc(whole);
         float* v = o.alloc((size_t)B * Tc * d);
         float* at = o.alloc((size_t)B * Tc * d);
         float* ff = o.alloc((size_t)B * Tc * 4 * d);
@@ -250,10 +253,12 @@ struct TkWhisperGraph {
         for (int l = 0; l < h.n_audio_layer; ++l) {
             const TkWhLayerIdx& L = m.enc[l];
             o.layernorm(x, R, d, W[L.ln1_w], W[L.ln1_b], hb);
-            o.gemm(lin(hb, R, d, d, W[L.q_w], W[L.q_b], d, q, d));
-            o.gemm(lin(hb, R, d, d, W[L.k_w], nullptr, d, k, d));
+            const int images = o.takes_images(W[L.q_w], W[L.k_w], W[L.o_w], Tc, d, nh) ? 1 : 0;
+            { TkGemm gq = lin(hb, R, d, d, W[L.q_w], W[L.q_b], d, q, d); gq.c_image = images; o.gemm(gq); }
+            { TkGemm gk = lin(hb, R, d, d, W[L.k_w], nullptr, d, k, d); gk.c_image = images; o.gemm(gk); }
             o.gemm(lin(hb, R, d, d, W[L.v_w], W[L.v_b], d, v, d));
-            attention(o, q, k, v, at, B, Tc, Tc, (int64_t)Tc * d, (int64_t)Tc * d, d, nh, sc);
+            if (images) o.attend_images(q, k, v, at, B, Tc, d, nh);
+            else attention(o, q, k, v, at, B, Tc, Tc, (int64_t)Tc * d, (int64_t)Tc * d, d, nh, sc);
             o.gemm(lin(at, R, d, d, W[L.o_w], W[L.o_b], d, x, d, 0, x, d));
             o.layernorm(x, R, d, W[L.ln2_w], W[L.ln2_b], hb);
             { TkGemm g1 = lin(hb, R, d, d, W[L.fc1_w], W[L.fc1_b], 4 * d, ff, 4 * d, TK_ACT_GELU); g1.c_feeds_linear = 1; o.gemm(g1); }

@@ -53,6 +53,7 @@ struct TkTiledGemm {
     int seg_ldc[3];
     const float* seg_bias[3];
     int seg_n[3];
+    int seg_img[3];          /* the segment's destination is the operand image of its output (k = its column), not rows */
     /* c_img: the output is ALSO written as the operand image of the next linear layer (K = n_valid), so no pack launch follows */
     float* c_img;
     /* ln_x: the activations are the layer norm of its rows ([nrows][K], dense), made by every workgroup for itself (f32 tiles, ks == 1, at most TK_TW_LN_ROWS rows of at

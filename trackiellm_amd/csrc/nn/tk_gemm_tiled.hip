@@ -260,6 +260,8 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         const float bias = bp ? bp[ns] : 0.0f;
         float* outp = a.seg_out[seg];
         const int ldc = a.seg_ldc[seg];
+        const bool img = a.seg_img[seg];
+        const size_t img_col = (size_t)(ns >> 4) * 256 + (size_t)(ns & 3) * 64 + ((ns & 15) >> 2);
 #pragma unroll
         for (int m = 0; m < MT; ++m)
 #pragma unroll
@@ -268,7 +270,9 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                 if (row < rows_here) {
                     float v = acc[m][r];
                     if (bp || a.add_zero_bias) v = v + bias;
-                    outp[(size_t)(row0 + row) * ldc + ns] = tw_act(v, a.act);
+                    v = tw_act(v, a.act);
+                    if (img) outp[(size_t)((row0 + row) >> 4) * 16 * a.seg_n[seg] + img_col + (size_t)((row0 + row) & 15) * 4] = v;
+                    else outp[(size_t)(row0 + row) * ldc + ns] = v;
                 }
             }
         return;
