@@ -20,6 +20,28 @@ def test_cut_of_few_tiles_equals_staged(gpu, M, N, K, act, res):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,act,res", [
+    (257, 2048, 128, 2, False), (544, 1024, 128, 0, True), (543, 1024, 128, 3, True), (577, 992, 256, 1, True), (1441, 384, 384, 2, True), (2047, 288, 128, 0, False),   # tiles of 32 x 32
+    (1825, 2176, 512, 0, True), (1857, 2176, 512, 2, False), (3841, 1088, 1024, 1, True), (3872, 1056, 1024, 0, True),                            # of 64 x 32
+])
+def test_wide_tiles_equal_staged(gpu, M, N, K, act, res):
+    test_cut_of_few_tiles_equals_staged(gpu, M, N, K, act, res)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("ctx,width", [(100, 1024), (33, 1280), (97, 384)])
+def test_wide_tiles_and_images_in_an_encoder(gpu, ctx, width):
+    """a clip's encoder states do not depend on how many clips run with it: from 20 on its layers, and the images between them, are made in wide tiles"""
+    hp = gpu.WhisperHP(80, ctx, width, width // 64, 1, 8, width, width // 64, 1, 512)
+    asr = gpu.Asr(hp=hp, seed=4, max_batch=59)
+    pcm = np.random.default_rng(ctx).integers(-6000, 6000, (59, 320 * ctx)).astype(np.int16)
+    _, _, enc, logits = asr.transcribe_tokens(pcm, 1)
+    for b in (0, 7, 58):
+        _, _, one, lg = asr.transcribe_tokens(pcm[b:b + 1], 1)
+        assert np.array_equal(one[0].view(np.uint32), enc[b].view(np.uint32)) and np.array_equal(lg[0].view(np.uint32), logits[b].view(np.uint32))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("width", [64, 128, 384, 768, 1024, 1152])
 def test_norms_inside_products_of_a_few_rows(gpu, width):
     """a decoder's norms are made by the products behind them for up to four sequences and widths of 128 .. 1024 in steps of 128, as launches else: tokens and logits of

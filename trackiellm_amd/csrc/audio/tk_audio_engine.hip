@@ -508,6 +508,7 @@ struct TkAudioGpuOps {
             if (norm.live) pk.mark = a->arena_used; /* (the norm has no image below it) */
             cimg = raw_alloc(tk_tiled_gemm_scratch(nx));
             t.c_img = cimg;
+            t.out = nullptr; /* (fc2 has tiles: its K is a multiple of 128) */
         }
         if (!tk_launch_gemm_tiled(t, s)) tk_launch_gemm(g, s); /* not reached: tk_tiled_gemm_applies() admits only shapes the launcher takes */
         if (emit_img) { /* the image pair stays allocated from pk.mark up; the upper one is now the live image */

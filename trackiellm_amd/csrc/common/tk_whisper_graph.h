@@ -282,18 +282,18 @@ struct TkWhisperGraph {
         DecState s;
         s.B = B;
         for (int l = 0; l < h.n_text_layer; ++l) {
-            const TkWhLayerIdx& L = m.dec[l];
-            float* xk = o.alloc((size_t)B * Tc * dt);
-            float* xv = o.alloc((size_t)B * Tc * dt);
-            o.gemm(lin(enc, B * Tc, d, d, W[L.xk_w], nullptr, dt, xk, dt));
-            o.gemm(lin(enc, B * Tc, d, d, W[L.xv_w], W[L.xv_b], dt, xv, dt));
-            s.xk.push_back(xk); s.xv.push_back(xv);
+            s.xk.push_back(o.alloc((size_t)B * Tc * dt)); s.xv.push_back(o.alloc((size_t)B * Tc * dt));
             s.sk.push_back(o.alloc((size_t)B * h.n_text_ctx * dt));
             s.sv.push_back(o.alloc((size_t)B * h.n_text_ctx * dt));
         }
         s.x = o.alloc((size_t)B * dt); s.hb = o.alloc((size_t)B * dt); s.q = o.alloc((size_t)B * dt);
         s.k = o.alloc((size_t)B * dt); s.v = o.alloc((size_t)B * dt); s.at = o.alloc((size_t)B * dt);
         s.ff = o.alloc((size_t)B * 4 * dt);
+        for (int l = 0; l < h.n_text_layer; ++l) { /* all on one input, one behind the other: packed once, launched together */
+            const TkWhLayerIdx& L = m.dec[l];
+            o.gemm(lin(enc, B * Tc, d, d, W[L.xk_w], nullptr, dt, s.xk[l], dt));
+            o.gemm(lin(enc, B * Tc, d, d, W[L.xv_w], W[L.xv_b], dt, s.xv[l], dt));
+        }
         const int tmax = Tc > h.n_text_ctx ? Tc : h.n_text_ctx;
         s.sc = o.alloc((size_t)B * h.n_text_head * score_pitch(tmax));
         s.logits = o.alloc((size_t)B * h.n_vocab);

@@ -14,7 +14,7 @@
  * A wave owns one weight row tile of one K range and streams it as one piece per 32 k, PF pieces in flight in registers; a piece feeds
  * 8 MFMAs per M-tile.  The A image is staged through an LDS ring by LDS-DMA, 1 KiB per (16 k, M-tile), shared by the workgroup's
  * waves; a lane's operand of four consecutive MFMAs is one ds_read_b128.  Rows beyond 256 run as further workgroups (grid y) over the
- * same weights.  At 16 rows the f16 path is HBM-bound (2 B per weight); from 32 rows up the fp32 MFMA rate (157 TFLOP/s) bounds it.
+ * same weights; where that makes enough tiles of 32 x 32, a kernel without LDS takes f32 products instead (k_gemm_wide).  At 16 rows the f16 path is HBM-bound (2 B per weight); from 32 rows up the fp32 MFMA rate (157 TFLOP/s) bounds it.
  */
 #ifndef TK_GEMM_TILED_H
 #define TK_GEMM_TILED_H
@@ -54,7 +54,7 @@ struct TkTiledGemm {
     const float* seg_bias[3];
     int seg_n[3];
     int seg_img[3];          /* the segment's destination is the operand image of its output (k = its column), not rows */
-    /* c_img: the output is ALSO written as the operand image of the next linear layer (K = n_valid), so no pack launch follows */
+    /* c_img: the output is ALSO written as the operand image of the next linear layer (K = n_valid), so no pack launch follows; out may be null then */
     float* c_img;
     /* ln_x: the activations are the layer norm of its rows ([nrows][K], dense), made by every workgroup for itself (f32 tiles, ks == 1, at most TK_TW_LN_ROWS rows of at
      * most TK_TW_LN_MAX columns, K % 128 == 0); a_img is not read */
@@ -67,7 +67,7 @@ struct TkTiledGemm {
 /* false (nothing launched): K / ks is not a multiple of the ring granularity (128 k; 64 k from 129 rows per block on) or a field is inconsistent */
 bool tk_launch_gemm_tiled(const TkTiledGemm& g, hipStream_t s);
 /* how a launch is cut: M-tiles and waves (a tile of columns each) of a workgroup, and what follows from them.  mt 0: its own choice */
-struct TkTiledPlan { int mt, waves, groups, ny, pf, rk, slot_bytes; bool one; size_t lds; };
+struct TkTiledPlan { int mt, waves, groups, ny, pf, rk, slot_bytes; bool one; size_t lds; int wide = 0; /* k_gemm_wide's form */ };
 bool tk_gemm_tiled_plan(const TkTiledGemm& g, int mt, int waves, TkTiledPlan* plan);
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& g, const TkTiledPlan& plan, hipStream_t s);
 /* row-major f16 / f32 [N][K] (device) -> tiles; N is padded up to a multiple of 16 with zero rows, K must be a multiple of 32 */

@@ -5,10 +5,12 @@
 
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "../common/tk_exact_math.h"
 
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
 
 #define TK_TW_SLOT_BYTES 65536
@@ -36,6 +38,18 @@ __device__ __forceinline__ float tw_act(float v, int act) {
         case TK_ACT_GELU: return tk_geluf(v);
         case TK_ACT_SIGMOID: return tk_sigmoidf(v);
         default: return v;
+    }
+}
+
+template <int N> __device__ __forceinline__ void tw_act_all(float* v, int act) {
+    if (act == TK_ACT_SILU) {
+        tk_silu_all<N>(v);
+    } else if (act == TK_ACT_GELU) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = tk_geluf(v[i]);
+    } else if (act == TK_ACT_SIGMOID) {
+#pragma unroll
+        for (int i = 0; i < N; ++i) v[i] = tk_sigmoidf(v[i]);
     }
 }
 
@@ -260,7 +274,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         const float bias = bp ? bp[ns] : 0.0f;
         float* outp = a.seg_out[seg];
         const int ldc = a.seg_ldc[seg];
-        const bool img = a.seg_img[seg];
+        const bool img = WB == 4 && a.seg_img[seg];
         const size_t img_col = (size_t)(ns >> 4) * 256 + (size_t)(ns & 3) * 64 + ((ns & 15) >> 2);
 #pragma unroll
         for (int m = 0; m < MT; ++m)
@@ -290,8 +304,159 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                 if (a.bias || a.add_zero_bias) v = v + bias;
                 v = tw_act(v, a.act);
                 if (a.residual) v = v + a.residual[(size_t)(row0 + row) * a.ldr + n];
-                a.out[(size_t)(row0 + row) * a.ldc + n] = v;
+                if (WB == 2 || a.out) a.out[(size_t)(row0 + row) * a.ldc + n] = v;
                 if (a.c_img) a.c_img[(size_t)((row0 + row) >> 4) * 16 * a.n_valid + img_col + (size_t)((row0 + row) & 15) * 4] = v;
+            }
+        }
+}
+
+/*
+ * Many rows: a wave makes 32 MI x 32 NI of the output alone, on v_mfma_f32_32x32x2_f32 (the same chain, two k an instruction), both operands from the caches straight
+ * into registers, PF stages of KS k in flight: no LDS, no barrier, nothing that waves wait for each other with.  Step s of a 16-k group takes k = 2 s, 2 s + 1: lane half
+ * h = l / 32 holds groups g = h and 2 + h of the image and of the weight tiles, a float4 each.  An operand float4 feeds 4 MI or 4 NI MFMAs of 64 cycles, where the ring
+ * kernel above reads LDS once for 4 of 32: fp32 MFMAs and LDS reads take turns on a SIMD.
+ * Images are made with the operands exchanged: a lane then holds one row, and lanes l, l + 32 swap halves so that each stores the 16 bytes of a group.
+ * Form <1, 1> has the smaller tiles, and so more of them; form <2, 1> reads a third less, which counts for matrices that the L2 does not hold (tk_gemm_tiled_plan).
+ * 48 000 rows, ring -> here, us (the fp32 MFMAs alone): 384 x 384 183 -> 139 (93), 1152 x 384 475 -> 346 (278), 1536 x 384 with GELU 610 -> 469 (370), 384 x 1536 560 -> 513
+ * (370); 1500 rows: 23.2 -> 17.6, 31.6 -> 25.2 and 38.2 -> 30.4 of the last three.  What is left is the last round of tiles and the first requests of each.
+ */
+template <int MI, int NI, int KS, int PF>
+__global__ __launch_bounds__(256, MI * NI == 4 ? 3 : MI * NI == 2 ? 4 : 5) void k_gemm_wide(TkTiledGemm a, int ncol /* tiles of 32 NI columns */, int total /* waves' tiles */, int per_xcd) {
+    constexpr int V = KS / 8; /* float4 per 32 rows and stage */
+    /* consecutive workgroups go to different XCDs: each takes a run of them, whose rows stay in its L2 */
+    const int wg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    const int lane = threadIdx.x & 63, id = wg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (id >= total) return;
+    const int h = lane >> 5, l32 = lane & 31, l16 = lane & 15, up = (lane >> 4) & 1;
+    const int blk = id / ncol, row0 = blk * 32 * MI;
+    int rt = (id - blk * ncol) * 2 * NI, seg = 0, col_base = 0;
+    while (seg < a.nseg - 1 && rt >= a.row_tiles[seg]) { rt -= a.row_tiles[seg]; col_base += a.row_tiles[seg] * TK_TW_ROWS_PER_TILE; ++seg; }
+    const unsigned a_pitch = (unsigned)a.a_ts * 4u, w_pitch = (unsigned)a.K * 64u; /* bytes of 16 rows */
+    const int tiles_here = (a.nrows - row0 + 15) / 16;
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void*)(a.a_img + (size_t)(row0 / 16) * a.a_ts), 0, (unsigned)(tiles_here < 2 * MI ? tiles_here : 2 * MI) * a_pitch, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.tiles[seg] + (size_t)rt * w_pitch), 0, 2u * NI * w_pitch, 0x00020000);
+    unsigned a_at[MI], w_at[NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+        const int tile = 2 * i + up;
+        a_at[i] = (unsigned)(tile < tiles_here ? tile : tiles_here - 1) * a_pitch + (unsigned)(h * 256 + l16 * 16);
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) w_at[i] = (unsigned)(2 * i + up) * w_pitch + (unsigned)((h * 16 + l16) * 32);
+
+    v4f aq[PF][MI][V], wq[PF][NI][V];
+    const int ns = a.K / KS;
+    auto load = [&](int s, v4f (*av)[V], v4f (*wv)[V]) {
+        s = s < ns ? s : ns - 1;
+#pragma unroll
+        for (int v = 0; v < V; ++v) { /* 16-k group v / 2 of the stage, half v % 2 of its groups */
+            const unsigned j = (unsigned)(s * (KS / 16) + v / 2);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) av[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(ar, a_at[i] + (v & 1) * 512, j * 1024, 0));
+#pragma unroll
+            for (int i = 0; i < NI; ++i) wv[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at[i] + (v & 1) * 1024, (j >> 1) * 2048 + (j & 1) * 16, 0));
+        }
+    };
+    v16f acc[MI][NI];
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int n = 0; n < NI; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][n][r] = 0.0f;
+    const bool image = a.c_img != nullptr || (a.per_seg && a.seg_img[seg]);
+    auto products = [&](auto swapped) {
+#pragma unroll
+        for (int s = 0; s < PF - 1; ++s) load(s, aq[s], wq[s]);
+#pragma unroll 1
+        for (int s = 0; s < ns; s += PF) {
+#pragma unroll
+            for (int u = 0; u < PF; ++u) {
+                load(s + u + PF - 1, aq[(u + PF - 1) % PF], wq[(u + PF - 1) % PF]);
+#pragma unroll
+                for (int v = 0; v < V; v += 2)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int b = 0; b < 2; ++b)
+#pragma unroll
+                            for (int i = 0; i < MI; ++i)
+#pragma unroll
+                                for (int n = 0; n < NI; ++n) {
+                                    const float x = aq[u][i][v + b][t], w = wq[u][n][v + b][t];
+                                    acc[i][n] = swapped.value ? __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, acc[i][n], 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, acc[i][n], 0, 0, 0);
+                                }
+                /* the requests spread over the products: in front of them they hold these up, behind them (where the compiler puts them) they come late */
+#pragma unroll
+                for (int i = 0; i < (MI + NI) * V; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, MI * NI * V * 4 / ((MI + NI) * V), 0);
+                    __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    };
+    const int col0 = rt * TK_TW_ROWS_PER_TILE; /* in the segment */
+    const float* bias = a.per_seg ? a.seg_bias[seg] : a.bias;
+    if (bias && !a.per_seg) bias += col_base;
+    const bool add_bias = bias || a.add_zero_bias;
+    if (image) {
+        products(std::true_type{});
+        float* img = a.per_seg ? a.seg_out[seg] : a.c_img;
+        const int cols = a.per_seg ? a.seg_n[seg] : a.n_valid, c0 = a.per_seg ? col0 : col_base + col0;
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int n = 0; n < NI; ++n) {
+                const int row = row0 + 32 * i + l32;
+                float v[16];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    v4f b = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if (bias) b = *(const v4f*)(bias + col0 + 32 * n + 8 * q + 4 * h);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[4 * q + r] = add_bias ? acc[i][n][4 * q + r] + b[r] : acc[i][n][4 * q + r];
+                }
+                tw_act_all<16>(v, a.act);
+#pragma unroll
+                for (int q = 0; q < 2; ++q)
+#pragma unroll
+                    for (int g = 0; g < 4; g += 2) {
+                        v4f o;
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) { /* t = 2 b + h of groups g, g + 1: the lower lanes take g, the upper g + 1 */
+                            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[8 * q + 4 * b + g]), __float_as_uint(v[8 * q + 4 * b + g + 1]), false, false);
+                            o[2 * b] = __uint_as_float(x[0]);
+                            o[2 * b + 1] = __uint_as_float(x[1]);
+                        }
+                        if (row < a.nrows) *(v4f*)(img + (size_t)(row >> 4) * 16 * cols + (size_t)(((c0 >> 4) + 2 * n + q) * 256 + (g + h) * 64 + (row & 15) * 4)) = o;
+                    }
+            }
+        return;
+    }
+    products(std::false_type{});
+    float* out = a.per_seg ? a.seg_out[seg] + col0 : a.out + col_base + col0;
+    const int ldc = a.per_seg ? a.seg_ldc[seg] : a.ldc;
+    const float* res = a.residual ? a.residual + col_base + col0 : nullptr;
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int n = 0; n < NI; ++n) {
+            const int c = 32 * n + l32;
+            const float b = bias ? bias[col0 + c] : 0.0f;
+            float v[16], rs[16];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = row0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (res) rs[r] = row < a.nrows ? res[(size_t)row * a.ldr + c] : 0.0f;
+                v[r] = add_bias ? acc[i][n][r] + b : acc[i][n][r];
+            }
+            tw_act_all<16>(v, a.act);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = row0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+                if (res) v[r] = v[r] + rs[r];
+                if (row < a.nrows) out[(size_t)row * ldc + c] = v[r];
             }
         }
 }
@@ -384,6 +549,8 @@ static bool tw_valid(const TkTiledGemm& a) {
     if (a.nseg < 1 || a.nseg > 3 || a.ks < 1 || a.K <= 0 || a.K % (32 * a.ks) || a.nrows <= 0 || (a.wbytes != 2 && a.wbytes != 4) || (a.ks > 1 && a.nrows > TK_TW_MAX_BLOCK_ROWS)) return false;
     if ((a.per_seg || a.c_img) && a.ks != 1) return false;
     if (a.per_seg && (a.residual || a.c_img)) return false;
+    if (!a.per_seg && !a.out && (!a.c_img || a.wbytes == 2)) return false;
+    if (a.per_seg && a.wbytes == 2 && (a.seg_img[0] || a.seg_img[1] || a.seg_img[2])) return false;
     if (a.ln_x && (a.ks != 1 || a.wbytes != 4 || a.K > TK_TW_LN_MAX || a.nrows > TK_TW_LN_ROWS || a.K % 128)) return false;
     return !(a.c_img && (a.n_valid % 16 || a.nseg != 1));
 }
@@ -397,13 +564,14 @@ static int tw_row_tiles(const TkTiledGemm& a) {
 static bool tw_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
     if ((mt != 1 && mt != 2 && mt != 4 && mt != 6 && mt != 8 && mt != 16) || waves < 1 || waves > 8) return false;
     const int row_tiles = tw_row_tiles(a), Kr = a.K / a.ks;
+    *p = TkTiledPlan{};
     p->mt = mt;
     p->waves = waves;
     p->groups = (row_tiles + waves - 1) / waves;
     p->ny = (a.nrows + mt * TK_TW_ROWS_PER_TILE - 1) / (mt * TK_TW_ROWS_PER_TILE);
     /* k per ring slot: the largest multiple of 32 PF that divides the K range and fits a 64 KiB slot (rk / 16 * mt KiB) — a whole short
      * range in one slot (`one`, up to 128 KiB) needs no ring.
-     * Many row blocks of 128 rows (the Whisper encoder's linears, 48000 rows): 32 KiB slots and two weight pieces in flight instead, so
+     * Many row blocks of 128 rows (of products that are none of k_gemm_wide's): 32 KiB slots and two weight pieces in flight instead, so
      * that TWO workgroups share a CU and one's ring fill and epilogue run under the other's MFMAs. */
     const bool twin = p->ny > 1 && (mt == 8 || mt == 6) && Kr % 64 == 0;
     p->one = mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES;
@@ -441,13 +609,22 @@ static float tw_cost(const TkTiledGemm& a, const TkTiledPlan& p) {
 }
 
 static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p);
+bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p);
 bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
     if (!tw_valid(a)) return false;
     if (mt > 0) return tw_plan(a, mt, waves, p);
+    /* Many rows: tiles of 32 x 32 without LDS, from 544 of them on (a chip has 1024 SIMDs).  Ring / wide time, 22 matrices at 260 .. 2000 rows: up to 384 tiles 0.4 .. 0.9
+     * (1152 x 384 1.2), 432 .. 576 0.8 .. 1.3, from 640 on 1.1 .. 1.6.  Form 2 where the weights are more than an XCD's L2 holds and there are tiles to spare: 5120 x 1280
+     * at 1500 and 12 000 rows 203 -> 179 and 1395 -> 1150 us; 512 rows 74 -> 86, 1536 x 384 at 48 000 rows 469 -> 485. */
+    if (a.nrows > TK_TW_MAX_BLOCK_ROWS) {
+        const int64_t tiles = (int64_t)((a.nrows + 31) / 32) * (tw_row_tiles(a) / 2);
+        const bool large = (size_t)tw_row_tiles(a) * 16 * (size_t)a.K * 4 > (4u << 20);
+        if (tiles >= 544 && tk_gemm_wide_plan(a, large && tiles >= 3840 ? 2 : 1, p)) return true;
+    }
     if (!tw_usual(a, p)) return false;
     /* As many rows as possible behind one reading of the weights is what counts where these are large.  Small matrices (up to 24 MB: they come from the caches) of few
      * tiles leave most of the chip idle that way: fewer M-tiles a workgroup, where that is clearly quicker by the costs, measured 384 x 384 at 32, 256 and 1500 rows
-     * 7.8 -> 5.6, 41 -> 5.4, 26.5 -> 10.4 us, 384 x 1536 20.3 -> 11.9, 123 -> 12.0, 87 -> 36.  No cut reads rows of the image that the usual one does not. */
+     * 7.8 -> 5.6, 41 -> 5.4, 26.5 -> 10.4 us, 384 x 1536 at 32 and 256 20.3 -> 11.9, 123 -> 12.0.  No cut reads rows of the image that the usual one does not. */
     const TkTiledPlan usual = *p;
     if ((size_t)tw_row_tiles(a) * 16 * (size_t)a.K * (size_t)a.wbytes > 24000000u || (int64_t)tw_row_tiles(a) * usual.ny * a.ks >= 4096) return true;
     float least = 0.93f * tw_cost(a, usual);
@@ -468,7 +645,7 @@ static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
     mt = rows_blk > 128 ? 16 : rows_blk > 64 ? 8 : rows_blk > 32 ? 4 : rows_blk > 16 ? 2 : 1;
     if (mt == 16 && a.nrows > TK_TW_MAX_BLOCK_ROWS && (a.K / a.ks) % 64 == 0) {
         /* many row blocks: two workgroups per CU (below), 512 at a time on the chip; of 128- and 96-row blocks the one whose last round
-         * wastes less (N = 384 at 48 000 rows: 1 125 workgroups = 3 rounds of 8 M-tiles against 1 500 = 3 rounds of 6) */
+         * wastes less (N = 376 at 48 000 rows: 1 125 workgroups = 3 rounds of 8 M-tiles against 1 500 = 3 rounds of 6) */
         const long wg_per_blk = (row_tiles + 7) / 8;
         const long slots = 2L * tk_tiled_num_cu();
         const long c8 = (((a.nrows + 127) / 128) * wg_per_blk + slots - 1) / slots * 8;
@@ -496,7 +673,30 @@ static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
     return tw_plan(a, mt, row_tiles < 8 ? row_tiles : 8, p);
 }
 
+/* the cut of k_gemm_wide's form 1 (32 x 32 of the output a wave) or 2 (64 x 32); false: not a product it takes */
+bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p) {
+    static const struct { int mi, ni; } forms[] = {{0, 0}, {1, 1}, {2, 1}};
+    if (!tw_valid(a) || form < 1 || form > 2 || a.wbytes != 4 || a.ks != 1 || a.ln_x || (a.c_img && (a.out || a.residual)) || a.K % 128) return false;
+    const int per = 2 * forms[form].ni;
+    for (int i = 0; i < a.nseg; ++i)
+        if (a.row_tiles[i] % per || (a.per_seg && a.seg_n[i] != a.row_tiles[i] * 16)) return false;
+    if (!a.per_seg && a.n_valid != tw_row_tiles(a) * 16) return false;
+    *p = TkTiledPlan{};
+    p->wide = form;
+    p->groups = tw_row_tiles(a) / per;
+    p->ny = (a.nrows + 32 * forms[form].mi - 1) / (32 * forms[form].mi);
+    return (int64_t)p->groups * p->ny < 0x7fffff00;
+}
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipStream_t s) {
+    if (p.wide) {
+        TkTiledPlan w; /* (the cut follows from the form) */
+        if (!tk_gemm_wide_plan(a, p.wide, &w)) return false;
+        const int total = w.groups * w.ny, per = ((total + 3) / 4 + 7) / 8;
+        const dim3 wgrid((unsigned)per * 8);
+        if (p.wide == 1) hipLaunchKernelGGL((k_gemm_wide<1, 1, 32, 2>), wgrid, dim3(256), 0, s, a, w.groups, total, per);
+        else hipLaunchKernelGGL((k_gemm_wide<2, 1, 16, 2>), wgrid, dim3(256), 0, s, a, w.groups, total, per);
+        return hipGetLastError() == hipSuccess;
+    }
     const int row_tiles = tw_row_tiles(a);
     if (a.ln_x) {
         if (p.mt != 1 || !p.one) return false;
