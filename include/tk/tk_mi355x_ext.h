@@ -263,6 +263,9 @@ TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_f32_form(int M, int N, int K,
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_conv_direct(int device, const int shape[15], const int* cut, const float* x0, const float* x1, const float* w, const float* bias,
                                                           const float* residual, float* y, int* used);
 
+/* test hook: n floats rounded to binary16 on the device, as the kernels do it (common/tk_exact_math.h: tk_f32_to_f16) */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_f32_to_f16(int device, const float* x, int n, uint16_t* bits);
+
 /* test hook: the blocks that a product of the layer-list decoders is cut into (csrc/nn/tk_gemm_image.h): rows x K against N x K, operands f32 or bf16;
  * swiglu: N = gate and up rows together; experts > 0: every row goes to `top` of them; max_slabs: parts of k at most.  form = rows, columns and LDS
  * stages of a block, parts of k; stages = 0: the kernel for few rows.  No GPU involved. */

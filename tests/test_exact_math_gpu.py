@@ -41,3 +41,22 @@ def test_activations_of_the_kernels_are_the_hosts(gpu, act, form):
     for n in (0, 7, 15):
         same = (c[:, n].view(np.uint32) == want.view(np.uint32)) | (np.isnan(c[:, n]) & np.isnan(want))
         assert same.all(), [(float(v[i]), float(c[i, n]), float(want[i])) for i in np.flatnonzero(~same)[:5]]
+
+
+@pytest.mark.gpu
+def test_f16_rounding_of_the_kernels_is_the_host_arithmetic(gpu):
+    """every 16-bit result's neighbourhood: halfway points and one unit to either side, subnormals, overflow, infinities, NaN of both signs"""
+    half = np.arange(0, 0x7C01, dtype=np.uint16).view(np.float16).astype(np.float32)
+    half[-1] = 65536.0  # the value that infinity stands for in the spacing of the last finite ones
+    mid = ((half[:-1].astype(np.float64) + half[1:]) / 2).astype(np.float32)  # exact
+    near = [(t.view(np.int32) + d).view(np.float32) for t in (half, mid) for d in (-1, 0, 1)]
+    bits = np.random.default_rng(8).integers(0, 1 << 32, 1 << 18, np.uint64).astype(np.uint32).view(np.float32)
+    x = np.concatenate(near + [-t for t in near] + [bits, np.array([0x7F800000, 0xFF800000, 0x7FC00000, 0xFFC00000, 0x7F800001, 0xFFBFFFFF, 0, 0x80000000, 1, 0x80000001], np.uint32).view(np.float32)])
+    got = np.zeros(len(x), np.uint16)
+    gpu.check(gpu.lib().tk_mi355x_f32_to_f16(0, x.ctypes.data_as(C.POINTER(C.c_float)), len(x), got.ctypes.data_as(C.POINTER(C.c_uint16))))
+    with np.errstate(all="ignore"):
+        want = x.astype(np.float16).view(np.uint16)
+    nan = np.isnan(x)
+    want[nan] = np.where(np.signbit(x[nan]), 0xFE00, 0x7E00)
+    bad = np.flatnonzero(got != want)
+    assert len(bad) == 0, [(hex(int(x.view(np.uint32)[i])), hex(int(got[i])), hex(int(want[i]))) for i in bad[:5]]

@@ -255,6 +255,29 @@ tk_error_code_t tk_mi355x_conv_direct(int device, const int shape[15], const int
     return !fits ? TK_ERROR_INVALID_ARGUMENT : ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
 }
 
+static __global__ __launch_bounds__(256) void k_f32_to_f16(const float* __restrict__ x, int n, uint16_t* __restrict__ bits) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) bits[i] = tk_f32_to_f16(x[i]);
+}
+
+tk_error_code_t tk_mi355x_f32_to_f16(int device, const float* x, int n, uint16_t* bits) {
+    if (!x || !bits || n < 1 || n > 1 << 28) return TK_ERROR_INVALID_ARGUMENT;
+    int have = 0;
+    if (hipGetDeviceCount(&have) != hipSuccess || have <= 0) return TK_ERROR_GPU_DEVICE_NOT_FOUND;
+    if (device < 0 || device >= have || hipSetDevice(device) != hipSuccess) return TK_ERROR_INVALID_ARGUMENT;
+    float* dx = nullptr;
+    uint16_t* db = nullptr;
+    bool ok = hipMalloc((void**)&dx, (size_t)n * 4) == hipSuccess && hipMalloc((void**)&db, (size_t)n * 2) == hipSuccess &&
+              hipMemcpy(dx, x, (size_t)n * 4, hipMemcpyHostToDevice) == hipSuccess;
+    if (ok) {
+        hipLaunchKernelGGL(k_f32_to_f16, dim3((n + 255) / 256), dim3(256), 0, nullptr, dx, n, db);
+        ok = hipGetLastError() == hipSuccess && hipMemcpy(bits, db, (size_t)n * 2, hipMemcpyDeviceToHost) == hipSuccess;
+    }
+    if (dx) (void)hipFree(dx);
+    if (db) (void)hipFree(db);
+    return ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
+}
+
 tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]) {
     if (rows <= 0 || N <= 0 || K <= 0 || experts < 0 || (experts > 0 && (top < 1 || top > experts)) || !form) return TK_ERROR_INVALID_ARGUMENT;
     const int to = swiglu ? 32 : 16;
