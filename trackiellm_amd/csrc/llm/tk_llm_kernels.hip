@@ -21,6 +21,7 @@
 
 #include "../common/tk_ggml_blocks.h"
 #include "../common/tk_sample_device.h"
+#include "../nn/tk_image_device.h"
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
@@ -196,23 +197,13 @@ void tk_launch_embed(const void* embd, int type, int D, const int32_t* tok, int 
 /* ------------------------------------------------------------------------------------------
  * shared device helpers
  * ------------------------------------------------------------------------------------------ */
-__device__ __forceinline__ float wave_xor_f(float v, int mask) { return __shfl_xor(v, mask, TK_WAVE); }
-
-/* canonical sum of 256 per-thread partials (oracle: orc_sum256) */
-__device__ __forceinline__ float block_sum256(float v, float* red /* >= 4 floats LDS */) {
-    for (int s = 32; s >= 1; s >>= 1) v = v + wave_xor_f(v, s);
-    const int w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 0) red[w] = v;
-    __syncthreads();
-    float r = ((red[0] + red[1]) + red[2]) + red[3];
-    __syncthreads();
-    return r;
-}
-
 /*
  * Quantise one 8-element chunk (chunk index c of the row) to the aq/ad/abs images.
  * Must be called by all 32 lanes of a half-wave that together hold one 256-block
- * (lane order == chunk order), so the block amax / sub-block sums come from shuffles.
+ * (lane order == chunk order), so the block amax / sub-block sums come from lane exchanges on the vector
+ * pipe: the magnitude's maximum by row rotations, then the sign of its first element from two ballots.  As butterflies of (magnitude, value, index)
+ * through LDS permutes this was a chain of sixteen LDS round
+ * trips: k_rmsnorm_q8 at 16 rows 6.3 -> 5.6 us, k_quant_q8 at 256 rows of 14336 8.1 -> 7.0, the mat-vec launches that quantise for themselves - 0.4 .. 0.6.
  */
 __device__ __forceinline__ void quantize_chunk8(const float* v, int c, int slot, TkActQ8 out) {
     if (out.af) { /* the f16-weight matmuls' input: the same values rounded through f16, in the tiled GEMM's operand-image order (csrc/nn/tk_gemm_tiled.h) */
@@ -220,24 +211,23 @@ __device__ __forceinline__ void quantize_chunk8(const float* v, int c, int slot,
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int k16 = 8 * (c & 1) + i; /* position inside the group of 16: g = k16 % 4, t = k16 / 4 */
-            dst[(k16 & 3) * 64 + (k16 >> 2)] = tk_f16_to_f32(tk_f32_to_f16(v[i]));
+            dst[(k16 & 3) * 64 + (k16 >> 2)] = (float)__builtin_bit_cast(_Float16, tk_f32_to_f16(v[i]));
         }
     }
     /* ggml's quantize_row_q8_K_ref: the signed value of the block's FIRST element of largest magnitude (element index = 8 x chunk-in-block + i),
      * iscale = -127 / max, q = min(127, nearest_int(iscale * x)), d = 1 / iscale */
-    float amax = 0.0f, mval = 0.0f;
-    int midx = 8 * (c & 31);
+    float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const float ax = tk_fabsf(v[i]);
-        if (ax > amax) { amax = ax; mval = v[i]; midx = 8 * (c & 31) + i; }
-    }
+    for (int i = 0; i < 8; ++i) amax = tk_max2(tk_fabsf(v[i]), amax); /* a NaN does not enter */
+    const float mine = amax;
+    amax = tk_row32_max(amax);
+    bool neg = false;
 #pragma unroll
-    for (int s = 1; s <= 16; s <<= 1) {
-        const float oa = wave_xor_f(amax, s), ov = wave_xor_f(mval, s);
-        const int oi = __shfl_xor(midx, s, TK_WAVE);
-        if (oa > amax || (oa == amax && oi < midx)) { amax = oa; mval = ov; midx = oi; }
-    }
+    for (int i = 7; i >= 0; --i) neg = tk_fabsf(v[i]) == amax ? v[i] < 0.0f : neg;
+    const uint64_t who64 = __ballot(mine == amax), neg64 = __ballot(neg);
+    const bool upper = (threadIdx.x & 32) != 0;
+    const uint32_t who = upper ? (uint32_t)(who64 >> 32) : (uint32_t)who64, negs = upper ? (uint32_t)(neg64 >> 32) : (uint32_t)neg64;
+    const float mval = (negs >> __builtin_ctz(who)) & 1u ? -amax : amax; /* lanes are chunks in order: the first that holds the maximum decides */
     const float iscale = amax > 0.0f ? tk_divf(-127.0f, mval) : 0.0f;
     int q[8];
     int sum = 0;
@@ -253,8 +243,8 @@ __device__ __forceinline__ void quantize_chunk8(const float* v, int c, int slot,
     const int mt = slot >> 4, sl = slot & 15; /* M-tile and slot inside it */
     /* image order [K/64][4 g][16 slot][2 sub-blocks][8]: c = 4 * sub-block + g; a lane's operand of one x64 MFMA is one 16-byte read */
     *(uint2*)(out.aq + mt * out.aq_ts + (size_t)(c >> 3) * 1024 + ((size_t)(c & 3) * TK_ROW_SLOTS + sl) * 16 + ((c >> 2) & 1) * 8) = make_uint2(lo, hi);
-    sum += __shfl_xor(sum, 1, TK_WAVE);
-    sum += __shfl_xor(sum, 2, TK_WAVE);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xf, 0xf, false); /* lane ^ 1, lane ^ 2 */
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xf, 0xf, false);
     if ((c & 3) == 0) { /* sub-block sum as two int8: sum = 64 * h + l, l in [0, 63], h in [-64, 63]  (|sum| <= 32 * 127) */
         int8_t* mb = out.abs + mt * out.abs_ts + (size_t)(c >> 5) * 256 + (size_t)sl * 8 + ((c >> 2) & 7);
         mb[0] = (int8_t)(sum & 63);
@@ -317,8 +307,8 @@ __global__ __launch_bounds__(1024) void k_rmsnorm_q8(float* __restrict__ x, cons
 #pragma unroll
             for (int i = 0; i < 4; ++i) ss = tk_fmaf(v[i], v[i], ss);
         }
-    /* canonical sum of the 256 chains (block_sum256's arithmetic, carried by the first four waves of a wider workgroup) */
-    for (int s = 32; s >= 1; s >>= 1) ss = ss + wave_xor_f(ss, s);
+    /* canonical sum of the 256 chains (oracle: orc_sum256), carried by the first four waves of a wider workgroup */
+    ss = tk_wave_butterfly_sum(ss);
     if (t < 256 && (t & 63) == 0) red[t >> 6] = ss;
     __syncthreads();
     const float tot = ((red[0] + red[1]) + red[2]) + red[3];
@@ -674,7 +664,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
 #pragma unroll
                         for (int i = 0; i < 4; ++i) ss = tk_fmaf(v[i], v[i], ss);
                     }
-                    for (int sh = 32; sh >= 1; sh >>= 1) ss = ss + wave_xor_f(ss, sh);
+                    ss = tk_wave_butterfly_sum(ss);
                     if (lane == 0) red[vw] = ss;
                 }
                 __syncthreads();
@@ -1638,12 +1628,33 @@ bool tk_gemv_fuses_producer(int nrows, int K, int ks, int fks) {
 
 /* ------------------------------------------------------------------------------------------
  * q/k/v: sum K-split partials, RoPE (adjacent pairs), append K/V (f16) to the cache.
- * grid (n_kv_head, nrows); 256 threads = one q pair each (4 q heads x 64 pairs per kv head).
+ * grid (n_kv_head, nrows); a thread = one pair of a query head, the key or the value.  The slabs are the traffic (25 MB at 256 rows of 4 x 6144) and
+ * the launch is a few trips to them: a pair's slabs are requested together, 8 bytes a lane (10.9 -> 7.2 us).
  * ------------------------------------------------------------------------------------------ */
-__device__ __forceinline__ float sum_partials(const float* partial, int ks, int n_total, int row, int col) {
-    float o = partial[(int64_t)row * n_total + col];
-    for (int s = 1; s < ks; ++s) o = o + partial[((int64_t)s * TK_MAX_ROWS + row) * n_total + col];
+/* the K-split sums of columns col, col + 1 (col even, pitches multiples of 64): every slab requested before the first add, slabs added in ascending
+ * order.  The number of slabs is a compile-time number inside each case: loads under a test of their own (eight, for any ks) are waited for at every join. */
+template <int KS> __device__ __forceinline__ float2 sum_slabs_pair(const float* row0, int64_t pitch, uint32_t col) {
+    float2 v[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) v[s] = *(const float2*)((const uint8_t*)(row0 + s * pitch) + col * 4u); /* wave-uniform base, 32-bit lane offset */
+    float2 o = v[0];
+#pragma unroll
+    for (int s = 1; s < KS; ++s) { o.x = o.x + v[s].x; o.y = o.y + v[s].y; }
     return o;
+}
+__device__ __forceinline__ float2 sum_partials_pair(const float* partial, int ks, int n_total, int row, int col) {
+    const float* p = partial + (int64_t)row * n_total;
+    const int64_t pitch = (int64_t)TK_MAX_ROWS * n_total;
+    switch (ks) {
+    case 1: return sum_slabs_pair<1>(p, pitch, (uint32_t)col);
+    case 2: return sum_slabs_pair<2>(p, pitch, (uint32_t)col);
+    case 3: return sum_slabs_pair<3>(p, pitch, (uint32_t)col);
+    case 4: return sum_slabs_pair<4>(p, pitch, (uint32_t)col);
+    case 5: return sum_slabs_pair<5>(p, pitch, (uint32_t)col);
+    case 6: return sum_slabs_pair<6>(p, pitch, (uint32_t)col);
+    case 7: return sum_slabs_pair<7>(p, pitch, (uint32_t)col);
+    default: return sum_slabs_pair<8>(p, pitch, (uint32_t)col); /* TK_RMS_MAX_KS: TkLlmModel::init admits no more */
+    }
 }
 
 __global__ void k_qkv_rope_append(const float* partial, int ks, int n_total, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
@@ -1656,31 +1667,23 @@ __global__ void k_qkv_rope_append(const float* partial, int ks, int n_total, int
     const float* cs = rope_cos + (int64_t)p * half;
     const float* sn = rope_sin + (int64_t)p * half;
     const int64_t cbase = ((((int64_t)layer * max_seq + sq) * n_kv_head + kvh) * max_ctx + p) * head_dim; /* [layer][seq][kv head][ctx][dim] */
-    for (int idx = threadIdx.x; idx < (grp + 1) * half; idx += blockDim.x) {
+    for (int idx = threadIdx.x; idx < (grp + 2) * half; idx += blockDim.x) {
         const int hsel = idx / half, i = idx % half;
-        if (hsel < grp) {
-            const int col = (kvh * grp + hsel) * head_dim + 2 * i;
-            const float a = sum_partials(partial, ks, n_total, r, col);
-            const float b = sum_partials(partial, ks, n_total, r, col + 1);
-            qbuf[(int64_t)r * QD + col] = tk_fmaf(-b, sn[i], a * cs[i]);
-            qbuf[(int64_t)r * QD + col + 1] = tk_fmaf(a, sn[i], b * cs[i]);
-        } else {
-            const int col = QD + kvh * head_dim + 2 * i;
-            const float a = sum_partials(partial, ks, n_total, r, col);
-            const float b = sum_partials(partial, ks, n_total, r, col + 1);
-            kcache[cbase + 2 * i] = tk_f32_to_f16(tk_fmaf(-b, sn[i], a * cs[i]));
-            kcache[cbase + 2 * i + 1] = tk_f32_to_f16(tk_fmaf(a, sn[i], b * cs[i]));
-            const int vcol = QD + KVD + kvh * head_dim + 2 * i;
-            vcache[cbase + 2 * i] = tk_f32_to_f16(sum_partials(partial, ks, n_total, r, vcol));
-            vcache[cbase + 2 * i + 1] = tk_f32_to_f16(sum_partials(partial, ks, n_total, r, vcol + 1));
-        }
+        const int col = hsel < grp ? (kvh * grp + hsel) * head_dim + 2 * i : (hsel == grp ? QD : QD + KVD) + kvh * head_dim + 2 * i;
+        const float c = cs[i], sv = sn[i];
+        const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+        const float2 rot = {tk_fmaf(-ab.y, sv, ab.x * c), tk_fmaf(ab.x, sv, ab.y * c)};
+        if (hsel < grp) *(float2*)(qbuf + (int64_t)r * QD + col) = rot;
+        else if (hsel == grp) *(uint32_t*)(kcache + cbase + 2 * i) = (uint32_t)tk_f32_to_f16(rot.x) | ((uint32_t)tk_f32_to_f16(rot.y) << 16);
+        else *(uint32_t*)(vcache + cbase + 2 * i) = (uint32_t)tk_f32_to_f16(ab.x) | ((uint32_t)tk_f32_to_f16(ab.y) << 16);
     }
 }
 
 void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
                                const float* rope_sin, const int32_t* seq, const int32_t* pos, int nrows, float* qbuf, uint16_t* kcache,
                                uint16_t* vcache, int layer, int max_seq, int max_ctx, hipStream_t s) {
-    hipLaunchKernelGGL(k_qkv_rope_append, dim3(n_kv_head, nrows), dim3(256), 0, s, partial, ks, n_total, n_head, n_kv_head, head_dim, rope_cos,
+    const int items = (n_head / n_kv_head + 2) * (head_dim / 2); /* a multiple of 32 */
+    hipLaunchKernelGGL(k_qkv_rope_append, dim3(n_kv_head, nrows), dim3(items < 512 ? (items + 63) / 64 * 64 : 512), 0, s, partial, ks, n_total, n_head, n_kv_head, head_dim, rope_cos,
                        rope_sin, seq, pos, qbuf, kcache, vcache, layer, max_seq, max_ctx);
 }
 
@@ -1705,18 +1708,6 @@ void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int n_
 /* ring slots (template parameter SLOTS, 2 everywhere): the next chunk lands while the current one is used.  Wide passes (256 rows x 128
  * cached positions, profiles/r02_attention_variants.txt: 2 x 64 rows 53.5 us, 8 x 32 rows 86 us) want a small LDS footprint — workgroups per
  * CU pay, not bytes in flight per workgroup; narrow ones gain nothing from a deeper ring either (profiles/r03_attention_slots.txt) */
-__device__ __forceinline__ float sum_partials_wide(const float* partial, int ks, int n_total, int row, int col) {
-    float p[TK_RMS_MAX_KS];
-#pragma unroll
-    for (int s = 0; s < TK_RMS_MAX_KS; ++s)
-        if (s < ks) p[s] = partial[((int64_t)s * TK_MAX_ROWS + row) * n_total + col];
-    float o = p[0];
-#pragma unroll
-    for (int s = 1; s < TK_RMS_MAX_KS; ++s)
-        if (s < ks) o = o + p[s];
-    return o;
-}
-
 /* stage rows [row0, row0 + 32) of one (sequence, kv head) cache run into an LDS slot; rows past `last_row` are clamped (their
  * content is never used).  swz: XOR-swizzle the 16-byte pieces of a row by the row number (K); plain copy otherwise (V).
  * Every wave issues exactly chunk_bytes / 4096 one-KiB pieces: the counted waits rely on it. */
@@ -1739,10 +1730,7 @@ __device__ __forceinline__ void att_stage(const uint16_t* run, int row0, int las
 }
 
 template <int GQ, bool FUSED, int HD /* head_dim when it is 64 or 128 (loops unroll, LDS reads batch), 0 = any */, int CH /* positions per ring slot */, int SLOTS = 2>
-#ifndef TK_ATT_WAVES
-#define TK_ATT_WAVES 1
-#endif
-__global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __restrict__ qbuf, const float* __restrict__ partial, int ks, int n_total,
+__global__ __launch_bounds__(256) void k_attention(const float* __restrict__ qbuf, const float* __restrict__ partial, int ks, int n_total,
                                                     const float* __restrict__ rope_cos, const float* __restrict__ rope_sin,
                                                     uint16_t* __restrict__ kcache, uint16_t* __restrict__ vcache, const int32_t* __restrict__ seq,
                                                     const int32_t* __restrict__ pos, int n_head, int n_kv_head, int head_dim_rt, int layer, int max_seq,
@@ -1796,26 +1784,20 @@ __global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __
     if (FUSED) {
         const float* cs = rope_cos + (int64_t)p * half;
         const float* sn = rope_sin + (int64_t)p * half;
+#pragma unroll 1 /* the passes side by side take 150 registers: three workgroups a CU where the LDS holds seven */
         for (int idx = t; idx < (GQ + 2) * half; idx += 256) {
             const int hsel = idx / half, i = idx % half;
+            const int col = hsel < GQ ? (hb * GQ + hsel) * head_dim + 2 * i : (hsel == GQ ? QD : QD + KVD) + kvh * head_dim + 2 * i;
+            const float c = cs[i], sv = sn[i];
+            const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+            const float2 rot = {tk_fmaf(-ab.y, sv, ab.x * c), tk_fmaf(ab.x, sv, ab.y * c)};
             if (hsel < GQ) {
-                const int col = (hb * GQ + hsel) * head_dim + 2 * i;
-                const float a = sum_partials_wide(partial, ks, n_total, r, col), b = sum_partials_wide(partial, ks, n_total, r, col + 1);
-                qs[hsel * head_dim + 2 * i] = tk_fmaf(-b, sn[i], a * cs[i]);
-                qs[hsel * head_dim + 2 * i + 1] = tk_fmaf(a, sn[i], b * cs[i]);
-            } else if (hsel == GQ) {
-                const int col = QD + kvh * head_dim + 2 * i;
-                const float a = sum_partials_wide(partial, ks, n_total, r, col), b = sum_partials_wide(partial, ks, n_total, r, col + 1);
-                const uint16_t k0 = tk_f32_to_f16(tk_fmaf(-b, sn[i], a * cs[i])), k1 = tk_f32_to_f16(tk_fmaf(a, sn[i], b * cs[i]));
-                const uint32_t kk = (uint32_t)k0 | ((uint32_t)k1 << 16);
-                *(uint32_t*)(kcache + run0 + (int64_t)p * head_dim + 2 * i) = kk;
-                *(uint32_t*)(own + 2 * i) = kk;
+                *(float2*)(qs + hsel * head_dim + 2 * i) = rot;
             } else {
-                const int col = QD + KVD + kvh * head_dim + 2 * i;
-                const uint16_t v0 = tk_f32_to_f16(sum_partials_wide(partial, ks, n_total, r, col)), v1 = tk_f32_to_f16(sum_partials_wide(partial, ks, n_total, r, col + 1));
-                const uint32_t vv = (uint32_t)v0 | ((uint32_t)v1 << 16);
-                *(uint32_t*)(vcache + run0 + (int64_t)p * head_dim + 2 * i) = vv;
-                *(uint32_t*)(own + head_dim + 2 * i) = vv;
+                const float2 kv = hsel == GQ ? rot : ab;
+                const uint32_t both = (uint32_t)tk_f32_to_f16(kv.x) | ((uint32_t)tk_f32_to_f16(kv.y) << 16);
+                *(uint32_t*)((hsel == GQ ? kcache : vcache) + run0 + (int64_t)p * head_dim + 2 * i) = both;
+                *(uint32_t*)(own + (hsel == GQ ? 0 : head_dim) + 2 * i) = both;
             }
         }
     } else {
@@ -1863,12 +1845,10 @@ __global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __
     }
     /* row maximum per head: thread idx = h * CHUNK + rr served head h in every chunk (GQ * CHUNK <= 256 threads: one idx per thread) */
     if (CH <= 64) {
-        float m = mx;
-        for (int s = CH / 2; s >= 1; s >>= 1) m = tk_fmaxf(m, wave_xor_f(m, s)); /* over the CHUNK lanes of one head */
+        const float m = CH == 64 ? tk_wave_max(mx) : tk_row32_max(mx); /* over the CHUNK lanes of one head */
         if ((lane & (CH - 1)) == 0 && t < GQ * CH) red[t / CH] = m;
     } else { /* a head's CHUNK threads span CH / 64 whole waves: per-wave maxima, joined below (a maximum does not depend on the order) */
-        float m = mx;
-        for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, wave_xor_f(m, s));
+        const float m = tk_wave_max(mx);
         if (lane == 0) red[TK_ATT_MAX_GRP + wave] = m; /* the second row of red[4][GQ <= 4]: free until the epilogue's lpart, which lives in the ring */
     }
     __syncthreads(); /* every score is written */
@@ -2015,24 +1995,18 @@ __global__ __launch_bounds__(1024) void k_attention_narrow(const float* __restri
         const float* cs = rope_cos + (int64_t)p * half;
         const float* sn = rope_sin + (int64_t)p * half;
         const int hsel = t / half, i = t % half;
+        const int col = hsel < GQ ? (hb * GQ + hsel) * HD + 2 * i : (hsel == GQ ? QD : QD + KVD) + kvh * HD + 2 * i;
+        const float c = cs[i], sv = sn[i];
+        const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+        const float2 rot = {tk_fmaf(-ab.y, sv, ab.x * c), tk_fmaf(ab.x, sv, ab.y * c)};
         if (hsel < GQ) {
-            const int col = (hb * GQ + hsel) * HD + 2 * i;
-            const float a = sum_partials_wide(partial, ks, n_total, r, col), b = sum_partials_wide(partial, ks, n_total, r, col + 1);
-            qs[hsel * HD + 2 * i] = tk_fmaf(-b, sn[i], a * cs[i]);
-            qs[hsel * HD + 2 * i + 1] = tk_fmaf(a, sn[i], b * cs[i]);
-        } else if (hsel == GQ) {
-            const int col = QD + kvh * HD + 2 * i;
-            const float a = sum_partials_wide(partial, ks, n_total, r, col), b = sum_partials_wide(partial, ks, n_total, r, col + 1);
-            const uint16_t k0 = tk_f32_to_f16(tk_fmaf(-b, sn[i], a * cs[i])), k1 = tk_f32_to_f16(tk_fmaf(a, sn[i], b * cs[i]));
-            const uint32_t kk = (uint32_t)k0 | ((uint32_t)k1 << 16);
-            if ((hb * GQ) % (n_head / n_kv_head) == 0) *(uint32_t*)(kcache + run0 + (int64_t)p * HD + 2 * i) = kk; /* one workgroup of the KV group appends */
-            *(uint32_t*)(own + 2 * i) = kk;
+            *(float2*)(qs + hsel * HD + 2 * i) = rot;
         } else {
-            const int col = QD + KVD + kvh * HD + 2 * i;
-            const uint16_t v0 = tk_f32_to_f16(sum_partials_wide(partial, ks, n_total, r, col)), v1 = tk_f32_to_f16(sum_partials_wide(partial, ks, n_total, r, col + 1));
-            const uint32_t vv = (uint32_t)v0 | ((uint32_t)v1 << 16);
-            if ((hb * GQ) % (n_head / n_kv_head) == 0) *(uint32_t*)(vcache + run0 + (int64_t)p * HD + 2 * i) = vv;
-            *(uint32_t*)(own + HD + 2 * i) = vv;
+            const float2 kv = hsel == GQ ? rot : ab;
+            const uint32_t both = (uint32_t)tk_f32_to_f16(kv.x) | ((uint32_t)tk_f32_to_f16(kv.y) << 16);
+            if ((hb * GQ) % (n_head / n_kv_head) == 0) /* one workgroup of the KV group appends */
+                *(uint32_t*)((hsel == GQ ? kcache : vcache) + run0 + (int64_t)p * HD + 2 * i) = both;
+            *(uint32_t*)(own + (hsel == GQ ? 0 : HD) + 2 * i) = both;
         }
     }
     const float att_scale = tk_divf(1.0f, tk_sqrtf((float)HD));
@@ -2072,7 +2046,7 @@ __global__ __launch_bounds__(1024) void k_attention_narrow(const float* __restri
             mx = tk_fmaxf(mx, sv);
         }
     }
-    for (int s2 = 32; s2 >= 1; s2 >>= 1) mx = tk_fmaxf(mx, wave_xor_f(mx, s2));
+    mx = tk_wave_max(mx);
     if (lane == 0) red[wave] = mx;
     __syncthreads(); /* every score and every wave maximum is written */
     if (t < GQ) {
@@ -2321,7 +2295,7 @@ __global__ __launch_bounds__((256 / HD) * 256) void k_attention_prefill(const fl
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        for (int s = 8; s >= 1; s >>= 1) mx[i] = tk_fmaxf(mx[i], wave_xor_f(mx[i], s));
+        mx[i] = tk_row16_max(mx[i]);
         if (n16 == 0) mred[w * 16 + 4 * G + i] = mx[i];
     }
     __syncthreads();
@@ -2450,7 +2424,8 @@ __global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict
         for (int idx = t; idx < (GQ + (last ? 2 : 0)) * HALF; idx += 256) {
             const int hsel = idx / HALF, i = idx % HALF;
             const int col = hsel < GQ ? (kvh * GQ + hsel) * HD + 2 * i : (hsel == GQ ? QD : QD + KVD) + kvh * HD + 2 * i;
-            const float a = sum_partials(partial, ks, n_total, r, col), bb = sum_partials(partial, ks, n_total, r, col + 1);
+            const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+            const float a = ab.x, bb = ab.y;
             if (hsel < GQ) {
                 qs[hsel * HD + 2 * i] = tk_fmaf(-bb, sn[i], a * cs[i]);
                 qs[hsel * HD + 2 * i + 1] = tk_fmaf(a, sn[i], bb * cs[i]);
@@ -2527,7 +2502,7 @@ __global__ __launch_bounds__(64) void k_att_pv_chain(const float* __restrict__ s
 #pragma unroll
         for (int u = 0; u < 16; ++u) m = tk_fmaxf(m, sv[u]);
     }
-    for (int sft = 32; sft >= 1; sft >>= 1) m = tk_fmaxf(m, wave_xor_f(m, sft));
+    m = tk_wave_max(m);
     const int nj = T > j ? (T - j + 3) / 4 : 0; /* positions j, j + 4, ... of this class */
     /* The chain: a lane owns two dims (head_dim 64: the upper half-wave mirrors the lower).  Chunks of 32 class positions, two register
      * sets: a chunk's value rows are requested a chunk before the chain reaches them; the scores of a chunk are requested two chunks ahead

@@ -89,6 +89,28 @@ __device__ __forceinline__ TkPair tk_halves(float v) {
     const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return TkPair{__uint_as_float(p[0]), __uint_as_float(p[1])};
 }
+/* sum of the wave's lanes in the canonical butterfly order (lane ^ 32, ^ 16, ^ 8, ^ 4, ^ 2, ^ 1; the oracles' 256-sum), in every lane.  After lane ^ 8 a
+ * row repeats every 8 lanes, so a rotation by 4 IS lane ^ 4.  The six steps as LDS permutes were a chain of six LDS round trips. */
+__device__ __forceinline__ float tk_wave_butterfly_sum(float v) {
+    const TkPair h = tk_halves(v);
+    const TkPair r = tk_rows(h.a + h.b);
+    v = r.a + r.b;
+    v += tk_dpp<0x128>(v);
+    v += tk_dpp<0x124>(v);
+    v += tk_dpp<0x4E>(v);
+    v += tk_dpp<0xB1>(v);
+    return v;
+}
+__device__ __forceinline__ float tk_max2(float a, float b) { return a > b ? a : b; }
+/* maximum over the 16 lanes of a row, the 32 lanes of a half-wave, the wave (no NaN among the values), in every lane of it */
+__device__ __forceinline__ float tk_row16_max(float v) {
+    v = tk_max2(v, tk_dpp<0x128>(v));
+    v = tk_max2(v, tk_dpp<0x124>(v));
+    v = tk_max2(v, tk_dpp<0x122>(v));
+    return tk_max2(v, tk_dpp<0x121>(v));
+}
+__device__ __forceinline__ float tk_row32_max(float v) { const TkPair p = tk_rows(tk_row16_max(v)); return tk_max2(p.a, p.b); }
+__device__ __forceinline__ float tk_wave_max(float v) { const TkPair p = tk_halves(tk_row32_max(v)); return tk_max2(p.a, p.b); }
 __device__ __forceinline__ float tk_row32_sum(float v) { const TkPair p = tk_rows(tk_row16_sum(v)); return p.a + p.b; }
 __device__ __forceinline__ float tk_wave_sum(float v) { const TkPair p = tk_halves(tk_row32_sum(v)); return p.a + p.b; }
 /* over the four lanes l % 16 + 16 g */
