@@ -260,6 +260,23 @@ __device__ __forceinline__ void quantize_chunk8(const float* v, int c, int slot,
     if ((c & 31) == 0) out.ad[mt * out.ad_ts + (size_t)(c >> 5) * TK_ROW_SLOTS + sl] = amax > 0.0f ? tk_divf(1.0f, iscale) : 0.0f;
 }
 
+/* Which row and 2048-column piece a workgroup of k_swiglu_q8 / k_quant_q8 takes.  The images hold the 16 rows of an M-tile side by side, 8 of every 128
+ * bytes from each: rows quantised on different XCDs leave every line as partial writes of several L2 caches.  Workgroups go to the XCDs in turn (block % 8),
+ * so the 16 rows of a (M-tile, piece) take one residue; blocks past the last row leave at once.  k_quant_q8 at 256 rows of 14336 7.0 -> 5.6 us,
+ * k_swiglu_q8 20.6 -> 13.8.  Below 16 such units some XCDs would take twice the others' work (16 rows of 14336: 4.6 us row by row, 4.8 by units); for
+ * k_rmsnorm_q8, whose time is its slabs, the order changes nothing. */
+struct TkQuantBlock { int row, piece; };
+__host__ __device__ __forceinline__ int quant_units(int nrows, int pieces) { return (nrows + 15) / 16 * pieces; }
+__host__ __device__ __forceinline__ int quant_blocks(int nrows, int pieces) {
+    const int units = quant_units(nrows, pieces);
+    return units < 16 ? nrows * pieces : 8 * 16 * ((units + 7) / 8);
+}
+__device__ __forceinline__ TkQuantBlock quant_block(int b, int nrows, int pieces) {
+    if (quant_units(nrows, pieces) < 16) return TkQuantBlock{b / pieces, b % pieces};
+    const int unit = (b & 7) + 8 * (b >> 7); /* b = 128 j + 8 r + x: row r of unit 8 j + x */
+    return TkQuantBlock{unit / pieces * 16 + ((b >> 3) & 15), unit % pieces};
+}
+
 /* ------------------------------------------------------------------------------------------
  * residual add (sum of K-split partials, ascending) + RMSNorm + Q8 quantise.  One WG per row.
  *
@@ -2762,10 +2779,10 @@ void tk_launch_attention(const float* qbuf, const float* partial, int ks, int n_
 /* KSM = the most K-split slabs an instantiation handles: the slab loads are held in registers before the first add, and the gate | up
  * projection of the canonical plan has ONE slab — with room for eight the kernel needs 130 registers (3 waves per SIMD), with one 40 */
 template <int KSM>
-__global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks, int FF, TkActQ8 out) {
-    const int r = blockIdx.y;
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= FF / 8) return; /* FF/8 is a multiple of 32: whole half-waves drop out together */
+__global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks, int FF, int nrows, TkActQ8 out) {
+    const TkQuantBlock qb = quant_block(blockIdx.x, nrows, (FF / 8 + 255) / 256);
+    const int r = qb.row, c = qb.piece * 256 + threadIdx.x;
+    if (r >= nrows || c >= FF / 8) return; /* FF/8 is a multiple of 32: whole half-waves drop out together */
     /* 8 gate and 8 up values as 16-byte loads, every K-split slab requested before the first add (slabs added in ascending order) */
     v4f g[2], u[2];
     {
@@ -2789,10 +2806,10 @@ __global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks,
 }
 
 /* the Q8 quantisation alone, for h = silu(gate) * up that the wide gate | up launch has formed in its epilogue (TkGemvArgs::swiglu) */
-__global__ __launch_bounds__(256) void k_quant_q8(const float* __restrict__ hbuf, int FF, TkActQ8 out) {
-    const int r = blockIdx.y;
-    const int c = blockIdx.x * 256 + threadIdx.x;
-    if (c >= FF / 8) return; /* FF/8 is a multiple of 32: whole half-waves drop out together */
+__global__ __launch_bounds__(256) void k_quant_q8(const float* __restrict__ hbuf, int FF, int nrows, TkActQ8 out) {
+    const TkQuantBlock qb = quant_block(blockIdx.x, nrows, (FF / 8 + 255) / 256);
+    const int r = qb.row, c = qb.piece * 256 + threadIdx.x;
+    if (r >= nrows || c >= FF / 8) return; /* FF/8 is a multiple of 32: whole half-waves drop out together */
     const float* row = hbuf + (int64_t)r * FF + 8 * c;
     const v4f a = *(const v4f*)row, b = *(const v4f*)(row + 4);
     float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
@@ -2800,7 +2817,7 @@ __global__ __launch_bounds__(256) void k_quant_q8(const float* __restrict__ hbuf
 }
 
 void tk_launch_quant_q8(const float* hbuf, int FF, int nrows, TkActQ8 out, hipStream_t s) {
-    hipLaunchKernelGGL(k_quant_q8, dim3((FF / 8 + 255) / 256, nrows), dim3(256), 0, s, hbuf, FF, out);
+    hipLaunchKernelGGL(k_quant_q8, dim3(quant_blocks(nrows, (FF / 8 + 255) / 256)), dim3(256), 0, s, hbuf, FF, nrows, out);
 }
 
 bool tk_gemv_fuses_swiglu(int nrows, int ks, int type_gate, int type_up) {
@@ -2808,8 +2825,9 @@ bool tk_gemv_fuses_swiglu(int nrows, int ks, int type_gate, int type_up) {
 }
 
 void tk_launch_swiglu_q8(const float* partial, int ks, int FF, int nrows, TkActQ8 out, hipStream_t s) {
-    if (ks == 1) hipLaunchKernelGGL((k_swiglu_q8<1>), dim3((FF / 8 + 255) / 256, nrows), dim3(256), 0, s, partial, ks, FF, out);
-    else hipLaunchKernelGGL((k_swiglu_q8<TK_RMS_MAX_KS>), dim3((FF / 8 + 255) / 256, nrows), dim3(256), 0, s, partial, ks, FF, out);
+    const dim3 grid(quant_blocks(nrows, (FF / 8 + 255) / 256));
+    if (ks == 1) hipLaunchKernelGGL((k_swiglu_q8<1>), grid, dim3(256), 0, s, partial, ks, FF, nrows, out);
+    else hipLaunchKernelGGL((k_swiglu_q8<TK_RMS_MAX_KS>), grid, dim3(256), 0, s, partial, ks, FF, nrows, out);
 }
 
 /* ------------------------------------------------------------------------------------------
