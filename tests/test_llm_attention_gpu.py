@@ -325,3 +325,34 @@ def test_prompt_chunks_of_a_long_prompt_bit_exact(mistral_long):
     gk, gv = sess.kv_read(0, 3, 0, n)
     wk, wv = orc.kv_read(0, 3, 0, n)
     assert np.array_equal(gk, wk) and np.array_equal(gv, wv)
+
+
+@pytest.mark.parametrize("head_dim,grp", [(128, 4), (128, 2), (64, 4)])
+def test_long_form_of_one_row_is_the_fused_kernels_bit_for_bit(gpu, monkeypatch, head_dim, grp):
+    """one row from position 256 on in windows up to 2048 (scores, chains, join inside the o projection) and two rows from 512: where a class's rows fill
+    their chunks of 64 or spill by one (256, 257, 767 .. 769, 1023 .. 1025), more rows than are in flight, the window's last position"""
+    hp = gpu.LlmHParams(2, 1024, 8, 8 // grp, head_dim, 1024, 512, 1e-5, 10000.0, 0, 0, 0, 0, 1)
+    model = gpu.LlmModel(hp).fill_synthetic(4)
+    hp, window = model.hparams, 1300
+    rng = np.random.default_rng(head_dim + grp)
+    kv = [(f16_bits(rng, (window, hp.n_kv_head, head_dim), 0.6), f16_bits(rng, (window, hp.n_kv_head, head_dim), 1.0)) for _ in range(4)]
+    runs = {}
+    for off in ("0", "1"):
+        monkeypatch.setenv("TK_MI355X_NO_LONG_ATT", off)
+        sess = gpu.LlmSession(model, 2, window)
+        for layer in range(2):
+            for s in range(2):
+                sess.kv_write(layer, s, 0, *kv[2 * layer + s])
+        for rows, ctx in [(1, c) for c in (1299, 1100, 1025, 1024, 1023, 769, 768, 767, 515, 257, 256)] + [(2, 1299), (2, 1024), (2, 512)]:  # downwards: a step writes its own position
+            want_form = 3 if off == "0" and gpu.lib().tk_mi355x_device_cu_count(0) == 256 else None
+            if want_form:
+                assert gpu.attention_plan(rows, hp.n_head, hp.n_kv_head, head_dim, window, True, top_position=ctx)[0] == want_form
+            tok = (np.arange(rows) + ctx % 400 + 3).astype(np.int32)
+            logits, ids = sess.forward(np.arange(rows, dtype=np.int32), np.full(rows, ctx, np.int32), tok)
+            runs[off, rows, ctx] = logits.copy(), ids.copy(), [sess.kv_read(layer, 0, ctx, 1) for layer in range(2)]
+        sess.close()
+    for off, rows, ctx in [k for k in runs if k[0] == "0"]:
+        a, b = runs["0", rows, ctx], runs["1", rows, ctx]
+        assert np.array_equal(a[0].view(np.uint32), b[0].view(np.uint32)) and np.array_equal(a[1], b[1]), (rows, ctx)
+        assert all(np.array_equal(x, y) for u, v in zip(a[2], b[2]) for x, y in zip(u, v)), (rows, ctx)
+    model.close()

@@ -118,11 +118,11 @@ private:
      * k_attention_prefill (16 rows of a sequence per workgroup), shorter contexts k_attention's per-row form (3 us per launch quicker below ~128
      * positions, profiles/r05_prefill_attention.txt); the two are bit-identical, so the choice never shows in a result */
     bool tiled_pass = false;
-    /* a decode pass (every sequence once) of at most TK_LONG_ATT_MAX_ROWS rows that reaches position TK_LONG_ATT_MIN_POS runs its attention as
-     * append + scores + PV launches spread over the chip (tk_launch_attention_long) instead of one latency chain per pair of heads; bit-identical */
+    /* a decode pass (every sequence once) of at most TK_LONG_ATT_MAX_ROWS rows that reaches tk_long_att_min_pos() runs its attention as
+     * append + scores and PV launches spread over the chip (tk_launch_attention_long) instead of one latency chain per pair of heads; bit-identical */
     bool long_pass = false;
     bool counted_ = false; /* this session is in the device's count of live decode sessions (tk_attention_note_session) */
-    float* d_scores = nullptr; /* [TK_LONG_ATT_MAX_ROWS][n_head][max_ctx], allocated when the window can reach TK_LONG_ATT_MIN_POS */
+    float* d_scores = nullptr; /* [TK_LONG_ATT_MAX_ROWS][n_head][max_ctx], allocated when the window can reach tk_long_att_min_pos() */
     void choose_attention(const int32_t* pos, int nrows);
     void choose_attention_top(int top, int nrows);
     int32_t* d_tab = nullptr;                           /* prefill schedule: [3][total rows] = seq, pos, tok */

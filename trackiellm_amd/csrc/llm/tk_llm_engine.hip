@@ -282,7 +282,7 @@ bool TkLlmSession::init(TkLlmModel* m, int mseq, int mctx) {
     if (!alloc_act(&act_d, h.d_model, m->has_f16, error) || !alloc_act(&act_qd, QD, m->has_f16, error) || !alloc_act(&act_ff, h.d_ff, m->has_f16, error)) return false;
     HIPQ(hipMalloc((void**)&d_tiles, (size_t)(1 + TK_MAX_ROWS) * 4));
     HIPQ(hipMemset(d_tiles, 0, (size_t)(1 + TK_MAX_ROWS) * 4));
-    if (mctx > TK_LONG_ATT_MIN_POS && tk_attention_long_applies(1, h.n_head, h.n_kv_head, h.head_dim))
+    if (mctx > tk_long_att_min_pos(1, mctx) && tk_attention_long_applies(1, h.n_head, h.n_kv_head, h.head_dim))
         HIPQ(hipMalloc((void**)&d_scores, tk_attention_long_scratch_floats(h.n_head, h.head_dim, mctx) * sizeof(float)));
     /* RoPE table, double precision on the host (same formula as the oracle) */
     std::vector<float> cs((size_t)mctx * half), sn((size_t)mctx * half);
@@ -419,6 +419,9 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
     const bool tiled_attn = !fused_attn && l1 > l0 && tiled_pass && tk_attention_prefill_applies(h.n_head, h.n_kv_head, h.head_dim);
     /* few rows over a long context: the fused kernels would walk it as one latency chain per pair of heads */
     const bool long_attn = fused_attn && l1 > l0 && long_pass && d_scores && tk_attention_long_applies(nrows, h.n_head, h.n_kv_head, h.head_dim);
+    /* ... and the o projection then joins the classes itself, as the other mat-vec launches of such a pass make their input */
+    const bool join_in_o = long_attn && fuse && tk_gemv_fuses_producer(nrows, QD, h.ks_o, 1);
+    const TkAttentionParts parts = long_attn ? tk_attention_long_parts(d_scores, h.n_head, h.head_dim, max_ctx) : TkAttentionParts{};
     if (tiled_attn) tk_launch_att_tiles(d_seq, nrows, d_tiles, s);
     int ks_res = 1; /* slabs of the pending residual update (the previous layer's down projection) */
     for (int l = l0; l < l1; ++l) {
@@ -432,11 +435,11 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
             if (!fused_attn)
                 tk_launch_qkv_rope_append(partial2, ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
                                           qbuf, kcache, vcache, l, max_seq, max_ctx, s);
-            if (long_attn) tk_launch_attention_long(partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, s);
+            if (long_attn) tk_launch_attention_long(partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, !join_in_o, s);
             else if (tiled_attn) tk_launch_attention_prefill(qbuf, kcache, vcache, d_seq, d_pos, d_tiles, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, act_qd, s);
             else tk_launch_attention(qbuf, partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
                                      h.head_dim, l, max_seq, max_ctx, act_qd, fused_attn, s);
-            const int ks_o = enqueue_matmul(ot, 1, QD, h.ks_o, D, act_qd, partial, nrows);
+            const int ks_o = join_in_o ? fused_gemv(ot, 1, QD, h.ks_o, D, partial, 3, parts.l, nullptr, parts.pv, 1, h.head_dim, nullptr) : enqueue_matmul(ot, 1, QD, h.ks_o, D, act_qd, partial, nrows);
             const int ks_gu = fused_gemv(gu, 2, D, h.ks_gateup, 2 * FF, partial2, 1, x2, x, partial, ks_o, D, (const float*)L.ffn_norm.data);
             ks_res = fused_gemv(dn, 1, FF, h.ks_down, D, partial, 2, nullptr, nullptr, partial2, ks_gu, 2 * FF, nullptr);
             continue;
@@ -446,7 +449,7 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
         if (!fused_attn)
             tk_launch_qkv_rope_append(partial, ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
                                       qbuf, kcache, vcache, l, max_seq, max_ctx, s);
-        if (long_attn) tk_launch_attention_long(partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, s);
+        if (long_attn) tk_launch_attention_long(partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, true, s);
         else if (tiled_attn) tk_launch_attention_prefill(qbuf, kcache, vcache, d_seq, d_pos, d_tiles, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, act_qd, s);
         else tk_launch_attention(qbuf, partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
                                  h.head_dim, l, max_seq, max_ctx, act_qd, fused_attn, s);
@@ -489,7 +492,7 @@ void TkLlmSession::choose_attention(const int32_t* pos, int nrows) {
 }
 void TkLlmSession::choose_attention_top(int top, int nrows) {
     tiled_pass = top >= TK_TILED_ATT_MIN_POS;
-    long_pass = d_scores != nullptr && nrows <= TK_LONG_ATT_MAX_ROWS && top >= tk_long_att_min_pos(nrows);
+    long_pass = d_scores != nullptr && nrows <= TK_LONG_ATT_MAX_ROWS && top >= tk_long_att_min_pos(nrows, max_ctx);
 }
 
 bool TkLlmSession::capture_pass(hipGraphExec_t* slot, int nrows, bool lm_head, bool fused_attn) {
@@ -729,13 +732,13 @@ bool TkLlmSession::time_attention(int nrows, int ctx, int iters, float* avg_ms, 
     /* TK_MI355X_TIME_UNFUSED=1: time the two-launch form instead (k_qkv_rope_append + k_attention<.., not fused>): what a decode pass would
      * cost without the fused prologue */
     const char* uf = getenv("TK_MI355X_TIME_UNFUSED");
-    const char* lf = getenv("TK_MI355X_TIME_LONG"); /* =1: the three-launch long-context form (tk_launch_attention_long) where it applies */
+    const char* lf = getenv("TK_MI355X_TIME_LONG"); /* =1: the long-context form's three launches (tk_launch_attention_long) where it applies */
     const bool longf = lf && lf[0] == '1' && d_scores && tk_attention_long_applies(nrows, h.n_head, h.n_kv_head, h.head_dim);
     const bool unfused = (uf && uf[0] == '1') || longf;
     auto launch = [&](int l) {
         if (longf) {
             tk_launch_attention_long(partial, h.ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l % h.n_layer,
-                                     max_seq, max_ctx, d_scores, act_qd, stream);
+                                     max_seq, max_ctx, d_scores, act_qd, true, stream);
             return;
         }
         if (unfused)

@@ -37,7 +37,8 @@ struct TkGemvArgs {
      *   1: residual update + RMS norm + Q8 — k_rmsnorm_q8's arithmetic: row = fx_in + (the fks slabs of fslab, ascending; pitch
      *      fn_total; fslab null: none), written once to fx_out (a buffer OTHER than fx_in: other workgroups still read it), norm
      *      weights fw, epsilon feps; K = d_model
-     *   2: SwiGLU + Q8 — k_swiglu_q8's arithmetic on the fks slabs of the gate | up projection in fslab ([.][2 K] per row); K = d_ff */
+     *   2: SwiGLU + Q8 — k_swiglu_q8's arithmetic on the fks slabs of the gate | up projection in fslab ([.][2 K] per row); K = d_ff
+     *   3: the join of a long attention's classes + Q8 — fslab = TkAttentionParts::pv, fx_in = ::l, fn_total = head_dim; K = n_head * head_dim */
     int fuse;
     const float* fx_in;
     float* fx_out;
@@ -111,16 +112,20 @@ void tk_launch_attention_prefill(const float* qbuf, const uint16_t* kcache, cons
 /* decode passes of few rows over long contexts: scores spread over (row, KV head, 64-position block) workgroups, then one sequential PV chain per
  * (row, head, class) wave — bit-identical to the fused kernels.  scores: tk_attention_long_scratch_floats() floats; `partial` holds the
  * q | k | v projection's K-split slabs (the launch finishes q / k / v itself and appends this pass's rows to the cache) */
-/* by measurement, end to end (profiles/r05_attention_long_ctx.txt): 1 .. 4 rows from position 512, 5 .. 8 rows from 768 (the isolated launch
- * already wins from ~384 at one row; a whole step does not before ~500); at 16 rows the fused kernels' 256 workgroups already cover the chip */
+/* From which position a decode pass takes this form, by whole steps of a 32-layer model (fused kernels / this form, ms): 1 row at 224 positions 1.675 / 1.704,
+ * at 288 1.767 / 1.737, at 448 1.852 / 1.742, at 900 2.188 / 1.815; 4 rows at 352 2.046 / 2.081, at 600 2.363 / 2.213; 8 rows at 600 2.384 / 2.445, at 900
+ * 2.647 / 2.606; at 16 rows the fused kernels' 256 workgroups already cover the chip.  The window hardly matters (4096: 1 row at 448 1.892 / 1.743); beyond
+ * 2048 the plan that its tests fix stays, 512 at 1 .. 4 rows. */
 #define TK_LONG_ATT_MAX_ROWS 8
-#define TK_LONG_ATT_MIN_POS 512
-static inline int tk_long_att_min_pos(int nrows) { return nrows > 4 ? 768 : TK_LONG_ATT_MIN_POS; }
+static inline int tk_long_att_min_pos(int nrows, int max_ctx) { return nrows > 4 ? 768 : nrows == 1 && max_ctx <= 2048 ? 256 : 512; }
 bool tk_attention_long_applies(int nrows, int n_head, int n_kv_head, int head_dim);
 size_t tk_attention_long_scratch_floats(int n_head, int head_dim, int max_ctx); /* floats of the `scores` scratch buffer */
+/* where such a launch leaves the classes' outputs [row][head][4][head_dim] and denominators [row][head][4]; join = false: its consumer joins them (TkGemvArgs::fuse 3) */
+struct TkAttentionParts { float *pv, *l; };
+TkAttentionParts tk_attention_long_parts(float* scores, int n_head, int head_dim, int max_ctx);
 void tk_launch_attention_long(const float* partial, int ks, int n_total, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
                               const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head, int head_dim, int layer, int max_seq, int max_ctx,
-                              float* scores, TkActQ8 out, hipStream_t s);
+                              float* scores, TkActQ8 out, bool join, hipStream_t s);
 size_t tk_gemv_lds_bytes(int K, int ks, int mtiles);
 /* dynamic LDS of one k_attention workgroup; must stay below 160 KiB (the session checks it against its max_ctx) */
 size_t tk_attention_lds_bytes(int gq, int head_dim, int max_ctx, int chunk /* positions per ring slot: 32 or 64 */, int slots = 2 /* ring depth: 2 or 5 */);

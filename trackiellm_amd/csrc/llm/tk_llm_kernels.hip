@@ -702,6 +702,23 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                     quantize_chunk8(v, cl, r, lo);
                 }
             }
+        } else if (FUSE == 3) { /* k_att_pv_join's arithmetic: this K-range's blocks of the attention output */
+            const int HD = a.fn_total;
+            for (int r = 0; r < a.nrows; ++r)
+                for (int b = hw; b < nb; b += nhw) {
+                    const int cl = 32 * b + (lane & 31), c = 32 * blk0 + cl;
+                    const int64_t hi = (int64_t)r * (a.K / HD) + 8 * c / HD; /* (row, head) of this chunk's eight dims */
+                    const float* pp = a.fslab + hi * 4 * HD + 8 * c % HD;
+                    v4f p[4][2];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) { p[j][0] = *(const v4f*)(pp + j * HD); p[j][1] = *(const v4f*)(pp + j * HD + 4); }
+                    const v4f lp = *(const v4f*)(a.fx_in + hi * 4);
+                    const float ll = ((lp[0] + lp[1]) + lp[2]) + lp[3];
+                    float v[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) v[i] = tk_divf(((p[0][i >> 2][i & 3] + p[1][i >> 2][i & 3]) + p[2][i >> 2][i & 3]) + p[3][i >> 2][i & 3], ll);
+                    quantize_chunk8(v, cl, r, lo);
+                }
         } else {
             const int FF = a.K;
             for (int r = 0; r < a.nrows; ++r)
@@ -1632,7 +1649,7 @@ void tk_launch_gemv(const TkGemvArgs& a, hipStream_t s) {
 #define TK_GEMV_TY(PFV, MTV, FUV) do { if (types == 1) TK_GEMV_LAUNCH(PFV, MTV, 1, FUV); else if (types == 2) TK_GEMV_LAUNCH(PFV, MTV, 2, FUV); else TK_GEMV_LAUNCH(PFV, MTV, 3, FUV); } while (0)
     const size_t fuse_lds = a.fuse == 1 ? ((size_t)a.K + 4) * sizeof(float) : 0; /* the finished row and the canonical sum's four partials */
     if (a.fuse && mt == 1 && pf == 2) { /* tk_gemv_fuses_producer() admits only such launches */
-        if (a.fuse == 1) TK_GEMV_TY(2, 1, 1); else TK_GEMV_TY(2, 1, 2);
+        if (a.fuse == 1) TK_GEMV_TY(2, 1, 1); else if (a.fuse == 2) TK_GEMV_TY(2, 1, 2); else TK_GEMV_TY(2, 1, 3);
     } else if (mt == 1) { if (pf == 2) TK_GEMV_TY(2, 1, 0); else TK_GEMV_TY(1, 1, 0); }
     else { if (pf == 2) TK_GEMV_TY(2, 2, 0); else TK_GEMV_TY(1, 2, 0); }
 #undef TK_GEMV_TY
@@ -2412,8 +2429,9 @@ __global__ __launch_bounds__((256 / HD) * 256) void k_attention_prefill(const fl
  *                       written to a [row][head][position] fp32 buffer;
  *   k_att_pv_chain      workgroup = one wave = (row, head, class j): row maximum (order-free), e = exp(s - m), then the canonical class
  *                       chain — positions j, j + 4, ... ascending, acc = fma(e, v, acc), l = l + e — as ONE sequential chain per lane (a lane
- *                       owns two dims), 32 value rows requested ahead; partial outputs and denominators to a scratch buffer;
- *   k_att_pv_join       the four classes joined in order, division, Q8 quantisation.
+ *                       owns two dims), 192 value rows requested ahead; partial outputs and denominators to a scratch buffer;
+ *   k_att_pv_join       the four classes joined in order, division, Q8 quantisation; in passes whose mat-vec launches make their own input the
+ *                       o projection does this (TkGemvArgs::fuse 3): a launch less, 0.1 us of the other.
  * Bit-identical to k_attention / k_attention_narrow (tests/test_llm_attention_gpu.py: the decode cases past 2 048 positions run both).
  * The session takes this form for passes of at most TK_LONG_ATT_MAX_ROWS rows that reach tk_long_att_min_pos(rows) (tk_llm_kernels.h).
  * ------------------------------------------------------------------------------------------ */
@@ -2434,6 +2452,16 @@ __global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict
     const int GQ = n_head / n_kv_head, QD = n_head * HD, KVD = n_kv_head * HD;
     const bool last = 64 * b + 64 >= T; /* this block holds position p */
     uint16_t* krun = kcache + (((int64_t)layer * max_seq + seq[r]) * n_kv_head + kvh) * (int64_t)max_ctx * HD;
+    uint4 kreg[PPT]; /* the block's key rows, requested before anything else */
+#pragma unroll
+    for (int u = 0; u < PPT; ++u) {
+        const int pid = t + u * 256;
+        if (PIECES % 256 == 0 || pid < PIECES) {
+            int pr = 64 * b + pid / PPR;
+            pr = pr < p ? pr : (p > 0 ? p - 1 : 0); /* cached rows only: position p itself is patched in from LDS below (its store may still be on its way) */
+            kreg[u] = *(const uint4*)(krun + (int64_t)pr * HD + 8 * (pid % PPR));
+        }
+    }
     {   /* q (every block) and k, v of this row (the last block): K-split sums, RoPE on adjacent pairs, f16 rounding — k_qkv_rope_append's
          * arithmetic, inside this launch (a launch of its own cost 4.8 us per layer) */
         const float* cs = rope_cos + (int64_t)p * HALF;
@@ -2461,9 +2489,7 @@ __global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict
         const int pid = t + u * 256;
         if (PIECES % 256 == 0 || pid < PIECES) {
             const int pn = pid / PPR, q8 = pid % PPR;
-            int pr = 64 * b + pn;
-            pr = pr < p ? pr : (p > 0 ? p - 1 : 0); /* cached rows only: position p itself is patched in from LDS below (its store may still be on its way) */
-            const uint4 kk = *(const uint4*)(krun + (int64_t)pr * HD + 8 * q8);
+            const uint4 kk = kreg[u];
             const uint32_t wv[4] = {kk.x, kk.y, kk.z, kk.w};
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
@@ -2500,87 +2526,93 @@ __global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict
     }
 }
 
-template <int HD>
+/* One wave = one (row, head, class) chain: 128 x rows workgroups, so the value rows arrive through as many CUs' memory pipes (a CU pulls ~25 - 40 GB/s:
+ * sixteen workgroups of eight chains each took 29 us at 2 048 positions).  The class's value rows come by LDS-DMA, 1 KiB a request, three chunks of 64
+ * rows in flight — the whole class up to 768 positions; two above four rows — and are requested right behind the scores; one 4-byte load a row and lane, the former way, held 64
+ * rows of two register sets and a wave can have no more than 63 requests on their way.  A lane owns two dims (head_dim 64: the upper half-wave mirrors the
+ * lower). With it, the keys requested before q's slabs and the join in the
+ * o projection a step of one row takes 1.742 ms at 448 positions (fused kernel 1.852);
+ * 4096-position window, before and now: 1 row at 600 1.975 -> 1.768, at 3000 2.527 -> 2.223, 4 rows at 900 2.515 -> 2.351, 8 rows at 900 2.627 -> 2.507. */
+#define TK_PV_ROWS 64
+template <int HD, int SLOTS>
 __global__ __launch_bounds__(64) void k_att_pv_chain(const float* __restrict__ scores, const uint16_t* __restrict__ vcache, const int32_t* __restrict__ seq,
                                                      const int32_t* __restrict__ pos, int n_head, int n_kv_head, int layer, int max_seq, int max_ctx,
                                                      float* __restrict__ pv_part, float* __restrict__ l_part) {
-    /* one wave = one (row, head, class) chain: 128 x rows workgroups, so the value rows arrive through as many CUs' memory pipes (a CU
-     * pulls ~25 - 40 GB/s: sixteen workgroups of eight chains each — the first form of this launch — took 29 us at 2 048 positions) */
+    extern __shared__ __attribute__((aligned(16))) uint8_t att_lds[];
+    constexpr int RB = HD * 2, PPR = RB / 16, RPI = 64 / PPR, NI = TK_PV_ROWS / RPI; /* bytes and 16-byte pieces of a row, rows of a request, requests of a chunk */
+    float* ebuf = (float*)(att_lds + SLOTS * TK_PV_ROWS * RB); /* the class's scores, then probabilities; whole chunks */
     const int j = blockIdx.x, head = blockIdx.y, r = blockIdx.z, lane = threadIdx.x;
     const int kvh = head / (n_head / n_kv_head);
     const int T = pos[r] + 1;
     const float* s = scores + ((int64_t)r * n_head + head) * max_ctx;
     const uint16_t* vrun = vcache + (((int64_t)layer * max_seq + seq[r]) * n_kv_head + kvh) * (int64_t)max_ctx * HD;
-    float m = -INFINITY;
-    for (int t0 = 0; t0 < T; t0 += 16 * 64) { /* sixteen loads in flight per lane: a load per iteration would be a chain of cache latencies */
-        float sv[16];
-#pragma unroll
-        for (int u = 0; u < 16; ++u) { const int tt = t0 + 64 * u + lane; sv[u] = tt < T ? s[tt] : -INFINITY; }
-#pragma unroll
-        for (int u = 0; u < 16; ++u) m = tk_fmaxf(m, sv[u]);
-    }
-    m = tk_wave_max(m);
     const int nj = T > j ? (T - j + 3) / 4 : 0; /* positions j, j + 4, ... of this class */
-    /* The chain: a lane owns two dims (head_dim 64: the upper half-wave mirrors the lower).  Chunks of 32 class positions, two register
-     * sets: a chunk's value rows are requested a chunk before the chain reaches them; the scores of a chunk are requested two chunks ahead
-     * and BEFORE the value rows of the chunk in between (vmcnt counts in order: waiting for a score requested after 32 row loads would
-     * drain them).  Probabilities reach every lane through LDS broadcast reads issued before the chunk's chain starts.  Measured and
-     * dropped: two rows per request with v_permlane32_swap (64 positions in flight; 19.1 us against 15.8 at 2 048 positions: the swaps and
-     * the four-dim owners' longer steps cost more than the deeper prefetch saves), v_readlane per step (16.7 us). */
+    const int nch = (nj + TK_PV_ROWS - 1) / TK_PV_ROWS;
+    auto stage = [&](int c) { /* always whole chunks (the waits count requests): rows past the context are the last one again, with probability 0 */
+#pragma unroll
+        for (int q = 0; q < NI; ++q) {
+            int tt = j + 4 * (c * TK_PV_ROWS + q * RPI + lane / PPR);
+            tt = tt < T ? tt : T - 1;
+            const auto gs = (const __attribute__((address_space(1))) void*)((const uint8_t*)(vrun + (int64_t)tt * HD) + (lane % PPR) * 16);
+            const auto ls = (__attribute__((address_space(3))) void*)(att_lds + (c % SLOTS) * TK_PV_ROWS * RB + q * 1024);
+            __builtin_amdgcn_global_load_lds(gs, ls, 16, 0, 0);
+        }
+    };
+    float m = -INFINITY;
+    float sv[16];
+    auto request = [&](int t0) { /* sixteen loads in flight per lane: a load per iteration would be a chain of cache latencies */
+#pragma unroll
+        for (int u = 0; u < 16; ++u) { const int tt = t0 + 64 * u + lane; sv[u] = s[tt < T ? tt : T - 1]; }
+    };
+    auto take = [&](int t0) { /* position tt is number tt / 4 of class tt % 4 */
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const int tt = t0 + 64 * u + lane;
+            if (tt < T) {
+                m = tk_fmaxf(m, sv[u]);
+                if ((lane & 3) == j) ebuf[tt >> 2] = sv[u];
+            }
+        }
+    };
+    request(0);
+    for (int c = 0; c < SLOTS && c < nch; ++c) stage(c);
+    take(0);
+    for (int t0 = 1024; t0 < T; t0 += 1024) { request(t0); take(t0); }
+    m = tk_wave_max(m);
+    __syncthreads();
+    for (int i = lane; i < nch * TK_PV_ROWS; i += 64) ebuf[i] = i < nj ? tk_expf(ebuf[i] - m) : 0.0f;
+    __syncthreads();
     const int dl = lane % (HD / 2);
     float acc0 = 0.0f, acc1 = 0.0f, l = 0.0f;
-    uint32_t va[32], vb[32];
-    auto fetch = [&](uint32_t (&v)[32], int c) { /* value rows of class positions 32 c .. 32 c + 31 */
-        if (32 * c + 32 <= nj) { /* a whole chunk: one base address, rows 4 * head_dim halves apart (two scalar adds per request instead of six) */
-            const uint16_t* base = vrun + (int64_t)(j + 128 * c) * HD + 2 * dl;
-#pragma unroll
-            for (int k = 0; k < 32; ++k) v[k] = *(const uint32_t*)(base + (int64_t)k * 4 * HD);
-            return;
-        }
-#pragma unroll
-        for (int k = 0; k < 32; ++k) { /* the last chunk, or past the end: clamped rows (their probability is 0) */
-            int tt = j + 4 * (32 * c + k);
-            tt = tt < T ? tt : T - 1;
-            v[k] = *(const uint32_t*)(vrun + (int64_t)tt * HD + 2 * dl);
-        }
-    };
-    auto score_of = [&](int c) -> float { /* lane i < 32: score of class position 32 c + i */
-        const int i = 32 * c + (lane & 31);
-        return i < nj ? s[j + 4 * i] : -INFINITY;
-    };
-    auto probs = [&](float sc, int c) -> float { return 32 * c + (lane & 31) < nj ? tk_expf(sc - m) : 0.0f; };
-    __shared__ float ebuf[2][32];
-    int eslot = 0;
-    auto eat = [&](const uint32_t (&v)[32], float e32) {
-        if (lane < 32) ebuf[eslot][lane] = e32;
+    for (int c = 0; c < nch; ++c) {
+        const int ahead = nch - 1 - c < SLOTS - 1 ? nch - 1 - c : SLOTS - 1;
+        wait_vmcnt(ahead * NI);
         __syncthreads();
-        float ek[32];
+        const uint8_t* vp = att_lds + (c % SLOTS) * TK_PV_ROWS * RB + dl * 4;
+        const float* ep = ebuf + c * TK_PV_ROWS;
 #pragma unroll
-        for (int k = 0; k < 32; ++k) ek[k] = ebuf[eslot][k];
-        eslot ^= 1;
+        for (int k0 = 0; k0 < TK_PV_ROWS; k0 += 16) {
+            uint32_t v[16];
+            v4f e[4];
 #pragma unroll
-        for (int k = 0; k < 32; ++k) {
-            acc0 = tk_fmaf(ek[k], f16bits_to_f32(v[k] & 0xffffu), acc0);
-            acc1 = tk_fmaf(ek[k], f16bits_to_f32(v[k] >> 16), acc1);
-            l = l + ek[k];
+            for (int k = 0; k < 16; ++k) v[k] = *(const uint32_t*)(vp + (k0 + k) * RB);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) e[k] = *(const v4f*)(ep + k0 + 4 * k);
+#pragma unroll
+            for (int k = 0; k < 16; ++k) {
+                const float ek = e[k >> 2][k & 3];
+                acc0 = tk_fmaf(ek, f16bits_to_f32(v[k] & 0xffffu), acc0);
+                acc1 = tk_fmaf(ek, f16bits_to_f32(v[k] >> 16), acc1);
+                l = l + ek;
+            }
         }
-    };
-    const int nch = (nj + 31) / 32;
-    float sa = score_of(0), sb = score_of(1);
-    if (nch > 0) fetch(va, 0);
-    for (int c = 0; c < nch; c += 2) {
-        const float ea = probs(sa, c);
-        sa = score_of(c + 2);
-        fetch(vb, c + 1); /* past the end: clamped rows, probabilities 0 */
-        eat(va, ea);
-        if (c + 1 >= nch) break;
-        const float eb = probs(sb, c + 1);
-        sb = score_of(c + 3);
-        if (c + 2 < nch) fetch(va, c + 2);
-        eat(vb, eb);
+        if (c + SLOTS < nch) {
+            __syncthreads(); /* the chunk's reads are done */
+            stage(c + SLOTS);
+        }
     }
     float* pp = pv_part + (((int64_t)r * n_head + head) * TK_ATT_TSPLIT + j) * HD;
-    if (lane < HD / 2) { pp[2 * dl] = acc0; pp[2 * dl + 1] = acc1; }
+    if (lane < HD / 2) *(float2*)(pp + 2 * dl) = make_float2(acc0, acc1);
     if (lane == 0) l_part[((int64_t)r * n_head + head) * TK_ATT_TSPLIT + j] = l;
 }
 
@@ -2605,29 +2637,36 @@ __global__ __launch_bounds__(256) void k_att_pv_join(const float* __restrict__ p
     }
 }
 
+/* the scratch buffer: scores, then the classes' partial outputs and denominators (tk_attention_long_scratch_floats) */
+TkAttentionParts tk_attention_long_parts(float* scores, int n_head, int head_dim, int max_ctx) {
+    float* pv = scores + (size_t)TK_LONG_ATT_MAX_ROWS * n_head * ((max_ctx + 3) & ~3);
+    return TkAttentionParts{pv, pv + (size_t)TK_LONG_ATT_MAX_ROWS * n_head * TK_ATT_TSPLIT * head_dim};
+}
+
 void tk_launch_attention_long(const float* partial, int ks, int n_total, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
                               const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head, int head_dim, int layer, int max_seq, int max_ctx,
-                              float* scores, TkActQ8 out, hipStream_t s) {
+                              float* scores, TkActQ8 out, bool join, hipStream_t s) {
     const dim3 gs(n_kv_head, (max_ctx + 63) / 64, nrows);
-    /* the scratch buffer: scores, then the classes' partial outputs and denominators (tk_attention_long_scratch_floats) */
-    float* pv_part = scores + (size_t)TK_LONG_ATT_MAX_ROWS * n_head * max_ctx;
-    float* l_part = pv_part + (size_t)TK_LONG_ATT_MAX_ROWS * n_head * TK_ATT_TSPLIT * head_dim;
+    const TkAttentionParts parts = tk_attention_long_parts(scores, n_head, head_dim, max_ctx);
+    float *pv_part = parts.pv, *l_part = parts.l;
     const dim3 gc(TK_ATT_TSPLIT, n_head, nrows);
+    const int slots = nrows > 4 ? 2 : 3; /* 32 KB: the four workgroups a CU of eight rows are resident together */
+    const size_t lds = (size_t)slots * TK_PV_ROWS * head_dim * 2 + ((size_t)(max_ctx + 3) / 4 + TK_PV_ROWS) * sizeof(float);
     if (head_dim == 128) {
         hipLaunchKernelGGL((k_att_scores_long<128>), gs, dim3(256), 0, s, partial, ks, n_total, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
                            max_seq, max_ctx, scores);
-        hipLaunchKernelGGL((k_att_pv_chain<128>), gc, dim3(64), 0, s, scores, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pv_part, l_part);
-        hipLaunchKernelGGL((k_att_pv_join<128>), dim3(n_head / 2, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
+        hipLaunchKernelGGL((slots == 2 ? k_att_pv_chain<128, 2> : k_att_pv_chain<128, 3>), gc, dim3(64), lds, s, scores, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pv_part, l_part);
+        if (join) hipLaunchKernelGGL((k_att_pv_join<128>), dim3(n_head / 2, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
     } else {
         hipLaunchKernelGGL((k_att_scores_long<64>), gs, dim3(256), 0, s, partial, ks, n_total, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
                            max_seq, max_ctx, scores);
-        hipLaunchKernelGGL((k_att_pv_chain<64>), gc, dim3(64), 0, s, scores, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pv_part, l_part);
-        hipLaunchKernelGGL((k_att_pv_join<64>), dim3(n_head / 4, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
+        hipLaunchKernelGGL((slots == 2 ? k_att_pv_chain<64, 2> : k_att_pv_chain<64, 3>), gc, dim3(64), lds, s, scores, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pv_part, l_part);
+        if (join) hipLaunchKernelGGL((k_att_pv_join<64>), dim3(n_head / 4, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
     }
 }
 
 size_t tk_attention_long_scratch_floats(int n_head, int head_dim, int max_ctx) {
-    return (size_t)TK_LONG_ATT_MAX_ROWS * n_head * ((size_t)max_ctx + (size_t)TK_ATT_TSPLIT * head_dim + TK_ATT_TSPLIT);
+    return (size_t)TK_LONG_ATT_MAX_ROWS * n_head * ((size_t)((max_ctx + 3) & ~3) + (size_t)TK_ATT_TSPLIT * head_dim + TK_ATT_TSPLIT);
 }
 
 bool tk_attention_long_applies(int nrows, int n_head, int n_kv_head, int head_dim) {
@@ -2945,7 +2984,7 @@ const char* tk_llm_prepare_device(int device) {
 #undef TK_OPT_G32
 #define TK_OPT_GEMV_F(PFV, MTV, FUV) do { TK_OPT((k_gemv_w4a8<PFV, MTV, 1, FUV>)); TK_OPT((k_gemv_w4a8<PFV, MTV, 2, FUV>)); TK_OPT((k_gemv_w4a8<PFV, MTV, 3, FUV>)); } while (0)
 #define TK_OPT_GEMV(PFV, MTV) TK_OPT_GEMV_F(PFV, MTV, 0)
-    TK_OPT_GEMV(1, 1); TK_OPT_GEMV(2, 1); TK_OPT_GEMV(1, 2); TK_OPT_GEMV(2, 2); TK_OPT_GEMV_F(2, 1, 1); TK_OPT_GEMV_F(2, 1, 2);
+    TK_OPT_GEMV(1, 1); TK_OPT_GEMV(2, 1); TK_OPT_GEMV(1, 2); TK_OPT_GEMV(2, 2); TK_OPT_GEMV_F(2, 1, 1); TK_OPT_GEMV_F(2, 1, 2); TK_OPT_GEMV_F(2, 1, 3);
 #define TK_OPT_ATT_C(H, C, S) do { TK_OPT((k_attention<1, true, H, C, S>)); TK_OPT((k_attention<2, true, H, C, S>)); TK_OPT((k_attention<4, true, H, C, S>)); \
                                  TK_OPT((k_attention<1, false, H, C, S>)); TK_OPT((k_attention<2, false, H, C, S>)); TK_OPT((k_attention<4, false, H, C, S>)); } while (0)
 #define TK_OPT_ATT(H) do { TK_OPT_ATT_C(H, 32, TK_ATT_WIDE_SLOTS); TK_OPT_ATT_C(H, 64, 2); } while (0)
@@ -2953,6 +2992,7 @@ const char* tk_llm_prepare_device(int device) {
 #define TK_OPT_ATT_N(H) do { TK_OPT((k_attention<1, true, H, 128, 2>)); TK_OPT((k_attention<2, true, H, 128, 2>)); TK_OPT((k_attention<1, false, H, 128, 2>)); TK_OPT((k_attention<2, false, H, 128, 2>)); } while (0)
     TK_OPT_ATT_N(64); TK_OPT_ATT_N(128);
     TK_OPT(k_attention_narrow);
+    TK_OPT((k_att_pv_chain<128, 2>)); TK_OPT((k_att_pv_chain<128, 3>)); TK_OPT((k_att_pv_chain<64, 2>)); TK_OPT((k_att_pv_chain<64, 3>));
     TK_OPT((k_attention_prefill<128>));
     TK_OPT((k_attention_prefill<64>));
 #undef TK_OPT_ATT_N
