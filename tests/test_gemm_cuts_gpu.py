@@ -29,6 +29,38 @@ def test_wide_tiles_equal_staged(gpu, M, N, K, act, res):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 8704, 128), (63, 8736, 384), (64, 9216, 256), (65, 5824, 1024), (96, 5856, 640), (127, 4384, 128), (129, 3520, 512),
+                                   (161, 17472, 256), (255, 16384, 256), (256, 20480, 128), (300, 2048, 128)])
+def test_wide_tiles_of_f16_weights_equal_staged(gpu, M, N, K):
+    """from 33 rows on, in both forms: last tiles of 1 .. 64 rows, one to eight requests of 128 k"""
+    rng = np.random.default_rng(M + N + K)
+    a, w = rng.normal(0, 1, (M, K)).astype(np.float32), (rng.normal(0, 1, (N, K)) * K ** -0.5).astype(np.float32)
+    cs, ct = np.empty((M, N), np.float32), np.empty((M, N), np.float32)
+    p = lambda x: x.ctypes.data_as(C.c_void_p)
+    gpu.check(gpu.lib().tk_mi355x_gemm_pair(0, M, N, K, p(a), p(w), None, None, 0, 1, p(cs), p(ct)))
+    assert np.array_equal(cs.view(np.uint32), ct.view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_wide_tiles_in_parts_of_k(gpu):
+    """a layer of f16 weights (q | k | v, o and down in 4, 4 and 7 parts of k): a position's logits do not depend on how many rows its pass has, whether up
+    to 32 (the LDS ring) or more"""
+    hp = gpu.MISTRAL_7B()
+    hp.n_layer = 1
+    model = gpu.LlmModel(hp).fill_synthetic(4, f16=True)
+    rng = np.random.default_rng(2)
+    n = 256
+    seq, pos, tok = np.arange(n, dtype=np.int32), np.zeros(n, np.int32), rng.integers(3, hp.vocab, n).astype(np.int32)
+    sess = gpu.LlmSession(model, n, 4)
+    want = np.concatenate([sess.forward(seq[i:i + 32], pos[i:i + 32], tok[i:i + 32])[0].copy() for i in range(0, n, 32)])
+    for rows in (33, 64, 65, 97, 128, 160, 255, 256):
+        got, _ = sess.forward(seq[:rows], pos[:rows], tok[:rows])
+        assert np.array_equal(got.view(np.uint32), want[:rows].view(np.uint32)), rows
+    sess.close()
+    model.close()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("ctx,width", [(100, 1024), (33, 1280), (97, 384)])
 def test_wide_tiles_and_images_in_an_encoder(gpu, ctx, width):
     """a clip's encoder states do not depend on how many clips run with it: from 20 on its layers, and the images between them, are made in wide tiles"""

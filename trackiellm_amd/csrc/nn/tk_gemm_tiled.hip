@@ -9,6 +9,7 @@
 
 #include "../common/tk_exact_math.h"
 
+typedef _Float16 tw_v8h __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef unsigned v4u __attribute__((ext_vector_type(4)));
@@ -316,22 +317,29 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
  * h = l / 32 holds groups g = h and 2 + h of the image and of the weight tiles, a float4 each.  An operand float4 feeds 4 MI or 4 NI MFMAs of 64 cycles, where the ring
  * kernel above reads LDS once for 4 of 32: fp32 MFMAs and LDS reads take turns on a SIMD.
  * Images are made with the operands exchanged: a lane then holds one row, and lanes l, l + 32 swap halves so that each stores the 16 bytes of a group.
+ * f16 weights (K-split parts side by side, the rows of a tile column in one workgroup) are converted in front of each product, on its pipe: 256 rows x 4096 x 28672 533 ->
+ * 491 us (393), 136 rows of a 4096-wide layer 1.20 -> 0.77 ms.
  * Form <1, 1> has the smaller tiles, and so more of them; form <2, 1> reads a third less, which counts for matrices that the L2 does not hold (tk_gemm_tiled_plan).
  * 48 000 rows, ring -> here, us (the fp32 MFMAs alone): 384 x 384 183 -> 139 (93), 1152 x 384 475 -> 346 (278), 1536 x 384 with GELU 610 -> 469 (370), 384 x 1536 560 -> 513
  * (370); 1500 rows: 23.2 -> 17.6, 31.6 -> 25.2 and 38.2 -> 30.4 of the last three.  What is left is the last round of tiles and the first requests of each.
  */
-template <int MI, int NI, int KS, int PF>
-__global__ __launch_bounds__(256, MI * NI == 4 ? 3 : MI * NI == 2 ? 4 : 5) void k_gemm_wide(TkTiledGemm a, int ncol /* tiles of 32 NI columns */, int total /* waves' tiles */, int per_xcd) {
-    constexpr int V = KS / 8; /* float4 per 32 rows and stage */
+template <int WB, int MI, int NI, int KS, int PF>
+__global__ __launch_bounds__(256, MI * NI == 2 || PF > 2 ? 4 : 5) void k_gemm_wide(TkTiledGemm a, int ncol /* tiles of 32 NI columns */, int nrow /* tiles of 32 MI rows */, int total /* waves' tiles */,
+                                                                                  int per_xcd) {
+    constexpr int V = KS / 8;               /* float4 per 32 rows and stage */
+    constexpr int WV = WB == 4 ? V : V / 2; /* 16-byte pieces of weights per 32 columns and stage */
     /* consecutive workgroups go to different XCDs: each takes a run of them, whose rows stay in its L2 */
     const int wg = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     const int lane = threadIdx.x & 63, id = wg * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (id >= total) return;
     const int h = lane >> 5, l32 = lane & 31, l16 = lane & 15, up = (lane >> 4) & 1;
-    const int blk = id / ncol, row0 = blk * 32 * MI;
-    int rt = (id - blk * ncol) * 2 * NI, seg = 0, col_base = 0;
+    /* f32: the columns of a tile row by row (the weights are small and stay); f16: the rows of a tile column side by side, so that a workgroup's waves share their
+     * weights, then the columns, then the parts of k */
+    const int blk = WB == 4 ? id / ncol : id % nrow, row0 = blk * 32 * MI;
+    const int colk = id / nrow, ksi = WB == 4 ? 0 : colk / ncol;
+    int rt = (WB == 4 ? id - blk * ncol : colk - ksi * ncol) * 2 * NI, seg = 0, col_base = 0;
     while (seg < a.nseg - 1 && rt >= a.row_tiles[seg]) { rt -= a.row_tiles[seg]; col_base += a.row_tiles[seg] * TK_TW_ROWS_PER_TILE; ++seg; }
-    const unsigned a_pitch = (unsigned)a.a_ts * 4u, w_pitch = (unsigned)a.K * 64u; /* bytes of 16 rows */
+    const unsigned a_pitch = (unsigned)a.a_ts * 4u, w_pitch = (unsigned)a.K * 16u * WB; /* bytes of 16 rows */
     const int tiles_here = (a.nrows - row0 + 15) / 16;
     const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void*)(a.a_img + (size_t)(row0 / 16) * a.a_ts), 0, (unsigned)(tiles_here < 2 * MI ? tiles_here : 2 * MI) * a_pitch, 0x00020000);
     const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.tiles[seg] + (size_t)rt * w_pitch), 0, 2u * NI * w_pitch, 0x00020000);
@@ -342,19 +350,22 @@ __global__ __launch_bounds__(256, MI * NI == 4 ? 3 : MI * NI == 2 ? 4 : 5) void 
         a_at[i] = (unsigned)(tile < tiles_here ? tile : tiles_here - 1) * a_pitch + (unsigned)(h * 256 + l16 * 16);
     }
 #pragma unroll
-    for (int i = 0; i < NI; ++i) w_at[i] = (unsigned)(2 * i + up) * w_pitch + (unsigned)((h * 16 + l16) * 32);
+    for (int i = 0; i < NI; ++i) w_at[i] = (unsigned)(2 * i + up) * w_pitch + (unsigned)((h * 16 + l16) * 8 * WB);
 
-    v4f aq[PF][MI][V], wq[PF][NI][V];
-    const int ns = a.K / KS;
-    auto load = [&](int s, v4f (*av)[V], v4f (*wv)[V]) {
-        s = s < ns ? s : ns - 1;
+    v4f aq[PF][MI][V], wq[PF][NI][WV];
+    const int ns = (WB == 4 ? a.K : a.K / a.ks) / KS, s0 = ksi * ns;
+    auto load = [&](int s, v4f (*av)[V], v4f (*wv)[WV]) {
+        s = s0 + (s < ns ? s : ns - 1);
 #pragma unroll
         for (int v = 0; v < V; ++v) { /* 16-k group v / 2 of the stage, half v % 2 of its groups */
             const unsigned j = (unsigned)(s * (KS / 16) + v / 2);
 #pragma unroll
             for (int i = 0; i < MI; ++i) av[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(ar, a_at[i] + (v & 1) * 512, j * 1024, 0));
 #pragma unroll
-            for (int i = 0; i < NI; ++i) wv[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at[i] + (v & 1) * 1024, (j >> 1) * 2048 + (j & 1) * 16, 0));
+            for (int i = 0; i < NI; ++i) {
+                if (WB == 4) wv[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at[i] + (v & 1) * 1024, (j >> 1) * 2048 + (j & 1) * 16, 0));
+                else if (v % 4 < 2) wv[i][v / 4 * 2 + v % 2] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at[i] + (v & 1) * 512, (j >> 1) * 1024, 0));
+            }
         }
     };
     v16f acc[MI][NI];
@@ -383,13 +394,16 @@ __global__ __launch_bounds__(256, MI * NI == 4 ? 3 : MI * NI == 2 ? 4 : 5) void 
                             for (int i = 0; i < MI; ++i)
 #pragma unroll
                                 for (int n = 0; n < NI; ++n) {
-                                    const float x = aq[u][i][v + b][t], w = wq[u][n][v + b][t];
+                                    const float x = aq[u][i][v + b][t];
+                                    float w;
+                                    if (WB == 4) w = wq[u][n][WB == 4 ? v + b : 0][t];
+                                    else w = (float)__builtin_bit_cast(tw_v8h, wq[u][n][v / 4 * 2 + b])[4 * (v / 2 % 2) + t]; /* a piece: t of both 16-k groups */
                                     acc[i][n] = swapped.value ? __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, acc[i][n], 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, acc[i][n], 0, 0, 0);
                                 }
                 /* the requests spread over the products: in front of them they hold these up, behind them (where the compiler puts them) they come late */
 #pragma unroll
-                for (int i = 0; i < (MI + NI) * V; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, MI * NI * V * 4 / ((MI + NI) * V), 0);
+                for (int i = 0; i < MI * V + NI * WV; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, MI * NI * V * 4 / (MI * V + NI * WV), 0);
                     __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -400,7 +414,7 @@ __global__ __launch_bounds__(256, MI * NI == 4 ? 3 : MI * NI == 2 ? 4 : 5) void 
     const float* bias = a.per_seg ? a.seg_bias[seg] : a.bias;
     if (bias && !a.per_seg) bias += col_base;
     const bool add_bias = bias || a.add_zero_bias;
-    if (image) {
+    if (WB == 4 && image) {
         products(std::true_type{});
         float* img = a.per_seg ? a.seg_out[seg] : a.c_img;
         const int cols = a.per_seg ? a.seg_n[seg] : a.n_valid, c0 = a.per_seg ? col0 : col_base + col0;
@@ -435,7 +449,7 @@ __global__ __launch_bounds__(256, MI * NI == 4 ? 3 : MI * NI == 2 ? 4 : 5) void 
         return;
     }
     products(std::false_type{});
-    float* out = a.per_seg ? a.seg_out[seg] + col0 : a.out + col_base + col0;
+    float* out = a.per_seg ? a.seg_out[seg] + col0 : a.out + (WB == 2 ? (size_t)ksi * a.slab_rows * a.ldc : 0) + col_base + col0;
     const int ldc = a.per_seg ? a.seg_ldc[seg] : a.ldc;
     const float* res = a.residual ? a.residual + col_base + col0 : nullptr;
 #pragma unroll
@@ -616,7 +630,16 @@ bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p)
     /* Many rows: tiles of 32 x 32 without LDS, from 544 of them on (a chip has 1024 SIMDs).  Ring / wide time, 22 matrices at 260 .. 2000 rows: up to 384 tiles 0.4 .. 0.9
      * (1152 x 384 1.2), 432 .. 576 0.8 .. 1.3, from 640 on 1.1 .. 1.6.  Form 2 where the weights are more than an XCD's L2 holds and there are tiles to spare: 5120 x 1280
      * at 1500 and 12 000 rows 203 -> 179 and 1395 -> 1150 us; 512 rows 74 -> 86, 1536 x 384 at 48 000 rows 469 -> 485. */
-    if (a.nrows > TK_TW_MAX_BLOCK_ROWS) {
+    /* f16 weights, from 33 rows on: ring / wide time of a 4096-wide layer (6144, 4096, 28672 and 4096 columns in 4, 4, 1 and 7 parts of k): 40 rows 1.01, 64 1.02, 96 1.30,
+     * 128 1.07, 136 1.55, 192 1.35, 256 1.14; at 24 and 32 rows 0.93 and 0.90.  Form 2 does a step of its 64 rows in 0.96 of the time that two tiles of form 1 take, but has
+     * half as many tiles to spread: 256 rows x 4096, 6144, 28672 columns 72.7, 105.5, 530 us against 76.8, 109.1, 491. */
+    if (a.wbytes == 2 && a.nrows > 2 * TK_TW_ROWS_PER_TILE) {
+        const int64_t cols = (int64_t)(tw_row_tiles(a) / 2) * a.ks, simds = 4 * (int64_t)tk_tiled_num_cu();
+        const int64_t one = (a.nrows + 31) / 32 * cols, two = (a.nrows + 63) / 64 * cols;
+        const int form = 1.92f * (float)((two + simds - 1) / simds) < (float)((one + simds - 1) / simds) ? 2 : 1;
+        if (one >= 544 && tk_gemm_wide_plan(a, form, p)) return true;
+    }
+    if (a.wbytes == 4 && a.nrows > TK_TW_MAX_BLOCK_ROWS) {
         const int64_t tiles = (int64_t)((a.nrows + 31) / 32) * (tw_row_tiles(a) / 2);
         const bool large = (size_t)tw_row_tiles(a) * 16 * (size_t)a.K * 4 > (4u << 20);
         if (tiles >= 544 && tk_gemm_wide_plan(a, large && tiles >= 3840 ? 2 : 1, p)) return true;
@@ -676,7 +699,7 @@ static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
 /* the cut of k_gemm_wide's form 1 (32 x 32 of the output a wave) or 2 (64 x 32); false: not a product it takes */
 bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p) {
     static const struct { int mi, ni; } forms[] = {{0, 0}, {1, 1}, {2, 1}};
-    if (!tw_valid(a) || form < 1 || form > 2 || a.wbytes != 4 || a.ks != 1 || a.ln_x || (a.c_img && (a.out || a.residual)) || a.K % 128) return false;
+    if (!tw_valid(a) || form < 1 || form > 2 || (a.wbytes == 4 && a.ks != 1) || a.ln_x || (a.c_img && (a.wbytes == 2 || a.out || a.residual)) || a.K % (128 * a.ks)) return false;
     const int per = 2 * forms[form].ni;
     for (int i = 0; i < a.nseg; ++i)
         if (a.row_tiles[i] % per || (a.per_seg && a.seg_n[i] != a.row_tiles[i] * 16)) return false;
@@ -685,16 +708,21 @@ bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p) {
     p->wide = form;
     p->groups = tw_row_tiles(a) / per;
     p->ny = (a.nrows + 32 * forms[form].mi - 1) / (32 * forms[form].mi);
-    return (int64_t)p->groups * p->ny < 0x7fffff00;
+    return (int64_t)p->groups * p->ny * a.ks < 0x7fffff00;
 }
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipStream_t s) {
     if (p.wide) {
         TkTiledPlan w; /* (the cut follows from the form) */
         if (!tk_gemm_wide_plan(a, p.wide, &w)) return false;
-        const int total = w.groups * w.ny, per = ((total + 3) / 4 + 7) / 8;
+        const int total = w.groups * w.ny * a.ks, per = ((total + 3) / 4 + 7) / 8;
         const dim3 wgrid((unsigned)per * 8);
-        if (p.wide == 1) hipLaunchKernelGGL((k_gemm_wide<1, 1, 32, 2>), wgrid, dim3(256), 0, s, a, w.groups, total, per);
-        else hipLaunchKernelGGL((k_gemm_wide<2, 1, 16, 2>), wgrid, dim3(256), 0, s, a, w.groups, total, per);
+#define TK_TW_WIDE(WBV, MIV, KSV, PFV) hipLaunchKernelGGL((k_gemm_wide<WBV, MIV, 1, KSV, PFV>), wgrid, dim3(256), 0, s, a, w.groups, w.ny, total, per)
+        if (a.wbytes == 2) {
+            if (p.wide == 1) TK_TW_WIDE(2, 1, 32, 4);
+            else TK_TW_WIDE(2, 2, 32, 2);
+        } else if (p.wide == 1) TK_TW_WIDE(4, 1, 32, 2);
+        else TK_TW_WIDE(4, 2, 16, 2);
+#undef TK_TW_WIDE
         return hipGetLastError() == hipSuccess;
     }
     const int row_tiles = tw_row_tiles(a);
