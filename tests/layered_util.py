@@ -206,6 +206,16 @@ def close(got, want, tol):
     return rel_rms(got, want, 1.0 if tol < 1e-3 else 0.9) < tol
 
 
+def image_parts(f32, rows, n, k):
+    """in how many parts of k a product of few rows is made whose consumer adds up to eight"""
+    import ctypes as C
+    import trackiellm_amd as tk
+    form = (C.c_int * 4)()
+    kt = 16 if f32 else 32
+    assert tk.lib().tk_mi355x_gemm_image_form(int(f32), rows, n, (k + kt - 1) // kt * kt, 0, 0, 0, 8, form) == 0
+    return form[3]
+
+
 # width, feed-forward, rows of passes whose products take every block form of the kernel for many rows (held in test_gemm_cpu.py)
 LARGE_PRODUCTS = [(2064, 8190, 901), (2064, 8190, 1303), (1040, 5000, 1100), (1040, 2000, 2047), (528, 1500, 1100), (528, 1500, 300), (528, 700, 81),
                   (1040, 300, 2047), (1296, 5000, 600), (2576, 300, 2047)]

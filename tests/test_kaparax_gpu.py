@@ -427,3 +427,22 @@ def test_products_in_large_blocks(gpu, width, ff, rows, dtype, tol):
     whole = s.forward_streams([0] * rows, range(rows), toks)[0]
     parts = [s.forward_streams([1] * len(toks[i:i + 61]), range(i, i + len(toks[i:i + 61])), toks[i:i + 61])[0] for i in range(0, rows, 61)]
     assert U.rel_rms(whole, np.concatenate(parts)) < tol
+
+
+@pytest.mark.parametrize("dtype,tol", [("float32", F32), ("bfloat16", 0.007)])
+@pytest.mark.parametrize("width,ff", [(528, 2085), (1040, 2048), (2048, 2400)])
+def test_products_of_few_rows_in_parts_of_k(gpu, width, ff, dtype, tol):
+    """passes of 1 .. 64 rows (one to four tiles of them), whose down product (and, at 2048, the mixers' too) is made in two parts of k, of even and odd numbers of
+    k tiles, against the same rows in one pass of 150, which takes another kernel; tolerances as above"""
+    n = width // 16
+    f32 = dtype == "float32"
+    assert U.image_parts(f32, 40, width, ff) == 2 and U.image_parts(f32, 40, width, 32 * (15 if f32 else 62)) == 1 and U.image_parts(f32, 1, 2064, 8192) == 1
+    cfg = kaparax(width, 64, [serial(chunked(n, n, 16, 16, 16, 48, 2, 20.0), (ff, 7.0))])
+    m = gpu.LlmModel(config=cfg, dtype=dtype, seed=3)
+    toks = tokens_for(cfg, 150, 5)
+    s = gpu.LlmSession(m, 5, 192)
+    whole = s.forward_streams([0] * 150, range(150), toks)[0]
+    for q, r in ((1, 64), (2, 40), (3, 17), (4, 1)):
+        last = 150 if r > 1 else 6
+        parts = [s.forward_streams([q] * len(toks[i:min(i + r, last)]), range(i, min(i + r, last)), toks[i:min(i + r, last)])[0] for i in range(0, last, r)]
+        assert U.rel_rms(whole[:last], np.concatenate(parts)) < tol, r

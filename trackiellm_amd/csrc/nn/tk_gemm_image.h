@@ -41,7 +41,7 @@ struct TkImgGemm {
     /* f32 output: out[row][n], n < n_valid; columns [copy0, copy1) are also written, as T, to the image copy_img at k = n - copy0 */
     float* out;
     int ldc, n_valid;
-    /* K-split (wide kernel, f32 output without copied columns): up to max_slabs partial results, slab i at out + i * slab_floats, which the
+    /* K-split (f32 output without copied columns): up to max_slabs partial results, slab i at out + i * slab_floats, which the
      * consumer adds in ascending order; the launcher reports how many it wrote.  0 / 1: none. */
     int max_slabs;
     size_t slab_floats;

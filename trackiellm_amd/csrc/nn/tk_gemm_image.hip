@@ -46,13 +46,16 @@ __device__ __forceinline__ void store_act(const TkImgGemm& a, int64_t row, int n
     if (n < a.act_valid) tk_img_put4((T*)a.act_img, row, n, a.act_ktiles, h);
 }
 
-/* ---- skinny: MT M-tiles of rows, NT column tiles per workgroup, K interleaved over the waves in pieces of U tiles ---- */
+/* ---- skinny: MT M-tiles of rows, NT column tiles per workgroup, K interleaved over the waves in pieces of U tiles ----
+ * Loads of three M-tiles are three (33 .. 48 rows; four, one of them twice: 40 rows x 2048 x 16384 gate and up 17.2 -> 15.8 us, x 32000 34.2 -> 28.6). */
 template <typename T, int MT, int NT, int WAVES, bool SWIGLU, bool GROUPED>
 __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
-    constexpr int U = MT >= 4 ? 2 : 4;
+    constexpr int U = MT >= 3 ? 2 : 4;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ktiles = a.K / TkImg<T>::KT;
+    const int k0 = GROUPED ? 0 : (int)((int64_t)ktiles * blockIdx.z / gridDim.z), k1 = GROUPED ? ktiles : (int)((int64_t)ktiles * (blockIdx.z + 1) / gridDim.z);
+    if (!GROUPED && !SWIGLU) a.out += blockIdx.z * a.slab_floats;
     int m0 = blockIdx.y * MT, mlive = (a.nrows + 15) / 16 - m0;
     const uint8_t* wbase = (const uint8_t*)a.w;
     if (GROUPED) {
@@ -80,26 +83,26 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
     auto load = [&](int c) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int kt = c + u < ktiles ? c + u : ktiles - 1;
+            const int kt = c + u < k1 ? c + u : k1 - 1;
 #pragma unroll
             for (int n = 0; n < NT; ++n) wq[u][n] = ldg16_stream(wp[n] + (size_t)kt * 1024);
 #pragma unroll
             for (int m = 0; m < MT; ++m) aq[u][m] = ldg16(ap[m] + (size_t)kt * 1024);
         }
     };
-    int c = wave * U;
-    if (c < ktiles) load(c);
-    while (c < ktiles) {
+    int c = k0 + wave * U;
+    if (c < k1) load(c);
+    while (c < k1) {
         tk_v4u w0[U][NT], a0[U][MT];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
             for (int n = 0; n < NT; ++n) w0[u][n] = wq[u][n];
 #pragma unroll
-            for (int m = 0; m < MT; ++m) a0[u][m] = c + u < ktiles ? aq[u][m] : zero;
+            for (int m = 0; m < MT; ++m) a0[u][m] = c + u < k1 ? aq[u][m] : zero;
         }
         const int next = c + WAVES * U;
-        if (next < ktiles) load(next);
+        if (next < k1) load(next);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -338,6 +341,13 @@ WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
     return best;
 }
 
+/* A product of few rows in two parts of k, where its column tiles leave half of the CUs idle and each part is a piece for every wave: 40 rows x 2048 x 8192 19.7 ->
+ * 13.0 us, x 2048 7.2 -> 5.9 (three parts 14.8 and 6.6, four 13.0 and 6.0, eight 13.4 and 7.3); steps of a 2048-wide model at 1, 16, 64 rows 488 -> 451, 540 -> 506,
+ * 909 -> 828 us.  256 column tiles: 486 -> 489, 532 -> 537, 920 -> 920.  The rows do not enter, so that a row's result does not depend on the others of its step. */
+int skinny_parts(const TkImgGemm& g, bool swiglu, bool grouped) {
+    return !swiglu && !grouped && g.max_slabs > 1 && g.N / 16 <= 128 && g.K / tk_img_kt(g.type) >= 64 ? 2 : 1;
+}
+
 template <typename T, bool SWIGLU, bool GROUPED>
 const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
     const int ntiles = g.N / 16;
@@ -345,8 +355,10 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
     if (mtiles <= 4) {
         /* GROUPED: one block per table entry */
         const int gy = GROUPED ? g.max_blocks : 1;
-#define TK_SK(MT, NT, WV) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, gy), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
-#define TK_SKM(NT, WV) do { if (mtiles <= 1) TK_SK(1, NT, WV); else if (mtiles <= 2) TK_SK(2, NT, WV); else TK_SK(4, NT, WV); } while (0)
+        const int parts = skinny_parts(g, SWIGLU, GROUPED);
+        if (slabs) *slabs = parts;
+#define TK_SK(MT, NT, WV) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, gy, parts), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
+#define TK_SKM(NT, WV) do { if (mtiles <= 1) TK_SK(1, NT, WV); else if (mtiles <= 2) TK_SK(2, NT, WV); else if (mtiles <= 3) TK_SK(3, NT, WV); else TK_SK(4, NT, WV); } while (0)
         if (SWIGLU || ntiles * gy >= 1024) {
             if (ntiles * gy >= 2048) TK_SKM(2, 4); else TK_SKM(2, 8);
         } else {
@@ -377,7 +389,7 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
 void tk_gemm_image_form(const TkImgGemm& g, int form[4]) {
     const bool grouped = g.max_blocks > 0;
     form[0] = 64; form[1] = form[2] = 0; form[3] = 1;
-    if ((grouped ? g.block_tiles : (g.nrows + 15) / 16) <= 4) return;
+    if ((grouped ? g.block_tiles : (g.nrows + 15) / 16) <= 4) { form[3] = skinny_parts(g, g.swiglu != 0, grouped); return; }
     const WidePick p = pick_wide(g, g.swiglu != 0, grouped);
     const WideForm& w = wide_forms[p.form];
     form[0] = 16 * w.mb; form[1] = 16 * w.nb; form[2] = w.ring; form[3] = p.ks;
