@@ -291,6 +291,23 @@ def test_many_heads_and_sequences(gpu, tmp_path, dim, vdim):
         assert close(np.array(rows), c.want(p)[0], F32)
 
 
+@pytest.mark.parametrize("rows", [25, 26, 40])
+def test_steps_around_the_change_of_the_mixers_workgroups(gpu, rows):
+    """attention of 2 kv heads beside 8 delta heads, 128 wide: eight waves a workgroup up to 256 of them, four beyond.  Sequences of 150 positions and of one,
+    against the same positions in one pass each, which takes other kernels; the bf16 tolerance of sums in another order, as for the products"""
+    cfg = config(128, 64, [layer(attention(4, 2, 128, 128, 64, 130, 2), delta(8, 4, 128, 128, 4), dense(64))] * 2)
+    m = gpu.LlmModel(config=cfg, dtype="bfloat16", seed=9)
+    s = gpu.LlmSession(m, rows, 192)
+    n = [150 if i % 3 else 1 for i in range(rows)]
+    toks = [tokens_for(cfg, n[i] + 1, i) for i in range(rows)]
+    for i in range(rows):
+        s.forward_rows([i] * n[i], range(n[i]), toks[i][:-1], [], want_logits=False)
+    got, _ = s.forward_rows(range(rows), n, [t[-1] for t in toks], range(rows))
+    one = gpu.LlmSession(m, 1, 192)
+    want = np.concatenate([one.forward_rows([0] * (n[i] + 1), range(n[i] + 1), toks[i], [n[i]])[0] for i in range(rows)])
+    assert U.rel_rms(got, want) < 0.02
+
+
 def test_wanted_rows_only(cases):
     c = cases("odd")
     toks = tokens_for(c.cfg, 100)

@@ -1864,7 +1864,11 @@ static int delta_ct_log2(const TkDeltaArgs& d) {
 }
 
 bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, const TkPassTab& t, int nrows, hipStream_t s) {
-    const int b = attn_bucket(a), ctl = delta_ct_log2(d), waves = attn_row_waves(a, nrows), threads = 64 * waves;
+    const int b = attn_bucket(a), ctl = delta_ct_log2(d);
+    /* 168 registers at heads of 128: a CU holds one workgroup of eight waves or three of four.  Eight, the shorter chain of pages, while every workgroup has a CU:
+     * steps of an eight-layer model of 2 + 8 workgroups a row over 400 positions, with eight / four: 25 rows 673 / 674, 32 746 / 715, 40 774 / 741, 52 873 / 815 us; over 20
+     * positions 16 rows 511 / 521, 26 626 / 619.  4 + 16 a row: 12 rows 542 / 538, 16 564 / 543, 25 707 / 671. */
+    const int waves = (int64_t)(attn_row_blocks(a) + d.heads) * nrows > 256 ? 4 : attn_row_waves(a, nrows), threads = 64 * waves;
     const int rg = threads >> ctl, rpt = rg ? (d.dim + rg - 1) / rg : 1 << 20;
     if (type != TK_IMG_BF16 || b > 128 || rpt > (waves == 8 ? 8 : 16) || d.vdim > threads) return false;
     const dim3 grid(attn_row_blocks(a) + d.heads, nrows);
