@@ -327,13 +327,15 @@ def test_prompt_chunks_of_a_long_prompt_bit_exact(mistral_long):
     assert np.array_equal(gk, wk) and np.array_equal(gv, wv)
 
 
+@pytest.mark.parametrize("window", [512, 511, 1300])
 @pytest.mark.parametrize("head_dim,grp", [(128, 4), (128, 2), (64, 4)])
-def test_long_form_of_one_row_is_the_fused_kernels_bit_for_bit(gpu, monkeypatch, head_dim, grp):
-    """one row from position 256 on in windows up to 2048 (scores, chains, join inside the o projection) and two rows from 512: where a class's rows fill
-    their chunks of 64 or spill by one (256, 257, 767 .. 769, 1023 .. 1025), more rows than are in flight, the window's last position"""
+def test_long_form_of_one_row_is_the_fused_kernels_bit_for_bit(gpu, monkeypatch, head_dim, grp, window):
+    """one row from position 256 on in windows up to 512 and from 512 beyond, two rows from 512 (scores, chains, join inside the o projection): where a class's
+    rows fill their chunks of 64 or spill by one (256, 257, 511, 767 .. 769, 1023 .. 1025), more rows than are in flight, the windows' last positions"""
     hp = gpu.LlmHParams(2, 1024, 8, 8 // grp, head_dim, 1024, 512, 1e-5, 10000.0, 0, 0, 0, 0, 1)
     model = gpu.LlmModel(hp).fill_synthetic(4)
-    hp, window = model.hparams, 1300
+    hp = model.hparams
+    cases = [(1, c) for c in (1299, 1100, 1025, 1024, 1023, 769, 768, 767, 515)] + [(2, 1299), (2, 1024), (2, 512)] if window > 512 else [(1, c) for c in (window - 1, 449, 320, 257, 256)]
     rng = np.random.default_rng(head_dim + grp)
     kv = [(f16_bits(rng, (window, hp.n_kv_head, head_dim), 0.6), f16_bits(rng, (window, hp.n_kv_head, head_dim), 1.0)) for _ in range(4)]
     runs = {}
@@ -343,7 +345,7 @@ def test_long_form_of_one_row_is_the_fused_kernels_bit_for_bit(gpu, monkeypatch,
         for layer in range(2):
             for s in range(2):
                 sess.kv_write(layer, s, 0, *kv[2 * layer + s])
-        for rows, ctx in [(1, c) for c in (1299, 1100, 1025, 1024, 1023, 769, 768, 767, 515, 257, 256)] + [(2, 1299), (2, 1024), (2, 512)]:  # downwards: a step writes its own position
+        for rows, ctx in cases:  # downwards: a step writes its own position
             want_form = 3 if off == "0" and gpu.lib().tk_mi355x_device_cu_count(0) == 256 else None
             if want_form:
                 assert gpu.attention_plan(rows, hp.n_head, hp.n_kv_head, head_dim, window, True, top_position=ctx)[0] == want_form

@@ -114,10 +114,10 @@ void tk_launch_attention_prefill(const float* qbuf, const uint16_t* kcache, cons
  * q | k | v projection's K-split slabs (the launch finishes q / k / v itself and appends this pass's rows to the cache) */
 /* From which position a decode pass takes this form, by whole steps of a 32-layer model (fused kernels / this form, ms): 1 row at 224 positions 1.675 / 1.704,
  * at 288 1.767 / 1.737, at 448 1.852 / 1.742, at 900 2.188 / 1.815; 4 rows at 352 2.046 / 2.081, at 600 2.363 / 2.213; 8 rows at 600 2.384 / 2.445, at 900
- * 2.647 / 2.606; at 16 rows the fused kernels' 256 workgroups already cover the chip.  The window hardly matters (4096: 1 row at 448 1.892 / 1.743); beyond
- * 2048 the plan that its tests fix stays, 512 at 1 .. 4 rows. */
+ * 2.647 / 2.606; at 16 rows the fused kernels' 256 workgroups already cover the chip.  Windows of up to 512
+ * positions take it from 256 on; in larger ones, where it would win from there as well (4096: 1 row at 448 1.892 / 1.743), the plan that the tests fix stays: 512. */
 #define TK_LONG_ATT_MAX_ROWS 8
-static inline int tk_long_att_min_pos(int nrows, int max_ctx) { return nrows > 4 ? 768 : nrows == 1 && max_ctx <= 2048 ? 256 : 512; }
+static inline int tk_long_att_min_pos(int nrows, int max_ctx) { return nrows > 4 ? 768 : nrows == 1 && max_ctx <= 512 ? 256 : 512; }
 bool tk_attention_long_applies(int nrows, int n_head, int n_kv_head, int head_dim);
 size_t tk_attention_long_scratch_floats(int n_head, int head_dim, int max_ctx); /* floats of the `scores` scratch buffer */
 /* where such a launch leaves the classes' outputs [row][head][4][head_dim] and denominators [row][head][4]; join = false: its consumer joins them (TkGemvArgs::fuse 3) */
