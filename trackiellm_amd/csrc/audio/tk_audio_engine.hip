@@ -9,6 +9,7 @@
 #include "../nn/tk_attention_images.h"
 #include "../nn/tk_gemm_tiled.h"
 #include "../nn/tk_nn_kernels.h"
+#include "../nn/tk_image_device.h"
 
 /* Every stream of the library keeps the default priority: work on streams of different priorities has been seen to hang. */
 static inline hipError_t tk_create_perception_stream(hipStream_t* s) { return hipStreamCreateWithFlags(s, hipStreamNonBlocking); }
@@ -54,7 +55,7 @@ __global__ void k_power(const float* ri, int64_t rows, int nb, float* out) {
  * one workgroup, now 7 + 4. */
 #define TK_MEL_PARTS 64
 __device__ __forceinline__ float mel_block_max(float mx, float* red) { /* 256 threads */
-    for (int s = 32; s >= 1; s >>= 1) mx = tk_fmaxf(mx, __shfl_xor(mx, s, 64));
+    mx = tk_wave_max(mx);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = mx;
     __syncthreads();
     return tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
@@ -242,7 +243,7 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
         for (int j = 0; j < NS; ++j)
             if (k0 + tk + 256 * j < Tk) m = tk_fmaxf(m, e[j]);
     }
-    for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, __shfl_xor(m, s, 64));
+    m = tk_wave_max(m);
     if (lane == 0) red[wave & 3] = m;
     __syncthreads();
     m = tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
                 if (FORM == AT1_LONG && wave < 4) sc[at1_place(k0 + tk + 256 * j)] = e[j];
             }
     }
-    for (int w = 32; w >= 1; w >>= 1) s = s + __shfl_xor(s, w, 64);
+    s = tk_wave_butterfly_sum(s);
     if (lane == 0) red[4 + (wave & 3)] = s;
     __syncthreads();
     const float tot = ((red[4] + red[5]) + red[6]) + red[7];

@@ -8,6 +8,7 @@
 #include <type_traits>
 
 #include "../common/tk_exact_math.h"
+#include "tk_image_device.h"
 
 typedef _Float16 tw_v8h __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -73,9 +74,7 @@ __device__ __forceinline__ void tw_layernorm(const TkTiledGemm& a, int row0, int
     const int D = a.K;
     auto fold = [&](float (&s)[4]) {
 #pragma unroll
-        for (int m = 32; m >= 1; m >>= 1)
-#pragma unroll
-            for (int w = 0; w < 4; ++w) s[w] = s[w] + __shfl_xor(s[w], m, 64);
+        for (int w = 0; w < 4; ++w) s[w] = tk_wave_butterfly_sum(s[w]);
         return ((s[0] + s[1]) + s[2]) + s[3];
     };
     for (int r = wave; r < rows; r += nw) {

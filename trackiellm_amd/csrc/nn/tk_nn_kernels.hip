@@ -5,6 +5,7 @@
 
 #include "../common/tk_exact_math.h"
 #include "../common/tk_sample_device.h"
+#include "tk_image_device.h"
 
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -1323,7 +1324,7 @@ void tk_launch_copy_cols(const float* x, int rows, int C, int ldx, float* y, int
 }
 
 __device__ __forceinline__ float nn_block_sum256(float v, float* red) {
-    for (int s = 32; s >= 1; s >>= 1) v = v + __shfl_xor(v, s, 64);
+    v = tk_wave_butterfly_sum(v);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
     float r = ((red[0] + red[1]) + red[2]) + red[3];
@@ -1401,7 +1402,7 @@ __global__ __launch_bounds__(256) void k_softmax_rows(float* x, int cols, int ld
     const int n = cols;
     float m = -INFINITY;
     for (int i = threadIdx.x; i < n; i += 256) m = tk_fmaxf(m, xr[i]);
-    for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, __shfl_xor(m, s, 64));
+    m = tk_wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     m = tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
@@ -1425,7 +1426,7 @@ __global__ __launch_bounds__(256) void k_softmax_rows_reg(float* x, int cols, in
         v[u] = i < cols ? xr[i] : -INFINITY;
         if (i < cols) m = tk_fmaxf(m, v[u]);
     }
-    for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, __shfl_xor(m, s, 64));
+    m = tk_wave_max(m);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
     __syncthreads();
     m = tk_fmaxf(tk_fmaxf(red[0], red[1]), tk_fmaxf(red[2], red[3]));
@@ -1461,7 +1462,7 @@ __global__ __launch_bounds__(256) void k_softmax_rows_wave(float* x, int64_t row
             m = tk_fmaxf(tk_fmaxf(tk_fmaxf(tk_fmaxf(m, v[u].x), v[u].y), v[u].z), v[u].w);
         }
     }
-    for (int s = 32; s >= 1; s >>= 1) m = tk_fmaxf(m, __shfl_xor(m, s, 64));
+    m = tk_wave_max(m);
     float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, p3 = 0.0f;
 #pragma unroll
     for (int u = 0; u < 8; ++u)
