@@ -1208,3 +1208,35 @@ def test_runner_long_prompt_through_the_reference_surface(gpu):
     loader.unload(h)
     loader.close()
     orc.close()
+
+
+@pytest.mark.parametrize("nrows", [1, 3, 40, 130, 256])
+def test_quantised_rows_with_ties_zeros_and_tiny_values(gpu, nrows):
+    """the first element of largest magnitude decides a block's sign, wherever its equals of the other sign stand: in the same run of 8, in another one of the
+    half-wave, at its ends; a row of zeros and one of subnormal halves.  Through the embedding of layer 0 (norm weights 1): inside the mat-vec launch (1 row), as a
+    launch (3 and more), logits bit for bit the oracle's"""
+    hp = gpu.TINY()
+    rng = np.random.default_rng(5)
+    pairs = [(0, 255), (0, 1), (7, 8), (8, 15), (100, 101), (127, 128), (248, 7), (255, 248), (64, 192), (31, 32), (200, 17)]
+    rows = rng.uniform(-0.5, 0.5, (hp.vocab, 256)).astype(np.float16)
+    for i, (a, b) in enumerate(pairs):
+        for j, sign in enumerate((1.0, -1.0)):
+            rows[2 * i + j, a], rows[2 * i + j, b] = 0.75 * sign, -0.75 * sign
+    rows[22] = 0.0
+    rows[23] = (rng.integers(-3, 4, 256) * 2.0 ** -24).astype(np.float16)
+    rows[24], rows[25] = 0.25, -0.25
+    model, orc = gpu.LlmModel(hp).fill_synthetic(4), O.OracleLlm(oracle_cfg_from(gpu.LlmModel(hp).fill_synthetic(4).hparams, 8, nrows), seed=4)
+    for m in (model, orc):
+        m.set_tensor(-1, 0, 1, rows)
+        m.set_tensor(0, 0, 0, np.ones(256, np.float32))
+    sess = gpu.LlmSession(model, nrows, 8)
+    seq, pos = np.arange(nrows, dtype=np.int32), np.zeros(nrows, np.int32)
+    for first in range(0, 26, nrows):
+        tok = ((first + np.arange(nrows)) % 40).astype(np.int32)
+        want, wam = orc.forward(seq, pos, tok)
+        got, gam = sess.forward(seq, pos, tok)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), (first, np.abs(got - want).max())
+        assert np.array_equal(gam, wam)
+    sess.close()
+    model.close()
+    orc.close()
