@@ -308,6 +308,24 @@ def test_steps_around_the_change_of_the_mixers_workgroups(gpu, rows):
     assert U.rel_rms(got, want) < 0.02
 
 
+@pytest.mark.parametrize("att,dim,vdim", [((128, 128, 64), 128, 128), ((64, 64, 16), 64, 128), ((24, 40, 12), 20, 36), ((128, 100, 64), 256, 64), ((48, 64, 8), 9, 7)])
+def test_a_row_of_a_step_does_not_depend_on_its_workgroups(gpu, att, dim, vdim):
+    """25 rows take eight waves a workgroup (250 of them), 26 rows four: the same chains of pages and row groups, the same bits.  Contexts of one page to eleven, so that a
+    wave has no page, one or two of either of its chains"""
+    cfg = config(128, 64, [layer(attention(4, 2, *att, 700, 2), delta(8, 4, dim, vdim, 4), dense(64))] * 2)
+    m = gpu.LlmModel(config=cfg, dtype="bfloat16", seed=9)
+    n = [(1, 70, 300, 470, 640, 699)[i % 6] for i in range(26)]
+    toks = [tokens_for(cfg, n[i] + 1, i) for i in range(26)]
+
+    def step(rows):
+        s = gpu.LlmSession(m, 26, 768)
+        for i in range(26):
+            s.forward_rows([i] * n[i], range(n[i]), toks[i][:-1], [], want_logits=False)
+        return s.forward_rows(range(rows), n[:rows], [t[-1] for t in toks[:rows]], range(rows))[0].copy()
+    eight, four = step(25), step(26)
+    assert np.isfinite(eight).all() and np.array_equal(eight.view(np.uint32), four[:25].view(np.uint32))
+
+
 def test_wanted_rows_only(cases):
     c = cases("odd")
     toks = tokens_for(c.cfg, 100)

@@ -693,8 +693,30 @@ __global__ __launch_bounds__(256, B * sizeof(T) >= 512 ? 1 : 2) void k_attn_tile
     if (q < n) attn_store<T, VT>(a, f.o, row0 + q, h, g, a.out_scale / f.l);
 }
 
-/* decoding: one row x up to 16 query heads of one kv head per workgroup, pages dealt to the waves (and to `splits` workgroups), merged in LDS */
-template <typename T, int B, int WAVES, bool FULL>
+/* a chain's result to and from the LDS: so [n][VT][64], sm and sl [n][64] behind it */
+template <typename T, int VT>
+__device__ __forceinline__ void flash_leave(const Flash<T, VT>& f, uint8_t* lds, int n, int to, int lane) {
+    tk_v4f* so = (tk_v4f*)lds;
+    float *sm = (float*)(so + n * VT * 64), *sl = sm + n * 64;
+#pragma unroll
+    for (int i = 0; i < VT; ++i) so[(to * VT + i) * 64 + lane] = f.o[i];
+    sm[to * 64 + lane] = f.m; sl[to * 64 + lane] = f.l;
+}
+template <typename T, int VT>
+__device__ __forceinline__ void flash_take(Flash<T, VT>& f, const uint8_t* lds, int n, int from, int lane) {
+    const tk_v4f* so = (const tk_v4f*)lds;
+    const float *sm = (const float*)(so + n * VT * 64), *sl = sm + n * 64;
+    const float m2 = sm[from * 64 + lane], mn = fmaxf(f.m, m2), ms = mn == -INFINITY ? 0.0f : mn;
+    const float c1 = __builtin_amdgcn_exp2f(f.m - ms), c2 = __builtin_amdgcn_exp2f(m2 - ms);
+    f.l = f.l * c1 + sl[from * 64 + lane] * c2;
+    f.m = mn;
+#pragma unroll
+    for (int i = 0; i < VT; ++i) f.o[i] = f.o[i] * c1 + so[(from * VT + i) * 64 + lane] * c2;
+}
+
+/* decoding: one row x up to 16 query heads of one kv head per workgroup, pages dealt to CHAINS chains (and to `splits` workgroups), merged in LDS.  A wave
+ * takes one chain, or (CHAINS = 2 WAVES) chain WAVES + w, then w: the order of every sum is that of CHAINS waves. */
+template <typename T, int B, int WAVES, bool FULL, int CHAINS = WAVES>
 __device__ __forceinline__ void attn_row(const TkAttnArgs& a, const TkPassTab& t, int block, int row, int split, int splits, float* scratch, uint8_t* lds) {
     constexpr int DT = B / TkImg<T>::KT, VT = B / 16, SZ = sizeof(T);
     constexpr bool AHEAD = SZ == 2 && B <= 128; /* a page's values are requested together with its keys */
@@ -710,59 +732,55 @@ __device__ __forceinline__ void attn_row(const TkAttnArgs& a, const TkPassTab& t
     for (int d = 0; d < DT; ++d)
         if (d < nd) qf[d] = *(const tk_v4u*)((const uint8_t*)a.q + (((size_t)row * a.heads + h) * a.kv.dim_pad) * SZ + d * 64 + g * 16);
     Flash<T, VT> f;
-    f.init();
     const PageWalk walk(a, pos, pos);
     const int low = first_visible(a, pos);
-    for (int i = split * WAVES + wave; i < walk.count; i += WAVES * splits) {
-        const size_t page = (size_t)t.page_of[(size_t)seq * t.max_pages + walk.page(i)] * a.kv_heads + kvh;
-        const uint8_t* kp = (const uint8_t*)a.kv.k + (page * TK_PAGE + (lane & 15)) * a.kv.dim_pad * SZ + g * 16;
-        const uint8_t* vp = (const uint8_t*)a.kv.v + (page * a.kv.vdim_pad + (lane & 15)) * TK_PAGE * SZ + 4 * g * SZ;
-        const int k0 = walk.page(i) * TK_PAGE;
-        auto vload = [&](int vt, int j) { return *(const VF*)(vp + ((size_t)16 * vt * TK_PAGE + 16 * j) * SZ); };
-        tk_v4u kf[AHEAD ? 4 : 1][AHEAD ? DT : 1];
-        VF vf[AHEAD ? VT : 1][4];
-        if (AHEAD) {
+    static_assert(CHAINS == WAVES || CHAINS == 2 * WAVES, "a wave has one chain or two");
+#pragma unroll 1
+    for (int part = CHAINS / WAVES - 1; part >= 0; --part) {
+        f.init();
+        for (int i = split * CHAINS + part * WAVES + wave; i < walk.count; i += CHAINS * splits) {
+            const size_t page = (size_t)t.page_of[(size_t)seq * t.max_pages + walk.page(i)] * a.kv_heads + kvh;
+            const uint8_t* kp = (const uint8_t*)a.kv.k + (page * TK_PAGE + (lane & 15)) * a.kv.dim_pad * SZ + g * 16;
+            const uint8_t* vp = (const uint8_t*)a.kv.v + (page * a.kv.vdim_pad + (lane & 15)) * TK_PAGE * SZ + 4 * g * SZ;
+            const int k0 = walk.page(i) * TK_PAGE;
+            auto vload = [&](int vt, int j) { return *(const VF*)(vp + ((size_t)16 * vt * TK_PAGE + 16 * j) * SZ); };
+            tk_v4u kf[AHEAD ? 4 : 1][AHEAD ? DT : 1];
+            VF vf[AHEAD ? VT : 1][4];
+            if (AHEAD) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int d = 0; d < DT; ++d)
+                        if (d < nd) kf[j][d] = *(const tk_v4u*)(kp + (size_t)16 * j * a.kv.dim_pad * SZ + d * 64);
+#pragma unroll
+                for (int i2 = 0; i2 < VT; ++i2)
+                    if (i2 < nv)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) vf[i2][j] = vload(i2, j);
+            }
+            tk_v4f s[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                s[j] = tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int d = 0; d < DT; ++d)
-                    if (d < nd) kf[j][d] = *(const tk_v4u*)(kp + (size_t)16 * j * a.kv.dim_pad * SZ + d * 64);
-#pragma unroll
-            for (int i2 = 0; i2 < VT; ++i2)
-                if (i2 < nv)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) vf[i2][j] = vload(i2, j);
+                    if (d < nd) s[j] = TkImg<T>::mma(AHEAD ? kf[AHEAD ? j : 0][AHEAD ? d : 0] : *(const tk_v4u*)(kp + (size_t)16 * j * a.kv.dim_pad * SZ + d * 64), qf[d], s[j]);
+            }
+            mask_scores<T>(s, a, k0, g, pos, low, pos, low);
+            f.update(s, nv, [&](int vt, int j) { return AHEAD ? vf[AHEAD ? vt : 0][j] : vload(vt, j); });
         }
-        tk_v4f s[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            s[j] = tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int d = 0; d < DT; ++d)
-                if (d < nd) s[j] = TkImg<T>::mma(AHEAD ? kf[AHEAD ? j : 0][AHEAD ? d : 0] : *(const tk_v4u*)(kp + (size_t)16 * j * a.kv.dim_pad * SZ + d * 64), qf[d], s[j]);
-        }
-        mask_scores<T>(s, a, k0, g, pos, low, pos, low);
-        f.update(s, nv, [&](int vt, int j) { return AHEAD ? vf[AHEAD ? vt : 0][j] : vload(vt, j); });
+        if (part > 0) flash_leave(f, lds, CHAINS / 2, wave, lane); /* every lane reads back what it wrote */
+    }
+    if (CHAINS > WAVES) {
+        flash_take(f, lds, CHAINS / 2, wave, lane);
+        __syncthreads();
     }
     /* the upper half of the waves into the lower half, and again */
-    tk_v4f* so = (tk_v4f*)lds; /* [WAVES / 2][VT][64] */
-    float *sm = (float*)(so + WAVES / 2 * VT * 64), *sl = sm + WAVES / 2 * 64;
 #pragma unroll
     for (int half = WAVES / 2; half >= 1; half >>= 1) {
-        if (wave >= half && wave < 2 * half) {
-#pragma unroll
-            for (int i = 0; i < VT; ++i) so[((wave - half) * VT + i) * 64 + lane] = f.o[i];
-            sm[(wave - half) * 64 + lane] = f.m; sl[(wave - half) * 64 + lane] = f.l;
-        }
+        if (wave >= half && wave < 2 * half) flash_leave(f, lds, CHAINS / 2, wave - half, lane);
         __syncthreads();
-        if (wave < half) {
-            const float m2 = sm[wave * 64 + lane], mn = fmaxf(f.m, m2), ms = mn == -INFINITY ? 0.0f : mn;
-            const float c1 = __builtin_amdgcn_exp2f(f.m - ms), c2 = __builtin_amdgcn_exp2f(m2 - ms);
-            f.l = f.l * c1 + sl[wave * 64 + lane] * c2;
-            f.m = mn;
-#pragma unroll
-            for (int i = 0; i < VT; ++i) f.o[i] = f.o[i] * c1 + so[(wave * VT + i) * 64 + lane] * c2;
-        }
+        if (wave < half) flash_take(f, lds, CHAINS / 2, wave, lane);
         __syncthreads();
     }
     if (wave != 0 || q >= gq) return;
@@ -775,7 +793,7 @@ __device__ __forceinline__ void attn_row(const TkAttnArgs& a, const TkPassTab& t
 #pragma unroll
             for (int r = 0; r < 4; ++r) out[2 + 16 * i + 4 * g + r] = f.o[i][r];
 }
-template <int B, int WAVES> constexpr size_t attn_row_lds() { return (size_t)WAVES / 2 * (B / 16 * 1024 + 512); }
+template <int B, int CHAINS> constexpr size_t attn_row_lds() { return (size_t)CHAINS / 2 * (B / 16 * 1024 + 512); }
 
 template <typename T, int B, int WAVES, bool FULL>
 __global__ __launch_bounds__(64 * WAVES, B == 256 ? 1 : 2) void k_attn_rows(TkAttnArgs a, TkPassTab t, int splits, float* scratch) {
@@ -1128,20 +1146,21 @@ __global__ __launch_bounds__(256) void k_delta_out(TkDeltaArgs d) {
     }
 }
 
-/* one token of one head: the state is read once and written once, a thread holds RPT rows x 4 columns of it.
+/* one token of one head: the state is read once and written once, a thread holds RPT rows x 4 columns of it, PARTS times: its sums are those of
+ * PARTS x THREADS threads (of which the further ones hold rows of the state only: dim, vdim <= 256 <= THREADS).
  * o = S_new^T q = (g S)^T q + (k . q) u, so both reductions over the key rows run on the decayed old state at once. */
-template <typename T, int THREADS, int RPT>
+template <typename T, int THREADS, int RPT, int PARTS = 1>
 __device__ __forceinline__ void delta_row(const TkDeltaArgs& d, const TkPassTab& t, int h, int row, int ct_log2, float* step_lds) {
     const int tid = threadIdx.x, kvh = h / (d.heads / d.kv_heads), vp = (d.vdim + 3) & ~3;
-    const int ct = tid & ((1 << ct_log2) - 1), rg = tid >> ct_log2, RG = THREADS >> ct_log2;
+    const int ct = tid & ((1 << ct_log2) - 1), rg = tid >> ct_log2, RG1 = THREADS >> ct_log2, RG = RG1 * PARTS;
     const bool live = 4 * ct < vp;
     const int seg = t.seg[row], in = t.seg_in[seg], out = t.seg_out[seg];
     float *red = step_lds, *lq = red + 16, *lk = lq + d.dim, *lg = lk + d.dim, *lu = red + 16 + (3 * d.dim + 3) / 4 * 4, *pk = lu + vp, *pq = pk + RG * vp;
-    tk_v4f S[RPT];
+    tk_v4f S[PARTS * RPT]; /* [i of row group rg + RG1 p] at p RPT + i */
     const float* sin = d.state + ((size_t)(in < 0 ? 0 : in) * d.heads + h) * d.dim * vp + 4 * ct;
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-        const int e = rg + RG * i;
+    for (int i = 0; i < PARTS * RPT; ++i) {
+        const int e = rg + RG1 * (i / RPT) + RG * (i % RPT);
         S[i] = in >= 0 && live && e < d.dim ? *(const tk_v4f*)(sin + (size_t)e * vp) : tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
     float kq = 0.0f;
@@ -1151,13 +1170,16 @@ __device__ __forceinline__ void delta_row(const TkDeltaArgs& d, const TkPassTab&
         kq += q * k;
     }
     kq = block_sum(kq, red); /* also orders the LDS writes above before the reads below */
-    tk_v4f ak = {0.0f, 0.0f, 0.0f, 0.0f}, aq = ak;
 #pragma unroll
-    for (int i = 0; i < RPT; ++i) {
-        const int e = rg + RG * i;
-        if (e < d.dim) { S[i] *= lg[e]; ak += S[i] * lk[e]; aq += S[i] * lq[e]; }
+    for (int p = 0; p < PARTS; ++p) {
+        tk_v4f ak = {0.0f, 0.0f, 0.0f, 0.0f}, aq = ak;
+#pragma unroll
+        for (int i = p * RPT; i < (p + 1) * RPT; ++i) {
+            const int e = rg + RG1 * p + RG * (i % RPT);
+            if (e < d.dim) { S[i] *= lg[e]; ak += S[i] * lk[e]; aq += S[i] * lq[e]; }
+        }
+        if (live) { *(tk_v4f*)(pk + (rg + RG1 * p) * vp + 4 * ct) = ak; *(tk_v4f*)(pq + (rg + RG1 * p) * vp + 4 * ct) = aq; }
     }
-    if (live) { *(tk_v4f*)(pk + rg * vp + 4 * ct) = ak; *(tk_v4f*)(pq + rg * vp + 4 * ct) = aq; }
     __syncthreads();
     const float beta = d.beta[(size_t)row * d.heads + h];
     float o = 0.0f, ss = 0.0f;
@@ -1175,8 +1197,8 @@ __device__ __forceinline__ void delta_row(const TkDeltaArgs& d, const TkPassTab&
         const tk_v4f u = *(const tk_v4f*)(lu + 4 * ct);
         float* so = d.state + ((size_t)out * d.heads + h) * d.dim * vp + 4 * ct;
 #pragma unroll
-        for (int i = 0; i < RPT; ++i) {
-            const int e = rg + RG * i;
+        for (int i = 0; i < PARTS * RPT; ++i) {
+            const int e = rg + RG1 * (i / RPT) + RG * (i % RPT);
             if (e < d.dim) *(tk_v4f*)(so + (size_t)e * vp) = S[i] + u * lk[e];
         }
     }
@@ -1199,11 +1221,11 @@ __global__ __launch_bounds__(THREADS) void k_delta_step(TkDeltaArgs d, TkPassTab
 }
 
 /* a decode step's attention and delta rule side by side: the first na workgroups of a row are attention's, the others one delta head each */
-template <typename T, int B, int WAVES, int RPT, bool FULL>
-__global__ __launch_bounds__(64 * WAVES, 2) void k_mixers_step(TkAttnArgs a, TkDeltaArgs d, TkPassTab t, int na, int ct_log2) {
+template <typename T, int B, int WAVES, int CHAINS, int RPT, bool FULL>
+__global__ __launch_bounds__(64 * WAVES, WAVES == 4 && FULL ? 3 : 2) void k_mixers_step(TkAttnArgs a, TkDeltaArgs d, TkPassTab t, int na, int ct_log2) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    if ((int)blockIdx.x < na) attn_row<T, B, WAVES, FULL>(a, t, blockIdx.x, blockIdx.y, 0, 1, nullptr, lds);
-    else delta_row<T, 64 * WAVES, RPT>(d, t, blockIdx.x - na, blockIdx.y, ct_log2, (float*)lds);
+    if ((int)blockIdx.x < na) attn_row<T, B, WAVES, FULL, CHAINS>(a, t, blockIdx.x, blockIdx.y, 0, 1, nullptr, lds);
+    else delta_row<T, 64 * WAVES, RPT, CHAINS / WAVES>(d, t, blockIdx.x - na, blockIdx.y, ct_log2, (float*)lds);
 }
 
 __global__ void k_swap_state(TkPassTab t, int n) {
@@ -1871,19 +1893,21 @@ static int delta_ct_log2(const TkDeltaArgs& d) {
 
 bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, const TkPassTab& t, int nrows, hipStream_t s) {
     const int b = attn_bucket(a), ctl = delta_ct_log2(d);
-    /* 168 registers at heads of 128: a CU holds one workgroup of eight waves or three of four.  Eight, the shorter chain of pages, while every workgroup has a CU:
-     * steps of an eight-layer model of 2 + 8 workgroups a row over 400 positions, with eight / four: 25 rows 673 / 674, 32 746 / 715, 40 774 / 741, 52 873 / 815 us; over 20
-     * positions 16 rows 511 / 521, 26 626 / 619.  4 + 16 a row: 12 rows 542 / 538, 16 564 / 543, 25 707 / 671. */
-    const int waves = (int64_t)(attn_row_blocks(a) + d.heads) * nrows > 256 ? 4 : attn_row_waves(a, nrows), threads = 64 * waves;
-    const int rg = threads >> ctl, rpt = rg ? (d.dim + rg - 1) / rg : 1 << 20;
-    if (type != TK_IMG_BF16 || b > 128 || rpt > (waves == 8 ? 8 : 16) || d.vdim > threads) return false;
+    /* Waves for the chains.  168 registers at heads of 128: a CU holds one workgroup of eight waves or three of four.  Eight, one chain each, while every workgroup has a CU;
+     * four beyond, two chains each, so that a row's sums do not depend on how many rows its step has.  Steps of an eight-layer model of 2 + 8 workgroups a row over 400 positions,
+     * with eight / four: 32 rows 770 / 740, 40 805 / 766, 52 897 / 838, 80 1049 / 1006 us; over 20 positions 26 rows 672 / 664.  4 + 16 a row: 16 rows 620 / 603, 25 746 / 719. */
+    const int chains = attn_row_waves(a, nrows), waves = (int64_t)(attn_row_blocks(a) + d.heads) * nrows > 256 ? 4 : chains, threads = 64 * waves;
+    const int rg = 64 * chains >> ctl, rpt = rg ? (d.dim + rg - 1) / rg : 1 << 20;
+    if (type != TK_IMG_BF16 || b > 128 || rpt > (chains == 8 ? 8 : 16) || d.vdim > threads) return false;
     const dim3 grid(attn_row_blocks(a) + d.heads, nrows);
-    const size_t dl = delta_row_lds(d, threads, ctl);
-#define TK_STEP(B, W, R) do { const size_t al = attn_row_lds<B, W>(); \
-        if (attn_full(a)) hipLaunchKernelGGL((k_mixers_step<TkBf16, B, W, R, true>), grid, dim3(threads), al > dl ? al : dl, s, a, d, t, attn_row_blocks(a), ctl); \
-        else hipLaunchKernelGGL((k_mixers_step<TkBf16, B, W, R, false>), grid, dim3(threads), al > dl ? al : dl, s, a, d, t, attn_row_blocks(a), ctl); } while (0)
-    if (b == 64) { if (waves == 8) TK_STEP(64, 8, 8); else TK_STEP(64, 4, 16); }
-    else { if (waves == 8) TK_STEP(128, 8, 8); else TK_STEP(128, 4, 16); }
+    const size_t dl = delta_row_lds(d, 64 * chains, ctl);
+#define TK_STEP(B, W, C, R) do { const size_t al = attn_row_lds<B, C>(); \
+        if (attn_full(a)) hipLaunchKernelGGL((k_mixers_step<TkBf16, B, W, C, R, true>), grid, dim3(threads), al > dl ? al : dl, s, a, d, t, attn_row_blocks(a), ctl); \
+        else hipLaunchKernelGGL((k_mixers_step<TkBf16, B, W, C, R, false>), grid, dim3(threads), al > dl ? al : dl, s, a, d, t, attn_row_blocks(a), ctl); } while (0)
+#define TK_STEP_B(B) do { if (chains == 4) TK_STEP(B, 4, 4, 16); else if (waves == 8) TK_STEP(B, 8, 8, 8); else TK_STEP(B, 4, 8, 8); } while (0)
+    if (b == 64) TK_STEP_B(64);
+    else TK_STEP_B(128);
+#undef TK_STEP_B
 #undef TK_STEP
     return true;
 }
