@@ -1146,7 +1146,7 @@ __global__ __launch_bounds__(256) void k_delta_out(TkDeltaArgs d) {
     }
 }
 
-/* one token of one head: the state is read once and written once, a thread holds RPT rows x 4 columns of it, PARTS times: its sums are those of
+/* one token of one head: the state is read once and written once, a thread holds RPT rows x 4 columns of it, in PARTS row groups whose sums are those of
  * PARTS x THREADS threads (of which the further ones hold rows of the state only: dim, vdim <= 256 <= THREADS).
  * o = S_new^T q = (g S)^T q + (k . q) u, so both reductions over the key rows run on the decayed old state at once. */
 template <typename T, int THREADS, int RPT, int PARTS = 1>
@@ -1156,11 +1156,11 @@ __device__ __forceinline__ void delta_row(const TkDeltaArgs& d, const TkPassTab&
     const bool live = 4 * ct < vp;
     const int seg = t.seg[row], in = t.seg_in[seg], out = t.seg_out[seg];
     float *red = step_lds, *lq = red + 16, *lk = lq + d.dim, *lg = lk + d.dim, *lu = red + 16 + (3 * d.dim + 3) / 4 * 4, *pk = lu + vp, *pq = pk + RG * vp;
-    tk_v4f S[PARTS * RPT]; /* [i of row group rg + RG1 p] at p RPT + i */
+    tk_v4f S[RPT]; /* row group rg + RG1 p has S[p], S[p + PARTS], ... */
     const float* sin = d.state + ((size_t)(in < 0 ? 0 : in) * d.heads + h) * d.dim * vp + 4 * ct;
 #pragma unroll
-    for (int i = 0; i < PARTS * RPT; ++i) {
-        const int e = rg + RG1 * (i / RPT) + RG * (i % RPT);
+    for (int i = 0; i < RPT; ++i) {
+        const int e = rg + RG1 * i;
         S[i] = in >= 0 && live && e < d.dim ? *(const tk_v4f*)(sin + (size_t)e * vp) : tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
     }
     float kq = 0.0f;
@@ -1174,8 +1174,8 @@ __device__ __forceinline__ void delta_row(const TkDeltaArgs& d, const TkPassTab&
     for (int p = 0; p < PARTS; ++p) {
         tk_v4f ak = {0.0f, 0.0f, 0.0f, 0.0f}, aq = ak;
 #pragma unroll
-        for (int i = p * RPT; i < (p + 1) * RPT; ++i) {
-            const int e = rg + RG1 * p + RG * (i % RPT);
+        for (int i = p; i < RPT; i += PARTS) {
+            const int e = rg + RG1 * i;
             if (e < d.dim) { S[i] *= lg[e]; ak += S[i] * lk[e]; aq += S[i] * lq[e]; }
         }
         if (live) { *(tk_v4f*)(pk + (rg + RG1 * p) * vp + 4 * ct) = ak; *(tk_v4f*)(pq + (rg + RG1 * p) * vp + 4 * ct) = aq; }
@@ -1197,8 +1197,8 @@ __device__ __forceinline__ void delta_row(const TkDeltaArgs& d, const TkPassTab&
         const tk_v4f u = *(const tk_v4f*)(lu + 4 * ct);
         float* so = d.state + ((size_t)out * d.heads + h) * d.dim * vp + 4 * ct;
 #pragma unroll
-        for (int i = 0; i < PARTS * RPT; ++i) {
-            const int e = rg + RG1 * (i / RPT) + RG * (i % RPT);
+        for (int i = 0; i < RPT; ++i) {
+            const int e = rg + RG1 * i;
             if (e < d.dim) *(tk_v4f*)(so + (size_t)e * vp) = S[i] + u * lk[e];
         }
     }
@@ -1904,7 +1904,7 @@ bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, 
 #define TK_STEP(B, W, C, R) do { const size_t al = attn_row_lds<B, C>(); \
         if (attn_full(a)) hipLaunchKernelGGL((k_mixers_step<TkBf16, B, W, C, R, true>), grid, dim3(threads), al > dl ? al : dl, s, a, d, t, attn_row_blocks(a), ctl); \
         else hipLaunchKernelGGL((k_mixers_step<TkBf16, B, W, C, R, false>), grid, dim3(threads), al > dl ? al : dl, s, a, d, t, attn_row_blocks(a), ctl); } while (0)
-#define TK_STEP_B(B) do { if (chains == 4) TK_STEP(B, 4, 4, 16); else if (waves == 8) TK_STEP(B, 8, 8, 8); else TK_STEP(B, 4, 8, 8); } while (0)
+#define TK_STEP_B(B) do { if (chains == 4) TK_STEP(B, 4, 4, 16); else if (waves == 8) TK_STEP(B, 8, 8, 8); else TK_STEP(B, 4, 8, 16); } while (0)
     if (b == 64) TK_STEP_B(64);
     else TK_STEP_B(128);
 #undef TK_STEP_B
