@@ -271,6 +271,10 @@ TK_API TK_NODISCARD tk_error_code_t tk_mi355x_f32_to_f16(int device, const float
  * stages of a block, parts of k; stages = 0: the kernel for few rows.  No GPU involved. */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]);
 
+/* test hook: such a product of float32 matrices x [rows][K], w [N][K] (rounded to bf16 where f32 is 0) with up to max_slabs partial results: out [max_slabs][rows][N], of
+ * which *slabs are written. */
+TK_API TK_NODISCARD tk_error_code_t tk_mi355x_gemm_image(int device, int f32, int rows, int N, int K, int max_slabs, const float* x, const float* w, float* out, int* slabs);
+
 #ifdef __cplusplus
 }
 #endif

@@ -207,7 +207,7 @@ def close(got, want, tol):
 
 
 def image_parts(f32, rows, n, k):
-    """in how many parts of k a product of few rows is made whose consumer adds up to eight"""
+    """by how many workgroups a column tile a product of few rows is made whose consumer adds up to eight slabs"""
     import ctypes as C
     import trackiellm_amd as tk
     form = (C.c_int * 4)()

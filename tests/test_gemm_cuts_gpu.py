@@ -86,3 +86,29 @@ def test_norms_inside_products_of_a_few_rows(gpu, width):
         i2, m2, e2, l2 = asr.transcribe_tokens(pcm[:n], 5)
         assert np.array_equal(i2, ids[:n]) and np.array_equal(l2.view(np.uint32), logits[:n].view(np.uint32))
         assert np.array_equal(m2.view(np.uint32), mel[:n].view(np.uint32)) and np.array_equal(e2.view(np.uint32), enc[:n].view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("N,K", [(2048, 2048), (528, 2085), (1040, 4160), (50, 8192), (2033, 8190), (16, 3000)])
+@pytest.mark.parametrize("rows", [1, 16, 17, 32, 33, 48, 49, 64])
+def test_slabs_of_a_product_of_few_rows_add_up_to_the_whole(gpu, rows, N, K, f32):
+    """two workgroups a column tile, their slabs added in order: the bits of one workgroup, at one to four tiles of rows, columns that fill no tile, k pieces of every
+    remainder over the waves"""
+    rng = np.random.default_rng(rows + N + K)
+    x, w = rng.normal(0, 1, (rows, K)).astype(np.float32), (rng.normal(0, 1, (N, K)) * K ** -0.5).astype(np.float32)
+    p = lambda t: t.ctypes.data_as(C.c_void_p)
+
+    def product(most):
+        out, n = np.full((8, rows, N), np.nan, np.float32), C.c_int(0)
+        gpu.check(gpu.lib().tk_mi355x_gemm_image(0, f32, rows, N, K, most, p(x), p(w), p(out), C.byref(n)))
+        assert np.isnan(out[n.value:]).all()
+        s = out[0]
+        for i in range(1, n.value):
+            s = s + out[i]
+        return s, n.value
+    whole, one = product(1)
+    parts, n = product(8)
+    assert one == 1 and n > 1
+    assert np.array_equal(parts.view(np.uint32), whole.view(np.uint32))
+    assert np.linalg.norm(whole - x.astype(np.float64) @ w.astype(np.float64).T) < (1e-5 if f32 else 1e-2) * np.linalg.norm(whole)

@@ -432,7 +432,7 @@ def test_products_in_large_blocks(gpu, width, ff, rows, dtype, tol):
 @pytest.mark.parametrize("dtype,tol", [("float32", F32), ("bfloat16", 0.007)])
 @pytest.mark.parametrize("width,ff", [(528, 2085), (1040, 2048), (2048, 2400)])
 def test_products_of_few_rows_in_parts_of_k(gpu, width, ff, dtype, tol):
-    """passes of 1 .. 64 rows (one to four tiles of them), whose down product (and, at 2048, the mixers' too) is made in two parts of k, of even and odd numbers of
+    """passes of 1 .. 64 rows (one to four tiles of them), whose down product (and, at 2048, the mixers' too) is made by two workgroups a column tile, of even and odd numbers of
     k tiles, against the same rows in one pass of 150, which takes another kernel; tolerances as above"""
     n = width // 16
     f32 = dtype == "float32"

@@ -278,6 +278,36 @@ tk_error_code_t tk_mi355x_f32_to_f16(int device, const float* x, int n, uint16_t
     return ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
 }
 
+tk_error_code_t tk_mi355x_gemm_image(int device, int f32, int rows, int N, int K, int max_slabs, const float* x, const float* w, float* out, int* slabs) {
+    if (rows < 1 || N < 1 || K < 1 || rows > 16384 || N > 65536 || K > 65536 || max_slabs < 1 || max_slabs > 8 || !x || !w || !out || !slabs) return TK_ERROR_INVALID_ARGUMENT;
+    int n = 0;
+    if (hipGetDeviceCount(&n) != hipSuccess || n <= 0) return TK_ERROR_GPU_DEVICE_NOT_FOUND;
+    if (device < 0 || device >= n || hipSetDevice(device) != hipSuccess) return TK_ERROR_INVALID_ARGUMENT;
+    const int type = f32 ? TK_IMG_F32 : TK_IMG_BF16, kp = tk_img_pad_k(type, K), np = (N + 15) / 16 * 16;
+    const size_t slab = ((size_t)rows * N + 3) / 4 * 4;
+    TkImgGemm g{};
+    g.type = type; g.K = kp; g.N = np; g.nrows = rows; g.ldc = g.n_valid = N; g.max_slabs = max_slabs; g.slab_floats = slab;
+    float *dx = nullptr, *dw = nullptr, *dy = nullptr;
+    void *ix = nullptr, *iw = nullptr;
+    auto put = [](float** d, const float* h, size_t n) { return hipMalloc((void**)d, n * 4) == hipSuccess && hipMemcpy(*d, h, n * 4, hipMemcpyHostToDevice) == hipSuccess; };
+    auto image = [&](void** img, const float* src, int64_t r) {
+        const size_t bytes = tk_img_bytes(type, r, K);
+        if (hipMalloc(img, bytes) != hipSuccess || hipMemset(*img, 0, bytes) != hipSuccess) return false;
+        tk_launch_put_image(type, src, 1, r, K, *img, kp / tk_img_kt(type), 0, 0, -1, nullptr);
+        return hipGetLastError() == hipSuccess;
+    };
+    bool ok = put(&dx, x, (size_t)rows * K) && put(&dw, w, (size_t)N * K) && image(&ix, dx, rows) && image(&iw, dw, N) &&
+              hipMalloc((void**)&dy, slab * max_slabs * 4) == hipSuccess && !tk_gemm_image_prepare_device();
+    if (ok) {
+        g.w = iw; g.a = ix; g.out = dy;
+        ok = !tk_launch_gemm_image(g, nullptr, slabs) && hipGetLastError() == hipSuccess && hipDeviceSynchronize() == hipSuccess;
+        for (int i = 0; ok && i < *slabs; ++i) ok = hipMemcpy(out + (size_t)i * rows * N, dy + i * slab, (size_t)rows * N * 4, hipMemcpyDeviceToHost) == hipSuccess;
+    }
+    void* ptrs[] = {dx, dw, dy, ix, iw};
+    for (void* q : ptrs) if (q) (void)hipFree(q);
+    return ok ? TK_SUCCESS : TK_ERROR_GPU_ROCM_ERROR;
+}
+
 tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int swiglu, int experts, int top, int max_slabs, int form[4]) {
     if (rows <= 0 || N <= 0 || K <= 0 || experts < 0 || (experts > 0 && (top < 1 || top > experts)) || !form) return TK_ERROR_INVALID_ARGUMENT;
     const int to = swiglu ? 32 : 16;

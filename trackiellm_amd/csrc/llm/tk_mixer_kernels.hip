@@ -171,7 +171,16 @@ __global__ __launch_bounds__(512) void k_post_norm(TkSubOut o, TkNorm norm, TkNo
         }
     } else {
         y.load(o.y + (size_t)row * o.ld, width);
-        for (int i = 1; i < o.slabs; ++i) {
+        int i = 1;
+        if (NV <= 2)
+            for (; i + 3 < o.slabs; i += 4) { /* four slabs, one trip to the caches */
+                Row<VEC, NV> w[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) w[j].load(o.y + (i + j) * o.slab_floats + (size_t)row * o.ld, width);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) y.each(width, [&](int g, int e, int) { y.v[g][e] += w[j].v[g][e]; });
+            }
+        for (; i < o.slabs; ++i) {
             z.load(o.y + i * o.slab_floats + (size_t)row * o.ld, width);
             y.each(width, [&](int g, int e, int) { y.v[g][e] += z.v[g][e]; });
         }

@@ -64,7 +64,8 @@ struct TkImgGemm {
 /* nullptr, or why the arguments are refused (nothing is launched then) */
 const char* tk_launch_gemm_image(const TkImgGemm& g, hipStream_t s, int* slabs = nullptr);
 
-/* rows, columns and LDS stages of the blocks that a launch with these sizes takes, and its k parts; stages = 0: the skinny kernel.  Reads no pointer. */
+/* rows, columns and LDS stages of the blocks that a launch with these sizes takes, and its k parts (few rows: workgroups
+ * of a column tile); stages = 0: the skinny kernel.  Reads no pointer. */
 void tk_gemm_image_form(const TkImgGemm& g, int form[4]);
 
 /* row blocks of `rows` rows sent to `top` of `experts` each: tiles of a block, the most there can be, and how many to expect (an expert's last block is half

@@ -47,16 +47,16 @@ __device__ __forceinline__ void store_act(const TkImgGemm& a, int64_t row, int n
 }
 
 /* ---- skinny: MT M-tiles of rows, NT column tiles per workgroup, K interleaved over the waves in pieces of U tiles ----
- * Loads of three M-tiles are three (33 .. 48 rows; four, one of them twice: 40 rows x 2048 x 16384 gate and up 17.2 -> 15.8 us, x 32000 34.2 -> 28.6). */
-template <typename T, int MT, int NT, int WAVES, bool SWIGLU, bool GROUPED>
+ * Loads of three M-tiles are three (33 .. 48 rows; four, one of them twice: 40 rows x 2048 x 16384 gate and up 17.2 -> 15.8 us, x 32000 34.2 -> 28.6).
+ * PARTS = 2: the waves of a column tile in two workgroups (skinny_parts), each wave with two pieces on their way.  The first workgroup adds its waves up in slab 0, each wave
+ * of the second has a slab of its own: added in ascending order, they are the sum that one workgroup of all waves makes. */
+template <typename T, int MT, int NT, int WAVES, int PARTS, bool SWIGLU, bool GROUPED>
 __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
-    constexpr int U = MT >= 3 ? 2 : 4;
+    static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && !SWIGLU && !GROUPED), "slabs are of plain products");
+    constexpr int U = MT >= 3 ? 2 : 4, STEP = PARTS * WAVES * U, AHEAD = PARTS;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ktiles = a.K / TkImg<T>::KT;
-    /* one part of k or two (skinny_parts); a division by the number of parts took 0.4 us of every launch */
-    const int k0 = !GROUPED && blockIdx.z ? ktiles >> 1 : 0, k1 = !GROUPED && gridDim.z > 1 && blockIdx.z == 0 ? ktiles >> 1 : ktiles;
-    if (!GROUPED && !SWIGLU) a.out += blockIdx.z * a.slab_floats;
     int m0 = blockIdx.y * MT, mlive = (a.nrows + 15) / 16 - m0;
     const uint8_t* wbase = (const uint8_t*)a.w;
     if (GROUPED) {
@@ -79,38 +79,53 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) acc[n][m] = tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
     const tk_v4u zero = {0, 0, 0, 0};
-    tk_v4u wq[U][NT], aq[U][MT];
+    tk_v4u wq[AHEAD][U][NT], aq[AHEAD][U][MT];
     /* tiles past the end re-read the last one against a zero activation: no branch around a load */
-    auto load = [&](int c) {
+    auto load = [&](int p, int c) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int kt = c + u < k1 ? c + u : k1 - 1;
+            const int kt = c + u < ktiles ? c + u : ktiles - 1;
 #pragma unroll
-            for (int n = 0; n < NT; ++n) wq[u][n] = ldg16_stream(wp[n] + (size_t)kt * 1024);
+            for (int n = 0; n < NT; ++n) wq[p][u][n] = ldg16_stream(wp[n] + (size_t)kt * 1024);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) aq[u][m] = ldg16(ap[m] + (size_t)kt * 1024);
+            for (int m = 0; m < MT; ++m) aq[p][u][m] = ldg16(ap[m] + (size_t)kt * 1024);
         }
     };
-    int c = k0 + wave * U;
-    if (c < k1) load(c);
-    while (c < k1) {
-        tk_v4u w0[U][NT], a0[U][MT];
+    int c = ((PARTS > 1 ? (int)blockIdx.z * WAVES : 0) + wave) * U;
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
+    for (int p = 0; p < AHEAD; ++p)
+        if (PARTS > 1 || c < ktiles) load(p, c + p * STEP);
+    while (c < ktiles) {
 #pragma unroll
-            for (int n = 0; n < NT; ++n) w0[u][n] = wq[u][n];
+        for (int p = 0; p < AHEAD; ++p) {
+            tk_v4u w0[U][NT], a0[U][MT];
 #pragma unroll
-            for (int m = 0; m < MT; ++m) a0[u][m] = c + u < k1 ? aq[u][m] : zero;
+            for (int u = 0; u < U; ++u) {
+#pragma unroll
+                for (int n = 0; n < NT; ++n) w0[u][n] = wq[p][u][n];
+#pragma unroll
+                for (int m = 0; m < MT; ++m) a0[u][m] = c + u < ktiles ? aq[p][u][m] : zero;
+            }
+            const int next = c + AHEAD * STEP;
+            if (PARTS > 1 || next < ktiles) load(p, next);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) acc[n][m] = TkImg<T>::mma(w0[u][n], a0[u][m], acc[n][m]);
+            c += STEP;
+            if (c >= ktiles) break;
         }
-        const int next = c + WAVES * U;
-        if (next < k1) load(next);
+    }
+    if (PARTS > 1 && blockIdx.z) {
+        a.out += (size_t)(1 + wave) * a.slab_floats;
 #pragma unroll
-        for (int u = 0; u < U; ++u)
-#pragma unroll
-            for (int n = 0; n < NT; ++n)
-#pragma unroll
-                for (int m = 0; m < MT; ++m) acc[n][m] = TkImg<T>::mma(w0[u][n], a0[u][m], acc[n][m]);
-        c = next;
+        for (int m = 0; m < MT; ++m) {
+            const int64_t row = (int64_t)(m0 + m) * 16 + (lane & 15);
+            if (m < mlive && row < a.nrows) store_f32<T>(a, row, n0 * 16 + 4 * (lane >> 4), acc[0][m]);
+        }
+        return;
     }
     /* partial sums of the waves, ascending */
     tk_v4f* red = (tk_v4f*)lds;
@@ -342,11 +357,14 @@ WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
     return best;
 }
 
-/* A product of few rows in two parts of k, where its column tiles leave half of the CUs idle and each part is a piece for every wave: 40 rows x 2048 x 8192 19.7 ->
- * 13.0 us, x 2048 7.2 -> 5.9 (three parts 14.8 and 6.6, four 13.0 and 6.0, eight 13.4 and 7.3); steps of a 2048-wide model at 1, 16, 64 rows 488 -> 451, 540 -> 506,
- * 909 -> 828 us.  256 column tiles: 486 -> 489, 532 -> 537, 920 -> 920.  The rows do not enter, so that a row's result does not depend on the others of its step. */
+/* A product of few rows by two workgroups a column tile, in TK_SKINNY_SLABS slabs, where its column tiles leave half of the CUs idle and there is work for every wave.  Steps of
+ * an eight-layer model 2048 wide with one workgroup / two: 1 row 539 / 529 us, 16 rows 599 / 590, 40 rows 816 / 781, 64 rows 894 / 836; three and four pieces of a wave on their
+ * way are no quicker than two.  256 column tiles (4096 wide): 1 row 531 / 546, 40 rows 822 / 838.  The rows do not enter, so that a row's result does not depend on the others
+ * of its step. */
+#define TK_SKINNY_WAVES 8
+#define TK_SKINNY_SLABS (1 + TK_SKINNY_WAVES / 2)
 int skinny_parts(const TkImgGemm& g, bool swiglu, bool grouped) {
-    return !swiglu && !grouped && g.max_slabs > 1 && g.N / 16 <= 128 && g.K / tk_img_kt(g.type) >= 64 ? 2 : 1;
+    return !swiglu && !grouped && g.max_slabs >= TK_SKINNY_SLABS && g.N / 16 <= 128 && g.K / tk_img_kt(g.type) >= 64 ? 2 : 1;
 }
 
 template <typename T, bool SWIGLU, bool GROUPED>
@@ -357,13 +375,15 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
         /* GROUPED: one block per table entry */
         const int gy = GROUPED ? g.max_blocks : 1;
         const int parts = skinny_parts(g, SWIGLU, GROUPED);
-        if (slabs) *slabs = parts;
-#define TK_SK(MT, NT, WV) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, gy, parts), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
-#define TK_SKM(NT, WV) do { if (mtiles <= 1) TK_SK(1, NT, WV); else if (mtiles <= 2) TK_SK(2, NT, WV); else if (mtiles <= 3) TK_SK(3, NT, WV); else TK_SK(4, NT, WV); } while (0)
+        if (slabs) *slabs = parts > 1 ? TK_SKINNY_SLABS : 1;
+#define TK_SK(MT, NT, WV, P) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, P, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, gy, P), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
+#define TK_SKM(NT, WV, P) do { if (mtiles <= 1) TK_SK(1, NT, WV, P); else if (mtiles <= 2) TK_SK(2, NT, WV, P); else if (mtiles <= 3) TK_SK(3, NT, WV, P); else TK_SK(4, NT, WV, P); } while (0)
         if (SWIGLU || ntiles * gy >= 1024) {
-            if (ntiles * gy >= 2048) TK_SKM(2, 4); else TK_SKM(2, 8);
+            if (ntiles * gy >= 2048) TK_SKM(2, 4, 1); else TK_SKM(2, 8, 1);
+        } else if (parts > 1) {
+            if constexpr (!SWIGLU && !GROUPED) TK_SKM(1, TK_SKINNY_WAVES / 2, 2);
         } else {
-            TK_SKM((SWIGLU ? 2 : 1), 8);
+            TK_SKM((SWIGLU ? 2 : 1), TK_SKINNY_WAVES, 1);
         }
 #undef TK_SKM
 #undef TK_SK
