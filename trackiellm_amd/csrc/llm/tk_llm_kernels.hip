@@ -1234,17 +1234,17 @@ __device__ __forceinline__ void unpack_q6_x32(const FragQ6& f0, const FragQ6& f1
     o.dmin = 0.0f;
 }
 
-/* s_waitcnt vmcnt(n) alone (expcnt / lgkmcnt untouched): until all but this wave's n youngest vector-memory operations are done.  The
+/* s_waitcnt vmcnt(N) alone (expcnt / lgkmcnt untouched): until all but this wave's N youngest vector-memory operations are done.  The
  * LDS-DMA pieces of a chunk are invisible to the compiler's own wait insertion, so the ring is guarded by hand. */
-__device__ __forceinline__ void wait_vmcnt(int n) {
-#define TK_VMW(k) case k: __builtin_amdgcn_s_waitcnt(0x0F70 | ((k) & 15) | (((k) >> 4) << 14)); break;
-    switch (n) {
-        TK_VMW(0) TK_VMW(1) TK_VMW(2) TK_VMW(3) TK_VMW(4) TK_VMW(5) TK_VMW(6) TK_VMW(7) TK_VMW(8) TK_VMW(9) TK_VMW(10) TK_VMW(11) TK_VMW(12)
-        TK_VMW(13) TK_VMW(14) TK_VMW(15) TK_VMW(16) TK_VMW(17) TK_VMW(18) TK_VMW(19) TK_VMW(20) TK_VMW(21) TK_VMW(22) TK_VMW(23) TK_VMW(24)
-        TK_VMW(25) TK_VMW(26) TK_VMW(27) TK_VMW(28)
-        default: __builtin_amdgcn_s_waitcnt(0x0F70); break;
-    }
-#undef TK_VMW
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N <= 63, "the counter has six bits");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
+/* until all but its `left` youngest batches of N requests are done; left <= MOST */
+template <int N, int MOST> __device__ __forceinline__ void wait_batches(int left) {
+    if constexpr (MOST == 0) wait_vmcnt<0>();
+    else if (left >= MOST) wait_vmcnt<N * MOST>();
+    else wait_batches<N, MOST - 1>(left);
 }
 
 #define TK_MFMA32 __builtin_amdgcn_mfma_i32_32x32x32_i8
@@ -1801,7 +1801,6 @@ __global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __
     const int nchunk = (T + CH - 1) / CH;
     const int total = 2 * nchunk;              /* the stream: K chunks 0 .. nchunk - 1, then V chunks 0 .. nchunk - 1 */
     const int last_row = max_ctx - 1;
-    const int ppw = slot_bytes / 4096;         /* DMA pieces per wave and chunk */
     const int ppr = rb / 16;
     auto issue = [&](int j) { /* chunk j of the stream into slot j % SLOTS; always issued (a chunk with nothing cached yet re-reads clamped rows) */
         const bool is_k = j < nchunk;
@@ -1811,8 +1810,8 @@ __global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __
     /* before touching chunk j: all but the chunks issued after it have landed; everybody is done with chunk j - 1, whose slot takes
      * chunk j + SLOTS - 1 */
     auto acquire = [&](int j) {
-        const int ahead = total - 1 - j < SLOTS - 2 ? total - 1 - j : SLOTS - 2;
-        wait_vmcnt(ahead * ppw);
+        static_assert(SLOTS == 2, "two slots: nothing is issued behind the chunk that is waited for");
+        wait_vmcnt<0>();
         __syncthreads();
         if (j + SLOTS - 1 < total) issue(j + SLOTS - 1);
     };
@@ -2432,7 +2431,7 @@ __global__ __launch_bounds__((256 / HD) * 256) void k_attention_prefill(const fl
  *                       written to a [row][head][position] fp32 buffer;
  *   k_att_pv_chain      workgroup = one wave = (row, head, class j): row maximum (order-free), e = exp(s - m), then the canonical class
  *                       chain — positions j, j + 4, ... ascending, acc = fma(e, v, acc), l = l + e — as ONE sequential chain per lane (a lane
- *                       owns two dims), 192 value rows requested ahead; partial outputs and denominators to a scratch buffer;
+ *                       owns two dims), up to 192 value rows on their way; partial outputs and denominators to a scratch buffer;
  *   k_att_pv_join       the four classes joined in order, division, Q8 quantisation; in passes whose mat-vec launches make their own input the
  *                       o projection does this (TkGemvArgs::fuse 3): a launch less, 0.1 us of the other.
  * Bit-identical to k_attention / k_attention_narrow (tests/test_llm_attention_gpu.py: the decode cases past 2 048 positions run both).
@@ -2531,11 +2530,12 @@ __global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict
 
 /* One wave = one (row, head, class) chain: 128 x rows workgroups, so the value rows arrive through as many CUs' memory pipes (a CU pulls ~25 - 40 GB/s:
  * sixteen workgroups of eight chains each took 29 us at 2 048 positions).  The class's value rows come by LDS-DMA, 1 KiB a request, three chunks of 64
- * rows in flight — the whole class up to 768 positions; two above four rows — and are requested right behind the scores; one 4-byte load a row and lane, the former way, held 64
- * rows of two register sets and a wave can have no more than 63 requests on their way.  A lane owns two dims (head_dim 64: the upper half-wave mirrors the
- * lower). With it, the keys requested before q's slabs and the join in the
+ * rows in flight, two above four rows; one 4-byte load a row and lane, the former way, held 64 rows of two register sets and a wave can have no more than 63 requests
+ * on their way.  The first chunks are requested right behind the scores and waited for with them; from then on a chunk's wait leaves the chunks behind it on their way
+ * (waiting for all: 1 row at 3000 positions 2.306 -> 2.274 ms a call of a 32-layer model, at 4000 2.481 -> 2.436, 4 rows at 3000 2.927 -> 2.855; up to 900 the same).  A lane
+ * owns two dims (head_dim 64: the upper half-wave mirrors the lower).  With it, the keys requested before q's slabs and the join in the
  * o projection a step of one row takes 1.742 ms at 448 positions (fused kernel 1.852);
- * 4096-position window, before and now: 1 row at 600 1.975 -> 1.768, at 3000 2.527 -> 2.223, 4 rows at 900 2.515 -> 2.351, 8 rows at 900 2.627 -> 2.507. */
+ * 4096-position window, one load a row and lane / LDS-DMA: 1 row at 600 1.975 / 1.768, at 3000 2.527 / 2.223, 4 rows at 900 2.515 / 2.351, 8 rows at 900 2.627 / 2.507. */
 #define TK_PV_ROWS 64
 template <int HD, int SLOTS>
 __global__ __launch_bounds__(64) void k_att_pv_chain(const float* __restrict__ scores, const uint16_t* __restrict__ vcache, const int32_t* __restrict__ seq,
@@ -2589,7 +2589,7 @@ __global__ __launch_bounds__(64) void k_att_pv_chain(const float* __restrict__ s
     float acc0 = 0.0f, acc1 = 0.0f, l = 0.0f;
     for (int c = 0; c < nch; ++c) {
         const int ahead = nch - 1 - c < SLOTS - 1 ? nch - 1 - c : SLOTS - 1;
-        wait_vmcnt(ahead * NI);
+        wait_batches<NI, SLOTS - 1>(ahead);
         __syncthreads();
         const uint8_t* vp = att_lds + (c % SLOTS) * TK_PV_ROWS * RB + dl * 4;
         const float* ep = ebuf + c * TK_PV_ROWS;
@@ -2653,7 +2653,7 @@ void tk_launch_attention_long(const float* partial, int ks, int n_total, const f
     const TkAttentionParts parts = tk_attention_long_parts(scores, n_head, head_dim, max_ctx);
     float *pv_part = parts.pv, *l_part = parts.l;
     const dim3 gc(TK_ATT_TSPLIT, n_head, nrows);
-    const int slots = nrows > 4 ? 2 : 3; /* 32 KB: the four workgroups a CU of eight rows are resident together */
+    const int slots = nrows > 4 ? 2 : 3; /* 32 KB: the four workgroups a CU of eight rows are resident together (calls with two / three: 8 rows at 900 positions 2.62 / 2.79 ms, at 3000 3.37 / 3.74, 6 at 900 2.54 / 2.56) */
     const size_t lds = (size_t)slots * TK_PV_ROWS * head_dim * 2 + ((size_t)(max_ctx + 3) / 4 + TK_PV_ROWS) * sizeof(float);
     if (head_dim == 128) {
         hipLaunchKernelGGL((k_att_scores_long<128>), gs, dim3(256), 0, s, partial, ks, n_total, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
