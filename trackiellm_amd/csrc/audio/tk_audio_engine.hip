@@ -511,7 +511,7 @@ struct TkAudioGpuOps {
             t.c_img = cimg;
             t.out = nullptr; /* (fc2 has tiles: its K is a multiple of 128) */
         }
-        if (!tk_launch_gemm_tiled(t, s)) tk_launch_gemm(g, s); /* not reached: tk_tiled_gemm_applies() admits only shapes the launcher takes */
+        if (!tk_launch_gemm_tiled(t, s)) a->launch_error = "tiled GEMM launch refused"; /* not reached: tk_tiled_gemm_applies() admits only shapes the launcher takes */
         if (emit_img) { /* the image pair stays allocated from pk.mark up; the upper one is now the live image */
             pk.img = cimg; pk.A = g.C; pk.M = g.M; pk.K = g.N; pk.lda = g.ldc; pk.live = true;
             norm.live = false;
