@@ -699,6 +699,7 @@ static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
 bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p) {
     static const struct { int mi, ni; } forms[] = {{0, 0}, {1, 1}, {2, 1}};
     if (!tw_valid(a) || form < 1 || form > 2 || (a.wbytes == 4 && a.ks != 1) || a.ln_x || (a.c_img && (a.wbytes == 2 || a.out || a.residual)) || a.K % (128 * a.ks)) return false;
+    if (a.ks > 1 && (a.bias || a.residual || a.act || a.add_zero_bias)) return false; /* parts of k are sums alone */
     const int per = 2 * forms[form].ni;
     for (int i = 0; i < a.nseg; ++i)
         if (a.row_tiles[i] % per || (a.per_seg && a.seg_n[i] != a.row_tiles[i] * 16)) return false;
