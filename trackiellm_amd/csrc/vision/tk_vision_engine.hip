@@ -295,6 +295,15 @@ struct TkGpuOps {
         else hipLaunchKernelGGL((k_stem<false>), grid, dim3(256), 0, s, a, frame_bytes, x.p, x.H, x.W, y.H, y.W, d->model->wp[0], d->model->b[0], sp.act, y.p, y.ld);
         return true;
     }
+    /* the network's input tensor, of frames that no stem kernel takes */
+    void preprocess(const TkT& x) {
+        for (int b = 0; frames && b < x.B; ++b) {
+            TkPreprocessArgs f = *frames;
+            f.src += frame_bytes * b;
+            f.dst = x.p + (size_t)b * x.H * x.W * 3;
+            tk_launch_preprocess(f, s);
+        }
+    }
     /* A concatenation's copied and upsampled parts are not written: the convolution behind it reads them where they are (two sources).  Any other reader has them
      * written first. */
     struct Part { TkT x, y; int shift; };
@@ -389,7 +398,10 @@ struct TkGpuOps {
     }
     void run(const TkT& x, int idx, const TkT& y, const TkT* res) {
         const TkConvSpec& sp = d->model->specs[idx];
-        if (idx == 0 && stem(x, y)) return;
+        if (idx == 0) {
+            if (stem(x, y)) return;
+            preprocess(x);
+        }
         if (direct(x, idx, y, res)) return;
         settle(x);
         if (res) settle(*res);
@@ -789,17 +801,16 @@ bool TkDetector::detect(int B, const uint8_t* const* frames, uint32_t w, uint32_
     a.src = frame_dev; a.in_w = w; a.in_h = h; a.in_stride = stride; a.bpp = bpp;
     a.dst = input; a.out_w = in_w; a.out_h = in_h; a.nhwc = model->generic ? 0 : 1; /* a file's graph takes planar NCHW */
     for (int c = 0; c < 3; ++c) { a.mean[c] = mean[c]; a.std_dev[c] = std_dev[c]; }
-    const bool in_stem = !model->generic && model->wp[0]; /* else as a launch of its own per frame */
     for (int b = 0; b < B; ++b) {
         HIPQ(hipMemcpyAsync(frame_dev + fb * b, frames[b], fb, hipMemcpyHostToDevice, stream));
-        if (in_stem) continue;
+        if (!model->generic) continue; /* the network takes the frames (TkGpuOps::run) */
         TkPreprocessArgs f = a;
         f.src = frame_dev + fb * b;
         f.dst = input + (size_t)b * in_h * in_w * 3;
         tk_launch_preprocess(f, stream);
     }
     last_w = w; last_h = h; last_stride = stride; last_B = B;
-    if (!enqueue(B, in_stem ? &a : nullptr)) return false;
+    if (!enqueue(B, model->generic ? nullptr : &a)) return false;
     return fetch(B, out);
 }
 
