@@ -136,6 +136,11 @@ TK_API TK_NODISCARD tk_error_code_t tk_mi355x_detector_set_max_batch(tk_object_d
  * frame does not depend on the frames that share its job (the kernel that evaluates a layer is chosen by the layer, never by the batch). */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_detector_set_fast_contraction(tk_object_detector_t* detector, int on);
 TK_API void tk_mi355x_detector_share_stats(const tk_object_detector_t* detector, uint64_t* handles, uint64_t* batches, uint64_t* frames, uint64_t* widest);
+
+/* test hook for the shared detector's waiting (csrc/common/tk_arrivals.h), on a clock of its own: `n` requests, request i of caller[i] not before at[i] microseconds nor
+ * before that caller's last one is served; a job of b requests takes job_us + b frame_us.  Returns the number of jobs, their sizes and when they began in sizes / begins [n];
+ * -1: bad arguments.  No GPU involved. */
+TK_API int tk_mi355x_arrivals_simulate(int callers, int wait_us, int job_us, int frame_us, int max_batch, int n, const int* caller, const int64_t* at, int* sizes, int64_t* begins);
 /* ONNX detector file (tk_object_detector_config_t.model_path, src/vision/tk_object_detector.c:93-152): parse the Conv initialisers
  * (no ONNX Runtime, no GPU) and check them against the YOLOv8n graph this path runs; n_convs / n_params optional */
 TK_API TK_NODISCARD tk_error_code_t tk_mi355x_onnx_probe(const char* path, int32_t* n_convs, int64_t* n_params);

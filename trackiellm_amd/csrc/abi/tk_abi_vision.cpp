@@ -28,12 +28,14 @@ static std::string file_identity(const std::string& path) {
            std::to_string((unsigned long long)st.st_ino);
 }
 
-/* ---- per-model-file registry (DESIGN.md 5): every tk_object_detector_t opened on the same file / device / geometry shares ONE set of weights
+/* ---- per-model-file registry: every tk_object_detector_t opened on the same file / device / geometry shares ONE set of weights
  * and ONE batched engine.  The reference's API is one frame per call and per handle (src/vision/tk_object_detector.c:182-219); K cortex
  * handles that each own a detector at batch 1 ran K small networks side by side.  Here a call enqueues its frame, a scheduler thread coalesces
  * the frames that are waiting (same geometry and thresholds) into one batched detect() — the way csrc/llm/tk_llm_batcher does for runners — and
  * every caller gets exactly what it would get alone: the engine's arithmetic is per frame (tests/test_vision_gpu.py: batch == singles).
  * The per-box attributes of tk_vision_pipeline_process_frame run inside the same job, while the batch's frames are still on the device. */
+#include "../common/tk_arrivals.h"
+
 #include <chrono>
 #include <condition_variable>
 #include <deque>
@@ -41,6 +43,7 @@ static std::string file_identity(const std::string& path) {
 #include <thread>
 
 #define TK_DET_SHARED_MAX_BATCH 32
+#define TK_DET_SHARED_WAIT_US 400 /* for the others of a burst: less than the network takes for a frame */
 
 struct DetReq {
     const uint8_t* frame = nullptr;
@@ -49,6 +52,7 @@ struct DetReq {
     bool fast = false;           /* tk_mi355x_detector_set_fast_contraction: requests of one kind share a job */
     bool want_attr = false;      /* classify the first `max_objects` boxes (0 = all) while the frame is resident */
     uint32_t max_objects = 0;
+    int caller = -1;             /* TkArrivals: the handle */
     std::vector<TkDetection> dets;
     std::vector<int32_t> color, door;
     bool have_attr = false, ok = false, done = false;
@@ -71,6 +75,8 @@ struct SharedDetector {
     std::thread th;
     bool stop = false;
     int handles = 0;
+    TkArrivals arrivals{TK_DET_SHARED_WAIT_US};
+    static int64_t now_us() { return std::chrono::duration_cast<std::chrono::microseconds>(std::chrono::steady_clock::now().time_since_epoch()).count(); }
     uint64_t n_batches = 0, n_frames = 0, widest = 0;
 
     ~SharedDetector() {
@@ -96,18 +102,17 @@ struct SharedDetector {
     }
     void run() {
         std::unique_lock<std::mutex> lk(mu);
-        int expect = 1;
         for (;;) {
             cv_req.wait(lk, [&] { return stop || !q.empty(); });
             if (stop) break;
-            /* give the other callers a moment to arrive, as many as there were last time: those of the last job and those that came while it ran.  (Waiting for every
-             * handle there is made a lone caller beside idle handles wait the 400 us each time, as long as half a network of one frame.) */
-            if (expect > 1) {
-                const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(400);
-                while ((int)q.size() < expect && !stop)
-                    if (cv_req.wait_until(lk, until) == std::cv_status::timeout) break;
-                if (stop) break;
-            }
+            const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(arrivals.wait_us());
+            const int64_t from = now_us();
+            while (arrivals.awaited(from) > 0 && (int)q.size() < TK_DET_SHARED_MAX_BATCH && !stop)
+                if (cv_req.wait_until(lk, until) == std::cv_status::timeout) {
+                    arrivals.waited_in_vain(from);
+                    break;
+                }
+            if (stop) break;
             std::vector<DetReq*> job;
             DetReq* first = q.front();
             for (auto it = q.begin(); it != q.end() && (int)job.size() < TK_DET_SHARED_MAX_BATCH;) {
@@ -154,8 +159,11 @@ struct SharedDetector {
             n_batches++;
             n_frames += job.size();
             if (job.size() > widest) widest = job.size();
-            for (DetReq* r : job) r->done = true;
-            expect = (int)(job.size() + q.size()) < TK_DET_SHARED_MAX_BATCH ? (int)(job.size() + q.size()) : TK_DET_SHARED_MAX_BATCH;
+            const int64_t at = now_us();
+            for (DetReq* r : job) {
+                r->done = true;
+                arrivals.served(r->caller, at);
+            }
             cv_done.notify_all();
         }
         /* whoever is still waiting is told so */
@@ -166,6 +174,7 @@ struct SharedDetector {
     void submit(DetReq* r) {
         std::unique_lock<std::mutex> lk(mu);
         q.push_back(r);
+        arrivals.submitted(r->caller, now_us());
         cv_req.notify_all();
         cv_done.wait(lk, [&] { return r->done; });
     }
@@ -175,6 +184,7 @@ static std::mutex g_det_mu;
 static std::map<std::string, std::weak_ptr<SharedDetector>> g_det_registry;
 
 struct tk_object_detector_s {
+    int caller = -1;                    /* this handle in sh->arrivals */
     std::shared_ptr<SharedDetector> sh; /* weights + the coalescing engine, shared by every handle of the same file */
     std::unique_ptr<TkDetector> own;    /* a private engine on the shared weights: only for the batch / raw-tensor entry points (tk_mi355x_detector_*) */
     std::vector<const char*> labels;
@@ -185,7 +195,7 @@ struct tk_object_detector_s {
     std::vector<std::vector<TkDetection>> last;
     ~tk_object_detector_s() {
         own.reset(); /* before the weights it reads */
-        if (sh) { std::lock_guard<std::mutex> lk(sh->mu); sh->handles--; }
+        if (sh) { std::lock_guard<std::mutex> lk(sh->mu); sh->handles--; sh->arrivals.remove(caller); }
     }
     TkDetector* priv(int max_batch, std::string* err) {
         if (own && own->max_batch >= max_batch) return own.get();
@@ -252,7 +262,7 @@ tk_error_code_t tk_object_detector_create(tk_object_detector_t** out_detector, c
             sh->th = std::thread([raw] { raw->run(); });
             g_det_registry[key] = sh;
         }
-        { std::lock_guard<std::mutex> hl(sh->mu); sh->handles++; }
+        { std::lock_guard<std::mutex> hl(sh->mu); sh->handles++; d->caller = sh->arrivals.add(); }
         d->sh = sh;
         std::string gerr;
         if (!sh->grow_for_handles(&gerr)) return vfail(TK_ERROR_GPU_MEMORY, gerr); /* (d's destructor takes the handle back) */
@@ -341,7 +351,7 @@ tk_error_code_t tk_mi355x_detector_detect_batch(tk_object_detector_t* d, int n, 
     if (n == 1 && !d->own) {
         /* the reference's one-frame call: through the shared engine, coalesced with the other handles' frames */
         DetReq r;
-        r.frame = frames[0].data; r.w = frames[0].width; r.h = frames[0].height; r.stride = pitch(frames[0]); r.bpp = bpp; r.conf = d->conf; r.iou = d->iou; r.fast = d->fast;
+        r.frame = frames[0].data; r.w = frames[0].width; r.h = frames[0].height; r.stride = pitch(frames[0]); r.bpp = bpp; r.conf = d->conf; r.iou = d->iou; r.fast = d->fast; r.caller = d->caller;
         if (r.w < 2 || r.h < 2 || r.stride < r.w * bpp) return vfail(TK_ERROR_INFERENCE_FAILED, "frame geometry invalid (need w,h >= 2 and stride >= w*bpp)");
         d->sh->submit(&r);
         if (!r.ok) return vfail(TK_ERROR_INFERENCE_FAILED, r.err);
@@ -417,6 +427,62 @@ tk_error_code_t tk_mi355x_detector_forward_graph(tk_object_detector_t* d, int ba
     memcpy(out, o.data(), o.size() * 4);
     if (!e->fetch(batch, &d->last)) return vfail(TK_ERROR_INFERENCE_FAILED, e->error); /* for last_boxes */
     return TK_SUCCESS;
+}
+
+int tk_mi355x_arrivals_simulate(int callers, int wait_us, int job_us, int frame_us, int max_batch, int n, const int* caller, const int64_t* at, int* sizes, int64_t* begins) {
+    if (callers < 1 || max_batch < 1 || n < 1 || !caller || !at || !sizes || !begins) return -1;
+    TkArrivals a(wait_us);
+    for (int i = 0; i < callers; ++i) a.add();
+    std::vector<std::deque<int64_t>> todo(callers); /* a caller's requests: not before this time, nor before its last one is served */
+    for (int i = 0; i < n; ++i) {
+        if (caller[i] < 0 || caller[i] >= callers) return -1;
+        todo[caller[i]].push_back(at[i]);
+    }
+    const int64_t never = INT64_MAX;
+    std::vector<int64_t> free_at(callers, 0);
+    std::vector<bool> in(callers, false);
+    int64_t now = 0;
+    int jobs = 0, left = n, queued = 0;
+    auto next = [&](int* who) { /* the next request to come */
+        int64_t t = never;
+        for (int i = 0; i < callers; ++i) {
+            if (in[i] || todo[i].empty()) continue;
+            const int64_t s = todo[i].front() > free_at[i] ? todo[i].front() : free_at[i];
+            if (s < t) { t = s; *who = i; }
+        }
+        return t;
+    };
+    auto arrive = [&](int64_t until) { /* all that come up to then */
+        int who = 0;
+        for (int64_t t; (t = next(&who)) <= until && t != never;) { a.submitted(who, t); in[who] = true; ++queued; }
+    };
+    while (left > 0) {
+        int who = 0;
+        arrive(now);
+        if (queued == 0) now = next(&who), arrive(now);
+        const int64_t from = now;
+        while (a.awaited(from) > 0 && queued < max_batch) {
+            const int64_t t = next(&who);
+            if (t > from + a.wait_us()) { now = from + a.wait_us(); a.waited_in_vain(from); break; }
+            now = t;
+            arrive(now);
+        }
+        int size = 0;
+        std::vector<int> job;
+        for (int i = 0; i < callers && size < max_batch; ++i)
+            if (in[i]) { job.push_back(i); ++size; }
+        sizes[jobs] = size;
+        begins[jobs++] = now;
+        const int64_t end = now + job_us + (int64_t)frame_us * size;
+        for (int i : job) todo[i].pop_front(); /* (its next request is later than `end`) */
+        for (int i : job) free_at[i] = end;
+        for (int64_t t; (t = next(&who)) < end && t != never;) { a.submitted(who, t); in[who] = true; ++queued; }
+        now = end;
+        for (int i : job) { a.served(i, now); in[i] = false; }
+        queued -= size;
+        left -= size;
+    }
+    return jobs;
 }
 
 int tk_mi355x_detector_is_graph(const tk_object_detector_t* d) { return d && d->sh && d->sh->model.generic ? 1 : 0; }
@@ -625,7 +691,7 @@ tk_error_code_t tk_vision_pipeline_process_frame(tk_vision_pipeline_t* pipeline,
             DetReq r;
             const uint32_t bpp = (uint32_t)bytes_per_pixel(video_frame);
             r.frame = video_frame->data; r.w = video_frame->width; r.h = video_frame->height; r.stride = video_frame->stride ? video_frame->stride : video_frame->width * bpp;
-            r.bpp = bpp; r.conf = d->conf; r.iou = d->iou; r.fast = d->fast; r.want_attr = bpp == 3 && r.stride == r.w * 3; r.max_objects = pipeline->max_objects;
+            r.bpp = bpp; r.conf = d->conf; r.iou = d->iou; r.fast = d->fast; r.caller = d->caller; r.want_attr = bpp == 3 && r.stride == r.w * 3; r.max_objects = pipeline->max_objects;
             ok = r.w >= 2 && r.h >= 2 && r.stride >= r.w * bpp;
             if (ok) {
                 d->sh->submit(&r);
