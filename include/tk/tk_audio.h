@@ -118,6 +118,8 @@ TK_API int32_t tk_mi355x_asr_suppress_table(tk_asr_whisper_context_t* ctx, uint8
  * engine whose scheduler coalesces their one-utterance calls (tk_asr_whisper_process_audio).  Counters of this context's shared engine: live
  * contexts, batched jobs run, utterances they carried, the widest job.  Any pointer may be NULL. */
 TK_API void tk_mi355x_asr_share_stats(const tk_asr_whisper_context_t* ctx, uint64_t* handles, uint64_t* batches, uint64_t* utterances, uint64_t* widest);
+/* pinned host memory that this context's engine holds for mel, encoder states and logits on their way out */
+TK_API uint64_t tk_mi355x_asr_staging_bytes(const tk_asr_whisper_context_t* ctx);
 /* whisper.cpp's decoding policy, which the reference's wrapper arms with temperature_inc 0.2 / entropy_thold 2.4 / logprob_thold -1.0
  * (src/audio/tk_asr_whisper.c:126-138; partial results: no fallback, :137).  OFF by default: the plain greedy decode is what the parity suite pins.
  *   transcribe_policy: the forced decode of transcribe_tokens with the token of every step picked by temperature (0 = arg max; > 0 = one draw from

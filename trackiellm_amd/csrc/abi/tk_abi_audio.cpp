@@ -493,6 +493,12 @@ void tk_mi355x_asr_share_stats(const tk_asr_whisper_context_t* c, uint64_t* hand
     if (widest) *widest = c->sh->widest;
 }
 
+uint64_t tk_mi355x_asr_staging_bytes(const tk_asr_whisper_context_t* c) {
+    if (!c || !c->sh) return 0;
+    std::lock_guard<std::mutex> lk(c->sh->eng_mu);
+    return c->sh->eng ? (uint64_t)c->sh->eng->staging_bytes() : 0;
+}
+
 tk_error_code_t tk_mi355x_asr_set_fast_contraction(tk_asr_whisper_context_t* c, int on) {
     if (!c) return TK_ERROR_INVALID_ARGUMENT;
     c->fast = on != 0;

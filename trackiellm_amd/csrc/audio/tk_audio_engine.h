@@ -47,6 +47,7 @@ public:
     bool fast = false;
     std::string error;
     hipStream_t stream = nullptr;
+    size_t staging_bytes() const { return aux_floats * sizeof(float); } /* pinned memory held for outputs beside the tokens */
     ~TkAsr();
     bool init(TkWhisperModel* m, int max_batch);
     /* pcm[B][n_samples] (host), greedy decode of exactly n_steps tokens after the start-of-transcript prompt;
@@ -81,12 +82,14 @@ private:
     int32_t* wh_state = nullptr;     /* [max_batch][TK_WH_STATE_INTS] */
     float* lp_dev = nullptr;         /* [n_text_ctx][max_batch] log-probabilities of a policy / reference-parameter decode */
     bool ensure_decode_buffers();
-    enum { TK_ASR_AUX_KEPT = 16 << 20 };
-    float* aux_host = nullptr;       /* pinned: what a call copies out beside its tokens */
-    size_t aux_floats = 0;
+    enum { TK_ASR_AUX_MIN = 1 << 20, TK_ASR_AUX_MAX = 16 << 20 }; /* floats */
+    float* aux_host = nullptr;       /* pinned: what a call copies out beside its tokens passes through it */
+    size_t aux_floats = 0;           /* grows in powers of two up to TK_ASR_AUX_MAX */
     hipStream_t aux_stream = nullptr;
-    hipEvent_t aux_ready = nullptr, aux_done = nullptr;
+    hipEvent_t aux_ready = nullptr, aux_done[2] = {nullptr, nullptr};
     bool aux_reserve(size_t floats);
+    struct Copy { float* to; const float* from; size_t n; };
+    bool aux_copy(const Copy* parts, int n, float* through, size_t room);
     std::vector<float> pick_logprobs; /* [total steps][B], read back by transcribe_policy */
 };
 

@@ -748,7 +748,7 @@ TkAsr::~TkAsr() {
     if (aux_stream) (void)hipStreamSynchronize(aux_stream);
     if (aux_host) (void)hipHostFree(aux_host);
     if (aux_ready) (void)hipEventDestroy(aux_ready);
-    if (aux_done) (void)hipEventDestroy(aux_done);
+    for (hipEvent_t e : aux_done) if (e) (void)hipEventDestroy(e);
     if (aux_stream) (void)hipStreamDestroy(aux_stream);
     if (stream) (void)hipStreamDestroy(stream);
 }
@@ -862,18 +862,46 @@ bool TkAsr::transcribe_ref(int B, const int16_t* pcm, int n_samples, const int32
     return ok && copied;
 }
 
-/* pinned memory of the last call's outputs is kept up to TK_ASR_AUX_KEPT floats; what is larger is given back by the next smaller call */
+/* pinned memory for a call's outputs beside its tokens: kept, so that it is pinned a few times in a context's life, and 64 MB at most; calls that have more to copy take it
+ * in turns (aux_copy) */
 bool TkAsr::aux_reserve(size_t floats) {
     if (!aux_stream) HIPQ(tk_create_perception_stream(&aux_stream));
     if (!aux_ready) HIPQ(hipEventCreateWithFlags(&aux_ready, hipEventDisableTiming));
-    if (!aux_done) HIPQ(hipEventCreateWithFlags(&aux_done, hipEventDisableTiming));
-    if (floats <= aux_floats && (aux_floats <= TK_ASR_AUX_KEPT || floats > TK_ASR_AUX_KEPT)) return true;
+    for (hipEvent_t& e : aux_done)
+        if (!e) HIPQ(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    size_t want = TK_ASR_AUX_MIN;
+    while (want < floats && want < TK_ASR_AUX_MAX) want *= 2;
+    if (want <= aux_floats) return true;
     if (aux_host) (void)hipHostFree(aux_host);
     aux_host = nullptr;
     aux_floats = 0;
-    HIPQ(hipHostMalloc((void**)&aux_host, floats * 4, hipHostMallocDefault));
-    aux_floats = floats;
+    HIPQ(hipHostMalloc((void**)&aux_host, want * 4, hipHostMallocDefault));
+    aux_floats = want;
     return true;
+}
+
+/* device arrays to the caller's memory through two halves of `room` pinned floats: one is on its way while the other is emptied */
+bool TkAsr::aux_copy(const Copy* parts, int n, float* through, size_t room) {
+    const size_t half = room / 2;
+    Copy busy[2] = {};
+    int slot = 0;
+    auto empty = [&](int i) {
+        if (busy[i].n == 0) return true;
+        HIPQ(hipEventSynchronize(aux_done[i]));
+        memcpy(busy[i].to, busy[i].from, busy[i].n * 4);
+        busy[i].n = 0;
+        return true;
+    };
+    for (int p = 0; p < n; ++p)
+        for (size_t at = 0; at < parts[p].n; at += half, slot ^= 1) {
+            if (!empty(slot)) return false;
+            const size_t count = parts[p].n - at < half ? parts[p].n - at : half;
+            float* mid = through + slot * half;
+            HIPQ(hipMemcpyAsync(mid, parts[p].from + at, count * 4, hipMemcpyDeviceToHost, aux_stream));
+            HIPQ(hipEventRecord(aux_done[slot], aux_stream));
+            busy[slot] = Copy{parts[p].to + at, mid, count};
+        }
+    return empty(slot) && empty(slot ^ 1);
 }
 
 bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* prompt, int n_prompt, int n_steps, int32_t* tokens_out,
@@ -883,6 +911,8 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     if (n_samples < 0 || n_samples > h.n_samples()) { error = "audio longer than the model window"; return false; }
     if (n_prompt < 1 || n_prompt + n_steps > h.n_text_ctx) { error = "prompt + steps exceed the text context"; return false; }
     HIPQ(hipSetDevice(model->device));
+    const size_t n_mel = mel_out ? (size_t)B * h.n_frames() * h.n_mels : 0, n_enc = enc_out ? (size_t)B * h.n_audio_ctx * h.n_audio_state : 0, n_lg = first_logits ? (size_t)B * h.n_vocab : 0;
+    if (n_mel + n_enc + n_lg > 0 && !aux_reserve(n_mel + n_enc + n_lg)) return false;
     size_t need = (size_t)B * (n_samples > 0 ? n_samples : 1);
     if (need > pcm_cap) need = (size_t)max_batch * (size_t)h.n_samples(); /* once: the engine's whole batch of full windows (0.96 MB each) */
     if (need > pcm_cap) {
@@ -903,18 +933,21 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     ops.long_ok = false;
     HIPQ(hipGetLastError());
     /* The mel, the encoder's output and the first logits travel to pinned memory on a stream of their own, and from there to the caller while the decoder's steps run:
-     * copies to pageable memory in between held back the launches behind them (one clip: 0.5 ms of 7). */
-    const size_t n_mel = mel_out ? (size_t)B * h.n_frames() * h.n_mels : 0, n_enc = enc_out ? (size_t)B * h.n_audio_ctx * h.n_audio_state : 0, n_lg = first_logits ? (size_t)B * h.n_vocab : 0;
-    float *mel_at = nullptr, *enc_at = nullptr, *lg_at = nullptr;
+     * copies to pageable memory in between held back the launches behind them (one clip: 0.5 ms of 7).  What does not fit goes in pieces once the steps are enqueued; logits
+     * that take more than half of the pinned memory go straight to the caller's. */
+    float* const lg_at = n_lg <= aux_floats / 2 ? aux_host : first_logits;
+    float* const mel_at = aux_host + (lg_at == aux_host ? n_lg : 0);
+    const size_t room = aux_floats - (size_t)(mel_at - aux_host);
+    const bool whole = n_mel + n_enc <= room;
     struct Wait { TkAsr* a; ~Wait() { if (a->aux_stream) (void)hipStreamSynchronize(a->aux_stream); } } wait{this}; /* whatever happens below */
-    if (n_mel + n_enc + n_lg > 0) {
-        if (!aux_reserve(n_mel + n_enc + n_lg)) return false;
-        mel_at = aux_host; enc_at = mel_at + n_mel; lg_at = enc_at + n_enc;
+    if (n_mel + n_enc > 0) {
         HIPQ(hipEventRecord(aux_ready, stream));
         HIPQ(hipStreamWaitEvent(aux_stream, aux_ready, 0));
-        if (n_mel) HIPQ(hipMemcpyAsync(mel_at, ml, n_mel * 4, hipMemcpyDeviceToHost, aux_stream));
-        if (n_enc) HIPQ(hipMemcpyAsync(enc_at, enc, n_enc * 4, hipMemcpyDeviceToHost, aux_stream));
-        HIPQ(hipEventRecord(aux_done, aux_stream));
+        if (whole) {
+            if (n_mel) HIPQ(hipMemcpyAsync(mel_at, ml, n_mel * 4, hipMemcpyDeviceToHost, aux_stream));
+            if (n_enc) HIPQ(hipMemcpyAsync(mel_at + n_mel, enc, n_enc * 4, hipMemcpyDeviceToHost, aux_stream));
+            HIPQ(hipEventRecord(aux_done[0], aux_stream));
+        }
     }
     /* The whole greedy loop is enqueued without touching the host: prompt tokens and positions sit in device tables uploaded once, step p
      * reads its token from the prompt table or from the previous step's arg-max slot and writes its own arg-max into slot p of an output
@@ -960,15 +993,18 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
         }
     }
     ops.flush();
-    if (n_mel + n_enc > 0) {
-        HIPQ(hipEventSynchronize(aux_done));
+    if (!whole) {
+        const Copy parts[2] = {{mel_out, ml, n_mel}, {enc_out, enc, n_enc}};
+        if (!aux_copy(parts, 2, mel_at, room)) return false;
+    } else if (n_mel + n_enc > 0) {
+        HIPQ(hipEventSynchronize(aux_done[0]));
         if (n_mel) memcpy(mel_out, mel_at, n_mel * 4);
-        if (n_enc) memcpy(enc_out, enc_at, n_enc * 4);
+        if (n_enc) memcpy(enc_out, mel_at + n_mel, n_enc * 4);
     }
     std::vector<int32_t> outs((size_t)steps_run * B);
     HIPQ(hipMemcpyAsync(outs.data(), out_tab + (size_t)(n_prompt - 1) * B, outs.size() * 4, hipMemcpyDeviceToHost, stream));
     HIPQ(hipStreamSynchronize(stream)); /* host_tab and outs live until here */
-    if (n_lg) memcpy(first_logits, lg_at, n_lg * 4);
+    if (n_lg && lg_at != first_logits) memcpy(first_logits, lg_at, n_lg * 4);
     for (int step = 0; step < n_steps; ++step)
         for (int b = 0; b < B; ++b) tokens_out[(size_t)b * n_steps + step] = step < steps_run ? outs[(size_t)step * B + b] : pick.eot;
     HIPQ(hipGetLastError());
