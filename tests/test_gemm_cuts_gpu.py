@@ -42,6 +42,14 @@ def test_wide_tiles_of_f16_weights_equal_staged(gpu, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(33, 32768, 128), (63, 32800, 384), (64, 33792, 256), (65, 27328, 128), (96, 27360, 640), (97, 20480, 256), (127, 12288, 1024), (129, 16384, 512),
+                                   (161, 13696, 384), (255, 10240, 256), (256, 6144, 512), (256, 10272, 128)])
+def test_wide_tiles_of_f16_weights_equal_staged_where_they_are_taken(gpu, M, N, K):
+    """two tiles and more for each of the chip's 1024 SIMDs, in both forms: last tiles of 1 .. 64 rows, one to eight requests of 128 k"""
+    test_wide_tiles_of_f16_weights_equal_staged(gpu, M, N, K)
+
+
+@pytest.mark.gpu
 def test_wide_tiles_in_parts_of_k(gpu):
     """a layer of f16 weights (q | k | v, o and down in 4, 4 and 7 parts of k): a position's logits do not depend on how many rows its pass has, whether up
     to 32 (the LDS ring) or more"""

@@ -14,7 +14,7 @@
  * A wave owns one weight row tile of one K range and streams it as one piece per 32 k, PF pieces in flight in registers; a piece feeds
  * 8 MFMAs per M-tile.  The A image is staged through an LDS ring by LDS-DMA, 1 KiB per (16 k, M-tile), shared by the workgroup's
  * waves; a lane's operand of four consecutive MFMAs is one ds_read_b128.  Rows beyond 256 run as further workgroups (grid y) over the
- * same weights; where that makes enough tiles of 32 x 32, a kernel without LDS takes
+ * same weights; where there are enough tiles of 32 x 32, a kernel without LDS takes
  * the products instead (k_gemm_wide), those of f16 weights from 33 rows on.  At 16 rows the f16 path is HBM-bound (2 B per weight); from 32 rows up the fp32 MFMA rate (157 TFLOP/s) bounds it.
  */
 #ifndef TK_GEMM_TILED_H

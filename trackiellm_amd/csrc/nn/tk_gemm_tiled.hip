@@ -629,14 +629,18 @@ bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p)
     /* Many rows: tiles of 32 x 32 without LDS, from 544 of them on (a chip has 1024 SIMDs).  Ring / wide time, 22 matrices at 260 .. 2000 rows: up to 384 tiles 0.4 .. 0.9
      * (1152 x 384 1.2), 432 .. 576 0.8 .. 1.3, from 640 on 1.1 .. 1.6.  Form 2 where the weights are more than an XCD's L2 holds and there are tiles to spare: 5120 x 1280
      * at 1500 and 12 000 rows 203 -> 179 and 1395 -> 1150 us; 512 rows 74 -> 86, 1536 x 384 at 48 000 rows 469 -> 485. */
-    /* f16 weights, from 33 rows on: ring / wide time of a 4096-wide layer (6144, 4096, 28672 and 4096 columns in 4, 4, 1 and 7 parts of k): 40 rows 1.01, 64 1.02, 96 1.30,
-     * 128 1.07, 136 1.55, 192 1.35, 256 1.14; at 24 and 32 rows 0.93 and 0.90.  Form 2 does a step of its 64 rows in 0.96 of the time that two tiles of form 1 take, but has
-     * half as many tiles to spread: 256 rows x 4096, 6144, 28672 columns 72.7, 105.5, 530 us against 76.8, 109.1, 491. */
+    /* f16 weights, from 33 rows on, where the chip's SIMDs get two tiles each; beyond 64 rows, which the ring kernel reads more than once, one and a half, or two and a half of
+     * short parts of k.  By ring / wide time of 400 products, 512 .. 5120 wide, 33 .. 256 rows: up to 64 rows 0.34 .. 1.02 below the line, 1.06 .. 1.35 above; beyond 0.35 ..
+     * 1.00 and 0.93 .. 2.3.  Layers' products by the ring / as chosen: 1536 wide at 33 rows 47 / 47 us (all in wide tiles 55), 2048 at 96 143 / 127, 4096 at 64 296 / 296 (314),
+     * at 160 1026 / 682.  Form 2
+     * does a step of its 64 rows in 0.96 of the time that two tiles of form 1 take, but has half as many tiles to spread: 256 rows x 4096, 6144, 28672 columns 72.7, 105.5,
+     * 530 us against 76.8, 109.1, 491. */
     if (a.wbytes == 2 && a.nrows > 2 * TK_TW_ROWS_PER_TILE) {
         const int64_t cols = (int64_t)(tw_row_tiles(a) / 2) * a.ks, simds = 4 * (int64_t)tk_tiled_num_cu();
         const int64_t one = (a.nrows + 31) / 32 * cols, two = (a.nrows + 63) / 64 * cols;
         const int form = 1.92f * (float)((two + simds - 1) / simds) < (float)((one + simds - 1) / simds) ? 2 : 1;
-        if (one >= 544 && tk_gemm_wide_plan(a, form, p)) return true;
+        const int64_t least = a.nrows <= 64 ? 2 * simds : a.K / a.ks >= 512 ? simds * 3 / 2 : simds * 5 / 2;
+        if (one >= least && tk_gemm_wide_plan(a, form, p)) return true;
     }
     if (a.wbytes == 4 && a.nrows > TK_TW_MAX_BLOCK_ROWS) {
         const int64_t tiles = (int64_t)((a.nrows + 31) / 32) * (tw_row_tiles(a) / 2);
