@@ -392,7 +392,8 @@ struct TkAudioGpuOps {
      * by a GEMM that writes into the matrix it was made from. */
     struct { const float* A = nullptr; int M = 0, K = 0, lda = 0; float* img = nullptr; size_t mark = 0; bool live = false; } pk;
     /* Decoder steps of few sequences: a norm is not launched; the linear layers on it make it themselves (TkTiledGemm::ln_x).  pk then names its output, which nobody else
-     * reads, and has no image.  A layer that cannot take it has it launched first. */
+     * reads, and has no image.  A layer that cannot take it has it launched first.  Up to TK_TW_LN_ROWS sequences: calls of 40 steps for 1, 2, 4, 6, 8, 16 clips, norms
+     * launched / in the products: 13.36 / 12.34, 14.39 / 13.28, 16.08 / 15.45, 17.31 / 17.27, 18.92 / 19.24, 23.65 / 26.00 ms. */
     struct { const float *x = nullptr, *w = nullptr, *b = nullptr; float* y = nullptr; bool live = false, used = false; } norm;
     static bool norm_fits(int rows, int D) { return rows <= TK_TW_LN_ROWS && D <= TK_TW_LN_MAX && D % 128 == 0; }
     void make_norm() { /* as a launch after all, with its image */

@@ -244,7 +244,9 @@ bool tk_conv_plan_ok(const TkConvDirect& c, const TkConvPlan& plan) {
 
 /* Costs in cycles, fitted to 18 000 launches (the detector's 3 x 3 layers at 1, 3, 8 and 32 frames, every cut): the choice takes 1.4 % more than the best cut in the
  * mean, 15 % at most.  A workgroup's latency is its patch, its chains (32 cycles an MFMA) and its epilogue; the CU's further ones take turns on the pipe, which their
- * vector instructions share.  Five, six or seven waves load the SIMDs unevenly (64 -> 80 channels, 32 frames: 247 us with five, 190 with four). */
+ * vector instructions share.  Five, six or seven waves load the SIMDs unevenly (64 -> 80 channels, 32 frames: 247 us with five, 190 with four).  The layers fitted are those of a
+ * network of 640 x 640; whole calls of others, by the GEMM kernels / here: 320 x 320, 1 and 16 frames 779 / 405, 1914 / 1249 us; 512 x 288, 1 and 6 766 / 418, 1207 / 733;
+ * 416 x 416, 2 and 16 847 / 496, 2269 / 1690; 1280 x 736, 1 and 16 1095 / 624, 8167 / 5361. */
 static float cd_plan(const TkConvDirect& c, int only_mt, int only_waves, TkConvPlan* plan) {
     const int ntiles = (c.N + 15) / 16;
     const float G = (float)(c.k * c.k * c.C / 16);

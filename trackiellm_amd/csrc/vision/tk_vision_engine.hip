@@ -365,8 +365,9 @@ struct TkGpuOps {
         return tk_launch_conv_direct(c, plan, s);
     }
     /* The last 18 layers are six chains of three, box and class branch of each scale: their first layers in one launch, then the second, then the third.  One frame:
-     * 18 launches of 170 us, now three of 73.  Up to four frames of 80 x 80: at 32 each layer fills the chip, and in one launch the largest patch (256 channels) would
-     * set how many workgroups a CU holds (1055 us for the first layers, 676 one by one). */
+     * 18 launches of 170 us, now three of 73.  Up to eight frames' worth of an 80 x 80 map: where each layer fills the chip, the largest patch (256 channels) of one launch
+     * sets how many workgroups a CU holds (32 frames: 1055 us for the first layers, 676 one by one).  Calls in sets / one by one: 640 x 640, 1 frame 491 / 565 us, 4 frames
+     * 938 / 1035, 8 frames 1553 / 1653, 16 frames 2764 / 2861; 1280 x 736, 2 frames 1070 / 1147, 6 frames 2390 / 2333, 16 frames 5853 / 5428. */
     struct Layer { TkT x, y; int idx; };
     std::vector<Layer> heads[3];
     bool defer(const TkT& x, int idx, const TkT& y, const TkT* res) {
@@ -378,7 +379,7 @@ struct TkGpuOps {
                 TkConvDirect c[TK_CONV_SET];
                 bool ok = stage.size() == TK_CONV_SET;
                 for (size_t i = 0; ok && i < stage.size(); ++i) ok = describe(stage[i].x, stage[i].idx, stage[i].y, nullptr, &c[i]);
-                ok = ok && (int64_t)c[0].B * c[0].H * c[0].W <= 4 * 6400;
+                ok = ok && (int64_t)c[0].B * c[0].H * c[0].W <= 8 * 6400;
                 TkConvPlan p[TK_CONV_SET];
                 if (ok && d->plans[x.B][stage[0].idx].mt == 0) {
                     ok = tk_conv_direct_plan_set(c, TK_CONV_SET, p);
