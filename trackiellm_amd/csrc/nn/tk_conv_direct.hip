@@ -43,7 +43,7 @@ template <int V> struct CdCount { static constexpr int value = V; };
  * instructions share: 71 % of it at 80 x 80 x 64 x 32 frames (139 us; the GEMM kernels 162), 57 % at 40 x 40 (43 us; 54), where patches and epilogues are a larger part.
  * Weights come from the L2 once per tile of pixels, operands from the LDS: a padding of 16 bytes a pixel turns 16 pixels into 16 different groups of banks.
  */
-template <int P, int MT /* 16-pixel tiles a wave */, int PF /* pieces of weights in flight */, int RD /* operand sets, divides PF: read RD - 1 groups ahead */>
+template <int P, int MT /* 16-pixel tiles a wave */, int PF /* pieces of weights in flight, even: operands are read a group ahead, into two sets */>
 __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdSet<P> set) {
     extern __shared__ __attribute__((aligned(16))) float cd_lds[];
     int pi = 0;
@@ -124,31 +124,29 @@ __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdSet<P> s
         const int py = cd_quot(pp, a.by_tw), px = pp - py * a.tw;
         base[m] = (const char*)cd_lds + ((py * a.pw + px) * c.stride * a.cp4 + g) * 16;
     }
-    v4f acc[MT], op[RD][MT];
+    v4f acc[MT], op[2][MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     auto read = [&](int set, int at) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) op[set][m] = *(const v4f*)(base[m] + at);
     };
-    auto group = [&](int u, int next) { /* operand set u % RD, weights w[u]; next: where the operands RD - 1 groups on lie */
-        read((u + RD - 1) % RD, next);
+    auto group = [&](int u, int next) { /* operand set u % 2, weights w[u]; next: where the next group's operands lie */
+        read((u + 1) % 2, next);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[u % RD][m][t], w[u][t], acc[m], 0, 0, 0);
+            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[u % 2][m][t], w[u][t], acc[m], 0, 0, 0);
     };
     int q = 0;
     v4i at = table[0], at_next = table[1];
-#pragma unroll
-    for (int i = 0; i < RD - 1; ++i) read(i, at[i]);
+    read(0, at[0]);
     for (; q + PF <= G; q += PF) {
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            constexpr int AHEAD = RD - 1;
-            const int next = at[(u + AHEAD) & 3];
-            if (((u + AHEAD) & 3) == 3) { at = at_next; at_next = table[(q + u + AHEAD + 5) >> 2]; }
+            const int next = at[(u + 1) & 3];
+            if (((u + 1) & 3) == 3) { at = at_next; at_next = table[(q + u + 6) >> 2]; }
             group(u, next);
             w[u] = *(const v4f*)(wp + (size_t)(q + u + PF) * 1024 + lane * 16);
         }
@@ -156,9 +154,8 @@ __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdSet<P> s
 #pragma unroll
     for (int u = 0; u < PF - 1; ++u)
         if (q + u < G) {
-            constexpr int AHEAD = RD - 1;
-            const int next = at[(u + AHEAD) & 3];
-            if (((u + AHEAD) & 3) == 3) { at = at_next; at_next = table[(q + u + AHEAD + 5) >> 2]; }
+            const int next = at[(u + 1) & 3];
+            if (((u + 1) & 3) == 3) { at = at_next; at_next = table[(q + u + 6) >> 2]; }
             group(u, next);
         }
 
@@ -306,8 +303,8 @@ bool tk_conv_direct_prepare_device() {
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return false;
     if (g_cd_opted[dev].load(std::memory_order_acquire)) return true;
     std::lock_guard<std::mutex> lk(g_cd_mu);
-    const void* fns[6] = {(const void*)k_conv_direct<1, 1, 8, 2>, (const void*)k_conv_direct<1, 2, 8, 2>, (const void*)k_conv_direct<1, 4, 4, 2>,
-                          (const void*)k_conv_direct<TK_CONV_SET, 1, 8, 2>, (const void*)k_conv_direct<TK_CONV_SET, 2, 8, 2>, (const void*)k_conv_direct<TK_CONV_SET, 4, 4, 2>};
+    const void* fns[6] = {(const void*)k_conv_direct<1, 1, 8>, (const void*)k_conv_direct<1, 2, 8>, (const void*)k_conv_direct<1, 4, 4>,
+                          (const void*)k_conv_direct<TK_CONV_SET, 1, 8>, (const void*)k_conv_direct<TK_CONV_SET, 2, 8>, (const void*)k_conv_direct<TK_CONV_SET, 4, 4>};
     for (const void* f : fns)
         if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, TK_CD_LDS) != hipSuccess) return false;
     g_cd_opted[dev].store(true, std::memory_order_release);
@@ -334,9 +331,9 @@ static bool cd_launch(const TkConvDirect* c, const TkConvPlan* p, int n, hipStre
     if (!tk_conv_direct_prepare_device()) return false;
     const dim3 grid(blocks, 1, c[0].B), block(64 * p[0].wm * p[0].wn);
     switch (p[0].mt) {
-        case 1: hipLaunchKernelGGL((k_conv_direct<P, 1, 8, 2>), grid, block, lds, s, set); break;
-        case 2: hipLaunchKernelGGL((k_conv_direct<P, 2, 8, 2>), grid, block, lds, s, set); break;
-        default: hipLaunchKernelGGL((k_conv_direct<P, 4, 4, 2>), grid, block, lds, s, set); break;
+        case 1: hipLaunchKernelGGL((k_conv_direct<P, 1, 8>), grid, block, lds, s, set); break;
+        case 2: hipLaunchKernelGGL((k_conv_direct<P, 2, 8>), grid, block, lds, s, set); break;
+        default: hipLaunchKernelGGL((k_conv_direct<P, 4, 4>), grid, block, lds, s, set); break;
     }
     return true;
 }

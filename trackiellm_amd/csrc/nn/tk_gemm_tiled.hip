@@ -311,9 +311,9 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
 }
 
 /*
- * Many rows: a wave makes 32 MI x 32 NI of the output alone, on v_mfma_f32_32x32x2_f32 (the same chain, two k an instruction), both operands from the caches straight
+ * Many rows: a wave makes 32 MI x 32 of the output alone, on v_mfma_f32_32x32x2_f32 (the same chain, two k an instruction), both operands from the caches straight
  * into registers, PF stages of KS k in flight: no LDS, no barrier, nothing that waves wait for each other with.  Step s of a 16-k group takes k = 2 s, 2 s + 1: lane half
- * h = l / 32 holds groups g = h and 2 + h of the image and of the weight tiles, a float4 each.  An operand float4 feeds 4 MI or 4 NI MFMAs of 64 cycles, where the ring
+ * h = l / 32 holds groups g = h and 2 + h of the image and of the weight tiles, a float4 each.  An operand float4 feeds 4 or 4 MI MFMAs of 64 cycles, where the ring
  * kernel above reads LDS once for 4 of 32: fp32 MFMAs and LDS reads take turns on a SIMD.
  * Images are made with the operands exchanged: a lane then holds one row, and lanes l, l + 32 swap halves so that each stores the 16 bytes of a group.
  * f16 weights (K-split parts side by side, the rows of a tile column in one workgroup) are converted in front of each product, on its pipe: 256 rows x 4096 x 28672 533 ->
@@ -322,8 +322,8 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
  * 48 000 rows, ring -> here, us (the fp32 MFMAs alone): 384 x 384 183 -> 139 (93), 1152 x 384 475 -> 346 (278), 1536 x 384 with GELU 610 -> 469 (370), 384 x 1536 560 -> 513
  * (370); 1500 rows: 23.2 -> 17.6, 31.6 -> 25.2 and 38.2 -> 30.4 of the last three.  What is left is the last round of tiles and the first requests of each.
  */
-template <int WB, int MI, int NI, int KS, int PF>
-__global__ __launch_bounds__(256, MI * NI == 2 || PF > 2 ? 4 : 5) void k_gemm_wide(TkTiledGemm a, int ncol /* tiles of 32 NI columns */, int nrow /* tiles of 32 MI rows */, int total /* waves' tiles */,
+template <int WB, int MI, int KS, int PF>
+__global__ __launch_bounds__(256, MI == 2 || PF > 2 ? 4 : 5) void k_gemm_wide(TkTiledGemm a, int ncol /* tiles of 32 columns */, int nrow /* tiles of 32 MI rows */, int total /* waves' tiles */,
                                                                                   int per_xcd) {
     constexpr int V = KS / 8;               /* float4 per 32 rows and stage */
     constexpr int WV = WB == 4 ? V : V / 2; /* 16-byte pieces of weights per 32 columns and stage */
@@ -336,44 +336,38 @@ __global__ __launch_bounds__(256, MI * NI == 2 || PF > 2 ? 4 : 5) void k_gemm_wi
      * weights, then the columns, then the parts of k */
     const int blk = WB == 4 ? id / ncol : id % nrow, row0 = blk * 32 * MI;
     const int colk = id / nrow, ksi = WB == 4 ? 0 : colk / ncol;
-    int rt = (WB == 4 ? id - blk * ncol : colk - ksi * ncol) * 2 * NI, seg = 0, col_base = 0;
+    int rt = (WB == 4 ? id - blk * ncol : colk - ksi * ncol) * 2, seg = 0, col_base = 0;
     while (seg < a.nseg - 1 && rt >= a.row_tiles[seg]) { rt -= a.row_tiles[seg]; col_base += a.row_tiles[seg] * TK_TW_ROWS_PER_TILE; ++seg; }
     const unsigned a_pitch = (unsigned)a.a_ts * 4u, w_pitch = (unsigned)a.K * 16u * WB; /* bytes of 16 rows */
     const int tiles_here = (a.nrows - row0 + 15) / 16;
     const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void*)(a.a_img + (size_t)(row0 / 16) * a.a_ts), 0, (unsigned)(tiles_here < 2 * MI ? tiles_here : 2 * MI) * a_pitch, 0x00020000);
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.tiles[seg] + (size_t)rt * w_pitch), 0, 2u * NI * w_pitch, 0x00020000);
-    unsigned a_at[MI], w_at[NI];
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.tiles[seg] + (size_t)rt * w_pitch), 0, 2u * w_pitch, 0x00020000);
+    unsigned a_at[MI];
 #pragma unroll
     for (int i = 0; i < MI; ++i) {
         const int tile = 2 * i + up;
         a_at[i] = (unsigned)(tile < tiles_here ? tile : tiles_here - 1) * a_pitch + (unsigned)(h * 256 + l16 * 16);
     }
-#pragma unroll
-    for (int i = 0; i < NI; ++i) w_at[i] = (unsigned)(2 * i + up) * w_pitch + (unsigned)((h * 16 + l16) * 8 * WB);
+    const unsigned w_at = (unsigned)up * w_pitch + (unsigned)((h * 16 + l16) * 8 * WB);
 
-    v4f aq[PF][MI][V], wq[PF][NI][WV];
+    v4f aq[PF][MI][V], wq[PF][WV];
     const int ns = (WB == 4 ? a.K : a.K / a.ks) / KS, s0 = ksi * ns;
-    auto load = [&](int s, v4f (*av)[V], v4f (*wv)[WV]) {
+    auto load = [&](int s, v4f (*av)[V], v4f* wv) {
         s = s0 + (s < ns ? s : ns - 1);
 #pragma unroll
         for (int v = 0; v < V; ++v) { /* 16-k group v / 2 of the stage, half v % 2 of its groups */
             const unsigned j = (unsigned)(s * (KS / 16) + v / 2);
 #pragma unroll
             for (int i = 0; i < MI; ++i) av[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(ar, a_at[i] + (v & 1) * 512, j * 1024, 0));
-#pragma unroll
-            for (int i = 0; i < NI; ++i) {
-                if (WB == 4) wv[i][v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at[i] + (v & 1) * 1024, (j >> 1) * 2048 + (j & 1) * 16, 0));
-                else if (v % 4 < 2) wv[i][v / 4 * 2 + v % 2] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at[i] + (v & 1) * 512, (j >> 1) * 1024, 0));
-            }
+            if (WB == 4) wv[v] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at + (v & 1) * 1024, (j >> 1) * 2048 + (j & 1) * 16, 0));
+            else if (v % 4 < 2) wv[v / 4 * 2 + v % 2] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(wr, w_at + (v & 1) * 512, (j >> 1) * 1024, 0));
         }
     };
-    v16f acc[MI][NI];
+    v16f acc[MI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int n = 0; n < NI; ++n)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][n][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
     const bool image = a.c_img != nullptr || (a.per_seg && a.seg_img[seg]);
     auto products = [&](auto swapped) {
 #pragma unroll
@@ -390,19 +384,17 @@ __global__ __launch_bounds__(256, MI * NI == 2 || PF > 2 ? 4 : 5) void k_gemm_wi
 #pragma unroll
                         for (int b = 0; b < 2; ++b)
 #pragma unroll
-                            for (int i = 0; i < MI; ++i)
-#pragma unroll
-                                for (int n = 0; n < NI; ++n) {
-                                    const float x = aq[u][i][v + b][t];
-                                    float w;
-                                    if (WB == 4) w = wq[u][n][WB == 4 ? v + b : 0][t];
-                                    else w = (float)__builtin_bit_cast(tw_v8h, wq[u][n][v / 4 * 2 + b])[4 * (v / 2 % 2) + t]; /* a piece: t of both 16-k groups */
-                                    acc[i][n] = swapped.value ? __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, acc[i][n], 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, acc[i][n], 0, 0, 0);
-                                }
+                            for (int i = 0; i < MI; ++i) {
+                                const float x = aq[u][i][v + b][t];
+                                float w;
+                                if (WB == 4) w = wq[u][WB == 4 ? v + b : 0][t];
+                                else w = (float)__builtin_bit_cast(tw_v8h, wq[u][v / 4 * 2 + b])[4 * (v / 2 % 2) + t]; /* a piece: t of both 16-k groups */
+                                acc[i] = swapped.value ? __builtin_amdgcn_mfma_f32_32x32x2f32(w, x, acc[i], 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x2f32(x, w, acc[i], 0, 0, 0);
+                            }
                 /* the requests spread over the products: in front of them they hold these up, behind them (where the compiler puts them) they come late */
 #pragma unroll
-                for (int i = 0; i < MI * V + NI * WV; ++i) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, MI * NI * V * 4 / (MI * V + NI * WV), 0);
+                for (int i = 0; i < MI * V + WV; ++i) {
+                    __builtin_amdgcn_sched_group_barrier(0x008, MI * V * 4 / (MI * V + WV), 0);
                     __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                 }
                 __builtin_amdgcn_sched_barrier(0);
@@ -418,33 +410,31 @@ __global__ __launch_bounds__(256, MI * NI == 2 || PF > 2 ? 4 : 5) void k_gemm_wi
         float* img = a.per_seg ? a.seg_out[seg] : a.c_img;
         const int cols = a.per_seg ? a.seg_n[seg] : a.n_valid, c0 = a.per_seg ? col0 : col_base + col0;
 #pragma unroll
-        for (int i = 0; i < MI; ++i)
+        for (int i = 0; i < MI; ++i) {
+            const int row = row0 + 32 * i + l32;
+            float v[16];
 #pragma unroll
-            for (int n = 0; n < NI; ++n) {
-                const int row = row0 + 32 * i + l32;
-                float v[16];
+            for (int q = 0; q < 4; ++q) {
+                v4f b = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (bias) b = *(const v4f*)(bias + col0 + 8 * q + 4 * h);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    v4f b = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if (bias) b = *(const v4f*)(bias + col0 + 32 * n + 8 * q + 4 * h);
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) v[4 * q + r] = add_bias ? acc[i][n][4 * q + r] + b[r] : acc[i][n][4 * q + r];
-                }
-                tw_act_all<16>(v, a.act);
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int g = 0; g < 4; g += 2) {
-                        v4f o;
-#pragma unroll
-                        for (int b = 0; b < 2; ++b) { /* t = 2 b + h of groups g, g + 1: the lower lanes take g, the upper g + 1 */
-                            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[8 * q + 4 * b + g]), __float_as_uint(v[8 * q + 4 * b + g + 1]), false, false);
-                            o[2 * b] = __uint_as_float(x[0]);
-                            o[2 * b + 1] = __uint_as_float(x[1]);
-                        }
-                        if (row < a.nrows) *(v4f*)(img + (size_t)(row >> 4) * 16 * cols + (size_t)(((c0 >> 4) + 2 * n + q) * 256 + (g + h) * 64 + (row & 15) * 4)) = o;
-                    }
+                for (int r = 0; r < 4; ++r) v[4 * q + r] = add_bias ? acc[i][4 * q + r] + b[r] : acc[i][4 * q + r];
             }
+            tw_act_all<16>(v, a.act);
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+#pragma unroll
+                for (int g = 0; g < 4; g += 2) {
+                    v4f o;
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) { /* t = 2 b + h of groups g, g + 1: the lower lanes take g, the upper g + 1 */
+                        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[8 * q + 4 * b + g]), __float_as_uint(v[8 * q + 4 * b + g + 1]), false, false);
+                        o[2 * b] = __uint_as_float(x[0]);
+                        o[2 * b + 1] = __uint_as_float(x[1]);
+                    }
+                    if (row < a.nrows) *(v4f*)(img + (size_t)(row >> 4) * 16 * cols + (size_t)(((c0 >> 4) + q) * 256 + (g + h) * 64 + (row & 15) * 4)) = o;
+                }
+        }
         return;
     }
     products(std::false_type{});
@@ -452,26 +442,23 @@ __global__ __launch_bounds__(256, MI * NI == 2 || PF > 2 ? 4 : 5) void k_gemm_wi
     const int ldc = a.per_seg ? a.seg_ldc[seg] : a.ldc;
     const float* res = a.residual ? a.residual + col_base + col0 : nullptr;
 #pragma unroll
-    for (int i = 0; i < MI; ++i)
+    for (int i = 0; i < MI; ++i) {
+        const float b = bias ? bias[col0 + l32] : 0.0f;
+        float v[16], rs[16];
 #pragma unroll
-        for (int n = 0; n < NI; ++n) {
-            const int c = 32 * n + l32;
-            const float b = bias ? bias[col0 + c] : 0.0f;
-            float v[16], rs[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = row0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (res) rs[r] = row < a.nrows ? res[(size_t)row * a.ldr + c] : 0.0f;
-                v[r] = add_bias ? acc[i][n][r] + b : acc[i][n][r];
-            }
-            tw_act_all<16>(v, a.act);
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = row0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
-                if (res) v[r] = v[r] + rs[r];
-                if (row < a.nrows) out[(size_t)row * ldc + c] = v[r];
-            }
+        for (int r = 0; r < 16; ++r) {
+            const int row = row0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (res) rs[r] = row < a.nrows ? res[(size_t)row * a.ldr + l32] : 0.0f;
+            v[r] = add_bias ? acc[i][r] + b : acc[i][r];
         }
+        tw_act_all<16>(v, a.act);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = row0 + 32 * i + 8 * (r >> 2) + 4 * h + (r & 3);
+            if (res) v[r] = v[r] + rs[r];
+            if (row < a.nrows) out[(size_t)row * ldc + l32] = v[r];
+        }
+    }
 }
 
 /* ---- operand preparation ---- */
@@ -701,17 +688,15 @@ static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p) {
 
 /* the cut of k_gemm_wide's form 1 (32 x 32 of the output a wave) or 2 (64 x 32); false: not a product it takes */
 bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p) {
-    static const struct { int mi, ni; } forms[] = {{0, 0}, {1, 1}, {2, 1}};
     if (!tw_valid(a) || form < 1 || form > 2 || (a.wbytes == 4 && a.ks != 1) || a.ln_x || (a.c_img && (a.wbytes == 2 || a.out || a.residual)) || a.K % (128 * a.ks)) return false;
     if (a.ks > 1 && (a.bias || a.residual || a.act || a.add_zero_bias)) return false; /* parts of k are sums alone */
-    const int per = 2 * forms[form].ni;
     for (int i = 0; i < a.nseg; ++i)
-        if (a.row_tiles[i] % per || (a.per_seg && a.seg_n[i] != a.row_tiles[i] * 16)) return false;
+        if (a.row_tiles[i] % 2 || (a.per_seg && a.seg_n[i] != a.row_tiles[i] * 16)) return false;
     if (!a.per_seg && a.n_valid != tw_row_tiles(a) * 16) return false;
     *p = TkTiledPlan{};
     p->wide = form;
-    p->groups = tw_row_tiles(a) / per;
-    p->ny = (a.nrows + 32 * forms[form].mi - 1) / (32 * forms[form].mi);
+    p->groups = tw_row_tiles(a) / 2;
+    p->ny = (a.nrows + 32 * form - 1) / (32 * form);
     return (int64_t)p->groups * p->ny * a.ks < 0x7fffff00;
 }
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipStream_t s) {
@@ -720,7 +705,7 @@ bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipSt
         if (!tk_gemm_wide_plan(a, p.wide, &w)) return false;
         const int total = w.groups * w.ny * a.ks, per = ((total + 3) / 4 + 7) / 8;
         const dim3 wgrid((unsigned)per * 8);
-#define TK_TW_WIDE(WBV, MIV, KSV, PFV) hipLaunchKernelGGL((k_gemm_wide<WBV, MIV, 1, KSV, PFV>), wgrid, dim3(256), 0, s, a, w.groups, w.ny, total, per)
+#define TK_TW_WIDE(WBV, MIV, KSV, PFV) hipLaunchKernelGGL((k_gemm_wide<WBV, MIV, KSV, PFV>), wgrid, dim3(256), 0, s, a, w.groups, w.ny, total, per)
         if (a.wbytes == 2) {
             if (p.wide == 1) TK_TW_WIDE(2, 1, 32, 4);
             else TK_TW_WIDE(2, 2, 32, 2);
