@@ -62,6 +62,21 @@ def test_a_lone_caller_waits_once_for_idle_ones():
     assert jobs_of(32, [(3, t) for t in at]) == [(1, at[0] + 400)] + [(1, t) for t in at[1:]]
 
 
+@pytest.mark.parametrize("callers", [2, 3, 8])
+@pytest.mark.parametrize("gap", [0, 100, 3000])
+def test_handles_that_one_thread_uses_in_turn_do_not_wait_for_each_other(callers, gap):
+    """a call, `gap`, the next handle's call: each of them is waited for twice at most"""
+    step = 550 + gap
+    at, requests = 1000, []
+    for i in range(10 * callers):
+        got = jobs_of(callers, requests + [(i % callers, at)])
+        requests.append((i % callers, at))
+        begin = got[-1][1]
+        assert got[-1][0] == 1 and begin - at in (0, 400)
+        assert begin == at or i < 2 * callers
+        at = begin + step
+
+
 @pytest.mark.parametrize("gap", [900, 2500])
 def test_a_caller_that_has_been_served_is_not_waited_for(gap):
     """bursts of one, then the seven others `gap` later: the seven are one job, which begins when the last of them is in (or the first one's job ends)"""
