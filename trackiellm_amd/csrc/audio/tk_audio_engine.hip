@@ -913,7 +913,7 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     if (n_prompt < 1 || n_prompt + n_steps > h.n_text_ctx) { error = "prompt + steps exceed the text context"; return false; }
     HIPQ(hipSetDevice(model->device));
     const size_t n_mel = mel_out ? (size_t)B * h.n_frames() * h.n_mels : 0, n_enc = enc_out ? (size_t)B * h.n_audio_ctx * h.n_audio_state : 0, n_lg = first_logits ? (size_t)B * h.n_vocab : 0;
-    if (n_mel + n_enc + n_lg > 0 && !aux_reserve(n_mel + n_enc + n_lg)) return false;
+    if (n_mel + n_enc + n_lg > 0 && aux_host && !aux_reserve(n_mel + n_enc + n_lg)) return false; /* (may give memory back, which waits for the device) */
     size_t need = (size_t)B * (n_samples > 0 ? n_samples : 1);
     if (need > pcm_cap) need = (size_t)max_batch * (size_t)h.n_samples(); /* once: the engine's whole batch of full windows (0.96 MB each) */
     if (need > pcm_cap) {
@@ -936,6 +936,7 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     /* The mel, the encoder's output and the first logits travel to pinned memory on a stream of their own, and from there to the caller while the decoder's steps run:
      * copies to pageable memory in between held back the launches behind them (one clip: 0.5 ms of 7).  What does not fit goes in pieces once the steps are enqueued; logits
      * that take more than half of the pinned memory go straight to the caller's. */
+    if (n_mel + n_enc + n_lg > 0 && !aux_reserve(n_mel + n_enc + n_lg)) return false; /* the first time: pinned while the encoder runs */
     float* const lg_at = n_lg <= aux_floats / 2 ? aux_host : first_logits;
     float* const mel_at = aux_host + (lg_at == aux_host ? n_lg : 0);
     const size_t room = aux_floats - (size_t)(mel_at - aux_host);
