@@ -1,0 +1,45 @@
+"""Whole prompts (prefill) against the same rows through passes of at most 256 rows (forward, which other tests hold to the oracle): the sampled ids, and the logits of the
+position behind each prompt, which read every key and value the prompt left, bit for bit.  Totals at the edges of the wide kernel's parts (96 and 128 rows) and of a pass (2048)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def models(gpu):
+    made = {}
+
+    def get(name):
+        if name not in made:
+            hp = {"tiny": gpu.TINY(), "tiny-f16": gpu.TINY(),
+                  "wide": gpu.LlmHParams(2, 1024, 8, 2, 128, 2048, 512, 1e-5, 10000.0, 0, 0, 0, 0, 1),
+                  "wide-f16": gpu.LlmHParams(2, 1024, 8, 2, 128, 2048, 512, 1e-5, 10000.0, 0, 0, 0, 0, 1)}[name]
+            made[name] = gpu.LlmModel(hp).fill_synthetic(4, f16=name.endswith("f16"))
+        return made[name]
+    return get
+
+
+@pytest.mark.parametrize("model", ["tiny", "tiny-f16", "wide", "wide-f16"])
+@pytest.mark.parametrize("nseq,n_prompt", [(1, 1), (1, 2), (2, 1), (3, 1), (5, 2), (1, 33), (3, 65), (1, 257), (3, 96), (9, 32), (1, 385), (256, 2), (2, 300), (7, 130), (32, 32), (41, 25), (3, 683), (64, 33), (1, 2100)])
+def test_prefill_equals_passes_of_256_rows(gpu, models, model, nseq, n_prompt):
+    m = models(model)
+    vocab = m.hparams.vocab
+    rng = np.random.default_rng(nseq * 1000 + n_prompt)
+    toks = rng.integers(3, vocab, (nseq, n_prompt)).astype(np.int32)
+    follow = rng.integers(3, vocab, nseq).astype(np.int32)
+    seq, pos = np.repeat(np.arange(nseq, dtype=np.int32), n_prompt), np.tile(np.arange(n_prompt, dtype=np.int32), nseq)
+    one, other = gpu.LlmSession(m, nseq, n_prompt + 4), gpu.LlmSession(m, nseq, n_prompt + 4)
+    for _ in range(2):  # a second call finds the first one's caches and buffers
+        first = one.prefill(toks)
+    ids, _ = one.decode(nseq, 1)
+    got, got_ids = one.forward(np.arange(nseq, dtype=np.int32), np.full(nseq, n_prompt, np.int32), follow)
+    flat, picked = toks.ravel(), np.zeros(nseq * n_prompt, np.int32)
+    for r in range(0, flat.size, 256):
+        _, picked[r:r + 256] = other.forward(seq[r:r + 256], pos[r:r + 256], flat[r:r + 256])
+    want_first = picked[n_prompt - 1::n_prompt]
+    _, want_ids = other.forward(np.arange(nseq, dtype=np.int32), np.full(nseq, n_prompt, np.int32), want_first)
+    want, _ = other.forward(np.arange(nseq, dtype=np.int32), np.full(nseq, n_prompt, np.int32), follow)
+    assert np.array_equal(first, want_first)
+    assert np.array_equal(ids[0], want_ids)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.abs(got - want).max()

@@ -102,11 +102,17 @@ public:
 
 private:
     friend class TkLlmPipe; /* tk_llm_pipe.h: a pipeline stage enqueues layer ranges of this session between its hand-off kernels */
+    const float* last_x = nullptr; /* where the last caches-only enqueue_range left the residual stream in front of its last layer */
     int last_ks_res = 1;    /* slabs of the residual update the last enqueue_range left pending in `partial` */
     void enqueue_pass(int nrows, bool lm_head, bool fused_attn);
-    void enqueue_range(int nrows, int l0, int l1, bool embed, bool fold_out, bool lm_head, bool fused_attn);
+    void enqueue_range(int nrows, int l0, int l1, bool embed, bool fold_out, bool lm_head, bool fused_attn, bool caches_only = false);
+    int enqueue_layer_tail(const TkLlmLayer& L, float* xs, int nrows);
+    void enqueue_head(float* xs, int ks_res, int nrows);
+    void enqueue_pick(int nrows);
     int enqueue_matmul(const TkDevTensor* const* t, int nseg, int K, int ks, int n_total, const TkActQ8& act, float* out, int nrows);
     uint16_t *kcache = nullptr, *vcache = nullptr;
+    int pass_rows = 0; /* rows of prefill()'s passes, and of every buffer a pass of rows writes */
+    float *x_last = nullptr, *q_last = nullptr; /* [TK_MAX_ROWS][..]: what prefill() keeps of the rows it samples */
     float *x = nullptr, *x2 = nullptr, *qbuf = nullptr, *partial = nullptr, *partial2 = nullptr, *rope_cos = nullptr, *rope_sin = nullptr;
     TkActQ8 act_d{}, act_qd{}, act_ff{};
     hipGraphExec_t graph_exec[2][TK_MAX_ROWS + 1] = {}; /* [long_pass][row count]: decode pass (head + sampling, every sequence once) */
@@ -125,8 +131,8 @@ private:
     float* d_scores = nullptr; /* [TK_LONG_ATT_MAX_ROWS][n_head][max_ctx], allocated when the window can reach tk_long_att_min_pos() */
     void choose_attention(const int32_t* pos, int nrows);
     void choose_attention_top(int top, int nrows);
-    int32_t* d_tab = nullptr;                           /* prefill schedule: [3][total rows] = seq, pos, tok */
-    int32_t* d_tiles = nullptr;                         /* [1 + TK_MAX_ROWS] 16-row tiles of a multi-position pass (k_att_tiles) */
+    int32_t* d_tab = nullptr;                           /* prefill schedule: [3][rows of all passes, then the sampled ones] = seq, pos, tok */
+    int32_t* d_tiles = nullptr;                         /* [1 + pass_rows] 16-row tiles of a multi-position pass (k_att_tiles) */
     size_t tab_cap = 0;
     bool capture_pass(hipGraphExec_t* slot, int nrows, bool lm_head, bool fused_attn);
     hipGraphExec_t* decode_slot(int nrows, int top) override;

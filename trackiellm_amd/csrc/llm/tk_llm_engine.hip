@@ -223,20 +223,21 @@ bool TkLlmModel::ready() const {
 
 /* ------------------------------------------------------------------ session ---------------- */
 
-static bool alloc_act(TkActQ8* a, int K, bool want_f16, std::string& error) {
+static bool alloc_act(TkActQ8* a, int K, int rows, bool want_f16, std::string& error) {
+    const size_t tiles = (size_t)(rows + TK_ROW_SLOTS - 1) / TK_ROW_SLOTS + TK_SPARE_TILES;
     a->aq_ts = TK_AQ_BYTES(K); a->ad_ts = TK_AD_FLOATS(K); a->abs_ts = TK_ABS_BYTES(K);
     a->af = nullptr; a->af_ts = (size_t)K * TK_ROW_SLOTS;
-    if (want_f16 && hipMalloc((void**)&a->af, (size_t)TK_MAX_ROWS * K * 4) != hipSuccess) { error = "out of device memory (f16 activation buffers)"; return false; }
-    if (a->af) (void)hipMemset(a->af, 0, (size_t)TK_MAX_ROWS * K * 4);
-    if (hipMalloc((void**)&a->aq, TK_MAX_TILES * a->aq_ts) != hipSuccess || hipMalloc((void**)&a->ad, TK_MAX_TILES * a->ad_ts * 4) != hipSuccess ||
-        hipMalloc((void**)&a->abs, TK_MAX_TILES * a->abs_ts) != hipSuccess || hipMalloc((void**)&a->abs16, TK_MAX_TILES * a->abs_ts * 2) != hipSuccess) {
+    if (want_f16 && hipMalloc((void**)&a->af, tiles * a->af_ts * 4) != hipSuccess) { error = "out of device memory (f16 activation buffers)"; return false; }
+    if (a->af) (void)hipMemset(a->af, 0, tiles * a->af_ts * 4);
+    if (hipMalloc((void**)&a->aq, tiles * a->aq_ts) != hipSuccess || hipMalloc((void**)&a->ad, tiles * a->ad_ts * 4) != hipSuccess ||
+        hipMalloc((void**)&a->abs, tiles * a->abs_ts) != hipSuccess || hipMalloc((void**)&a->abs16, tiles * a->abs_ts * 2) != hipSuccess) {
         error = "out of device memory (activation buffers)";
         return false;
     }
-    (void)hipMemset(a->aq, 0, TK_MAX_TILES * a->aq_ts);
-    (void)hipMemset(a->ad, 0, TK_MAX_TILES * a->ad_ts * 4);
-    (void)hipMemset(a->abs, 0, TK_MAX_TILES * a->abs_ts);
-    (void)hipMemset(a->abs16, 0, TK_MAX_TILES * a->abs_ts * 2);
+    (void)hipMemset(a->aq, 0, tiles * a->aq_ts);
+    (void)hipMemset(a->ad, 0, tiles * a->ad_ts * 4);
+    (void)hipMemset(a->abs, 0, tiles * a->abs_ts);
+    (void)hipMemset(a->abs16, 0, tiles * a->abs_ts * 2);
     return true;
 }
 static void free_act(TkActQ8* a) {
@@ -259,7 +260,10 @@ bool TkLlmSession::init(TkLlmModel* m, int mseq, int mctx) {
         error = "max_ctx too large: the attention kernel keeps one score row per query head of a KV group in LDS (about 9000 positions for 4 x 128)";
         return false;
     }
-    if (!init_tables(m->device, h.vocab, TK_MAX_ROWS, 0, nullptr)) return false;
+    /* a prompt's pass: as many rows as prefill() can hand to it, in whole parts of the wide kernel */
+    const int64_t most = (int64_t)(mseq < TK_MAX_ROWS ? mseq : TK_MAX_ROWS) * mctx;
+    pass_rows = most >= TK_PASS_ROWS ? TK_PASS_ROWS : most <= TK_MAX_ROWS ? TK_MAX_ROWS : (int)(most + 127) / 128 * 128;
+    if (!init_tables(m->device, h.vocab, pass_rows, 0, nullptr)) return false;
     tk_attention_note_session(m->device, +1);
     counted_ = true;
     const int QD = h.n_head * h.head_dim, KVD = h.n_kv_head * h.head_dim, half = h.head_dim / 2;
@@ -268,20 +272,23 @@ bool TkLlmSession::init(TkLlmModel* m, int mseq, int mctx) {
     HIPQ(hipMalloc((void**)&vcache, kv * 2));
     HIPQ(hipMemset(kcache, 0, kv * 2));
     HIPQ(hipMemset(vcache, 0, kv * 2));
-    HIPQ(hipMalloc((void**)&x, (size_t)TK_MAX_ROWS * h.d_model * 4));
-    HIPQ(hipMalloc((void**)&qbuf, (size_t)TK_MAX_ROWS * QD * 4));
-    size_t pmax = (size_t)h.ks_qkv * (QD + 2 * KVD);
-    pmax = std::max(pmax, (size_t)h.ks_o * h.d_model);
-    pmax = std::max(pmax, (size_t)h.ks_gateup * 2 * h.d_ff);
-    pmax = std::max(pmax, (size_t)h.ks_down * h.d_model);
-    HIPQ(hipMalloc((void**)&partial, pmax * TK_MAX_ROWS * 4));
+    HIPQ(hipMalloc((void**)&x, (size_t)pass_rows * h.d_model * 4));
+    HIPQ(hipMalloc((void**)&qbuf, (size_t)pass_rows * QD * 4));
+    HIPQ(hipMalloc((void**)&x_last, (size_t)TK_MAX_ROWS * h.d_model * 4));
+    HIPQ(hipMalloc((void**)&q_last, (size_t)TK_MAX_ROWS * QD * 4));
+    /* K-split slabs, TK_SLAB_ROWS rows apart; the last one ends with the pass */
+    auto slabs = [&](int ks, int cols, int rows) { return ((size_t)(ks - 1) * TK_SLAB_ROWS + rows) * (size_t)cols; };
+    auto partial_floats = [&](int rows) {
+        return std::max(std::max(slabs(h.ks_qkv, QD + 2 * KVD, rows), slabs(h.ks_o, h.d_model, rows)), std::max(slabs(h.ks_gateup, 2 * h.d_ff, rows), slabs(h.ks_down, h.d_model, rows)));
+    };
+    HIPQ(hipMalloc((void**)&partial, partial_floats(pass_rows) * 4));
     /* twins for passes whose mat-vec launches run their producer themselves (enqueue_range): such a launch reads one (x, slab) pair while
      * its workgroups write the other */
-    HIPQ(hipMalloc((void**)&x2, (size_t)TK_MAX_ROWS * h.d_model * 4));
-    HIPQ(hipMalloc((void**)&partial2, pmax * TK_MAX_ROWS * 4));
-    if (!alloc_act(&act_d, h.d_model, m->has_f16, error) || !alloc_act(&act_qd, QD, m->has_f16, error) || !alloc_act(&act_ff, h.d_ff, m->has_f16, error)) return false;
-    HIPQ(hipMalloc((void**)&d_tiles, (size_t)(1 + TK_MAX_ROWS) * 4));
-    HIPQ(hipMemset(d_tiles, 0, (size_t)(1 + TK_MAX_ROWS) * 4));
+    HIPQ(hipMalloc((void**)&x2, (size_t)TK_GEMV_FUSE_MAX_ROWS * h.d_model * 4));
+    HIPQ(hipMalloc((void**)&partial2, partial_floats(TK_GEMV_FUSE_MAX_ROWS) * 4));
+    if (!alloc_act(&act_d, h.d_model, pass_rows, m->has_f16, error) || !alloc_act(&act_qd, QD, pass_rows, m->has_f16, error) || !alloc_act(&act_ff, h.d_ff, pass_rows, m->has_f16, error)) return false;
+    HIPQ(hipMalloc((void**)&d_tiles, (size_t)(1 + pass_rows) * 4));
+    HIPQ(hipMemset(d_tiles, 0, (size_t)(1 + pass_rows) * 4));
     if (mctx > tk_long_att_min_pos(1, mctx) && tk_attention_long_applies(1, h.n_head, h.n_kv_head, h.head_dim))
         HIPQ(hipMalloc((void**)&d_scores, tk_attention_long_scratch_floats(h.n_head, h.head_dim, mctx) * sizeof(float)));
     /* RoPE table, double precision on the host (same formula as the oracle) */
@@ -311,7 +318,7 @@ TkLlmSession::~TkLlmSession() {
     for (auto& v : graph_exec) for (auto& g : v) if (g) (void)hipGraphExecDestroy(g);
     for (auto& v : graph_prefill) for (auto& g : v) if (g) (void)hipGraphExecDestroy(g);
     for (auto& v : graph_head_nf) for (auto& g : v) if (g) (void)hipGraphExecDestroy(g);
-    void* ptrs[] = {kcache, vcache, x, x2, qbuf, partial, partial2, rope_cos, rope_sin, d_tab, d_tiles, d_scores};
+    void* ptrs[] = {kcache, vcache, x, x2, x_last, qbuf, q_last, partial, partial2, rope_cos, rope_sin, d_tab, d_tiles, d_scores};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     free_act(&act_d); free_act(&act_qd); free_act(&act_ff);
 }
@@ -350,7 +357,8 @@ static void set_act(TkGemvArgs& a, const TkActQ8& q) {
 
 static TkGemvSeg seg_of(const TkDevTensor& t) { return TkGemvSeg{t.data, t.type, (int)(t.rows / TK_TILE_ROWS)}; }
 
-void TkLlmSession::enqueue_pass(int nrows, bool lm_head, bool fused_attn) { enqueue_range(nrows, 0, model->hp.n_layer, true, false, lm_head, fused_attn); }
+/* a pass without a head is read through the caches alone: its last layer ends with them */
+void TkLlmSession::enqueue_pass(int nrows, bool lm_head, bool fused_attn) { enqueue_range(nrows, 0, model->hp.n_layer, true, false, lm_head, fused_attn, !lm_head); }
 
 /* layers [l0, l1) of one pass.  embed: the residual stream starts from the token embeddings (first pipeline stage), otherwise x
  * already holds it.  fold_out: finish the last layer's residual update so x is the complete stream (it leaves this GPU).
@@ -363,7 +371,7 @@ int TkLlmSession::enqueue_matmul(const TkDevTensor* const* t, int nseg, int K, i
     if (t[0]->type == TK_TYPE_F16) {
         TkTiledGemm f{};
         for (int i = 0; i < nseg; ++i) { f.tiles[i] = t[i]->data; f.row_tiles[i] = (int)(t[i]->rows / TK_TILE_ROWS); }
-        f.nseg = nseg; f.wbytes = 2; f.K = K; f.ks = ks; f.ldc = n_total; f.n_valid = n_total; f.nrows = nrows; f.slab_rows = TK_MAX_ROWS;
+        f.nseg = nseg; f.wbytes = 2; f.K = K; f.ks = ks; f.ldc = n_total; f.n_valid = n_total; f.nrows = nrows; f.slab_rows = TK_SLAB_ROWS;
         f.a_img = act.af; f.a_ts = act.af_ts; f.out = out;
         /* shapes were validated when the model was installed (K a multiple of 256 ks); a refusal here would leave the slab unwritten, so it is
          * recorded and fails the pass (forward / decode / capture_pass check launch_error) instead of producing garbage silently */
@@ -384,7 +392,44 @@ static bool producer_fusion_enabled() {
     return !(nf && nf[0] == '1');
 }
 
-void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fold_out, bool lm_head, bool fused_attn) {
+/* a layer behind its attention (whose output act_qd holds): o projection, norm, MLP; the slabs of the residual update xs still lacks stay in `partial` */
+int TkLlmSession::enqueue_layer_tail(const TkLlmLayer& L, float* xs, int nrows) {
+    const TkLlmHParams& h = model->hp;
+    const int D = h.d_model, QD = h.n_head * h.head_dim, FF = h.d_ff;
+    hipStream_t s = stream;
+    const TkDevTensor* ot[1] = {&L.o};
+    const TkDevTensor* gu[2] = {&L.gate, &L.up};
+    const TkDevTensor* dn[1] = {&L.down};
+    const int ks_o = enqueue_matmul(ot, 1, QD, h.ks_o, D, act_qd, partial, nrows);
+    tk_launch_rmsnorm_q8(xs, partial, ks_o, D, (const float*)L.ffn_norm.data, h.rms_eps, D, nrows, act_d, s);
+    if (tk_gemv_fuses_swiglu(nrows, h.ks_gateup, L.gate.type, L.up.type)) { /* wide pass: SwiGLU in the launch's epilogue, `partial` holds h [rows][FF] */
+        TkGemvArgs a{};
+        a.seg[0] = seg_of(L.gate); a.seg[1] = seg_of(L.up);
+        a.nseg = 2; a.K = D; a.ks = 1; a.n_total = FF; a.nrows = nrows; a.swiglu = 1;
+        set_act(a, act_d); a.out = partial;
+        tk_launch_gemv(a, s);
+        tk_launch_quant_q8(partial, FF, nrows, act_ff, s);
+    } else {
+        const int ks_gu = enqueue_matmul(gu, 2, D, h.ks_gateup, 2 * FF, act_d, partial, nrows);
+        tk_launch_swiglu_q8(partial, ks_gu, FF, nrows, act_ff, s);
+    }
+    return enqueue_matmul(dn, 1, FF, h.ks_down, D, act_ff, partial, nrows);
+}
+
+/* the final norm, the logits matrix and the pick of the rows xs + the slabs in `partial` (ks_res == 0: none) */
+void TkLlmSession::enqueue_head(float* xs, int ks_res, int nrows) {
+    const TkLlmHParams& h = model->hp;
+    const int D = h.d_model;
+    const TkDevTensor* lm[1] = {&model->output};
+    tk_launch_rmsnorm_q8(xs, ks_res ? partial : nullptr, ks_res, D, (const float*)model->out_norm.data, h.rms_eps, D, nrows, act_d, stream);
+    (void)enqueue_matmul(lm, 1, D, 1, h.vocab, act_d, logits, nrows);
+    enqueue_pick(nrows);
+}
+void TkLlmSession::enqueue_pick(int nrows) {
+    tk_launch_argmax(logits, model->hp.vocab, nrows, d_mask, d_mask_row, d_samp, d_tok, d_pos, d_nsteps, d_hist, TK_MAX_ROWS, stream);
+}
+
+void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fold_out, bool lm_head, bool fused_attn, bool caches_only) {
     const TkLlmHParams& h = model->hp;
     const int D = h.d_model, QD = h.n_head * h.head_dim, KVD = h.n_kv_head * h.head_dim, FF = h.d_ff;
     hipStream_t s = stream;
@@ -427,14 +472,15 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
     for (int l = l0; l < l1; ++l) {
         const TkLlmLayer& L = model->layers[l];
         const TkDevTensor* qkv[3] = {&L.q, &L.k, &L.v};
-        const TkDevTensor* ot[1] = {&L.o};
-        const TkDevTensor* gu[2] = {&L.gate, &L.up};
-        const TkDevTensor* dn[1] = {&L.down};
         if (fuse) {
+            const TkDevTensor* ot[1] = {&L.o};
+            const TkDevTensor* gu[2] = {&L.gate, &L.up};
+            const TkDevTensor* dn[1] = {&L.down};
             const int ks_qkv = fused_gemv(qkv, 3, D, h.ks_qkv, QD + 2 * KVD, partial2, 1, x, x2, l == l0 ? nullptr : partial, ks_res, D, (const float*)L.attn_norm.data);
             if (!fused_attn)
                 tk_launch_qkv_rope_append(partial2, ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
                                           qbuf, kcache, vcache, l, max_seq, max_ctx, s);
+            if (caches_only && l == l1 - 1) { last_x = x2; return; }
             if (long_attn) tk_launch_attention_long(partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, !join_in_o, s);
             else if (tiled_attn) tk_launch_attention_prefill(qbuf, kcache, vcache, d_seq, d_pos, d_tiles, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, act_qd, s);
             else tk_launch_attention(qbuf, partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
@@ -449,37 +495,23 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
         if (!fused_attn)
             tk_launch_qkv_rope_append(partial, ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
                                       qbuf, kcache, vcache, l, max_seq, max_ctx, s);
+        if (caches_only && l == l1 - 1) { last_x = x; return; }
         if (long_attn) tk_launch_attention_long(partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, true, s);
         else if (tiled_attn) tk_launch_attention_prefill(qbuf, kcache, vcache, d_seq, d_pos, d_tiles, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, act_qd, s);
         else tk_launch_attention(qbuf, partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
                                  h.head_dim, l, max_seq, max_ctx, act_qd, fused_attn, s);
-        const int ks_o = enqueue_matmul(ot, 1, QD, h.ks_o, D, act_qd, partial, nrows);
-        tk_launch_rmsnorm_q8(x, partial, ks_o, D, (const float*)L.ffn_norm.data, h.rms_eps, D, nrows, act_d, s);
-        if (tk_gemv_fuses_swiglu(nrows, h.ks_gateup, L.gate.type, L.up.type)) { /* wide pass: SwiGLU in the launch's epilogue, `partial` holds h [rows][FF] */
-            TkGemvArgs a{};
-            a.seg[0] = seg_of(L.gate); a.seg[1] = seg_of(L.up);
-            a.nseg = 2; a.K = D; a.ks = 1; a.n_total = FF; a.nrows = nrows; a.swiglu = 1;
-            set_act(a, act_d); a.out = partial;
-            tk_launch_gemv(a, s);
-            tk_launch_quant_q8(partial, FF, nrows, act_ff, s);
-        } else {
-            const int ks_gu = enqueue_matmul(gu, 2, D, h.ks_gateup, 2 * FF, act_d, partial, nrows);
-            tk_launch_swiglu_q8(partial, ks_gu, FF, nrows, act_ff, s);
-        }
-        ks_res = enqueue_matmul(dn, 1, FF, h.ks_down, D, act_ff, partial, nrows);
+        ks_res = enqueue_layer_tail(L, x, nrows);
     }
     last_ks_res = ks_res;
     if (!lm_head) { /* prompt rows whose logits nobody reads (K/V are already appended), or a pipeline stage that hands x on */
         if (fold_out && l1 > l0) tk_launch_residual_fold(x, partial, ks_res, D, D, nrows, s);
         return;
     }
-    const TkDevTensor* lm[1] = {&model->output};
-    if (fuse) (void)fused_gemv(lm, 1, D, 1, h.vocab, logits, 1, x, x2, l1 > l0 ? partial : nullptr, ks_res, D, (const float*)model->out_norm.data);
-    else {
-        tk_launch_rmsnorm_q8(x, l1 > l0 ? partial : nullptr, ks_res, D, (const float*)model->out_norm.data, h.rms_eps, D, nrows, act_d, s);
-        (void)enqueue_matmul(lm, 1, D, 1, h.vocab, act_d, logits, nrows);
-    }
-    tk_launch_argmax(logits, h.vocab, nrows, d_mask, d_mask_row, d_samp, d_tok, d_pos, d_nsteps, d_hist, TK_MAX_ROWS, s);
+    if (fuse) {
+        const TkDevTensor* lm[1] = {&model->output};
+        (void)fused_gemv(lm, 1, D, 1, h.vocab, logits, 1, x, x2, l1 > l0 ? partial : nullptr, ks_res, D, (const float*)model->out_norm.data);
+        enqueue_pick(nrows);
+    } else enqueue_head(x, l1 > l0 ? ks_res : 0, nrows);
 }
 
 #ifndef TK_TILED_ATT_MIN_POS
@@ -592,48 +624,70 @@ __global__ void k_stage_rows(const int32_t* __restrict__ tab, int n, int stride,
     if (i < n) { seq[i] = tab[i]; pos[i] = tab[stride + i]; tok[i] = tab[2 * stride + i]; }
 }
 
-/* Prompt rows that nobody samples from (all but the last token of every prompt): the whole schedule — (sequence, position, token) of
- * every row of every pass — is uploaded once, each pass is one tiny staging launch + one replay of a captured pass (no lm_head,
- * rope/append as its own kernel so a pass may hold several positions of one sequence), and the host synchronises once, in the final
- * sampling pass.  Same kernels, same order, same arithmetic as forward(): bit-identical results. */
+/* the residual stream and the query of every sequence's last position that rows [off, off + n) of the schedule hold; one workgroup a sequence */
+__global__ __launch_bounds__(256) void k_keep_last(const float* __restrict__ x, float* __restrict__ x_last, int D, const float* __restrict__ q, float* __restrict__ q_last, int QD,
+                                                   int64_t off, int n, int n_prompt) {
+    const int64_t r = (int64_t)blockIdx.x * n_prompt + n_prompt - 1 - off;
+    if (r < 0 || r >= n) return;
+    for (int i = threadIdx.x; i < D; i += 256) x_last[(int64_t)blockIdx.x * D + i] = x[r * D + i];
+    for (int i = threadIdx.x; i < QD; i += 256) q_last[(int64_t)blockIdx.x * QD + i] = q[r * QD + i];
+}
+
+/* Whole prompts: the schedule — (sequence, position, token) of every row of every pass — is uploaded once; a pass is a tiny staging launch and its layers' launches
+ * (rope/append as its own kernel so a pass may hold several positions of one sequence), enqueued as they are: a pass of hundreds of rows runs longer than the host takes
+ * to enqueue it, and a graph per row count would be captured for every new length.  Nobody reads what the last layer makes of a row that is not sampled, so passes end
+ * with its keys and values, and its attention, MLP and the head run once, over the last position of every prompt (k_keep_last).  The arithmetic of every row is
+ * forward()'s: bit-identical results. */
 bool TkLlmSession::prefill(int nseq, int n_prompt, const int32_t* tokens, int32_t* first_tokens_host) {
     if (nseq <= 0 || nseq > TK_MAX_ROWS || nseq > max_seq) { error = "nseq must be in [1, min(256, max_seq)]"; return false; }
     if (n_prompt <= 0 || n_prompt >= max_ctx) { error = "prompt does not fit the context"; return false; }
     for (int64_t i = 0; i < (int64_t)nseq * n_prompt; ++i)
         if (tokens[i] < 0 || tokens[i] >= model->hp.vocab) { error = "row out of range (sequence id, position or token id)"; return false; }
     HIPQ(hipSetDevice(model->device));
-    /* all but the last prompt token: up to 256 rows per pass, positions ascending inside a sequence so causality holds inside a pass */
-    const int64_t total = (int64_t)nseq * (n_prompt - 1);
-    if (total > 0) {
-        std::vector<int32_t> tab((size_t)3 * total);
-        int64_t k = 0;
-        for (int s = 0; s < nseq; ++s)
-            for (int p = 0; p + 1 < n_prompt; ++p, ++k) {
-                tab[k] = s; tab[total + k] = p; tab[2 * total + k] = tokens[(size_t)s * n_prompt + p];
-            }
-        if ((int64_t)tab_cap < 3 * total) {
-            if (d_tab) (void)hipFree(d_tab);
-            d_tab = nullptr;
-            HIPQ(hipMalloc((void**)&d_tab, (size_t)3 * total * 4));
-            tab_cap = (size_t)3 * total;
+    const TkLlmHParams& h = model->hp;
+    const int QD = h.n_head * h.head_dim, KVD = h.n_kv_head * h.head_dim, last = h.n_layer - 1;
+    /* every position of every prompt, sequence by sequence (ascending, so causality holds inside a pass and from pass to pass), then the sampled rows again */
+    const int64_t total = (int64_t)nseq * n_prompt, cols = total + nseq;
+    std::vector<int32_t> tab((size_t)3 * cols);
+    for (int64_t s = 0; s < nseq; ++s)
+        for (int64_t p = 0; p < n_prompt; ++p) {
+            const int64_t k = s * n_prompt + p;
+            tab[k] = (int32_t)s; tab[cols + k] = (int32_t)p; tab[2 * cols + k] = tokens[k];
+            if (p + 1 == n_prompt) { tab[total + s] = (int32_t)s; tab[cols + total + s] = (int32_t)p; tab[2 * cols + total + s] = tokens[k]; }
         }
-        HIPQ(hipMemcpyAsync(d_tab, tab.data(), (size_t)3 * total * 4, hipMemcpyHostToDevice, stream));
-        HIPQ(hipStreamSynchronize(stream)); /* `tab` is pageable host memory that dies with this scope */
-        const bool use_graph = graphs_enabled();
-        for (int64_t off = 0; off < total; off += TK_MAX_ROWS) {
-            const int n = (int)std::min<int64_t>(TK_MAX_ROWS, total - off);
-            choose_attention(tab.data() + total + off, n);
-            if (use_graph && !capture_pass(&graph_prefill[tiled_pass][n], n, false, false)) return false;
-            hipLaunchKernelGGL(k_stage_rows, dim3((n + 255) / 256), dim3(256), 0, stream, d_tab + off, n, (int)total, d_seq, d_pos, d_tok);
-            if (use_graph) HIPQ(hipGraphLaunch(graph_prefill[tiled_pass][n], stream));
-            else { launch_error.clear(); enqueue_pass(n, false, false); if (!launch_error.empty()) { error = launch_error; return false; } }
-        }
-        HIPQ(hipGetLastError());
+    if ((int64_t)tab_cap < 3 * cols) {
+        if (d_tab) (void)hipFree(d_tab);
+        d_tab = nullptr;
+        tab_cap = 0;
+        HIPQ(hipMalloc((void**)&d_tab, (size_t)3 * cols * 4));
+        tab_cap = (size_t)3 * cols;
     }
-    /* last prompt token of every sequence: row r == sequence r, sampled -> decode() continues from here */
-    std::vector<int32_t> sq(nseq), ps(nseq), tk(nseq);
-    for (int s = 0; s < nseq; ++s) { sq[s] = s; ps[s] = n_prompt - 1; tk[s] = tokens[(size_t)s * n_prompt + n_prompt - 1]; }
-    return forward(nseq, sq.data(), ps.data(), tk.data(), nullptr, first_tokens_host, true);
+    HIPQ(hipMemcpyAsync(d_tab, tab.data(), (size_t)3 * cols * 4, hipMemcpyHostToDevice, stream));
+    HIPQ(hipMemsetAsync(d_nsteps, 0, TK_MAX_ROWS * 4, stream));
+    HIPQ(hipStreamSynchronize(stream)); /* `tab` is pageable host memory that dies with this scope */
+    if (!stage_sampling(nseq, nullptr, nullptr, nullptr)) return false;
+    auto stage = [&](int64_t at, int n) { hipLaunchKernelGGL(k_stage_rows, dim3((n + 255) / 256), dim3(256), 0, stream, d_tab + at, n, (int)cols, d_seq, d_pos, d_tok); };
+    launch_error.clear();
+    /* passes of as many whole parts of the wide kernel as there are, in equal shares */
+    const int64_t n_passes = (total + pass_rows - 1) / pass_rows;
+    const int share = (int)std::min<int64_t>(pass_rows, ((total + n_passes - 1) / n_passes + 127) / 128 * 128);
+    for (int64_t off = 0; off < total; off += share) {
+        const int n = (int)std::min<int64_t>(share, total - off);
+        choose_attention(tab.data() + cols + off, n);
+        stage(off, n);
+        enqueue_range(n, 0, h.n_layer, true, false, false, false, true);
+        hipLaunchKernelGGL(k_keep_last, dim3(nseq), dim3(256), 0, stream, last_x, x_last, h.d_model, qbuf, q_last, QD, off, n, n_prompt);
+    }
+    /* the last layer of the sampled rows alone: their queries over the caches, which now hold every position */
+    stage(total, nseq);
+    tk_launch_attention(q_last, partial, h.ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nseq, h.n_head, h.n_kv_head, h.head_dim, last, max_seq, max_ctx,
+                        act_qd, false, stream);
+    enqueue_head(x_last, enqueue_layer_tail(model->layers[last], x_last, nseq), nseq);
+    if (!launch_error.empty()) { error = launch_error; (void)hipStreamSynchronize(stream); return false; }
+    HIPQ(hipGetLastError());
+    if (first_tokens_host) HIPQ(hipMemcpyAsync(first_tokens_host, d_tok, nseq * 4, hipMemcpyDeviceToHost, stream));
+    HIPQ(hipStreamSynchronize(stream));
+    return true;
 }
 
 bool TkLlmSession::time_gemv(int layer, int which, int nrows, int iters, float* avg_ms, double* algo_bytes) {

@@ -302,7 +302,7 @@ __global__ __launch_bounds__(1024) void k_rmsnorm_q8(float* __restrict__ x, cons
             v4f p[TK_RMS_MAX_KS];
 #pragma unroll
             for (int s = 0; s < TK_RMS_MAX_KS; ++s)
-                if (s < ks) p[s] = *(const v4f*)(partial + ((int64_t)s * TK_MAX_ROWS + r) * n_total + 4 * g);
+                if (s < ks) p[s] = *(const v4f*)(partial + ((int64_t)s * TK_SLAB_ROWS + r) * n_total + 4 * g);
             v4f o = p[0];
 #pragma unroll
             for (int s = 1; s < TK_RMS_MAX_KS; ++s)
@@ -353,7 +353,7 @@ __global__ __launch_bounds__(256) void k_residual_fold(float* __restrict__ x, co
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (4 * g >= D) return;
     v4f o = *(const v4f*)(partial + (int64_t)r * n_total + 4 * g);
-    for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + ((int64_t)s * TK_MAX_ROWS + r) * n_total + 4 * g);
+    for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + ((int64_t)s * TK_SLAB_ROWS + r) * n_total + 4 * g);
     v4f* xp = (v4f*)(x + (int64_t)r * D + 4 * g);
     *xp = *xp + o;
 }
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                         v4f p[TK_RMS_MAX_KS];
 #pragma unroll
                         for (int sl = 0; sl < TK_RMS_MAX_KS; ++sl)
-                            if (sl < a.fks) p[sl] = *(const v4f*)(a.fslab + ((int64_t)sl * TK_MAX_ROWS + r) * a.fn_total + 4 * gi);
+                            if (sl < a.fks) p[sl] = *(const v4f*)(a.fslab + ((int64_t)sl * TK_SLAB_ROWS + r) * a.fn_total + 4 * gi);
                         v4f o = p[0];
 #pragma unroll
                         for (int sl = 1; sl < TK_RMS_MAX_KS; ++sl)
@@ -730,7 +730,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
 #pragma unroll
                         for (int sl = 0; sl < TK_RMS_MAX_KS; ++sl)
                             if (sl < a.fks) {
-                                const float* row = a.fslab + ((int64_t)sl * TK_MAX_ROWS + r) * (2 * (int64_t)FF);
+                                const float* row = a.fslab + ((int64_t)sl * TK_SLAB_ROWS + r) * (2 * (int64_t)FF);
                                 pg[sl][0] = *(const v4f*)(row + 8 * c); pg[sl][1] = *(const v4f*)(row + 8 * c + 4);
                                 pu[sl][0] = *(const v4f*)(row + FF + 8 * c); pu[sl][1] = *(const v4f*)(row + FF + 8 * c + 4);
                             }
@@ -847,7 +847,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
             /* default-policy stores: the <= 1 MB of slabs of a narrow pass stay in L2 / the Infinity Cache for the consumer kernel, which is one
              * load latency long (decode step 2.277 -> 2.207 ms at 16 rows, 2.108 -> 2.038 ms at 1 row against non-temporal stores,
              * profiles/r03_smallbatch_variants.txt); the wide kernels keep non-temporal stores (29 MB per launch would only evict) */
-            if (row < a.nrows) a.out[((size_t)ksi * TK_MAX_ROWS + row) * a.n_total + n] = acc[m][r];
+            if (row < a.nrows) a.out[((size_t)ksi * TK_SLAB_ROWS + row) * a.n_total + n] = acc[m][r];
         }
 }
 
@@ -1126,14 +1126,14 @@ __global__ __launch_bounds__(NT == 2 ? 256 : 512) void k_gemm_w4a8(TkGemvArgs a,
             for (int r = 0; r < 4; ++r) {
                 const int mt = rot == 0 ? m : (m < MT / 2 ? m + rot : m - rot); /* register slot m holds M-tile m ^ rot (the half-swap: MT = 6 is no power of two) */
                 const int row = mt * TK_ROW_SLOTS + 4 * g + r;
-                if (row < a.nrows) __builtin_nontemporal_store(acc[w][m][r], &a.out[((size_t)ksi * TK_MAX_ROWS + row) * a.n_total + n]);
+                if (row < a.nrows) __builtin_nontemporal_store(acc[w][m][r], &a.out[((size_t)ksi * TK_SLAB_ROWS + row) * a.n_total + n]);
             }
     }
 }
 
 
 /* ------------------------------------------------------------------------------------------
- * Wide passes (193..256 rows by default, from 129 with TK_MI355X_G32_FROM=129): the same arithmetic on v_mfma_i32_32x32x32_i8.
+ * Wide passes (from 193 rows, or from 129 with TK_MI355X_G32_FROM=129): the same arithmetic on v_mfma_i32_32x32x32_i8.
  *
  * Why: per (16 rows x 16 weight rows x 256 k) the 16x16x64 formulation above issues 8 int8 MFMAs + 1 f16 MFMA (9 x 8 issue cycles) and four
  * ds_read_b128; the 32x32x32 form does the same multiply-adds with HALF the MFMA issue slots and HALF the LDS operand bytes per MAC (one
@@ -1275,8 +1275,7 @@ __device__ __forceinline__ void load_atile32(ATile32& T, const Ptrs32& p, int t)
 
 /* one 256-k block: this wave's 32 weight rows x its four 32-row M-tiles.  T arrives holding tile 0's operands; the operands of tile
  * t + 1 are requested as soon as the MFMAs of tile t have issued — into the same registers — and land while tile t is finished on the VALU. */
-/* MTW = 32-row M-tiles a workgroup's row range holds: 3 for passes of 129..192 rows (two halves of 96 rows), 4 for 193..256 — a pass of 160
- * rows walks 3 + 3 tiles, not 4 + 4 (round 5: the 129th row cost + 63 %, profiles/r05_width_curve.txt).  A compile-time bound: 48 or 64
+/* MTW = 32-row M-tiles a workgroup's row range holds, 4 or 3 (tk_launch_gemv).  A compile-time bound: 48 or 64
  * accumulators and no branch in the loop.  (One tile fewer for the second half of 129..160- and 193..224-row passes as a scalar `break` in the
  * unrolled loop was built too: 108 - 392 bytes of spill per lane at the 256-register budget of two workgroups per CU; not kept.) */
 template <bool Q4, int MTW, typename Hook>
@@ -1403,16 +1402,17 @@ __device__ __forceinline__ void g32_k_loop(const uint8_t* tile, size_t tile_byte
     }
 }
 
-/* 193..256 rows (129..192 as MTW = 3 under TK_MI355X_G32_FROM; and one row half alone).  A workgroup = 4 waves, one per SIMD = four pairs of weight tiles (128 weight rows) x ONE half
- * of the pass's rows (128 rows = four 32-row M-tiles per wave); the two row halves of the same weights are two workgroups that share a CU
- * (73 KiB of ring each) and nothing else.  The SIMD's two resident waves therefore belong to DIFFERENT workgroups: no barrier couples
+/* A workgroup = 4 waves, one per SIMD = four pairs of weight tiles (128 weight rows) x ONE part of the pass's rows (128 or 96 rows = MTW 32-row M-tiles per wave).  Two
+ * workgroups share a CU (73 KiB of ring each) and nothing else.  The SIMD's two resident waves therefore belong to DIFFERENT workgroups: no barrier couples
  * them, so one's weight unpack (190 VALU instructions, no MFMA) drifts under the other's MFMA phases.  With both halves in one 8-wave
  * workgroup the block barrier re-aligned the partners every 256 k — both unpacked at once, then the later one finished alone:
  * 8750 cycles per block against 4352 of matrix pipe (profiles/r03_gemm32_segments.txt).
- * blockIdx -> (half, unit): consecutive workgroup ids go round the 8 XCDs, so the two halves of a unit are 8 ids apart: same XCD, same
- * L2 — the second half's weight requests hit the lines the first one brought in. */
+ * blockIdx -> (part, unit): consecutive workgroup ids go round the 8 XCDs, so the parts of a unit are 8 ids apart: same XCD, same
+ * L2 — the further parts' weight requests hit the lines the first one brought in.
+ * Passes of more than 256 rows take as many parts as they need: 256 rows alone are 448 (gate | up, down), 384 (q | k | v) or 256 (o) workgroups on 512 slots, with a ramp and
+ * a tail each.  A prompt of 8 192 rows through 32 layers, 4096 wide: passes of 256 rows 6.3 ms each, of 2 048 rows 41. */
 template <int TYPES, int MTW>
-__global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups, int total_row_tiles, int n_halves) {
+__global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups, int total_row_tiles, int n_parts) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int MT = TK_G32_MT;
     constexpr int CH = MT * TK_RING_TILE_BYTES;   /* one block of the ring */
@@ -1421,17 +1421,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
     const int pair = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nb = a.K / a.ks / 256;
     const int nblk_total = a.K / 256;
-    int half = 0, unit = blockIdx.x;
-    if (n_halves == 2) {
-        const int units = gridDim.x >> 1, body = (units >> 3) << 4; /* ids below `body`: XCD-aligned pairs; the rest (units not a multiple of 8) adjacent */
+    int rpart = 0, unit = blockIdx.x;
+    if (n_parts > 1) {
+        const int units = gridDim.x / n_parts, body = (units & ~7) * n_parts; /* ids below `body`: a unit's parts on one XCD; the rest (units not a multiple of 8) adjacent */
         if ((int)blockIdx.x < body) {
             const int x = blockIdx.x & 7, idx = blockIdx.x >> 3;
-            half = idx & 1;
-            unit = (idx >> 1) * 8 + x;
+            rpart = idx % n_parts;
+            unit = idx / n_parts * 8 + x;
         } else {
             const int r = blockIdx.x - body;
-            half = r & 1;
-            unit = (body >> 1) + (r >> 1);
+            rpart = r % n_parts;
+            unit = (units & ~7) + r / n_parts;
         }
     }
     const int ksi = unit % a.ks;
@@ -1464,10 +1464,10 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
     /* ring staging: of the half's eight 16-row M-tiles, `pair` and `pair + 4` belong to this wave.  The int8 image (4 x 1 KiB pieces per
      * tile, every lane takes part: no exec masking, so the issue can sit between the MFMA phases of the tile loop) in four parts of two
      * pieces; the f16 sub-block sums (32 lanes) and the block scales (4 lanes) separately at the top of a block */
-    /* rows of the pass as 32-row tiles: each half takes MTW of them (rows beyond the pass are computed on whatever the image holds and never stored) */
-    const int t32_0 = half * MTW; /* this half's first 32-row tile */
-    const int m0 = 2 * t32_0;     /* the half's first 16-row M-tile in the pass's activation images */
-    /* the ring is staged whole (eight 16-row M-tiles per block) whatever MTW: the images of all sixteen M-tiles exist (TK_MAX_ROWS), a tile nobody
+    /* rows of the pass as 32-row tiles: each part takes MTW of them (rows beyond the pass are computed on whatever the image holds and never stored) */
+    const int t32_0 = rpart * MTW; /* this part's first 32-row tile */
+    const int m0 = 2 * t32_0;     /* the part's first 16-row M-tile in the pass's activation images */
+    /* the ring is staged whole (eight 16-row M-tiles per block) whatever MTW: the images hold TK_SPARE_TILES M-tiles more than a pass, a tile nobody
      * reads costs L2 -> LDS bytes only, and a branch around the DMA issue inside the tile loop costs registers (148 bytes of spill per lane measured) */
     /* addresses = wave-uniform base (SGPR pair) + this lane's 32-bit offset, formed where they are used: the compiler otherwise hoists five
      * 64-bit per-lane addresses out of the K loop and holds ten registers for them across it (the asm keeps the offset opaque per use) */
@@ -1545,7 +1545,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
                 const int rl = 8 * i + (lane >> 3);
                 const v4f v = *(const v4f*)(sp + rl * 32 + 4 * (lane & 7));
                 const int row = (t32_0 + t) * 32 + rl;
-                if (row < a.nrows) *(v4f*)&a.out[((size_t)ksi * TK_MAX_ROWS + row) * a.n_total + n0] = v;
+                if (row < a.nrows) *(v4f*)&a.out[((size_t)ksi * TK_SLAB_ROWS + row) * a.n_total + n0] = v;
             }
         }
     }
@@ -1601,16 +1601,21 @@ void tk_launch_gemv(const TkGemvArgs& a, hipStream_t s) {
     /* 129..192 rows: the 16x16x64 kernel at ten / twelve M-tiles (its time grows by ~0.4 ms per 32 rows: 3.3 / 3.7 ms per decode step's launch set
      * against 4.2 of the 32x32x32 kernel at three tiles per half, profiles/r06_width_curve.txt); TK_MI355X_G32_FROM=129 keeps the round-5 split */
     if (a.nrows >= tk_g32_from()) {
-        /* tk_g32_from() .. 256 rows: the 32x32x32 kernel, one type per wave (a mixed q / k / v launch needs no split): four (weight-tile pair) slots per
-         * workgroup, one workgroup per row half */
+        /* from tk_g32_from() rows on: the 32x32x32 kernel, one type per wave (a mixed q / k / v launch needs no split): four (weight-tile pair) slots per
+         * workgroup, one workgroup per part of the rows */
         const int pairs = a.swiglu ? a.seg[0].row_tiles : row_tiles / 2; /* every segment holds a multiple of 4 row tiles: pairs never straddle segments */
         const int g32 = (pairs + 3) / 4;
-        const int n_halves = a.nrows > 8 * TK_ROW_SLOTS ? 2 : 1;
-        const int tiles32 = (a.nrows + 31) / 32; /* 5..8 at 129..256 rows: two halves of 3 (<= 192 rows) or 4 tiles */
+        /* parts of 128 rows (four 32-row tiles a wave) or of 96, whichever makes the shorter pass: a block costs a wave its weights' unpack, worth one and a half
+         * tiles, and its tiles (1 980 and 1 315 cycles).  Prompts of 260, 288, 544 rows through 16 layers, all parts of 128 / by this rule: 5.20 / 4.75, 5.38 / 4.92,
+         * 8.71 / 8.47 ms; one part alone always holds four tiles */
+        const int tiles32 = (a.nrows + 31) / 32;
+        const int parts4 = (tiles32 + 3) / 4, parts3 = (tiles32 + 2) / 3;
+        const bool four = parts4 == 1 || 11 * parts4 <= 9 * parts3;
+        const int n_parts = four ? parts4 : parts3;
         const size_t ldsb = (size_t)2 * TK_G32_MT * TK_RING_TILE_BYTES;
-        const dim3 grid(g32 * a.ks * n_halves);
-#define TK_G32_LAUNCH_M(TYV, MTWV) hipLaunchKernelGGL((k_gemm32_w4a8<TYV, MTWV>), grid, dim3(256), ldsb, s, a, g32, row_tiles, n_halves)
-#define TK_G32_LAUNCH(TYV) do { if (n_halves == 1 || tiles32 > 6) TK_G32_LAUNCH_M(TYV, 4); else TK_G32_LAUNCH_M(TYV, 3); } while (0)
+        const dim3 grid(g32 * a.ks * n_parts);
+#define TK_G32_LAUNCH_M(TYV, MTWV) hipLaunchKernelGGL((k_gemm32_w4a8<TYV, MTWV>), grid, dim3(256), ldsb, s, a, g32, row_tiles, n_parts)
+#define TK_G32_LAUNCH(TYV) do { if (four) TK_G32_LAUNCH_M(TYV, 4); else TK_G32_LAUNCH_M(TYV, 3); } while (0)
         if (types == 1) TK_G32_LAUNCH(1);
         else if (types == 2) TK_G32_LAUNCH(2);
         else TK_G32_LAUNCH(3);
@@ -1678,7 +1683,7 @@ template <int KS> __device__ __forceinline__ float2 sum_slabs_pair(const float* 
 }
 __device__ __forceinline__ float2 sum_partials_pair(const float* partial, int ks, int n_total, int row, int col) {
     const float* p = partial + (int64_t)row * n_total;
-    const int64_t pitch = (int64_t)TK_MAX_ROWS * n_total;
+    const int64_t pitch = (int64_t)TK_SLAB_ROWS * n_total;
     switch (ks) {
     case 1: return sum_slabs_pair<1>(p, pitch, (uint32_t)col);
     case 2: return sum_slabs_pair<2>(p, pitch, (uint32_t)col);
@@ -2175,32 +2180,39 @@ __global__ __launch_bounds__(1024) void k_attention_narrow(const float* __restri
  * wave w computes score tile w of every 64-position block and owns PV class j = w.  Keys sit in LDS in B-operand order (lane group g's
  * dims g, g + 4, ... contiguous), values row-major with padded rows; both are fetched one block ahead into registers.
  * ------------------------------------------------------------------------------------------ */
-__global__ __launch_bounds__(256) void k_att_tiles(const int32_t* __restrict__ seq, int nrows, int32_t* __restrict__ tiles) {
-    __shared__ int sq[TK_MAX_ROWS], run0[TK_MAX_ROWS], cnt[TK_MAX_ROWS];
-    const int t = threadIdx.x;
-    sq[t] = t < nrows ? seq[t] : -1;
-    __syncthreads();
-    run0[t] = (t < nrows && (t == 0 || sq[t] != sq[t - 1])) ? t : 0; /* start of the run a row belongs to: running maximum of the starts */
-    __syncthreads();
-    for (int d = 1; d < TK_MAX_ROWS; d <<= 1) {
-        const int v = t >= d ? (run0[t] > run0[t - d] ? run0[t] : run0[t - d]) : run0[t];
+#define TK_AT_THREADS 1024
+#define TK_AT_PER (TK_PASS_ROWS / TK_AT_THREADS)
+/* a[i] = op(a[0 .. i]) for i < n; every thread of the workgroup takes part and holds rows t, t + blockDim.x, .. */
+template <typename Op> __device__ __forceinline__ void att_tiles_scan(int* a, int n, Op op) {
+    const int t = threadIdx.x, w = blockDim.x;
+    for (int d = 1; d < n; d <<= 1) {
+        int v[TK_AT_PER];
+#pragma unroll
+        for (int k = 0; k < TK_AT_PER; ++k) { const int i = t + k * w; v[k] = i < n ? (i >= d ? op(a[i], a[i - d]) : a[i]) : 0; }
         __syncthreads();
-        run0[t] = v;
-        __syncthreads();
-    }
-    const bool head = t < nrows && ((t - run0[t]) & 15) == 0; /* a tile starts every 16 rows of a run */
-    int len = 0;
-    if (head) { len = 1; while (len < 16 && t + len < nrows && sq[t + len] == sq[t]) ++len; }
-    cnt[t] = head ? 1 : 0;
-    __syncthreads();
-    for (int d = 1; d < TK_MAX_ROWS; d <<= 1) { /* inclusive prefix sum: the tile's index */
-        const int v = t >= d ? cnt[t] + cnt[t - d] : cnt[t];
-        __syncthreads();
-        cnt[t] = v;
+#pragma unroll
+        for (int k = 0; k < TK_AT_PER; ++k) { const int i = t + k * w; if (i < n) a[i] = v[k]; }
         __syncthreads();
     }
-    if (head) tiles[cnt[t]] = t | (len << 16); /* tiles[1 ..] */
-    if (t == TK_MAX_ROWS - 1) tiles[0] = cnt[t];
+}
+__global__ __launch_bounds__(TK_AT_THREADS) void k_att_tiles(const int32_t* __restrict__ seq, int nrows, int32_t* __restrict__ tiles) {
+    __shared__ int sq[TK_PASS_ROWS], run0[TK_PASS_ROWS], cnt[TK_PASS_ROWS];
+    const int t = threadIdx.x, w = blockDim.x;
+    for (int i = t; i < nrows; i += w) sq[i] = seq[i];
+    __syncthreads();
+    for (int i = t; i < nrows; i += w) run0[i] = i == 0 || sq[i] != sq[i - 1] ? i : 0; /* start of the run a row belongs to: running maximum of the starts */
+    __syncthreads();
+    att_tiles_scan(run0, nrows, [](int x, int y) { return x > y ? x : y; });
+    for (int i = t; i < nrows; i += w) cnt[i] = ((i - run0[i]) & 15) == 0 ? 1 : 0; /* a tile starts every 16 rows of a run */
+    __syncthreads();
+    att_tiles_scan(cnt, nrows, [](int x, int y) { return x + y; }); /* the tile's number, from 1 */
+    for (int i = t; i < nrows; i += w) {
+        if (((i - run0[i]) & 15) != 0) continue;
+        int len = 1;
+        while (len < 16 && i + len < nrows && sq[i + len] == sq[i]) ++len;
+        tiles[cnt[i]] = i | (len << 16); /* tiles[1 ..] */
+    }
+    if (t == 0) tiles[0] = cnt[nrows - 1];
 }
 
 template <int HD>
@@ -2691,7 +2703,7 @@ bool tk_attention_prefill_applies(int n_head, int n_kv_head, int head_dim) {
 }
 
 void tk_launch_att_tiles(const int32_t* seq, int nrows, int32_t* tiles, hipStream_t s) {
-    hipLaunchKernelGGL(k_att_tiles, dim3(1), dim3(TK_MAX_ROWS), 0, s, seq, nrows, tiles);
+    hipLaunchKernelGGL(k_att_tiles, dim3(1), dim3(nrows < TK_AT_THREADS ? (nrows + 63) / 64 * 64 : TK_AT_THREADS), 0, s, seq, nrows, tiles);
 }
 
 void tk_launch_attention_prefill(const float* qbuf, const uint16_t* kcache, const uint16_t* vcache, const int32_t* seq, const int32_t* pos,
@@ -2832,7 +2844,7 @@ __global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks,
 #pragma unroll
         for (int s = 0; s < KSM; ++s)
             if (s < ks) {
-                const float* row = partial + ((int64_t)s * TK_MAX_ROWS + r) * (2 * (int64_t)FF);
+                const float* row = partial + ((int64_t)s * TK_SLAB_ROWS + r) * (2 * (int64_t)FF);
                 pg[s][0] = *(const v4f*)(row + 8 * c); pg[s][1] = *(const v4f*)(row + 8 * c + 4);
                 pu[s][0] = *(const v4f*)(row + FF + 8 * c); pu[s][1] = *(const v4f*)(row + FF + 8 * c + 4);
             }

@@ -37,7 +37,7 @@
  *                                      the A operand of the MFMA that contracts them with the 6-bit mins
  *      abs16: f16   [K/256][2][16][8]  the same sums as sum = 2 hh + ll (|hh| <= 2032, ll in {0, 1}: exact in f16) — the batched kernel
  *                                      contracts them with (2 m_j, m_j) in ONE v_mfma_f32_16x16x32_f16 (exact: every partial sum < 2^24)
- *  "row slot" b < 16 is a (sequence, position) row of the current pass; a pass holds up to TK_MAX_TILES such
+ *  "row slot" b < 16 is a (sequence, position) row of the current pass; a caller's pass holds up to TK_MAX_TILES such
  *  16-row M-tiles (row r lives in tile r / 16, slot r % 16), each with its own aq / ad / abs image.
  */
 #ifndef TK_LLM_LAYOUT_H
@@ -49,8 +49,14 @@
 #define TK_Q4K_TILE_BYTES 2304
 #define TK_Q6K_TILE_BYTES 3360
 #define TK_ROW_SLOTS 16  /* rows of one MFMA M-tile */
-#define TK_MAX_TILES 16   /* M-tiles per pass: a weight tile is unpacked once and multiplied against all of them */
+#define TK_MAX_TILES 16   /* M-tiles per caller's pass: a weight tile is unpacked once and multiplied against all of them */
 #define TK_MAX_ROWS (TK_ROW_SLOTS * TK_MAX_TILES)
+/* Rows of a whole prompt's pass (TkLlmSession::prefill), several times a caller's pass: a launch of 256 rows fills the chip's workgroup slots to 0.5 (o) .. 0.875 (gate | up)
+ * and pays its ramp and its tail for those rows alone.  256 prompts of 32 positions, 32 layers 4096 wide, in passes of 256, 512, 1024, 2048 rows: 216, 191, 175, 166 ms.
+ * K-split slabs are TK_SLAB_ROWS rows apart in every pass. */
+#define TK_PASS_ROWS 2048
+#define TK_SLAB_ROWS TK_PASS_ROWS
+#define TK_SPARE_TILES 8 /* M-tiles behind a pass's last that the images hold: a part of 96 rows stages eight tiles */
 
 /* per M-tile sizes; tile m of a buffer starts at m * (these) */
 #define TK_AQ_BYTES(K) ((size_t)(K) * TK_ROW_SLOTS)

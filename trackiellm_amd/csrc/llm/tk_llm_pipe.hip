@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void k_pipe_send_x(const float* __restrict__ x
         v4f v = *(const v4f*)(x + (int64_t)r * D + 4 * g);
         if (partial) {
             v4f o = *(const v4f*)(partial + (int64_t)r * n_total + 4 * g);
-            for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + ((int64_t)s * TK_MAX_ROWS + r) * n_total + 4 * g);
+            for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + ((int64_t)s * TK_SLAB_ROWS + r) * n_total + 4 * g);
             v = v + o;
         }
         const int64_t at = (int64_t)r * (D / 4) + g;

@@ -37,7 +37,7 @@ struct TkTiledGemm {
     int ldc;                 /* row pitch of out (and of the K-split slabs) */
     int n_valid;             /* columns actually stored (N; the last tile may be padding) */
     int nrows;
-    int slab_rows;           /* rows per K-split slab (ks > 1): TK_MAX_ROWS of the LLM path */
+    int slab_rows;           /* rows per K-split slab (ks > 1), at least nrows: TK_SLAB_ROWS of the LLM path */
     const float* a_img;
     size_t a_ts;             /* floats between M-tiles of the image = 16 K */
     float* out;

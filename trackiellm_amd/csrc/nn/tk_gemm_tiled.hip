@@ -546,7 +546,7 @@ bool tk_gemm_tiled_prepare_device() {
 }
 
 static bool tw_valid(const TkTiledGemm& a) {
-    if (a.nseg < 1 || a.nseg > 3 || a.ks < 1 || a.K <= 0 || a.K % (32 * a.ks) || a.nrows <= 0 || (a.wbytes != 2 && a.wbytes != 4) || (a.ks > 1 && a.nrows > TK_TW_MAX_BLOCK_ROWS)) return false;
+    if (a.nseg < 1 || a.nseg > 3 || a.ks < 1 || a.K <= 0 || a.K % (32 * a.ks) || a.nrows <= 0 || (a.wbytes != 2 && a.wbytes != 4) || (a.ks > 1 && a.nrows > a.slab_rows)) return false;
     if ((a.per_seg || a.c_img) && a.ks != 1) return false;
     if (a.per_seg && (a.residual || a.c_img)) return false;
     if (!a.per_seg && !a.out && (!a.c_img || a.wbytes == 2)) return false;
