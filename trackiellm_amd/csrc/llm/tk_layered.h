@@ -96,7 +96,8 @@ protected:
 
 private:
     struct Seq { int len = 0, prev = -1, side = 0; std::vector<int32_t> pages; };
-    struct Pass { int nrows = 0, nseg = 0, nruns = 0, nchunks = 0, shortest = 1 << 30, ntiles = 0, nblocks = 0, nsums = 0; bool single = true, singles = true; }; /* all segments, or any, are single rows */
+    struct Pass { int nrows = 0, nseg = 0, nruns = 0, nchunks = 0, shortest = 1 << 30, ntiles = 0, nblocks = 0, nsums = 0; bool single = true, singles = true; /* all segments, or any, are single rows */
+                  int n_last = -1, last_tiles = 0; }; /* >= 0: the wanted rows, which alone go through the last layer behind its mixers; the attention tiles that hold one */
     TkLayeredModel* m_ = nullptr;
     std::mutex mu_; /* seqs_, free_pages_, host page table */
     std::vector<Seq> seqs_;
@@ -105,15 +106,15 @@ private:
     int n_pages_ = 0, max_pages_ = 0;
     std::vector<int32_t> live_; /* sequences of rows 0 .. of the last pass decode() may continue from */
     std::vector<void*> owned_;
-    int32_t *h_tab_ = nullptr, *d_tab_ = nullptr, *d_pages_ = nullptr, *d_out_rows_ = nullptr, *d_tiles_ = nullptr, *d_blocks_ = nullptr, *d_otok_ = nullptr;
+    int32_t *h_tab_ = nullptr, *d_tab_ = nullptr, *d_pages_ = nullptr, *d_out_rows_ = nullptr, *d_tiles_ = nullptr, *d_last_tiles_ = nullptr, *d_blocks_ = nullptr, *d_otok_ = nullptr;
     int ret_heads_ = 0; /* most heads of a retention layer (0: none) */
     int retention_rows(int nrows) const;
     size_t tab_ints_ = 0;
     TkPassTab tab_{};
-    float *x_ = nullptr, *proj_ = nullptr, *low_ = nullptr, *y_ = nullptr, *router_ = nullptr, *scratch_ = nullptr;
+    float *x_ = nullptr, *x_last_ = nullptr, *proj_ = nullptr, *low_ = nullptr, *y_ = nullptr, *router_ = nullptr, *scratch_ = nullptr;
     float *sums_ = nullptr, *chunks_ = nullptr;
     float *dq_ = nullptr, *dk_ = nullptr, *dv_ = nullptr, *dg_ = nullptr, *db_ = nullptr, *do_ = nullptr;
-    void *img_x_ = nullptr, *img_low_ = nullptr, *img_mix_ = nullptr, *img_ff_ = nullptr, *img_gather_ = nullptr, *img_head_ = nullptr, *q_ = nullptr;
+    void *img_x_ = nullptr, *img_low_ = nullptr, *img_mix_ = nullptr, *img_ff_ = nullptr, *img_gather_ = nullptr, *img_head_ = nullptr, *img_last_ = nullptr, *q_ = nullptr;
     TkMoeTab moe_{};
     struct Rope { float *c, *s; };
     std::map<std::pair<int, double>, Rope> rope_;
@@ -132,7 +133,8 @@ private:
     void gemm(const TkImgGemm& g, int* slabs = nullptr);
     size_t y_floats_ = 0;
     void enqueue_layers(const Pass& p);
-    void enqueue_head(int n, const int32_t* d_rows, int32_t* tok, int32_t* pos);
+    void enqueue_head(const float* x, int n, const int32_t* d_rows, int32_t* tok, int32_t* pos);
+    void choose_last_rows(Pass* p, int n_out);
     void enqueue_moe(const TkLayerSpec& s, const TkLayeredLayer& L, int nrows);
     bool run(int nrows, const int32_t* seq, const int32_t* pos, const int32_t* tok, float* logits_host, int32_t* argmax_host, bool head,
              const uint32_t* const* row_masks, const TkSampleRow* row_samp, int n_out, const int32_t* out_rows);

@@ -72,9 +72,9 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     const int64_t want = ((int64_t)mseq * mctx + 63) / 64 * 64;
     const int R = (int)std::max<int64_t>(TK_MAX_ROWS, std::min<int64_t>(PASS_ROWS, want));
     const int max_tiles = R / 64 + mseq;
-    /* tables behind the base's rows: segment of a row, segments, wanted rows, attention tiles, retention blocks */
+    /* tables behind the base's rows: segment of a row, segments, wanted rows, attention tiles (all, and the wanted rows'), retention blocks */
     int32_t* ext = nullptr;
-    const size_t block_ints = sizeof(TkRetentionBlock) / 4, extra = (size_t)R + 4 * (size_t)mseq + 2 * (size_t)(R / TK_DELTA_CHUNKED) + R + (2 + block_ints) * (size_t)max_tiles;
+    const size_t block_ints = sizeof(TkRetentionBlock) / 4, extra = (size_t)R + 4 * (size_t)mseq + 2 * (size_t)(R / TK_DELTA_CHUNKED) + R + (4 + block_ints) * (size_t)max_tiles;
     if (!init_tables(m->device, c.vocab, R, extra, &ext)) return false;
     tab_ints_ = 3 * (size_t)R + extra;
     d_tab_ = d_seq;
@@ -88,6 +88,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     tab_.chunked = p; p += 2 * (size_t)(R / TK_DELTA_CHUNKED);
     d_out_rows_ = p; p += R;
     d_tiles_ = p; p += 2 * (size_t)max_tiles;
+    d_last_tiles_ = p; p += 2 * (size_t)max_tiles;
     d_blocks_ = p;
     HIPQ(hipHostMalloc((void**)&h_tab_, tab_ints_ * 4, hipHostMallocDefault));
     memset(h_tab_, 0, tab_ints_ * 4);
@@ -98,7 +99,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     h_pages_.assign((size_t)mseq * max_pages_, 0);
     for (int i = n_pages_ - 1; i >= 0; --i) free_pages_.push_back(i);
 
-    size_t proj = 16, low = 16, mix = 0, lowk = 0, q = 0, dq = 0, dv = 0, dg = 0, dh = 0, ff = 0, scratch = 0, E = 0, gather = 0, moe_ff = 0, assign = 0, moe_rows = 0, sums = 0, chunks = 0;
+    size_t proj = 16, low = 16, mix = 0, mix_last = 0, lowk = 0, q = 0, dq = 0, dv = 0, dg = 0, dh = 0, ff = 0, scratch = 0, E = 0, gather = 0, moe_ff = 0, assign = 0, moe_rows = 0, sums = 0, chunks = 0;
     for (const TkLayerSpec& s : c.layers)
         for (const TkBranchSpec& b : s.branches)
             if (b.kind == TkBranchSpec::RETENTION) ret_heads_ = std::max(ret_heads_, b.retention.heads);
@@ -111,6 +112,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
         proj = std::max(proj, (size_t)proj_pitch(L.in.N));
         low = std::max(low, (size_t)L.low.N);
         mix = std::max(mix, tk_img_bytes(type, R, L.out.cols));
+        if (l + 1 == c.layers.size()) mix_last = tk_img_bytes(type, TK_MAX_ROWS, L.out.cols);
         if (L.low_cols) lowk = std::max(lowk, tk_img_bytes(type, R, L.low_cols));
         st_[l].resize(s.branches.size());
         for (size_t b = 0; b < s.branches.size(); ++b) {
@@ -165,7 +167,7 @@ bool TkLayeredSession::init(TkLayeredModel* m, int mseq, int mctx, int pool_toke
     }
     const size_t yrows = std::max<size_t>({(size_t)R, moe_rows, 8 * TK_MAX_ROWS}); /* a product of up to 256 rows may be split over k into eight slabs */
     y_floats_ = yrows * c.width;
-    if (!alloc((void**)&x_, (size_t)R * c.width * 4) || !alloc((void**)&proj_, (size_t)R * proj * 4, true) || !alloc((void**)&low_, (size_t)R * low * 4, true) ||
+    if (!alloc((void**)&x_, (size_t)R * c.width * 4) || !alloc((void**)&x_last_, (size_t)TK_MAX_ROWS * c.width * 4) || !alloc(&img_last_, mix_last, true) || !alloc((void**)&proj_, (size_t)R * proj * 4, true) || !alloc((void**)&low_, (size_t)R * low * 4, true) ||
         !alloc((void**)&y_, yrows * c.width * 4, true) || !alloc(&img_x_, tk_img_bytes(type, R, c.width), true) || !alloc(&img_low_, lowk, true) ||
         !alloc(&img_mix_, mix, true) || !alloc(&img_ff_, std::max(ff, moe_ff), true) || !alloc(&img_head_, tk_img_bytes(type, TK_MAX_ROWS, c.width), true) ||
         !alloc(&q_, (size_t)R * q * esz, true) || !alloc((void**)&dq_, (size_t)R * dq * 4) || !alloc((void**)&dk_, (size_t)R * dq * 4) || !alloc((void**)&dv_, (size_t)R * dv * 4) ||
@@ -336,14 +338,33 @@ void TkLayeredSession::enqueue_moe(const TkLayerSpec& s, const TkLayeredLayer& L
     gemm(d);
 }
 
+/* Nobody reads what the last layer makes of a row whose logits are not wanted, so behind its mixers (which leave keys, values and states) only the wanted rows go on, side by
+ * side.  Not where they are most of the pass: a launch that takes them out is 4 us. */
+void TkLayeredSession::choose_last_rows(Pass* p, int n_out) {
+    if (streams_ || p->single || n_out > TK_MAX_ROWS || 2 * n_out > p->nrows) return;
+    p->n_last = n_out;
+    const int32_t *out = h_tab_ + (d_out_rows_ - d_tab_), *tiles = h_tab_ + (d_tiles_ - d_tab_);
+    int32_t* last = h_tab_ + (d_last_tiles_ - d_tab_);
+    for (int t = 0, i = 0; t < p->ntiles && i < n_out; ++t) { /* both ascend */
+        const int32_t r0 = tiles[2 * t], nr = tiles[2 * t + 1];
+        if (out[i] >= r0 + nr) continue;
+        last[2 * p->last_tiles] = r0; last[2 * p->last_tiles + 1] = nr;
+        ++p->last_tiles;
+        while (i < n_out && out[i] < r0 + nr) ++i;
+    }
+}
+
 void TkLayeredSession::enqueue_layers(const Pass& p) {
     const TkLayeredConfig& c = m_->cfg;
-    const int type = m_->type, D = c.width, kt = tk_img_kt(type), xkt = tk_img_pad_k(type, D) / kt, n = p.nrows;
+    const int type = m_->type, D = c.width, kt = tk_img_kt(type), xkt = tk_img_pad_k(type, D) / kt;
+    int n = p.nrows;
+    float* x = x_;
     hipStream_t s = stream;
     tk_launch_layer_embed(type, m_->embed, D, c.embed_scale, d_tok, n, x_, m_->layers[0].pre1, c.eps, img_x_, xkt, s);
     for (size_t l = 0; l < c.layers.size(); ++l) {
         const TkLayerSpec& spec = c.layers[l];
         const TkLayeredLayer& L = m_->layers[l];
+        const bool part = p.n_last >= 0 && l + 1 == c.layers.size();
         const TkNorm after = l + 1 < c.layers.size() ? m_->layers[l + 1].pre1 : TkNorm{}; /* on the next layer's input: fused into this layer's last kernel */
         const int pitch = proj_pitch(L.in.N);
         TkImgGemm g{};
@@ -397,7 +418,7 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             const TkDeltaArgs* d = di < ds.size() ? &ds[di] : nullptr;
             tk_launch_mixer_prep(type, proj_, pitch, a, d, tab_, n, s);
             if (!p.single) {
-                if (a) tk_launch_attn_tiles(type, *a, tab_, d_tiles_, p.ntiles, s);
+                if (a && (!part || p.last_tiles)) tk_launch_attn_tiles(type, *a, tab_, part ? d_last_tiles_ : d_tiles_, part ? p.last_tiles : p.ntiles, s);
                 if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, p.shortest, p.nruns, p.nchunks, n, s);
                 continue;
             }
@@ -406,15 +427,21 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             if (a) tk_launch_attn_rows(type, *a, tab_, n, splits, scratch_, s);
             if (d) tk_launch_delta_step(type, *d, tab_, n, s);
         }
+        if (part) {
+            if (p.n_last == 0) return;
+            tk_launch_take_rows(d_out_rows_, p.n_last, x_, x_last_, D, img_mix_, img_last_, L.out.K / kt, s);
+            n = p.n_last;
+            x = x_last_;
+        }
         TkImgGemm o{};
-        o.type = type; o.w = L.out.img; o.a = img_mix_; o.K = L.out.K; o.N = L.out.N; o.nrows = n; o.out = y_; o.ldc = D; o.n_valid = D;
+        o.type = type; o.w = L.out.img; o.a = part ? img_last_ : img_mix_; o.K = L.out.K; o.N = L.out.N; o.nrows = n; o.out = y_; o.ldc = D; o.n_valid = D;
         /* products whose result goes to a norm may come in slabs, as many as y_ holds */
         const size_t slab = (size_t)n * D;
         const int most = slab % 4 == 0 ? (int)std::min<size_t>(8, y_floats_ / slab) : 1;
         int slabs = 1;
         o.max_slabs = most; o.slab_floats = slab;
         gemm(o, &slabs);
-        tk_launch_post_norm(type, TkSubOut{y_, D, slabs, slab, L.out_bias, 1.0f, nullptr, nullptr, 0}, L.norm1, spec.mlp.kind == TkMlpSpec::NONE ? after : L.pre2, c.eps, D, n, x_, img_x_, xkt, s);
+        tk_launch_post_norm(type, TkSubOut{y_, D, slabs, slab, L.out_bias, 1.0f, nullptr, nullptr, 0}, L.norm1, spec.mlp.kind == TkMlpSpec::NONE ? after : L.pre2, c.eps, D, n, x, img_x_, xkt, s);
         if (spec.mlp.kind == TkMlpSpec::DENSE) {
             TkImgGemm u{};
             u.type = type; u.w = L.gate_up.img; u.a = img_x_; u.K = L.gate_up.K; u.N = L.gate_up.N; u.nrows = n;
@@ -425,19 +452,19 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             w.type = type; w.w = L.down.img; w.a = img_ff_; w.K = L.down.K; w.N = L.down.N; w.nrows = n; w.out = y_; w.ldc = D; w.n_valid = D;
             w.max_slabs = most; w.slab_floats = slab;
             gemm(w, &slabs);
-            tk_launch_post_norm(type, TkSubOut{y_, D, slabs, slab, nullptr, 0.0f, nullptr, nullptr, 0}, L.norm2, after, c.eps, D, n, x_, img_x_, xkt, s);
+            tk_launch_post_norm(type, TkSubOut{y_, D, slabs, slab, nullptr, 0.0f, nullptr, nullptr, 0}, L.norm2, after, c.eps, D, n, x, img_x_, xkt, s);
         } else if (spec.mlp.kind == TkMlpSpec::MOE) {
             enqueue_moe(spec, L, n);
-            tk_launch_post_norm(type, TkSubOut{y_, D, 1, 0, nullptr, 0.0f, moe_.slot, moe_.weight, spec.mlp.top}, L.norm2, after, c.eps, D, n, x_, img_x_, xkt, s);
+            tk_launch_post_norm(type, TkSubOut{y_, D, 1, 0, nullptr, 0.0f, moe_.slot, moe_.weight, spec.mlp.top}, L.norm2, after, c.eps, D, n, x, img_x_, xkt, s);
         }
         if (streams_) (void)hipMemcpyAsync(streams_ + l * (size_t)n * D, x_, (size_t)n * D * 4, hipMemcpyDeviceToHost, s);
     }
 }
 
-void TkLayeredSession::enqueue_head(int n, const int32_t* d_rows, int32_t* tok, int32_t* pos) {
+void TkLayeredSession::enqueue_head(const float* x, int n, const int32_t* d_rows, int32_t* tok, int32_t* pos) {
     const TkLayeredConfig& c = m_->cfg;
     const int type = m_->type;
-    tk_launch_rows_norm(type, x_, d_rows, n, m_->final_norm, c.eps, c.width, img_head_, m_->head.K / tk_img_kt(type), stream);
+    tk_launch_rows_norm(type, x, d_rows, n, m_->final_norm, c.eps, c.width, img_head_, m_->head.K / tk_img_kt(type), stream);
     TkImgGemm g{};
     g.type = type; g.w = m_->head.img; g.a = img_head_; g.K = m_->head.K; g.N = m_->head.N; g.nrows = n; g.out = logits; g.ldc = c.vocab; g.n_valid = c.vocab;
     gemm(g);
@@ -451,7 +478,7 @@ void TkLayeredSession::enqueue_decode(int nrows) {
     Pass p;
     p.nrows = p.nseg = nrows;
     enqueue_layers(p);
-    enqueue_head(nrows, nullptr, d_tok, d_pos);
+    enqueue_head(x_, nrows, nullptr, d_tok, d_pos);
     tk_launch_swap_state(tab_, nrows, stream);
 }
 
@@ -473,6 +500,7 @@ bool TkLayeredSession::run(int nrows, const int32_t* seq, const int32_t* pos, co
     }
     if (!out_rows)
         for (int i = 0; i < n_out; ++i) h_tab_[(size_t)(d_out_rows_ - d_tab_) + i] = i;
+    choose_last_rows(&p, head ? n_out : 0);
     HIPQ(hipMemcpyAsync(d_tab_, h_tab_, tab_ints_ * 4, hipMemcpyHostToDevice, stream));
     HIPQ(hipMemsetAsync(d_nsteps, 0, TK_MAX_ROWS * 4, stream));
     launch_error.clear();
@@ -491,7 +519,7 @@ bool TkLayeredSession::run(int nrows, const int32_t* seq, const int32_t* pos, co
         for (int o = 0; head && o < n_out; o += TK_MAX_ROWS) {
             const int k = std::min(TK_MAX_ROWS, n_out - o);
             if (!stage_sampling(k, h_tab_ + (d_out_rows_ - d_tab_) + o, row_masks, row_samp)) return false;
-            enqueue_head(k, d_out_rows_ + o, d_otok_, nullptr);
+            enqueue_head(p.n_last >= 0 ? x_last_ : x_, k, p.n_last >= 0 ? nullptr : d_out_rows_ + o, d_otok_, nullptr);
             if (logits_host) HIPQ(hipMemcpyAsync(logits_host + (size_t)o * vocab_, logits, (size_t)k * vocab_ * 4, hipMemcpyDeviceToHost, stream));
             if (argmax_host) HIPQ(hipMemcpyAsync(argmax_host + o, d_otok_, k * 4, hipMemcpyDeviceToHost, stream));
         }

@@ -130,6 +130,8 @@ struct TkSubOut {
 };
 /* x += norm(output); the image of next(x), the next sublayer's input */
 void tk_launch_post_norm(int type, const TkSubOut& o, const TkNorm& norm, const TkNorm& next, float eps, int width, int nrows, float* x, void* img, int ktiles, hipStream_t s);
+/* the listed rows of the residual stream and of an image, side by side */
+void tk_launch_take_rows(const int32_t* rows, int n, const float* x, float* x_out, int width, const void* img, void* img_out, int ktiles, hipStream_t s);
 /* norm of the listed rows (null: rows 0 .. n - 1) as an image */
 void tk_launch_rows_norm(int type, const float* x, const int32_t* rows, int n, const TkNorm& norm, float eps, int width, void* img, int ktiles, hipStream_t s);
 

@@ -1814,6 +1814,21 @@ __global__ __launch_bounds__(256) void k_moe_gather(const tk_v4u* img, tk_v4u* o
     out[((size_t)(slot >> 4) * ktiles + p / 4) * 64 + (slot & 15) + 16 * (p % 4)] = img[((size_t)(row >> 4) * ktiles + p / 4) * 64 + (row & 15) + 16 * (p % 4)];
 }
 
+/* rows[i] of the residual stream and of an operand image to row i of others: 16-byte pieces, first the stream's, then the image's */
+__global__ __launch_bounds__(256) void k_take_rows(const int32_t* rows, const float* x, float* x_out, int width, const tk_v4u* img, tk_v4u* img_out, int ktiles) {
+    const int i = blockIdx.y, row = rows[i], nx = (width + 3) / 4;
+    int p = blockIdx.x * 256 + threadIdx.x;
+    if (p < nx) {
+        const float* from = x + (size_t)row * width;
+        float* to = x_out + (size_t)i * width;
+        for (int c = 4 * p; c < width && c < 4 * p + 4; ++c) to[c] = from[c];
+        return;
+    }
+    p -= nx; /* piece: k tile p / 4, lane group p % 4 */
+    if (p >= ktiles * 4) return;
+    img_out[((size_t)(i >> 4) * ktiles + p / 4) * 64 + (i & 15) + 16 * (p % 4)] = img[((size_t)(row >> 4) * ktiles + p / 4) * 64 + (row & 15) + 16 * (p % 4)];
+}
+
 } // namespace
 
 /* ------------------------------------------------------------------ launchers -------------- */
@@ -2012,6 +2027,9 @@ void tk_launch_moe_select(const float* logits, int ld, int experts, int top, int
 }
 void tk_launch_moe_gather(const void* img, void* gathered, int ktiles, int top, int nrows, const TkMoeTab& t, hipStream_t s) {
     hipLaunchKernelGGL(k_moe_gather, dim3(nrows * top, (ktiles * 4 + 255) / 256), dim3(256), 0, s, (const tk_v4u*)img, (tk_v4u*)gathered, ktiles, top, t);
+}
+void tk_launch_take_rows(const int32_t* rows, int n, const float* x, float* x_out, int width, const void* img, void* img_out, int ktiles, hipStream_t s) {
+    hipLaunchKernelGGL(k_take_rows, dim3(((width + 3) / 4 + ktiles * 4 + 255) / 256, n), dim3(256), 0, s, rows, x, x_out, width, (const tk_v4u*)img, (tk_v4u*)img_out, ktiles);
 }
 void tk_launch_swap_state(const TkPassTab& t, int n, hipStream_t s) { hipLaunchKernelGGL(k_swap_state, dim3((n + 255) / 256), dim3(256), 0, s, t, n); }
 
