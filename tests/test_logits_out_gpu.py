@@ -1,0 +1,43 @@
+"""Logits on their way to the caller: up to 1 MiB in one copy, more in pieces of 256 KiB through pinned memory of 32, which longer ones pass several times.  The same rows eight at a
+time, bit for bit; several sessions at once, each from a thread of its own."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+VOCAB = 32000
+
+
+@pytest.fixture(scope="module")
+def model(gpu):
+    return gpu.LlmModel(gpu.LlmHParams(1, 256, 8, 2, 64, 512, VOCAB, 1e-5, 10000.0, 0, 0, 0, 0, 1)).fill_synthetic(4)
+
+
+def passes(gpu, model, rows, width, seed, session=None):
+    s = session or gpu.LlmSession(model, 256, 8)
+    toks = np.random.default_rng(seed).integers(3, VOCAB, rows).astype(np.int32)
+    out = [s.forward(np.arange(r, min(r + width, rows)), np.zeros(min(width, rows - r)), toks[r:r + width]) for r in range(0, rows, width)]
+    return np.concatenate([o[0] for o in out]), np.concatenate([o[1] for o in out])
+
+
+@pytest.mark.parametrize("rows", [1, 8, 9, 33, 65, 66, 131, 256])
+def test_logits_of_many_rows(gpu, model, rows):
+    got, ids = passes(gpu, model, rows, 256, rows)
+    want, want_ids = passes(gpu, model, rows, 8, rows)
+    assert np.array_equal(got.view(np.uint32), want.view(np.uint32)) and np.array_equal(ids, want_ids)
+
+
+def test_sessions_in_threads(gpu, model):
+    rows = [70, 130, 33]
+    got = [None] * len(rows)
+    sessions = [gpu.LlmSession(model, 256, 8) for _ in rows]
+
+    def work(i):
+        got[i] = [passes(gpu, model, rows[i], 256, 7 + k, sessions[i])[0] for k in range(3)]
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(rows))]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    for i, n in enumerate(rows):
+        for k in range(3):
+            assert np.array_equal(got[i][k].view(np.uint32), passes(gpu, model, n, 8, 7 + k)[0].view(np.uint32))

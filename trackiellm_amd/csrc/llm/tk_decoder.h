@@ -18,6 +18,12 @@
 #include "../common/tk_sample.h"
 #include "tk_llm_layout.h"
 
+/* logits on their way to the caller (TkDecodeSession::copy_out) */
+#define TK_OUT_PIECE ((size_t)256 << 10)
+#define TK_OUT_GROUPS 8  /* workgroups of a piece */
+#define TK_OUT_PIECES 32 /* pieces the pinned memory holds */
+#define TK_OUT_DIRECT ((size_t)1 << 20)
+
 class TkDecodeSession;
 
 class TkDecoderModel {
@@ -84,6 +90,8 @@ protected:
     /* records what `enqueue` launches into *slot (kept when it is there already) */
     bool capture(hipGraphExec_t* slot, const std::function<void()>& enqueue);
     static bool graphs_enabled();
+    /* dev -> host behind what the stream holds.  Up to TK_OUT_DIRECT bytes the copy is enqueued as it is; more is in `host` when this returns */
+    bool copy_out(void* host, const void* dev, size_t bytes);
     bool rows_in_range(int nrows, const int32_t* seq, const int32_t* pos, const int32_t* tok);
 
     /* hooks of decode(): before the loop (host positions of the rows), then per step, `top` = the step's highest position: the graph slot the step
@@ -95,6 +103,9 @@ protected:
 
 private:
     int32_t* d_block_ = nullptr;
+    uint8_t* out_ring_ = nullptr; /* pinned: TK_OUT_PIECES pieces, and of each the number of the batch that arrived last */
+    unsigned* d_out_done_ = nullptr;
+    unsigned out_epoch_ = 1;
 };
 
 /* capture is one at a time per process: other host threads keep calling allocation and copy APIs meanwhile (relaxed mode) */

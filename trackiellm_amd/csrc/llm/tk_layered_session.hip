@@ -512,7 +512,7 @@ bool TkLayeredSession::run(int nrows, const int32_t* seq, const int32_t* pos, co
         } else {
             enqueue_decode(nrows);
         }
-        if (logits_host) HIPQ(hipMemcpyAsync(logits_host, logits, (size_t)nrows * vocab_ * 4, hipMemcpyDeviceToHost, stream));
+        if (logits_host && !copy_out(logits_host, logits, (size_t)nrows * vocab_ * 4)) return false;
         if (argmax_host) HIPQ(hipMemcpyAsync(argmax_host, d_tok, nrows * 4, hipMemcpyDeviceToHost, stream));
     } else {
         enqueue_layers(p);
@@ -520,7 +520,7 @@ bool TkLayeredSession::run(int nrows, const int32_t* seq, const int32_t* pos, co
             const int k = std::min(TK_MAX_ROWS, n_out - o);
             if (!stage_sampling(k, h_tab_ + (d_out_rows_ - d_tab_) + o, row_masks, row_samp)) return false;
             enqueue_head(p.n_last >= 0 ? x_last_ : x_, k, p.n_last >= 0 ? nullptr : d_out_rows_ + o, d_otok_, nullptr);
-            if (logits_host) HIPQ(hipMemcpyAsync(logits_host + (size_t)o * vocab_, logits, (size_t)k * vocab_ * 4, hipMemcpyDeviceToHost, stream));
+            if (logits_host && launch_error.empty() && !copy_out(logits_host + (size_t)o * vocab_, logits, (size_t)k * vocab_ * 4)) return false;
             if (argmax_host) HIPQ(hipMemcpyAsync(argmax_host + o, d_otok_, k * 4, hipMemcpyDeviceToHost, stream));
         }
     }

@@ -577,7 +577,7 @@ bool TkLlmSession::forward(int nrows, const int32_t* seq, const int32_t* pos, co
         for (int i = 0; i < n_out && argmax_host; ++i) argmax_host[i] = ids[out_rows[i]];
         return true;
     }
-    if (logits_host) HIPQ(hipMemcpyAsync(logits_host, logits, (size_t)nrows * model->hp.vocab * 4, hipMemcpyDeviceToHost, stream));
+    if (logits_host && !copy_out(logits_host, logits, (size_t)nrows * vocab_ * 4)) return false;
     if (argmax_host) HIPQ(hipMemcpyAsync(argmax_host, d_tok, nrows * 4, hipMemcpyDeviceToHost, stream));
     HIPQ(hipStreamSynchronize(stream));
     return true;
