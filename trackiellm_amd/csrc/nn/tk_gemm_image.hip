@@ -29,15 +29,18 @@ __device__ __forceinline__ void store_f32(const TkImgGemm& a, int64_t row, int n
 }
 
 /* 1 / (1 + e^-z): what becomes bf16 next by the hardware's exponential and reciprocal (1 ulp of float32 each), five instructions where expf and a division take some forty, which
- * stood between a block's last product and the next block's first: 1785 x 16384 x 2048 (gate | up) 123 -> 114 us.  Errors against 64 bits of whole models: unchanged */
+ * stood between a block's last product and the next block's first: 1785 x 16384 x 2048 (gate | up) 122 -> 114 us (and 111 with store_act's addresses, below).  Errors against 64 bits of whole models: unchanged */
 template <typename T> __device__ __forceinline__ float act_sigmoid(float z) {
     return sizeof(T) == 4 ? tk_sigmoid32(z) : __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
 }
 template <typename T> __device__ __forceinline__ float act_silu(float z) { return sizeof(T) == 4 ? tk_silu32(z) : z * act_sigmoid<T>(z); }
 
-/* gate and up tiles of the same 16 columns -> the gated activation in the next product's operand image */
+/* gate and up tiles of the same 16 columns -> the gated activation in the next product's operand image: M-tile mt, columns 16 ct .. 16 ct + 15, both the same for all lanes, so that
+ * the address is a scalar one and a lane's constant offset (row and column of a lane through tk_img_index are two 64-bit products each) */
 template <typename T>
-__device__ __forceinline__ void store_act(const TkImgGemm& a, int64_t row, int n, tk_v4f gate, tk_v4f up) {
+__device__ __forceinline__ void store_act(const TkImgGemm& a, int mt, int ct, int lane, tk_v4f gate, tk_v4f up) {
+    constexpr int PER = TkImg<T>::KT / 16, EP = TkImg<T>::EP; /* tiles of 16 columns in a k tile */
+    const int n = ct * 16 + 4 * (lane >> 4);
     tk_v4f h;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -50,7 +53,8 @@ __device__ __forceinline__ void store_act(const TkImgGemm& a, int64_t row, int n
         }
         h[r] = n + r < a.act_valid ? y : 0.0f;
     }
-    if (n < a.act_valid) tk_img_put4((T*)a.act_img, row, n, a.act_ktiles, h);
+    T* const tile = (T*)a.act_img + ((size_t)mt * a.act_ktiles + ct / PER) * (1024 / sizeof(T)) + ct % PER * 256;
+    if (n < a.act_valid) tk_img_put4_at(tile + ((lane & 15) + 16 * ((lane >> 4) * 4 / EP)) * EP + (lane >> 4) * 4 % EP, h);
 }
 
 /* ---- skinny: MT M-tiles of rows, NT column tiles per workgroup, K interleaved over the waves in pieces of U tiles ----
@@ -152,7 +156,7 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
         const int64_t row = (int64_t)(m0 + m) * 16 + (lane & 15);
         if (m >= mlive || (!GROUPED && row >= a.nrows)) continue;
         if (SWIGLU) {
-            if (n0 + 2 * n < ntot) store_act<T>(a, row, (n0 / 2 + n) * 16 + 4 * (lane >> 4), total(2 * n, m), total(2 * n + 1, m));
+            if (n0 + 2 * n < ntot) store_act<T>(a, m0 + m, n0 / 2 + n, lane, total(2 * n, m), total(2 * n + 1, m));
         } else if (n0 + n < ntot) {
             store_f32<T>(a, row, (n0 + n) * 16 + 4 * (lane >> 4), total(n, m));
         }
@@ -287,7 +291,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_wide(TkImgGemm a, int nbl
         if (SWIGLU) {
 #pragma unroll
             for (int n = 0; n < NW / 2; ++n)
-                if (n0 + wn + 2 * n < ntot) store_act<T>(a, row, ((n0 + wn) / 2 + n) * 16 + 4 * (lane >> 4), acc[2 * n][m], acc[2 * n + 1 < NW ? 2 * n + 1 : 0][m]);
+                if (n0 + wn + 2 * n < ntot) store_act<T>(a, m0 + wm + m, (n0 + wn) / 2 + n, lane, acc[2 * n][m], acc[2 * n + 1 < NW ? 2 * n + 1 : 0][m]);
         } else {
 #pragma unroll
             for (int n = 0; n < NW; ++n)

@@ -49,13 +49,15 @@ template <typename T>
 __device__ __forceinline__ void tk_img_put(T* img, int64_t row, int k, int ktiles, float v) { img[tk_img_index<T>(row, k, ktiles)] = TkImg<T>::from(v); }
 
 /* four consecutive k, k % 4 == 0 */
-__device__ __forceinline__ void tk_img_put4(float* img, int64_t row, int k, int ktiles, tk_v4f v) { *(tk_v4f*)(img + tk_img_index<float>(row, k, ktiles)) = v; }
-__device__ __forceinline__ void tk_img_put4(TkBf16* img, int64_t row, int k, int ktiles, tk_v4f v) {
+__device__ __forceinline__ void tk_img_put4_at(float* at, tk_v4f v) { *(tk_v4f*)at = v; }
+__device__ __forceinline__ void tk_img_put4_at(TkBf16* at, tk_v4f v) {
     tk_v2u p;
     p[0] = (uint32_t)tk_bf16_bits(v[0]) | (uint32_t)tk_bf16_bits(v[1]) << 16;
     p[1] = (uint32_t)tk_bf16_bits(v[2]) | (uint32_t)tk_bf16_bits(v[3]) << 16;
-    *(tk_v2u*)(img + tk_img_index<TkBf16>(row, k, ktiles)) = p;
+    *(tk_v2u*)at = p;
 }
+template <typename T>
+__device__ __forceinline__ void tk_img_put4(T* img, int64_t row, int k, int ktiles, tk_v4f v) { tk_img_put4_at(img + tk_img_index<T>(row, k, ktiles), v); }
 
 /* eight consecutive k, k % 8 == 0 */
 __device__ __forceinline__ void tk_img_put8(float* img, int64_t row, int k, int ktiles, tk_v4f a, tk_v4f b) { tk_img_put4(img, row, k, ktiles, a); tk_img_put4(img, row, k + 4, ktiles, b); }
