@@ -418,8 +418,10 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             const TkDeltaArgs* d = di < ds.size() ? &ds[di] : nullptr;
             tk_launch_mixer_prep(type, proj_, pitch, a, d, tab_, n, s);
             if (!p.single) {
-                if (a && (!part || p.last_tiles)) tk_launch_attn_tiles(type, *a, tab_, part ? d_last_tiles_ : d_tiles_, part ? p.last_tiles : p.ntiles, s);
-                if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, p.shortest, p.nruns, p.nchunks, n, s);
+                const int32_t* tiles = part ? d_last_tiles_ : d_tiles_;
+                const int ntiles = part ? p.last_tiles : p.ntiles;
+                if (d) tk_launch_delta_scan(type, *d, tab_, p.nseg, p.shortest, p.nruns, p.nchunks, n, s, a, tiles, ntiles);
+                else if (a && ntiles) tk_launch_attn_tiles(type, *a, tab_, tiles, ntiles, s);
                 continue;
             }
             const int splits = a ? tk_attn_rows_splits(*a, visible[ai], n) : 1;

@@ -105,7 +105,8 @@ size_t tk_attn_rows_scratch_floats(const TkAttnArgs& a, int nrows, int splits);
 #define TK_DELTA_CHUNKED 40
 #define TK_DELTA_LONG 72
 #define TK_DELTA_MANY 224
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_runs /* <= 256 */, int n_chunks, int nrows, hipStream_t s);
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_runs /* <= 256 */, int n_chunks, int nrows, hipStream_t s,
+                          const TkAttnArgs* beside = nullptr, const int32_t* tiles = nullptr, int n_tiles = 0 /* tk_launch_attn_tiles' work, done on the way */);
 /* scratch of a pass of at most `rows` rows: its chunks, and one that is partly filled per segment (16 heads of 128, 2048 rows: 78 MB) */
 size_t tk_delta_chunk_floats(int heads, int dim, int rows);
 /* the same for passes whose segments are single rows: one launch */

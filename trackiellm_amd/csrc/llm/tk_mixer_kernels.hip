@@ -3,6 +3,7 @@
 
 #include <math.h>
 
+#include <algorithm>
 #include <atomic>
 #include <mutex>
 
@@ -616,12 +617,11 @@ __device__ __forceinline__ void attn_store(const TkAttnArgs& a, const tk_v4f (&o
 template <typename T, int B> constexpr bool attn_two_buffers() { return sizeof(T) == 2 || B < 256; }
 
 template <typename T, int B, bool FULL /* head sizes fill the bucket */>
-__global__ __launch_bounds__(256, B * sizeof(T) >= 512 ? 1 : 2) void k_attn_tiles(TkAttnArgs a, TkPassTab t, const int32_t* tiles) {
+__device__ __forceinline__ void attn_tile(const TkAttnArgs& a, const TkPassTab& t, const int32_t* tiles, int tile, int h, uint8_t* lds) {
     constexpr int DT = B / TkImg<T>::KT, VT = B / 16, SZ = sizeof(T);
     typedef typename VFrag<T>::type VF;
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4;
-    const int row0 = tiles[2 * blockIdx.x], n = tiles[2 * blockIdx.x + 1], h = blockIdx.y, kvh = h / (a.heads / a.kv_heads);
+    const int row0 = tiles[2 * tile], n = tiles[2 * tile + 1], kvh = h / (a.heads / a.kv_heads);
     const int nd = FULL ? DT : a.kv.dim_pad / TkImg<T>::KT, nv = FULL ? VT : a.kv.vdim_pad / 16;
     const int krow = a.kv.dim_pad * SZ + 16, vrow = TK_PAGE * SZ + 16; /* LDS pitches: rows start in different banks */
     const int buf = TK_PAGE * krow + a.kv.vdim_pad * vrow;
@@ -700,6 +700,11 @@ __global__ __launch_bounds__(256, B * sizeof(T) >= 512 ? 1 : 2) void k_attn_tile
         if (!TWO) __syncthreads(); /* the only buffer is free again */
     }
     if (q < n) attn_store<T, VT>(a, f.o, row0 + q, h, g, a.out_scale / f.l);
+}
+template <typename T, int B, bool FULL>
+__global__ __launch_bounds__(256, B * sizeof(T) >= 512 ? 1 : 2) void k_attn_tiles(TkAttnArgs a, TkPassTab t, const int32_t* tiles) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    attn_tile<T, B, FULL>(a, t, tiles, blockIdx.x, blockIdx.y, lds);
 }
 
 /* a chain's result to and from the LDS: so [n][VT][64], sm and sl [n][64] behind it */
@@ -1027,12 +1032,14 @@ __global__ __launch_bounds__(256) void k_delta_chunk(TkDeltaArgs d, TkPassTab t,
  * The zeros of T and B must not meet an infinity or NaN, which would reach the tokens before its own.  A test per chunk cost 18 us on top of the 108, so a
  * second launch (AGAIN, 5 us) looks at the states that the first has left, where what is not finite stays (0 x infinity is NaN): it walks columns that
  * have any once more, without those zeros, and leaves at once otherwise. */
+struct DeltaChainLds { tk_v4f pu[2][4][64], po[2][4][64]; };
 template <int DP, bool AGAIN>
-__global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t) {
+__device__ __forceinline__ void delta_chain(const TkDeltaArgs& d, const TkPassTab& t, int h, int block, int run, DeltaChainLds& m) {
     constexpr int NT = DP / 64, AHEAD = 3;
-    __shared__ tk_v4f pu[2][4][64], po[2][4][64];
+    tk_v4f (&pu)[2][4][64] = m.pu;
+    tk_v4f (&po)[2][4][64] = m.po;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4;
-    const int h = blockIdx.x, seg = t.chunked[2 * blockIdx.z], vp = (d.vdim + 3) & ~3, col = blockIdx.y * 16 + (lane & 15);
+    const int seg = t.chunked[2 * run], vp = (d.vdim + 3) & ~3, col = block * 16 + (lane & 15);
     const int row0 = t.seg_row0[seg], n = t.seg_n[seg], in = t.seg_in[seg], out = t.seg_out[seg];
     const bool live = col < d.vdim;
     const int nc = (n + DC - 1) / DC;
@@ -1047,7 +1054,7 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
         }
     struct Ops { tk_v4f w[NT], q[NT], k[NT], g[NT]; float t, b, v; } ops[AHEAD + 1];
     const size_t step = (size_t)d.heads * delta_chunk_floats(DP);
-    const float* const base = d.chunks + ((size_t)t.chunked[2 * blockIdx.z + 1] * d.heads + h) * delta_chunk_floats(DP);
+    const float* const base = d.chunks + ((size_t)t.chunked[2 * run + 1] * d.heads + h) * delta_chunk_floats(DP);
     auto fetch = [&](Ops& o, int c) {
         const float* p = base + (size_t)c * step;
         const int tile = wave * NT;
@@ -1065,7 +1072,7 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
         /* past the run's end, and in columns that do not exist, any number will do: their T is zero, their results are not stored */
         o.v = d.v[((size_t)(row0 + (tt < n ? tt : c * DC)) * d.heads + h) * d.vdim + (live ? col : 0)];
     };
-    const int ot = tid >> 4, oc = blockIdx.y * 16 + (tid & 15); /* the output element this thread finishes */
+    const int ot = tid >> 4, oc = block * 16 + (tid & 15); /* the output element this thread finishes */
     auto finish = [&](int c) {
         const int l = (ot >> 2) * 16 + (tid & 15), b = c & 1;
         const float o = ((po[b][0][l][ot & 3] + po[b][1][l][ot & 3]) + po[b][2][l][ot & 3]) + po[b][3][l][ot & 3];
@@ -1134,6 +1141,25 @@ __global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t)
                 const int e = (wave * NT + i) * 16 + 4 * g + r;
                 if (e < d.dim) d.state[(((size_t)out * d.heads + h) * d.dim + e) * vp + col] = S[i][r];
             }
+}
+template <int DP, bool AGAIN>
+__global__ __launch_bounds__(256) void k_delta_chain(TkDeltaArgs d, TkPassTab t) {
+    __shared__ DeltaChainLds m;
+    delta_chain<DP, AGAIN>(d, t, blockIdx.x, blockIdx.y, blockIdx.z, m);
+}
+
+/* The chain, which is latency on a few CUs, and the tiles of the attention branch beside it in one launch: the chain's workgroups come first and so have CUs of their own as long as
+ * there are any, and its waves go first where a tile's share their SIMDs.  2047 tokens, 16 heads of 128 each: 110 + 60 us one behind the other, 124 side by side. */
+template <typename T, int B, int DP>
+__global__ __launch_bounds__(256, 2) void k_chain_and_tiles(TkDeltaArgs d, TkAttnArgs a, TkPassTab t, const int32_t* tiles, int n_tiles, int blocks /* of a head's columns */, int chains) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int id = blockIdx.x;
+    if (id < chains) {
+        __builtin_amdgcn_s_setprio(3);
+        delta_chain<DP, false>(d, t, id % d.heads, id / d.heads % blocks, id / d.heads / blocks, *(DeltaChainLds*)lds);
+    } else {
+        attn_tile<T, B, true>(a, t, tiles, (id - chains) % n_tiles, (id - chains) / n_tiles, lds);
+    }
 }
 
 /* o over its root mean square, times the norm's weight, times the gate: one wave per (row, head) */
@@ -1866,10 +1892,14 @@ static int attn_bucket(const TkAttnArgs& a) {
 
 static bool attn_full(const TkAttnArgs& a) { return a.kv.dim_pad == attn_bucket(a) && a.kv.vdim_pad == attn_bucket(a); }
 
+static size_t attn_tiles_lds(int type, const TkAttnArgs& a) {
+    const size_t sz = type == TK_IMG_F32 ? 4 : 2;
+    return (TK_PAGE * (a.kv.dim_pad * sz + 16) + a.kv.vdim_pad * (TK_PAGE * sz + 16)) * (type == TK_IMG_F32 && attn_bucket(a) == 256 ? 1 : 2);
+}
 void tk_launch_attn_tiles(int type, const TkAttnArgs& a, const TkPassTab& t, const int32_t* tiles, int n_tiles, hipStream_t s) {
     const int b = attn_bucket(a);
     const dim3 grid(n_tiles, a.heads);
-    const size_t sz = type == TK_IMG_F32 ? 4 : 2, lds = (TK_PAGE * (a.kv.dim_pad * sz + 16) + a.kv.vdim_pad * (TK_PAGE * sz + 16)) * (type == TK_IMG_F32 && b == 256 ? 1 : 2);
+    const size_t lds = attn_tiles_lds(type, a);
 #define TK_TILES(T, B, F) hipLaunchKernelGGL((k_attn_tiles<T, B, F>), grid, dim3(256), lds, s, a, t, tiles)
 #define TK_TILES_B(T, F) do { if (b == 64) TK_TILES(T, 64, F); else if (b == 128) TK_TILES(T, 128, F); else TK_TILES(T, 256, F); } while (0)
     if (type == TK_IMG_F32) TK_TILES_B(float, false);
@@ -1938,18 +1968,27 @@ bool tk_launch_mixers_step(int type, const TkAttnArgs& a, const TkDeltaArgs& d, 
 
 size_t tk_delta_chunk_floats(int heads, int dim, int rows) { return (size_t)(rows / DC + rows / TK_DELTA_CHUNKED) * heads * delta_chunk_floats(delta_pad(dim)); }
 
-void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_runs, int n_chunks, int nrows, hipStream_t s) {
+void tk_launch_delta_scan(int type, const TkDeltaArgs& d, const TkPassTab& t, int n_segments, int shortest, int n_runs, int n_chunks, int nrows, hipStream_t s, const TkAttnArgs* beside,
+                          const int32_t* tiles, int n_tiles) {
     const int below = n_runs > 0 ? TK_DELTA_CHUNKED : 1 << 30;
+    /* the attention branch's tiles beside the chain, where that leaves CUs idle and both have the head sizes of the joint kernel */
+    const int vb = (d.vdim + 15) / 16, chains = d.heads * vb * n_runs, pad = delta_pad(d.dim);
+    const bool joint = beside && n_tiles > 0 && chains > 0 && chains <= 256 && type == TK_IMG_BF16 && attn_full(*beside) && attn_bucket(*beside) == pad && pad <= 128;
+    if (beside && n_tiles > 0 && !joint) tk_launch_attn_tiles(type, *beside, t, tiles, n_tiles, s);
     if (n_runs > 0) {
-        const dim3 chunks(d.heads, n_chunks), chain(d.heads, (d.vdim + 15) / 16, n_runs); /* heads first: a head's workgroups share an XCD's L2 */
+        const dim3 chunks(d.heads, n_chunks), chain(d.heads, vb, n_runs); /* heads first: a head's workgroups share an XCD's L2 */
+#define TK_JOINT(DP) hipLaunchKernelGGL((k_chain_and_tiles<TkBf16, DP, DP>), dim3(chains + n_tiles * beside->heads), dim3(256), std::max(attn_tiles_lds(type, *beside), sizeof(DeltaChainLds)), s, d, *beside, t, \
+                                        tiles, n_tiles, vb, chains)
 #define TK_CHUNKED(DP) do { hipLaunchKernelGGL((k_delta_chunk<DP>), chunks, dim3(256), 0, s, d, t, n_runs); \
-        hipLaunchKernelGGL((k_delta_chain<DP, false>), chain, dim3(256), 0, s, d, t); hipLaunchKernelGGL((k_delta_chain<DP, true>), chain, dim3(256), 0, s, d, t); } while (0)
+        if (!joint) hipLaunchKernelGGL((k_delta_chain<DP, false>), chain, dim3(256), 0, s, d, t); else if constexpr (DP <= 128) TK_JOINT(DP); \
+        hipLaunchKernelGGL((k_delta_chain<DP, true>), chain, dim3(256), 0, s, d, t); } while (0)
         switch (delta_pad(d.dim)) {
             case 64: TK_CHUNKED(64); break;
             case 128: TK_CHUNKED(128); break;
             default: TK_CHUNKED(256);
         }
 #undef TK_CHUNKED
+#undef TK_JOINT
     }
     if (shortest < below) {
         const bool many = (int64_t)((d.vdim + 15) / 16) * d.heads * n_segments >= 512;
@@ -2042,6 +2081,7 @@ const char* tk_mixer_prepare_device() {
     std::lock_guard<std::mutex> lk(mu);
     hipError_t e = hipSuccess;
     auto opt = [&](const void* f) { if (e == hipSuccess) e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024); };
+    opt((const void*)k_chain_and_tiles<TkBf16, 64, 64>); opt((const void*)k_chain_and_tiles<TkBf16, 128, 128>);
     opt((const void*)k_attn_tiles<float, 64, false>); opt((const void*)k_attn_tiles<float, 128, false>); opt((const void*)k_attn_tiles<float, 256, false>);
     opt((const void*)k_attn_tiles<TkBf16, 64, false>); opt((const void*)k_attn_tiles<TkBf16, 128, false>); opt((const void*)k_attn_tiles<TkBf16, 256, false>);
     opt((const void*)k_attn_tiles<TkBf16, 64, true>); opt((const void*)k_attn_tiles<TkBf16, 128, true>); opt((const void*)k_attn_tiles<TkBf16, 256, true>);
