@@ -437,7 +437,8 @@ __device__ __forceinline__ void delta_unit(const TkDeltaArgs& d, const TkPassTab
         if (row >= nrows) break;
         float ss = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) { y[r][i] = tk_silu32(y[r][i]); ss += y[r][i] * y[r][i]; } /* silu(0) = 0 past the head */
+        for (int i = 0; i < 4; ++i)
+            if (64 * i < n) { y[r][i] = tk_silu32(y[r][i]); ss += y[r][i] * y[r][i]; } /* (silu(0) = 0 past the head.)  Some 35 instructions each in a kernel that is vector work */
         float f = 1.0f;
         if (which < 2) {
             f = 1.0f / sqrtf(tk_wave_sum(ss) + d.unit_eps);
