@@ -38,6 +38,8 @@ public:
 /* floats of scratch that a TkAsr of up to `max_batch` clips works in */
 size_t tk_asr_arena_floats(const TkWhisperHP& hp, const TkWhManifest& man, int max_batch);
 
+#define TK_ASR_SPAN_ROWS 128 /* rows (sequences x positions) of a pass over a prompt, where there are fewer sequences */
+
 class TkAsr {
 public:
     TkWhisperModel* model = nullptr;

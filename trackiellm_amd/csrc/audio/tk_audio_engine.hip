@@ -141,19 +141,19 @@ __device__ __forceinline__ float at1_score(const float* kp, int blk, int Tk, int
     return a + 0.0f;
 }
 
-/* scores [sequences][heads][pitch] of a long context: grid (64-key blocks / 4, heads, sequences), a block of keys per wave */
+/* scores [rows][heads][pitch] of a long context: grid (64-key blocks / 4, heads, rows), a block of keys per wave; row i `group` + b is a row of sequence b */
 __global__ __launch_bounds__(256) void k_attend1_scores(const float* q, const float* k, float* scores, int Tk, int pitch, int64_t q_bstride, int64_t kv_bstride, int d, int hd,
-                                                        float scale) {
+                                                        int group, float scale) {
     extern __shared__ __attribute__((aligned(16))) uint8_t att1_lds[];
-    const int h = blockIdx.y, b = blockIdx.z, lane = threadIdx.x & 63;
+    const int h = blockIdx.y, row = blockIdx.z, b = (int)gridDim.z > group ? (int)((unsigned)row % (unsigned)group) : row, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     float* qs = (float*)(att1_lds + 4 * TK_AT1_RING);
-    for (int i = threadIdx.x; i < hd; i += 256) qs[i] = q[(int64_t)b * q_bstride + (int64_t)h * hd + i];
+    for (int i = threadIdx.x; i < hd; i += 256) qs[i] = q[(int64_t)row * q_bstride + (int64_t)h * hd + i];
     __syncthreads();
     const int blk = blockIdx.x * 4 + wave;
     if (blk * 64 >= Tk) return;
     const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, blk, Tk, d, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
-    if (blk * 64 + lane < Tk) scores[((int64_t)b * gridDim.y + h) * pitch + blk * 64 + lane] = a;
+    if (blk * 64 + lane < Tk) scores[((int64_t)row * gridDim.y + h) * pitch + blk * 64 + lane] = a;
 }
 
 /* tasks of a thread in a round of V (kernel below), and what a round takes of C columns: the whole of a self attention's usual context at once */
@@ -167,9 +167,12 @@ enum { AT1_SELF, AT1_HELD, AT1_LONG };
 template <int FORM>
 __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, const float* k, const float* v, const float* scores, int pitch, float* out, int Tk,
                                                            int64_t q_bstride, int64_t kv_bstride, int d, int hd, int split, float scale, int sc_at /* bytes */,
-                                                           float* img /* optional: out also as the tiled GEMM's operand image [B rows][K = d] */) {
+                                                           int more /* keys that each position of a span sees beyond the one before */,
+                                                           float* img /* optional: out also as the tiled GEMM's operand image [rows][K = d] */) {
     extern __shared__ __attribute__((aligned(16))) uint8_t att1_lds[];
-    const int h = blockIdx.x / split, part = blockIdx.x % split, b = blockIdx.y, t0 = threadIdx.x, lane = t0 & 63;
+    /* grid (heads * split, sequences, positions) */
+    const int h = blockIdx.x / split, part = blockIdx.x % split, b = blockIdx.y, row = blockIdx.z * gridDim.y + b, t0 = threadIdx.x, lane = t0 & 63;
+    Tk += (int)blockIdx.z * more;
     const int wave = __builtin_amdgcn_readfirstlane(t0 >> 6);
     float* vbuf = (float*)att1_lds;         /* a round of V; before it the waves' rings of K */
     float* sc = (float*)(att1_lds + sc_at); /* [Tk rounded up to 16] */
@@ -182,7 +185,7 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
     constexpr bool SELF = FORM == AT1_SELF;
     constexpr int NS = SELF ? TK_AT1_SELF / 256 : TK_AT1_HELD / 256;
     float e[NS];
-    const float* sp = scores + ((int64_t)b * (gridDim.x / split) + h) * pitch;
+    const float* sp = scores + ((int64_t)row * (gridDim.x / split) + h) * pitch;
     auto load_scores = [&](int k0) {
 #pragma unroll
         for (int j = 0; j < NS; ++j) { const int t = k0 + (t0 & 255) + 256 * j; e[j] = sp[t < Tk ? t : Tk - 1]; }
@@ -223,7 +226,7 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
     load_v(0);
     __builtin_amdgcn_sched_barrier(0);
     if (SELF) {
-        const float* qp = q + (int64_t)b * q_bstride + (int64_t)h * hd;
+        const float* qp = q + (int64_t)row * q_bstride + (int64_t)h * hd;
         for (int i = t0; i < hd; i += 64 * TK_AT1_NW) qs[i] = qp[i];
         __syncthreads();
         if (wave * 64 < Tk) {
@@ -329,8 +332,8 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
         if (c0 - col >= C || g != 0) break;
         const int kk = h * hd + part * C + c0;
         const float r = acc[w][0] + 0.0f;
-        out[(int64_t)b * q_bstride + kk] = r;
-        if (img) img[(int64_t)(b >> 4) * 16 * d + (int64_t)(kk >> 4) * 256 + (kk & 3) * 64 + (b & 15) * 4 + ((kk & 15) >> 2)] = r;
+        out[(int64_t)row * q_bstride + kk] = r;
+        if (img) img[(int64_t)(row >> 4) * 16 * d + (int64_t)(kk >> 4) * 256 + (kk & 3) * 64 + (row & 15) * 4 + ((kk & 15) >> 2)] = r;
     }
 }
 /* bytes in front of the weights: the rings of K or a round of V, whichever is more */
@@ -346,21 +349,23 @@ static bool at1_prepare_device() {
            hipFuncSetAttribute((const void*)k_attend1<AT1_LONG>, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess &&
            hipFuncSetAttribute((const void*)k_attend1_scores, hipFuncAttributeMaxDynamicSharedMemorySize, most) == hipSuccess;
 }
-/* scores: scratch [B][nh][pitch] */
-static bool at1_launch(const float* q, const float* k, const float* v, float* scores, int pitch, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh,
-                       float* img, hipStream_t s) {
-    const int hd = d / nh;
+/* n positions of B sequences, rows position by position; the first sees Tk keys, each next one `more` further ones (0, or 1 with at most TK_AT1_SELF keys for the last).
+ * scores: scratch [B n][nh][pitch] */
+static bool at1_launch(const float* q, const float* k, const float* v, float* scores, int pitch, float* out, int B, int n, int Tk, int more, int64_t q_bstride, int64_t kv_bstride,
+                       int d, int nh, float* img, hipStream_t s) {
+    const int hd = d / nh, most = Tk + (n - 1) * more;
+    if (n < 1 || (more != 0 && (more != 1 || most > TK_AT1_SELF))) return false;
     const float scale = tk_divf(1.0f, tk_sqrtf((float)hd));
     int split = 1; /* workgroups per head: 16 outputs each at least, while all of them run at once */
-    while (hd % (32 * split) == 0 && 2 * split * nh * B <= 256) split *= 2;
-    const dim3 grid(nh * split, B), block(64 * TK_AT1_NW);
-    const int sc_at = at1_buffer(Tk, hd / split);
-    const size_t lds = (size_t)sc_at + (size_t)(((Tk + 15) & ~15) + hd + 8) * 4; /* <= 128 KiB + 3 KiB, 96 KiB + 10 KiB, 96 KiB + 50 KiB */
-    if (Tk <= TK_AT1_SELF) {
-        hipLaunchKernelGGL((k_attend1<AT1_SELF>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img);
+    while (hd % (32 * split) == 0 && 2 * split * nh * B * n <= 256) split *= 2;
+    const dim3 grid(nh * split, B, n), block(64 * TK_AT1_NW);
+    const int sc_at = at1_buffer(most, hd / split);
+    const size_t lds = (size_t)sc_at + (size_t)(((most + 15) & ~15) + hd + 8) * 4; /* <= 128 KiB + 3 KiB, 96 KiB + 10 KiB, 96 KiB + 50 KiB */
+#define TK_AT1(FORM) hipLaunchKernelGGL((k_attend1<FORM>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, more, img)
+    if (most <= TK_AT1_SELF) {
+        TK_AT1(AT1_SELF);
     } else {
-        hipLaunchKernelGGL(k_attend1_scores, dim3(((Tk + 63) / 64 + 3) / 4, nh, B), dim3(256), 4 * TK_AT1_RING + (size_t)hd * 4, s, q, k, scores, Tk, pitch, q_bstride, kv_bstride, d, hd, scale);
-#define TK_AT1(FORM) hipLaunchKernelGGL((k_attend1<FORM>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, img)
+        hipLaunchKernelGGL(k_attend1_scores, dim3(((Tk + 63) / 64 + 3) / 4, nh, B * n), dim3(256), 4 * TK_AT1_RING + (size_t)hd * 4, s, q, k, scores, Tk, pitch, q_bstride, kv_bstride, d, hd, B, scale);
         if (Tk <= TK_AT1_HELD) TK_AT1(AT1_HELD); else TK_AT1(AT1_LONG);
 #undef TK_AT1
     }
@@ -473,7 +478,8 @@ struct TkAudioGpuOps {
         }
         /* does the output overlap the packed matrix (an in-place layer)?  Then the image is stale once the launch has run */
         const float* c0 = g.C;
-        const float* c1 = g.C + (size_t)(g.M - 1) * g.ldc + g.N;
+        const int c_rows = g.c_group > 0 && g.c_group < g.M ? g.c_group : g.M;
+        const float* c1 = g.C + (size_t)(c_rows - 1) * g.ldc + (g.c_group > 0 ? (size_t)((g.M - 1) / g.c_group) * (size_t)g.c_gstride : 0) + g.N;
         const float* a0 = g.A;
         const float* a1 = g.A + (size_t)(g.M - 1) * g.lda + g.K;
         const bool in_place = c0 < a1 && a0 < c1;
@@ -490,10 +496,12 @@ struct TkAudioGpuOps {
             const int i = pend.n++;
             t.tiles[i] = a->model->wt[(size_t)idx]; t.row_tiles[i] = g.N / 16;
             t.seg_out[i] = g.C; t.seg_ldc[i] = g.ldc; t.seg_bias[i] = g.bias; t.seg_n[i] = g.N; t.seg_img[i] = g.c_image;
+            t.seg_group[i] = g.c_group; t.seg_gstride[i] = g.c_gstride;
             if (pend.n == 3) flush();
             return; /* none of these layers writes into its own input: `plain` excludes in-place layers */
         }
         flush();
+        if (g.c_group) a->launch_error = "rows in groups need a plain layer"; /* not reached: keys and values are written into caches, by layers without a residual */
         TkTiledGemm t{};
         t.tiles[0] = a->model->wt[(size_t)idx]; t.row_tiles[0] = (g.N + 15) / 16; t.nseg = 1; t.wbytes = 4;
         t.K = g.K; t.ks = 1; t.ldc = g.ldc; t.n_valid = g.N; t.nrows = g.M; t.slab_rows = 0;
@@ -542,7 +550,19 @@ struct TkAudioGpuOps {
         const int hd = d / nh;
         if (hd > 256 || (hd & 15) || (d & 3) || Tk < 1 || Tk > TK_AT1_MAX_KEYS) return false; /* the three-launch form takes what does not fit */
         float* img = (short_pass(B) && d % 128 == 0 && q_bstride == d) ? image_for(out, B, d, d) : nullptr; /* the output projection's input, packed on the way out */
-        return at1_launch(q, k, v, scores, pitch, out, B, Tk, q_bstride, kv_bstride, d, nh, img, s);
+        return at1_launch(q, k, v, scores, pitch, out, B, 1, Tk, 0, q_bstride, kv_bstride, d, nh, img, s);
+    }
+    /* positions of a prompt that one pass takes: as many as make TK_ASR_SPAN_ROWS rows.  0, for one by one as they are decoded, where a layer's widths are not those of the
+     * kernels that know of several, or where the span's keys need scores from a launch of their own */
+    static int span(const TkWhisperHP& h, int B) {
+        const int dt = h.n_text_state, hd = dt / h.n_text_head;
+        if (dt % 128 || hd > 256 || (hd & 15) || h.n_text_ctx > TK_AT1_SELF || h.n_audio_ctx > TK_AT1_MAX_KEYS) return 0;
+        return B < TK_ASR_SPAN_ROWS ? TK_ASR_SPAN_ROWS / B : 1;
+    }
+    void attend_span(const float* q, const float* k, const float* v, float* out, int B, int n, int Tk, bool causal, int64_t q_bstride, int64_t kv_bstride, int d, int nh, float* scores, int pitch) {
+        drop_image();
+        float* img = image_for(out, B * n, d, d);
+        if (!at1_launch(q, k, v, scores, pitch, out, B, n, Tk, causal ? 1 : 0, q_bstride, kv_bstride, d, nh, img, s)) a->launch_error = "decoder attention launch refused";
     }
     /* an encoder layer's attention on operand images: 16 rows of a head in one workgroup, no score matrix.  All contexts it has registers for take it (three launches
      * and their score matrix else): at 1500 positions and six heads 97 -> 56 us a layer for one clip, 2106 -> 1194 us for 32 */
@@ -584,7 +604,6 @@ struct TkAudioGpuOps {
         } else {
             tk_launch_pick_rows(x, rows, cols, ld, out, pk, s);
         }
-        a->pick.step++;
     }
     void frames(const int16_t* pcm, int B, int n_samples, int pcm_stride, int n_total, int T, const float* window, float* out) {
         drop_image();
@@ -626,6 +645,7 @@ struct TkAudioSizeOps {
     bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int d, int, float*, int) { image(B, d); return true; }
     bool takes_images(const float*, const float*, const float*, int, int, int) { return false; }
     void attend_images(const float*, const float*, const float*, float*, int, int, int, int) {}
+    void attend_span(const float*, const float*, const float*, float*, int B, int n, int, bool, int64_t, int64_t, int d, int, float*, int) { image(B * n, d); }
     bool attend_fused(const float*, const float*, const float*, float*, int, int, int, int64_t, int64_t, int, int) { return false; } /* sized for the exact form */
     void add_rows(float*, const float*, int, int, int) {}
     void embed_rows(const float*, const float*, const int32_t*, const int32_t*, int, int, float*) {}
@@ -762,8 +782,10 @@ size_t tk_asr_arena_floats(const TkWhisperHP& hp, const TkWhManifest& man, int m
     TkWhisperGraph<TkAudioSizeOps> g{hp, man, nullw.data()};
     float* ml = g.mel(so, nullptr, mb, 0, 0);
     float* enc = g.encode(so, ml, mb);
-    auto st = g.begin_decode(so, enc, mb);
+    const int rows = mb > TK_ASR_SPAN_ROWS ? mb : TK_ASR_SPAN_ROWS;
+    auto st = g.begin_decode(so, enc, mb, rows);
     so.alloc_i32((size_t)3 * hp.n_text_ctx * mb);
+    st.B = rows; /* a pass's widest images */
     g.decode_step(so, st, 0);
     return so.peak + 4096;
 }
@@ -930,7 +952,7 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     ops.long_ok = true;
     float* ml = g.mel(ops, pcm_dev, B, n_samples, n_samples);
     float* enc = g.encode(ops, ml, B);
-    auto st = g.begin_decode(ops, enc, B);
+    auto st = g.begin_decode(ops, enc, B, B > TK_ASR_SPAN_ROWS ? B : TK_ASR_SPAN_ROWS);
     ops.long_ok = false;
     HIPQ(hipGetLastError());
     /* The mel, the encoder's output and the first logits travel to pinned memory on a stream of their own, and from there to the caller while the decoder's steps run:
@@ -971,11 +993,19 @@ bool TkAsr::transcribe(int B, const int16_t* pcm, int n_samples, const int32_t* 
     HIPQ(hipMemcpyAsync(tok_tab, host_tab.data(), host_tab.size() * 4, hipMemcpyHostToDevice, stream));
     int steps_run = n_steps; /* sampled positions really enqueued */
     std::vector<int32_t> st_host;
+    /* the prompt's positions several at a time (a pass is bound by its chains and launches, whose number this halves for a prompt of two: 17 positions
+     * of one clip 230 us less of 4.8 ms, of 32 clips 320 us of 6.5); logits of the sampled position alone */
+    const int span = TkAudioGpuOps::span(h, B);
     for (int p = 0; p < total; ++p) {
         st.tok = p < n_prompt ? tok_tab + (size_t)p * B : out_tab + (size_t)(p - 1) * B;
         st.pos = pos_tab + (size_t)p * B;
-        st.next = out_tab + (size_t)p * B;
-        g.decode_step(ops, st, p);
+        const int left = (n_prompt < total ? n_prompt : total) - p, n = left < span ? left : span;
+        const int at = n > 1 ? p + n - 1 : p; /* the pass's last position */
+        st.next = out_tab + (size_t)at * B;
+        pick.step = at;
+        if (n > 1 || (n == 1 && at < n_prompt - 1)) g.prompt_span(ops, st, p, n, at == n_prompt - 1);
+        else g.decode_step(ops, st, p);
+        p = at;
         if (p == n_prompt - 1 && first_logits) {
             ops.flush();
             HIPQ(hipMemcpyAsync(lg_at, st.logits, n_lg * 4, hipMemcpyDeviceToHost, stream)); /* (the next step writes them again) */

@@ -18,6 +18,7 @@
  *     their linear layers wrote as operand images (TkGemm::c_image; same arithmetic); `out` then feeds linear layer `o` only
  *   bool attend_fused(...): optional one-kernel form of attention() for many query rows (the GPU's opt-in fast contraction: NOT the same
  *     arithmetic, ~1e-6 of scale off; the oracle and the exact path return false)
+ *   void attend_span(...): attention of n positions of every sequence (a causal span, or all keys for all), for prompt_span() alone
  *   void add_rows(float* x, const float* add, int rows, int D, int add_rows);
  *   void embed_rows(const float* table, const float* pos, const int32_t* idx, const int32_t* pos_idx, int rows, int D, float* out);
  *   void argmax_rows(const float* x, int rows, int cols, int ld, int32_t* out);
@@ -277,7 +278,9 @@ struct TkWhisperGraph {
         int32_t *tok, *pos, *next;
     };
 
-    DecState begin_decode(Ops& o, const float* enc, int B) const {
+    /* rows: of the widest pass, at least B */
+    DecState begin_decode(Ops& o, const float* enc, int B, int rows = 0) const {
+        if (rows < B) rows = B;
         const int Tc = h.n_audio_ctx, d = h.n_audio_state, dt = h.n_text_state;
         DecState s;
         s.B = B;
@@ -286,43 +289,62 @@ struct TkWhisperGraph {
             s.sk.push_back(o.alloc((size_t)B * h.n_text_ctx * dt));
             s.sv.push_back(o.alloc((size_t)B * h.n_text_ctx * dt));
         }
-        s.x = o.alloc((size_t)B * dt); s.hb = o.alloc((size_t)B * dt); s.q = o.alloc((size_t)B * dt);
-        s.k = o.alloc((size_t)B * dt); s.v = o.alloc((size_t)B * dt); s.at = o.alloc((size_t)B * dt);
-        s.ff = o.alloc((size_t)B * 4 * dt);
+        s.x = o.alloc((size_t)rows * dt); s.hb = o.alloc((size_t)rows * dt); s.q = o.alloc((size_t)rows * dt);
+        s.k = o.alloc((size_t)rows * dt); s.v = o.alloc((size_t)rows * dt); s.at = o.alloc((size_t)rows * dt);
+        s.ff = o.alloc((size_t)rows * 4 * dt);
         for (int l = 0; l < h.n_text_layer; ++l) { /* all on one input, one behind the other: packed once, launched together */
             const TkWhLayerIdx& L = m.dec[l];
             o.gemm(lin(enc, B * Tc, d, d, W[L.xk_w], nullptr, dt, s.xk[l], dt));
             o.gemm(lin(enc, B * Tc, d, d, W[L.xv_w], W[L.xv_b], dt, s.xv[l], dt));
         }
         const int tmax = Tc > h.n_text_ctx ? Tc : h.n_text_ctx;
-        s.sc = o.alloc((size_t)B * h.n_text_head * score_pitch(tmax));
+        s.sc = o.alloc((size_t)rows * h.n_text_head * score_pitch(tmax));
         s.logits = o.alloc((size_t)B * h.n_vocab);
         s.tok = o.alloc_i32(B); s.pos = o.alloc_i32(B); s.next = o.alloc_i32(B);
         return s;
     }
 
     /* one decoder step at position p for all B sequences: tokens in s.tok, positions in s.pos (== p); argmax -> s.next */
-    void decode_step(Ops& o, DecState& s, int p) const {
+    void decode_step(Ops& o, DecState& s, int p) const { pass<false>(o, s, p, 1, true); }
+    /* positions p .. p + n - 1 of a prompt in one pass, rows position by position: row i B + b of s.tok and s.pos.  `sampled`: the last of them is, argmax -> s.next;
+     * else the last layer ends at its keys and values.  For backends with attend_span() */
+    void prompt_span(Ops& o, DecState& s, int p, int n, bool sampled) const { pass<true>(o, s, p, n, sampled); }
+
+private:
+    template <bool SPAN> void pass(Ops& o, DecState& s, int p, int n, bool sampled) const {
         const int B = s.B, Tc = h.n_audio_ctx, dt = h.n_text_state, nh = h.n_text_head, ctx = h.n_text_ctx;
-        o.embed_rows(W[m.tok_emb], W[m.dec_pos], s.tok, s.pos, B, dt, s.x);
+        int R = B * n; /* rows */
+        float *x = s.x, *q = s.q;
+        o.embed_rows(W[m.tok_emb], W[m.dec_pos], s.tok, s.pos, R, dt, x);
         for (int l = 0; l < h.n_text_layer; ++l) {
             const TkWhLayerIdx& L = m.dec[l];
-            o.layernorm(s.x, B, dt, W[L.ln1_w], W[L.ln1_b], s.hb);
-            o.gemm(lin(s.hb, B, dt, dt, W[L.q_w], W[L.q_b], dt, s.q, dt));
-            /* k, v of this position go straight into the caches (row p of every sequence) */
-            o.gemm(lin(s.hb, B, dt, dt, W[L.k_w], nullptr, dt, s.sk[l] + (size_t)p * dt, ctx * dt));
-            o.gemm(lin(s.hb, B, dt, dt, W[L.v_w], W[L.v_b], dt, s.sv[l] + (size_t)p * dt, ctx * dt));
-            attention(o, s.q, s.sk[l], s.sv[l], s.at, B, 1, p + 1, dt, (int64_t)ctx * dt, dt, nh, s.sc);
-            o.gemm(lin(s.at, B, dt, dt, W[L.o_w], W[L.o_b], dt, s.x, dt, 0, s.x, dt));
-            o.layernorm(s.x, B, dt, W[L.lnx_w], W[L.lnx_b], s.hb);
-            o.gemm(lin(s.hb, B, dt, dt, W[L.xq_w], W[L.xq_b], dt, s.q, dt));
-            attention(o, s.q, s.xk[l], s.xv[l], s.at, B, 1, Tc, dt, (int64_t)Tc * dt, dt, nh, s.sc);
-            o.gemm(lin(s.at, B, dt, dt, W[L.xo_w], W[L.xo_b], dt, s.x, dt, 0, s.x, dt));
-            o.layernorm(s.x, B, dt, W[L.ln2_w], W[L.ln2_b], s.hb);
-            { TkGemm g1 = lin(s.hb, B, dt, dt, W[L.fc1_w], W[L.fc1_b], 4 * dt, s.ff, 4 * dt, TK_ACT_GELU); g1.c_feeds_linear = 1; o.gemm(g1); }
-            o.gemm(lin(s.ff, B, 4 * dt, 4 * dt, W[L.fc2_w], W[L.fc2_b], dt, s.x, dt, 0, s.x, dt));
+            const bool last = SPAN && l == h.n_text_layer - 1;
+            o.layernorm(x, R, dt, W[L.ln1_w], W[L.ln1_b], s.hb);
+            if (sampled || !last) o.gemm(lin(s.hb, R, dt, dt, W[L.q_w], W[L.q_b], dt, q, dt));
+            /* k, v of these positions go straight into the caches (rows p .. of every sequence) */
+            TkGemm gk = lin(s.hb, R, dt, dt, W[L.k_w], nullptr, dt, s.sk[l] + (size_t)p * dt, ctx * dt);
+            TkGemm gv = lin(s.hb, R, dt, dt, W[L.v_w], W[L.v_b], dt, s.sv[l] + (size_t)p * dt, ctx * dt);
+            if (n > 1) { gk.c_group = gv.c_group = B; gk.c_gstride = gv.c_gstride = dt; }
+            o.gemm(gk);
+            o.gemm(gv);
+            if (last) { /* behind its keys and values: the sampled rows */
+                if (!sampled) return;
+                x += (size_t)(n - 1) * B * dt; q += (size_t)(n - 1) * B * dt;
+                p += n - 1; n = 1; R = B;
+            }
+            if constexpr (SPAN) o.attend_span(q, s.sk[l], s.sv[l], s.at, B, n, p + 1, true, dt, (int64_t)ctx * dt, dt, nh, s.sc, score_pitch(p + n));
+            else attention(o, q, s.sk[l], s.sv[l], s.at, B, 1, p + 1, dt, (int64_t)ctx * dt, dt, nh, s.sc);
+            o.gemm(lin(s.at, R, dt, dt, W[L.o_w], W[L.o_b], dt, x, dt, 0, x, dt));
+            o.layernorm(x, R, dt, W[L.lnx_w], W[L.lnx_b], s.hb);
+            o.gemm(lin(s.hb, R, dt, dt, W[L.xq_w], W[L.xq_b], dt, q, dt));
+            if constexpr (SPAN) o.attend_span(q, s.xk[l], s.xv[l], s.at, B, n, Tc, false, dt, (int64_t)Tc * dt, dt, nh, s.sc, score_pitch(Tc));
+            else attention(o, q, s.xk[l], s.xv[l], s.at, B, 1, Tc, dt, (int64_t)Tc * dt, dt, nh, s.sc);
+            o.gemm(lin(s.at, R, dt, dt, W[L.xo_w], W[L.xo_b], dt, x, dt, 0, x, dt));
+            o.layernorm(x, R, dt, W[L.ln2_w], W[L.ln2_b], s.hb);
+            { TkGemm g1 = lin(s.hb, R, dt, dt, W[L.fc1_w], W[L.fc1_b], 4 * dt, s.ff, 4 * dt, TK_ACT_GELU); g1.c_feeds_linear = 1; o.gemm(g1); }
+            o.gemm(lin(s.ff, R, 4 * dt, 4 * dt, W[L.fc2_w], W[L.fc2_b], dt, x, dt, 0, x, dt));
         }
-        o.layernorm(s.x, B, dt, W[m.dec_ln_w], W[m.dec_ln_b], s.hb);
+        o.layernorm(x, B, dt, W[m.dec_ln_w], W[m.dec_ln_b], s.hb);
         o.gemm(lin(s.hb, B, dt, dt, W[m.tok_emb], nullptr, h.n_vocab, s.logits, h.n_vocab));
         o.argmax_rows(s.logits, B, h.n_vocab, h.n_vocab, s.next);
     }
