@@ -399,13 +399,21 @@ struct TkAudioGpuOps {
     /* Decoder steps of few sequences: a norm is not launched; the linear layers on it make it themselves (TkTiledGemm::ln_x).  pk then names its output, which nobody else
      * reads, and has no image.  A layer that cannot take it has it launched first.  Up to TK_TW_LN_ROWS sequences: calls of 40 steps for 1, 2, 4, 6, 8, 16 clips, norms
      * launched / in the products: 13.36 / 12.34, 14.39 / 13.28, 16.08 / 15.45, 17.31 / 17.27, 18.92 / 19.24, 23.65 / 26.00 ms. */
-    struct { const float *x = nullptr, *w = nullptr, *b = nullptr; float* y = nullptr; bool live = false, used = false; } norm;
+    /* Other norms of a whole number of 128 columns wait for their first reader: a layer with tiles gets an operand image and no rows (48 000 rows of 384 columns: 70 -> 28 us),
+     * anything else the rows. */
+    struct { const float *x = nullptr, *w = nullptr, *b = nullptr; float* y = nullptr; bool live = false, used = false, in_products = false; } norm;
     static bool norm_fits(int rows, int D) { return rows <= TK_TW_LN_ROWS && D <= TK_TW_LN_MAX && D % 128 == 0; }
-    void make_norm() { /* as a launch after all, with its image */
+    void make_norm(bool image) { /* as a launch after all */
         const int M = pk.M, K = pk.K;
-        norm.live = false;
-        float* img = image_for(norm.y, M, K, K);
-        tk_launch_layernorm(norm.x, M, K, norm.w, norm.b, TK_WH_LN_EPS, norm.y, s, img);
+        norm.live = pk.live = false;
+        if (image) tk_launch_layernorm_image(norm.x, M, K, norm.w, norm.b, TK_WH_LN_EPS, image_for(norm.y, M, K, K), s);
+        else tk_launch_layernorm(norm.x, M, K, norm.w, norm.b, TK_WH_LN_EPS, norm.y, s);
+    }
+    /* columns of a convolution wait for their reader in the same way */
+    struct { const float* x = nullptr; int B = 0, T = 0, C = 0, ldx = 0, kw = 0, stride = 0, pad = 0; float* col = nullptr; } cols;
+    void make_columns() {
+        if (cols.col) tk_launch_im2col1d(cols.x, cols.B, cols.T, cols.C, cols.ldx, cols.kw, cols.stride, cols.pad, cols.col, s);
+        cols.col = nullptr;
     }
     /* linear layers on the SAME packed input (q / k / v of a layer, the cross keys and values) are collected — up to three — and go out as ONE
      * launch with a destination per segment (q | k | v: the query buffer and row p of the two caches); anything else flushes the batch first */
@@ -421,7 +429,8 @@ struct TkAudioGpuOps {
     }
     void drop_image() {
         flush();
-        if (norm.live && !norm.used) make_norm(); /* (its readers are not linear layers) */
+        make_columns();
+        if (norm.live && !norm.used) make_norm(false); /* (its readers are not linear layers) */
         if (pk.live && !norm.live) a->arena_used = pk.mark;
         pk.live = norm.live = false;
     }
@@ -463,18 +472,23 @@ struct TkAudioGpuOps {
         }
         const int idx = tk_tiled_gemm_applies(g) ? a->model->tensor_of(g.B) : -1;
         if (idx < 0 || !a->model->wt[(size_t)idx]) {
-            if (norm.live) make_norm();
+            if (norm.live) make_norm(false);
             drop_image();
             tk_launch_gemm(g, s);
             return;
         }
         if (norm.live && !(pk.A == g.A && pk.M == g.M && pk.K == g.K && pk.lda == g.lda)) drop_image();
         if (!(pk.live && pk.A == g.A && pk.M == g.M && pk.K == g.K && pk.lda == g.lda)) {
+            const bool columns = cols.col == g.A && g.K == cols.kw * cols.C && g.lda == g.K && cols.C % 16 == 0;
+            if (columns) cols.col = nullptr;
             drop_image();
             pk.mark = a->arena_used;
             pk.img = raw_alloc(tk_tiled_gemm_scratch(g));
-            tk_launch_pack_a(g.A, g.M, g.K, g.lda, 0, pk.img, s);
+            if (columns) tk_launch_im2col1d_image(cols.x, cols.B, cols.T, cols.C, cols.ldx, cols.kw, cols.stride, cols.pad, pk.img, s);
+            else tk_launch_pack_a(g.A, g.M, g.K, g.lda, 0, pk.img, s);
             pk.A = g.A; pk.M = g.M; pk.K = g.K; pk.lda = g.lda; pk.live = true;
+        } else if (norm.live && !norm.in_products) {
+            make_norm(true);
         }
         /* does the output overlap the packed matrix (an in-place layer)?  Then the image is stale once the launch has run */
         const float* c0 = g.C;
@@ -533,16 +547,16 @@ struct TkAudioGpuOps {
         norm.used = true;
         t.ln_x = norm.x; t.ln_w = norm.w; t.ln_b = norm.b; t.ln_eps = TK_WH_LN_EPS;
     }
-    void im2col1d(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* col) { drop_image(); tk_launch_im2col1d(x, B, T, C, ldx, kw, stride, pad, col, s); }
+    void im2col1d(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* col) {
+        drop_image();
+        cols.x = x; cols.B = B; cols.T = T; cols.C = C; cols.ldx = ldx; cols.kw = kw; cols.stride = stride; cols.pad = pad; cols.col = col;
+    }
     void layernorm(const float* x, int rows, int D, const float* w, const float* b, float* y) {
         drop_image();
-        if (!long_ok && norm_fits(rows, D)) { /* a decoder step's: it feeds linear layers only */
-            norm.x = x; norm.w = w; norm.b = b; norm.y = y; norm.live = true; norm.used = false;
-            pk.A = y; pk.M = rows; pk.K = D; pk.lda = D; pk.img = nullptr; pk.mark = a->arena_used; pk.live = true;
-            return;
-        }
-        float* img = D % 128 == 0 && !(a->fast && long_ok) ? image_for(y, rows, D, D) : nullptr; /* a norm feeds linear layers: packed on the way out */
-        tk_launch_layernorm(x, rows, D, w, b, TK_WH_LN_EPS, y, s, img);
+        if (D % 128) { tk_launch_layernorm(x, rows, D, w, b, TK_WH_LN_EPS, y, s); return; }
+        norm.x = x; norm.w = w; norm.b = b; norm.y = y; norm.live = true; norm.used = false;
+        norm.in_products = !long_ok && norm_fits(rows, D); /* a decoder step's */
+        pk.A = y; pk.M = rows; pk.K = D; pk.lda = D; pk.img = nullptr; pk.mark = a->arena_used; pk.live = true;
     }
     void softmax_rows(float* x, int rows, int cols, int ld) { drop_image(); tk_launch_softmax_rows(x, rows, cols, ld, s); }
     bool attend1(const float* q, const float* k, const float* v, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh, float* scores, int pitch) {

@@ -234,12 +234,12 @@ struct TkWhisperGraph {
     float* encode(Ops& o, const float* ml, int B) const {
         const int T = h.n_frames(), Tc = h.n_audio_ctx, d = h.n_audio_state, nh = h.n_audio_head;
         float* col1 = o.alloc((size_t)B * T * 3 * h.n_mels);
-        o.im2col1d(ml, B, T, h.n_mels, h.n_mels, 3, 1, 1, col1);
         float* x1 = o.alloc((size_t)B * T * d);
+        o.im2col1d(ml, B, T, h.n_mels, h.n_mels, 3, 1, 1, col1);
         o.gemm(lin(col1, B * T, 3 * h.n_mels, 3 * h.n_mels, W[m.conv1_w], W[m.conv1_b], d, x1, d, TK_ACT_GELU));
         float* col2 = o.alloc((size_t)B * Tc * 3 * d);
-        o.im2col1d(x1, B, T, d, d, 3, 2, 1, col2);
         float* x = o.alloc((size_t)B * Tc * d);
+        o.im2col1d(x1, B, T, d, d, 3, 2, 1, col2);
         o.gemm(lin(col2, B * Tc, 3 * d, 3 * d, W[m.conv2_w], W[m.conv2_b], d, x, d, TK_ACT_GELU));
         o.add_rows(x, W[m.enc_pos], B * Tc, d, Tc);
         float* hb = o.alloc((size_t)B * Tc * d);

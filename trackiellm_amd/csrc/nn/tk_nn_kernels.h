@@ -47,6 +47,8 @@ void tk_launch_upsample2x(const float* x, int B, int H, int W, int C, int ldx, f
 void tk_launch_copy_cols(const float* x, int rows, int C, int ldx, float* y, int ldy, hipStream_t s);
 /* rows of [T][C] (row pitch ldx) -> col[b*To + t][(kx*C + c)], kernel width kw, zero padding `pad` on both ends */
 void tk_launch_im2col1d(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* col, hipStream_t s);
+/* as the tiled GEMM's operand image, C % 16 == 0 */
+void tk_launch_im2col1d_image(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* img, hipStream_t s);
 /* out[r][:] = table[idx[r]][:] + pos[(pos0[r])][:] */
 void tk_launch_embed_rows(const float* table, const float* pos, const int32_t* idx, const int32_t* pos_idx, int rows, int D, float* out, hipStream_t s);
 void tk_launch_argmax_rows(const float* x, int rows, int cols, int ld, int32_t* out, hipStream_t s);
@@ -63,7 +65,9 @@ void tk_launch_pick_rows(const float* x, int rows, int cols, int ld, int32_t* ou
 #define TK_WH_STATE_INTS 8
 struct TkWhFilter { const uint8_t* suppress; int32_t* state; int32_t beg, eot, tid0; };
 void tk_launch_pick_rows_filtered(const float* x, int rows, int cols, int ld, int32_t* out, const TkPick& pk, const TkWhFilter& f, hipStream_t s);
-void tk_launch_layernorm(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, hipStream_t s, float* img = nullptr /* optional: also the tiled GEMM's operand image of y */);
+void tk_launch_layernorm(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, hipStream_t s);
+/* as the tiled GEMM's operand image (csrc/nn/tk_gemm_tiled.h), D % 16 == 0; the rows of a last tile that are not there are left as they are */
+void tk_launch_layernorm_image(const float* x, int rows, int D, const float* w, const float* b, float eps, float* img, hipStream_t s);
 void tk_launch_softmax_rows(float* x, int rows, int cols, int ld, hipStream_t s);
 void tk_launch_add_rows(float* x, const float* add, int rows, int D, int add_rows, hipStream_t s);
 

@@ -1333,7 +1333,7 @@ __device__ __forceinline__ float nn_block_sum256(float v, float* red) {
 }
 
 /* y = ((x - mean) * rstd) * w + b ; sums in the canonical 256-partial order */
-/* img (optional): the rows are ALSO written as the tiled GEMM's operand image (csrc/nn/tk_gemm_tiled.h: element (row, k = 16 j + 4 t + g) at
+/* img: the rows are written as the tiled GEMM's operand image instead (csrc/nn/tk_gemm_tiled.h: element (row, k = 16 j + 4 t + g) at
  * [row / 16][j][g][row % 16][t]) — the linear layer behind a norm then needs no pack launch */
 __global__ __launch_bounds__(256) void k_layernorm(const float* x, int D, const float* w, const float* b, float eps, float* y, float* img) {
     __shared__ float red[4];
@@ -1349,8 +1349,8 @@ __global__ __launch_bounds__(256) void k_layernorm(const float* x, int D, const 
     float* ir = img ? img + (r >> 4) * 16 * (int64_t)D + (r & 15) * 4 : nullptr;
     for (int i = threadIdx.x; i < D; i += 256) {
         const float v = ((xr[i] - mean) * rstd) * w[i] + b[i];
-        y[r * D + i] = v;
         if (ir) ir[(int64_t)(i >> 4) * 256 + (i & 3) * 64 + ((i & 15) >> 2)] = v;
+        else y[r * D + i] = v;
     }
 }
 /* rows of up to 256 NV columns: k_layernorm on registers (thread j owns elements j, j + 256, ...), in the same order.  The row, w and b are requested
@@ -1384,11 +1384,73 @@ __global__ __launch_bounds__(256) void k_layernorm_reg(const float* x, int D, co
         const int i = threadIdx.x + 256 * u;
         if (i >= D) break;
         const float o = ((v[u] - mean) * rstd) * wv[u] + bv[u];
-        y[r * D + i] = o;
         if (ir) ir[(int64_t)(i >> 4) * 256 + (i & 3) * 64 + ((i & 15) >> 2)] = o;
+        else y[r * D + i] = o;
     }
 }
-void tk_launch_layernorm(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, hipStream_t s, float* img) {
+/* The image of 16 rows of up to 256 NV columns (multiples of 128), a wave a row: the 256 partial sums as four in a lane, folded in k_layernorm's order.  Bound by memory: a
+ * row alone writes 4 of the 64 bytes that lie together in the image, so the tile passes through LDS (rows 4 floats apart beyond their columns: 16 rows and four
+ * neighbours of them are in 64 banks).  48 000 rows of 384: 70 us a row in four waves, which wrote the rows too (alone 41), now 28 (148 MB) */
+template <int NV>
+__global__ __launch_bounds__(1024) void k_layernorm_tile(const float* x, int rows, int D, const float* w, const float* b, float eps, float* img) {
+    extern __shared__ __attribute__((aligned(16))) float ln_tile[]; /* [16][D + 4] */
+    const int lane = threadIdx.x & 63, r = threadIdx.x >> 6, pitch = D + 4;
+    const int64_t row = (int64_t)blockIdx.x * 16 + r;
+    const float* xr = x + (row < rows ? row : rows - 1) * D;
+    float v[NV][4], wv[NV][4], bv[NV][4];
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            int i = 256 * u + 64 * p + lane;
+            i = i < D ? i : D - 1;
+            v[u][p] = xr[i]; wv[u][p] = w[i]; bv[u][p] = b[i];
+        }
+    auto fold = [&](float (&s)[4]) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) s[p] = tk_wave_butterfly_sum(s[p]);
+        return ((s[0] + s[1]) + s[2]) + s[3];
+    };
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f}, q[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+            if (256 * u + 64 * p + lane < D) s[p] = s[p] + v[u][p];
+    const float mean = tk_divf(fold(s), (float)D);
+#pragma unroll
+    for (int p = 0; p < 4; ++p)
+#pragma unroll
+        for (int u = 0; u < NV; ++u)
+            if (256 * u + 64 * p + lane < D) { const float d = v[u][p] - mean; q[p] = tk_fmaf(d, d, q[p]); }
+    const float var = tk_divf(fold(q), (float)D);
+    const float rstd = tk_divf(1.0f, tk_sqrtf(var + eps));
+#pragma unroll
+    for (int u = 0; u < NV; ++u)
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+            const int i = 256 * u + 64 * p + lane;
+            if (i < D) ln_tile[r * pitch + i] = ((v[u][p] - mean) * rstd) * wv[u][p] + bv[u][p];
+        }
+    __syncthreads();
+    /* wave r: the 16-k groups j = r, r + 16, ...; lane (g, row) the four k = 16 j + 4 t + g */
+    const int g = lane >> 4, n = lane & 15;
+    if ((int64_t)blockIdx.x * 16 + n >= rows) return;
+    for (int j = r; j < D >> 4; j += 16) {
+        const float* f = ln_tile + n * pitch + 16 * j + g;
+        *(float4*)(img + (int64_t)blockIdx.x * 16 * D + j * 256 + lane * 4) = make_float4(f[0], f[4], f[8], f[12]);
+    }
+}
+void tk_launch_layernorm_image(const float* x, int rows, int D, const float* w, const float* b, float eps, float* img, hipStream_t s) {
+    const dim3 tiles((rows + 15) / 16);
+    const size_t lds = (size_t)16 * (D + 4) * 4; /* 60 KiB at 960 columns; more than 64 need leave */
+    if (D <= 512 && D % 64 == 0) hipLaunchKernelGGL((k_layernorm_tile<2>), tiles, dim3(1024), lds, s, x, rows, D, w, b, eps, img);
+    else if (D <= 960 && D % 64 == 0) hipLaunchKernelGGL((k_layernorm_tile<4>), tiles, dim3(1024), lds, s, x, rows, D, w, b, eps, img);
+    else if (D <= 1280) hipLaunchKernelGGL((k_layernorm_reg<5>), dim3(rows), dim3(256), 0, s, x, D, w, b, eps, (float*)nullptr, img);
+    else hipLaunchKernelGGL(k_layernorm, dim3(rows), dim3(256), 0, s, x, D, w, b, eps, (float*)nullptr, img);
+}
+void tk_launch_layernorm(const float* x, int rows, int D, const float* w, const float* b, float eps, float* y, hipStream_t s) {
+    float* const img = nullptr;
     if (D <= 512) hipLaunchKernelGGL((k_layernorm_reg<2>), dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
     else if (D <= 1280) hipLaunchKernelGGL((k_layernorm_reg<5>), dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
     else hipLaunchKernelGGL(k_layernorm, dim3(rows), dim3(256), 0, s, x, D, w, b, eps, y, img);
@@ -1523,6 +1585,27 @@ void tk_launch_im2col1d(const float* x, int B, int T, int C, int ldx, int kw, in
     int64_t blocks = (total + 255) / 256;
     if (blocks > 16384) blocks = 16384;
     hipLaunchKernelGGL(k_im2col1d, dim3((unsigned)blocks), dim3(256), 0, s, x, B, T, C, ldx, kw, stride, pad, To, col);
+}
+/* the column matrix as the tiled GEMM's operand image, C % 16 == 0: a wave makes 16 rows of a 16-k group, which lie in one tap.  32 clips of 1500 positions, 1152 k: columns
+ * and their packing 330 us, here 110 (147 MB read, 221 written) */
+__global__ __launch_bounds__(256) void k_im2col1d_image(const float* x, int64_t rows, int T, int C, int ldx, int groups, int stride, int pad, int To, float* img) {
+    const int64_t id = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); /* (M-tile, 16-k group) */
+    const int64_t mt = id / groups, row = mt * 16 + (threadIdx.x & 15);
+    const int j = (int)(id - mt * groups), g = (threadIdx.x >> 4) & 3, kx = 16 * j / C, c = 16 * j - kx * C + g;
+    if (row >= rows) return;
+    const int64_t b = row / To;
+    const int it = (int)(row - b * To) * stride + kx - pad;
+    float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (it >= 0 && it < T) {
+        const float* p = x + (b * T + it) * ldx + c;
+        v = make_float4(p[0], p[4], p[8], p[12]);
+    }
+    *(float4*)(img + id * 256 + (threadIdx.x & 63) * 4) = v;
+}
+void tk_launch_im2col1d_image(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* img, hipStream_t s) {
+    const int To = (T + 2 * pad - kw) / stride + 1, groups = kw * C / 16;
+    const int64_t rows = (int64_t)B * To, waves = (rows + 15) / 16 * groups;
+    hipLaunchKernelGGL(k_im2col1d_image, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, s, x, rows, T, C, ldx, groups, stride, pad, To, img);
 }
 
 __global__ void k_embed_rows(const float* table, const float* pos, const int32_t* idx, const int32_t* pos_idx, int D, float* out) {
