@@ -591,7 +591,7 @@ struct TkAudioGpuOps {
     void attend_images(const float* q, const float* k, const float* v, float* out, int B, int Tc, int d, int nh) {
         drop_image();
         float* img = image_for(out, B * Tc, d, d);
-        if (!tk_launch_attention_images(q, k, v, img, B, nh, Tc, Tc, d, tk_divf(1.0f, tk_sqrtf((float)(d / nh))), s)) a->launch_error = "attention launch refused";
+        if (!tk_launch_attention_images(q, k, v, img, B, nh, Tc, Tc, d, s)) a->launch_error = "attention launch refused";
     }
     /* the opt-in fast contraction's attention (TkAsr::fast): Q K^T, softmax and P V of a long pass in one kernel, no score matrix in HBM */
     bool attend_fused(const float* q, const float* k, const float* v, float* out, int B, int Tq, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh) {

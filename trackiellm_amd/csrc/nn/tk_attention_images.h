@@ -16,6 +16,6 @@ static inline bool tk_attention_images_fits(int Tq, int Tk, int d, int nh) {
     return Tq >= 1 && Tk >= 1 && Tk <= TK_AIM_MAX_KEYS && nh >= 1 && d == nh * 64;
 }
 /* q_img [B Tq][d], k_img [B Tk][d], out_img [B Tq][d]: images; v [B Tk][d] rows.  false (nothing launched): sizes it does not take */
-bool tk_launch_attention_images(const float* q_img, const float* k_img, const float* v, float* out_img, int B, int nh, int Tq, int Tk, int d, float scale, hipStream_t s);
+bool tk_launch_attention_images(const float* q_img, const float* k_img, const float* v, float* out_img, int B, int nh, int Tq, int Tk, int d, hipStream_t s);
 
 #endif

@@ -11,19 +11,24 @@ typedef float v4f __attribute__((ext_vector_type(4)));
  *   scores: S^T = K Q^T a tile of 16 keys at a time, K's rows handed over in the order 4 b + a for row 4 a + b, so that the accumulator a
  *     lane gets back (rows 4 g .. 4 g + 3 of its column) is keys 4 t + g, t = 0 .. 3, of its query: the layout of P as an operand of P V.
  *     They stay in registers (4 U float4 a lane) until the product needs them.
- *   softmax: the tree's levels 32 .. 4 are inside a lane, 2 and 1 between the four lanes of a query, the quarters meet in LDS.  Division by
- *     the row's sum: q = e y with y = RN(1 / sum), then two corrections by the exact remainder — the first leaves q within an ulp, the
- *     second rounds it correctly — as long as no remainder is subnormal (e >= 2^-100); the division itself otherwise.
+ *   softmax: the tree's levels 32 .. 4 are inside a lane, 2 and 1 between the four lanes of a query, the quarters meet in LDS.  Scores are
+ *     held unscaled: the scale 1 / 8 is a power of two, so (x / 8) - m rounds once, as one fma (a subnormal x / 8 does too, up to differences
+ *     below 2^-100, whose exponential is 1 either way).  Division by the row's sum: y = RN(1 / sum), yl what is missing of it, q = e y + e yl
+ *     within an ulp, and one correction by the exact remainder rounds it correctly (1.6e9 pairs, among them mantissas of nearly all ones and zeros,
+ *     compared with the division on a CPU: all equal) — as long as no remainder is subnormal (e >= 2^-100); the
+ *     division itself otherwise.
  *   output: P goes through LDS 256 keys at a time, two buffers; wave w makes columns 16 w .. 16 w + 15, one chain over all keys.
- * Bound by the fp32 matrix pipe, which fp32 vector instructions share: at 16 rows x 1500 keys 24.3 k cycles of MFMA and about 10 k of
- * exponentials and divisions per SIMD, 16 us; 32 clips of 1500 positions x 6 heads take 1194 us (three launches: 797 + 736 + 574), of which the
- * products alone are 725 us at the rate of a large one.
+ * Bound by the fp32 matrix pipe, which vector instructions share: at 16 rows x 1500 keys 24.3 k cycles of MFMA and 2400 vector instructions of
+ * four cycles per SIMD, nearly all of them exponentials and divisions: 97 % of its time.  32 clips of 1500 positions x 6 heads take 1205 us (three
+ * launches: 797 + 736 + 574), of which the products alone are 725 us at the rate of a large one.  With two corrections a division, a scale and a
+ * vector address for each tile of K, 1240 us; two forms of the exponential, one without the test for values below -87, cost more than they save.
  */
 template <int U>
 __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const float* q_img, const float* k_img, const float* v, float* out_img, int nh, int Tq, int Tk, int d,
-                                                                         int tiles, int total, int per_xcd, float scale) {
+                                                                         int tiles, int total, int per_xcd) {
     __shared__ v4f ring[2][16 * 64];
     __shared__ float top[4][16], sum[4][16];
+    constexpr float scale = 0.125f; /* 1 / sqrt(64) */
     /* consecutive workgroups go to different XCDs: each XCD takes a run of them, so that a head's K and V (768 KB) are read into few L2s */
     const int id = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
     if (id >= total) return;
@@ -43,13 +48,18 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
     const int64_t k0 = (int64_t)b * Tk;
     const __amdgpu_buffer_rsrc_t kr = __builtin_amdgcn_make_buffer_rsrc((void*)(k_img + (size_t)(k0 >> 4) * group), 0, (unsigned)((k0 + Tk + 15) / 16 - (k0 >> 4)) * (unsigned)group * 4u, 0x00020000);
     const int k_odd = (int)(k0 & 15), key_of_row = 4 * (n & 3) + (n >> 2), k_first = 16 * (4 * wave) + key_of_row;
-    auto load_k = [&](int i, v4f* f) { /* tile i of the wave */
-        int key = k_first + 16 * (16 * (i >> 2) + (i & 3));
-        if (i >= 4 * U - 4) key = key < Tk ? key : Tk - 1;
-        key += k_odd;
-        const unsigned at = (unsigned)(key >> 4) * (unsigned)(64 * d) + (unsigned)(key & 15) * 16u + (unsigned)g * 256u;
+    auto k_place = [&](int key) { key += k_odd; return (unsigned)(key >> 4) * (unsigned)(64 * d) + (unsigned)(key & 15) * 16u + (unsigned)g * 256u; };
+    const unsigned k_at = k_place(k_first);
+    auto load_k = [&](int i, v4f* f) { /* tile i of the wave: 16 keys on is 16 rows of the image on */
+        const int step = 16 * (i >> 2) + (i & 3);
+        unsigned at = k_at, from = 4 * h * 1024 + (unsigned)step * (unsigned)(64 * d);
+        if (i >= 4 * U - 4) {
+            const int key = k_first + 16 * step;
+            at = k_place(key < Tk ? key : Tk - 1);
+            from = 4 * h * 1024;
+        }
 #pragma unroll
-        for (int j = 0; j < 4; ++j) f[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(kr, at + j * 1024, 4 * h * 1024, 0));
+        for (int j = 0; j < 4; ++j) f[j] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(kr, at + j * 1024, from, 0));
     };
     v4f sc[4 * U];
     float m = -INFINITY, low = INFINITY;
@@ -66,7 +76,7 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
                 for (int t = 0; t < 4; ++t) a = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[i & 1][j][t], qf[j][t], a, 0, 0, 0);
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                float x = a[t] * scale;
+                float x = a[t];
                 if (i >= 4 * U - 4) { /* keys that are not there: exp is 0 */
                     const bool there = 16 * (16 * (U - 1) + 4 * wave + (i & 3)) + 4 * t + g < Tk;
                     low = __builtin_fminf(low, there ? x : INFINITY);
@@ -84,10 +94,10 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
     m = tk_fmaxf(m, __shfl_xor(m, 32, 64));
     if (lane < 16) top[wave][lane] = m;
     __syncthreads();
-    m = tk_fmaxf(tk_fmaxf(top[0][n], top[1][n]), tk_fmaxf(top[2][n], top[3][n]));
+    m = tk_fmaxf(tk_fmaxf(top[0][n], top[1][n]), tk_fmaxf(top[2][n], top[3][n])) * scale;
 
     /* every e of the wave is 2^-100 or more (or none: the keys that are not there) */
-    const bool tame = __all(low - m >= -69.0f);
+    const bool tame = __all(low * scale - m >= -69.0f);
     v4f part[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -96,7 +106,7 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
         for (int u = 0; u < U; ++u) {
 #pragma unroll
             for (int t = 0; t < 4; ++t) {
-                const float e = tk_expf_below(sc[4 * u + i][t] - m);
+                const float e = tk_expf_below(tk_fmaf(sc[4 * u + i][t], scale, -m));
                 sc[4 * u + i][t] = e;
                 s[t] = s[t] + e;
             }
@@ -116,7 +126,7 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
     if (lane < 16) sum[wave][lane] = quarter;
     __syncthreads();
     const float tot = ((sum[0][n] + sum[1][n]) + sum[2][n]) + sum[3][n];
-    const float inv = tk_divf(1.0f, tot);
+    const float inv = tk_divf(1.0f, tot), rest = inv * tk_fmaf(-tot, inv, 1.0f);
 
     auto put = [&](int u) { /* the wave's four tiles of 256 keys */
 #pragma unroll
@@ -126,8 +136,7 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     const float e = sc[4 * u + i][t];
-                    float x = e * inv;
-                    x = tk_fmaf(tk_fmaf(-tot, x, e), inv, x);
+                    const float x = tk_fmaf(e, inv, e * rest);
                     p[t] = tk_fmaf(tk_fmaf(-tot, x, e), inv, x);
                 }
             } else {
@@ -185,12 +194,12 @@ __global__ __launch_bounds__(256, U > 4 ? 3 : 4) void k_attention_images(const f
     }
 }
 
-bool tk_launch_attention_images(const float* q_img, const float* k_img, const float* v, float* out_img, int B, int nh, int Tq, int Tk, int d, float scale, hipStream_t s) {
+bool tk_launch_attention_images(const float* q_img, const float* k_img, const float* v, float* out_img, int B, int nh, int Tq, int Tk, int d, hipStream_t s) {
     if (B < 1 || !tk_attention_images_fits(Tq, Tk, d, nh)) return false;
     const int tiles = (Tq + 15) / 16;
     const int64_t total = (int64_t)B * nh * tiles, per = (total + 7) / 8;
     if (per * 8 > 0x7fffffff) return false;
-#define TK_AIM(U) hipLaunchKernelGGL((k_attention_images<U>), dim3((unsigned)(per * 8)), dim3(256), 0, s, q_img, k_img, v, out_img, nh, Tq, Tk, d, tiles, (int)total, (int)per, scale)
+#define TK_AIM(U) hipLaunchKernelGGL((k_attention_images<U>), dim3((unsigned)(per * 8)), dim3(256), 0, s, q_img, k_img, v, out_img, nh, Tq, Tk, d, tiles, (int)total, (int)per)
     switch ((Tk + 255) / 256) {
         case 1: TK_AIM(1); break;
         case 2: TK_AIM(2); break;
