@@ -175,7 +175,7 @@ struct CpuAudioOps {
             for (int i = 0; i < D; ++i) y[(int64_t)r * D + i] = ((xr[i] - mean) * rstd) * w[i] + b[i];
         }
     }
-    bool attend1(const float*, const float*, const float*, float*, int, int, int64_t, int64_t, int, int, float*, int) { return false; }
+    bool attend1(const float*, const float*, const float*, float*, int, int, int64_t, int64_t, int, int, int, float*, int) { return false; }
     bool takes_images(const float*, const float*, const float*, int, int, int) { return false; }
     void attend_images(const float*, const float*, const float*, float*, int, int, int, int) {}
     bool attend_fused(const float*, const float*, const float*, float*, int, int, int, int64_t, int64_t, int, int) { return false; }

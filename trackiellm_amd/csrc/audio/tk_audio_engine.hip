@@ -110,14 +110,14 @@ __device__ __forceinline__ void at1_dma(const float* src, uint8_t* lds) {
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src, (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
 }
 /* the score of key 64 blk + lane (of the last key where there is none); q [hd] in LDS, hd * 256 bytes of ring per wave or 16 KiB, whichever is less */
-__device__ __forceinline__ float at1_score(const float* kp, int blk, int Tk, int d, int hd, float scale, const float* qs, uint8_t* ring, int lane) {
+__device__ __forceinline__ float at1_score(const float* kp, int blk, int Tk, int64_t kv_row, int hd, float scale, const float* qs, uint8_t* ring, int lane) {
     const int unit = (lane & 3) ^ ((lane >> 4) & 3), nsl = hd >> 4;
     const float* src[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         int row = blk * 64 + p * 16 + (lane >> 2);
         row = row < Tk ? row : Tk - 1;
-        src[p] = kp + (int64_t)row * d + unit * 4;
+        src[p] = kp + row * kv_row + unit * 4;
     }
     float a = 0.0f;
     for (int s0 = 0; s0 < nsl; s0 += 4) {
@@ -142,7 +142,7 @@ __device__ __forceinline__ float at1_score(const float* kp, int blk, int Tk, int
 }
 
 /* scores [rows][heads][pitch] of a long context: grid (64-key blocks / 4, heads, rows), a block of keys per wave; row i `group` + b is a row of sequence b */
-__global__ __launch_bounds__(256) void k_attend1_scores(const float* q, const float* k, float* scores, int Tk, int pitch, int64_t q_bstride, int64_t kv_bstride, int d, int hd,
+__global__ __launch_bounds__(256) void k_attend1_scores(const float* q, const float* k, float* scores, int Tk, int pitch, int64_t q_bstride, int64_t kv_bstride, int64_t kv_row, int hd,
                                                         int group, float scale) {
     extern __shared__ __attribute__((aligned(16))) uint8_t att1_lds[];
     const int h = blockIdx.y, row = blockIdx.z, b = (int)gridDim.z > group ? (int)((unsigned)row % (unsigned)group) : row, lane = threadIdx.x & 63;
@@ -152,7 +152,7 @@ __global__ __launch_bounds__(256) void k_attend1_scores(const float* q, const fl
     __syncthreads();
     const int blk = blockIdx.x * 4 + wave;
     if (blk * 64 >= Tk) return;
-    const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, blk, Tk, d, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
+    const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, blk, Tk, kv_row, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
     if (blk * 64 + lane < Tk) scores[((int64_t)row * gridDim.y + h) * pitch + blk * 64 + lane] = a;
 }
 
@@ -166,7 +166,7 @@ __device__ __forceinline__ int at1_place(int k) { return (k & ~15) | (k & 3) << 
 enum { AT1_SELF, AT1_HELD, AT1_LONG };
 template <int FORM>
 __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, const float* k, const float* v, const float* scores, int pitch, float* out, int Tk,
-                                                           int64_t q_bstride, int64_t kv_bstride, int d, int hd, int split, float scale, int sc_at /* bytes */,
+                                                           int64_t q_bstride, int64_t kv_bstride, int64_t kv_row, int d, int hd, int split, float scale, int sc_at /* bytes */,
                                                            int more /* keys that each position of a span sees beyond the one before */,
                                                            float* img /* optional: out also as the tiled GEMM's operand image [rows][K = d] */) {
     extern __shared__ __attribute__((aligned(16))) uint8_t att1_lds[];
@@ -204,7 +204,7 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
             for (int t = 0; t < 4; ++t) {
                 int row = (kb0 + (kq >> 2)) * 16 + 4 * t + (kq & 3);
                 row = row < Tk ? row : Tk - 1;
-                vv[i][t] = *(const at1_f32x4*)(vp + (int64_t)row * d + 4 * x);
+                vv[i][t] = *(const at1_f32x4*)(vp + row * kv_row + 4 * x);
             }
         }
     };
@@ -230,7 +230,7 @@ __global__ __launch_bounds__(64 * TK_AT1_NW) void k_attend1(const float* q, cons
         for (int i = t0; i < hd; i += 64 * TK_AT1_NW) qs[i] = qp[i];
         __syncthreads();
         if (wave * 64 < Tk) {
-            const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, wave, Tk, d, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
+            const float a = at1_score(k + (int64_t)b * kv_bstride + (int64_t)h * hd, wave, Tk, kv_row, hd, scale, qs, att1_lds + wave * TK_AT1_RING, lane);
             if (t0 < Tk) sc[t0] = a;
         }
         __syncthreads();
@@ -351,7 +351,7 @@ static bool at1_prepare_device() {
 }
 /* n positions of B sequences, rows position by position; the first sees Tk keys, each next one `more` further ones (0, or 1 with at most TK_AT1_SELF keys for the last).
  * scores: scratch [B n][nh][pitch] */
-static bool at1_launch(const float* q, const float* k, const float* v, float* scores, int pitch, float* out, int B, int n, int Tk, int more, int64_t q_bstride, int64_t kv_bstride,
+static bool at1_launch(const float* q, const float* k, const float* v, float* scores, int pitch, float* out, int B, int n, int Tk, int more, int64_t q_bstride, int64_t kv_bstride, int64_t kv_row,
                        int d, int nh, float* img, hipStream_t s) {
     const int hd = d / nh, most = Tk + (n - 1) * more;
     if (n < 1 || (more != 0 && (more != 1 || most > TK_AT1_SELF))) return false;
@@ -361,11 +361,11 @@ static bool at1_launch(const float* q, const float* k, const float* v, float* sc
     const dim3 grid(nh * split, B, n), block(64 * TK_AT1_NW);
     const int sc_at = at1_buffer(most, hd / split);
     const size_t lds = (size_t)sc_at + (size_t)(((most + 15) & ~15) + hd + 8) * 4; /* <= 128 KiB + 3 KiB, 96 KiB + 10 KiB, 96 KiB + 50 KiB */
-#define TK_AT1(FORM) hipLaunchKernelGGL((k_attend1<FORM>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, d, hd, split, scale, sc_at, more, img)
+#define TK_AT1(FORM) hipLaunchKernelGGL((k_attend1<FORM>), grid, block, lds, s, q, k, v, scores, pitch, out, Tk, q_bstride, kv_bstride, kv_row, d, hd, split, scale, sc_at, more, img)
     if (most <= TK_AT1_SELF) {
         TK_AT1(AT1_SELF);
     } else {
-        hipLaunchKernelGGL(k_attend1_scores, dim3(((Tk + 63) / 64 + 3) / 4, nh, B * n), dim3(256), 4 * TK_AT1_RING + (size_t)hd * 4, s, q, k, scores, Tk, pitch, q_bstride, kv_bstride, d, hd, B, scale);
+        hipLaunchKernelGGL(k_attend1_scores, dim3(((Tk + 63) / 64 + 3) / 4, nh, B * n), dim3(256), 4 * TK_AT1_RING + (size_t)hd * 4, s, q, k, scores, Tk, pitch, q_bstride, kv_bstride, kv_row, hd, B, scale);
         if (Tk <= TK_AT1_HELD) TK_AT1(AT1_HELD); else TK_AT1(AT1_LONG);
 #undef TK_AT1
     }
@@ -492,8 +492,7 @@ struct TkAudioGpuOps {
         }
         /* does the output overlap the packed matrix (an in-place layer)?  Then the image is stale once the launch has run */
         const float* c0 = g.C;
-        const int c_rows = g.c_group > 0 && g.c_group < g.M ? g.c_group : g.M;
-        const float* c1 = g.C + (size_t)(c_rows - 1) * g.ldc + (g.c_group > 0 ? (size_t)((g.M - 1) / g.c_group) * (size_t)g.c_gstride : 0) + g.N;
+        const float* c1 = g.C + (size_t)(g.M - 1) * g.ldc + g.N;
         const float* a0 = g.A;
         const float* a1 = g.A + (size_t)(g.M - 1) * g.lda + g.K;
         const bool in_place = c0 < a1 && a0 < c1;
@@ -510,12 +509,10 @@ struct TkAudioGpuOps {
             const int i = pend.n++;
             t.tiles[i] = a->model->wt[(size_t)idx]; t.row_tiles[i] = g.N / 16;
             t.seg_out[i] = g.C; t.seg_ldc[i] = g.ldc; t.seg_bias[i] = g.bias; t.seg_n[i] = g.N; t.seg_img[i] = g.c_image;
-            t.seg_group[i] = g.c_group; t.seg_gstride[i] = g.c_gstride;
             if (pend.n == 3) flush();
             return; /* none of these layers writes into its own input: `plain` excludes in-place layers */
         }
         flush();
-        if (g.c_group) a->launch_error = "rows in groups need a plain layer"; /* not reached: keys and values are written into caches, by layers without a residual */
         TkTiledGemm t{};
         t.tiles[0] = a->model->wt[(size_t)idx]; t.row_tiles[0] = (g.N + 15) / 16; t.nseg = 1; t.wbytes = 4;
         t.K = g.K; t.ks = 1; t.ldc = g.ldc; t.n_valid = g.N; t.nrows = g.M; t.slab_rows = 0;
@@ -559,12 +556,12 @@ struct TkAudioGpuOps {
         pk.A = y; pk.M = rows; pk.K = D; pk.lda = D; pk.img = nullptr; pk.mark = a->arena_used; pk.live = true;
     }
     void softmax_rows(float* x, int rows, int cols, int ld) { drop_image(); tk_launch_softmax_rows(x, rows, cols, ld, s); }
-    bool attend1(const float* q, const float* k, const float* v, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int d, int nh, float* scores, int pitch) {
+    bool attend1(const float* q, const float* k, const float* v, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int kv_row, int d, int nh, float* scores, int pitch) {
         drop_image();
         const int hd = d / nh;
         if (hd > 256 || (hd & 15) || (d & 3) || Tk < 1 || Tk > TK_AT1_MAX_KEYS) return false; /* the three-launch form takes what does not fit */
         float* img = (short_pass(B) && d % 128 == 0 && q_bstride == d) ? image_for(out, B, d, d) : nullptr; /* the output projection's input, packed on the way out */
-        return at1_launch(q, k, v, scores, pitch, out, B, 1, Tk, 0, q_bstride, kv_bstride, d, nh, img, s);
+        return at1_launch(q, k, v, scores, pitch, out, B, 1, Tk, 0, q_bstride, kv_bstride, kv_row, d, nh, img, s);
     }
     /* positions of a prompt that one pass takes: as many as make TK_ASR_SPAN_ROWS rows.  0, for one by one as they are decoded, where a layer's widths are not those of the
      * kernels that know of several, or where the span's keys need scores from a launch of their own */
@@ -573,10 +570,10 @@ struct TkAudioGpuOps {
         if (dt % 128 || hd > 256 || (hd & 15) || h.n_text_ctx > TK_AT1_SELF || h.n_audio_ctx > TK_AT1_MAX_KEYS) return 0;
         return B < TK_ASR_SPAN_ROWS ? TK_ASR_SPAN_ROWS / B : 1;
     }
-    void attend_span(const float* q, const float* k, const float* v, float* out, int B, int n, int Tk, bool causal, int64_t q_bstride, int64_t kv_bstride, int d, int nh, float* scores, int pitch) {
+    void attend_span(const float* q, const float* k, const float* v, float* out, int B, int n, int Tk, bool causal, int64_t q_bstride, int64_t kv_bstride, int kv_row, int d, int nh, float* scores, int pitch) {
         drop_image();
         float* img = image_for(out, B * n, d, d);
-        if (!at1_launch(q, k, v, scores, pitch, out, B, n, Tk, causal ? 1 : 0, q_bstride, kv_bstride, d, nh, img, s)) a->launch_error = "decoder attention launch refused";
+        if (!at1_launch(q, k, v, scores, pitch, out, B, n, Tk, causal ? 1 : 0, q_bstride, kv_bstride, kv_row, d, nh, img, s)) a->launch_error = "decoder attention launch refused";
     }
     /* an encoder layer's attention on operand images: 16 rows of a head in one workgroup, no score matrix.  All contexts it has registers for take it (three launches
      * and their score matrix else): at 1500 positions and six heads 97 -> 56 us a layer for one clip, 2106 -> 1194 us for 32 */
@@ -656,10 +653,10 @@ struct TkAudioSizeOps {
     void im2col1d(const float*, int, int, int, int, int, int, int, float*) {}
     void layernorm(const float*, int rows, int D, const float*, const float*, float*) { image(rows, D); }
     void softmax_rows(float*, int, int, int) {}
-    bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int d, int, float*, int) { image(B, d); return true; }
+    bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int, int d, int, float*, int) { image(B, d); return true; }
     bool takes_images(const float*, const float*, const float*, int, int, int) { return false; }
     void attend_images(const float*, const float*, const float*, float*, int, int, int, int) {}
-    void attend_span(const float*, const float*, const float*, float*, int B, int n, int, bool, int64_t, int64_t, int d, int, float*, int) { image(B * n, d); }
+    void attend_span(const float*, const float*, const float*, float*, int B, int n, int, bool, int64_t, int64_t, int, int d, int, float*, int) { image(B * n, d); }
     bool attend_fused(const float*, const float*, const float*, float*, int, int, int, int64_t, int64_t, int, int) { return false; } /* sized for the exact form */
     void add_rows(float*, const float*, int, int, int) {}
     void embed_rows(const float*, const float*, const int32_t*, const int32_t*, int, int, float*) {}

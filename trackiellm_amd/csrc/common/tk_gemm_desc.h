@@ -28,10 +28,6 @@ struct TkGemm {
     int c_feeds_linear;
     /* C [(M + 15) / 16 * 16][N] takes the matrix as an operand image (csrc/nn/tk_gemm_tiled.h) instead of rows: only for a backend that offered attention on images */
     int c_image;
-    /* c_group > 0: row r of C lies at (r % c_group) ldc + (r / c_group) c_gstride (several positions of several sequences into their caches): only for a backend that
-     * offered passes of several positions */
-    int c_group;
-    int64_t c_gstride;
     /* implicit im2col (im_C > 0): A is a convolution's NHWC input [B][im_H][im_W] pixels of pitch im_ldx; GEMM row m = (b, oy, ox) over
      * im_Ho x im_Wo outputs and column k = (ky im_kw + kx) im_C + c address it directly (zero outside the image), K = kh kw im_C.
      * Same values in the same order as the explicit column matrix; lda, batch and b_kn are unused */

@@ -207,15 +207,15 @@ struct TkWhisperGraph {
     /* row pitch of the scores scratch: whole 128-byte lines per row (1500 keys -> 1504 floats would do for 16-byte groups; 1536 keeps every
      * row, and every 128-column tile of it, on cache-line boundaries: Q.K^T's stores and the row kernels' 16-byte groups never straddle) */
     static int score_pitch(int Tk) { return (Tk + 31) & ~31; }
-    /* attention over `Tk` keys for `Tq` queries per batch element; q/k/v/out row pitch = d; scores scratch [B*nh][Tq][score_pitch(Tk)] */
+    /* attention over `Tk` keys for `Tq` queries per batch element; q/out row pitch = d, k/v row pitch kv_row; scores scratch [B*nh][Tq][score_pitch(Tk)] */
     void attention(Ops& o, const float* q, const float* k, const float* v, float* out, int B, int Tq, int Tk, int64_t q_bstride, int64_t kv_bstride,
-                   int d, int nh, float* scores) const {
+                   int kv_row, int d, int nh, float* scores) const {
         const int hd = d / nh;
-        if (Tq == 1 && o.attend1(q, k, v, out, B, Tk, q_bstride, kv_bstride, d, nh, scores, score_pitch(Tk))) return; /* decoder steps: same arithmetic */
-        if (Tq > 1 && o.attend_fused(q, k, v, out, B, Tq, Tk, q_bstride, kv_bstride, d, nh)) return; /* opt-in fast path only */
+        if (Tq == 1 && o.attend1(q, k, v, out, B, Tk, q_bstride, kv_bstride, kv_row, d, nh, scores, score_pitch(Tk))) return; /* decoder steps: same arithmetic */
+        if (Tq > 1 && kv_row == d && o.attend_fused(q, k, v, out, B, Tq, Tk, q_bstride, kv_bstride, d, nh)) return; /* opt-in fast path only */
         const int Tp = score_pitch(Tk);
         TkGemm s{};
-        s.A = q; s.B = k; s.C = scores; s.M = Tq; s.N = Tk; s.K = hd; s.lda = d; s.ldb = d; s.ldc = Tp; s.b_kn = 0; s.act = 0;
+        s.A = q; s.B = k; s.C = scores; s.M = Tq; s.N = Tk; s.K = hd; s.lda = d; s.ldb = kv_row; s.ldc = Tp; s.b_kn = 0; s.act = 0;
         s.alpha = tk_divf(1.0f, tk_sqrtf((float)hd));
         s.batch = B * nh; s.batch_inner = nh;
         s.sA = hd; s.sB = hd; s.sC = (int64_t)Tq * Tp;
@@ -223,7 +223,7 @@ struct TkWhisperGraph {
         o.gemm(s);
         o.softmax_rows(scores, B * nh * Tq, Tk, Tp);
         TkGemm p{};
-        p.A = scores; p.B = v; p.C = out; p.M = Tq; p.N = hd; p.K = Tk; p.lda = Tp; p.ldb = d; p.ldc = d; p.b_kn = 1; p.act = 0; p.alpha = 1.0f;
+        p.A = scores; p.B = v; p.C = out; p.M = Tq; p.N = hd; p.K = Tk; p.lda = Tp; p.ldb = kv_row; p.ldc = d; p.b_kn = 1; p.act = 0; p.alpha = 1.0f;
         p.batch = B * nh; p.batch_inner = nh;
         p.sA = (int64_t)Tq * Tp; p.sB = hd; p.sC = hd;
         p.sA2 = (int64_t)nh * Tq * Tp; p.sB2 = kv_bstride; p.sC2 = q_bstride;
@@ -259,7 +259,7 @@ struct TkWhisperGraph {
             { TkGemm gk = lin(hb, R, d, d, W[L.k_w], nullptr, d, k, d); gk.c_image = images; o.gemm(gk); }
             o.gemm(lin(hb, R, d, d, W[L.v_w], W[L.v_b], d, v, d));
             if (images) o.attend_images(q, k, v, at, B, Tc, d, nh);
-            else attention(o, q, k, v, at, B, Tc, Tc, (int64_t)Tc * d, (int64_t)Tc * d, d, nh, sc);
+            else attention(o, q, k, v, at, B, Tc, Tc, (int64_t)Tc * d, (int64_t)Tc * d, d, d, nh, sc);
             o.gemm(lin(at, R, d, d, W[L.o_w], W[L.o_b], d, x, d, 0, x, d));
             o.layernorm(x, R, d, W[L.ln2_w], W[L.ln2_b], hb);
             { TkGemm g1 = lin(hb, R, d, d, W[L.fc1_w], W[L.fc1_b], 4 * d, ff, 4 * d, TK_ACT_GELU); g1.c_feeds_linear = 1; o.gemm(g1); }
@@ -273,7 +273,7 @@ struct TkWhisperGraph {
     struct DecState {
         int B = 0;
         std::vector<float*> xk, xv; /* per layer [B][ctx][dt] */
-        std::vector<float*> sk, sv; /* per layer self caches [B][n_text_ctx][dt] */
+        std::vector<float*> sk, sv; /* per layer self caches [n_text_ctx][B][dt]: a pass's rows, position by position, lie in one piece */
         float *x, *hb, *q, *k, *v, *at, *ff, *sc, *logits;
         int32_t *tok, *pos, *next;
     };
@@ -312,7 +312,7 @@ struct TkWhisperGraph {
 
 private:
     template <bool SPAN> void pass(Ops& o, DecState& s, int p, int n, bool sampled) const {
-        const int B = s.B, Tc = h.n_audio_ctx, dt = h.n_text_state, nh = h.n_text_head, ctx = h.n_text_ctx;
+        const int B = s.B, Tc = h.n_audio_ctx, dt = h.n_text_state, nh = h.n_text_head;
         int R = B * n; /* rows */
         float *x = s.x, *q = s.q;
         o.embed_rows(W[m.tok_emb], W[m.dec_pos], s.tok, s.pos, R, dt, x);
@@ -321,24 +321,21 @@ private:
             const bool last = SPAN && l == h.n_text_layer - 1;
             o.layernorm(x, R, dt, W[L.ln1_w], W[L.ln1_b], s.hb);
             if (sampled || !last) o.gemm(lin(s.hb, R, dt, dt, W[L.q_w], W[L.q_b], dt, q, dt));
-            /* k, v of these positions go straight into the caches (rows p .. of every sequence) */
-            TkGemm gk = lin(s.hb, R, dt, dt, W[L.k_w], nullptr, dt, s.sk[l] + (size_t)p * dt, ctx * dt);
-            TkGemm gv = lin(s.hb, R, dt, dt, W[L.v_w], W[L.v_b], dt, s.sv[l] + (size_t)p * dt, ctx * dt);
-            if (n > 1) { gk.c_group = gv.c_group = B; gk.c_gstride = gv.c_gstride = dt; }
-            o.gemm(gk);
-            o.gemm(gv);
+            /* k, v of these positions go straight into the caches */
+            o.gemm(lin(s.hb, R, dt, dt, W[L.k_w], nullptr, dt, s.sk[l] + (size_t)p * B * dt, dt));
+            o.gemm(lin(s.hb, R, dt, dt, W[L.v_w], W[L.v_b], dt, s.sv[l] + (size_t)p * B * dt, dt));
             if (last) { /* behind its keys and values: the sampled rows */
                 if (!sampled) return;
                 x += (size_t)(n - 1) * B * dt; q += (size_t)(n - 1) * B * dt;
                 p += n - 1; n = 1; R = B;
             }
-            if constexpr (SPAN) o.attend_span(q, s.sk[l], s.sv[l], s.at, B, n, p + 1, true, dt, (int64_t)ctx * dt, dt, nh, s.sc, score_pitch(p + n));
-            else attention(o, q, s.sk[l], s.sv[l], s.at, B, 1, p + 1, dt, (int64_t)ctx * dt, dt, nh, s.sc);
+            if constexpr (SPAN) o.attend_span(q, s.sk[l], s.sv[l], s.at, B, n, p + 1, true, dt, dt, B * dt, dt, nh, s.sc, score_pitch(p + n));
+            else attention(o, q, s.sk[l], s.sv[l], s.at, B, 1, p + 1, dt, dt, B * dt, dt, nh, s.sc);
             o.gemm(lin(s.at, R, dt, dt, W[L.o_w], W[L.o_b], dt, x, dt, 0, x, dt));
             o.layernorm(x, R, dt, W[L.lnx_w], W[L.lnx_b], s.hb);
             o.gemm(lin(s.hb, R, dt, dt, W[L.xq_w], W[L.xq_b], dt, q, dt));
-            if constexpr (SPAN) o.attend_span(q, s.xk[l], s.xv[l], s.at, B, n, Tc, false, dt, (int64_t)Tc * dt, dt, nh, s.sc, score_pitch(Tc));
-            else attention(o, q, s.xk[l], s.xv[l], s.at, B, 1, Tc, dt, (int64_t)Tc * dt, dt, nh, s.sc);
+            if constexpr (SPAN) o.attend_span(q, s.xk[l], s.xv[l], s.at, B, n, Tc, false, dt, (int64_t)Tc * dt, dt, dt, nh, s.sc, score_pitch(Tc));
+            else attention(o, q, s.xk[l], s.xv[l], s.at, B, 1, Tc, dt, (int64_t)Tc * dt, dt, dt, nh, s.sc);
             o.gemm(lin(s.at, R, dt, dt, W[L.xo_w], W[L.xo_b], dt, x, dt, 0, x, dt));
             o.layernorm(x, R, dt, W[L.ln2_w], W[L.ln2_b], s.hb);
             { TkGemm g1 = lin(s.hb, R, dt, dt, W[L.fc1_w], W[L.fc1_b], 4 * dt, s.ff, 4 * dt, TK_ACT_GELU); g1.c_feeds_linear = 1; o.gemm(g1); }

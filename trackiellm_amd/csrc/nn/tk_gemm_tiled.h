@@ -55,8 +55,6 @@ struct TkTiledGemm {
     const float* seg_bias[3];
     int seg_n[3];
     int seg_img[3];          /* the segment's destination is the operand image of its output (k = its column), not rows */
-    int seg_group[3];        /* > 0: row r at (r % seg_group) seg_ldc + (r / seg_group) seg_gstride; not with an image, nor beyond TK_TW_MAX_BLOCK_ROWS rows */
-    int64_t seg_gstride[3];
     /* c_img: the output is ALSO written as the operand image of the next linear layer (K = n_valid), so no pack launch follows; out may be null then */
     float* c_img;
     /* ln_x: the activations are the layer norm of its rows ([nrows][K], dense), made by every workgroup for itself (f32 tiles, ks == 1, at most TK_TW_LN_ROWS rows of at

@@ -155,8 +155,6 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
     const float* const end_res = split || per_seg ? nullptr : a.residual;
     const bool end_img = WB == 4 && per_seg && of(a.seg_img), add_bias = end_bias || a.add_zero_bias;
     float* const c_img = split || per_seg ? nullptr : a.c_img;
-    const int group = per_seg ? of(a.seg_group) : 0;
-    const int64_t gstride = per_seg ? of(a.seg_gstride) : 0;
 
     const int ppslot = gps * MT;
     const uint32_t voff = lane * 16;
@@ -311,9 +309,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                 continue;
             }
             if (end_res) v = v + (EARLY ? res[EARLY ? m : 0][r] : end_res[at * a.ldr + n]);
-            size_t to = at * end_ldc;
-            if (group > 0) { const uint32_t i = (uint32_t)at / (uint32_t)group; to = (at - (size_t)i * group) * end_ldc + i * (size_t)gstride; }
-            if (WB == 2 || end_out) end_out[to + n] = v;
+            if (WB == 2 || end_out) end_out[at * end_ldc + n] = v;
             if (c_img) c_img[tile] = v;
         }
 }
@@ -557,8 +553,6 @@ static bool tw_valid(const TkTiledGemm& a) {
     if (a.nseg < 1 || a.nseg > 3 || a.ks < 1 || a.K <= 0 || a.K % (32 * a.ks) || a.nrows <= 0 || (a.wbytes != 2 && a.wbytes != 4) || (a.ks > 1 && a.nrows > a.slab_rows)) return false;
     if ((a.per_seg || a.c_img) && a.ks != 1) return false;
     if (a.per_seg && (a.residual || a.c_img)) return false;
-    for (int i = 0; i < a.nseg; ++i)
-        if (a.seg_group[i] != 0 && (a.seg_group[i] < 0 || !a.per_seg || a.seg_img[i] || a.nrows > TK_TW_MAX_BLOCK_ROWS)) return false;
     if (!a.per_seg && !a.out && (!a.c_img || a.wbytes == 2)) return false;
     if (a.per_seg && a.wbytes == 2 && (a.seg_img[0] || a.seg_img[1] || a.seg_img[2])) return false;
     if (a.ln_x && (a.ks != 1 || a.wbytes != 4 || a.K > TK_TW_LN_MAX || a.nrows > TK_TW_LN_ROWS || a.K % 128)) return false;
