@@ -68,7 +68,7 @@ struct TkTiledGemm {
 /* false (nothing launched): K / ks is not a multiple of the ring granularity (128 k; 64 k from 129 rows per block on) or a field is inconsistent */
 bool tk_launch_gemm_tiled(const TkTiledGemm& g, hipStream_t s);
 /* how a launch is cut: M-tiles and waves (a tile of columns each) of a workgroup, and what follows from them.  mt 0: its own choice */
-struct TkTiledPlan { int mt, waves, groups, ny, pf, rk, slot_bytes; bool one; size_t lds; int wide = 0; /* k_gemm_wide's form */ };
+struct TkTiledPlan { int mt, waves, groups, ny, pf, rk, slot_bytes; bool one; size_t lds; bool reg = false; /* operands of the rows in registers, without LDS */ int wide = 0; /* k_gemm_wide's form */ };
 bool tk_gemm_tiled_plan(const TkTiledGemm& g, int mt, int waves, TkTiledPlan* plan);
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& g, const TkTiledPlan& plan, hipStream_t s);
 /* row-major f16 / f32 [N][K] (device) -> tiles; N is padded up to a multiple of 16 with zero rows, K must be a multiple of 32 */

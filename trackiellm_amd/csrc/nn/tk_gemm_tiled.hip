@@ -61,7 +61,9 @@ template <int N> __device__ __forceinline__ void tw_act_all(float* v, int act) {
  * behind the staging and lets the first weights of every PF chunks wait for all requests; where the activations of the whole K range fit the LDS
  * (ONE: multiples of 128 k, up to 2048 at one M-tile, 1024 at two) there is no staging in the loop, and four pieces of weights stay in flight, eight
  * where k is a multiple of 256 from 512 on.
- * Cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us and 51872 x 384 24.0 -> 22.0 with four, 384 x 1536 13.9 -> 10.2 with eight; at 32 rows
+ * A wave by itself in its workgroup (REG: f32, one M-tile; the launcher's rule says when) shares no activations: it fetches its operands as it does its weights, straight into
+ * registers, and its chain starts with the first of both instead of behind a whole image in LDS and a barrier.
+ * In LDS, cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us and 51872 x 384 24.0 -> 22.0 with four, 384 x 1536 13.9 -> 10.2 with eight; at 32 rows
  * 8.6 -> 7.9, 30.0 -> 27.0 with four, 20.8 -> 18.9 (ring).  Twelve pieces: 384 x 384 at 1 row 5.6 (a wave's requests queue in front of the activations
  * of the others). */
 /*
@@ -117,7 +119,7 @@ __device__ __forceinline__ void tw_layernorm(const TkTiledGemm& a, int row0, int
 }
 
 template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */,
-          bool LN = false /* the activations are made here (MT = 1, ONE) */>
+          bool LN = false /* the activations are made here (MT = 1, ONE) */, bool REG = false /* and each wave fetches its own into registers, like its weights (MT = 1, ONE) */>
 __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, int total_row_tiles, int rk /* k per ring slot */, int slot_bytes /* ring slot pitch */) {
     constexpr int LPC = WB == 4 ? 2 : 1; /* 16-byte requests per piece and lane */
     constexpr int PIECE = 512 * WB;      /* bytes of one (row tile, 32 k) piece */
@@ -196,7 +198,21 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                 }
         }
     };
-    if (LN) {
+    /* REG: operands of chunk c, two 16-k groups; rows that are not there: the last one again */
+    v4f aq[REG ? PF : 1][2];
+    const int rows_tile = rows_here < TK_TW_ROWS_PER_TILE ? rows_here : TK_TW_ROWS_PER_TILE, arow = (lane & 15) < rows_tile ? lane & 15 : rows_tile - 1;
+    const float* const abase = a_img + (size_t)k0 * 16 + ((lane & 48) + arow) * 4;
+    auto aload = [&](int c, v4f* dst) {
+        const v4f* p = (const v4f*)(abase + (size_t)(c < nchunk ? c : nchunk - 1) * 512);
+        dst[0] = p[0];
+        dst[1] = p[64];
+    };
+    if (REG) {
+        if (!active) return;
+#pragma unroll
+        for (int i = 0; i < PF; ++i) { aload(i, aq[REG ? i : 0]); wload(i, wq[i]); }
+        load_end();
+    } else if (LN) {
         if (active) {
 #pragma unroll
             for (int i = 0; i < PF; ++i) wload(i, wq[i]);
@@ -208,7 +224,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
     } else {
         stage(0, 0);
     }
-    if (!LN && !active) { /* no tile of its own: its share of the staging */
+    if (!LN && !REG && !active) { /* no tile of its own: its share of the staging */
         for (int s = 0; s < nslots; ++s) {
             tw_wait_vmcnt(0);
             __syncthreads();
@@ -216,7 +232,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         }
         return;
     }
-    if (!LN) {
+    if (!LN && !REG) {
         load_end();
 #pragma unroll
         for (int i = 0; i < PF; ++i) wload(i, wq[i]);
@@ -226,7 +242,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
     for (int s = 0; s < (ONE ? 1 : nslots); ++s) {
         /* slot s has landed once all but the PF * LPC youngest requests are done: those are weight requests issued after its DMA
          * (cps >= PF chunks follow every slot's DMA, the PF initial ones the first) */
-        if (!LN) {
+        if (!LN && !REG) {
             tw_wait_vmcnt(PF * LPC);
             __syncthreads();
         }
@@ -242,7 +258,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
 #pragma unroll
                 for (int h = 0; h < 2; ++h) o.a[h][i] = *(const v4f*)(ap + (h * MT + i) * 1024);
         };
-        read(ops[0], 0, 0);
+        if (!REG) read(ops[0], 0, 0);
 #pragma unroll 1
         for (int cc = 0; cc < cps; cc += PF) {
 #pragma unroll
@@ -265,8 +281,14 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                      * chains alternate (a chain step's 40-cycle dependent latency hides behind the other chain's MFMA) */
                     const int step = u * PAIRS + p, m = p * PAIR;
                     Ops& o = ops[step & 1];
-                    if (p + 1 < PAIRS) read(ops[(step + 1) & 1], cc + u, m + PAIR);
-                    else read(ops[(step + 1) & 1], cc + u + 1, 0);
+                    if (REG) {
+                        o.a[0][0] = aq[REG ? u : 0][0];
+                        o.a[1][0] = aq[REG ? u : 0][1];
+                    } else if (p + 1 < PAIRS) {
+                        read(ops[(step + 1) & 1], cc + u, m + PAIR);
+                    } else {
+                        read(ops[(step + 1) & 1], cc + u + 1, 0);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                     {
                         v4f d[PAIR];
@@ -283,6 +305,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                     }
                 }
                 if (WB == 4 && ONE) wload(c + PF, wq[u]);
+                if (REG) aload(c + PF, aq[REG ? u : 0]);
             }
         }
     }
@@ -578,7 +601,8 @@ static bool tw_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
      * Many row blocks of 128 rows (of products that are none of k_gemm_wide's): 32 KiB slots and two weight pieces in flight instead, so
      * that TWO workgroups share a CU and one's ring fill and epilogue run under the other's MFMAs. */
     const bool twin = p->ny > 1 && (mt == 8 || mt == 6) && Kr % 64 == 0;
-    p->one = mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES;
+    p->reg = mt == 1 && waves == 1 && Kr % 128 == 0 && a.wbytes == 4 && !a.ln_x; /* a wave by itself shares nothing */
+    p->one = p->reg || (mt <= 2 && Kr % 128 == 0 && (size_t)Kr * mt * 64 <= 2 * TK_TW_SLOT_BYTES);
     /* whole range: eight pieces of weights in flight where they divide it, but not all of it at once: 51872 x 256, f32, 1 and 32 rows 14.9 and 18.9 us with
      * four, 18.2 and 22.6 with eight */
     p->pf = mt == 16 || mt == 6 || twin ? 2 : p->one && Kr % 256 == 0 && Kr > 256 ? 8 : 4;
@@ -588,7 +612,7 @@ static bool tw_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
         if (Kr % c == 0) p->rk = c;
     if (p->rk == 0) return false;
     p->slot_bytes = twin ? slot_kib * 1024 : TK_TW_SLOT_BYTES;
-    p->lds = p->one ? (size_t)Kr * mt * 64 : (size_t)2 * p->slot_bytes;
+    p->lds = p->reg ? 0 : p->one ? (size_t)Kr * mt * 64 : (size_t)2 * p->slot_bytes;
     return true;
 }
 
@@ -598,7 +622,7 @@ static bool tw_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
 static float tw_cost(const TkTiledGemm& a, const TkTiledPlan& p) {
     const int row_tiles = tw_row_tiles(a), Kr = a.K / a.ks;
     const float rounds = (float)p.groups * (float)p.ny * (float)a.ks * (1.0f / 256.0f), up = ceilf(rounds);
-    int side_by_side = (int)(163840 / p.lds) < 16 / p.waves ? (int)(163840 / p.lds) : 16 / p.waves;
+    int side_by_side = (int)(163840 / (p.lds + 1)) < 16 / p.waves ? (int)(163840 / p.lds) : 16 / p.waves;
     if (side_by_side < 1) side_by_side = 1;
     const int per = (p.waves + 3) / 4;
     const float kib = (float)p.lds * (1.0f / 1024.0f), waits = p.one ? 0.0f : (float)(Kr / p.rk) * 1012.0f;
@@ -637,6 +661,13 @@ bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p)
         const int64_t tiles = (int64_t)((a.nrows + 31) / 32) * (tw_row_tiles(a) / 2);
         const bool large = (size_t)tw_row_tiles(a) * 16 * (size_t)a.K * 4 > (4u << 20);
         if (tiles >= 544 && tk_gemm_wide_plan(a, large && tiles >= 3840 ? 2 : 1, p)) return true;
+    }
+    /* Up to five tiles of 16 x 16 for eight SIMDs: a wave each, operands in registers.  LDS (the best of 1, 2, 4, 8 waves) / registers, us, cold weights: 1 row x 384, 1152,
+     * 1536 columns of 384 k 4.9, 5.2, 5.2 / 4.3, 4.4, 4.4, x 384 of 1536 k 11.0 / 9.1, x 1280 of 1280 9.9 / 8.1, x 5120 of 1280 (320 tiles) 10.2 / 9.5; 32 rows 5.7, 5.8, 5.8 / 5.0,
+     * 5.1, 5.2, 11.7 / 9.7, 10.4 / 8.8, 15.1 / 14.6 (640 tiles); beyond, 128 rows x 1536 of 384 (768) 6.4 / 6.7, x 2048 of 512 (1024) 8.1 / 9.7, 48 x 5120 of 1280 (960) 14.9 / 17.8. */
+    if (a.wbytes == 4 && !a.ln_x && a.ks == 1) {
+        const int64_t tiles = (int64_t)((a.nrows + TK_TW_ROWS_PER_TILE - 1) / TK_TW_ROWS_PER_TILE) * tw_row_tiles(a);
+        if (2 * tiles <= 5 * (int64_t)tk_tiled_num_cu() && tw_plan(a, 1, 1, p) && p->reg) return true;
     }
     if (!tw_usual(a, p)) return false;
     /* As many rows as possible behind one reading of the weights is what counts where these are large.  Small matrices (up to 24 MB: they come from the caches) of few
@@ -728,7 +759,10 @@ bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipSt
 #define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
 #define TK_TW_WB(MTV, ONEV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, ONEV, PFV); else TK_TW_LAUNCH(MTV, 4, ONEV, PFV); } while (0)
     switch (p.mt) {
-        case 1: if (p.one) { if (p.pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
+        case 1: if (p.reg) {
+                if (p.pf == 8) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 8, false, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+                else hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 4, false, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+            } else if (p.one) { if (p.pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
         case 2: if (p.one) { if (p.pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
         case 4: TK_TW_WB(4, false, 4); break;
         case 6: TK_TW_WB(6, false, 2); break;
