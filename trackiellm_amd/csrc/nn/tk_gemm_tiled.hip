@@ -69,10 +69,11 @@ template <int N> __device__ __forceinline__ void tw_act_all(float* v, int act) {
 /*
  * Layer norm of the workgroup's rows into the one slot of activations (TkTiledGemm::ln_x): a wave a row, k_layernorm's arithmetic in its order — 256 partial sums over
  * columns p, p + 256, ..., folded within groups of 64 by halves, the four groups left to right — with the four groups side by side in a wave's lanes.  A decoder step of
- * one sequence has 13 norms; as launches of their own they took 2.9 us each, and the 12 products behind them waited for a trip to memory more.
+ * one sequence has 13 norms; as launches of their own they took 2.9 us each, and the 12 products behind them waited for a trip to memory more.  Registers and requests for
+ * no more columns than the form is for: 384 columns in the form for 1024 6.4 us a product of a step and 21.9 one of 51 864 columns, in that for 512 6.1 and 19.5.
  */
+template <int NV /* times 256 columns, at most */>
 __device__ __forceinline__ void tw_layernorm(const TkTiledGemm& a, int row0, int rows, float* image, int wave, int nw, int lane) {
-    constexpr int NV = TK_TW_LN_MAX / 256;
     const int D = a.K;
     auto fold = [&](float (&s)[4]) {
 #pragma unroll
@@ -119,7 +120,7 @@ __device__ __forceinline__ void tw_layernorm(const TkTiledGemm& a, int row0, int
 }
 
 template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */,
-          bool LN = false /* the activations are made here (MT = 1, ONE) */, bool REG = false /* and each wave fetches its own into registers, like its weights (MT = 1, ONE) */>
+          int LN = 0 /* the activations are made here, norms of up to LN times 256 columns (MT = 1, ONE) */, bool REG = false /* and each wave fetches its own into registers, like its weights (MT = 1, ONE) */>
 __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, int total_row_tiles, int rk /* k per ring slot */, int slot_bytes /* ring slot pitch */) {
     constexpr int LPC = WB == 4 ? 2 : 1; /* 16-byte requests per piece and lane */
     constexpr int PIECE = 512 * WB;      /* bytes of one (row tile, 32 k) piece */
@@ -218,7 +219,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
             for (int i = 0; i < PF; ++i) wload(i, wq[i]);
             load_end();
         }
-        tw_layernorm(a, row0, rows_here, (float*)lds, wave, nw, lane);
+        tw_layernorm<LN ? LN : 1>(a, row0, rows_here, (float*)lds, wave, nw, lane);
         __syncthreads();
         if (!active) return;
     } else {
@@ -565,8 +566,10 @@ bool tk_gemm_tiled_prepare_device() {
     TK_TW_OPT(1, true, 4); TK_TW_OPT(1, true, 8); TK_TW_OPT(2, true, 4); TK_TW_OPT(2, true, 8);
     TK_TW_OPT(1, false, 4); TK_TW_OPT(2, false, 4); TK_TW_OPT(4, false, 4); TK_TW_OPT(8, false, 4); TK_TW_OPT(16, false, 2); TK_TW_OPT(8, false, 2); TK_TW_OPT(6, false, 2);
 #undef TK_TW_OPT
-    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 4, true>);
-    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 8, true>);
+    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 4, 2>);
+    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 8, 2>);
+    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 4, 4>);
+    if (e == hipSuccess) e = tw_opt_in(k_gemm_tiled<1, 4, true, 8, 4>);
     if (e != hipSuccess) return false;
     g_tw_opted[dev].store(true, std::memory_order_release);
     return true;
@@ -752,16 +755,18 @@ bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipSt
     const int row_tiles = tw_row_tiles(a);
     if (a.ln_x) {
         if (p.mt != 1 || !p.one) return false;
-        if (p.pf == 8) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 8, true>), dim3(p.groups, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
-        else hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 4, true>), dim3(p.groups, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+#define TK_TW_LN(PFV, NV) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, PFV, NV>), dim3(p.groups, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
+        if (a.K <= 512) { if (p.pf == 8) TK_TW_LN(8, 2); else TK_TW_LN(4, 2); }
+        else { if (p.pf == 8) TK_TW_LN(8, 4); else TK_TW_LN(4, 4); }
+#undef TK_TW_LN
         return true;
     }
 #define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
 #define TK_TW_WB(MTV, ONEV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, ONEV, PFV); else TK_TW_LAUNCH(MTV, 4, ONEV, PFV); } while (0)
     switch (p.mt) {
         case 1: if (p.reg) {
-                if (p.pf == 8) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 8, false, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
-                else hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 4, false, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+                if (p.pf == 8) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 8, 0, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
+                else hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 4, 0, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
             } else if (p.one) { if (p.pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
         case 2: if (p.one) { if (p.pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
         case 4: TK_TW_WB(4, false, 4); break;
