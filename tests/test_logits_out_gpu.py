@@ -41,3 +41,26 @@ def test_sessions_in_threads(gpu, model):
     for i, n in enumerate(rows):
         for k in range(3):
             assert np.array_equal(got[i][k].view(np.uint32), passes(gpu, model, n, 8, 7 + k)[0].view(np.uint32))
+
+
+def test_halves_sent_in_any_order(gpu, model):
+    """eight halves of the pinned memory, freed and sent again by whichever thread takes a half's last piece: one behind a later one is still waited for"""
+    rows = 256
+    s = gpu.LlmSession(model, 256, 8)
+    want = passes(gpu, model, rows, 8, 3)[0]
+    stop = threading.Event()
+
+    def busy():  # threads that hold the others up in the middle of a piece
+        a = np.zeros(1 << 22, np.uint8)
+        while not stop.is_set():
+            a[:] = a + 1
+    others = [threading.Thread(target=busy) for _ in range(12)]
+    [t.start() for t in others]
+    try:
+        for _ in range(60):
+            got = passes(gpu, model, rows, 256, 3, s)[0]
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+    finally:
+        stop.set()
+        [t.join() for t in others]
+    s.close()

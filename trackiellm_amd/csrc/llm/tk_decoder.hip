@@ -111,8 +111,10 @@ bool TkDecodeSession::copy_out(void* host, const void* dev, size_t bytes) {
     }
     constexpr size_t HALF = TK_OUT_PIECES / 2;
     const size_t n = (bytes + TK_OUT_PIECE - 1) / TK_OUT_PIECE;
-    std::atomic<size_t> next{0}, sent{0}; /* pieces taken by a thread; pieces on their way */
+    std::atomic<size_t> next{0}; /* pieces taken by a thread */
     std::vector<std::atomic<unsigned>> left((n + HALF - 1) / HALF); /* pieces of each half-ring not yet taken away */
+    std::vector<std::atomic<bool>> on_way(left.size()); /* of each by itself: they are sent in the order in which threads free their places, which is any order */
+    for (auto& w : on_way) w.store(false, std::memory_order_relaxed);
     std::atomic<int> failed{hipSuccess};
     unsigned* const there = (unsigned*)(out_ring_ + TK_OUT_PIECES * TK_OUT_PIECE);
     const unsigned epoch0 = out_epoch_;
@@ -124,16 +126,16 @@ bool TkDecodeSession::copy_out(void* host, const void* dev, size_t bytes) {
                            d_out_done_ + slot, there + slot, epoch0 + (unsigned)g);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) { failed.store(e); return; }
-        sent.store(g * HALF + pieces, std::memory_order_release);
+        on_way[g].store(true, std::memory_order_release);
     };
-    auto arrived = [&](size_t i) { return i < sent.load(std::memory_order_acquire) && __atomic_load_n(there + i % TK_OUT_PIECES, __ATOMIC_ACQUIRE) == epoch0 + (unsigned)(i / HALF); };
+    auto arrived = [&](size_t i) { return on_way[i / HALF].load(std::memory_order_acquire) && __atomic_load_n(there + i % TK_OUT_PIECES, __ATOMIC_ACQUIRE) == epoch0 + (unsigned)(i / HALF); };
     auto wait = [&](size_t i) { /* as the runtime waits: actively, and politely once it takes long; a stream that has ended without the piece has failed */
         const auto t0 = std::chrono::steady_clock::now();
         for (unsigned spin = 1; !arrived(i); ++spin) {
             if (failed.load() != hipSuccess) return false;
             std::this_thread::yield();
             if (spin % 256) continue;
-            if (i < sent.load()) {
+            if (on_way[i / HALF].load()) {
                 const hipError_t e = hipStreamQuery(stream);
                 if (e != hipErrorNotReady && !arrived(i)) { failed.store(e == hipSuccess ? hipErrorUnknown : e); return false; }
             }
