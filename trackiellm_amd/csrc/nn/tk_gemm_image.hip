@@ -63,7 +63,7 @@ __device__ __forceinline__ void store_act(const TkImgGemm& a, int mt, int ct, in
  * of the second has a slab of its own: added in ascending order, they are the sum that one workgroup of all waves makes. */
 template <typename T, int MT, int NT, int WAVES, int PARTS, bool SWIGLU, bool GROUPED>
 __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
-    static_assert(PARTS == 1 || (PARTS == 2 && NT == 1 && !SWIGLU && !GROUPED), "slabs are of plain products");
+    static_assert(PARTS == 1 || (PARTS == 2 && !SWIGLU && !GROUPED), "slabs are of plain products");
     constexpr int U = MT >= 3 ? 2 : 4, STEP = PARTS * WAVES * U, AHEAD = PARTS;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -132,10 +132,12 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
     if (PARTS > 1 && blockIdx.z) {
         a.out += (size_t)(1 + wave) * a.slab_floats;
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            const int64_t row = (int64_t)(m0 + m) * 16 + (lane & 15);
-            if (m < mlive && row < a.nrows) store_f32<T>(a, row, n0 * 16 + 4 * (lane >> 4), acc[0][m]);
-        }
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const int64_t row = (int64_t)(m0 + m) * 16 + (lane & 15);
+                if (m < mlive && row < a.nrows && n0 + n < ntot) store_f32<T>(a, row, (n0 + n) * 16 + 4 * (lane >> 4), acc[n][m]);
+            }
         return;
     }
     /* partial sums of the waves, ascending */
@@ -370,12 +372,14 @@ WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
 
 /* A product of few rows by two workgroups a column tile, in TK_SKINNY_SLABS slabs, where its column tiles leave half of the CUs idle and there is work for every wave:
  * 40 rows x 2048 x 8192 19.7 -> 13.9 us, x 2048 7.2 -> 6.1.  Steps of an eight-layer model 2048 wide with one workgroup / two: 1 row 539 / 529 us, 16 rows 599 / 590, 40 rows
- * 816 / 781, 64 rows 894 / 836; three and four pieces of a wave on their way are no quicker than two.  256 column tiles (4096 wide): 1 row 531 / 546, 40 rows 822 / 838.  The
- * rows do not enter, so that a row's result does not depend on the others of its step. */
+ * 816 / 781, 64 rows 894 / 836; three and four pieces of a wave on their way are no quicker than two.  256 column tiles (4096 wide), one tile a workgroup: 1 row 531 / 546, 40 rows 822 / 838; from 17 rows
+ * on in workgroups of two tiles, which read the rows' activations half as often: the products of a step of a four-layer model 4096 wide at 40 and 60 rows 550 / 532 and 606 / 590 us.
+ * The slabs add up to the bits of one workgroup, so a row's result does not depend on which it was. */
 #define TK_SKINNY_WAVES 8
 #define TK_SKINNY_SLABS (1 + TK_SKINNY_WAVES / 2)
 int skinny_parts(const TkImgGemm& g, bool swiglu, bool grouped) {
-    return !swiglu && !grouped && g.max_slabs >= TK_SKINNY_SLABS && g.N / 16 <= 128 && g.K / tk_img_kt(g.type) >= 64 ? 2 : 1;
+    const int most = g.nrows > 16 && g.K / tk_img_kt(g.type) >= 128 ? 256 : 128;
+    return !swiglu && !grouped && g.max_slabs >= TK_SKINNY_SLABS && g.N / 16 <= most && g.K / tk_img_kt(g.type) >= 64 ? 2 : 1;
 }
 
 template <typename T, bool SWIGLU, bool GROUPED>
@@ -388,15 +392,26 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
         const int parts = skinny_parts(g, SWIGLU, GROUPED);
         if (slabs) *slabs = parts > 1 ? TK_SKINNY_SLABS : 1;
 #define TK_SK(MT, NT, WV, P) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, P, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, gy, P), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
-#define TK_SKM(NT, WV, P) do { if (mtiles <= 1) TK_SK(1, NT, WV, P); else if (mtiles <= 2) TK_SK(2, NT, WV, P); else if (mtiles <= 3) TK_SK(3, NT, WV, P); else TK_SK(4, NT, WV, P); } while (0)
-        if (SWIGLU || ntiles * gy >= 1024) {
+#define TK_SKM2(NT, WV, P) do { if (mtiles <= 2) TK_SK(2, NT, WV, P); else if (mtiles <= 3) TK_SK(3, NT, WV, P); else TK_SK(4, NT, WV, P); } while (0)
+#define TK_SKM(NT, WV, P) do { if (mtiles <= 1) TK_SK(1, NT, WV, P); else TK_SKM2(NT, WV, P); } while (0)
+        /* Column tiles of a workgroup: every workgroup reads its rows' activations again, which from two M-tiles on is more than its weights and comes from the L2s.  So four
+         * where that leaves 384 workgroups and more, two where it leaves 192.  4096 x 28672 (gate and up) at 20, 40, 60 rows with two / four 47.9 / 41.5, 51.2 / 45.6, 60.9 / 48.4
+         * us, x 32000 50.8 / 43.4, 55.5 / 49.7, 68.3 / 53.5 (at 1 row 40.0 / 41.9); x 7440 with one / two at 1, 20, 40, 60 rows 13.6 / 11.9, 17.3 / 14.5, 21.2 / 16.2, 23.7 / 18.9. */
+        if (!GROUPED && mtiles >= 2 && ntiles >= 1536) {
+            TK_SKM2(4, 4, 1);
+        } else if (!GROUPED && !SWIGLU && ntiles >= 384 && ntiles < 1024) {
+            TK_SKM(2, 8, 1);
+        } else if (SWIGLU || ntiles * gy >= 1024) {
             if (ntiles * gy >= 2048) TK_SKM(2, 4, 1); else TK_SKM(2, 8, 1);
         } else if (parts > 1) {
-            if constexpr (!SWIGLU && !GROUPED) TK_SKM(1, TK_SKINNY_WAVES / 2, 2);
+            if constexpr (!SWIGLU && !GROUPED) {
+                if (ntiles > 128) TK_SKM2(2, TK_SKINNY_WAVES / 2, 2); else TK_SKM(1, TK_SKINNY_WAVES / 2, 2);
+            }
         } else {
             TK_SKM((SWIGLU ? 2 : 1), TK_SKINNY_WAVES, 1);
         }
 #undef TK_SKM
+#undef TK_SKM2
 #undef TK_SK
         return nullptr;
     }
