@@ -28,15 +28,11 @@ __device__ __forceinline__ void store_f32(const TkImgGemm& a, int64_t row, int n
             if (n + r >= a.copy0 && n + r < a.copy1) tk_img_put((T*)a.copy_img, row, n + r - a.copy0, a.copy_ktiles, v[r]);
 }
 
-/* 1 / (1 + e^-z): what becomes bf16 next by the hardware's exponential and reciprocal (1 ulp of float32 each), five instructions where expf and a division take some forty, which
- * stood between a block's last product and the next block's first: 1785 x 16384 x 2048 (gate | up) 122 -> 114 us (and 111 with store_act's addresses, below).  Errors against 64 bits of whole models: unchanged */
-template <typename T> __device__ __forceinline__ float act_sigmoid(float z) {
-    return sizeof(T) == 4 ? tk_sigmoid32(z) : __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-1.4426950408889634f * z));
-}
-template <typename T> __device__ __forceinline__ float act_silu(float z) { return sizeof(T) == 4 ? tk_silu32(z) : z * act_sigmoid<T>(z); }
-
 /* gate and up tiles of the same 16 columns -> the gated activation in the next product's operand image: M-tile mt, columns 16 ct .. 16 ct + 15, both the same for all lanes, so that
- * the address is a scalar one and a lane's constant offset (row and column of a lane through tk_img_index are two 64-bit products each) */
+ * the address is a scalar one and a lane's constant offset (row and column of a lane through tk_img_index are two 64-bit products each: 2047 x 28672 x 4096
+ * (gate | up) 429 -> 426 us).
+ * expf and the division, some forty instructions of an element that becomes bf16 next, stand between a block's last product and the next block's first.  The hardware's exponential and
+ * reciprocal would take 21 us off that product, but with the exponent's rounding they are up to |z| units of 2^-24 off. */
 template <typename T>
 __device__ __forceinline__ void store_act(const TkImgGemm& a, int mt, int ct, int lane, tk_v4f gate, tk_v4f up) {
     constexpr int PER = TkImg<T>::KT / 16, EP = TkImg<T>::EP; /* tiles of 16 columns in a k tile */
@@ -47,9 +43,9 @@ __device__ __forceinline__ void store_act(const TkImgGemm& a, int mt, int ct, in
         float y;
         if (a.act_clamped) {
             const float g = fminf(gate[r], a.act_limit), u = fminf(fmaxf(up[r], -a.act_limit), a.act_limit);
-            y = g * act_sigmoid<T>(a.act_slope * g) * (u + a.act_shift);
+            y = g * tk_sigmoid32(a.act_slope * g) * (u + a.act_shift);
         } else {
-            y = act_silu<T>(gate[r]) * up[r];
+            y = tk_silu32(gate[r]) * up[r];
         }
         h[r] = n + r < a.act_valid ? y : 0.0f;
     }
