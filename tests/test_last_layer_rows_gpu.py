@@ -49,3 +49,30 @@ def test_wanted_rows_of_the_last_layer(gpu, name, lengths, dtype):
     assert none is None
     nxt = [x.forward_rows(range(len(ns)), ns, toks[n:], range(len(ns)))[0] for x in (s, t, u)]
     assert U.rel_rms(nxt[1], nxt[0]) < TOL[dtype] and U.rel_rms(nxt[2], nxt[0]) < TOL[dtype]
+
+
+# 32 wide: products over the width are one chain in every kernel, so that the head's sums don't depend on how many rows it takes; those of the last layer's other products do
+NARROW = {
+    "delta": config(32, 96, [layer(attention(4, 2, 64, 64, 32, 70, 2), delta(4, 2, 64, 64, 4), dense(576))] * 2),
+    "deep": config(32, 96, [layer(attention(4, 2, 64, 64, 32, 70, 2), delta(4, 2, 64, 64, 4), dense(4096))]),
+    "odd": config(31, 131, [layer(attention(4, 2, 24, 40, 12, 33, 3), delta(3, 3, 20, 36, 3), dense(1070))] * 2),
+    "experts": config(32, 96, [layer(attention(4, 2, 64, 64, 32, 70, 2), delta(4, 2, 64, 64, 4), moe(448, 8, 2))] * 2),
+    "retention last": kaparax(32, 96, [serial(chunked(4, 2, 64, 64, 32, 48, 4, 15.0), (64, 2.0)), serial(retention(4, 64, 64, 64, [0.9, 0.99, 0.5, 0.8]), (640, 2.0))]),
+}
+
+
+@pytest.mark.parametrize("dtype", sorted(TOL))
+@pytest.mark.parametrize("lengths", ["one", "few", "many", "long"])
+@pytest.mark.parametrize("name", sorted(NARROW))
+def test_a_rows_logits_do_not_depend_on_which_others_are_wanted(gpu, name, lengths, dtype):
+    """bit for bit those of a pass that wants all"""
+    cfg, ns = NARROW[name], LENGTHS[lengths]
+    m = gpu.LlmModel(config=cfg, dtype=dtype, seed=9)
+    n = sum(ns)
+    seq, pos, toks, out = np.repeat(np.arange(len(ns)), ns), np.concatenate([np.arange(k) for k in ns]), tokens_for(cfg, n + len(ns)), wanted(lengths, ns, n)
+    s, t = (gpu.LlmSession(m, len(ns), max(ns) + 8) for _ in range(2))
+    whole, _ = s.forward_rows(seq, pos, toks[:n], range(n))
+    some, _ = t.forward_rows(seq, pos, toks[:n], out)
+    assert np.array_equal(some.view(np.uint32), whole[out].view(np.uint32))
+    nxt = [x.forward_rows(range(len(ns)), ns, toks[n:], range(len(ns)))[0] for x in (s, t)]
+    assert np.array_equal(nxt[0].view(np.uint32), nxt[1].view(np.uint32))

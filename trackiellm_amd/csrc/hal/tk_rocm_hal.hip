@@ -313,7 +313,7 @@ tk_error_code_t tk_mi355x_gemm_image_form(int f32, int rows, int N, int K, int s
     const int to = swiglu ? 32 : 16;
     TkImgGemm g{};
     g.type = f32 ? TK_IMG_F32 : TK_IMG_BF16; g.K = tk_img_pad_k(g.type, K); g.N = (N + to - 1) / to * to; g.n_valid = N; g.nrows = rows; g.swiglu = swiglu != 0; g.max_slabs = max_slabs;
-    if (experts) tk_img_expert_blocks(rows, top, experts, &g);
+    if (experts) tk_img_expert_blocks(rows, rows, top, experts, &g);
     tk_gemm_image_form(g, form);
     return TK_SUCCESS;
 }

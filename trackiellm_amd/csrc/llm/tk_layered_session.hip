@@ -317,15 +317,15 @@ void TkLayeredSession::gemm(const TkImgGemm& g, int* slabs) {
         if (launch_error.empty()) launch_error = e;
 }
 
-void TkLayeredSession::enqueue_moe(const TkLayerSpec& s, const TkLayeredLayer& L, int nrows) {
+void TkLayeredSession::enqueue_moe(const TkLayerSpec& s, const TkLayeredLayer& L, int nrows, int as_rows) {
     const TkMlpSpec& f = s.mlp;
     const int type = m_->type, D = m_->cfg.width, kt = tk_img_kt(type), xkt = tk_img_pad_k(type, D) / kt, fkt = L.down.K / kt;
     TkImgGemm g{};
-    g.type = type; g.w = L.router.img; g.a = img_x_; g.K = L.router.K; g.N = L.router.N; g.nrows = nrows;
+    g.type = type; g.w = L.router.img; g.a = img_x_; g.K = L.router.K; g.N = L.router.N; g.nrows = nrows; g.as_rows = as_rows;
     g.out = router_; g.ldc = L.router.N; g.n_valid = f.experts;
     gemm(g);
     TkImgGemm u{};
-    tk_img_expert_blocks(nrows, f.top, f.experts, &u);
+    tk_img_expert_blocks(nrows, as_rows, f.top, f.experts, &u);
     tk_launch_moe_select(router_, L.router.N, f.experts, f.top, f.groups, f.keep, nrows, u.block_tiles, moe_, stream);
     tk_launch_moe_gather(img_x_, img_gather_, xkt, f.top, nrows, moe_, stream);
     u.type = type; u.w = L.gate_up.img; u.a = img_gather_; u.K = L.gate_up.K; u.N = L.gate_up.N;
@@ -339,7 +339,8 @@ void TkLayeredSession::enqueue_moe(const TkLayerSpec& s, const TkLayeredLayer& L
 }
 
 /* Nobody reads what the last layer makes of a row whose logits are not wanted, so behind its mixers (which leave keys, values and states) only the wanted rows go on, side by
- * side.  Not where they are most of the pass: a launch that takes them out is 4 us. */
+ * side, through products that make the whole pass's sums of them (TkImgGemm::as_rows): a row's logits do not depend on which others are wanted.  Not where they are most of
+ * the pass: a launch that takes them out is 4 us. */
 void TkLayeredSession::choose_last_rows(Pass* p, int n_out) {
     if (streams_ || p->single || n_out > TK_MAX_ROWS || 2 * n_out > p->nrows) return;
     p->n_last = n_out;
@@ -436,27 +437,27 @@ void TkLayeredSession::enqueue_layers(const Pass& p) {
             x = x_last_;
         }
         TkImgGemm o{};
-        o.type = type; o.w = L.out.img; o.a = part ? img_last_ : img_mix_; o.K = L.out.K; o.N = L.out.N; o.nrows = n; o.out = y_; o.ldc = D; o.n_valid = D;
-        /* products whose result goes to a norm may come in slabs, as many as y_ holds */
-        const size_t slab = (size_t)n * D;
-        const int most = slab % 4 == 0 ? (int)std::min<size_t>(8, y_floats_ / slab) : 1;
+        o.type = type; o.w = L.out.img; o.a = part ? img_last_ : img_mix_; o.K = L.out.K; o.N = L.out.N; o.nrows = n; o.as_rows = p.nrows; o.out = y_; o.ldc = D; o.n_valid = D;
+        /* products whose result goes to a norm may come in slabs, as many as y_ holds of a whole pass */
+        const size_t slab = ((size_t)n * D + 3) / 4 * 4, whole = (size_t)p.nrows * D;
+        const int most = whole % 4 == 0 ? (int)std::min<size_t>(8, y_floats_ / whole) : 1;
         int slabs = 1;
         o.max_slabs = most; o.slab_floats = slab;
         gemm(o, &slabs);
         tk_launch_post_norm(type, TkSubOut{y_, D, slabs, slab, L.out_bias, 1.0f, nullptr, nullptr, 0}, L.norm1, spec.mlp.kind == TkMlpSpec::NONE ? after : L.pre2, c.eps, D, n, x, img_x_, xkt, s);
         if (spec.mlp.kind == TkMlpSpec::DENSE) {
             TkImgGemm u{};
-            u.type = type; u.w = L.gate_up.img; u.a = img_x_; u.K = L.gate_up.K; u.N = L.gate_up.N; u.nrows = n;
+            u.type = type; u.w = L.gate_up.img; u.a = img_x_; u.K = L.gate_up.K; u.N = L.gate_up.N; u.nrows = n; u.as_rows = p.nrows;
             u.swiglu = 1; u.act_img = img_ff_; u.act_ktiles = L.down.K / kt; u.act_valid = spec.mlp.ff;
             if (spec.mlp.act == TkMlpSpec::CLAMPED) { u.act_clamped = 1; u.act_limit = spec.mlp.limit; u.act_slope = spec.mlp.slope; u.act_shift = spec.mlp.shift; }
             gemm(u);
             TkImgGemm w{};
-            w.type = type; w.w = L.down.img; w.a = img_ff_; w.K = L.down.K; w.N = L.down.N; w.nrows = n; w.out = y_; w.ldc = D; w.n_valid = D;
+            w.type = type; w.w = L.down.img; w.a = img_ff_; w.K = L.down.K; w.N = L.down.N; w.nrows = n; w.as_rows = p.nrows; w.out = y_; w.ldc = D; w.n_valid = D;
             w.max_slabs = most; w.slab_floats = slab;
             gemm(w, &slabs);
             tk_launch_post_norm(type, TkSubOut{y_, D, slabs, slab, nullptr, 0.0f, nullptr, nullptr, 0}, L.norm2, after, c.eps, D, n, x, img_x_, xkt, s);
         } else if (spec.mlp.kind == TkMlpSpec::MOE) {
-            enqueue_moe(spec, L, n);
+            enqueue_moe(spec, L, n, p.nrows);
             tk_launch_post_norm(type, TkSubOut{y_, D, 1, 0, nullptr, 0.0f, moe_.slot, moe_.weight, spec.mlp.top}, L.norm2, after, c.eps, D, n, x, img_x_, xkt, s);
         }
         if (streams_) (void)hipMemcpyAsync(streams_ + l * (size_t)n * D, x_, (size_t)n * D * 4, hipMemcpyDeviceToHost, s);

@@ -57,6 +57,9 @@ struct TkImgGemm {
     const TkImgBlock* blocks;
     const int32_t* n_blocks;
     int max_blocks, block_tiles;
+    /* rows that were taken out of a pass of as_rows (grouped: of as_blocks row blocks at most): the sums are those, bit for bit, that the product over the whole pass makes
+     * of them, whatever kernel that takes.  0: these rows are the pass */
+    int as_rows, as_blocks;
     int live_blocks;     /* how many are expected to be live (0: all of max_blocks); for the choice of a form only */
     size_t group_bytes;  /* between the weight images of two groups */
 };
@@ -68,13 +71,16 @@ const char* tk_launch_gemm_image(const TkImgGemm& g, hipStream_t s, int* slabs =
  * of a column tile); stages = 0: the skinny kernel.  Reads no pointer. */
 void tk_gemm_image_form(const TkImgGemm& g, int form[4]);
 
-/* row blocks of `rows` rows sent to `top` of `experts` each: tiles of a block, the most there can be, and how many to expect (an expert's last block is half
+/* row blocks of `rows` rows, taken out of a pass of `as_rows`, sent to `top` of `experts` each: tiles of a block, the most there can be, and how many to expect (an expert's last block is half
  * the time there) */
-static inline void tk_img_expert_blocks(int64_t rows, int top, int experts, TkImgGemm* g) {
-    const int64_t assign = rows * top, per = assign / experts, used = experts < assign ? experts : assign;
+static inline void tk_img_expert_blocks(int64_t rows, int64_t as_rows, int top, int experts, TkImgGemm* g) {
+    const int64_t per = as_rows * top / experts;
     g->block_tiles = per <= 16 ? 1 : per <= 32 ? 2 : per <= 64 ? 4 : 8;
-    g->max_blocks = (int)(used + assign / (16 * g->block_tiles));
-    g->live_blocks = g->max_blocks - (int)(used / 2);
+    auto used = [&](int64_t r) { return experts < r * top ? experts : (int)(r * top); };
+    auto most = [&](int64_t r) { return (int)(used(r) + r * top / (16 * g->block_tiles)); };
+    g->max_blocks = most(rows);
+    g->as_blocks = most(as_rows);
+    g->live_blocks = g->max_blocks - used(rows) / 2;
 }
 
 /* opts the kernels into their dynamic LDS on the calling thread's current device; nullptr or an error string.  Idempotent, thread-safe. */

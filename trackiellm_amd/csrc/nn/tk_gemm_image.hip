@@ -340,19 +340,24 @@ float wide_us(const WideForm& w, bool f32, int64_t blocks, float k /* thousands 
     if (w.per_cu == 1) return (float)((blocks + 255) / 256) * one;
     return (float)(blocks / 512) * two + (blocks % 512 == 0 ? 0.0f : blocks % 512 <= 256 ? one : two);
 }
+/* rows and row blocks whose sums a launch makes (TkImgGemm::as_rows) */
+int order_rows(const TkImgGemm& g) { return std::max(g.nrows, g.as_rows); }
+int order_tiles(const TkImgGemm& g, bool grouped) { return grouped ? g.block_tiles : (order_rows(g) + 15) / 16; }
+
 struct WidePick { int form, ks; };
-WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
-    const int ntiles = g.N / 16, mtiles = (g.nrows + 15) / 16;
+/* ks: parts of k, 0 for its own choice.  A row's sums depend on the parts alone, not on the blocks */
+WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped, int rows, int parts) {
+    const int ntiles = g.N / 16, mtiles = (rows + 15) / 16;
     /* k in parts whose sums the consumer adds, at least 16 k tiles each: it reads, and this kernel writes, a slab more per part */
-    const int kt = tk_img_kt(g.type), most = swiglu || grouped || g.max_slabs < 1 ? 1 : g.max_slabs;
-    const float slab_us = (float)((double)g.nrows * g.n_valid * 8e-6 / 5.0);
+    const int kt = tk_img_kt(g.type), most = parts ? parts : swiglu || grouped || g.max_slabs < 1 ? 1 : g.max_slabs;
+    const float slab_us = (float)((double)rows * g.n_valid * 8e-6 / 5.0);
     /* f32: no fewer parts than bring 128 x 128 blocks to two a CU, also where fewer would be a little quicker (0 - 20 us a product): shorter chains of sums,
      * 3 - 4 % less error in the logits of prompts of 150 - 300 rows */
-    int fewest = 1;
+    int fewest = parts ? parts : 1;
     const int64_t full = (int64_t)((mtiles + 7) / 8) * ((ntiles + 7) / 8);
-    if (g.type == TK_IMG_F32 && most > 1 && full < 256) fewest = (int)std::max<int64_t>(1, std::min<int64_t>({512 / full, most, g.K / kt / 16}));
+    if (!parts && g.type == TK_IMG_F32 && most > 1 && full < 256) fewest = (int)std::max<int64_t>(1, std::min<int64_t>({512 / full, most, g.K / kt / 16}));
     const int row_blocks = g.live_blocks > 0 && g.live_blocks < g.max_blocks ? g.live_blocks : g.max_blocks;
-    WidePick best{2, 1};
+    WidePick best{2, fewest};
     float least = 1e30f;
     for (int f = 0; f < (int)(sizeof wide_forms / sizeof wide_forms[0]); ++f) {
         const WideForm& w = wide_forms[f];
@@ -365,6 +370,10 @@ WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
     }
     return best;
 }
+WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
+    const WidePick whole = pick_wide(g, swiglu, grouped, order_rows(g), 0);
+    return grouped || order_rows(g) == g.nrows ? whole : pick_wide(g, swiglu, grouped, g.nrows, whole.ks);
+}
 
 /* A product of few rows by two workgroups a column tile, in TK_SKINNY_SLABS slabs, where its column tiles leave half of the CUs idle and there is work for every wave:
  * 40 rows x 2048 x 8192 19.7 -> 13.9 us, x 2048 7.2 -> 6.1.  Steps of an eight-layer model 2048 wide with one workgroup / two: 1 row 539 / 529 us, 16 rows 599 / 590, 40 rows
@@ -374,20 +383,20 @@ WidePick pick_wide(const TkImgGemm& g, bool swiglu, bool grouped) {
 #define TK_SKINNY_WAVES 8
 #define TK_SKINNY_SLABS (1 + TK_SKINNY_WAVES / 2)
 int skinny_parts(const TkImgGemm& g, bool swiglu, bool grouped) {
-    const int most = g.nrows > 16 && g.K / tk_img_kt(g.type) >= 128 ? 256 : 128;
+    const int most = order_rows(g) > 16 && g.K / tk_img_kt(g.type) >= 128 ? 256 : 128;
     return !swiglu && !grouped && g.max_slabs >= TK_SKINNY_SLABS && g.N / 16 <= most && g.K / tk_img_kt(g.type) >= 64 ? 2 : 1;
 }
 
 template <typename T, bool SWIGLU, bool GROUPED>
 const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
     const int ntiles = g.N / 16;
-    const int mtiles = GROUPED ? g.block_tiles : (g.nrows + 15) / 16;
+    const int mtiles = order_tiles(g, GROUPED);
     if (mtiles <= 4) {
-        /* GROUPED: one block per table entry */
-        const int gy = GROUPED ? g.max_blocks : 1;
+        /* GROUPED: one block per table entry; the waves of a workgroup, which share k out, by the whole pass's */
+        const int blocks = GROUPED ? g.max_blocks : 1, gy = GROUPED ? std::max(g.max_blocks, g.as_blocks) : 1;
         const int parts = skinny_parts(g, SWIGLU, GROUPED);
         if (slabs) *slabs = parts > 1 ? TK_SKINNY_SLABS : 1;
-#define TK_SK(MT, NT, WV, P) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, P, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, gy, P), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
+#define TK_SK(MT, NT, WV, P) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, P, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, blocks, P), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
 #define TK_SKM2(NT, WV, P) do { if (mtiles <= 2) TK_SK(2, NT, WV, P); else if (mtiles <= 3) TK_SK(3, NT, WV, P); else TK_SK(4, NT, WV, P); } while (0)
 #define TK_SKM(NT, WV, P) do { if (mtiles <= 1) TK_SK(1, NT, WV, P); else TK_SKM2(NT, WV, P); } while (0)
         /* Column tiles of a workgroup: every workgroup reads its rows' activations again, which from two M-tiles on is more than its weights and comes from the L2s.  So four
@@ -413,7 +422,7 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
     }
     const WidePick pick = pick_wide(g, SWIGLU, GROUPED);
     if (slabs) *slabs = pick.ks;
-#define TK_WD(MB, NB, WM, WN, RING) do { const int nbn = (ntiles + NB - 1) / NB, nbm = GROUPED ? g.max_blocks : (mtiles + MB - 1) / MB; \
+#define TK_WD(MB, NB, WM, WN, RING) do { const int nbn = (ntiles + NB - 1) / NB, nbm = GROUPED ? g.max_blocks : ((g.nrows + 15) / 16 + MB - 1) / MB; \
         hipLaunchKernelGGL((k_gemm_wide<T, MB, NB, WM, WN, RING, SWIGLU, GROUPED>), dim3(nbn * nbm * pick.ks), dim3(64 * WM * WN), (size_t)RING * wide_stage(MB, NB), s, g, nbn, nbm, pick.ks); } while (0)
     switch (pick.form) {
         case 0: if constexpr (!GROUPED) TK_WD(16, 16, 4, 2, 2); break;
@@ -432,7 +441,7 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
 void tk_gemm_image_form(const TkImgGemm& g, int form[4]) {
     const bool grouped = g.max_blocks > 0;
     form[0] = 64; form[1] = form[2] = 0; form[3] = 1;
-    if ((grouped ? g.block_tiles : (g.nrows + 15) / 16) <= 4) { form[3] = skinny_parts(g, g.swiglu != 0, grouped); return; }
+    if (order_tiles(g, grouped) <= 4) { form[3] = skinny_parts(g, g.swiglu != 0, grouped); return; }
     const WidePick p = pick_wide(g, g.swiglu != 0, grouped);
     const WideForm& w = wide_forms[p.form];
     form[0] = 16 * w.mb; form[1] = 16 * w.nb; form[2] = w.ring; form[3] = p.ks;
