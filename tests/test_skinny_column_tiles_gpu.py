@@ -4,6 +4,8 @@ import ctypes as C
 import numpy as np
 import pytest
 
+from layered_util import attention, config, delta, dense, layer
+
 pytestmark = pytest.mark.gpu
 
 
@@ -44,3 +46,21 @@ def test_slabs_of_two_column_tiles_add_up_to_the_whole(gpu, rows, N, f32, K):
     whole, one = product(gpu, x, w, 1, f32)
     parts, n = product(gpu, x, w, 8, f32)
     assert one == 1 and n == 5 and np.array_equal(parts.view(np.uint32), whole.view(np.uint32))
+
+
+@pytest.mark.parametrize("f32", [0, 1])
+@pytest.mark.parametrize("N", [2064, 6160, 24576, 28672, 32000, 33000])
+def test_a_rows_sums_are_those_of_a_step_of_fewer_rows(gpu, N, f32):
+    """bit for bit, within one depth of the loads (up to 32 rows, up to 64), which is also the order of k"""
+    x, w = operands(64, N, 528 if f32 else 1056, f32)
+    for few, more in ((1, 17), (16, 32), (33, 64)):
+        a, b = product(gpu, x[:few], w, 1, f32)[0], product(gpu, x[:more], w, 1, f32)[0]
+        assert np.array_equal(a.view(np.uint32), b[:few].view(np.uint32)), (few, more)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+def test_a_sequences_logits_are_those_of_a_step_of_fewer(gpu, dtype):
+    """the same for gate and up, 24 608 columns together"""
+    m = gpu.LlmModel(config=config(1056, 96, [layer(attention(4, 2, 64, 64, 32, 70, 2), delta(4, 2, 64, 64, 4), dense(12304))]), dtype=dtype, seed=9)
+    got = [gpu.LlmSession(m, 32, 8).forward_rows(range(n), [0] * n, range(n), range(n))[0] for n in (16, 17, 32)]
+    assert np.array_equal(got[0], got[2][:16]) and np.array_equal(got[1], got[2][:17])

@@ -56,11 +56,13 @@ __device__ __forceinline__ void store_act(const TkImgGemm& a, int mt, int ct, in
 /* ---- skinny: MT M-tiles of rows, NT column tiles per workgroup, K interleaved over the waves in pieces of U tiles ----
  * Loads of three M-tiles are three (33 .. 48 rows; four, one of them twice: 40 rows x 2048 x 16384 gate and up 17.2 -> 15.8 us, x 32000 34.2 -> 28.6).
  * PARTS = 2: the waves of a column tile in two workgroups (skinny_parts), each wave with two pieces on their way.  The first workgroup adds its waves up in slab 0, each wave
- * of the second has a slab of its own: added in ascending order, they are the sum that one workgroup of all waves makes. */
-template <typename T, int MT, int NT, int WAVES, int PARTS, bool SWIGLU, bool GROUPED>
+ * of the second has a slab of its own: added in ascending order, they are the sum that one workgroup of all waves makes.
+ * CHAINS = 2: each wave makes the sums of two waves one behind the other, so that four waves give the bits of eight. */
+template <typename T, int MT, int NT, int WAVES, int PARTS, int CHAINS, bool SWIGLU, bool GROUPED>
 __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
     static_assert(PARTS == 1 || (PARTS == 2 && !SWIGLU && !GROUPED), "slabs are of plain products");
-    constexpr int U = MT >= 3 ? 2 : 4, STEP = PARTS * WAVES * U, AHEAD = PARTS;
+    static_assert(CHAINS == 1 || (CHAINS == 2 && PARTS == 1), "two chains a wave: of products in one part");
+    constexpr int U = MT >= 3 ? 2 : 4, STEP = PARTS * CHAINS * WAVES * U, AHEAD = PARTS;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int ktiles = a.K / TkImg<T>::KT;
@@ -81,10 +83,13 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
 #pragma unroll
     for (int m = 0; m < MT; ++m) ap[m] = (const uint8_t*)a.a + (size_t)(m0 + (m < mlive ? m : 0)) * ktiles * 1024 + lane * 16;
     tk_v4f acc[NT][MT];
+    auto clear = [&] {
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+        for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[n][m] = tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+            for (int m = 0; m < MT; ++m) acc[n][m] = tk_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    };
+    clear();
     const tk_v4u zero = {0, 0, 0, 0};
     tk_v4u wq[AHEAD][U][NT], aq[AHEAD][U][MT];
     /* tiles past the end re-read the last one against a zero activation: no branch around a load */
@@ -102,29 +107,33 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
 #pragma unroll
     for (int p = 0; p < AHEAD; ++p)
         if (PARTS > 1 || c < ktiles) load(p, c + p * STEP);
-    while (c < ktiles) {
+    auto walk = [&](int c, int after /* where the next chain starts */) {
+        while (c < ktiles) {
 #pragma unroll
-        for (int p = 0; p < AHEAD; ++p) {
-            tk_v4u w0[U][NT], a0[U][MT];
+            for (int p = 0; p < AHEAD; ++p) {
+                tk_v4u w0[U][NT], a0[U][MT];
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
+                for (int u = 0; u < U; ++u) {
 #pragma unroll
-                for (int n = 0; n < NT; ++n) w0[u][n] = wq[p][u][n];
+                    for (int n = 0; n < NT; ++n) w0[u][n] = wq[p][u][n];
 #pragma unroll
-                for (int m = 0; m < MT; ++m) a0[u][m] = c + u < ktiles ? aq[p][u][m] : zero;
+                    for (int m = 0; m < MT; ++m) a0[u][m] = c + u < ktiles ? aq[p][u][m] : zero;
+                }
+                const int next = c + AHEAD * STEP;
+                if (PARTS > 1 || next < ktiles) load(p, next);
+                else if (CHAINS > 1 && after < ktiles) load(p, after);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int n = 0; n < NT; ++n)
+#pragma unroll
+                        for (int m = 0; m < MT; ++m) acc[n][m] = TkImg<T>::mma(w0[u][n], a0[u][m], acc[n][m]);
+                c += STEP;
+                if (c >= ktiles) break;
             }
-            const int next = c + AHEAD * STEP;
-            if (PARTS > 1 || next < ktiles) load(p, next);
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-#pragma unroll
-                for (int n = 0; n < NT; ++n)
-#pragma unroll
-                    for (int m = 0; m < MT; ++m) acc[n][m] = TkImg<T>::mma(w0[u][n], a0[u][m], acc[n][m]);
-            c += STEP;
-            if (c >= ktiles) break;
         }
-    }
+    };
+    if (CHAINS == 1) walk(c, ktiles);
     if (PARTS > 1 && blockIdx.z) {
         a.out += (size_t)(1 + wave) * a.slab_floats;
 #pragma unroll
@@ -138,25 +147,50 @@ __global__ __launch_bounds__(64 * WAVES) void k_gemm_skinny(TkImgGemm a) {
     }
     /* partial sums of the waves, ascending */
     tk_v4f* red = (tk_v4f*)lds;
+    auto put = [&] {
 #pragma unroll
-    for (int n = 0; n < NT; ++n)
+        for (int n = 0; n < NT; ++n)
 #pragma unroll
-        for (int m = 0; m < MT; ++m) red[((wave * NT + n) * MT + m) * 64 + lane] = acc[n][m];
-    __syncthreads();
-    auto total = [&](int n, int m) {
-        tk_v4f s = red[(n * MT + m) * 64 + lane];
-        for (int w = 1; w < WAVES; ++w) s += red[((w * NT + n) * MT + m) * 64 + lane];
+            for (int m = 0; m < MT; ++m) red[((wave * NT + n) * MT + m) * 64 + lane] = acc[n][m];
+        __syncthreads();
+    };
+    auto fold = [&](tk_v4f s, int w, int n, int m) {
+        for (; w < WAVES; ++w) s += red[((w * NT + n) * MT + m) * 64 + lane];
         return s;
     };
-    constexpr int UNITS = SWIGLU ? NT / 2 * MT : NT * MT;
-    for (int i = wave; i < UNITS; i += WAVES) {
-        const int n = i / MT, m = i % MT;
+    constexpr int HALVES = SWIGLU ? 2 : 1, UNITS = NT / HALVES * MT, MINE = (UNITS + WAVES - 1) / WAVES;
+    tk_v4f first[CHAINS > 1 ? MINE : 1][HALVES]; /* the sum of the first chains */
+    if (CHAINS == 1) put();
+    else {
+#pragma unroll 1
+        for (int r = 0; r < CHAINS; ++r) {
+            walk(c, r + 1 < CHAINS ? c + WAVES * U : ktiles);
+            if (r) __syncthreads();
+            put();
+            if (r + 1 == CHAINS) break;
+#pragma unroll
+            for (int j = 0; j < MINE; ++j) {
+                const int i = wave + j * WAVES < UNITS ? wave + j * WAVES : 0;
+#pragma unroll
+                for (int h = 0; h < HALVES; ++h) first[CHAINS > 1 ? j : 0][h] = fold(red[((HALVES * (i / MT) + h) * MT + i % MT) * 64 + lane], 1, HALVES * (i / MT) + h, i % MT);
+            }
+            clear();
+            c += WAVES * U;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < MINE; ++j) {
+        const int i = wave + j * WAVES, n = i / MT, m = i % MT;
+        if (i >= UNITS) break;
         const int64_t row = (int64_t)(m0 + m) * 16 + (lane & 15);
         if (m >= mlive || (!GROUPED && row >= a.nrows)) continue;
+        auto total = [&](int h) {
+            return CHAINS > 1 ? fold(first[CHAINS > 1 ? j : 0][h], 0, HALVES * n + h, m) : fold(red[((HALVES * n + h) * MT + m) * 64 + lane], 1, HALVES * n + h, m);
+        };
         if (SWIGLU) {
-            if (n0 + 2 * n < ntot) store_act<T>(a, m0 + m, n0 / 2 + n, lane, total(2 * n, m), total(2 * n + 1, m));
+            if (n0 + 2 * n < ntot) store_act<T>(a, m0 + m, n0 / 2 + n, lane, total(0), total(HALVES - 1));
         } else if (n0 + n < ntot) {
-            store_f32<T>(a, row, (n0 + n) * 16 + 4 * (lane >> 4), total(n, m));
+            store_f32<T>(a, row, (n0 + n) * 16 + 4 * (lane >> 4), total(0));
         }
     }
 }
@@ -396,16 +430,26 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
         const int blocks = GROUPED ? g.max_blocks : 1, gy = GROUPED ? std::max(g.max_blocks, g.as_blocks) : 1;
         const int parts = skinny_parts(g, SWIGLU, GROUPED);
         if (slabs) *slabs = parts > 1 ? TK_SKINNY_SLABS : 1;
-#define TK_SK(MT, NT, WV, P) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, P, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, blocks, P), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
+#define TK_SKC(MT, NT, WV, P, C) hipLaunchKernelGGL((k_gemm_skinny<T, MT, NT, WV, P, C, SWIGLU, GROUPED>), dim3((ntiles + NT - 1) / NT, blocks, P), dim3(64 * WV), (size_t)WV * NT * MT * 1024, s, g)
+#define TK_SK(MT, NT, WV, P) TK_SKC(MT, NT, WV, P, 1)
 #define TK_SKM2(NT, WV, P) do { if (mtiles <= 2) TK_SK(2, NT, WV, P); else if (mtiles <= 3) TK_SK(3, NT, WV, P); else TK_SK(4, NT, WV, P); } while (0)
 #define TK_SKM(NT, WV, P) do { if (mtiles <= 1) TK_SK(1, NT, WV, P); else TK_SKM2(NT, WV, P); } while (0)
-        /* Column tiles of a workgroup: every workgroup reads its rows' activations again, which from two M-tiles on is more than its weights and comes from the L2s.  So four
-         * where that leaves 384 workgroups and more, two where it leaves 192.  4096 x 28672 (gate and up) at 20, 40, 60 rows with two / four 47.9 / 41.5, 51.2 / 45.6, 60.9 / 48.4
-         * us, x 32000 50.8 / 43.4, 55.5 / 49.7, 68.3 / 53.5 (at 1 row 40.0 / 41.9); x 7440 with one / two at 1, 20, 40, 60 rows 13.6 / 11.9, 17.3 / 14.5, 21.2 / 16.2, 23.7 / 18.9. */
-        if (!GROUPED && mtiles >= 2 && ntiles >= 1536) {
-            TK_SKM2(4, 4, 1);
+        /* Column tiles of a workgroup: every workgroup reads its rows' activations again, which from two M-tiles on is more than its weights and comes from the L2s.  So two from 384
+         * on: 4096 x 7440 with one / two at 1, 20, 40, 60 rows 16.3 / 14.0, 19.0 / 15.9, 22.1 / 17.2, 25.1 / 19.0 us.  Four where workgroups of two are more than run at once (768
+         * of eight waves), at two M-tiles as long as those of four do (512 of four waves): 4096 x 24576, 28672, 32000 with two / four at 20 rows 39.2 / 42.8, 49.0 / 45.2,
+         * 50.2 / 47.4, at 60 rows 50.8 / 51.8, 63.8 / 55.6, 67.5 / 59.9; x 40960 59.2 / 61.6, 80.6 / 74.2.  Three M-tiles ask for less at a time and gain less, with two chains a wave and a
+         * long k nothing in the end: 4096 x 27648, 30720, 32000 at 40 rows 52.6 / 50.5, 54.5 / 55.2, 55.2 / 57.4, 2048 x 32000 29.4 / 27.4.
+         * Below 2048 tiles k is shared out in eight chains, from there on in four, whatever the rows: a row's sums are those of a step of fewer. */
+        const bool four = !GROUPED && mtiles >= 2 && ntiles > 1536 && (mtiles == 2 ? ntiles <= 2048 : mtiles > 3 || ntiles >= 2048 || ntiles <= 1792 || g.K <= 2048);
+        if (four) {
+            if constexpr (!GROUPED) {
+                if (ntiles >= 2048) TK_SKM2(4, 4, 1);
+                else if (mtiles <= 2) TK_SKC(2, 4, 4, 1, 2);
+                else if (mtiles <= 3) TK_SKC(3, 4, 4, 1, 2);
+                else TK_SKC(4, 4, 4, 1, 2);
+            }
         } else if (!GROUPED && !SWIGLU && ntiles >= 384 && ntiles < 1024) {
-            TK_SKM(2, 8, 1);
+            if constexpr (!GROUPED) TK_SKM(2, 8, 1);
         } else if (SWIGLU || ntiles * gy >= 1024) {
             if (ntiles * gy >= 2048) TK_SKM(2, 4, 1); else TK_SKM(2, 8, 1);
         } else if (parts > 1) {
@@ -418,6 +462,7 @@ const char* launch(const TkImgGemm& g, hipStream_t s, int* slabs) {
 #undef TK_SKM
 #undef TK_SKM2
 #undef TK_SK
+#undef TK_SKC
         return nullptr;
     }
     const WidePick pick = pick_wide(g, SWIGLU, GROUPED);
