@@ -43,3 +43,19 @@ def test_prefill_equals_passes_of_256_rows(gpu, models, model, nseq, n_prompt):
     assert np.array_equal(first, want_first)
     assert np.array_equal(ids[0], want_ids)
     assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), np.abs(got - want).max()
+
+
+@pytest.mark.parametrize("model", ["wide", "wide-f16"])
+@pytest.mark.parametrize("rows", [1, 2, 3, 40])
+def test_passes_without_a_head_leave_every_layers_keys_and_values(gpu, models, monkeypatch, model, rows):
+    """one position of each sequence whose logits nobody wants, as plain launches and as a graph, at row counts of either kind of product: what the next position reads is the same,
+    and what a pass with a head leaves"""
+    m = models(model)
+    toks = np.random.default_rng(rows).integers(3, m.hparams.vocab, (2, rows)).astype(np.int32)
+    got = {}
+    for name, graphs, head in (("head", "0", True), ("graph", "0", False), ("plain", "1", False)):
+        monkeypatch.setenv("TK_MI355X_NO_GRAPH", graphs)
+        s = gpu.LlmSession(m, rows, 8)
+        s.forward_rows(range(rows), [0] * rows, toks[0], range(rows) if head else [], want_logits=head)
+        got[name] = s.forward(np.arange(rows), np.ones(rows), toks[1])[0].view(np.uint32)
+    assert np.array_equal(got["graph"], got["head"]) and np.array_equal(got["plain"], got["head"])

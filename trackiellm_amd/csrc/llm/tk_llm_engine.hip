@@ -357,8 +357,8 @@ static void set_act(TkGemvArgs& a, const TkActQ8& q) {
 
 static TkGemvSeg seg_of(const TkDevTensor& t) { return TkGemvSeg{t.data, t.type, (int)(t.rows / TK_TILE_ROWS)}; }
 
-/* a pass without a head is read through the caches alone: its last layer ends with them */
-void TkLlmSession::enqueue_pass(int nrows, bool lm_head, bool fused_attn) { enqueue_range(nrows, 0, model->hp.n_layer, true, false, lm_head, fused_attn, !lm_head); }
+/* a pass without a head is read through the caches alone: its last layer ends with them, in front of the attention, which therefore can't be what appends to them */
+void TkLlmSession::enqueue_pass(int nrows, bool lm_head, bool fused_attn) { enqueue_range(nrows, 0, model->hp.n_layer, true, false, lm_head, lm_head && fused_attn, !lm_head); }
 
 /* layers [l0, l1) of one pass.  embed: the residual stream starts from the token embeddings (first pipeline stage), otherwise x
  * already holds it.  fold_out: finish the last layer's residual update so x is the complete stream (it leaves this GPU).
@@ -559,7 +559,7 @@ bool TkLlmSession::forward(int nrows, const int32_t* seq, const int32_t* pos, co
     hipGraphExec_t* slot = !graphs_enabled() ? nullptr
                            : !lm_head ? &graph_prefill[tiled_pass][nrows] : distinct ? &graph_exec[long_pass][nrows] : &graph_head_nf[tiled_pass][nrows];
     if (slot) {
-        if (!capture_pass(slot, nrows, lm_head, lm_head && distinct)) return false;
+        if (!capture_pass(slot, nrows, lm_head, distinct)) return false;
         HIPQ(hipGraphLaunch(*slot, stream));
     } else {
         launch_error.clear();
