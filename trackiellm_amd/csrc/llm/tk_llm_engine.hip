@@ -643,6 +643,11 @@ bool TkLlmSession::prefill(int nseq, int n_prompt, const int32_t* tokens, int32_
     if (n_prompt <= 0 || n_prompt >= max_ctx) { error = "prompt does not fit the context"; return false; }
     for (int64_t i = 0; i < (int64_t)nseq * n_prompt; ++i)
         if (tokens[i] < 0 || tokens[i] >= model->hp.vocab) { error = "row out of range (sequence id, position or token id)"; return false; }
+    if (n_prompt == 1) { /* a decode step, whose graph is there (or will be used): 32 layers 4096 wide, one prompt 1.61 ms, by the launches below 1.75; 16 prompts 1.93, 2.12 */
+        std::vector<int32_t> sq(nseq), ps(nseq, 0);
+        for (int s = 0; s < nseq; ++s) sq[s] = s;
+        return forward(nseq, sq.data(), ps.data(), tokens, nullptr, first_tokens_host, true);
+    }
     HIPQ(hipSetDevice(model->device));
     const TkLlmHParams& h = model->hp;
     const int QD = h.n_head * h.head_dim, KVD = h.n_kv_head * h.head_dim, last = h.n_layer - 1;
