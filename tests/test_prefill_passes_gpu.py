@@ -59,3 +59,23 @@ def test_passes_without_a_head_leave_every_layers_keys_and_values(gpu, models, m
         s.forward_rows(range(rows), [0] * rows, toks[0], range(rows) if head else [], want_logits=head)
         got[name] = s.forward(np.arange(rows), np.ones(rows), toks[1])[0].view(np.uint32)
     assert np.array_equal(got["graph"], got["head"]) and np.array_equal(got["plain"], got["head"])
+
+
+@pytest.mark.parametrize("ctx,rows", [(64, 256), (2100, 2048)])
+def test_memory_of_a_session(gpu, ctx, rows):
+    """what a pass of `rows` rows writes once: its K-split slabs, the residual stream, queries, activation images (their sums are 0.4 of their bytes), the logits of 256 rows and the caches;
+    a tenth and 48 MB for tables, what is kept of 256 sampled rows and the allocator's pages"""
+    import gc
+
+    import torch
+    m = gpu.LlmModel(gpu.LlmHParams(1, 4096, 32, 8, 128, 14336, 32000, 1e-5, 10000.0, 0, 0, 0, 0, 1)).fill_synthetic(4)
+    h = m.hparams
+    slabs = max(h.ks_qkv * 6144, h.ks_o * 4096, h.ks_gateup * 2 * 14336, h.ks_down * 4096)
+    need = 4 * rows * (slabs + 2 * 4096) + 1.4 * rows * (2 * 4096 + 14336) + 4 * 256 * 32000 + 4 * ctx * 1024
+    gc.collect()
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info(0)[0]
+    s = gpu.LlmSession(m, 1, ctx)
+    used = before - torch.cuda.mem_get_info(0)[0]
+    s.close()
+    assert used < 1.1 * need + (48 << 20), (used >> 20, int(need) >> 20)

@@ -112,6 +112,8 @@ private:
     int enqueue_matmul(const TkDevTensor* const* t, int nseg, int K, int ks, int n_total, const TkActQ8& act, float* out, int nrows);
     uint16_t *kcache = nullptr, *vcache = nullptr;
     int pass_rows = 0; /* rows of prefill()'s passes, and of every buffer a pass of rows writes */
+    int64_t pitch(int cols) const { return (int64_t)pass_rows * cols; } /* between the K-split slabs in `partial` */
+    static int64_t pitch2(int cols) { return (int64_t)TK_GEMV_FUSE_MAX_ROWS * cols; } /* .. in `partial2` */
     float *x_last = nullptr, *q_last = nullptr; /* [TK_MAX_ROWS][..]: what prefill() keeps of the rows it samples */
     float *x = nullptr, *x2 = nullptr, *qbuf = nullptr, *partial = nullptr, *partial2 = nullptr, *rope_cos = nullptr, *rope_sin = nullptr;
     TkActQ8 act_d{}, act_qd{}, act_ff{};

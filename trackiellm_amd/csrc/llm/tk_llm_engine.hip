@@ -276,16 +276,13 @@ bool TkLlmSession::init(TkLlmModel* m, int mseq, int mctx) {
     HIPQ(hipMalloc((void**)&qbuf, (size_t)pass_rows * QD * 4));
     HIPQ(hipMalloc((void**)&x_last, (size_t)TK_MAX_ROWS * h.d_model * 4));
     HIPQ(hipMalloc((void**)&q_last, (size_t)TK_MAX_ROWS * QD * 4));
-    /* K-split slabs, TK_SLAB_ROWS rows apart; the last one ends with the pass */
-    auto slabs = [&](int ks, int cols, int rows) { return ((size_t)(ks - 1) * TK_SLAB_ROWS + rows) * (size_t)cols; };
-    auto partial_floats = [&](int rows) {
-        return std::max(std::max(slabs(h.ks_qkv, QD + 2 * KVD, rows), slabs(h.ks_o, h.d_model, rows)), std::max(slabs(h.ks_gateup, 2 * h.d_ff, rows), slabs(h.ks_down, h.d_model, rows)));
-    };
-    HIPQ(hipMalloc((void**)&partial, partial_floats(pass_rows) * 4));
+    /* K-split slabs of a row */
+    const size_t in_slabs = std::max((size_t)h.ks_qkv * (QD + 2 * KVD), (size_t)h.ks_gateup * 2 * h.d_ff), out_slabs = (size_t)std::max(h.ks_o, h.ks_down) * h.d_model;
+    HIPQ(hipMalloc((void**)&partial, std::max(in_slabs, out_slabs) * pass_rows * 4));
     /* twins for passes whose mat-vec launches run their producer themselves (enqueue_range): such a launch reads one (x, slab) pair while
      * its workgroups write the other */
     HIPQ(hipMalloc((void**)&x2, (size_t)TK_GEMV_FUSE_MAX_ROWS * h.d_model * 4));
-    HIPQ(hipMalloc((void**)&partial2, partial_floats(TK_GEMV_FUSE_MAX_ROWS) * 4));
+    HIPQ(hipMalloc((void**)&partial2, in_slabs * TK_GEMV_FUSE_MAX_ROWS * 4));
     if (!alloc_act(&act_d, h.d_model, pass_rows, m->has_f16, error) || !alloc_act(&act_qd, QD, pass_rows, m->has_f16, error) || !alloc_act(&act_ff, h.d_ff, pass_rows, m->has_f16, error)) return false;
     HIPQ(hipMalloc((void**)&d_tiles, (size_t)(1 + pass_rows) * 4));
     HIPQ(hipMemset(d_tiles, 0, (size_t)(1 + pass_rows) * 4));
@@ -371,7 +368,7 @@ int TkLlmSession::enqueue_matmul(const TkDevTensor* const* t, int nseg, int K, i
     if (t[0]->type == TK_TYPE_F16) {
         TkTiledGemm f{};
         for (int i = 0; i < nseg; ++i) { f.tiles[i] = t[i]->data; f.row_tiles[i] = (int)(t[i]->rows / TK_TILE_ROWS); }
-        f.nseg = nseg; f.wbytes = 2; f.K = K; f.ks = ks; f.ldc = n_total; f.n_valid = n_total; f.nrows = nrows; f.slab_rows = TK_SLAB_ROWS;
+        f.nseg = nseg; f.wbytes = 2; f.K = K; f.ks = ks; f.ldc = n_total; f.n_valid = n_total; f.nrows = nrows; f.slab_rows = pass_rows;
         f.a_img = act.af; f.a_ts = act.af_ts; f.out = out;
         /* shapes were validated when the model was installed (K a multiple of 256 ks); a refusal here would leave the slab unwritten, so it is
          * recorded and fails the pass (forward / decode / capture_pass check launch_error) instead of producing garbage silently */
@@ -380,7 +377,7 @@ int TkLlmSession::enqueue_matmul(const TkDevTensor* const* t, int nseg, int K, i
     }
     TkGemvArgs a{};
     for (int i = 0; i < nseg; ++i) a.seg[i] = seg_of(*t[i]);
-    a.nseg = nseg; a.K = K; a.ks = ks; a.n_total = n_total; a.nrows = nrows;
+    a.nseg = nseg; a.K = K; a.ks = ks; a.n_total = n_total; a.slab_pitch = pitch(n_total); a.nrows = nrows;
     set_act(a, act); a.out = out;
     tk_launch_gemv(a, s);
     return ks;
@@ -401,7 +398,7 @@ int TkLlmSession::enqueue_layer_tail(const TkLlmLayer& L, float* xs, int nrows) 
     const TkDevTensor* gu[2] = {&L.gate, &L.up};
     const TkDevTensor* dn[1] = {&L.down};
     const int ks_o = enqueue_matmul(ot, 1, QD, h.ks_o, D, act_qd, partial, nrows);
-    tk_launch_rmsnorm_q8(xs, partial, ks_o, D, (const float*)L.ffn_norm.data, h.rms_eps, D, nrows, act_d, s);
+    tk_launch_rmsnorm_q8(xs, partial, ks_o, D, pitch(D), (const float*)L.ffn_norm.data, h.rms_eps, D, nrows, act_d, s);
     if (tk_gemv_fuses_swiglu(nrows, h.ks_gateup, L.gate.type, L.up.type)) { /* wide pass: SwiGLU in the launch's epilogue, `partial` holds h [rows][FF] */
         TkGemvArgs a{};
         a.seg[0] = seg_of(L.gate); a.seg[1] = seg_of(L.up);
@@ -411,7 +408,7 @@ int TkLlmSession::enqueue_layer_tail(const TkLlmLayer& L, float* xs, int nrows) 
         tk_launch_quant_q8(partial, FF, nrows, act_ff, s);
     } else {
         const int ks_gu = enqueue_matmul(gu, 2, D, h.ks_gateup, 2 * FF, act_d, partial, nrows);
-        tk_launch_swiglu_q8(partial, ks_gu, FF, nrows, act_ff, s);
+        tk_launch_swiglu_q8(partial, ks_gu, pitch(2 * FF), FF, nrows, act_ff, s);
     }
     return enqueue_matmul(dn, 1, FF, h.ks_down, D, act_ff, partial, nrows);
 }
@@ -421,7 +418,7 @@ void TkLlmSession::enqueue_head(float* xs, int ks_res, int nrows) {
     const TkLlmHParams& h = model->hp;
     const int D = h.d_model;
     const TkDevTensor* lm[1] = {&model->output};
-    tk_launch_rmsnorm_q8(xs, ks_res ? partial : nullptr, ks_res, D, (const float*)model->out_norm.data, h.rms_eps, D, nrows, act_d, stream);
+    tk_launch_rmsnorm_q8(xs, ks_res ? partial : nullptr, ks_res, D, pitch(D), (const float*)model->out_norm.data, h.rms_eps, D, nrows, act_d, stream);
     (void)enqueue_matmul(lm, 1, D, 1, h.vocab, act_d, logits, nrows);
     enqueue_pick(nrows);
 }
@@ -451,11 +448,12 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
                       tk_gemv_fuses_producer(nrows, D, h.ks_gateup, h.ks_o) && tk_gemv_fuses_producer(nrows, FF, h.ks_down, h.ks_gateup) &&
                       tk_gemv_fuses_producer(nrows, D, 1, h.ks_down);
     auto fused_gemv = [&](const TkDevTensor* const* t, int nseg, int K, int ks, int n_total, float* out, int mode, const float* xin, float* xout,
-                          const float* slab, int slab_ks, int slab_pitch, const float* w) {
+                          const float* slab, int slab_ks, int slab_cols, const float* w) {
         TkGemvArgs a{};
         for (int i = 0; i < nseg; ++i) a.seg[i] = seg_of(*t[i]);
         a.nseg = nseg; a.K = K; a.ks = ks; a.n_total = n_total; a.nrows = nrows; a.out = out;
-        a.fuse = mode; a.fx_in = xin; a.fx_out = xout; a.fslab = slab; a.fks = slab_ks; a.fn_total = slab_pitch; a.fw = w; a.feps = h.rms_eps;
+        a.slab_pitch = out == partial2 ? pitch2(n_total) : pitch(n_total); a.fslab_pitch = slab == partial2 ? pitch2(slab_cols) : pitch(slab_cols);
+        a.fuse = mode; a.fx_in = xin; a.fx_out = xout; a.fslab = slab; a.fks = slab_ks; a.fn_total = slab_cols; a.fw = w; a.feps = h.rms_eps;
         tk_launch_gemv(a, s);
         return ks;
     };
@@ -478,33 +476,33 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
             const TkDevTensor* dn[1] = {&L.down};
             const int ks_qkv = fused_gemv(qkv, 3, D, h.ks_qkv, QD + 2 * KVD, partial2, 1, x, x2, l == l0 ? nullptr : partial, ks_res, D, (const float*)L.attn_norm.data);
             if (!fused_attn)
-                tk_launch_qkv_rope_append(partial2, ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
+                tk_launch_qkv_rope_append(partial2, ks_qkv, QD + 2 * KVD, pitch2(QD + 2 * KVD), h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
                                           qbuf, kcache, vcache, l, max_seq, max_ctx, s);
             if (caches_only && l == l1 - 1) { last_x = x2; return; }
-            if (long_attn) tk_launch_attention_long(partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, !join_in_o, s);
+            if (long_attn) tk_launch_attention_long(partial2, ks_qkv, QD + 2 * KVD, pitch2(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, !join_in_o, s);
             else if (tiled_attn) tk_launch_attention_prefill(qbuf, kcache, vcache, d_seq, d_pos, d_tiles, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, act_qd, s);
-            else tk_launch_attention(qbuf, partial2, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
+            else tk_launch_attention(qbuf, partial2, ks_qkv, QD + 2 * KVD, pitch2(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
                                      h.head_dim, l, max_seq, max_ctx, act_qd, fused_attn, s);
             const int ks_o = join_in_o ? fused_gemv(ot, 1, QD, h.ks_o, D, partial, 3, parts.l, nullptr, parts.pv, 1, h.head_dim, nullptr) : enqueue_matmul(ot, 1, QD, h.ks_o, D, act_qd, partial, nrows);
             const int ks_gu = fused_gemv(gu, 2, D, h.ks_gateup, 2 * FF, partial2, 1, x2, x, partial, ks_o, D, (const float*)L.ffn_norm.data);
             ks_res = fused_gemv(dn, 1, FF, h.ks_down, D, partial, 2, nullptr, nullptr, partial2, ks_gu, 2 * FF, nullptr);
             continue;
         }
-        tk_launch_rmsnorm_q8(x, l == l0 ? nullptr : partial, ks_res, D, (const float*)L.attn_norm.data, h.rms_eps, D, nrows, act_d, s);
+        tk_launch_rmsnorm_q8(x, l == l0 ? nullptr : partial, ks_res, D, pitch(D), (const float*)L.attn_norm.data, h.rms_eps, D, nrows, act_d, s);
         const int ks_qkv = enqueue_matmul(qkv, 3, D, h.ks_qkv, QD + 2 * KVD, act_d, partial, nrows);
         if (!fused_attn)
-            tk_launch_qkv_rope_append(partial, ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
+            tk_launch_qkv_rope_append(partial, ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows,
                                       qbuf, kcache, vcache, l, max_seq, max_ctx, s);
         if (caches_only && l == l1 - 1) { last_x = x; return; }
-        if (long_attn) tk_launch_attention_long(partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, true, s);
+        if (long_attn) tk_launch_attention_long(partial, ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, d_scores, act_qd, true, s);
         else if (tiled_attn) tk_launch_attention_prefill(qbuf, kcache, vcache, d_seq, d_pos, d_tiles, nrows, h.n_head, h.n_kv_head, h.head_dim, l, max_seq, max_ctx, act_qd, s);
-        else tk_launch_attention(qbuf, partial, ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
+        else tk_launch_attention(qbuf, partial, ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
                                  h.head_dim, l, max_seq, max_ctx, act_qd, fused_attn, s);
         ks_res = enqueue_layer_tail(L, x, nrows);
     }
     last_ks_res = ks_res;
     if (!lm_head) { /* prompt rows whose logits nobody reads (K/V are already appended), or a pipeline stage that hands x on */
-        if (fold_out && l1 > l0) tk_launch_residual_fold(x, partial, ks_res, D, D, nrows, s);
+        if (fold_out && l1 > l0) tk_launch_residual_fold(x, partial, ks_res, D, pitch(D), D, nrows, s);
         return;
     }
     if (fuse) {
@@ -685,7 +683,7 @@ bool TkLlmSession::prefill(int nseq, int n_prompt, const int32_t* tokens, int32_
     }
     /* the last layer of the sampled rows alone: their queries over the caches, which now hold every position */
     stage(total, nseq);
-    tk_launch_attention(q_last, partial, h.ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nseq, h.n_head, h.n_kv_head, h.head_dim, last, max_seq, max_ctx,
+    tk_launch_attention(q_last, partial, h.ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nseq, h.n_head, h.n_kv_head, h.head_dim, last, max_seq, max_ctx,
                         act_qd, false, stream);
     enqueue_head(x_last, enqueue_layer_tail(model->layers[last], x_last, nseq), nseq);
     if (!launch_error.empty()) { error = launch_error; (void)hipStreamSynchronize(stream); return false; }
@@ -728,6 +726,7 @@ bool TkLlmSession::time_gemv(int layer, int which, int nrows, int iters, float* 
         }
         /* algorithmic bytes of one launch: the weight tiles once, the int8 activation images (+ block scales and sub-block sums) once,
          * the fp32 K-split partial outputs once */
+        a.slab_pitch = pitch(a.n_total);
         *bytes += (double)nrows * ((double)a.K + (double)a.K / 256.0 * (4.0 + 16.0)) + (double)a.ks * nrows * (double)a.n_total * 4.0;
         return a;
     };
@@ -796,14 +795,14 @@ bool TkLlmSession::time_attention(int nrows, int ctx, int iters, float* avg_ms, 
     const bool unfused = (uf && uf[0] == '1') || longf;
     auto launch = [&](int l) {
         if (longf) {
-            tk_launch_attention_long(partial, h.ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l % h.n_layer,
+            tk_launch_attention_long(partial, h.ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head, h.head_dim, l % h.n_layer,
                                      max_seq, max_ctx, d_scores, act_qd, true, stream);
             return;
         }
         if (unfused)
-            tk_launch_qkv_rope_append(partial, h.ks_qkv, QD + 2 * KVD, h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows, qbuf, kcache,
+            tk_launch_qkv_rope_append(partial, h.ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), h.n_head, h.n_kv_head, h.head_dim, rope_cos, rope_sin, d_seq, d_pos, nrows, qbuf, kcache,
                                       vcache, l % h.n_layer, max_seq, max_ctx, stream);
-        tk_launch_attention(qbuf, partial, h.ks_qkv, QD + 2 * KVD, rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
+        tk_launch_attention(qbuf, partial, h.ks_qkv, QD + 2 * KVD, pitch(QD + 2 * KVD), rope_cos, rope_sin, kcache, vcache, d_seq, d_pos, nrows, h.n_head, h.n_kv_head,
                             h.head_dim, l % h.n_layer, max_seq, max_ctx, act_qd, !unfused, stream);
     };
     *kv_bytes = (double)nrows * ctx * KVD * 2.0 * 2.0;

@@ -21,10 +21,10 @@ struct TkGemvArgs {
     TkGemvSeg seg[3];
     int nseg;
     int K;        /* reduction length, multiple of 256*ks */
-    int ks;       /* K-split count: partial sums land in out[ks][16][n_total] */
+    int ks;       /* K-split count: partial sums land in out + ksi * slab_pitch, [nrows][n_total] each */
     int n_total;  /* row pitch of `out`: the sum of rows over all segments of the matrix */
     int col0;     /* column of `out` where segment 0 starts (non-zero when a launch carries only some of the matrix's segments) */
-    int nrows;    /* live rows (<= TK_MAX_ROWS); rows 16.. use the second M-tile */
+    int nrows;    /* live rows (<= TK_PASS_ROWS); rows 16.. use the second M-tile */
     int swiglu;   /* 1 (only where tk_gemv_fuses_swiglu() says so): seg[0] = gate, seg[1] = up, out = h[nrows][n_total = d_ff] = silu(gate) * up */
     size_t aq_ts, ad_ts, abs_ts; /* M-tile strides of aq (bytes), ad (floats), abs (ints) */
     const int8_t* aq;
@@ -32,6 +32,7 @@ struct TkGemvArgs {
     const int8_t* abs; /* sub-block sums as (l, h) int8 images: [K/256][2][16][8] */
     const uint16_t* abs16; /* the same sums as two f16 images (sum = 2 hh + ll): [K/256][2][16][8] halves, M-tile stride abs_ts halves */
     float* out;
+    int64_t slab_pitch, fslab_pitch; /* floats between the slabs of out, of fslab */
     /* fuse != 0 (only where tk_gemv_fuses_producer() says so: passes of one or two rows, where a launch boundary costs more than the
      * producer's work repeated in every workgroup): the launch builds its int8 activation image in LDS itself and aq / ad / abs are unused.
      *   1: residual update + RMS norm + Q8 — k_rmsnorm_q8's arithmetic: row = fx_in + (the fks slabs of fslab, ascending; pitch
@@ -72,17 +73,17 @@ void tk_launch_repack(int type, const void* blocks, int64_t rows, int64_t K, uin
 /* step kernels */
 void tk_launch_embed(const void* embd, int type /* TK_TYPE_Q4_K or TK_TYPE_F16 */, int D, const int32_t* tok, int nrows, float* x, hipStream_t s);
 void tk_launch_synth_f16(uint64_t seed, uint64_t tensor_id, int64_t n, float scale, uint16_t* out, hipStream_t s);
-void tk_launch_rmsnorm_q8(float* x, const float* partial, int ks, int n_total_partial, const float* w, float eps, int D, int nrows,
+void tk_launch_rmsnorm_q8(float* x, const float* partial, int ks, int n_total_partial, int64_t pitch /* floats between slabs, here and below */, const float* w, float eps, int D, int nrows,
                           TkActQ8 out, hipStream_t s);
-void tk_launch_residual_fold(float* x, const float* partial, int ks, int n_total, int D, int nrows, hipStream_t s);
+void tk_launch_residual_fold(float* x, const float* partial, int ks, int n_total, int64_t pitch, int D, int nrows, hipStream_t s);
 void tk_launch_gemv(const TkGemvArgs& a, hipStream_t s);
-void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
+void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int64_t pitch, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
                                const float* rope_sin, const int32_t* seq, const int32_t* pos, int nrows, float* qbuf, uint16_t* kcache,
                                uint16_t* vcache, int layer, int max_seq, int max_ctx, hipStream_t s);
-void tk_launch_attention(const float* qbuf, const float* partial, int ks, int n_total, const float* rope_cos, const float* rope_sin,
+void tk_launch_attention(const float* qbuf, const float* partial, int ks, int n_total, int64_t pitch, const float* rope_cos, const float* rope_sin,
                          uint16_t* kcache, uint16_t* vcache, const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head,
                          int head_dim, int layer, int max_seq, int max_ctx, TkActQ8 out, bool fused, hipStream_t s);
-void tk_launch_swiglu_q8(const float* partial, int ks, int FF, int nrows, TkActQ8 out, hipStream_t s);
+void tk_launch_swiglu_q8(const float* partial, int ks, int64_t pitch, int FF, int nrows, TkActQ8 out, hipStream_t s);
 /* wide passes: the gate | up launch forms h = silu(gate) * up in its epilogue (half the slab bytes written and read back); then only the quantisation is left */
 /* rows up to which the norm / SwiGLU producer of a mat-vec launch runs inside it (TkGemvArgs::fuse) */
 #define TK_GEMV_FUSE_MAX_ROWS 2
@@ -102,7 +103,7 @@ void tk_attention_note_session(int device, int delta);
 TkAttentionPlan tk_attention_plan(int nrows, int n_head, int n_kv_head, int head_dim, int max_ctx, bool fused);
 
 /* multi-position passes (prompt chunks): 16 rows of a sequence per workgroup on the fp32 matrix pipe, bit-identical to k_attention's non-fused
- * form.  tiles: 1 + TK_MAX_ROWS ints built by tk_launch_att_tiles from the pass's sequence ids (once per pass); the cache must already hold
+ * form.  tiles: 1 + nrows ints built by tk_launch_att_tiles from the pass's sequence ids (once per pass); the cache must already hold
  * the pass's own K / V rows (tk_launch_qkv_rope_append) */
 bool tk_attention_prefill_applies(int n_head, int n_kv_head, int head_dim);
 void tk_launch_att_tiles(const int32_t* seq, int nrows, int32_t* tiles, hipStream_t s);
@@ -123,7 +124,7 @@ size_t tk_attention_long_scratch_floats(int n_head, int head_dim, int max_ctx); 
 /* where such a launch leaves the classes' outputs [row][head][4][head_dim] and denominators [row][head][4]; join = false: its consumer joins them (TkGemvArgs::fuse 3) */
 struct TkAttentionParts { float *pv, *l; };
 TkAttentionParts tk_attention_long_parts(float* scores, int n_head, int head_dim, int max_ctx);
-void tk_launch_attention_long(const float* partial, int ks, int n_total, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
+void tk_launch_attention_long(const float* partial, int ks, int n_total, int64_t pitch, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
                               const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head, int head_dim, int layer, int max_seq, int max_ctx,
                               float* scores, TkActQ8 out, bool join, hipStream_t s);
 size_t tk_gemv_lds_bytes(int K, int ks, int mtiles);

@@ -288,7 +288,7 @@ __device__ __forceinline__ TkQuantBlock quant_block(int b, int nrows, int pieces
  * chains read the finished row back from LDS, so how many threads loaded it does not enter the result.
  * ------------------------------------------------------------------------------------------ */
 #define TK_RMS_MAX_KS 8
-__global__ __launch_bounds__(1024) void k_rmsnorm_q8(float* __restrict__ x, const float* __restrict__ partial, int ks, int n_total,
+__global__ __launch_bounds__(1024) void k_rmsnorm_q8(float* __restrict__ x, const float* __restrict__ partial, int ks, int n_total, int64_t pitch,
                                                       const float* __restrict__ w, float eps, int D, TkActQ8 out) {
     extern __shared__ float sh[]; /* D floats + 4 */
     float* hbuf = sh;
@@ -302,7 +302,7 @@ __global__ __launch_bounds__(1024) void k_rmsnorm_q8(float* __restrict__ x, cons
             v4f p[TK_RMS_MAX_KS];
 #pragma unroll
             for (int s = 0; s < TK_RMS_MAX_KS; ++s)
-                if (s < ks) p[s] = *(const v4f*)(partial + ((int64_t)s * TK_SLAB_ROWS + r) * n_total + 4 * g);
+                if (s < ks) p[s] = *(const v4f*)(partial + s * pitch + (int64_t)r * n_total + 4 * g);
             v4f o = p[0];
 #pragma unroll
             for (int s = 1; s < TK_RMS_MAX_KS; ++s)
@@ -348,27 +348,27 @@ __global__ __launch_bounds__(1024) void k_rmsnorm_q8(float* __restrict__ x, cons
 
 /* x += (p_0 + p_1 + ... + p_{ks-1}), exactly the residual update k_rmsnorm_q8 performs before it normalises: used where the
  * residual stream leaves this GPU (pipeline-stage boundary) and the next layer's norm runs elsewhere */
-__global__ __launch_bounds__(256) void k_residual_fold(float* __restrict__ x, const float* __restrict__ partial, int ks, int n_total, int D) {
+__global__ __launch_bounds__(256) void k_residual_fold(float* __restrict__ x, const float* __restrict__ partial, int ks, int n_total, int64_t pitch, int D) {
     const int r = blockIdx.y;
     const int g = blockIdx.x * 256 + threadIdx.x;
     if (4 * g >= D) return;
     v4f o = *(const v4f*)(partial + (int64_t)r * n_total + 4 * g);
-    for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + ((int64_t)s * TK_SLAB_ROWS + r) * n_total + 4 * g);
+    for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + s * pitch + (int64_t)r * n_total + 4 * g);
     v4f* xp = (v4f*)(x + (int64_t)r * D + 4 * g);
     *xp = *xp + o;
 }
 
-void tk_launch_residual_fold(float* x, const float* partial, int ks, int n_total, int D, int nrows, hipStream_t s) {
-    hipLaunchKernelGGL(k_residual_fold, dim3((D / 4 + 255) / 256, nrows), dim3(256), 0, s, x, partial, ks, n_total, D);
+void tk_launch_residual_fold(float* x, const float* partial, int ks, int n_total, int64_t pitch, int D, int nrows, hipStream_t s) {
+    hipLaunchKernelGGL(k_residual_fold, dim3((D / 4 + 255) / 256, nrows), dim3(256), 0, s, x, partial, ks, n_total, pitch, D);
 }
 
-void tk_launch_rmsnorm_q8(float* x, const float* partial, int ks, int n_total_partial, const float* w, float eps, int D, int nrows,
+void tk_launch_rmsnorm_q8(float* x, const float* partial, int ks, int n_total_partial, int64_t pitch, const float* w, float eps, int D, int nrows,
                           TkActQ8 out, hipStream_t s) {
     int nthr = D / 4; /* one thread per 16-byte group of the row, 256 .. 1024 */
     nthr = nthr < 256 ? 256 : nthr > 1024 ? 1024 : (nthr + 255) / 256 * 256;
     /* (round 6: four-wave workgroups while several decode streams share the device — so that the norm fits beside other streams' resident mat-vec
      * workgroups instead of waiting for one to retire — measured SLOWER: 3.99 against 3.90 ms per step and group at 3 x 16 rows, profiles/r06_northstar_explore.txt) */
-    hipLaunchKernelGGL(k_rmsnorm_q8, dim3(nrows), dim3(nthr), (D + 4) * sizeof(float), s, x, partial, ks, n_total_partial, w, eps, D, out);
+    hipLaunchKernelGGL(k_rmsnorm_q8, dim3(nrows), dim3(nthr), (D + 4) * sizeof(float), s, x, partial, ks, n_total_partial, pitch, w, eps, D, out);
 }
 
 /* ------------------------------------------------------------------------------------------
@@ -662,7 +662,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                         v4f p[TK_RMS_MAX_KS];
 #pragma unroll
                         for (int sl = 0; sl < TK_RMS_MAX_KS; ++sl)
-                            if (sl < a.fks) p[sl] = *(const v4f*)(a.fslab + ((int64_t)sl * TK_SLAB_ROWS + r) * a.fn_total + 4 * gi);
+                            if (sl < a.fks) p[sl] = *(const v4f*)(a.fslab + sl * a.fslab_pitch + (int64_t)r * a.fn_total + 4 * gi);
                         v4f o = p[0];
 #pragma unroll
                         for (int sl = 1; sl < TK_RMS_MAX_KS; ++sl)
@@ -730,7 +730,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
 #pragma unroll
                         for (int sl = 0; sl < TK_RMS_MAX_KS; ++sl)
                             if (sl < a.fks) {
-                                const float* row = a.fslab + ((int64_t)sl * TK_SLAB_ROWS + r) * (2 * (int64_t)FF);
+                                const float* row = a.fslab + sl * a.fslab_pitch + r * (2 * (int64_t)FF);
                                 pg[sl][0] = *(const v4f*)(row + 8 * c); pg[sl][1] = *(const v4f*)(row + 8 * c + 4);
                                 pu[sl][0] = *(const v4f*)(row + FF + 8 * c); pu[sl][1] = *(const v4f*)(row + FF + 8 * c + 4);
                             }
@@ -847,7 +847,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
             /* default-policy stores: the <= 1 MB of slabs of a narrow pass stay in L2 / the Infinity Cache for the consumer kernel, which is one
              * load latency long (decode step 2.277 -> 2.207 ms at 16 rows, 2.108 -> 2.038 ms at 1 row against non-temporal stores,
              * profiles/r03_smallbatch_variants.txt); the wide kernels keep non-temporal stores (29 MB per launch would only evict) */
-            if (row < a.nrows) a.out[((size_t)ksi * TK_SLAB_ROWS + row) * a.n_total + n] = acc[m][r];
+            if (row < a.nrows) a.out[ksi * a.slab_pitch + (int64_t)row * a.n_total + n] = acc[m][r];
         }
 }
 
@@ -1126,7 +1126,7 @@ __global__ __launch_bounds__(NT == 2 ? 256 : 512) void k_gemm_w4a8(TkGemvArgs a,
             for (int r = 0; r < 4; ++r) {
                 const int mt = rot == 0 ? m : (m < MT / 2 ? m + rot : m - rot); /* register slot m holds M-tile m ^ rot (the half-swap: MT = 6 is no power of two) */
                 const int row = mt * TK_ROW_SLOTS + 4 * g + r;
-                if (row < a.nrows) __builtin_nontemporal_store(acc[w][m][r], &a.out[((size_t)ksi * TK_SLAB_ROWS + row) * a.n_total + n]);
+                if (row < a.nrows) __builtin_nontemporal_store(acc[w][m][r], &a.out[ksi * a.slab_pitch + (int64_t)row * a.n_total + n]);
             }
     }
 }
@@ -1545,7 +1545,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
                 const int rl = 8 * i + (lane >> 3);
                 const v4f v = *(const v4f*)(sp + rl * 32 + 4 * (lane & 7));
                 const int row = (t32_0 + t) * 32 + rl;
-                if (row < a.nrows) *(v4f*)&a.out[((size_t)ksi * TK_SLAB_ROWS + row) * a.n_total + n0] = v;
+                if (row < a.nrows) *(v4f*)&a.out[ksi * a.slab_pitch + (int64_t)row * a.n_total + n0] = v;
             }
         }
     }
@@ -1681,9 +1681,8 @@ template <int KS> __device__ __forceinline__ float2 sum_slabs_pair(const float* 
     for (int s = 1; s < KS; ++s) { o.x = o.x + v[s].x; o.y = o.y + v[s].y; }
     return o;
 }
-__device__ __forceinline__ float2 sum_partials_pair(const float* partial, int ks, int n_total, int row, int col) {
+__device__ __forceinline__ float2 sum_partials_pair(const float* partial, int ks, int n_total, int64_t pitch, int row, int col) {
     const float* p = partial + (int64_t)row * n_total;
-    const int64_t pitch = (int64_t)TK_SLAB_ROWS * n_total;
     switch (ks) {
     case 1: return sum_slabs_pair<1>(p, pitch, (uint32_t)col);
     case 2: return sum_slabs_pair<2>(p, pitch, (uint32_t)col);
@@ -1696,7 +1695,7 @@ __device__ __forceinline__ float2 sum_partials_pair(const float* partial, int ks
     }
 }
 
-__global__ void k_qkv_rope_append(const float* partial, int ks, int n_total, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
+__global__ void k_qkv_rope_append(const float* partial, int ks, int n_total, int64_t pitch, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
                                   const float* rope_sin, const int32_t* seq, const int32_t* pos, float* qbuf, uint16_t* kcache,
                                   uint16_t* vcache, int layer, int max_seq, int max_ctx) {
     const int kvh = blockIdx.x, r = blockIdx.y;
@@ -1710,7 +1709,7 @@ __global__ void k_qkv_rope_append(const float* partial, int ks, int n_total, int
         const int hsel = idx / half, i = idx % half;
         const int col = hsel < grp ? (kvh * grp + hsel) * head_dim + 2 * i : (hsel == grp ? QD : QD + KVD) + kvh * head_dim + 2 * i;
         const float c = cs[i], sv = sn[i];
-        const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+        const float2 ab = sum_partials_pair(partial, ks, n_total, pitch, r, col);
         const float2 rot = {tk_fmaf(-ab.y, sv, ab.x * c), tk_fmaf(ab.x, sv, ab.y * c)};
         if (hsel < grp) *(float2*)(qbuf + (int64_t)r * QD + col) = rot;
         else if (hsel == grp) *(uint32_t*)(kcache + cbase + 2 * i) = (uint32_t)tk_f32_to_f16(rot.x) | ((uint32_t)tk_f32_to_f16(rot.y) << 16);
@@ -1718,11 +1717,11 @@ __global__ void k_qkv_rope_append(const float* partial, int ks, int n_total, int
     }
 }
 
-void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
+void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int64_t pitch, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
                                const float* rope_sin, const int32_t* seq, const int32_t* pos, int nrows, float* qbuf, uint16_t* kcache,
                                uint16_t* vcache, int layer, int max_seq, int max_ctx, hipStream_t s) {
     const int items = (n_head / n_kv_head + 2) * (head_dim / 2); /* a multiple of 32 */
-    hipLaunchKernelGGL(k_qkv_rope_append, dim3(n_kv_head, nrows), dim3(items < 512 ? (items + 63) / 64 * 64 : 512), 0, s, partial, ks, n_total, n_head, n_kv_head, head_dim, rope_cos,
+    hipLaunchKernelGGL(k_qkv_rope_append, dim3(n_kv_head, nrows), dim3(items < 512 ? (items + 63) / 64 * 64 : 512), 0, s, partial, ks, n_total, pitch, n_head, n_kv_head, head_dim, rope_cos,
                        rope_sin, seq, pos, qbuf, kcache, vcache, layer, max_seq, max_ctx);
 }
 
@@ -1772,7 +1771,7 @@ template <int GQ, bool FUSED, int HD /* head_dim when it is 64 or 128 (loops unr
 #ifndef TK_ATT_WAVES
 #define TK_ATT_WAVES 1
 #endif
-__global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __restrict__ qbuf, const float* __restrict__ partial, int ks, int n_total,
+__global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __restrict__ qbuf, const float* __restrict__ partial, int ks, int n_total, int64_t pitch,
                                                     const float* __restrict__ rope_cos, const float* __restrict__ rope_sin,
                                                     uint16_t* __restrict__ kcache, uint16_t* __restrict__ vcache, const int32_t* __restrict__ seq,
                                                     const int32_t* __restrict__ pos, int n_head, int n_kv_head, int head_dim_rt, int layer, int max_seq,
@@ -1830,7 +1829,7 @@ __global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __
             const int hsel = idx / half, i = idx % half;
             const int col = hsel < GQ ? (hb * GQ + hsel) * head_dim + 2 * i : (hsel == GQ ? QD : QD + KVD) + kvh * head_dim + 2 * i;
             const float c = cs[i], sv = sn[i];
-            const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+            const float2 ab = sum_partials_pair(partial, ks, n_total, pitch, r, col);
             const float2 rot = {tk_fmaf(-ab.y, sv, ab.x * c), tk_fmaf(ab.x, sv, ab.y * c)};
             if (hsel < GQ) {
                 *(float2*)(qs + hsel * head_dim + 2 * i) = rot;
@@ -1992,7 +1991,7 @@ __global__ __launch_bounds__(256, TK_ATT_WAVES) void k_attention(const float* __
  * value phase (wave = one head x one of the four canonical interleaved partial sums), combine, quantise: six barriers.
  * Workgroup = (row, two query heads of one KV group); grid (n_head / 2, rows).
  * ------------------------------------------------------------------------------------------ */
-__global__ __launch_bounds__(1024) void k_attention_narrow(const float* __restrict__ partial, int ks, int n_total, const float* __restrict__ rope_cos,
+__global__ __launch_bounds__(1024) void k_attention_narrow(const float* __restrict__ partial, int ks, int n_total, int64_t pitch, const float* __restrict__ rope_cos,
                                                             const float* __restrict__ rope_sin, uint16_t* __restrict__ kcache, uint16_t* __restrict__ vcache,
                                                             const int32_t* __restrict__ seq, const int32_t* __restrict__ pos, int n_head, int n_kv_head, int layer,
                                                             int max_seq, int max_ctx, int cap, TkActQ8 out) {
@@ -2038,7 +2037,7 @@ __global__ __launch_bounds__(1024) void k_attention_narrow(const float* __restri
         const int hsel = t / half, i = t % half;
         const int col = hsel < GQ ? (hb * GQ + hsel) * HD + 2 * i : (hsel == GQ ? QD : QD + KVD) + kvh * HD + 2 * i;
         const float c = cs[i], sv = sn[i];
-        const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+        const float2 ab = sum_partials_pair(partial, ks, n_total, pitch, r, col);
         const float2 rot = {tk_fmaf(-ab.y, sv, ab.x * c), tk_fmaf(ab.x, sv, ab.y * c)};
         if (hsel < GQ) {
             *(float2*)(qs + hsel * HD + 2 * i) = rot;
@@ -2450,7 +2449,7 @@ __global__ __launch_bounds__((256 / HD) * 256) void k_attention_prefill(const fl
  * The session takes this form for passes of at most TK_LONG_ATT_MAX_ROWS rows that reach tk_long_att_min_pos(rows) (tk_llm_kernels.h).
  * ------------------------------------------------------------------------------------------ */
 template <int HD>
-__global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict__ partial, int ks, int n_total, const float* __restrict__ rope_cos,
+__global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict__ partial, int ks, int n_total, int64_t pitch, const float* __restrict__ rope_cos,
                                                          const float* __restrict__ rope_sin, uint16_t* __restrict__ kcache, uint16_t* __restrict__ vcache,
                                                          const int32_t* __restrict__ seq, const int32_t* __restrict__ pos, int n_head, int n_kv_head, int layer,
                                                          int max_seq, int max_ctx, float* __restrict__ scores) {
@@ -2483,7 +2482,7 @@ __global__ __launch_bounds__(256) void k_att_scores_long(const float* __restrict
         for (int idx = t; idx < (GQ + (last ? 2 : 0)) * HALF; idx += 256) {
             const int hsel = idx / HALF, i = idx % HALF;
             const int col = hsel < GQ ? (kvh * GQ + hsel) * HD + 2 * i : (hsel == GQ ? QD : QD + KVD) + kvh * HD + 2 * i;
-            const float2 ab = sum_partials_pair(partial, ks, n_total, r, col);
+            const float2 ab = sum_partials_pair(partial, ks, n_total, pitch, r, col);
             const float a = ab.x, bb = ab.y;
             if (hsel < GQ) {
                 qs[hsel * HD + 2 * i] = tk_fmaf(-bb, sn[i], a * cs[i]);
@@ -2658,7 +2657,7 @@ TkAttentionParts tk_attention_long_parts(float* scores, int n_head, int head_dim
     return TkAttentionParts{pv, pv + (size_t)TK_LONG_ATT_MAX_ROWS * n_head * TK_ATT_TSPLIT * head_dim};
 }
 
-void tk_launch_attention_long(const float* partial, int ks, int n_total, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
+void tk_launch_attention_long(const float* partial, int ks, int n_total, int64_t pitch, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
                               const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head, int head_dim, int layer, int max_seq, int max_ctx,
                               float* scores, TkActQ8 out, bool join, hipStream_t s) {
     const dim3 gs(n_kv_head, (max_ctx + 63) / 64, nrows);
@@ -2668,12 +2667,12 @@ void tk_launch_attention_long(const float* partial, int ks, int n_total, const f
     const int slots = nrows > 4 ? 2 : 3; /* 32 KB: the four workgroups a CU of eight rows are resident together (calls with two / three: 8 rows at 900 positions 2.62 / 2.79 ms, at 3000 3.37 / 3.74, 6 at 900 2.54 / 2.56) */
     const size_t lds = (size_t)slots * TK_PV_ROWS * head_dim * 2 + ((size_t)(max_ctx + 3) / 4 + TK_PV_ROWS) * sizeof(float);
     if (head_dim == 128) {
-        hipLaunchKernelGGL((k_att_scores_long<128>), gs, dim3(256), 0, s, partial, ks, n_total, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
+        hipLaunchKernelGGL((k_att_scores_long<128>), gs, dim3(256), 0, s, partial, ks, n_total, pitch, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
                            max_seq, max_ctx, scores);
         hipLaunchKernelGGL((slots == 2 ? k_att_pv_chain<128, 2> : k_att_pv_chain<128, 3>), gc, dim3(64), lds, s, scores, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pv_part, l_part);
         if (join) hipLaunchKernelGGL((k_att_pv_join<128>), dim3(n_head / 2, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
     } else {
-        hipLaunchKernelGGL((k_att_scores_long<64>), gs, dim3(256), 0, s, partial, ks, n_total, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
+        hipLaunchKernelGGL((k_att_scores_long<64>), gs, dim3(256), 0, s, partial, ks, n_total, pitch, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer,
                            max_seq, max_ctx, scores);
         hipLaunchKernelGGL((slots == 2 ? k_att_pv_chain<64, 2> : k_att_pv_chain<64, 3>), gc, dim3(64), lds, s, scores, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pv_part, l_part);
         if (join) hipLaunchKernelGGL((k_att_pv_join<64>), dim3(n_head / 4, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
@@ -2801,19 +2800,19 @@ TkAttentionPlan tk_attention_plan(int nrows, int n_head, int n_kv_head, int head
     return pl;
 }
 
-void tk_launch_attention(const float* qbuf, const float* partial, int ks, int n_total, const float* rope_cos, const float* rope_sin,
+void tk_launch_attention(const float* qbuf, const float* partial, int ks, int n_total, int64_t pitch, const float* rope_cos, const float* rope_sin,
                          uint16_t* kcache, uint16_t* vcache, const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head,
                          int head_dim, int layer, int max_seq, int max_ctx, TkActQ8 out, bool fused, hipStream_t s) {
     const TkAttentionPlan pl = tk_attention_plan(nrows, n_head, n_kv_head, head_dim, max_ctx, fused);
     if (pl.kernel == 1) {
-        hipLaunchKernelGGL(k_attention_narrow, dim3(n_head / 2, nrows), dim3(1024), pl.lds_bytes, s, partial, ks, n_total, rope_cos, rope_sin, kcache,
+        hipLaunchKernelGGL(k_attention_narrow, dim3(n_head / 2, nrows), dim3(1024), pl.lds_bytes, s, partial, ks, n_total, pitch, rope_cos, rope_sin, kcache,
                            vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx, pl.chunk, out);
         return;
     }
     const int gq = pl.gq, chunk = pl.chunk;
     const size_t lds = pl.lds_bytes;
 #define TK_ATT_LAUNCH_CH(G, F, H, C, S)                                                                                                       \
-    hipLaunchKernelGGL((k_attention<G, F, H, C, S>), dim3(n_head / gq, nrows), dim3(256), lds, s, qbuf, partial, ks, n_total, rope_cos, rope_sin, kcache, \
+    hipLaunchKernelGGL((k_attention<G, F, H, C, S>), dim3(n_head / gq, nrows), dim3(256), lds, s, qbuf, partial, ks, n_total, pitch, rope_cos, rope_sin, kcache, \
                        vcache, seq, pos, n_head, n_kv_head, head_dim, layer, max_seq, max_ctx, out)
 #define TK_ATT_LAUNCH_HD(G, F, H) do { if (chunk == 32) TK_ATT_LAUNCH_CH(G, F, H, 32, TK_ATT_WIDE_SLOTS); else if (chunk == 128 && G <= 2 && H != 0) TK_ATT_LAUNCH_CH((G <= 2 ? G : 2), F, (H ? H : 128), 128, 2); else TK_ATT_LAUNCH_CH(G, F, H, 64, 2); } while (0)
 #define TK_ATT_LAUNCH(G, F) do { if (head_dim == 128) TK_ATT_LAUNCH_HD(G, F, 128); else if (head_dim == 64) TK_ATT_LAUNCH_HD(G, F, 64); else TK_ATT_LAUNCH_HD(G, F, 0); } while (0)
@@ -2833,7 +2832,7 @@ void tk_launch_attention(const float* qbuf, const float* partial, int ks, int n_
 /* KSM = the most K-split slabs an instantiation handles: the slab loads are held in registers before the first add, and the gate | up
  * projection of the canonical plan has ONE slab — with room for eight the kernel needs 130 registers (3 waves per SIMD), with one 40 */
 template <int KSM>
-__global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks, int FF, int nrows, TkActQ8 out) {
+__global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks, int64_t pitch, int FF, int nrows, TkActQ8 out) {
     const TkQuantBlock qb = quant_block(blockIdx.x, nrows, (FF / 8 + 255) / 256);
     const int r = qb.row, c = qb.piece * 256 + threadIdx.x;
     if (r >= nrows || c >= FF / 8) return; /* FF/8 is a multiple of 32: whole half-waves drop out together */
@@ -2844,7 +2843,7 @@ __global__ __launch_bounds__(256) void k_swiglu_q8(const float* partial, int ks,
 #pragma unroll
         for (int s = 0; s < KSM; ++s)
             if (s < ks) {
-                const float* row = partial + ((int64_t)s * TK_SLAB_ROWS + r) * (2 * (int64_t)FF);
+                const float* row = partial + s * pitch + r * (2 * (int64_t)FF);
                 pg[s][0] = *(const v4f*)(row + 8 * c); pg[s][1] = *(const v4f*)(row + 8 * c + 4);
                 pu[s][0] = *(const v4f*)(row + FF + 8 * c); pu[s][1] = *(const v4f*)(row + FF + 8 * c + 4);
             }
@@ -2878,10 +2877,10 @@ bool tk_gemv_fuses_swiglu(int nrows, int ks, int type_gate, int type_up) {
     return nrows >= tk_g32_from() && ks == 1 && type_gate == type_up && (type_gate == TK_TYPE_Q4_K || type_gate == TK_TYPE_Q6_K); /* the 32x32x32 kernel's epilogue */
 }
 
-void tk_launch_swiglu_q8(const float* partial, int ks, int FF, int nrows, TkActQ8 out, hipStream_t s) {
+void tk_launch_swiglu_q8(const float* partial, int ks, int64_t pitch, int FF, int nrows, TkActQ8 out, hipStream_t s) {
     const dim3 grid(quant_blocks(nrows, (FF / 8 + 255) / 256));
-    if (ks == 1) hipLaunchKernelGGL((k_swiglu_q8<1>), grid, dim3(256), 0, s, partial, ks, FF, nrows, out);
-    else hipLaunchKernelGGL((k_swiglu_q8<TK_RMS_MAX_KS>), grid, dim3(256), 0, s, partial, ks, FF, nrows, out);
+    if (ks == 1) hipLaunchKernelGGL((k_swiglu_q8<1>), grid, dim3(256), 0, s, partial, ks, pitch, FF, nrows, out);
+    else hipLaunchKernelGGL((k_swiglu_q8<TK_RMS_MAX_KS>), grid, dim3(256), 0, s, partial, ks, pitch, FF, nrows, out);
 }
 
 /* ------------------------------------------------------------------------------------------

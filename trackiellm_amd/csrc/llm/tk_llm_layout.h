@@ -53,9 +53,8 @@
 #define TK_MAX_ROWS (TK_ROW_SLOTS * TK_MAX_TILES)
 /* Rows of a whole prompt's pass (TkLlmSession::prefill), several times a caller's pass: a launch of 256 rows fills the chip's workgroup slots to 0.5 (o) .. 0.875 (gate | up)
  * and pays its ramp and its tail for those rows alone.  256 prompts of 32 positions, 32 layers 4096 wide, in passes of 256, 512, 1024, 2048 rows: 216, 191, 175, 166 ms.
- * K-split slabs are TK_SLAB_ROWS rows apart in every pass. */
+ * K-split slabs are as many rows apart as a session's passes have at most: where those of 16 rows were 16 apart, the products of a step took 2 % longer. */
 #define TK_PASS_ROWS 2048
-#define TK_SLAB_ROWS TK_PASS_ROWS
 #define TK_SPARE_TILES 8 /* M-tiles behind a pass's last that the images hold: a part of 96 rows stages eight tiles */
 
 /* per M-tile sizes; tile m of a buffer starts at m * (these) */

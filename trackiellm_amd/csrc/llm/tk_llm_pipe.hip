@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256) void k_pipe_take_x(const TkPipeBlock* mine, Tk
 /* producer, last kernel of a pass: x + (p_0 + ... + p_{ks-1}) — the pending residual update, slabs added in ascending order exactly as
  * k_rmsnorm_q8 / k_residual_fold do — stored straight into a slot of the NEXT stage's mailbox; the last workgroup to arrive publishes the
  * slot.  grid (d_model / 1024, nrows) */
-__global__ __launch_bounds__(256) void k_pipe_send_x(const float* __restrict__ x, const float* __restrict__ partial, int ks, int n_total, int D, TkPipeBlock* next,
+__global__ __launch_bounds__(256) void k_pipe_send_x(const float* __restrict__ x, const float* __restrict__ partial, int ks, int n_total, int64_t pitch, int D, TkPipeBlock* next,
                                                       const TkPipeBlock* mine, TkPipeState* st, int slot_floats, int f16) {
     __shared__ int ok;
     const unsigned long long seq = st->sent_x + 1;
@@ -104,7 +104,7 @@ __global__ __launch_bounds__(256) void k_pipe_send_x(const float* __restrict__ x
         v4f v = *(const v4f*)(x + (int64_t)r * D + 4 * g);
         if (partial) {
             v4f o = *(const v4f*)(partial + (int64_t)r * n_total + 4 * g);
-            for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + ((int64_t)s * TK_SLAB_ROWS + r) * n_total + 4 * g);
+            for (int s = 1; s < ks; ++s) o = o + *(const v4f*)(partial + s * pitch + (int64_t)r * n_total + 4 * g);
             v = v + o;
         }
         const int64_t at = (int64_t)r * (D / 4) + g;
@@ -426,7 +426,7 @@ void TkLlmPipe::enqueue_stage(int nrows, bool take_ids, bool head, bool advance_
     s_->enqueue_range(nrows, l0, l1, first, false, sample, fused_attn);
     if (!last) {
         const float* partial = l1 > l0 ? s_->partial : nullptr;
-        hipLaunchKernelGGL(k_pipe_send_x, dim3((D / 4 + 255) / 256, nrows), dim3(256), 0, st, s_->x, partial, s_->last_ks_res, D, D, next_, mine_, st_, slot_floats,
+        hipLaunchKernelGGL(k_pipe_send_x, dim3((D / 4 + 255) / 256, nrows), dim3(256), 0, st, s_->x, partial, s_->last_ks_res, D, s_->pitch(D), D, next_, mine_, st_, slot_floats,
                            f16_ ? 1 : 0);
     } else if (sample && n_stages > 1) {
         hipLaunchKernelGGL(k_pipe_send_ids, dim3(1), dim3(256), 0, st, s_->d_tok, nrows, next_, mine_, st_);

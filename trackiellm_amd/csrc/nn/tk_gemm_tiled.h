@@ -8,7 +8,7 @@
  *     Producers either write it directly (the LLM's norm / activation kernels, csrc/llm/tk_llm_kernels.hip: quantize_chunk8) or
  *     tk_launch_pack_a() converts a row-major matrix.
  * Contract: per K-split slab one fp32 chain over k ascending from zero (the same chain k_gemm_f32 evaluates on the 32x32x2 MFMA, so the
- * two kernels agree bit for bit).  ks > 1: out[ks][TK_MAX_ROWS rows][ldc] partial slabs, summed in ascending order by the consumer
+ * two kernels agree bit for bit).  ks > 1: out[ks][slab_rows][ldc] partial slabs, summed in ascending order by the consumer
  * (LLM path); ks == 1: out[row][ldc] with the optional epilogue  v = act(acc + bias[n]) + residual[row][n].
  *
  * A wave owns one weight row tile of one K range and streams it as one piece per 32 k, PF pieces in flight in registers; a piece feeds
@@ -37,7 +37,7 @@ struct TkTiledGemm {
     int ldc;                 /* row pitch of out (and of the K-split slabs) */
     int n_valid;             /* columns actually stored (N; the last tile may be padding) */
     int nrows;
-    int slab_rows;           /* rows per K-split slab (ks > 1), at least nrows: TK_SLAB_ROWS of the LLM path */
+    int slab_rows;           /* rows per K-split slab (ks > 1), at least nrows */
     const float* a_img;
     size_t a_ts;             /* floats between M-tiles of the image = 16 K */
     float* out;
