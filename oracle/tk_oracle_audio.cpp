@@ -179,6 +179,7 @@ struct CpuAudioOps {
     bool takes_images(const float*, const float*, const float*, int, int, int) { return false; }
     void attend_images(const float*, const float*, const float*, float*, int, int, int, int) {}
     bool attend_fused(const float*, const float*, const float*, float*, int, int, int, int64_t, int64_t, int, int) { return false; }
+    void settle() {}
     void softmax_rows(float* x, int rows, int cols, int ld) {
         for (int r = 0; r < rows; ++r) {
             float* xr = x + (int64_t)r * ld;

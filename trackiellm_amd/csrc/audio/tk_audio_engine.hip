@@ -555,6 +555,7 @@ struct TkAudioGpuOps {
         norm.in_products = !long_ok && norm_fits(rows, D); /* a decoder step's */
         pk.A = y; pk.M = rows; pk.K = D; pk.lda = D; pk.img = nullptr; pk.mark = a->arena_used; pk.live = true;
     }
+    void settle() { drop_image(); }
     void softmax_rows(float* x, int rows, int cols, int ld) { drop_image(); tk_launch_softmax_rows(x, rows, cols, ld, s); }
     bool attend1(const float* q, const float* k, const float* v, float* out, int B, int Tk, int64_t q_bstride, int64_t kv_bstride, int kv_row, int d, int nh, float* scores, int pitch) {
         drop_image();
@@ -652,6 +653,7 @@ struct TkAudioSizeOps {
     }
     void im2col1d(const float*, int, int, int, int, int, int, int, float*) {}
     void layernorm(const float*, int rows, int D, const float*, const float*, float*) { image(rows, D); }
+    void settle() {}
     void softmax_rows(float*, int, int, int) {}
     bool attend1(const float*, const float*, const float*, float*, int B, int, int64_t, int64_t, int, int d, int, float*, int) { image(B, d); return true; }
     bool takes_images(const float*, const float*, const float*, int, int, int) { return false; }

@@ -12,6 +12,7 @@
  *   void gemm(const TkGemm&);
  *   void im2col1d(const float* x, int B, int T, int C, int ldx, int kw, int stride, int pad, float* col);
  *   void layernorm(const float* x, int rows, int D, const float* w, const float* b, float* y);
+ *   void settle(): everything before it is written where it was asked for (a backend may let outputs wait for their first reader among these ops and pass them on in another form)
  *   void softmax_rows(float* x, int rows, int cols, int ld);
  *   bool attend1(...): optional fused form of attention() for one query row per sequence (same arithmetic); false = not provided
  *   bool takes_images(...) / attend_images(...): optional one-kernel form of attention() for all rows of an encoder layer, on q and k that
@@ -267,6 +268,7 @@ struct TkWhisperGraph {
         }
         float* y = o.alloc((size_t)R * d);
         o.layernorm(x, R, d, W[m.enc_ln_w], W[m.enc_ln_b], y);
+        o.settle(); /* the caller's: rows */
         return y;
     }
 
