@@ -512,6 +512,7 @@ void TkLlmSession::enqueue_range(int nrows, int l0, int l1, bool embed, bool fol
     } else enqueue_head(x, l1 > l0 ? ks_res : 0, nrows);
 }
 
+/* fitted to passes of 256 rows; at the 2048 of a whole prompt it has not been measured anew */
 #ifndef TK_TILED_ATT_MIN_POS
 #define TK_TILED_ATT_MIN_POS 128
 #endif

@@ -1461,7 +1461,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
 
-    /* ring staging: of the half's eight 16-row M-tiles, `pair` and `pair + 4` belong to this wave.  The int8 image (4 x 1 KiB pieces per
+    /* ring staging: of the part's eight 16-row M-tiles, `pair` and `pair + 4` belong to this wave.  The int8 image (4 x 1 KiB pieces per
      * tile, every lane takes part: no exec masking, so the issue can sit between the MFMA phases of the tile loop) in four parts of two
      * pieces; the f16 sub-block sums (32 lanes) and the block scales (4 lanes) separately at the top of a block */
     /* rows of the pass as 32-row tiles: each part takes MTW of them (rows beyond the pass are computed on whatever the image holds and never stored) */

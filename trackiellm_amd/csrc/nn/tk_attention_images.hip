@@ -14,9 +14,8 @@ typedef float v4f __attribute__((ext_vector_type(4)));
  *   softmax: the tree's levels 32 .. 4 are inside a lane, 2 and 1 between the four lanes of a query, the quarters meet in LDS.  Scores are
  *     held unscaled: the scale 1 / 8 is a power of two, so (x / 8) - m rounds once, as one fma (a subnormal x / 8 does too, up to differences
  *     below 2^-100, whose exponential is 1 either way).  Division by the row's sum: y = RN(1 / sum), yl what is missing of it, q = e y + e yl
- *     within an ulp, and one correction by the exact remainder rounds it correctly (1.6e9 pairs, among them mantissas of nearly all ones and zeros,
- *     compared with the division on a CPU: all equal) — as long as no remainder is subnormal (e >= 2^-100); the
- *     division itself otherwise.
+ *     within an ulp, and q + y (e - q sum) rounds correctly: Markstein's theorem (1990) for a correctly rounded reciprocal and an exact remainder.
+ *     That is so as long as no remainder is subnormal (e >= 2^-100); the division itself otherwise.
  *   output: P goes through LDS 256 keys at a time, two buffers; wave w makes columns 16 w .. 16 w + 15, one chain over all keys.
  * Bound by the fp32 matrix pipe, which vector instructions share: at 16 rows x 1500 keys 24.3 k cycles of MFMA and 2400 vector instructions of
  * four cycles per SIMD, nearly all of them exponentials and divisions: 97 % of its time.  32 clips of 1500 positions x 6 heads take 1205 us (three
