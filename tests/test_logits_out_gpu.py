@@ -64,3 +64,43 @@ def test_halves_sent_in_any_order(gpu, model):
         stop.set()
         [t.join() for t in others]
     s.close()
+
+
+REFUSAL = r"""
+#include <dlfcn.h>
+#include <stddef.h>
+int hipHostMalloc(void** p, size_t n, unsigned flags) {
+    static int (*real)(void**, size_t, unsigned);
+    if (n >= ((size_t)8 << 20)) { *p = 0; return 2; /* hipErrorOutOfMemory */ }
+    if (!real) real = (int (*)(void**, size_t, unsigned))dlsym(dlopen("libamdhip64.so.7", RTLD_NOW | RTLD_NOLOAD), "hipHostMalloc");
+    return real(p, n, flags);
+}
+"""
+WITHOUT = r"""
+import ctypes, sys
+ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path[:0] = [sys.argv[2]]
+import numpy as np
+import trackiellm_amd as tk
+m = tk.LlmModel(tk.LlmHParams(1, 256, 8, 2, 64, 512, 32000, 1e-5, 10000.0, 0, 0, 0, 0, 1)).fill_synthetic(4)
+s = tk.LlmSession(m, 256, 8)
+print("open", flush=True)
+x = np.arange(3, 43, dtype=np.int32)
+np.save(sys.argv[3], s.forward(np.arange(40), np.zeros(40), x)[0])
+"""
+
+
+def test_a_session_without_pinned_memory(gpu, model, tmp_path):
+    """where the runtime refuses it (here: a definition in front of its own), a session opens all the same and its logits go by the plain copy"""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    shim, out = tmp_path / "refuse.so", tmp_path / "logits.npy"
+    (tmp_path / "refuse.c").write_text(REFUSAL)
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(shim), str(tmp_path / "refuse.c"), "-ldl"], check=True)
+    r = subprocess.run([sys.executable, "-c", WITHOUT, str(shim), root, str(out)], capture_output=True, text=True, timeout=60)
+    assert r.returncode == 0 and "open" in r.stdout, r.stderr[-1000:]
+    x = np.arange(3, 43, dtype=np.int32)
+    want = gpu.LlmSession(model, 256, 8).forward(np.arange(40), np.zeros(40), x)[0]
+    assert np.array_equal(np.load(out).view(np.uint32), want.view(np.uint32))

@@ -103,7 +103,7 @@ protected:
 
 private:
     int32_t* d_block_ = nullptr;
-    uint8_t* out_ring_ = nullptr; /* pinned, from the first large copy on: TK_OUT_PIECES pieces, and of each the number of the batch that arrived last */
+    uint8_t* out_ring_ = nullptr; /* pinned, null where there is none to be had: TK_OUT_PIECES pieces, and of each the number of the batch that arrived last */
     unsigned* d_out_done_ = nullptr;
     unsigned out_epoch_ = 1;
 };

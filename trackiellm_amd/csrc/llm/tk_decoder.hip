@@ -49,6 +49,13 @@ bool TkDecodeSession::init_tables(int device, int vocab, int row_cap, size_t ext
     if (extra_tab) *extra_tab = d_tok + row_cap;
     HIPQ(hipMalloc((void**)&logits, (size_t)TK_MAX_ROWS * vocab * 4));
     if ((size_t)TK_MAX_ROWS * vocab * 4 > TK_OUT_DIRECT) {
+        /* here, and not with the first large copy, of whose call it took 0.06 .. 0.7 ms.  None to be had: those copies are plain ones */
+        if (hipHostMalloc((void**)&out_ring_, TK_OUT_PIECES * (TK_OUT_PIECE + 4), hipHostMallocDefault) == hipSuccess) {
+            memset(out_ring_ + TK_OUT_PIECES * TK_OUT_PIECE, 0, TK_OUT_PIECES * 4);
+        } else {
+            out_ring_ = nullptr;
+            (void)hipGetLastError();
+        }
         HIPQ(hipMalloc((void**)&d_out_done_, TK_OUT_PIECES * 4));
         HIPQ(hipMemset(d_out_done_, 0, TK_OUT_PIECES * 4));
     }
@@ -103,14 +110,6 @@ __global__ __launch_bounds__(256) void k_send_out(const float* __restrict__ dev,
  * each piece to its place as it arrives.  Copies with an event a piece instead cost 13 us a piece on the stream.  The pinned memory is the session's and bounded (two halves,
  * one being filled while the other is taken away); nothing of it is handed out. */
 bool TkDecodeSession::copy_out(void* host, const void* dev, size_t bytes) {
-    if (bytes > TK_OUT_DIRECT && d_out_done_ && !out_ring_) { /* the first time, while the pass runs: sessions that hand out ids alone never need it.  None to be had: the plain copy */
-        if (hipHostMalloc((void**)&out_ring_, TK_OUT_PIECES * (TK_OUT_PIECE + 4), hipHostMallocDefault) == hipSuccess) {
-            memset(out_ring_ + TK_OUT_PIECES * TK_OUT_PIECE, 0, TK_OUT_PIECES * 4);
-        } else {
-            out_ring_ = nullptr;
-            (void)hipGetLastError();
-        }
-    }
     if (bytes <= TK_OUT_DIRECT || !out_ring_ || bytes % 4) {
         HIPQ(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream));
         return true;
