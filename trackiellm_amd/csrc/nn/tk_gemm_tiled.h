@@ -12,10 +12,11 @@
  * (LLM path); ks == 1: out[row][ldc] with the optional epilogue  v = act(acc + bias[n]) + residual[row][n].
  *
  * A wave owns one weight row tile of one K range and streams it as one piece per 32 k, PF pieces in flight in registers; a piece feeds
- * 8 MFMAs per M-tile.  The A image is staged through an LDS ring by LDS-DMA, 1 KiB per (16 k, M-tile), shared by the workgroup's
+ * 8 MFMAs per M-tile.  f16 weights of up to 128 rows: the A image comes from the caches straight into registers, as the weights do (tw_reg_plan).
+ * Else it is staged through an LDS ring by LDS-DMA, 1 KiB per (16 k, M-tile), shared by the workgroup's
  * waves; a lane's operand of four consecutive MFMAs is one ds_read_b128.  Rows beyond 256 run as further workgroups (grid y) over the
  * same weights; where there are enough tiles of 32 x 32, a kernel without LDS takes
- * the products instead (k_gemm_wide), those of f16 weights from 33 rows on.  At 16 rows the f16 path is HBM-bound (2 B per weight); from 32 rows up the fp32 MFMA rate (157 TFLOP/s) bounds it.
+ * the products instead (k_gemm_wide), those of f16 weights from 49 rows on.  At 16 rows the f16 path is HBM-bound (2 B per weight); from 32 rows up the fp32 MFMA rate (157 TFLOP/s) bounds it.
  */
 #ifndef TK_GEMM_TILED_H
 #define TK_GEMM_TILED_H
@@ -68,7 +69,7 @@ struct TkTiledGemm {
 /* false (nothing launched): K / ks is not a multiple of the ring granularity (128 k; 64 k from 129 rows per block on) or a field is inconsistent */
 bool tk_launch_gemm_tiled(const TkTiledGemm& g, hipStream_t s);
 /* how a launch is cut: M-tiles and waves (a tile of columns each) of a workgroup, and what follows from them.  mt 0: its own choice */
-struct TkTiledPlan { int mt, waves, groups, ny, pf, rk, slot_bytes; bool one; size_t lds; bool reg = false; /* operands of the rows in registers, without LDS */ int wide = 0; /* k_gemm_wide's form */ };
+struct TkTiledPlan { int mt, waves, groups, ny, pf, rk, slot_bytes; bool one; size_t lds; bool reg = false; /* operands of the rows in registers, without LDS: units of columns and parts in grid y, eight of them and the row blocks in grid x */ int wide = 0; /* k_gemm_wide's form */ };
 bool tk_gemm_tiled_plan(const TkTiledGemm& g, int mt, int waves, TkTiledPlan* plan);
 bool tk_launch_gemm_tiled_plan(const TkTiledGemm& g, const TkTiledPlan& plan, hipStream_t s);
 /* row-major f16 / f32 [N][K] (device) -> tiles; N is padded up to a multiple of 16 with zero rows, K must be a multiple of 32 */

@@ -61,8 +61,10 @@ template <int N> __device__ __forceinline__ void tw_act_all(float* v, int act) {
  * behind the staging and lets the first weights of every PF chunks wait for all requests; where the activations of the whole K range fit the LDS
  * (ONE: multiples of 128 k, up to 2048 at one M-tile, 1024 at two) there is no staging in the loop, and four pieces of weights stay in flight, eight
  * where k is a multiple of 256 from 512 on.
- * A wave by itself in its workgroup (REG: f32, one M-tile; the launcher's rule says when) shares no activations: it fetches its operands as it does its weights, straight into
- * registers, and its chain starts with the first of both instead of behind a whole image in LDS and a barrier.
+ * REG (the launcher's rules say when): a wave shares no activations, it fetches its operands as it does its weights, straight into registers, by scalar offsets, and its
+ * chain starts with the first of both instead of behind a whole image in LDS and a barrier; nothing waits for another wave, and no LDS read takes a turn from the MFMAs.
+ * f16: conversions in front of a piece's products, not between them, and the next operands' requests behind them (scattered, 8192 columns of 4096 k at 24 rows take 39.6 us,
+ * in order 35.7).  4096 x 28672 at 1, 24, 48 rows, ring -> here: 61 -> 42, 83 -> 68, 142 -> 97 us (floor of the weights 45, of the fp32 MFMAs on two tiles a SIMD 55 and 82).
  * In LDS, cold weights, N x K at 1 row: 384 x 384 5.4 -> 4.5 us and 51872 x 384 24.0 -> 22.0 with four, 384 x 1536 13.9 -> 10.2 with eight; at 32 rows
  * 8.6 -> 7.9, 30.0 -> 27.0 with four, 20.8 -> 18.9 (ring).  Twelve pieces: 384 x 384 at 1 row 5.6 (a wave's requests queue in front of the activations
  * of the others). */
@@ -120,7 +122,7 @@ __device__ __forceinline__ void tw_layernorm(const TkTiledGemm& a, int row0, int
 }
 
 template <int MT, int WB, bool ONE /* the whole K range in one slot */, int PF /* weight pieces in flight per wave; a ring slot holds a multiple of PF chunks (the launcher's rk), so piece c sits in register set c % PF */,
-          int LN = 0 /* the activations are made here, norms of up to LN times 256 columns (MT = 1, ONE) */, bool REG = false /* and each wave fetches its own into registers, like its weights (MT = 1, ONE) */>
+          int LN = 0 /* the activations are made here, norms of up to LN times 256 columns (MT = 1, ONE) */, bool REG = false /* and each wave fetches its own into registers, like its weights (ONE; f16: up to four M-tiles) */>
 __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, int total_row_tiles, int rk /* k per ring slot */, int slot_bytes /* ring slot pitch */) {
     constexpr int LPC = WB == 4 ? 2 : 1; /* 16-byte requests per piece and lane */
     constexpr int PIECE = 512 * WB;      /* bytes of one (row tile, 32 k) piece */
@@ -129,16 +131,18 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nw = blockDim.x >> 6;
     const int Kr = a.K / a.ks;
-    const int ksi = blockIdx.x % a.ks;
+    /* REG: the row blocks of a unit one behind the other on one XCD, which then has their weights */
+    const int unit = REG ? (int)(blockIdx.y * 8 + (blockIdx.x & 7)) : (int)blockIdx.x, block = REG ? (int)(blockIdx.x >> 3) : (int)blockIdx.y;
+    const int ksi = unit % a.ks;
     const int k0 = ksi * Kr;
     const int nslots = Kr / rk, cps = rk / 32, gps = rk / 16;
     /* grid y: the block of MT M-tiles this workgroup covers */
-    const int row0 = blockIdx.y * MT * TK_TW_ROWS_PER_TILE;
-    const float* a_img = a.a_img + (size_t)blockIdx.y * MT * a.a_ts;
+    const int row0 = block * MT * TK_TW_ROWS_PER_TILE;
+    const float* a_img = a.a_img + (size_t)block * MT * a.a_ts;
     const int rows_here = a.nrows - row0 < MT * TK_TW_ROWS_PER_TILE ? a.nrows - row0 : MT * TK_TW_ROWS_PER_TILE;
 
-    int rt = blockIdx.x / a.ks + wave * groups;
-    const bool active = rt < total_row_tiles;
+    int rt = unit / a.ks + wave * groups;
+    const bool active = (!REG || unit < groups * a.ks) && rt < total_row_tiles;
     if (!active) rt = 0;
     /* The segment by comparisons and selects, without an index into the arguments, and all that the end takes from them here: an argument is asked for
      * where it is used else, and each new line of them is a trip to memory of a chain of its own, in front of the weights and behind the sums (with bias and
@@ -176,13 +180,6 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
 #pragma unroll
         for (int r = 0; r < 4; ++r) acc[m][r] = 0.0f;
 
-    /* a request past the range re-reads the last piece: no branch around a load, static wait counts */
-    uint4 wq[PF][LPC];
-    auto wload = [&](int c, uint4* dst) {
-        const uint8_t* p = wbase + (size_t)(c < nchunk ? c : nchunk - 1) * PIECE;
-        dst[0] = tw_ldg_nt(p);
-        if (LPC == 2) dst[LPC - 1] = tw_ldg_nt(p + 16);
-    };
     /* bias and residual are on their way while the products run: one trip to memory less behind them (few rows: registers for all of it) */
     constexpr bool EARLY = MT <= 2;
     float bias = 0.0f, res[EARLY ? MT : 1][4] = {};
@@ -199,14 +196,35 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                 }
         }
     };
-    /* REG: operands of chunk c, two 16-k groups; rows that are not there: the last one again */
-    v4f aq[REG ? PF : 1][2];
-    const int rows_tile = rows_here < TK_TW_ROWS_PER_TILE ? rows_here : TK_TW_ROWS_PER_TILE, arow = (lane & 15) < rows_tile ? lane & 15 : rows_tile - 1;
-    const float* const abase = a_img + (size_t)k0 * 16 + ((lane & 48) + arow) * 4;
-    auto aload = [&](int c, v4f* dst) {
-        const v4f* p = (const v4f*)(abase + (size_t)(c < nchunk ? c : nchunk - 1) * 512);
-        dst[0] = p[0];
-        dst[1] = p[64];
+    /* REG: operands of chunk c, two 16-k groups of each M-tile; rows that are not there: the last one again.  Scalar offsets walk k: no vector instruction beside the products. */
+    v4f aq[REG ? PF : 1][REG ? MT : 1][2];
+    const int tiles_here = (rows_here + TK_TW_ROWS_PER_TILE - 1) / TK_TW_ROWS_PER_TILE;
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void*)(a_img + (size_t)k0 * 16), 0, ((unsigned)(tiles_here - 1) * (unsigned)a.a_ts + (unsigned)Kr * 16u) * 4u, 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)(of(a.tiles) + ((size_t)rt * nchunk_total + k0 / 32) * PIECE), 0, (unsigned)nchunk * PIECE, 0x00020000);
+    unsigned a_at[REG ? MT : 1];
+#pragma unroll
+    for (int m = 0; m < (REG ? MT : 0); ++m) {
+        const int t = m < tiles_here ? m : tiles_here - 1, rows = rows_here - t * TK_TW_ROWS_PER_TILE, last = rows < TK_TW_ROWS_PER_TILE ? rows - 1 : TK_TW_ROWS_PER_TILE - 1;
+        a_at[m] = (unsigned)t * (unsigned)a.a_ts * 4u + (unsigned)((lane & 48) + ((lane & 15) < last ? lane & 15 : last)) * 16u;
+    }
+    /* a request past the range re-reads the last piece: no branch around a load, static wait counts */
+    uint4 wq[PF][LPC];
+    auto wload = [&](int c, uint4* dst) {
+        if (REG) {
+#pragma unroll
+            for (int i = 0; i < LPC; ++i) dst[i] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(wr, lane * (8 * WB) + 16 * i, (unsigned)(c < nchunk ? c : nchunk - 1) * PIECE, 2));
+            return;
+        }
+        const uint8_t* p = wbase + (size_t)(c < nchunk ? c : nchunk - 1) * PIECE;
+        dst[0] = tw_ldg_nt(p);
+        if (LPC == 2) dst[LPC - 1] = tw_ldg_nt(p + 16);
+    };
+    auto aload = [&](int c, v4f (*dst)[2]) {
+        const unsigned at = (unsigned)(c < nchunk ? c : nchunk - 1) * 2048u;
+#pragma unroll
+        for (int m = 0; m < (REG ? MT : 0); ++m)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) dst[m][h] = __builtin_bit_cast(v4f, __builtin_amdgcn_raw_buffer_load_b128(ar, a_at[m] + h * 1024, at, 0));
     };
     if (REG) {
         if (!active) return;
@@ -250,7 +268,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
         if (!ONE && s + 1 < nslots) stage(s + 1, (s + 1) & 1);
         const uint8_t* slot = lds + (size_t)(ONE ? 0 : s & 1) * slot_bytes + lane * 16;
         /* operands of M-tiles m, m + 1 (m alone of MT = 1) and chunk cc of the slot; [k half][tile] */
-        constexpr int PAIR = MT == 1 ? 1 : 2, PAIRS = MT / PAIR;
+        constexpr int PAIR = MT == 1 ? 1 : REG ? MT : 2, PAIRS = MT / PAIR;
         struct Ops { v4f a[2][PAIR]; } ops[2];
         auto read = [&](Ops& o, int cc, int m) {
             const uint8_t* ap = slot + (size_t)(2 * (cc < cps ? cc : cps - 1)) * MT * 1024 + m * 1024;
@@ -276,6 +294,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                     wf[4] = __uint_as_float(w1.x); wf[5] = __uint_as_float(w1.y); wf[6] = __uint_as_float(w1.z); wf[7] = __uint_as_float(w1.w);
                 }
                 if (WB == 2 || !ONE) wload(c + PF, wq[u]);
+                if (REG && WB == 2) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int p = 0; p < PAIRS; ++p) {
                     /* the next pair's operand reads, the next chunk's behind the last pair, are issued before this pair's MFMAs; of two tiles the
@@ -283,8 +302,10 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                     const int step = u * PAIRS + p, m = p * PAIR;
                     Ops& o = ops[step & 1];
                     if (REG) {
-                        o.a[0][0] = aq[REG ? u : 0][0];
-                        o.a[1][0] = aq[REG ? u : 0][1];
+#pragma unroll
+                        for (int i = 0; i < PAIR; ++i)
+#pragma unroll
+                            for (int h = 0; h < 2; ++h) o.a[h][i] = aq[REG ? u : 0][REG ? m + i : 0][h];
                     } else if (p + 1 < PAIRS) {
                         read(ops[(step + 1) & 1], cc + u, m + PAIR);
                     } else {
@@ -307,6 +328,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiled(TkTiledGemm a, int groups, i
                 }
                 if (WB == 4 && ONE) wload(c + PF, wq[u]);
                 if (REG) aload(c + PF, aq[REG ? u : 0]);
+                if (REG && WB == 2) __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
@@ -639,6 +661,50 @@ static float tw_cost(const TkTiledGemm& a, const TkTiledPlan& p) {
     return pipe > weights ? pipe + 0.15f * weights : weights + 0.15f * pipe;
 }
 
+/*
+ * f16 weights, operands in registers: how many M-tiles a wave makes (1 .. 4) and how many waves share a workgroup.  The chip's SIMDs take (tile columns x parts of k x row
+ * blocks) in rounds; a wave of m M-tiles takes m + 1 units of time (its products, and the weights' way and conversion once), a lone one of four a quarter more; of equal
+ * ones the larger.  What that chooses is within 7 % of the best measured of m = 1 .. 4 with one, four and a CU's share of waves, for 16 matrices of 256 .. 8192 k at 1, 16, 24,
+ * 33, 64, 96, 128 rows, but for 1024 x 5632 at 128 rows (20.1 us; m = 1 18.7, the ring 25.7).  Ring or one LDS image / this, us: 4096 x 28672 at 1, 16, 24, 33, 64 rows 61 / 42, 52.7 / 50.6, 83 / 68, 142 / 97, 142 / 131;
+ * 14336 x 4096 in seven parts 25.4 / 24.2, (25.2 / 26.4), 43.5 / 35.7, 73 / 51, 74 / 70; 4096 x 4096 35 / 20, 36 / 21, 52 / 21, 84 / 22, 85 / 23; 2048 x 2048 in four parts
+ * 6.2 / 5.1, 6.5 / 5.4, 6.8 / 5.8, 9.0 / 7.7, 9.5 / 7.8; 256 x 768 4.4 / 3.8 .. 4.9 / 4.3.  The one in brackets stays with the image in LDS: rows that all 16 of a tile hold
+ * and parts of more than 1024 k, whose operands a CU's waves no longer find in its L1 (8192 x 28672 in four parts at 12 rows 98 / 103; at 8 rows 96 / 89).
+ * 65 .. 128 rows: up to one and a half tile columns a SIMD (4096 x 6144 in four parts at 96 rows 54 / 43; beyond, 4096 x 28672 at 96 and 128 rows 203 / 198 and 250 / 255).
+ * 49 .. 64 rows: behind k_gemm_wide's rule, where both are alike (4096 x 65536 269 / 268, x 40960 195 / 197).
+ */
+static int tk_tiled_num_cu();
+static bool tw_reg_plan(const TkTiledGemm& a, bool behind_wide, TkTiledPlan* p) {
+    const int Kr = a.K / a.ks, tiles = (a.nrows + TK_TW_ROWS_PER_TILE - 1) / TK_TW_ROWS_PER_TILE, row_tiles = tw_row_tiles(a);
+    if (a.wbytes != 2 || a.ln_x || Kr % 128 || tiles > 8 || (!behind_wide && tiles > 3)) return false;
+    const int64_t cus = tk_tiled_num_cu(), simds = 4 * cus, units = (int64_t)row_tiles * a.ks;
+    if (units > 400000 || (tiles > 4 && 2 * units > 3 * simds)) return false;
+    if (a.nrows > 8 && tiles == 1 && a.ks > 1 && Kr > 1024 && Kr <= 2048 && 2 * units > 3 * simds) return false;
+    int mt = 0;
+    int64_t least = 0;
+    for (int m = 1; m <= 4 && m <= tiles; ++m) {
+        const int64_t rounds = (units * ((tiles + m - 1) / m) + simds - 1) / simds, cost = rounds * (m + 1) * (m == 4 && rounds == 1 ? 5 : 4);
+        if (mt == 0 || cost <= least) { mt = m; least = cost; }
+    }
+    *p = TkTiledPlan{};
+    p->mt = mt;
+    p->ny = (tiles + mt - 1) / mt;
+    p->reg = p->one = true;
+    p->rk = Kr;
+    /* more waves than SIMDs and one row block: as many workgroups as CUs, whose waves share the operands that they find in its L1 (4096 x 28672 at 1 row 42.3 us, single
+     * waves 45.2); else a wave a workgroup, which spreads them evenly (4096 x 8192 at 24 rows 22.5, in twos 37.1) */
+    p->waves = 1;
+    p->groups = row_tiles;
+    if (p->ny == 1 && units > simds) {
+        int groups = (int)(cus / a.ks);
+        groups = groups < 1 ? 1 : groups > row_tiles ? row_tiles : groups;
+        while ((row_tiles + groups - 1) / groups > 8) groups *= 2;
+        p->waves = (row_tiles + groups - 1) / groups;
+        p->groups = groups;
+    }
+    /* one M-tile, no more waves than SIMDs: eight pieces of weights in flight (4096 x 4096 at 1 row 22.4 -> 19.9 us; 4096 x 6144 in four parts, 1536 waves, 11.9 -> 12.9) */
+    p->pf = mt == 1 && units * p->ny <= simds && Kr % 256 == 0 ? 8 : 4;
+    return true;
+}
 static bool tw_usual(const TkTiledGemm& a, TkTiledPlan* p);
 bool tk_gemm_wide_plan(const TkTiledGemm& a, int form, TkTiledPlan* p);
 bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p) {
@@ -653,12 +719,14 @@ bool tk_gemm_tiled_plan(const TkTiledGemm& a, int mt, int waves, TkTiledPlan* p)
      * at 160 1026 / 682.  Form 2
      * does a step of its 64 rows in 0.96 of the time that two tiles of form 1 take, but has half as many tiles to spread: 256 rows x 4096, 6144, 28672 columns 72.7, 105.5,
      * 530 us against 76.8, 109.1, 491. */
+    if (tw_reg_plan(a, false, p)) return true;
     if (a.wbytes == 2 && a.nrows > 2 * TK_TW_ROWS_PER_TILE) {
         const int64_t cols = (int64_t)(tw_row_tiles(a) / 2) * a.ks, simds = 4 * (int64_t)tk_tiled_num_cu();
         const int64_t one = (a.nrows + 31) / 32 * cols, two = (a.nrows + 63) / 64 * cols;
         const int form = 1.92f * (float)((two + simds - 1) / simds) < (float)((one + simds - 1) / simds) ? 2 : 1;
         const int64_t least = a.nrows <= 64 ? 2 * simds : a.K / a.ks >= 512 ? simds * 3 / 2 : simds * 5 / 2;
         if (one >= least && tk_gemm_wide_plan(a, form, p)) return true;
+        if (tw_reg_plan(a, true, p)) return true;
     }
     if (a.wbytes == 4 && a.nrows > TK_TW_MAX_BLOCK_ROWS) {
         const int64_t tiles = (int64_t)((a.nrows + 31) / 32) * (tw_row_tiles(a) / 2);
@@ -762,19 +830,24 @@ bool tk_launch_gemm_tiled_plan(const TkTiledGemm& a, const TkTiledPlan& p, hipSt
         return true;
     }
 #define TK_TW_LAUNCH(MTV, WBV, ONEV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, ONEV, PFV>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), p.lds, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
+#define TK_TW_LAUNCH_REG(MTV, WBV, PFV) hipLaunchKernelGGL((k_gemm_tiled<MTV, WBV, true, PFV, 0, true>), dim3(8 * p.ny, (p.groups * a.ks + 7) / 8), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes)
+#define TK_TW_REG(MTV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH_REG(MTV, 2, PFV); else TK_TW_LAUNCH_REG(MTV, 4, PFV); } while (0)
 #define TK_TW_WB(MTV, ONEV, PFV) do { if (a.wbytes == 2) TK_TW_LAUNCH(MTV, 2, ONEV, PFV); else TK_TW_LAUNCH(MTV, 4, ONEV, PFV); } while (0)
     switch (p.mt) {
-        case 1: if (p.reg) {
-                if (p.pf == 8) hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 8, 0, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
-                else hipLaunchKernelGGL((k_gemm_tiled<1, 4, true, 4, 0, true>), dim3(p.groups * a.ks, p.ny), dim3(64 * p.waves), 0, s, a, p.groups, row_tiles, p.rk, p.slot_bytes);
-            } else if (p.one) { if (p.pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
-        case 2: if (p.one) { if (p.pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
-        case 4: TK_TW_WB(4, false, 4); break;
+        case 1: if (p.reg) { if (p.pf == 8) TK_TW_REG(1, 8); else TK_TW_REG(1, 4); }
+                else if (p.one) { if (p.pf == 8) TK_TW_WB(1, true, 8); else TK_TW_WB(1, true, 4); } else TK_TW_WB(1, false, 4); break;
+        case 2: if (p.reg) TK_TW_LAUNCH_REG(2, 2, 4);
+                else if (p.one) { if (p.pf == 8) TK_TW_WB(2, true, 8); else TK_TW_WB(2, true, 4); } else TK_TW_WB(2, false, 4); break;
+        case 3: if (!p.reg) return false;
+                TK_TW_LAUNCH_REG(3, 2, 4); break;
+        case 4: if (p.reg) TK_TW_LAUNCH_REG(4, 2, 4); else TK_TW_WB(4, false, 4); break;
         case 6: TK_TW_WB(6, false, 2); break;
         case 8: if (p.pf == 2) TK_TW_WB(8, false, 2); else TK_TW_WB(8, false, 4); break;
         default: TK_TW_WB(16, false, 2); break;
     }
 #undef TK_TW_WB
+#undef TK_TW_REG
+#undef TK_TW_LAUNCH_REG
 #undef TK_TW_LAUNCH
     return true;
 }
