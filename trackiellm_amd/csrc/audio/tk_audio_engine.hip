@@ -1098,11 +1098,73 @@ bool TkVadModel::fill_synthetic(uint64_t seed) {
 }
 
 /* A workgroup per window, a lane per hidden unit: its chain over the window, relu, then one lane's chain over the hidden units.  Windows are read from, and probabilities
- * written to, pinned host memory: one launch and one wait make a call, where a copy, two launches, a copy and a wait took 47 us for 33 windows of 480.  What is left is the
- * launch, the trip over the bus and the chain of `window` fmas. */
+ * written to, pinned host memory: one launch and one wait make a call.  What is left is the launch, the trip over the bus and the chain of `window` fmas. */
+/* Windows of up to 480 samples (16 kHz): NW waves of P groups of four.  The chain goes from wave to wave: each has its P groups of four weights, all asked for at once, and then its share of the window in
+ * registers before its turn, so that a turn is its fmas and a hand-over through LDS.  One wave that fetched all weights had 40 groups in flight and read the window from LDS beside
+ * the chain (k_vad_long): load, chain, end 3.0, 6.6, 0.9 us of a window of 480, here 2.4, 1.8, 1.0; 33 windows from call to result 23.0 -> 17.8 us, 256 34.4 -> 30.8.  Weights in
+ * LDS 19.8 (an LDS read holds the wave's issue as long as four fmas), all 480 in one wave's registers, half of them accumulation registers, 19.8; five waves of 26 groups 18.05,
+ * eight of 16 18.3. */
+__global__ __launch_bounds__(256) void k_vad(const float* x, int window, int hidden, const float* __restrict__ w1, const float* __restrict__ b1, const float* __restrict__ w2,
+                                             const float* __restrict__ b2, float* prob) {
+    constexpr int NW = 4, P = 30;
+    __shared__ __attribute__((aligned(16))) float win[4 * NW * P], sums[64], w2s[64];
+    const int t = threadIdx.x, lane = t & 63, wave = __builtin_amdgcn_readfirstlane(t >> 6), groups = window >> 2, unit = lane < hidden ? lane : hidden - 1;
+    const int g0 = wave * P;
+    at1_f32x4 mine = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (t < groups) mine = ((const at1_f32x4*)(x + (int64_t)blockIdx.x * window))[t];
+    float w2v = 0.0f, b1v = 0.0f, b2v = 0.0f;
+    if (wave == 0) w2v = w2[unit];
+    if (wave == NW - 1) { b1v = b1[unit]; b2v = b2[0]; }
+    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc((void*)w1, 0, (unsigned)(window * hidden * 4), 0x00020000);
+    at1_f32x4 w[P], v[P];
+#pragma unroll
+    for (int i = 0; i < P; ++i) /* past the window: its last group again */
+        w[i] = __builtin_bit_cast(at1_f32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, unit * 16, (g0 + i < groups ? g0 + i : groups - 1) * hidden * 16, 0));
+    if (t < NW * P) ((at1_f32x4*)win)[t] = mine;
+    if (wave == 0) w2s[lane] = w2v;
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < P; ++i) v[i] = ((const at1_f32x4*)win)[g0 + i];
+    float acc = 0.0f;
+#pragma unroll 1
+    for (int s = 0; s < NW; ++s) {
+        if (s == wave) {
+            if (s) acc = sums[lane];
+            if (g0 + P <= groups) {
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc = tk_fmaf(v[i][j], w[i][j], acc);
+            } else {
+#pragma unroll
+                for (int i = 0; i < P; ++i)
+                    if (g0 + i < groups)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) acc = tk_fmaf(v[i][j], w[i][j], acc);
+            }
+            if (s == NW - 1) acc = tk_fmaxf(acc + b1v, 0.0f);
+            sums[lane] = acc;
+        }
+        if (s < NW - 1) __syncthreads();
+    }
+    if (wave < NW - 1) return;
+    float a = 0.0f;
+#pragma unroll
+    for (int k0 = 0; k0 < 64; k0 += 16) {
+        at1_f32x4 hv[4], wv[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) { hv[i] = ((const at1_f32x4*)sums)[k0 / 4 + i]; wv[i] = ((const at1_f32x4*)w2s)[k0 / 4 + i]; }
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (k0 + i < hidden) a = tk_fmaf(hv[i >> 2][i & 3], wv[i >> 2][i & 3], a);
+    }
+    if (lane == 0) prob[blockIdx.x] = tk_sigmoidf(a + b2v);
+}
+
+/* windows of more than 480 samples (48 kHz): three waves a SIMD hold no such shares */
 #define TK_VAD_AHEAD 20 /* groups of four weights on their way, twice */
-__global__ __launch_bounds__(64) void k_vad(const float* x, int window, int hidden, const float* __restrict__ w1, const float* __restrict__ b1, const float* __restrict__ w2,
-                                            const float* __restrict__ b2, float* prob) {
+__global__ __launch_bounds__(64) void k_vad_long(const float* x, int window, int hidden, const float* __restrict__ w1, const float* __restrict__ b1, const float* __restrict__ w2,
+                                                 const float* __restrict__ b2, float* prob) {
     extern __shared__ __attribute__((aligned(16))) float vad_lds[];
     float* hs = vad_lds + window; /* [hidden] behind the window */
     const int t = threadIdx.x, groups = window >> 2, unit = t < hidden ? t : hidden - 1;
@@ -1159,7 +1221,9 @@ bool TkVadModel::infer(const float* windows_host, int n, float* prob_host) {
     HIPQ(hipSetDevice(device));
     if (!stream) HIPQ(tk_create_perception_stream(&stream));
     auto launch = [&](Slot& s, int count) {
-        hipLaunchKernelGGL(k_vad, dim3(count), dim3(64), (size_t)(window + hidden) * 4, stream, s.x, window, hidden, w1, b1, w2, b2, s.x + (size_t)s.cap * window);
+        float* prob = s.x + (size_t)s.cap * window;
+        if (window <= 480) hipLaunchKernelGGL(k_vad, dim3(count), dim3(256), 0, stream, s.x, window, hidden, w1, b1, w2, b2, prob);
+        else hipLaunchKernelGGL(k_vad_long, dim3(count), dim3(64), (size_t)(window + hidden) * 4, stream, s.x, window, hidden, w1, b1, w2, b2, prob);
         return hipGetLastError();
     };
     if (n <= TK_VAD_CHUNK) {
