@@ -18,6 +18,7 @@
 #include <stdlib.h>
 
 #include <atomic>
+#include <type_traits>
 
 #include "../common/tk_ggml_blocks.h"
 #include "../common/tk_sample_device.h"
@@ -629,20 +630,23 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
         for (int r = 0; r < 4; ++r) acc[m][r] = 0.0f;
 
     /* The first PF weight tiles are requested before the activations are staged so HBM latency overlaps the LDS
-     * fill.  Loop bodies below contain NO conditional loads: hipcc then keeps counted vmcnt waits and the next
+     * fill (FUSE 2: behind what the image is made of).  Loop bodies below contain NO conditional loads: hipcc then keeps counted vmcnt waits and the next
      * group's tiles stay in flight under the current group's MFMAs (a branch around a load costs a vmcnt(0)). */
     constexpr bool HAS4 = (TYPES & 1) != 0, HAS6 = (TYPES & 2) != 0;
     const bool is4 = HAS4 && (!HAS6 || type == TK_TYPE_Q4_K);
     FragQ4 f4[HAS4 ? PF : 1];
     FragQ6 f6[HAS6 ? PF : 1];
-    if (HAS4 && is4) {
+    auto load_first = [&]() {
+        if (HAS4 && is4) {
 #pragma unroll
-        for (int u = 0; u < PF; ++u) f4[HAS4 ? u : 0] = load_q4(tile + (size_t)u * tile_bytes, lane);
-    }
-    if (HAS6 && !is4) {
+            for (int u = 0; u < PF; ++u) f4[HAS4 ? u : 0] = load_q4(tile + (size_t)u * tile_bytes, lane);
+        }
+        if (HAS6 && !is4) {
 #pragma unroll
-        for (int u = 0; u < PF; ++u) f6[HAS6 ? u : 0] = load_q6(tile + (size_t)u * tile_bytes, lane);
-    }
+            for (int u = 0; u < PF; ++u) f6[HAS6 ? u : 0] = load_q6(tile + (size_t)u * tile_bytes, lane);
+        }
+    };
+    if (FUSE != 2) load_first();
     if (FUSE != 0) {
         const int nw = nthr >> 6, hw = tid >> 5, nhw = nthr >> 5;
         TkActQ8 lo{}; /* the LDS image as quantize_chunk8's destination: same layout as the global one, block 0 = this K-range's first */
@@ -720,30 +724,41 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                     quantize_chunk8(v, cl, r, lo);
                 }
         } else {
+            /* A wave's requests are answered in order, and the weights come from HBM: the gate and up values in front of them, so that the image is made while the weights
+             * are on their way.  14336 x 4096 at one row, Q6_K / Q4_K: 13.2 -> 12.2, 10.5 -> 10.0 us.  Norms (FUSE 1), whose slabs are 64 .. 128 KB a workgroup, gain nothing or
+             * lose: gate | up 17.3 / 17.4, q | k | v 8.7 / 9.0 and 10.4 / 11.0; nor do joins (FUSE 3: 5.9 / 6.0). */
             const int FF = a.K;
-            for (int r = 0; r < a.nrows; ++r)
-                for (int b = hw; b < nb; b += nhw) {
-                    const int cl = 32 * b + (lane & 31), c = 32 * blk0 + cl;
-                    v4f g[2], u[2];
-                    {
-                        v4f pg[TK_RMS_MAX_KS][2], pu[TK_RMS_MAX_KS][2];
+            auto gated_rows = [&](auto slabs /* requested; from a.fks on the last one again */) {
+                constexpr int NS = slabs.value;
+                v4f pg[NS][2], pu[NS][2];
+                auto request = [&](int r, int b) { /* past the range: its last block again */
+                    const int c = 32 * (blk0 + (b < nb ? b : nb - 1)) + (lane & 31);
 #pragma unroll
-                        for (int sl = 0; sl < TK_RMS_MAX_KS; ++sl)
-                            if (sl < a.fks) {
-                                const float* row = a.fslab + sl * a.fslab_pitch + r * (2 * (int64_t)FF);
-                                pg[sl][0] = *(const v4f*)(row + 8 * c); pg[sl][1] = *(const v4f*)(row + 8 * c + 4);
-                                pu[sl][0] = *(const v4f*)(row + FF + 8 * c); pu[sl][1] = *(const v4f*)(row + FF + 8 * c + 4);
-                            }
-                        g[0] = pg[0][0]; g[1] = pg[0][1]; u[0] = pu[0][0]; u[1] = pu[0][1];
-#pragma unroll
-                        for (int sl = 1; sl < TK_RMS_MAX_KS; ++sl)
-                            if (sl < a.fks) { g[0] = g[0] + pg[sl][0]; g[1] = g[1] + pg[sl][1]; u[0] = u[0] + pu[sl][0]; u[1] = u[1] + pu[sl][1]; }
+                    for (int sl = 0; sl < NS; ++sl) {
+                        const float* row = a.fslab + (sl < a.fks ? sl : a.fks - 1) * a.fslab_pitch + r * (2 * (int64_t)FF);
+                        pg[sl][0] = *(const v4f*)(row + 8 * c); pg[sl][1] = *(const v4f*)(row + 8 * c + 4);
+                        pu[sl][0] = *(const v4f*)(row + FF + 8 * c); pu[sl][1] = *(const v4f*)(row + FF + 8 * c + 4);
                     }
-                    float v[8];
+                };
+                request(0, hw);
+                __builtin_amdgcn_sched_barrier(0);
+                load_first();
+                __builtin_amdgcn_sched_barrier(0);
+                for (int r = 0; r < a.nrows; ++r)
+                    for (int b = hw; b < nb; b += nhw) {
+                        if (r > 0 || b > hw) request(r, b);
+                        v4f g[2] = {pg[0][0], pg[0][1]}, u[2] = {pu[0][0], pu[0][1]};
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) v[i] = tk_siluf(g[i >> 2][i & 3]) * u[i >> 2][i & 3];
-                    quantize_chunk8(v, cl, r, lo);
-                }
+                        for (int sl = 1; sl < NS; ++sl)
+                            if (sl < a.fks) { g[0] = g[0] + pg[sl][0]; g[1] = g[1] + pg[sl][1]; u[0] = u[0] + pu[sl][0]; u[1] = u[1] + pu[sl][1]; }
+                        float v[8];
+#pragma unroll
+                        for (int i = 0; i < 8; ++i) v[i] = tk_siluf(g[i >> 2][i & 3]) * u[i >> 2][i & 3];
+                        quantize_chunk8(v, 32 * b + (lane & 31), r, lo);
+                    }
+            };
+            if (a.fks == 1) gated_rows(std::integral_constant<int, 1>{});
+            else gated_rows(std::integral_constant<int, TK_RMS_MAX_KS>{});
         }
         __builtin_amdgcn_s_waitcnt(0); /* the image's stores and the first weight tiles */
     } else {
