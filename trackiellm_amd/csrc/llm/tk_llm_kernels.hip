@@ -585,6 +585,12 @@ size_t tk_gemv_lds_bytes(int K, int ks, int mtiles) {
  * so (a) every CU streams the same number of 16-row tiles (+-1), (b) the K-range's int8 activations are
  * staged once per CU, (c) all waves of a CU walk disjoint contiguous tile runs.
  */
+/* s_waitcnt vmcnt(N) alone (expcnt / lgkmcnt untouched): until all but this wave's N youngest vector-memory operations are done.  The
+ * LDS-DMA pieces of a chunk are invisible to the compiler's own wait insertion, so the ring is guarded by hand. */
+template <int N> __device__ __forceinline__ void wait_vmcnt() {
+    static_assert(N >= 0 && N <= 63, "the counter has six bits");
+    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
+}
 /* TYPES: bit 0 = the launch contains Q4_K tiles, bit 1 = Q6_K tiles; single-type launches keep only one fragment ring in registers */
 /* FUSE (TkGemvArgs::fuse, MT = 1 only): 0 = the activation image comes from global memory; 1 / 2 = every workgroup forms it itself —
  * the norm's or SwiGLU's arithmetic, value for value what k_rmsnorm_q8 / k_swiglu_q8 write — under the latency of its first weight tiles */
@@ -630,7 +636,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
         for (int r = 0; r < 4; ++r) acc[m][r] = 0.0f;
 
     /* The first PF weight tiles are requested before the activations are staged so HBM latency overlaps the LDS
-     * fill (FUSE 2: behind what the image is made of).  Loop bodies below contain NO conditional loads: hipcc then keeps counted vmcnt waits and the next
+     * fill (FUSE 2, 3: behind what the image is made of).  Loop bodies below contain NO conditional loads: hipcc then keeps counted vmcnt waits and the next
      * group's tiles stay in flight under the current group's MFMAs (a branch around a load costs a vmcnt(0)). */
     constexpr bool HAS4 = (TYPES & 1) != 0, HAS6 = (TYPES & 2) != 0;
     const bool is4 = HAS4 && (!HAS6 || type == TK_TYPE_Q4_K);
@@ -646,7 +652,11 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
             for (int u = 0; u < PF; ++u) f6[HAS6 ? u : 0] = load_q6(tile + (size_t)u * tile_bytes, lane);
         }
     };
-    if (FUSE != 2) load_first();
+    if (FUSE < 2) load_first();
+    /* A wave's requests are answered in order, and the weights come from HBM: what FUSE 2 and 3 make the image of is asked for in front of them, so that it is made while they are
+     * on their way.  The first blocks in front of the loops: in a loop that requests, the compiler waits for all that is in flight.  14336 x 4096 at one row, Q6_K / Q4_K:
+     * 13.1 -> 12.2, 10.3 -> 9.2 us, two rows 15.0 -> 13.9, 12.0 -> 10.7; o after a long attention 5.7 -> 5.6, 7.0 -> 6.8.  Norms (FUSE 1), whose slabs are 64 .. 128 KB a
+     * workgroup, gain nothing: gate | up 16.9 / 17.1, q | k | v 8.6 / 8.7 and 10.2 / 10.5, with four weight tiles in flight 17.2, 9.0. */
     if (FUSE != 0) {
         const int nw = nthr >> 6, hw = tid >> 5, nhw = nthr >> 5;
         TkActQ8 lo{}; /* the LDS image as quantize_chunk8's destination: same layout as the global one, block 0 = this K-range's first */
@@ -655,9 +665,14 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
             const int D = a.K, ngrp4 = D / 4;
             float* hbuf = (float*)(lds_abs + MT * abs_ts); /* the finished row, then 4 floats of the canonical sum */
             float* red = hbuf + D;
-            /* norm weights of this half-wave's first block: requested before the reductions so their latency hides under them */
-            v4f wa0 = {0.0f, 0.0f, 0.0f, 0.0f}, wa1 = wa0;
-            if (hw < nb) { const int c = 32 * (blk0 + hw) + (lane & 31); wa0 = *(const v4f*)(a.fw + 8 * c); wa1 = *(const v4f*)(a.fw + 8 * c + 4); }
+            /* norm weights of this half-wave's first two blocks: requested before the reductions so their latency hides under them (gate | up: 16 blocks, 14 half-waves) */
+            v4f wa[2][2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int b = hw + i * nhw, c = 32 * (blk0 + (b < nb ? b : nb - 1)) + (lane & 31);
+                wa[i][0] = *(const v4f*)(a.fw + 8 * c);
+                wa[i][1] = *(const v4f*)(a.fw + 8 * c + 4);
+            }
             for (int r = 0; r < a.nrows; ++r) {
                 if (r > 0) __syncthreads(); /* hbuf and red are reused */
                 for (int gi = tid; gi < ngrp4; gi += nthr) { /* the row and ALL its slabs requested before the first add (k_rmsnorm_q8) */
@@ -694,7 +709,8 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                 for (int b = hw; b < nb; b += nhw) { /* a half-wave quantises one 256-block of this K-range */
                     const int cl = 32 * b + (lane & 31), c = 32 * blk0 + cl;
                     v4f w0, w1;
-                    if (b == hw) { w0 = wa0; w1 = wa1; }
+                    if (b == hw) { w0 = wa[0][0]; w1 = wa[0][1]; }
+                    else if (b == hw + nhw) { w0 = wa[1][0]; w1 = wa[1][1]; }
                     else { w0 = *(const v4f*)(a.fw + 8 * c); w1 = *(const v4f*)(a.fw + 8 * c + 4); }
                     const v4f h0 = *(const v4f*)(hbuf + 8 * c), h1 = *(const v4f*)(hbuf + 8 * c + 4);
                     float v[8];
@@ -708,25 +724,31 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
             }
         } else if (FUSE == 3) { /* k_att_pv_join's arithmetic: this K-range's blocks of the attention output */
             const int HD = a.fn_total;
-            for (int r = 0; r < a.nrows; ++r)
-                for (int b = hw; b < nb; b += nhw) {
-                    const int cl = 32 * b + (lane & 31), c = 32 * blk0 + cl;
-                    const int64_t hi = (int64_t)r * (a.K / HD) + 8 * c / HD; /* (row, head) of this chunk's eight dims */
-                    const float* pp = a.fslab + hi * 4 * HD + 8 * c % HD;
-                    v4f p[4][2];
+            v4f p[4][2], lp;
+            auto request = [&](int r, int b) { /* past the range: its last block again */
+                const int c = 32 * (blk0 + (b < nb ? b : nb - 1)) + (lane & 31);
+                const int64_t hi = (int64_t)r * (a.K / HD) + 8 * c / HD; /* (row, head) of this chunk's eight dims */
+                const float* pp = a.fslab + hi * 4 * HD + 8 * c % HD;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) { p[j][0] = *(const v4f*)(pp + j * HD); p[j][1] = *(const v4f*)(pp + j * HD + 4); }
-                    const v4f lp = *(const v4f*)(a.fx_in + hi * 4);
-                    const float ll = ((lp[0] + lp[1]) + lp[2]) + lp[3];
-                    float v[8];
+                for (int j = 0; j < 4; ++j) { p[j][0] = *(const v4f*)(pp + j * HD); p[j][1] = *(const v4f*)(pp + j * HD + 4); }
+                lp = *(const v4f*)(a.fx_in + hi * 4);
+            };
+            auto finish = [&](int r, int b) {
+                const float ll = ((lp[0] + lp[1]) + lp[2]) + lp[3];
+                float v[8];
 #pragma unroll
-                    for (int i = 0; i < 8; ++i) v[i] = tk_divf(((p[0][i >> 2][i & 3] + p[1][i >> 2][i & 3]) + p[2][i >> 2][i & 3]) + p[3][i >> 2][i & 3], ll);
-                    quantize_chunk8(v, cl, r, lo);
-                }
+                for (int i = 0; i < 8; ++i) v[i] = tk_divf(((p[0][i >> 2][i & 3] + p[1][i >> 2][i & 3]) + p[2][i >> 2][i & 3]) + p[3][i >> 2][i & 3], ll);
+                quantize_chunk8(v, 32 * b + (lane & 31), r, lo);
+            };
+            request(0, hw);
+            __builtin_amdgcn_sched_barrier(0);
+            load_first();
+            __builtin_amdgcn_sched_barrier(0);
+            if (hw < nb) finish(0, hw);
+            for (int b = hw + nhw; b < nb; b += nhw) { request(0, b); wait_vmcnt<0>(); finish(0, b); }
+            for (int r = 1; r < a.nrows; ++r)
+                for (int b = hw; b < nb; b += nhw) { request(r, b); wait_vmcnt<0>(); finish(r, b); }
         } else {
-            /* A wave's requests are answered in order, and the weights come from HBM: the gate and up values in front of them, so that the image is made while the weights
-             * are on their way.  14336 x 4096 at one row, Q6_K / Q4_K: 13.2 -> 12.2, 10.5 -> 10.0 us.  Norms (FUSE 1), whose slabs are 64 .. 128 KB a workgroup, gain nothing or
-             * lose: gate | up 17.3 / 17.4, q | k | v 8.7 / 9.0 and 10.4 / 11.0; nor do joins (FUSE 3: 5.9 / 6.0). */
             const int FF = a.K;
             auto gated_rows = [&](auto slabs /* requested; from a.fks on the last one again */) {
                 constexpr int NS = slabs.value;
@@ -744,18 +766,20 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                 __builtin_amdgcn_sched_barrier(0);
                 load_first();
                 __builtin_amdgcn_sched_barrier(0);
-                for (int r = 0; r < a.nrows; ++r)
-                    for (int b = hw; b < nb; b += nhw) {
-                        if (r > 0 || b > hw) request(r, b);
-                        v4f g[2] = {pg[0][0], pg[0][1]}, u[2] = {pu[0][0], pu[0][1]};
+                auto finish = [&](int r, int b) {
+                    v4f g[2] = {pg[0][0], pg[0][1]}, u[2] = {pu[0][0], pu[0][1]};
 #pragma unroll
-                        for (int sl = 1; sl < NS; ++sl)
-                            if (sl < a.fks) { g[0] = g[0] + pg[sl][0]; g[1] = g[1] + pg[sl][1]; u[0] = u[0] + pu[sl][0]; u[1] = u[1] + pu[sl][1]; }
-                        float v[8];
+                    for (int sl = 1; sl < NS; ++sl)
+                        if (sl < a.fks) { g[0] = g[0] + pg[sl][0]; g[1] = g[1] + pg[sl][1]; u[0] = u[0] + pu[sl][0]; u[1] = u[1] + pu[sl][1]; }
+                    float v[8];
 #pragma unroll
-                        for (int i = 0; i < 8; ++i) v[i] = tk_siluf(g[i >> 2][i & 3]) * u[i >> 2][i & 3];
-                        quantize_chunk8(v, 32 * b + (lane & 31), r, lo);
-                    }
+                    for (int i = 0; i < 8; ++i) v[i] = tk_siluf(g[i >> 2][i & 3]) * u[i >> 2][i & 3];
+                    quantize_chunk8(v, 32 * b + (lane & 31), r, lo);
+                };
+                if (hw < nb) finish(0, hw);
+                for (int b = hw + nhw; b < nb; b += nhw) { request(0, b); wait_vmcnt<0>(); finish(0, b); }
+                for (int r = 1; r < a.nrows; ++r)
+                    for (int b = hw; b < nb; b += nhw) { request(r, b); wait_vmcnt<0>(); finish(r, b); }
             };
             if (a.fks == 1) gated_rows(std::integral_constant<int, 1>{});
             else gated_rows(std::integral_constant<int, TK_RMS_MAX_KS>{});
@@ -1249,12 +1273,6 @@ __device__ __forceinline__ void unpack_q6_x32(const FragQ6& f0, const FragQ6& f1
     o.dmin = 0.0f;
 }
 
-/* s_waitcnt vmcnt(N) alone (expcnt / lgkmcnt untouched): until all but this wave's N youngest vector-memory operations are done.  The
- * LDS-DMA pieces of a chunk are invisible to the compiler's own wait insertion, so the ring is guarded by hand. */
-template <int N> __device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N <= 63, "the counter has six bits");
-    __builtin_amdgcn_s_waitcnt(0x0F70 | (N & 15) | ((N >> 4) << 14));
-}
 /* until all but its `left` youngest batches of N requests are done; left <= MOST */
 template <int N, int MOST> __device__ __forceinline__ void wait_batches(int left) {
     if constexpr (MOST == 0) wait_vmcnt<0>();
