@@ -180,6 +180,17 @@ def test_detector_full_frame_path_and_batch(gpu):
     assert det.detect(fr[0]) == []                                            # empty result set
 
 
+@pytest.mark.parametrize("n", [9, 12, 17])
+def test_frames_that_arrive_while_the_network_runs(gpu, n):
+    """large frames for a small network: the later ones are uploaded behind the first ones' launches; every frame's boxes are those it gives alone, call after call"""
+    rng = np.random.default_rng(n)
+    det = gpu.ObjectDetector(model="synthetic://yolov8n?seed=5&cls_bias=-1", width=320, height=320, conf=0.3, iou=0.5, max_batch=17)
+    for _ in range(2):
+        fr = [rng.integers(0, 256, (720, 1280, 3), dtype=np.uint8) for _ in range(n)]
+        res = det.detect_batch(fr)
+        assert res == [det.detect(f) for f in fr] and all(res) and res[0] != res[n - 1]
+
+
 @pytest.mark.skipif(not O.have_ref() or not os.path.exists(os.path.join(O.ROOT, "oracle", "_ref", "libtkref_attr.so")), reason="compiled reference not built")
 def test_box_attributes_equal_the_compiled_reference(gpu):
     """tk_classify_dominant_color / tk_classify_door_state on the GPU against the reference's own C compiled from its sources:

@@ -118,7 +118,19 @@ private:
     TkDetection* kept = nullptr;        /* in results */
     int32_t* n_kept = nullptr;
     bool begin_list();
+    bool network(int first, int B, const TkPreprocessArgs* frames); /* B frames through the network; candidates of frames first .. first + B - 1 */
+    bool suppress(int B);
+    bool upload(const uint8_t* const* frames, size_t frame_bytes, int first, int n, hipStream_t s);
+    hipStream_t upload_stream = nullptr; /* of a second part's frames; with the first call that has one */
+    hipEvent_t uploaded = nullptr;
 };
+
+/* How many of a call's B frames go to the device in front of the network; the others (B: none) while it runs on the first ones, and the network then takes them.  Frames
+ * come out of pageable memory at 24.5 GB/s and a pass of n frames at 640 x 640 takes about 380 + 117 n us: the part that makes the shortest call, where that saves a twentieth
+ * (below, two passes cost what they hide: 16 frames of 640 x 480 2.84 ms either way).  Fours of frames fill the layers' blocks better: 32 frames of 640 x 480 whole / 4 / 6 / 8 / 10
+ * first 5.25 / 4.83 / 4.95 / 4.84 / 4.93 ms; 64: 10.3 / 8.8 (8 first); 12 and 32 frames of 1280 x 720: 2.84 / 2.41, 7.55 / 6.23.  A frame's results do not depend on how many
+ * are beside it. */
+int tk_detector_first_part(int B, size_t frame_bytes, int in_w, int in_h);
 
 /* the same classification on a host frame (tightly packed RGB8), temporary device buffers on `device`: the reference's stand-alone
  * tk_classify_dominant_color / tk_classify_door_state entry points */

@@ -4,6 +4,8 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
+
 #include "../nn/tk_nn_kernels.h"
 
 /* Every stream of the library keeps the default priority: work on streams of different priorities has been seen to hang. */
@@ -660,12 +662,15 @@ __global__ __launch_bounds__(64) void k_yolo_scan(const tk_yolo_cand_t* cand, in
 
 TkDetector::~TkDetector() {
     if (model) (void)hipSetDevice(model->device);
+    if (upload_stream) (void)hipStreamSynchronize(upload_stream);
     if (stream) (void)hipStreamSynchronize(stream);
     void* ptrs[] = {frame_dev, arena, col, input, cand, order, n_cand, mask, results, list, n_list, attr_dev};
     for (void* p : ptrs) if (p) (void)hipFree(p);
     if (results_host) (void)hipHostFree(results_host);
     if (exec) exec->unload(); /* before its stream goes */
     if (stream) (void)hipStreamDestroy(stream);
+    if (upload_stream) (void)hipStreamDestroy(upload_stream);
+    if (uploaded) (void)hipEventDestroy(uploaded);
 }
 
 bool TkDetector::init(TkYoloModel* m, int w, int h, int mb) {
@@ -758,17 +763,7 @@ bool TkDetector::begin_list() {
     return true;
 }
 
-bool TkDetector::enqueue(int B, const TkPreprocessArgs* frames) {
-    if (!begin_list()) return false;
-    if (model->generic) {
-        if (!run_graph(B, nullptr)) return false;
-        hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, list, n_list, n_anchors, order, n_cand);
-        hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
-        hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept, n_list);
-        HIPQ(hipGetLastError());
-        list_clear = true;
-        return true;
-    }
+bool TkDetector::network(int first, int B, const TkPreprocessArgs* frames) {
     TkT x;
     x.p = input; x.B = B; x.H = in_h; x.W = in_w; x.C = 3; x.ld = 3;
     if (plans[B].empty()) plans[B].assign(model->specs.size(), TkConvPlan{});
@@ -778,12 +773,40 @@ bool TkDetector::enqueue(int B, const TkPreprocessArgs* frames) {
     ops.frame_bytes = frames ? (size_t)frames->in_stride * frames->in_h : 0;
     arena_used = 0;
     TkYoloV8n<TkGpuOps>::forward(ops, x, heads, model->nc);
-    hipLaunchKernelGGL(k_yolo_decode, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, heads[0], heads[1], heads[2], model->nc, n_anchors, conf, cand, list, n_list);
+    const size_t at = (size_t)first * n_anchors;
+    hipLaunchKernelGGL(k_yolo_decode, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, heads[0], heads[1], heads[2], model->nc, n_anchors, conf, cand + at, list + at, n_list + first);
+    HIPQ(hipGetLastError());
+    return true;
+}
+
+bool TkDetector::suppress(int B) {
     hipLaunchKernelGGL(k_yolo_rank, dim3((n_anchors + 63) / 64, B), dim3(256), 0, stream, list, n_list, n_anchors, order, n_cand);
     hipLaunchKernelGGL(k_yolo_mask, dim3(TK_YOLO_MAX_CAND / 256, TK_YOLO_MAX_CAND / 32, B), dim3(256), 0, stream, cand, n_anchors, order, n_cand, iou, mask);
     hipLaunchKernelGGL(k_yolo_scan, dim3(B), dim3(64), 0, stream, cand, n_anchors, order, n_cand, mask, kept, n_kept, n_list);
     HIPQ(hipGetLastError());
     list_clear = true;
+    return true;
+}
+
+bool TkDetector::enqueue(int B, const TkPreprocessArgs* frames) {
+    return begin_list() && (model->generic ? run_graph(B, nullptr) : network(0, B, frames)) && suppress(B);
+}
+
+int tk_detector_first_part(int B, size_t frame_bytes, int in_w, int in_h) {
+    const float up = (float)frame_bytes * (1.0f / 24.5e3f), per = 117.0f * ((float)in_w * (float)in_h / (640.0f * 640.0f));
+    auto net = [&](int n) { return 380.0f + per * (float)n; };
+    int best = B;
+    float least = 0.95f * (up * (float)B + net(B));
+    for (int f = 4; f < B; f += 4) {
+        const float us = up * (float)f + std::max(net(f), 100.0f /* launches */ + up * (float)(B - f)) + net(B - f);
+        if (us < least) { least = us; best = f; }
+    }
+    return best;
+}
+
+/* frames first .. first + n - 1 to their places on the device */
+bool TkDetector::upload(const uint8_t* const* frames, size_t frame_bytes, int first, int n, hipStream_t s) {
+    for (int b = first; b < first + n; ++b) HIPQ(hipMemcpyAsync(frame_dev + frame_bytes * b, frames[b], frame_bytes, hipMemcpyHostToDevice, s));
     return true;
 }
 
@@ -802,16 +825,32 @@ bool TkDetector::detect(int B, const uint8_t* const* frames, uint32_t w, uint32_
     a.src = frame_dev; a.in_w = w; a.in_h = h; a.in_stride = stride; a.bpp = bpp;
     a.dst = input; a.out_w = in_w; a.out_h = in_h; a.nhwc = model->generic ? 0 : 1; /* a file's graph takes planar NCHW */
     for (int c = 0; c < 3; ++c) { a.mean[c] = mean[c]; a.std_dev[c] = std_dev[c]; }
-    for (int b = 0; b < B; ++b) {
-        HIPQ(hipMemcpyAsync(frame_dev + fb * b, frames[b], fb, hipMemcpyHostToDevice, stream));
-        if (!model->generic) continue; /* the network takes the frames (TkGpuOps::run) */
-        TkPreprocessArgs f = a;
-        f.src = frame_dev + fb * b;
-        f.dst = input + (size_t)b * in_h * in_w * 3;
-        tk_launch_preprocess(f, stream);
-    }
     last_w = w; last_h = h; last_stride = stride; last_B = B;
-    if (!enqueue(B, model->generic ? nullptr : &a)) return false;
+    if (model->generic) {
+        if (!upload(frames, fb, 0, B, stream)) return false;
+        for (int b = 0; b < B; ++b) {
+            TkPreprocessArgs f = a;
+            f.src = frame_dev + fb * b;
+            f.dst = input + (size_t)b * in_h * in_w * 3;
+            tk_launch_preprocess(f, stream);
+        }
+        return enqueue(B) && fetch(B, out);
+    }
+    const int part = tk_detector_first_part(B, fb, in_w, in_h); /* the network takes the frames (TkGpuOps::run) */
+    if (part == B) return upload(frames, fb, 0, B, stream) && enqueue(B, &a) && fetch(B, out);
+    if (!upload_stream) {
+        HIPQ(tk_create_perception_stream(&upload_stream));
+        HIPQ(hipEventCreateWithFlags(&uploaded, hipEventDisableTiming));
+    }
+    if (!upload(frames, fb, 0, part, stream) || !begin_list() || !network(0, part, &a)) return false;
+    const bool there = upload(frames, fb, part, B - part, upload_stream);
+    if (!there || hipEventRecord(uploaded, upload_stream) != hipSuccess || hipStreamWaitEvent(stream, uploaded, 0) != hipSuccess) {
+        (void)hipStreamSynchronize(upload_stream); /* nothing reads the caller's frames any more */
+        if (there) error = "frames: the wait for their second part could not be enqueued";
+        return false;
+    }
+    a.src = frame_dev + fb * part;
+    if (!network(part, B - part, &a) || !suppress(B)) { (void)hipStreamSynchronize(upload_stream); return false; }
     return fetch(B, out);
 }
 
