@@ -379,8 +379,9 @@ int TkLlmSession::enqueue_matmul(const TkDevTensor* const* t, int nseg, int K, i
     for (int i = 0; i < nseg; ++i) a.seg[i] = seg_of(*t[i]);
     a.nseg = nseg; a.K = K; a.ks = ks; a.n_total = n_total; a.slab_pitch = pitch(n_total); a.nrows = nrows;
     set_act(a, act); a.out = out;
+    a.fold = tk_gemv_folds(a);
     tk_launch_gemv(a, s);
-    return ks;
+    return ks - a.fold + 1;
 }
 
 static bool producer_fusion_enabled() {

@@ -33,6 +33,7 @@ struct TkGemvArgs {
     const uint16_t* abs16; /* the same sums as two f16 images (sum = 2 hh + ll): [K/256][2][16][8] halves, M-tile stride abs_ts halves */
     float* out;
     int64_t slab_pitch, fslab_pitch; /* floats between the slabs of out, of fslab */
+    int fold;     /* wide passes: K ranges 0 .. fold - 1 are added up in slab 0 by the workgroups that make them, range fold + i goes to slab 1 + i (tk_gemv_folds(); 0, 1: none) */
     /* fuse != 0 (only where tk_gemv_fuses_producer() says so: passes of one or two rows, where a launch boundary costs more than the
      * producer's work repeated in every workgroup): the launch builds its int8 activation image in LDS itself and aq / ad / abs are unused.
      *   1: residual update + RMS norm + Q8 — k_rmsnorm_q8's arithmetic: row = fx_in + (the fks slabs of fslab, ascending; pitch
@@ -77,6 +78,8 @@ void tk_launch_rmsnorm_q8(float* x, const float* partial, int ks, int n_total_pa
                           TkActQ8 out, hipStream_t s);
 void tk_launch_residual_fold(float* x, const float* partial, int ks, int n_total, int64_t pitch, int D, int nrows, hipStream_t s);
 void tk_launch_gemv(const TkGemvArgs& a, hipStream_t s);
+/* TkGemvArgs::fold that this launch gains by: as many K ranges as a workgroup can walk while the others still finish no later than with a range each.  1: none */
+int tk_gemv_folds(const TkGemvArgs& a);
 void tk_launch_qkv_rope_append(const float* partial, int ks, int n_total, int64_t pitch, int n_head, int n_kv_head, int head_dim, const float* rope_cos,
                                const float* rope_sin, const int32_t* seq, const int32_t* pos, int nrows, float* qbuf, uint16_t* kcache,
                                uint16_t* vcache, int layer, int max_seq, int max_ctx, hipStream_t s);

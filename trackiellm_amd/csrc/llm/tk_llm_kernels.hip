@@ -1388,31 +1388,34 @@ __device__ __forceinline__ void g32_unpack(const typename G32Frag<Q4>::type& f0,
 }
 
 
-/* The K loop of one wave: its two weight tiles (32 weight rows) against its four 32-row M-tiles, block by block through the ring. */
+/* The K loop of one wave: its two weight tiles (32 weight rows) against its four 32-row M-tiles, block by block through the ring.  `at` blocks of the workgroup's `total`
+ * went before (at > 0: the first block of these is on its way already, in f0, f1 and slot s0); the block behind the last is requested while there is one. */
 template <bool Q4, int MTW, typename StageSmall, typename StagePart>
-__device__ __forceinline__ void g32_k_loop(const uint8_t* tile, size_t tile_bytes, ptrdiff_t tile_pitch, int nb, const uint8_t* ring, int slot_bytes, int lane,
-                                           float (&acc)[MTW][16], StageSmall&& stage_small, StagePart&& stage_part) {
-    typedef typename G32Frag<Q4>::type F;
-    F f0 = g32_load<Q4>(tile, lane), f1 = g32_load<Q4>(tile + tile_pitch, lane);
-    stage_small(0, 0);
-    for (int part = 0; part < 4; ++part) stage_part(0, 0, part);
+__device__ __forceinline__ void g32_k_loop(const uint8_t* tile, size_t tile_bytes, ptrdiff_t tile_pitch, int nb, int at, int total, int s0, const uint8_t* ring, int slot_bytes, int lane,
+                                           typename G32Frag<Q4>::type& f0, typename G32Frag<Q4>::type& f1, float (&acc)[MTW][16], StageSmall&& stage_small, StagePart&& stage_part) {
+    if (at == 0) {
+        f0 = g32_load<Q4>(tile, lane);
+        f1 = g32_load<Q4>(tile + tile_pitch, lane);
+        stage_small(0, s0);
+        for (int part = 0; part < 4; ++part) stage_part(0, s0, part);
+    }
 #pragma unroll 1
     for (int b = 0; b < nb; ++b) {
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        const bool more = b + 1 < nb;
+        const bool more = at + b + 1 < total;
         { /* a CU's two workgroups share its SIMDs under oldest-first arbitration: the older one runs near its solo rate, the younger one on what
            * is left and finishes alone (K loop 58 / 74 us for gate|up).  Issue priority that falls with progress lets the one that is behind
            * catch up: 63 / 71 us, launch set - 1..3 % (profiles/r03_gemm32_balance.txt) */
-            const int q = 4 * b / nb;
+            const int q = 4 * (at + b) / total;
             if (q == 0) __builtin_amdgcn_s_setprio(3);
             else if (q == 1) __builtin_amdgcn_s_setprio(2);
             else if (q == 2) __builtin_amdgcn_s_setprio(1);
             else __builtin_amdgcn_s_setprio(0);
         }
-        if (more) stage_small(b + 1, (b + 1) & 1);
+        if (more) stage_small(b + 1, (s0 + b + 1) & 1);
         const uint8_t* next = tile + (size_t)(more ? b + 1 : b) * tile_bytes; /* the last step re-requests its own tile: no branch around a load */
-        const Ptrs32 bp = block_ptrs32(ring + (b & 1) * slot_bytes, lane);
+        const Ptrs32 bp = block_ptrs32(ring + ((s0 + b) & 1) * slot_bytes, lane);
         ATile32 T;
         load_atile32<Q4>(T, bp, 0); /* tile 0's operands: their LDS latency hides under the unpack */
         __builtin_amdgcn_sched_barrier(0);
@@ -1426,15 +1429,20 @@ __device__ __forceinline__ void g32_k_loop(const uint8_t* tile, size_t tile_byte
         /* the ring's four staging parts ride on the tiles' MFMA phases: one per tile, the rest with the LAST tile when there are fewer than four
          * (with the first tile the same code needs 148 bytes of spill per lane) */
         gemm_block32<Q4, MTW>(o, T, bp, acc, [&](int t) {
-            stage_part(more ? b + 1 : b, (b + 1) & 1, t);
+            stage_part(more ? b + 1 : b, (s0 + b + 1) & 1, t);
             if (MTW < 4 && t == MTW - 1)
 #pragma unroll
-                for (int q = MTW; q < 4; ++q) stage_part(more ? b + 1 : b, (b + 1) & 1, q);
+                for (int q = MTW; q < 4; ++q) stage_part(more ? b + 1 : b, (s0 + b + 1) & 1, q);
         });
         __builtin_amdgcn_sched_barrier(0);
     }
 }
 
+/* all waves of the workgroup have read what they asked the LDS for; requests to memory stay on their way */
+__device__ __forceinline__ void g32_meet() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+/* FOLD (TkGemvArgs::fold): what a K range's slab costs is the norm behind it, which is bound by the slabs it reads: 2 048 rows of 4096, on average of o's four and down's
+ * seven, 50 us; 26 with one each, where a workgroup adds its ranges up itself.  The product's own time stays (down 345 -> 338 us): its workgroups come in as many rounds. */
 /* A workgroup = 4 waves, one per SIMD = four pairs of weight tiles (128 weight rows) x ONE part of the pass's rows (128 or 96 rows = MTW 32-row M-tiles per wave).  Two
  * workgroups share a CU (73 KiB of ring each) and nothing else.  The SIMD's two resident waves therefore belong to DIFFERENT workgroups: no barrier couples
  * them, so one's weight unpack (190 VALU instructions, no MFMA) drifts under the other's MFMA phases.  With both halves in one 8-wave
@@ -1444,35 +1452,44 @@ __device__ __forceinline__ void g32_k_loop(const uint8_t* tile, size_t tile_byte
  * L2 — the further parts' weight requests hit the lines the first one brought in.
  * Passes of more than 256 rows take as many parts as they need: 256 rows alone are 448 (gate | up, down), 384 (q | k | v) or 256 (o) workgroups on 512 slots, with a ramp and
  * a tail each.  A prompt of 8 192 rows through 32 layers, 4096 wide: passes of 256 rows 6.3 ms each, of 2 048 rows 41. */
-template <int TYPES, int MTW>
+template <int TYPES, int MTW, bool FOLD>
 __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups, int total_row_tiles, int n_parts) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int MT = TK_G32_MT;
     constexpr int CH = MT * TK_RING_TILE_BYTES;   /* one block of the ring */
     constexpr int OFF_AMN = MT * 4096, OFF_AD = MT * 4096 + MT * 512;
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
+    int lane = tid & 63;
     const int pair = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nb = a.K / a.ks / 256;
     const int nblk_total = a.K / 256;
-    int rpart = 0, unit = blockIdx.x;
+    /* FOLD: the first workgroups take the K ranges 0 .. fold - 1 one behind the other, the ones after them a range each */
+    int block = blockIdx.x, blocks = gridDim.x, k0 = 0, kdiv = a.ks, n_ranges = 1;
+    if (FOLD) {
+        const int per = groups * n_parts;
+        if (block < per) { blocks = per; kdiv = 1; n_ranges = a.fold; }
+        else { block -= per; blocks -= per; k0 = a.fold; kdiv = a.ks - a.fold; }
+    }
+    int rpart = 0, unit = block;
     if (n_parts > 1) {
-        const int units = gridDim.x / n_parts, body = (units & ~7) * n_parts; /* ids below `body`: a unit's parts on one XCD; the rest (units not a multiple of 8) adjacent */
-        if ((int)blockIdx.x < body) {
-            const int x = blockIdx.x & 7, idx = blockIdx.x >> 3;
+        const int units = blocks / n_parts, body = (units & ~7) * n_parts; /* ids below `body`: a unit's parts on one XCD; the rest (units not a multiple of 8) adjacent */
+        if (block < body) {
+            const int x = block & 7, idx = block >> 3;
             rpart = idx % n_parts;
             unit = idx / n_parts * 8 + x;
         } else {
-            const int r = blockIdx.x - body;
+            const int r = block - body;
             rpart = r % n_parts;
             unit = (units & ~7) + r / n_parts;
         }
     }
-    const int ksi = unit % a.ks;
-    const int blk0 = ksi * nb;
+    int ksi = k0 + unit % kdiv;
+    const int column = unit / kdiv, slab = FOLD ? (ksi < a.fold ? 0 : ksi - a.fold + 1) : ksi;
+    int blk0 = ksi * nb;
 
     /* a.swiglu (gate | up launches with one K range): the wave's 32 weight rows are gate tile i and up tile i — the same 16 hidden columns —
      * so its epilogue can form silu(gate) * up; the four waves of a workgroup take adjacent tiles (their stores join to 256 B per row) */
-    int rt = a.swiglu ? 4 * (unit / a.ks) + pair : 2 * (unit / a.ks + pair * groups); /* first of this wave's two row tiles */
+    int rt = a.swiglu ? 4 * column + pair : 2 * (column + pair * groups); /* first of this wave's two row tiles */
     const bool active = rt < (a.swiglu ? a.seg[0].row_tiles : total_row_tiles);
     if (!active) rt = 0;
     int seg = 0, row_base = 0;
@@ -1487,12 +1504,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
     const size_t tile_bytes = is4 ? (size_t)TK_Q4K_TILE_BYTES : (size_t)TK_Q6K_TILE_BYTES;
     const ptrdiff_t tile_pitch = a.swiglu ? a.seg[1].tiles - a.seg[0].tiles : (ptrdiff_t)((size_t)nblk_total * tile_bytes);
     const uint8_t* tile = a.seg[seg].tiles + ((size_t)rt * nblk_total + blk0) * tile_bytes;
-
-    float acc[MTW][16];
-#pragma unroll
-    for (int t = 0; t < MTW; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
 
     /* ring staging: of the part's eight 16-row M-tiles, `pair` and `pair + 4` belong to this wave.  The int8 image (4 x 1 KiB pieces per
      * tile, every lane takes part: no exec masking, so the issue can sit between the MFMA phases of the tile loop) in four parts of two
@@ -1530,55 +1541,91 @@ __global__ __launch_bounds__(256, 2) void k_gemm32_w4a8(TkGemvArgs a, int groups
         }
     };
 
-    if (!active) { /* a workgroup's spare wave slots (row tiles beyond the matrix) still stage their share of the ring */
-        stage_small(0, 0);
-        for (int part = 0; part < 4; ++part) stage_part(0, 0, part);
+    /* The K ranges of this workgroup (FOLD; else one), block by block without a stop: a range's first block is on its way while the range before is stored */
+    int s0 = 0;
+    FragQ4 f4[2];
+    FragQ6 f6[2];
 #pragma unroll 1
-        for (int b = 0; b < nb; ++b) {
-            __builtin_amdgcn_s_waitcnt(0);
-            __syncthreads();
-            if (b + 1 < nb) { stage_small(b + 1, (b + 1) & 1); for (int part = 0; part < 4; ++part) stage_part(b + 1, (b + 1) & 1, part); }
+    for (int range = 0; range < (FOLD ? n_ranges : 1); ++range) {
+        if (FOLD) asm volatile("" : "+v"(lane)); /* nothing that is made of it is kept from range to range: there is no register for that */
+        if (FOLD && range) {
+            blk0 += nb;
+            tile += (size_t)nb * tile_bytes;
+            s0 = (s0 + nb) & 1;
         }
-        return;
-    }
-    if (HAS4 && is4) g32_k_loop<true, MTW>(tile, tile_bytes, tile_pitch, nb, lds, CH, lane, acc, stage_small, stage_part);
-    if (HAS6 && !is4) g32_k_loop<false, MTW>(tile, tile_bytes, tile_pitch, nb, lds, CH, lane, acc, stage_small, stage_part);
-
-    /* Epilogue: 64 accumulator registers per lane.  Stored as they stand, a store instruction writes one dword per lane (two 128-byte row
-     * segments): 64 store instructions per wave, and the tail of the launch is store-ISSUE bound (exit - loop end 4 us of gate|up's 76).
-     * So each 32 x 32 tile goes through LDS once — into the 4 KiB ring regions THIS wave staged itself (M-tiles `pair` and `pair + 4` of
-     * the slot nobody reads any more: after the wave's own vmcnt(0) no DMA can land there, and LDS operations of one wave execute in order,
-     * so no barrier is needed) — and comes back as 16 bytes per lane: lane (row r8 = l >> 3, column group l & 7) holds four consecutive
-     * columns of one row, a store instruction writes eight whole 128-byte row segments, 16 instructions per wave instead of 64. */
-    {
-        __builtin_amdgcn_s_waitcnt(0);
-        uint8_t* scr[2] = {lds + (nb & 1) * CH + pair * 4096, lds + (nb & 1) * CH + (pair + 4) * 4096};
-        const int h = lane >> 5, n32 = lane & 31;
-        const int n0 = a.col0 + row_base + rt * TK_TILE_ROWS + 4 * (lane & 7);
-#pragma unroll
-        for (int t = 0; t < MTW; ++t) {
-            float* sp = (float*)scr[t & 1];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) sp[((r & 3) + 8 * (r >> 2) + 4 * h) * 32 + n32] = acc[t][r];
-            if (a.swiglu) { /* columns 0..15 of the tile are gate, 16..31 up, of hidden columns 16 rt ..: h = silu(gate) * up, what k_swiglu_q8 evaluates */
-#pragma unroll
-                for (int i = 0; i < 2; ++i) {
-                    const int rl = 16 * i + (lane >> 2), cg = 4 * (lane & 3);
-                    const v4f g = *(const v4f*)(sp + rl * 32 + cg), u = *(const v4f*)(sp + rl * 32 + 16 + cg);
-                    v4f hv;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) hv[j] = tk_siluf(g[j]) * u[j];
-                    const int row = (t32_0 + t) * 32 + rl;
-                    if (row < a.nrows) *(v4f*)&a.out[(size_t)row * a.n_total + rt * TK_TILE_ROWS + cg] = hv;
-                }
-                continue;
+        if (!active) { /* a workgroup's spare wave slots (row tiles beyond the matrix) still stage their share of the ring */
+            if (range == 0) {
+                stage_small(0, 0);
+                for (int part = 0; part < 4; ++part) stage_part(0, 0, part);
             }
+#pragma unroll 1
+            for (int b = 0; b < nb; ++b) {
+                __builtin_amdgcn_s_waitcnt(0);
+                __syncthreads();
+                if (range * nb + b + 1 < n_ranges * nb) { stage_small(b + 1, (s0 + b + 1) & 1); for (int part = 0; part < 4; ++part) stage_part(b + 1, (s0 + b + 1) & 1, part); }
+            }
+            if (FOLD) g32_meet();
+            continue;
+        }
+        float acc[MTW][16];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int rl = 8 * i + (lane >> 3);
-                const v4f v = *(const v4f*)(sp + rl * 32 + 4 * (lane & 7));
-                const int row = (t32_0 + t) * 32 + rl;
-                if (row < a.nrows) *(v4f*)&a.out[ksi * a.slab_pitch + (int64_t)row * a.n_total + n0] = v;
+        for (int t = 0; t < MTW; ++t)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[t][r] = 0.0f;
+        if (HAS4 && is4) g32_k_loop<true, MTW>(tile, tile_bytes, tile_pitch, nb, range * nb, n_ranges * nb, s0, lds, CH, lane, f4[0], f4[1], acc, stage_small, stage_part);
+        if (HAS6 && !is4) g32_k_loop<false, MTW>(tile, tile_bytes, tile_pitch, nb, range * nb, n_ranges * nb, s0, lds, CH, lane, f6[0], f6[1], acc, stage_small, stage_part);
+        if (FOLD) asm volatile("" : "+v"(lane));
+        /* Epilogue: 64 accumulator registers per lane.  Stored as they stand, a store instruction writes one dword per lane (two 128-byte row
+         * segments): 64 store instructions per wave, and the tail of the launch is store-ISSUE bound (exit - loop end 4 us of gate|up's 76).
+         * So each 32 x 32 tile goes through LDS once — into the 4 KiB ring regions THIS wave staged itself (M-tiles `pair` and `pair + 4` of
+         * the slot nobody reads any more: after the wave's own vmcnt(0) no DMA can land there, and LDS operations of one wave execute in order,
+         * so no barrier is needed) — and comes back as 16 bytes per lane: lane (row r8 = l >> 3, column group l & 7) holds four consecutive
+         * columns of one row, a store instruction writes eight whole 128-byte row segments, 16 instructions per wave instead of 64. */
+        {
+            /* FOLD: the other slot is filling with the next range's first block, so the one just read is used, once all waves are through with it */
+            if (FOLD) g32_meet();
+            else __builtin_amdgcn_s_waitcnt(0);
+            uint8_t* const idle = lds + ((s0 + nb - (FOLD ? 1 : 0)) & 1) * CH;
+            uint8_t* scr[2] = {idle + pair * 4096, idle + (pair + 4) * 4096};
+            const int h = lane >> 5, n32 = lane & 31;
+            const int n0 = a.col0 + row_base + rt * TK_TILE_ROWS + 4 * (lane & 7);
+            float* const out = a.out + slab * a.slab_pitch + n0;
+            const bool add = FOLD && range > 0;
+            v4f before[4]; /* the sum of the ranges so far, which this lane wrote; a tile's is asked for in front of the tile's way through the LDS */
+            auto ask = [&](int t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int row = (t32_0 + t) * 32 + 8 * i + (lane >> 3);
+                    before[i] = *(const v4f*)&out[(int64_t)(row < a.nrows ? row : a.nrows - 1) * a.n_total];
+                }
+            };
+#pragma unroll
+            for (int t = 0; t < MTW; ++t) {
+                float* sp = (float*)scr[t & 1];
+                if (add) ask(t);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) sp[((r & 3) + 8 * (r >> 2) + 4 * h) * 32 + n32] = acc[t][r];
+                if (a.swiglu) { /* columns 0..15 of the tile are gate, 16..31 up, of hidden columns 16 rt ..: h = silu(gate) * up, what k_swiglu_q8 evaluates */
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        const int rl = 16 * i + (lane >> 2), cg = 4 * (lane & 3);
+                        const v4f g = *(const v4f*)(sp + rl * 32 + cg), u = *(const v4f*)(sp + rl * 32 + 16 + cg);
+                        v4f hv;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) hv[j] = tk_siluf(g[j]) * u[j];
+                        const int row = (t32_0 + t) * 32 + rl;
+                        if (row < a.nrows) *(v4f*)&a.out[(size_t)row * a.n_total + rt * TK_TILE_ROWS + cg] = hv;
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int rl = 8 * i + (lane >> 3);
+                    v4f v = *(const v4f*)(sp + rl * 32 + 4 * (lane & 7));
+                    if (add) v = before[i] + v;
+                    const int row = (t32_0 + t) * 32 + rl;
+                    if (row < a.nrows) *(v4f*)&out[(int64_t)row * a.n_total] = v;
+                }
             }
         }
     }
@@ -1618,6 +1665,29 @@ static int tk_g32_from() {
     return v;
 }
 
+struct G32Shape { int columns, n_parts; bool four; };
+static G32Shape g32_shape(const TkGemvArgs& a) {
+    int row_tiles = 0;
+    for (int i = 0; i < a.nseg; ++i) row_tiles += a.seg[i].row_tiles;
+    const int pairs = a.swiglu ? a.seg[0].row_tiles : row_tiles / 2; /* every segment holds a multiple of 4 row tiles: pairs never straddle segments */
+    /* parts of 128 rows (four 32-row tiles a wave) or of 96, whichever makes the shorter pass: a block costs a wave its weights' unpack, worth one and a half
+     * tiles, and its tiles (1 980 and 1 315 cycles).  Prompts of 260, 288, 544 rows through 16 layers, all parts of 128 / by this rule: 5.20 / 4.75, 5.38 / 4.92,
+     * 8.71 / 8.47 ms; one part alone always holds four tiles */
+    const int tiles32 = (a.nrows + 31) / 32;
+    const int parts4 = (tiles32 + 3) / 4, parts3 = (tiles32 + 2) / 3;
+    const bool four = parts4 == 1 || 11 * parts4 <= 9 * parts3;
+    return G32Shape{(pairs + 3) / 4, four ? parts4 : parts3, four};
+}
+
+/* 512 workgroups run at once.  2 048 rows x 4096: o's and down's 512 blocks of columns and rows, four and seven ranges in one round; 1 024 rows: two and four ranges in
+ * one workgroup, the others one by one.  q | k | v, 768 blocks, could take three of its four ranges together: k_qkv_rope_append 43 -> 32 us, the product 148 -> 157; left as it is. */
+int tk_gemv_folds(const TkGemvArgs& a) {
+    if (a.nseg != 1 || a.ks < 2 || a.nrows < tk_g32_from()) return 1;
+    const G32Shape g = g32_shape(a);
+    const int64_t slots = 2 * TK_NUM_CU, units = (int64_t)g.columns * g.n_parts, rounds = (units * a.ks + slots - 1) / slots, longest = rounds / ((units + slots - 1) / slots);
+    return (int)(longest < 1 ? 1 : longest < a.ks ? longest : a.ks);
+}
+
 void tk_launch_gemv(const TkGemvArgs& a, hipStream_t s) {
     int row_tiles = 0;
     for (int i = 0; i < a.nseg; ++i) row_tiles += a.seg[i].row_tiles;
@@ -1636,23 +1706,19 @@ void tk_launch_gemv(const TkGemvArgs& a, hipStream_t s) {
     if (a.nrows >= tk_g32_from()) {
         /* from tk_g32_from() rows on: the 32x32x32 kernel, one type per wave (a mixed q / k / v launch needs no split): four (weight-tile pair) slots per
          * workgroup, one workgroup per part of the rows */
-        const int pairs = a.swiglu ? a.seg[0].row_tiles : row_tiles / 2; /* every segment holds a multiple of 4 row tiles: pairs never straddle segments */
-        const int g32 = (pairs + 3) / 4;
-        /* parts of 128 rows (four 32-row tiles a wave) or of 96, whichever makes the shorter pass: a block costs a wave its weights' unpack, worth one and a half
-         * tiles, and its tiles (1 980 and 1 315 cycles).  Prompts of 260, 288, 544 rows through 16 layers, all parts of 128 / by this rule: 5.20 / 4.75, 5.38 / 4.92,
-         * 8.71 / 8.47 ms; one part alone always holds four tiles */
-        const int tiles32 = (a.nrows + 31) / 32;
-        const int parts4 = (tiles32 + 3) / 4, parts3 = (tiles32 + 2) / 3;
-        const bool four = parts4 == 1 || 11 * parts4 <= 9 * parts3;
-        const int n_parts = four ? parts4 : parts3;
+        const G32Shape g = g32_shape(a);
+        const int g32 = g.columns, n_parts = g.n_parts;
+        const bool fold = a.fold > 1;
         const size_t ldsb = (size_t)2 * TK_G32_MT * TK_RING_TILE_BYTES;
-        const dim3 grid(g32 * a.ks * n_parts);
-#define TK_G32_LAUNCH_M(TYV, MTWV) hipLaunchKernelGGL((k_gemm32_w4a8<TYV, MTWV>), grid, dim3(256), ldsb, s, a, g32, row_tiles, n_parts)
-#define TK_G32_LAUNCH(TYV) do { if (four) TK_G32_LAUNCH_M(TYV, 4); else TK_G32_LAUNCH_M(TYV, 3); } while (0)
+        const dim3 grid(g32 * (fold ? a.ks - a.fold + 1 : a.ks) * n_parts);
+#define TK_G32_LAUNCH_M(TYV, MTWV, FO) hipLaunchKernelGGL((k_gemm32_w4a8<TYV, MTWV, FO>), grid, dim3(256), ldsb, s, a, g32, row_tiles, n_parts)
+#define TK_G32_LAUNCH_F(TYV, FO) do { if (g.four) TK_G32_LAUNCH_M(TYV, 4, FO); else TK_G32_LAUNCH_M(TYV, 3, FO); } while (0)
+#define TK_G32_LAUNCH(TYV) do { if (fold) TK_G32_LAUNCH_F(TYV, true); else TK_G32_LAUNCH_F(TYV, false); } while (0)
         if (types == 1) TK_G32_LAUNCH(1);
         else if (types == 2) TK_G32_LAUNCH(2);
-        else TK_G32_LAUNCH(3);
+        else TK_G32_LAUNCH_F(3, false);
 #undef TK_G32_LAUNCH
+#undef TK_G32_LAUNCH_F
 #undef TK_G32_LAUNCH_M
         return;
     }
@@ -3026,7 +3092,7 @@ const char* tk_llm_prepare_device(int device) {
 #define TK_OPT(fn) do { if (e == hipSuccess) e = opt_in_lds(fn); } while (0)
 #define TK_OPT_GEMM(MTV) do { TK_OPT((k_gemm_w4a8<MTV, 1, 1>)); TK_OPT((k_gemm_w4a8<MTV, 2, 1>)); TK_OPT((k_gemm_w4a8<MTV, 3, 1>)); } while (0)
     TK_OPT_GEMM(4); TK_OPT_GEMM(6); TK_OPT_GEMM(8); TK_OPT_GEMM(10); TK_OPT_GEMM(12); TK_OPT_GEMM(14); TK_OPT_GEMM(16);
-#define TK_OPT_G32(TYV) do { TK_OPT((k_gemm32_w4a8<TYV, 4>)); TK_OPT((k_gemm32_w4a8<TYV, 3>)); } while (0)
+#define TK_OPT_G32(TYV) do { TK_OPT((k_gemm32_w4a8<TYV, 4, false>)); TK_OPT((k_gemm32_w4a8<TYV, 3, false>)); if (TYV < 3) { TK_OPT((k_gemm32_w4a8<(TYV) & 1 ? 1 : 2, 4, true>)); TK_OPT((k_gemm32_w4a8<(TYV) & 1 ? 1 : 2, 3, true>)); } } while (0)
     TK_OPT_G32(1); TK_OPT_G32(2); TK_OPT_G32(3);
 #undef TK_OPT_G32
 #define TK_OPT_GEMV_F(PFV, MTV, FUV) do { TK_OPT((k_gemv_w4a8<PFV, MTV, 1, FUV>)); TK_OPT((k_gemv_w4a8<PFV, MTV, 2, FUV>)); TK_OPT((k_gemv_w4a8<PFV, MTV, 3, FUV>)); } while (0)
