@@ -64,6 +64,14 @@ def test_its_own_cut(gpu, size, k, stride):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("N,out,res", [(16, 0, 0), (80, 4, 8), (80, 2, 0), (80, 0, 3), (79, 1, 1), (78, 0, 2), (20, 12, 4)])
+def test_four_channels_of_a_pixel_at_once_and_one_by_one(gpu, N, out, res):
+    """outputs and residuals whose pixels are whole aligned fours of channels, and such that are not"""
+    check(gpu, 7, 2, 9, 11, 32, N, 3, 1, pad=(0, 0, out, res), res=True)
+    check(gpu, 8, 2, 9, 11, 32, N, 3, 2, (2, 1, 2, 2, 7), pad=(0, 0, out, 0), bias=False, act=0)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("up", [(0, 0), (1, 0), (0, 1), (1, 1)])
 def test_two_sources(gpu, up):
     check(gpu, 5, 2, 12, 18, 96, 40, 1, 1, split=32, up=up, pad=(4, 12, 0, 0))

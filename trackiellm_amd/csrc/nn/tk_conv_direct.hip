@@ -23,6 +23,7 @@ __device__ __forceinline__ int cd_quot(int n, uint32_t by) { return (int)__umulh
 struct CdArgs {
     TkConvDirect c;
     int wn, th, tw, pw, ph;      /* waves along channels; tile; patch */
+    int vec;                     /* output, residual: four channels of a pixel are an aligned 16 bytes */
     int tiles_x, tiles;          /* spatial tiles of a row, of an image */
     int cp4;                     /* float4 of a pixel in the LDS: C / 4 + 1 */
     uint32_t by_c4[2], by_pw, by_tw, by_wn, by_cj, by_tiles_x; /* cd_div() of a source's float4 of a pixel, ... */
@@ -40,7 +41,7 @@ template <int V> struct CdCount { static constexpr int value = V; };
 /*
  * What bounds it.  Few tiles (one frame): the chain, about 46 cycles an MFMA where the wave has nothing else to issue, behind one trip to memory for the patch and the
  * first weights (40 x 40 x 64, 576 k: 7.0 us, of which 2.8 are the chain; k_gemm_f32_t16 10.4, whose slabs are a trip each).  Many: the fp32 pipe, which vector
- * instructions share: 71 % of it at 80 x 80 x 64 x 32 frames (139 us; the GEMM kernels 162), 57 % at 40 x 40 (43 us; 54), where patches and epilogues are a larger part.
+ * instructions share: 73 % of it at 80 x 80 x 64 x 32 frames (136 us; the GEMM kernels 162), 60 % at 40 x 40 (41 us; 54), where patches and epilogues are a larger part.
  * Weights come from the L2 once per tile of pixels, operands from the LDS: a padding of 16 bytes a pixel turns 16 pixels into 16 different groups of banks.
  */
 template <int P, int MT /* 16-pixel tiles a wave */, int PF /* pieces of weights in flight, even: operands are read a group ahead, into two sets */>
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdSet<P> s
 #pragma unroll
         for (int t = 0; t < 4; ++t)
 #pragma unroll
-            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(op[u % 2][m][t], w[u][t], acc[m], 0, 0, 0);
+            for (int m = 0; m < MT; ++m) acc[m] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][t], op[u % 2][m][t], acc[m], 0, 0, 0);
     };
     int q = 0;
     v4i at = table[0], at_next = table[1];
@@ -159,32 +160,39 @@ __global__ __launch_bounds__(64 * TK_CD_MAX_WAVES) void k_conv_direct(CdSet<P> s
             group(u, next);
         }
 
-    const int n = ntile * 16 + r;
+    /* The weights are the rows of the MFMAs, so that a lane ends with four channels, 4 g .. 4 g + 3, of one pixel, r, of a tile: an address and a store instead of four, where
+     * vector instructions share the pipe */
+    const int n = ntile * 16 + 4 * g;
     if (n >= c.N) return;
-    const float bias = c.bias ? c.bias[n] : 0.0f;
     const bool silu = c.act == TK_ACT_SILU;
-    float* yb = c.y + (int64_t)b * c.Ho * c.Wo * c.ldy + n;
-    const float* rb = c.residual ? c.residual + (int64_t)b * c.Ho * c.Wo * c.ldr + n : nullptr;
+    float bias[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bias[i] = c.bias && n + i < c.N ? c.bias[n + i] : 0.0f;
+    const int64_t image = (int64_t)b * c.Ho * c.Wo;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
-        int at[4];
-        float res[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int p = (wm * MT + m) * 16 + 4 * g + i;
-            const int py = cd_quot(p, a.by_tw), px = p - py * a.tw;
-            const int oy = oy0 + py, ox = ox0 + px;
-            at[i] = py < a.th && oy < c.Ho && ox < c.Wo ? oy * c.Wo + ox : -1;
-            res[i] = rb && at[i] >= 0 ? rb[(int64_t)at[i] * c.ldr] : 0.0f;
-        }
+        const int p = (wm * MT + m) * 16 + r;
+        const int py = cd_quot(p, a.by_tw), px = p - py * a.tw;
+        const int oy = oy0 + py, ox = ox0 + px;
+        if (py >= a.th || oy >= c.Ho || ox >= c.Wo) continue;
+        const int64_t pix = image + oy * c.Wo + ox;
+        float* y = c.y + pix * c.ldy + n;
+        const float* res = c.residual ? c.residual + pix * c.ldr + n : nullptr;
+        v4f before = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (res && a.vec) before = *(const v4f*)res;
         float v[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = acc[m][i] + bias;
+        for (int i = 0; i < 4; ++i) v[i] = acc[m][i] + bias[i];
         if (silu) tk_silu_all<4>(v);
+        if (a.vec) {
+            v4f o;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            if (rb) v[i] = v[i] + res[i];
-            if (at[i] >= 0) yb[(int64_t)at[i] * c.ldy] = v[i];
+            for (int i = 0; i < 4; ++i) o[i] = res ? v[i] + before[i] : v[i];
+            *(v4f*)y = o;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (n + i < c.N) y[i] = res ? v[i] + res[i] : v[i];
         }
     }
 }
@@ -222,6 +230,8 @@ static bool cd_fill(const TkConvDirect& c, const TkConvPlan& p, CdArgs* a) {
     if ((p.mt != 1 && p.mt != 2 && p.mt != 4) || p.wm < 1 || p.wn < 1 || p.wm * p.wn > TK_CD_MAX_WAVES || p.th < 1 || p.tw < 1) return false;
     if (p.th * p.tw > 16 * p.mt * p.wm) return false;
     a->c = c;
+    auto whole = [](const void* q, int ld) { return !(((uintptr_t)q) & 15) && !(ld & 3); };
+    a->vec = !(c.N & 3) && whole(c.y, c.ldy) && whole(c.residual, c.residual ? c.ldr : 0);
     a->wn = p.wn; a->th = p.th; a->tw = p.tw;
     a->ph = (p.th - 1) * c.stride + c.k; a->pw = (p.tw - 1) * c.stride + c.k;
     a->tiles_x = (c.Wo + p.tw - 1) / p.tw;
@@ -239,11 +249,14 @@ bool tk_conv_plan_ok(const TkConvDirect& c, const TkConvPlan& plan) {
     return tk_conv_direct_takes(c) && cd_fill(c, plan, &a);
 }
 
-/* Costs in cycles, fitted to 18 000 launches (the detector's 3 x 3 layers at 1, 3, 8 and 32 frames, every cut): the choice takes 1.4 % more than the best cut in the
- * mean, 15 % at most.  A workgroup's latency is its patch, its chains (32 cycles an MFMA) and its epilogue; the CU's further ones take turns on the pipe, which their
- * vector instructions share.  Five, six or seven waves load the SIMDs unevenly (64 -> 80 channels, 32 frames: 247 us with five, 190 with four).  The layers fitted are those of a
- * network of 640 x 640; whole calls of others, by the GEMM kernels / here: 320 x 320, 1 and 16 frames 779 / 405, 1914 / 1249 us; 512 x 288, 1 and 6 766 / 418, 1207 / 733;
- * 416 x 416, 2 and 16 847 / 496, 2269 / 1690; 1280 x 736, 1 and 16 1095 / 624, 8167 / 5361. */
+/* Costs in cycles, fitted to 8 000 launches (the detector's 3 x 3 layers at 1, 8, 24 and 32 frames, every cut): the choice takes 1.1 % more than the best cut in the
+ * mean, 9 % at most; at 4, 12 and 16 frames, which were not fitted, 0.5, 1.7 and 2.4 %, the largest 24.  A workgroup's latency is its patch, its chains (32 cycles an MFMA) and
+ * its epilogue; the CU's further ones take turns on the pipe, which their vector instructions share, and hide no more of a latency than there are of them: a patch that leaves
+ * room for one workgroup is paid whole (64 -> 80 channels of 80 x 80, 32 frames: 246 us with 16 x 16 pixels, 185 with 16 x 8).  Five, six or seven waves load the SIMDs unevenly
+ * (the same layer: 247 us with five, 190 with four).  Two, four and five channel tiles a wave, which read the patch once for all of them, are no quicker (1 - 2 % at 80
+ * channels) but at 20 x 20 x 256 -> 80 (69 / 56 us).  The layers fitted are those of a network of 640 x 640; whole calls of others, by the GEMM kernels / here before this fit:
+ * 320 x 320, 1 and 16 frames 779 / 405, 1914 / 1249 us; 512 x 288, 1 and 6 766 / 418, 1207 / 733; 416 x 416, 2 and 16 847 / 496, 2269 / 1690; 1280 x 736, 1 and 16
+ * 1095 / 624, 8167 / 5361. */
 static float cd_plan(const TkConvDirect& c, int only_mt, int only_waves, TkConvPlan* plan) {
     const int ntiles = (c.N + 15) / 16;
     const float G = (float)(c.k * c.k * c.C / 16);
@@ -267,9 +280,11 @@ static float cd_plan(const TkConvDirect& c, int only_mt, int only_waves, TkConvP
                     const float rounds = (float)((c.Wo + tw - 1) / tw) * (float)((c.Ho + th - 1) / th) * (float)c.B * (float)((ntiles + wn - 1) / wn) * (1.0f / 256.0f);
                     const int side_by_side = (int)(TK_CD_LDS / lds) < 16 / w ? (int)(TK_CD_LDS / lds) : 16 / w;
                     const float per = (float)((w + 3) / 4 * mt), share = 0.25f * (float)(w * mt), kib = (float)lds * (1.0f / 1024.0f);
-                    float turns = side_by_side > 1 ? 0.57f * rounds + 0.43f * ceilf(rounds) : ceilf(rounds);
+                    const float latency = 370.0f + 57.0f * kib + per * (G * 4.0f * 32.0f + 33.0f), work = share * (G * 4.0f * 34.3f + 37.0f) + 9.7f * kib + 79.0f * (float)w;
+                    float turns = side_by_side > 1 ? 0.32f * rounds + 0.68f * ceilf(rounds) : ceilf(rounds);
                     turns = turns > 1.0f ? turns - 1.0f : 0.0f;
-                    const float cost = 28.0f * kib + per * (G * 4.0f * 32.0f + 49.0f) + turns * (share * (G * 4.0f * 37.0f + 28.0f) + 7.4f * kib + 51.0f * (float)w);
+                    const float alone = latency / (float)side_by_side; /* what is not hidden under the others' */
+                    const float cost = latency + turns * (work > alone ? work : alone);
                     if (cost < best) {
                         best = cost;
                         *plan = TkConvPlan{mt, wm, wn, th, tw};
