@@ -1,6 +1,7 @@
 /* tk_conv_direct.hip — see tk_conv_direct.h */
 #include "tk_conv_direct.h"
 
+#include <algorithm>
 #include <atomic>
 #include <math.h>
 #include <mutex>
@@ -330,10 +331,12 @@ template <int P>
 static bool cd_launch(const TkConvDirect* c, const TkConvPlan* p, int n, hipStream_t s) {
     CdSet<P> set;
     set.n = n;
-    int blocks = 0;
+    int blocks = 0, order[P];
     size_t lds = 0;
+    for (int i = 0; i < P; ++i) order[i] = i;
+    std::stable_sort(order, order + n, [&](int i, int j) { return c[i].k * c[i].k * c[i].C > c[j].k * c[j].C * c[j].k; });
     for (int i = 0; i < P; ++i) {
-        const int j = i < n ? i : 0;
+        const int j = order[i < n ? i : 0];
         CdArgs& a = set.a[i];
         if (!tk_conv_direct_takes(c[j]) || !cd_fill(c[j], p[j], &a) || c[j].B != c[0].B || p[j].mt != p[0].mt || p[j].wm * p[j].wn != p[0].wm * p[0].wn) return false;
         set.first[i] = blocks;
