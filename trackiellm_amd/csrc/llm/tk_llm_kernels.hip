@@ -516,6 +516,38 @@ __device__ __forceinline__ void mma_q4(const OpsQ4& o, const uint8_t* lds_act, c
     }
 }
 
+/* The same for up to four rows in slots 0, 4, 8 and 12, of which a lane has one result: one MFMA a sub-block and its scale on that result.  With sixteen rows a lane has four, and eight
+ * multiply-adds for each are what folding the scales into the operands costs (16 rows: 1.95 / 1.96 ms a step of a 32-layer model). */
+struct OpsQ4s { uint32_t q[8], sc_lo, sc_hi; long bm; float dw, dmin; };
+__device__ __forceinline__ void unpack_q4s(const FragQ4& f, int lane, OpsQ4s& o) {
+    const uint32_t qs[8] = {f.q0.x, f.q0.y, f.q0.z, f.q0.w, f.q1.x, f.q1.y, f.q1.z, f.q1.w};
+    uint32_t mn_lo, mn_hi;
+    q4k_scales(f.h, &o.sc_lo, &o.sc_hi, &mn_lo, &mn_hi);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o.q[j] = qs[j];
+    o.bm = (lane >> 4) == 0 ? (long)(((unsigned long)mn_hi << 32) | mn_lo) : 0L;
+    o.dw = f16bits_to_f32(f.h.x & 0xffffu);
+    o.dmin = f16bits_to_f32(f.h.x >> 16);
+}
+__device__ __forceinline__ void mma_q4s(const OpsQ4s& o, const uint8_t* lds_act, const uint8_t* lds_amn, const float* lds_ad, int blk, int lane, float& acc) {
+    const v4i zero = {0, 0, 0, 0};
+    const uint8_t* ap = lds_act + (size_t)blk * 4096 + lane * 16;
+    int P = 0;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const long a = *(const long*)(ap + (j >> 1) * 1024 + (j & 1) * 8);
+        const uint32_t lo = o.q[j] & 0x0F0F0F0Fu, hi = (o.q[j] >> 4) & 0x0F0F0F0Fu;
+        const v4i c = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, (long)(((unsigned long)hi << 32) | lo), zero, 0, 0, 0);
+        P = mad24((int)(((j < 4 ? o.sc_lo : o.sc_hi) >> (8 * (j & 3))) & 0xFFu), c[0], P);
+    }
+    const uint8_t* mp = lds_amn + (size_t)blk * 256 + (lane & 15) * 8;
+    const v4i cl = __builtin_amdgcn_mfma_i32_16x16x32_i8(*(const long*)mp, o.bm, zero, 0, 0, 0);
+    const v4i ch = __builtin_amdgcn_mfma_i32_16x16x32_i8(*(const long*)(mp + 128), o.bm, zero, 0, 0, 0);
+    const float da = lds_ad[blk * TK_ROW_SLOTS + 4 * (lane >> 4)];
+    acc = tk_fmaf(o.dw * da, (float)P, acc);
+    acc = tk_fmaf(-(o.dmin * da), (float)((ch[0] << 6) + cl[0]), acc);
+}
+
 /* Q6_K: int8 operands 4 (q - 32) and the sixteen int8 group scales (one per 16 k: two per sub-block, applied to the two
  * half-masked MFMA results of the sub-block) */
 struct OpsQ6 { long b[8]; uint32_t sc[4]; float dw; };
@@ -536,17 +568,17 @@ __device__ __forceinline__ void unpack_q6(const FragQ6& f, OpsQ6& o) {
     o.dw = f16bits_to_f32(f.d);
 }
 
-template <int MT>
+template <int MT, int R>
 __device__ __forceinline__ void mma_q6(const OpsQ6& o, const uint8_t* lds_act, const float* lds_ad, size_t act_ts, int ad_ts, int blk, int lane,
                                        float (*acc)[4]) {
     const int g = lane >> 4;
     const v4i zero = {0, 0, 0, 0};
     const long mask_a = (g < 2) ? -1L : 0L;
-    int P[MT][4];
+    int P[MT][R];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) P[m][r] = 0;
+        for (int r = 0; r < R; ++r) P[m][r] = 0;
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int e = j & 1;
@@ -560,14 +592,14 @@ __device__ __forceinline__ void mma_q6(const OpsQ6& o, const uint8_t* lds_act, c
             const v4i ca = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, ba, zero, 0, 0, 0);
             const v4i cb = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, bb, zero, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) P[m][r] = mad24(scb, cb[r], mad24(sca, ca[r], P[m][r]));
+            for (int r = 0; r < R; ++r) P[m][r] = mad24(scb, cb[r], mad24(sca, ca[r], P[m][r]));
         }
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) {
         const v4f da = *(const v4f*)(lds_ad + m * ad_ts + blk * TK_ROW_SLOTS + 4 * g);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
+        for (int r = 0; r < R; ++r) {
             const float s1f = (o.dw * da[r]) * 0.25f; /* operand bytes are 4*(q-32): exact power-of-two fold */
             acc[m][r] = tk_fmaf(s1f, (float)P[m][r], acc[m][r]);
         }
@@ -629,6 +661,9 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
     float* lds_ad = (float*)(lds + MT * act_ts);
     uint8_t* lds_abs = (uint8_t*)(lds_ad + MT * ad_ts); /* sub-block sums as (l, h) int8 images, 256 B per block */
 
+    /* FUSE: row i in slot 4 i, so that a lane's first result is the only one that is a row */
+    constexpr bool FEW = FUSE != 0;
+    constexpr int R = FEW ? 1 : 4;
     float acc[MT][4];
 #pragma unroll
     for (int m = 0; m < MT; ++m)
@@ -719,7 +754,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                         v[i] = (h0[i] * scale) * w0[i];
                         v[4 + i] = (h1[i] * scale) * w1[i];
                     }
-                    quantize_chunk8(v, cl, r, lo);
+                    quantize_chunk8(v, cl, 4 * r, lo);
                 }
             }
         } else if (FUSE == 3) { /* k_att_pv_join's arithmetic: this K-range's blocks of the attention output */
@@ -738,7 +773,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                 float v[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) v[i] = tk_divf(((p[0][i >> 2][i & 3] + p[1][i >> 2][i & 3]) + p[2][i >> 2][i & 3]) + p[3][i >> 2][i & 3], ll);
-                quantize_chunk8(v, 32 * b + (lane & 31), r, lo);
+                quantize_chunk8(v, 32 * b + (lane & 31), 4 * r, lo);
             };
             request(0, hw);
             __builtin_amdgcn_sched_barrier(0);
@@ -774,7 +809,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                     float v[8];
 #pragma unroll
                     for (int i = 0; i < 8; ++i) v[i] = tk_siluf(g[i >> 2][i & 3]) * u[i >> 2][i & 3];
-                    quantize_chunk8(v, 32 * b + (lane & 31), r, lo);
+                    quantize_chunk8(v, 32 * b + (lane & 31), 4 * r, lo);
                 };
                 if (hw < nb) finish(0, hw);
                 for (int b = hw + nhw; b < nb; b += nhw) { request(0, b); wait_vmcnt<0>(); finish(0, b); }
@@ -829,27 +864,35 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
 
     /* steady state per tile: unpack (frees the packed fragment) -> request the tile PF blocks ahead into the same registers ->
      * MFMAs; so a tile has PF - 1 blocks of MFMA time plus its own to arrive */
+    auto unpack = [&](const FragQ4& f, auto& o) {
+        if constexpr (FEW) unpack_q4s(f, lane, o);
+        else unpack_q4(f, lane, o);
+    };
+    auto multiply = [&](const auto& o, int blk) {
+        if constexpr (FEW) mma_q4s(o, lds_act, lds_abs, lds_ad, blk, lane, acc[0][0]);
+        else mma_q4<MT>(o, lds_act, lds_abs, lds_ad, act_ts, abs_ts, ad_ts, blk, lane, acc);
+    };
     if (HAS4 && is4) {
         const uint8_t* tp = tile + PF * tile_bytes; /* one moving wave-uniform pointer: no per-load 64-bit VGPR address chains */
 #pragma unroll 1
         for (int g = 0; g < ngrp - 1; ++g, tp += PF * tile_bytes) {
 #pragma unroll
             for (int u = 0; u < PF; ++u) {
-                OpsQ4 o;
+                typename std::conditional<FEW, OpsQ4s, OpsQ4>::type o;
                 __builtin_amdgcn_sched_barrier(0);
-                unpack_q4(f4[HAS4 ? u : 0], lane, o);
+                unpack(f4[HAS4 ? u : 0], o);
                 __builtin_amdgcn_sched_barrier(0);
                 f4[HAS4 ? u : 0] = load_q4(tp + u * tile_bytes, lane);
                 __builtin_amdgcn_sched_barrier(0);
-                mma_q4<MT>(o, lds_act, lds_abs, lds_ad, act_ts, abs_ts, ad_ts, g * PF + u, lane, acc);
+                multiply(o, g * PF + u);
             }
         }
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
-            OpsQ4 o;
+            typename std::conditional<FEW, OpsQ4s, OpsQ4>::type o;
             __builtin_amdgcn_sched_barrier(0);
-            unpack_q4(f4[HAS4 ? u : 0], lane, o);
-            mma_q4<MT>(o, lds_act, lds_abs, lds_ad, act_ts, abs_ts, ad_ts, (ngrp - 1) * PF + u, lane, acc);
+            unpack(f4[HAS4 ? u : 0], o);
+            multiply(o, (ngrp - 1) * PF + u);
         }
     }
     if (HAS6 && !is4) {
@@ -864,7 +907,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
                 __builtin_amdgcn_sched_barrier(0);
                 f6[HAS6 ? u : 0] = load_q6(tp + u * tile_bytes, lane);
                 __builtin_amdgcn_sched_barrier(0);
-                mma_q6<MT>(o, lds_act, lds_ad, act_ts, ad_ts, g * PF + u, lane, acc);
+                mma_q6<MT, R>(o, lds_act, lds_ad, act_ts, ad_ts, g * PF + u, lane, acc);
             }
         }
 #pragma unroll
@@ -872,7 +915,7 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
             OpsQ6 o;
             __builtin_amdgcn_sched_barrier(0);
             unpack_q6(f6[HAS6 ? u : 0], o);
-            mma_q6<MT>(o, lds_act, lds_ad, act_ts, ad_ts, (ngrp - 1) * PF + u, lane, acc);
+            mma_q6<MT, R>(o, lds_act, lds_ad, act_ts, ad_ts, (ngrp - 1) * PF + u, lane, acc);
         }
     }
 
@@ -881,8 +924,8 @@ __global__ __launch_bounds__(512) void k_gemv_w4a8(TkGemvArgs a, int groups, int
 #pragma unroll
     for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int row = m * TK_ROW_SLOTS + 4 * g + r;
+        for (int r = 0; r < R; ++r) {
+            const int row = R == 1 ? g : m * TK_ROW_SLOTS + 4 * g + r;
             /* default-policy stores: the <= 1 MB of slabs of a narrow pass stay in L2 / the Infinity Cache for the consumer kernel, which is one
              * load latency long (decode step 2.277 -> 2.207 ms at 16 rows, 2.108 -> 2.038 ms at 1 row against non-temporal stores,
              * profiles/r03_smallbatch_variants.txt); the wide kernels keep non-temporal stores (29 MB per launch would only evict) */
