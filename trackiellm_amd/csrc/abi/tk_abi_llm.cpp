@@ -536,7 +536,8 @@ tk_error_code_t tk_mi355x_attention_plan_at(int device, int nrows, int n_head, i
     if (top_position < 0 || top_position >= max_ctx) return TK_ERROR_INVALID_ARGUMENT;
     /* the session's per-pass choices (TkLlmSession::choose_attention_top) on top of the launcher's */
     if (fused) {
-        if (max_ctx > tk_long_att_min_pos(1, max_ctx) && tk_attention_long_applies(nrows, n_head, n_kv_head, head_dim) && top_position >= tk_long_att_min_pos(nrows, max_ctx)) {
+        if (max_ctx > tk_long_att_min_pos(1, n_head, head_dim, max_ctx) && tk_attention_long_applies(nrows, n_head, n_kv_head, head_dim) &&
+            top_position >= tk_long_att_min_pos(nrows, n_head, head_dim, max_ctx)) {
             out[0] = 3; out[1] = n_head / n_kv_head; out[2] = 64; out[3] = 1;
         }
     } else if (out[0] == 2 && top_position < 128) {

@@ -286,7 +286,7 @@ bool TkLlmSession::init(TkLlmModel* m, int mseq, int mctx) {
     if (!alloc_act(&act_d, h.d_model, pass_rows, m->has_f16, error) || !alloc_act(&act_qd, QD, pass_rows, m->has_f16, error) || !alloc_act(&act_ff, h.d_ff, pass_rows, m->has_f16, error)) return false;
     HIPQ(hipMalloc((void**)&d_tiles, (size_t)(1 + pass_rows) * 4));
     HIPQ(hipMemset(d_tiles, 0, (size_t)(1 + pass_rows) * 4));
-    if (mctx > tk_long_att_min_pos(1, mctx) && tk_attention_long_applies(1, h.n_head, h.n_kv_head, h.head_dim))
+    if ((mctx > tk_long_att_min_pos(1, h.n_head, h.head_dim, mctx) || tk_attention_one_launch_fits(1, h.n_head, h.head_dim, mctx)) && tk_attention_long_applies(1, h.n_head, h.n_kv_head, h.head_dim))
         HIPQ(hipMalloc((void**)&d_scores, tk_attention_long_scratch_floats(h.n_head, h.head_dim, mctx) * sizeof(float)));
     /* RoPE table, double precision on the host (same formula as the oracle) */
     std::vector<float> cs((size_t)mctx * half), sn((size_t)mctx * half);
@@ -524,7 +524,7 @@ void TkLlmSession::choose_attention(const int32_t* pos, int nrows) {
 }
 void TkLlmSession::choose_attention_top(int top, int nrows) {
     tiled_pass = top >= TK_TILED_ATT_MIN_POS;
-    long_pass = d_scores != nullptr && nrows <= TK_LONG_ATT_MAX_ROWS && top >= tk_long_att_min_pos(nrows, max_ctx);
+    long_pass = d_scores != nullptr && nrows <= TK_LONG_ATT_MAX_ROWS && top >= tk_long_att_min_pos(nrows, model->hp.n_head, model->hp.head_dim, max_ctx);
 }
 
 bool TkLlmSession::capture_pass(hipGraphExec_t* slot, int nrows, bool lm_head, bool fused_attn) {

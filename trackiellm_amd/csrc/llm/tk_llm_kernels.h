@@ -121,7 +121,14 @@ void tk_launch_attention_prefill(const float* qbuf, const uint16_t* kcache, cons
  * 2.647 / 2.606; at 16 rows the fused kernels' 256 workgroups already cover the chip.  Windows of up to 512
  * positions take it from 256 on; in larger ones, where it would win from there as well (4096: 1 row at 448 1.892 / 1.743), the plan that the tests fix stays: 512. */
 #define TK_LONG_ATT_MAX_ROWS 8
-static inline int tk_long_att_min_pos(int nrows, int max_ctx) { return nrows > 4 ? 768 : nrows == 1 && max_ctx <= 512 ? 256 : 512; }
+/* A window that fits the LDS, of as many rows as leave a CU to every (row, head, class), alone on its device: scores and chains in one launch, from the first position on.  Other
+ * forms / this, ms a step: 1 row at 4, 100, 220, 400 positions 1.500 / 1.461, 1.538 / 1.472, 1.599 / 1.497, 1.651 (two launches) / 1.546; 2 rows at 4, 32, 200, 400 1.753 / 1.757,
+ * 1.767 / 1.752, 1.849 / 1.812, 2.006 / 1.874. */
+bool tk_attention_one_launch_fits(int nrows, int n_head, int head_dim, int max_ctx);
+bool tk_attention_one_launch(int nrows, int n_head, int head_dim, int max_ctx); /* fits, and no other session is on the device */
+static inline int tk_long_att_min_pos(int nrows, int n_head, int head_dim, int max_ctx) {
+    return tk_attention_one_launch(nrows, n_head, head_dim, max_ctx) ? 0 : nrows > 4 ? 768 : nrows == 1 && max_ctx <= 512 ? 256 : 512;
+}
 bool tk_attention_long_applies(int nrows, int n_head, int n_kv_head, int head_dim);
 size_t tk_attention_long_scratch_floats(int n_head, int head_dim, int max_ctx); /* floats of the `scores` scratch buffer */
 /* where such a launch leaves the classes' outputs [row][head][4][head_dim] and denominators [row][head][4]; join = false: its consumer joins them (TkGemvArgs::fuse 3) */

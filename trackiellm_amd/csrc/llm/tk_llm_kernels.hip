@@ -2772,6 +2772,114 @@ __global__ __launch_bounds__(64) void k_att_pv_chain(const float* __restrict__ s
     if (lane == 0) l_part[((int64_t)r * n_head + head) * TK_ATT_TSPLIT + j] = l;
 }
 
+/* Both in one launch where the whole window fits the LDS, for as many rows as leave a CU to each workgroup: workgroup = (class, head, row), which makes the head's scores itself
+ * (every class makes them all: 460 x 128 products, against a launch and a trip to memory) and then walks its class.  Outputs as k_att_pv_chain's.  What bounds it is the way in: a CU
+ * takes 118 KB of keys for 460 positions, and 29 of values.  One row of 32 heads at 437 positions: 5.2 + 5.0 us in two launches, 6.9 here. */
+__host__ __device__ __forceinline__ int att_class_rows(int max_ctx) { return ((max_ctx + 3) / 4 + 15) & ~15; } /* value rows of a class */
+static size_t att_class_lds(int max_ctx) {
+    const size_t keys = (size_t)(max_ctx + 3) & ~3, values = (size_t)att_class_rows(max_ctx);
+    return (keys + values) * 256 + 128 * 4 + keys * 4 + values * 4 + 16 * 4 + 2 * 256;
+}
+__global__ __launch_bounds__(512) void k_att_class(const float* __restrict__ partial, int ks, int n_total, int64_t pitch, const float* __restrict__ rope_cos, const float* __restrict__ rope_sin,
+                                                   uint16_t* __restrict__ kcache, uint16_t* __restrict__ vcache, const int32_t* __restrict__ seq, const int32_t* __restrict__ pos, int n_head,
+                                                   int n_kv_head, int layer, int max_seq, int max_ctx, float* __restrict__ pv_part, float* __restrict__ l_part) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t att_lds[];
+    constexpr int HD = 128, RB = HD * 2, PPR = RB / 16, HALF = HD / 2;
+    const int j = blockIdx.x, head = blockIdx.y, r = blockIdx.z, t = threadIdx.x, lane = t & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int grp = n_head / n_kv_head, kvh = head / grp, QD = n_head * HD, KVD = n_kv_head * HD;
+    const int p = pos[r], T = p + 1, keys = (max_ctx + 3) & ~3, values = att_class_rows(max_ctx);
+    const int nj = T > j ? (T - j + 3) / 4 : 0; /* positions j, j + 4, ... of this class */
+    uint8_t* kbuf = att_lds;                            /* [keys][256 B], 16-byte pieces XOR-swizzled by the row number */
+    uint8_t* vbuf = kbuf + (size_t)keys * RB;           /* [values][256 B] */
+    float* qs = (float*)(vbuf + (size_t)values * RB);   /* [HD] */
+    float* sc = qs + HD;                                /* [keys] */
+    float* ebuf = sc + keys;                            /* [values] */
+    float* red = ebuf + values;                         /* [16] */
+    uint16_t* own = (uint16_t*)(red + 16);              /* [2][HD]: this row's own K and V */
+    const int64_t run0 = (((int64_t)layer * max_seq + seq[r]) * n_kv_head + kvh) * (int64_t)max_ctx * HD;
+    /* four rows a request; rows past the context are the last one of the window again (never used) */
+    auto request = [&](const uint16_t* run, int row, int piece, uint8_t* to) {
+        row = row < max_ctx - 1 ? row : max_ctx - 1;
+        const auto gs = (const __attribute__((address_space(1))) void*)((const uint8_t*)run + (int64_t)row * RB + piece * 16);
+        __builtin_amdgcn_global_load_lds(gs, (__attribute__((address_space(3))) void*)to, 16, 0, 0);
+    };
+    for (int pc = wave; 4 * pc < T; pc += 8) {
+        const int row = 4 * pc + (lane >> 4);
+        request(kcache + run0, row, (lane & 15) ^ (row & (PPR - 1)), kbuf + pc * 1024);
+    }
+    for (int pc = wave; 4 * pc < nj; pc += 8) request(vcache + run0, j + 4 * (4 * pc + (lane >> 4)), lane & 15, vbuf + pc * 1024);
+    if (t < 3 * HALF) { /* q, k and v of this row: K-split sums, RoPE, f16 rounding (k_attention's FUSED prologue); one workgroup of the KV group appends */
+        const int what = t / HALF, i = t % HALF;
+        const int col = what == 0 ? head * HD + 2 * i : (what == 1 ? QD : QD + KVD) + kvh * HD + 2 * i;
+        const float c = rope_cos[(int64_t)p * HALF + i], sn = rope_sin[(int64_t)p * HALF + i];
+        const float2 ab = sum_partials_pair(partial, ks, n_total, pitch, r, col);
+        const float2 rot = {tk_fmaf(-ab.y, sn, ab.x * c), tk_fmaf(ab.x, sn, ab.y * c)};
+        if (what == 0) {
+            *(float2*)(qs + 2 * i) = rot;
+        } else {
+            const float2 kv = what == 1 ? rot : ab;
+            const uint32_t both = (uint32_t)tk_f32_to_f16(kv.x) | ((uint32_t)tk_f32_to_f16(kv.y) << 16);
+            if (j == 0 && head % grp == 0) *(uint32_t*)((what == 1 ? kcache : vcache) + run0 + (int64_t)p * HD + 2 * i) = both;
+            *(uint32_t*)(own + (what - 1) * HD + 2 * i) = both;
+        }
+    }
+    const float att_scale = tk_divf(1.0f, tk_sqrtf((float)HD));
+    __builtin_amdgcn_s_waitcnt(0x0F70); /* vmcnt(0): this wave's pieces */
+    __syncthreads();
+    if (t < PPR) *(uint4*)(kbuf + p * RB + ((t ^ (p & (PPR - 1))) * 16)) = *(const uint4*)((const uint8_t*)own + t * 16);
+    else if (t >= 64 && t < 64 + PPR && (p & 3) == j) *(uint4*)(vbuf + (p >> 2) * RB + (t - 64) * 16) = *(const uint4*)((const uint8_t*)(own + HD) + (t - 64) * 16);
+    __syncthreads();
+    float mx = -INFINITY;
+    for (int rr = t; rr < T; rr += 512) { /* one fma chain over head_dim per position */
+        const uint8_t* kr = kbuf + rr * RB;
+        uint4 kv[PPR];
+#pragma unroll
+        for (int u = 0; u < PPR; ++u) kv[u] = *(const uint4*)(kr + ((u ^ (rr & (PPR - 1))) * 16));
+        float a = 0.0f;
+#pragma unroll
+        for (int u = 0; u < PPR; ++u) {
+            const v4f q0 = *(const v4f*)(qs + 8 * u), q1 = *(const v4f*)(qs + 8 * u + 4);
+            const uint32_t kw[4] = {kv[u].x, kv[u].y, kv[u].z, kv[u].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) a = tk_fmaf(e < 4 ? q0[e] : q1[e - 4], f16bits_to_f32((kw[e >> 1] >> (16 * (e & 1))) & 0xffffu), a);
+        }
+        const float sv = a * att_scale;
+        sc[rr] = sv;
+        mx = tk_fmaxf(mx, sv);
+    }
+    mx = tk_wave_max(mx);
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    float m = red[0];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) m = tk_fmaxf(m, red[w]); /* a maximum does not depend on the order */
+    const int padded = (nj + 15) & ~15;
+    for (int i = t; i < padded; i += 512) ebuf[i] = i < nj ? tk_expf(sc[j + 4 * i] - m) : 0.0f;
+    /* value rows past the class: probability 0 on finite numbers */
+    for (int i = nj * (RB / 4) + t; i < padded * (RB / 4); i += 512) ((uint32_t*)vbuf)[i] = 0;
+    __syncthreads();
+    if (wave >= 2) return;
+    float acc = 0.0f, l = 0.0f; /* a dim a lane */
+    const uint8_t* vp = vbuf + (64 * wave + lane) * 2;
+    for (int k0 = 0; k0 < padded; k0 += 16) {
+        uint16_t v[16];
+        v4f e[4];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = *(const uint16_t*)(vp + (k0 + k) * RB);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e[k] = *(const v4f*)(ebuf + k0 + 4 * k);
+#pragma unroll
+        for (int k = 0; k < 16; ++k) {
+            acc = tk_fmaf(e[k >> 2][k & 3], f16bits_to_f32(v[k]), acc);
+            l = l + e[k >> 2][k & 3];
+        }
+    }
+    const int64_t at = ((int64_t)r * n_head + head) * TK_ATT_TSPLIT + j;
+    pv_part[at * HD + 64 * wave + lane] = acc;
+    if (t == 0) l_part[at] = l;
+}
+
 /* the four classes of every head joined in order, divided, quantised: workgroup = (row, the 256 / head_dim heads of a Q8 block) */
 template <int HD>
 __global__ __launch_bounds__(256) void k_att_pv_join(const float* __restrict__ pv_part, const float* __restrict__ l_part, int n_head, TkActQ8 out) {
@@ -2799,6 +2907,14 @@ TkAttentionParts tk_attention_long_parts(float* scores, int n_head, int head_dim
     return TkAttentionParts{pv, pv + (size_t)TK_LONG_ATT_MAX_ROWS * n_head * TK_ATT_TSPLIT * head_dim};
 }
 
+bool tk_attention_one_launch_fits(int nrows, int n_head, int head_dim, int max_ctx) {
+    return head_dim == 128 && att_class_lds(max_ctx) <= TK_MAX_DYN_LDS && nrows * n_head * TK_ATT_TSPLIT <= TK_NUM_CU;
+}
+static bool tk_device_is_shared_by_sessions();
+bool tk_attention_one_launch(int nrows, int n_head, int head_dim, int max_ctx) {
+    return tk_attention_one_launch_fits(nrows, n_head, head_dim, max_ctx) && !tk_device_is_shared_by_sessions();
+}
+
 void tk_launch_attention_long(const float* partial, int ks, int n_total, int64_t pitch, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
                               const int32_t* seq, const int32_t* pos, int nrows, int n_head, int n_kv_head, int head_dim, int layer, int max_seq, int max_ctx,
                               float* scores, TkActQ8 out, bool join, hipStream_t s) {
@@ -2806,6 +2922,12 @@ void tk_launch_attention_long(const float* partial, int ks, int n_total, int64_t
     const TkAttentionParts parts = tk_attention_long_parts(scores, n_head, head_dim, max_ctx);
     float *pv_part = parts.pv, *l_part = parts.l;
     const dim3 gc(TK_ATT_TSPLIT, n_head, nrows);
+    if (tk_attention_one_launch(nrows, n_head, head_dim, max_ctx)) {
+        hipLaunchKernelGGL(k_att_class, gc, dim3(512), att_class_lds(max_ctx), s, partial, ks, n_total, pitch, rope_cos, rope_sin, kcache, vcache, seq, pos, n_head, n_kv_head, layer, max_seq, max_ctx,
+                           pv_part, l_part);
+        if (join) hipLaunchKernelGGL((k_att_pv_join<128>), dim3(n_head / 2, nrows), dim3(256), 0, s, pv_part, l_part, n_head, out);
+        return;
+    }
     const int slots = nrows > 4 ? 2 : 3; /* 32 KB: the four workgroups a CU of eight rows are resident together (calls with two / three: 8 rows at 900 positions 2.62 / 2.79 ms, at 3000 3.37 / 3.74, 6 at 900 2.54 / 2.56) */
     const size_t lds = (size_t)slots * TK_PV_ROWS * head_dim * 2 + ((size_t)(max_ctx + 3) / 4 + TK_PV_ROWS) * sizeof(float);
     if (head_dim == 128) {
@@ -3148,6 +3270,7 @@ const char* tk_llm_prepare_device(int device) {
 #define TK_OPT_ATT_N(H) do { TK_OPT((k_attention<1, true, H, 128, 2>)); TK_OPT((k_attention<2, true, H, 128, 2>)); TK_OPT((k_attention<1, false, H, 128, 2>)); TK_OPT((k_attention<2, false, H, 128, 2>)); } while (0)
     TK_OPT_ATT_N(64); TK_OPT_ATT_N(128);
     TK_OPT(k_attention_narrow);
+    TK_OPT(k_att_class);
     TK_OPT((k_att_pv_chain<128, 2>)); TK_OPT((k_att_pv_chain<128, 3>)); TK_OPT((k_att_pv_chain<64, 2>)); TK_OPT((k_att_pv_chain<64, 3>));
     TK_OPT((k_attention_prefill<128>));
     TK_OPT((k_attention_prefill<64>));
