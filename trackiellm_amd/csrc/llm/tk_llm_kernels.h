@@ -121,11 +121,12 @@ void tk_launch_attention_prefill(const float* qbuf, const uint16_t* kcache, cons
  * 2.647 / 2.606; at 16 rows the fused kernels' 256 workgroups already cover the chip.  Windows of up to 512
  * positions take it from 256 on; in larger ones, where it would win from there as well (4096: 1 row at 448 1.892 / 1.743), the plan that the tests fix stays: 512. */
 #define TK_LONG_ATT_MAX_ROWS 8
-/* A window that fits the LDS, of as many rows as leave a CU to every (row, head, class), alone on its device: scores and chains in one launch, from the first position on.  Other
+/* A window that fits the LDS, of as many rows as leave a CU to every (row, head, class): scores and chains in one launch, from the first position on.  Other
  * forms / this, ms a step: 1 row at 4, 100, 220, 400 positions 1.500 / 1.461, 1.538 / 1.472, 1.599 / 1.497, 1.651 (two launches) / 1.546; 2 rows at 4, 32, 200, 400 1.753 / 1.757,
- * 1.767 / 1.752, 1.849 / 1.812, 2.006 / 1.874. */
+ * 1.767 / 1.752, 1.849 / 1.812, 2.006 / 1.874.  Beside other sessions' steps a launch that asks for whole CUs waits for them: two, three and eight sessions of one row at 420 positions
+ * 2.321 / 2.303, 3.107 / 3.159, 8.64 / 8.77, two and three at 64 2.211 / 2.141, 3.777 / 3.609; three of two rows at 200 3.655 / 3.775, so two rows take it alone. */
 bool tk_attention_one_launch_fits(int nrows, int n_head, int head_dim, int max_ctx);
-bool tk_attention_one_launch(int nrows, int n_head, int head_dim, int max_ctx); /* fits, and no other session is on the device */
+bool tk_attention_one_launch(int nrows, int n_head, int head_dim, int max_ctx); /* fits; more than one row: and no other session is on the device */
 static inline int tk_long_att_min_pos(int nrows, int n_head, int head_dim, int max_ctx) {
     return tk_attention_one_launch(nrows, n_head, head_dim, max_ctx) ? 0 : nrows > 4 ? 768 : nrows == 1 && max_ctx <= 512 ? 256 : 512;
 }

@@ -2912,7 +2912,7 @@ bool tk_attention_one_launch_fits(int nrows, int n_head, int head_dim, int max_c
 }
 static bool tk_device_is_shared_by_sessions();
 bool tk_attention_one_launch(int nrows, int n_head, int head_dim, int max_ctx) {
-    return tk_attention_one_launch_fits(nrows, n_head, head_dim, max_ctx) && !tk_device_is_shared_by_sessions();
+    return tk_attention_one_launch_fits(nrows, n_head, head_dim, max_ctx) && (nrows == 1 || !tk_device_is_shared_by_sessions());
 }
 
 void tk_launch_attention_long(const float* partial, int ks, int n_total, int64_t pitch, const float* rope_cos, const float* rope_sin, uint16_t* kcache, uint16_t* vcache,
